@@ -66,6 +66,16 @@ def load():
     return lib
 
 
+def load_native():
+    """The extension module dcnv4_amd._native (csrc/binding), which is linked against the library above."""
+    try:
+        from . import _native
+    except ImportError as e:
+        raise ImportError(f"dcnv4_amd._native is missing or does not fit this torch ({e}): build it with "
+                          "`python dcnv4_amd/build.py`") from e
+    return _native
+
+
 def check(rc):
     """Maps a status code to the exception class the reference's pybind layer would raise."""
     if rc == OK:

@@ -8,10 +8,22 @@ from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from .. import ext
-from .launch_spec import find_spec_bwd, findspec, launch_options_for
+from .launch_spec import GFX950_TABLE, find_spec_bwd, findspec, launch_options_for
+
+_native_dcnv4 = ext._native.dcnv4
+_ext_functions = (ext.dcnv4_forward, ext.dcnv4_backward)
 
 
 class DCNv4Function(Function):
+    @staticmethod
+    def apply(*args):
+        # The C++ path (csrc/binding/operators.cpp) does what the two methods below do when the library is to choose the
+        # launch: host time of a small forward 15 -> 6 us, of forward + backward 65-130 -> 40-60 us.  They run for tuned
+        # table entries, whose options are set around the calls, and for programs that wrap ext's functions.
+        if GFX950_TABLE or ext.dcnv4_forward is not _ext_functions[0] or ext.dcnv4_backward is not _ext_functions[1]:
+            return super(DCNv4Function, DCNv4Function).apply(*args)
+        return _native_dcnv4(*args)
+
     @staticmethod
     @custom_fwd(device_type="cuda")
     def forward(ctx, input, offset_mask, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,

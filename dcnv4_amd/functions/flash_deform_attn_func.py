@@ -9,10 +9,27 @@ from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from .. import ext
-from .launch_spec import attn_launch_options_for, findspec_attn, findspec_attn_bwd
+from .launch_spec import GFX950_TABLE, attn_launch_options_for, findspec_attn, findspec_attn_bwd
+
+_native = ext._native
+_EXT = ("flash_deform_attn_forward", "flash_deform_attn_backward", "flash_deform_attn_forward_split", "flash_deform_attn_backward_split")
+_ext_functions = tuple(getattr(ext, name) for name in _EXT)
+
+
+def _interpreted():
+    """Whether a call goes through the methods below rather than csrc/binding/operators.cpp: there are tuned table entries,
+    whose options are set around the calls, or a program has wrapped one of ext's functions."""
+    return bool(GFX950_TABLE) or any(getattr(ext, name) is not f for name, f in zip(_EXT, _ext_functions))
 
 
 class FlashDeformAttnFunction(Function):
+    @staticmethod
+    def apply(value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K=8):
+        if _interpreted():
+            return super(FlashDeformAttnFunction, FlashDeformAttnFunction).apply(
+                value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K)
+        return _native.flash_deform_attn(value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K)
+
     @staticmethod
     @torch.autocast("cuda", enabled=True, dtype=torch.float16)
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K=8):
@@ -48,6 +65,13 @@ class FlashDeformAttnSplitFunction(Function):
     with the logits in front of the operator (DCNv4_op/DCNv4/modules/flash_deform_attn.py:132-133); here both steps
     happen while the kernels stage their rows, and the backward returns the two gradients autograd would derive
     through the ``cat`` and the cast."""
+
+    @staticmethod
+    def apply(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_logits, im2col_step, K=8):
+        args = (value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_logits, im2col_step, K)
+        if _interpreted():
+            return super(FlashDeformAttnSplitFunction, FlashDeformAttnSplitFunction).apply(*args)
+        return _native.flash_deform_attn_split(*args)
 
     @staticmethod
     @torch.autocast("cuda", enabled=True, dtype=torch.float16)
