@@ -17,13 +17,15 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "libdcnv4_gfx950.so")
 SOURCES = ["capi.hip", "dcnv4_kernels.hip", "dcnv4_tiled_gather.hip", "dcnv4_grad_value.hip", "dcnv4_backward_dual.hip", "fda_kernels.hip", "fda_grad_value.hip",
-           "depthwise_conv.hip", "layer_norm.hip", "center_feature.hip"]
-HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "launch.hpp"), os.path.join(CSRC, "dcnv4_tiled_gather.hpp"), os.path.join(CSRC, "dcnv4_grad_value.hpp"),
+           "depthwise_conv.hip", "layer_norm.hip", "center_feature.hip",
+           "linear.hip"]
+HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "mfma.hpp"), os.path.join(CSRC, "linear.hpp"), os.path.join(CSRC, "launch.hpp"), os.path.join(CSRC, "dcnv4_tiled_gather.hpp"), os.path.join(CSRC, "dcnv4_grad_value.hpp"),
            os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]
 
 BINDING = os.path.join(CSRC, "binding")
-BINDING_SOURCES = ["module.cpp", "operators.cpp"]
-BINDING_HEADERS = [os.path.join(BINDING, "binding.hpp"), os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]
+BINDING_SOURCES = ["module.cpp", "operators.cpp", "modules.cpp", "layers.cpp"]
+BINDING_HEADERS = [os.path.join(BINDING, "binding.hpp"), os.path.join(BINDING, "modules.hpp"), os.path.join(CSRC, "linear.hpp"),
+                   os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -86,7 +88,7 @@ def build(force=False, verbose=True):
     if force or _stale(NATIVE_PATH, binding + [LIB_PATH]):
         lib = os.path.join(_torch_paths(), "lib")
         _run([CXX, "-shared", "-o", NATIVE_PATH] + binding + ["-L" + HERE, "-ldcnv4_gfx950", "-L" + lib, "-lc10", "-lc10_hip",
-             "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], "link")
+             "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,$ORIGIN"], "link")
     if verbose:
         print("built", LIB_PATH, "and", NATIVE_PATH)
     return LIB_PATH

@@ -1,0 +1,233 @@
+// Inference of a FlashInternImage layer (dcnv4_amd/models/flash_intern_image.py InternImageLayer) as one call: the
+// module's parameters are read from C++ and its kernels enqueued back to back, intermediates in one allocation.
+//
+// A picture or a few are bound by the host: 415 launches through Python took 6.5 ms for a T variant whose kernels run
+// 2.2 ms.  Here a layer is seven (pre-norm) or eight launches: the two projections in front of the operator share one,
+// bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.
+#include <ATen/autocast_mode.h>
+
+#include "../linear.hpp"
+#include "modules.hpp"
+
+namespace dcn::binding {
+namespace {
+
+struct NormParams {
+  Tensor weight, bias;
+  float eps = 0.f;
+};
+
+// What the kernels need of a layer; load() says whether they take it.
+struct Layer {
+  NormParams norm1, norm2;
+  Tensor gamma1, gamma2;
+  Tensor value_w, value_b, offset_w, offset_b, output_w, output_b, dw_w, dw_b;
+  Tensor fc1_w, fc1_b, fc2_w, fc2_b;
+  int kernel = 0, pad = 0, dilation = 0, group = 0, group_channels = 0, remove_center = 0, dw_kernel = 0;
+  float offset_scale = 1.f;
+  bool post_norm = false;
+  int64_t channels = 0, row = 0, hidden = 0;
+
+  bool load(const Module &m, const Tensor &x);
+};
+
+bool same(const Tensor &t, const Tensor &x, int64_t elements, bool optional) {
+  if (!t.defined()) return optional;
+  return t.scalar_type() == x.scalar_type() && t.device() == x.device() && t.numel() == elements && t.is_contiguous() &&
+         (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
+}
+
+bool load_norm(const Module &sequential, const Tensor &x, int64_t channels, NormParams *out) {
+  const Module norm = sequential.child("0", kLayerNorm);
+  if (!norm || sequential.child("1")) return false;
+  out->weight = norm.parameter("weight");
+  out->bias = norm.parameter("bias");
+  out->eps = (float)norm.real("eps", -1.0);
+  return out->eps >= 0.f && same(out->weight, x, channels, false) && same(out->bias, x, channels, false);
+}
+
+bool load_linear(const Module &m, const Tensor &x, int64_t in, int64_t out, Tensor *w, Tensor *b) {
+  if (!m) return false;
+  *w = m.parameter("weight");
+  *b = m.parameter("bias");
+  return same(*w, x, in * out, false) && same(*b, x, out, true);
+}
+
+bool Layer::load(const Module &m, const Tensor &x) {
+  const int64_t c = channels = x.size(-1);
+  if (c % 8 != 0 || c > 4096) return false;
+  post_norm = m.truth("post_norm", false);
+  if (!idle(m.child("drop_path"), kDropPath)) return false;
+  if (!load_norm(m.child("norm1", kSequential), x, c, &norm1) || !load_norm(m.child("norm2", kSequential), x, c, &norm2)) return false;
+  if (m.truth("layer_scale", false)) {
+    gamma1 = m.parameter("gamma1");
+    gamma2 = m.parameter("gamma2");
+    if (!same(gamma1, x, c, false) || !same(gamma2, x, c, false)) return false;
+  }
+  const Module mlp = m.child("mlp", kMlp);
+  if (!mlp || !idle(mlp.child("drop"), kDropout)) return false;
+  const Module act = mlp.child("act", kGelu);
+  PyObject *approximate = act.attribute("approximate");
+  if (approximate == nullptr || PyUnicode_CompareWithASCIIString(approximate, "none") != 0) return false;
+  const Module fc1 = mlp.child("fc1", kLinear);
+  hidden = fc1.integer("out_features", 0);
+  if (hidden <= 0 || hidden % 8 != 0 || !load_linear(fc1, x, c, hidden, &fc1_w, &fc1_b) ||
+      !load_linear(mlp.child("fc2", kLinear), x, hidden, c, &fc2_w, &fc2_b))
+    return false;
+
+  const Module dcn = m.child("dcn", kDCNv4);
+  if (!dcn || dcn.truth("without_pointwise", true) || dcn.truth("center_feature_scale", true) || dcn.integer("stride", 0) != 1) return false;
+  kernel = (int)dcn.integer("kernel_size", 0);
+  pad = (int)dcn.integer("pad", -1);
+  dilation = (int)dcn.integer("dilation", 0);
+  group = (int)dcn.integer("group", 0);
+  group_channels = (int)dcn.integer("group_channels", 0);
+  remove_center = (int)dcn.integer("remove_center", 0);
+  offset_scale = (float)dcn.real("offset_scale", 1.0);
+  if (kernel <= 0 || dilation <= 0 || 2 * pad != dilation * (kernel - 1) || (int64_t)group * group_channels != c) return false;
+  const Module offset = dcn.child("offset_mask", kLinear);
+  row = offset.integer("out_features", 0);
+  if (row <= 0 || row % 8 != 0 || !load_linear(offset, x, c, row, &offset_w, &offset_b) ||
+      !load_linear(dcn.child("value_proj", kLinear), x, c, c, &value_w, &value_b) ||
+      !load_linear(dcn.child("output_proj", kLinear), x, c, c, &output_w, &output_b))
+    return false;
+  PyObject *dw = dcn.attribute("dw_kernel_size");
+  if (dw != nullptr && dw != Py_None) {
+    dw_kernel = (int)dcn.integer("dw_kernel_size", 0);
+    if (dw_kernel != 1 && dw_kernel != 3 && dw_kernel != 5 && dw_kernel != 7) return false;
+    const Module conv = dcn.child("offset_mask_dw", kConv2d);
+    if (!conv) return false;
+    dw_w = conv.parameter("weight");
+    dw_b = conv.parameter("bias");
+    if (!same(dw_w, x, c * dw_kernel * dw_kernel, false) || !same(dw_b, x, c, true)) return false;
+  }
+  return true;
+}
+
+void launch(int code, const LinearLaunch &l, void *stream) {
+  const hipError_t e = launch_linear(code, l, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) raise_runtime("linear layer launch: %s", hipGetErrorString(e));
+}
+
+Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w) {
+  OnDevice guard(x);
+  const int code = dtype_code(x, "input");
+  void *stream = stream_of(x);
+  const int64_t rows = (int64_t)batch * h * w, c = l.channels;
+  Tensor out = at::empty(x.sizes(), x.options());
+  // intermediates, each on a 256-byte boundary: the depthwise output (or a normalised input), value and the operator's output,
+  // offset rows, a projection's output, the stream between the two halves; the MLP's hidden tensor takes the place of the first four
+  auto span = [](int64_t elements) { return (elements * 2 + 255) / 256 * 256; };
+  const int64_t act = span(rows * c), om = span(rows * l.row), hid = span(rows * l.hidden);
+  const int64_t front = std::max(4 * act + om, hid);
+  const Tensor ws = workspace((size_t)(front + 2 * act), x);
+  char *base = static_cast<char *>(ws.data_ptr());
+  char *pre = base, *value = base + act, *sampled = base + 2 * act, *projected = base + 3 * act, *offsets = base + 4 * act;
+  char *hidden = base, *middle = base + front, *last = base + front + act;
+  const void *in = x.const_data_ptr();
+
+  auto norm = [&](const void *y, const NormParams &n, const Tensor &gamma, const void *residual, void *o) {
+    check(dcnv4_gfx950_layer_norm_residual_forward(y, residual, ptr(n.weight), ptr(n.bias), ptr(gamma), o, code, rows, (int)c, n.eps, stream));
+  };
+  auto linear = [&](const void *a, const Tensor &wt, const Tensor &b, int64_t k, int64_t n, bool gelu, const Tensor &gamma,
+                    const void *residual, void *o) {
+    LinearLaunch p = {};
+    p.p[0] = {a, ptr(wt), ptr(b), ptr(gamma), residual, o, (int)n};
+    p.count = 1; p.rows = rows; p.k = (int)k; p.gelu = gelu;
+    launch(code, p, stream);
+  };
+
+  // DCNv4 half
+  const void *source = in;
+  if (!l.post_norm) {
+    norm(in, l.norm1, Tensor(), nullptr, middle);
+    source = middle;
+  }
+  const void *offset_source = source;
+  if (l.dw_kernel != 0) {
+    check(dcnv4_gfx950_depthwise_conv_forward(source, ptr(l.dw_w), ptr(l.dw_b), pre, code, batch, h, w, (int)c, l.dw_kernel,
+                                              (l.dw_kernel - 1) / 2, stream));
+    offset_source = pre;
+  }
+  LinearLaunch both = {};
+  both.p[0] = {source, ptr(l.value_w), ptr(l.value_b), nullptr, nullptr, value, (int)c};
+  both.p[1] = {offset_source, ptr(l.offset_w), ptr(l.offset_b), nullptr, nullptr, offsets, (int)l.row};
+  both.count = 2; both.rows = rows; both.k = (int)c;
+  launch(code, both, stream);
+  check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
+                             l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
+  if (l.post_norm) {
+    linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, projected);
+    norm(projected, l.norm1, l.gamma1, in, middle);
+    linear(middle, l.fc1_w, l.fc1_b, c, l.hidden, true, Tensor(), nullptr, hidden);
+    linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
+    norm(last, l.norm2, l.gamma2, middle, out.data_ptr());
+  } else {
+    linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
+    norm(last, l.norm2, Tensor(), nullptr, middle);
+    linear(middle, l.fc1_w, l.fc1_b, c, l.hidden, true, Tensor(), nullptr, hidden);
+    linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, l.gamma2, last, out.data_ptr());
+  }
+  return out;
+}
+
+// linear(a, weight, bias, gamma, residual, gelu): act(a @ weight.T + bias) * gamma + residual; the last three may be None
+PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("linear", args, n, 6);
+  const Tensor &in = a.tensor(), &weight = a.tensor();
+  const Tensor bias = a.optional_tensor(), gamma = a.optional_tensor(), residual = a.optional_tensor();
+  const int gelu = a.integer();
+  check_tensor(in, "input");
+  check_tensor(weight, "weight", in.scalar_type());
+  if (in.dim() < 1 || weight.dim() != 2 || weight.size(1) != in.size(-1)) raise_runtime("weight must be (N, K) for an input (..., K)");
+  const int64_t k = weight.size(1), width = weight.size(0), rows = k ? in.numel() / k : 0;
+  const int code = dtype_code(in, "input");
+  if (!linear_fits(code, rows, (int)width, (int)k)) raise_runtime("linear takes 16-bit tensors of a depth and width in multiples of 8");
+  auto sizes = in.sizes().vec();
+  sizes.back() = width;
+  if (!same(in, in, in.numel(), false) || !same(weight, in, width * k, false) || !same(bias, in, width, true) ||
+      !same(gamma, in, width, true) || !same(residual, in, rows * width, true))
+    raise_runtime("bias, gamma and residual must be contiguous, 16-byte aligned and of the input's dtype");
+  OnDevice guard(in);
+  at::AutoGradMode no_grad(false);
+  Tensor out = at::empty(sizes, in.options());
+  LinearLaunch p = {};
+  p.p[0] = {in.data_ptr(), ptr(weight), ptr(bias), ptr(gamma), ptr(residual), out.data_ptr(), (int)width};
+  p.count = 1; p.rows = rows; p.k = (int)k; p.gelu = gelu;
+  launch(code, p, stream_of(in));
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// layer_inference(layer, x, h, w): the layer's output, or None where the composition of its modules has to run: gradients or
+// autocast, single precision, modules of other classes, hooks, dropout or stochastic depth at work.
+PyObject *py_layer_inference(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("layer_inference", args + 1, n - 1, 3);
+  const Tensor &x = a.tensor();
+  const int h = a.integer(), w = a.integer();
+  if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks()) Py_RETURN_NONE;
+  if (!x.is_cuda() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) || x.dim() != 3 || !x.is_contiguous() ||
+      x.numel() == 0 || x.size(1) != (int64_t)h * w || (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15) != 0)
+    Py_RETURN_NONE;
+  Layer layer;
+  if (!layer.load(Module(args[0]), x)) Py_RETURN_NONE;
+  const int batch = (int)x.size(0);
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    out = layer_inference(layer, x, batch, h, w);
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+}  // namespace
+
+PyMethodDef layer_methods[] = {
+    {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear)), METH_FASTCALL, nullptr},
+    {"layer_inference", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_layer_inference)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+}  // namespace dcn::binding

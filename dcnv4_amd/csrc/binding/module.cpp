@@ -1,7 +1,7 @@
 // The extension module dcnv4_amd._native and the helpers its files share.
 #include <cstdarg>
 
-#include "binding.hpp"
+#include "modules.hpp"
 
 namespace dcn::binding {
 
@@ -84,4 +84,13 @@ variable_list once_differentiable(variable_list grads) {
 static struct PyModuleDef native_module = {PyModuleDef_HEAD_INIT, "_native", "Host path of the gfx950 operators in C++.", -1,
                                            dcn::binding::operator_methods, nullptr, nullptr, nullptr, nullptr};
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&native_module); }
+PyMODINIT_FUNC PyInit__native(void) {
+  PyObject *m = PyModule_Create(&native_module);
+  if (m == nullptr) return nullptr;
+  for (PyMethodDef *methods : {dcn::binding::module_methods, dcn::binding::layer_methods})
+    if (PyModule_AddFunctions(m, methods) != 0) {
+      Py_DECREF(m);
+      return nullptr;
+    }
+  return m;
+}

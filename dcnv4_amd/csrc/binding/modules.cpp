@@ -1,0 +1,113 @@
+#include "modules.hpp"
+
+#include <unordered_map>
+
+namespace dcn::binding {
+namespace {
+
+PyObject *g_kinds[kModuleKinds] = {};
+PyObject *g_global_hooks[4] = {};
+
+// Interned attribute names, looked up by the address of the literal.
+PyObject *name_object(const char *name) {
+  static std::unordered_map<const char *, PyObject *> names;      // under the GIL
+  PyObject *&o = names[name];
+  if (o == nullptr) o = PyUnicode_InternFromString(name);
+  return o;
+}
+
+PyObject *dict_of(PyObject *o) {
+  PyObject **d = _PyObject_GetDictPtr(o);
+  return d != nullptr ? *d : nullptr;
+}
+
+PyObject *item(PyObject *dict, const char *name) {
+  return dict != nullptr && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, name_object(name)) : nullptr;
+}
+
+}  // namespace
+
+bool Module::is(ModuleKind kind) const { return o_ != nullptr && (PyObject *)Py_TYPE(o_) == g_kinds[kind]; }
+
+Module Module::child(const char *name) const {
+  PyObject *c = o_ != nullptr ? item(item(dict_of(o_), "_modules"), name) : nullptr;
+  return Module(c == Py_None ? nullptr : c);
+}
+
+Module Module::child(const char *name, ModuleKind kind) const {
+  const Module c = child(name);
+  return c.is(kind) && !c.hooked() ? c : Module();
+}
+
+Tensor Module::parameter(const char *name) const {
+  PyObject *p = o_ != nullptr ? item(item(dict_of(o_), "_parameters"), name) : nullptr;
+  return p != nullptr && THPVariable_Check(p) ? THPVariable_Unpack(p) : Tensor();
+}
+
+PyObject *Module::attribute(const char *name) const { return o_ != nullptr ? item(dict_of(o_), name) : nullptr; }
+
+long Module::integer(const char *name, long otherwise) const {
+  PyObject *a = attribute(name);
+  return a != nullptr && PyLong_Check(a) ? PyLong_AsLong(a) : otherwise;
+}
+
+double Module::real(const char *name, double otherwise) const {
+  PyObject *a = attribute(name);
+  return a != nullptr && (PyFloat_Check(a) || PyLong_Check(a)) ? PyFloat_AsDouble(a) : otherwise;
+}
+
+bool Module::truth(const char *name, bool otherwise) const {
+  PyObject *a = attribute(name);
+  return a == nullptr ? otherwise : PyObject_IsTrue(a) == 1;
+}
+
+bool Module::hooked() const {
+  PyObject *d = dict_of(o_);
+  for (const char *name : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}) {
+    PyObject *hooks = item(d, name);
+    if (hooks != nullptr && PyDict_Check(hooks) && PyDict_GET_SIZE(hooks) != 0) return true;
+  }
+  return false;
+}
+
+bool global_module_hooks() {
+  for (PyObject *hooks : g_global_hooks)
+    if (hooks != nullptr && PyDict_Check(hooks) && PyDict_GET_SIZE(hooks) != 0) return true;
+  return false;
+}
+
+bool idle(const Module &m, ModuleKind kind) {
+  if (!m || m.hooked()) return false;
+  if (m.is(kIdentity)) return true;
+  return m.is(kind) && (!m.truth("training", true) || m.real("p", 1.0) == 0.0);
+}
+
+namespace {
+
+// register_modules(*classes in the order of ModuleKind)
+PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != kModuleKinds) raise_runtime("register_modules takes %d classes, got %zd", (int)kModuleKinds, n);
+  for (int i = 0; i < kModuleKinds; ++i) {
+    Py_INCREF(args[i]);
+    Py_XSETREF(g_kinds[i], args[i]);
+  }
+  PyObject *m = PyImport_ImportModule("torch.nn.modules.module");
+  if (m == nullptr) throw python_error();
+  int i = 0;
+  for (const char *name : {"_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks"}) {
+    Py_XSETREF(g_global_hooks[i], PyObject_GetAttrString(m, name));
+    if (g_global_hooks[i] == nullptr) PyErr_Clear();
+    ++i;
+  }
+  Py_DECREF(m);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+}  // namespace
+
+PyMethodDef module_methods[] = {{"register_modules", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_register)), METH_FASTCALL, nullptr},
+                                {nullptr, nullptr, 0, nullptr}};
+
+}  // namespace dcn::binding

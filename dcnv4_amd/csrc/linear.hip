@@ -1,0 +1,246 @@
+// Linear layers on the matrix cores for 16-bit tensors, with what follows the product fused into its epilogue: bias, GELU,
+// layer scale, residual.  Two kernels:
+//
+//  linear_tiled_kernel: many rows.  A workgroup of four waves owns BM rows x BN features; both operands come in slices of 64
+//    along the depth, 16 bytes a lane, straight into LDS (two buffers, one barrier a slice: the next slice's loads are in
+//    flight while the matrix cores work on this one).  The 16-byte vectors of a row are stored at position
+//    vector ^ (row / 2 & 7), so the 16 rows that a fragment read touches fall into 16 different slots of 256 bytes and the
+//    read has no bank conflicts.  The features are the rows of the matrix instruction's result, so a lane ends up with
+//    four consecutive features of one row and stores 8 bytes.
+//  linear_few_rows_kernel: a picture or two at the later stages, where a launch has a handful of tiles and its time is load
+//    latency.  A workgroup owns 32 rows x 32 features; its four waves share the depth between them, take their fragments
+//    straight from memory and meet in LDS once.
+#include "linear.hpp"
+#include "mfma.hpp"
+
+namespace dcn {
+namespace {
+
+constexpr int kCus = 256;                        // MI355X
+constexpr int kSlice = 64;                       // depth of a slice: 128 bytes of a row
+constexpr int kRowVectors = kSlice * 2 / 16;     // 16-byte vectors of a row's slice
+
+// What a lane needs of a feature vector for its eight columns, read once.
+template <typename Tag>
+struct Columns {
+  float bias[8], gamma[8];
+  bool has_bias, has_gamma;
+  __device__ __forceinline__ Columns(const LinearProblem &q, int n, bool live) : has_bias(q.bias != nullptr), has_gamma(q.gamma != nullptr) {
+    if (has_bias && live) Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.bias) + n * 2), bias);
+    if (has_gamma && live) Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.gamma) + n * 2), gamma);
+  }
+};
+
+// The epilogue for eight consecutive features of one row: 16 bytes in and out.
+template <typename Tag>
+__device__ __forceinline__ void finish(const LinearProblem &q, const Columns<Tag> &col, int gelu, long long row, int n, float (&v)[8]) {
+  if (col.has_bias)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += col.bias[c];
+  if (gelu)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = gelu_exact(v[c]);
+  if (col.has_gamma)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] *= col.gamma[c];
+  const size_t at = ((size_t)row * q.n + n) * 2;
+  if (q.residual != nullptr) {
+    float r[8];
+    Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.residual) + at), r);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += r[c];
+  }
+  *reinterpret_cast<u32x4 *>(static_cast<char *>(q.out) + at) = Pack<Tag, 8>::encode(v);
+}
+
+template <typename Tag, int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
+  static_assert(WM * WN == 4 && BM % (16 * WM) == 0 && BN % (32 * WN) == 0 && BM % 32 == 0, "tile shape");
+  constexpr int MF = BM / WM / 16, NF = BN / WN / 16;
+  __shared__ u32x4 lds[2][(BM + BN) * kRowVectors];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t tile = xcd_contiguous_block(blockIdx.x, gridDim.x);
+  const int tm = tile / tiles_n;
+  int tn = tile % tiles_n;
+  const int which = tn >= tiles_n0;
+  const LinearProblem &q = p.p[which];
+  if (which) tn -= tiles_n0;
+  const long long m0 = (long long)tm * BM;
+  const int n0 = tn * BN, k = p.k;
+  const int live_m = (int)min((long long)BM, p.rows - m0), live_n = min(BN, q.n - n0);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * 2, (uint32_t)live_m * k * 2);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * 2, (uint32_t)live_n * k * 2);
+
+  // a wave's load covers eight rows of a tile: lane l takes row l / 8, position l & 7
+  const int row8 = lane >> 3, pos = lane & 7;
+  auto stage = [&](int k0, u32x4 *buf) {
+#pragma unroll
+    for (int i = 0; i < (BM + BN) / 32; ++i) {
+      const bool act = i < BM / 32;
+      const int base = (i * 4 + wave) * 8, row = base + row8;             // rows of the row tile, then of the feature tile
+      const int kk = k0 + (pos ^ ((row >> 1) & 7)) * 8;
+      const uint32_t off = (uint32_t)((act ? row : row - BM) * k + kk) * 2;
+      load_to_lds(act ? ra : rw, buf + base * kRowVectors, kk < k ? off : kDropOffset);
+    }
+  };
+  const int wm = wave / WN, wn = wave % WN, r16 = lane & 15, kb = lane >> 4;
+  auto fragment = [&](const u32x4 *buf, int row, int s) { return buf[row * kRowVectors + ((s * 4 + kb) ^ ((row >> 1) & 7))]; };
+
+  f32x4 acc[NF][MF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < MF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  stage(0, lds[0]);
+  int cur = 0;
+  for (int k0 = 0; k0 < k; k0 += kSlice, cur ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    u32x4 fm[2][MF], fn[2][NF];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int j = 0; j < MF; ++j) fm[s][j] = fragment(lds[cur], wm * (BM / WM) + j * 16 + r16, s);
+#pragma unroll
+      for (int i = 0; i < NF; ++i) fn[s][i] = fragment(lds[cur], BM + wn * (BN / WN) + i * 16 + r16, s);
+    }
+    if (k0 + kSlice < k) stage(k0 + kSlice, lds[cur ^ 1]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NF; ++i)
+#pragma unroll
+        for (int j = 0; j < MF; ++j) acc[i][j] = mfma_16x16x32<Tag>(fn[s][i], fm[s][j], acc[i][j]);
+  }
+  // Epilogue, sixteen rows of the wave at a time: the fragments are turned through the buffer that the last slice did not
+  // use (the wave's own part of it, so no barrier), each lane then holds eight consecutive features of a row, and a row's
+  // piece goes out as whole 128-byte lines.  Stored as the fragments lie, 8 bytes a lane, the 401408 x 448 x 112 product
+  // took 232 us.
+  constexpr int TN = BN / WN, kTurn = TN + 4;                 // floats per row: an odd number of 16-byte units
+  static_assert(16 * kTurn * 4 <= (BM + BN) * kRowVectors * 16 / 4, "the wave's part of a buffer holds sixteen rows");
+  constexpr int lanes_per_row = TN / 8, rows_per_pass = 64 / lanes_per_row;
+  float *turn = reinterpret_cast<float *>(lds[cur]) + wave * ((BM + BN) * kRowVectors * 16 / 4 / 4);
+  const int col = (lane % lanes_per_row) * 8, n = wn * TN + col;
+  const Columns<Tag> columns(q, n0 + n, n < live_n);
+#pragma unroll
+  for (int j = 0; j < MF; ++j) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) *reinterpret_cast<f32x4 *>(turn + r16 * kTurn + i * 16 + kb * 4) = acc[i][j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < 16 / rows_per_pass; ++u) {
+      const int r = u * rows_per_pass + lane / lanes_per_row, row = wm * (BM / WM) + j * 16 + r;
+      const f32x4 lo = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col), hi = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col + 4);
+      float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      if (row < live_m && n < live_n) finish<Tag>(q, columns, p.gelu, m0 + row, n0 + n, v);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+constexpr int kFewTile = 32;
+
+template <typename Tag>
+__global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
+  __shared__ __align__(16) float part[4][kFewTile][kFewTile + 4];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tm = blockIdx.x / tiles_n;
+  int tn = blockIdx.x % tiles_n;
+  const int which = tn >= tiles_n0;
+  const LinearProblem &q = p.p[which];
+  if (which) tn -= tiles_n0;
+  const int m0 = tm * kFewTile, n0 = tn * kFewTile, k = p.k;
+  const int live_m = (int)min((long long)kFewTile, p.rows - m0), live_n = min(kFewTile, q.n - n0);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * 2, (uint32_t)live_m * k * 2);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * 2, (uint32_t)live_n * k * 2);
+  const int r16 = lane & 15, kb = lane >> 4;
+  const int steps = (k + 31) / 32;
+
+  f32x4 acc[2][2] = {};
+  // wave w takes every fourth step of 32 along the depth
+#pragma unroll 4
+  for (int s = wave; s < steps; s += 4) {
+    const int kk = s * 32 + kb * 8;
+    u32x4 fm[2], fn[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t off = (uint32_t)((j * 16 + r16) * k + kk) * 2;
+      fm[j] = buffer_load<16>(ra, kk < k ? off : kDropOffset);
+      fn[j] = buffer_load<16>(rw, kk < k ? off : kDropOffset);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_16x16x32<Tag>(fn[i], fm[j], acc[i][j]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
+  __syncthreads();
+  if (threadIdx.x >= 128) return;
+  const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
+  const Columns<Tag> columns(q, n0 + n, n < live_n);
+  float v[8];
+#pragma unroll
+  for (int c = 0; c < 8; c += 4) {
+    f32x4 sum = *reinterpret_cast<const f32x4 *>(&part[0][row][n + c]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
+    v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
+  }
+  if (row < live_m && n < live_n) finish<Tag>(q, columns, p.gelu, m0 + row, n0 + n, v);
+}
+
+template <typename Tag, int BM, int BN, int WM, int WN>
+hipError_t launch_tiled(const LinearLaunch &p, hipStream_t stream) {
+  const long long tiles_m = (p.rows + BM - 1) / BM;
+  const int tiles_n0 = (p.p[0].n + BN - 1) / BN, tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + BN - 1) / BN : 0);
+  if (tiles_m * tiles_n > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((linear_tiled_kernel<Tag, BM, BN, WM, WN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p,
+                     tiles_n0, tiles_n);
+  return hipGetLastError();
+}
+
+template <typename Tag>
+hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
+  const int tiles_m = (int)((p.rows + kFewTile - 1) / kFewTile), tiles_n0 = (p.p[0].n + kFewTile - 1) / kFewTile;
+  const int tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kFewTile - 1) / kFewTile : 0);
+  hipLaunchKernelGGL((linear_few_rows_kernel<Tag>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p, tiles_n0, tiles_n);
+  return hipGetLastError();
+}
+
+// Which kernel and tile: enough workgroups for the 256 CUs first, then the widest tile whose padding does not cost more
+// than it saves.  Measured (fp16, tile rows x features; us):
+//   few rows against 64x64: 49 x 512 x 2048 9.5 / 11.1, 392 x 512 x 2048 9.8 / 11.4, 1568 x 256 x 1024 9.6 / 7.1
+//   128x64 against 128x128: 25088 x 448 x 448 17.7 / 18.9, 25088 x 1792 x 448 62.5 / 55.5, 6272 x 3584 x 896 59.3 / 51.4,
+//     6272 x 1512 x 896 25.4 / 30.1 (600 against 588 tiles of which the last round is a third full)
+//   256x64 where the width is not a multiple of 128: 401408 x 192 x 112 52.4 against 62.0
+template <typename Tag>
+hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
+  auto tiles = [&](int bm, int bn) {
+    long long n = 0;
+    for (int i = 0; i < p.count; ++i) n += (p.p[i].n + bn - 1) / bn;
+    return n * ((p.rows + bm - 1) / bm);
+  };
+  if (tiles(64, 64) < 64) return launch_few<Tag>(p, stream);
+  if (tiles(128, 64) < kCus) return launch_tiled<Tag, 64, 64, 2, 2>(p, stream);
+  const long long wide = tiles(128, 128), narrow = tiles(128, 64);
+  if (wide < 4 * kCus) return launch_tiled<Tag, 128, 64, 4, 1>(p, stream);
+  if (20 * wide <= 11 * narrow) return launch_tiled<Tag, 128, 128, 2, 2>(p, stream);
+  return launch_tiled<Tag, 256, 64, 4, 1>(p, stream);
+}
+
+}  // namespace
+
+bool linear_fits(int dtype, long long rows, int n, int k) {
+  return (dtype == F16::kCode || dtype == BF16::kCode) && rows > 0 && n > 0 && k > 0 && n % 8 == 0 && k % 8 == 0 && k <= (1 << 20) &&
+         rows * (long long)n < (1ll << 42) && (rows + 63) / 64 * ((n + 63) / 64) < (1ll << 30);
+}
+
+hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream) {
+  return dtype == F16::kCode ? launch_t<F16>(p, stream) : launch_t<BF16>(p, stream);
+}
+
+}  // namespace dcn

@@ -139,6 +139,12 @@ def flash_deform_attn_backward(value, spatial_shapes, level_start_index, samplin
                                               im2col_step, K, d_stride, block_thread)
 
 
+def linear_forward(input, weight, bias=None, gamma=None, residual=None, gelu=False):
+    """``act(input @ weight.T + bias) * gamma + residual`` for 16-bit tensors, ``act`` the exact GELU or nothing: the linear
+    layers of a FlashInternImage layer with what follows them, as one matrix-core kernel."""
+    return _native.linear(input, weight, bias, gamma, residual, bool(gelu))
+
+
 def depthwise_conv_forward(input, weight, bias, pad):
     """Depthwise convolution of an NHWC tensor, stride 1, dilation 1: the ``offset_mask_dw`` layer of a
     DCNv4 block (DCNv4_op/DCNv4/modules/dcnv4.py:67-75,121-123) without the permutes around it.

@@ -11,7 +11,9 @@ FlashInternImage config enables.
 import torch
 from torch import nn
 
+from .. import ext
 from ..functions import layer_norm_residual
+from ..functions.launch_spec import GFX950_TABLE
 from ..modules import DCNv4
 
 
@@ -128,6 +130,11 @@ class InternImageLayer(nn.Module):
         return residual + self.drop_path(layer_norm_residual(y, ln, gamma))
 
     def forward(self, x, shape):
+        if not torch.is_grad_enabled() and not GFX950_TABLE and ext.dcnv4_forward is _ext_forward:
+            # inference in one call (csrc/binding/layers.cpp) where the kernels take the layer as it is
+            y = ext._native.layer_inference(self, x, *shape)
+            if y is not None:
+                return y
         g1, g2 = (self.gamma1, self.gamma2) if self.layer_scale else (None, None)
         if self.post_norm:
             x = self._scaled_norm(self.norm1, g1, self.dcn(x, shape), x)
@@ -138,6 +145,11 @@ class InternImageLayer(nn.Module):
             y = self.mlp(layer_norm_residual(x, self.norm2[0]), shape)
             x = x + self.drop_path(y if g2 is None else g2 * y)
         return x
+
+
+_ext_forward = ext.dcnv4_forward
+ext._native.register_modules(nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Identity, nn.Conv2d, nn.Sequential, DropPath, DCNv4,
+                             MLPLayer)
 
 
 class InternImageBlock(nn.Module):
