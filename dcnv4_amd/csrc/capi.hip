@@ -294,6 +294,8 @@ int plan_grad_value_tiles(DcnLaunch *L, int dtype, int batch) {
   return fail(DCNV4_ERR_RUNTIME, "kernel with %d taps and %d group channels does not fit the tiled backward", L->Kp, D);
 }
 
+constexpr uint64_t kDirectForwardBytes = 2800u << 10;      // outputs up to this size go by the direct kernel
+
 bool tiled_gather_enabled() { return g_opt.gather != kOptPlain; }
 
 // Output tile, group chunk and input window of the LDS-tiled gather kernels.  Returns false (and
@@ -734,7 +736,13 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
     return rc;
   if (int rc = check_ptrs({value, offset_mask, output})) return rc;
   const int per = images_per_launch(pr, false);
-  const bool tiled = plan_gather_tiles(&pr.launch, pr.s, false);
+  // A small call is a chain of latencies: the direct kernel's lanes go to memory at once, where the tiled one first stages
+  // its window behind a barrier.  Measured (fp16 / fp32, us, direct against tiled): 1x7x7x512 5.6 / 5.3 against 10.8 / 9.3,
+  // 2x56x56x112 6.7 / 7.6 against 9.8 / 8.3, 8x28x28x128 6.6 / 8.7 against 9.8 / 8.3; at 8x56x56x64 they meet in fp16
+  // (10.6 / 14.5 against 10.2 / 11.5), at 1x100x152x160 the tiled one is ahead (15.9 / 23.1 against 14.2 / 17.8).
+  const bool small = g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 &&
+                     (uint64_t)batch * pr.img_out_elems * pr.s <= kDirectForwardBytes;
+  const bool tiled = !small && plan_gather_tiles(&pr.launch, pr.s, false);
   for (int b0 = 0; b0 < batch; b0 += per) {
     const int nb = std::min(per, batch - b0);
     DcnLaunch L = pr.launch;
