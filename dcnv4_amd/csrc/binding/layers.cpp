@@ -6,63 +6,51 @@
 // bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.
 #include <ATen/autocast_mode.h>
 
-#include "../linear.hpp"
-#include "modules.hpp"
+#include "layers.hpp"
 
 namespace dcn::binding {
-namespace {
 
-struct NormParams {
-  Tensor weight, bias;
-  float eps = 0.f;
-};
-
-// What the kernels need of a layer; load() says whether they take it.
-struct Layer {
-  NormParams norm1, norm2;
-  Tensor gamma1, gamma2;
-  Tensor value_w, value_b, offset_w, offset_b, output_w, output_b, dw_w, dw_b;
-  Tensor fc1_w, fc1_b, fc2_w, fc2_b;
-  int kernel = 0, pad = 0, dilation = 0, group = 0, group_channels = 0, remove_center = 0, dw_kernel = 0;
-  float offset_scale = 1.f;
-  bool post_norm = false;
-  int64_t channels = 0, row = 0, hidden = 0;
-
-  bool load(const Module &m, const Tensor &x);
-};
-
-bool same(const Tensor &t, const Tensor &x, int64_t elements, bool optional) {
+bool usable(const Tensor &t, const Tensor &x, at::ScalarType dtype, int64_t elements, bool optional) {
   if (!t.defined()) return optional;
-  return t.scalar_type() == x.scalar_type() && t.device() == x.device() && t.numel() == elements && t.is_contiguous() &&
+  return t.scalar_type() == dtype && t.device() == x.device() && t.numel() == elements && t.is_contiguous() &&
          (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
 }
 
-bool load_norm(const Module &sequential, const Tensor &x, int64_t channels, NormParams *out) {
+namespace {
+
+bool load_norm(const Module &sequential, const Tensor &x, at::ScalarType dtype, int64_t channels, NormParams *out) {
   const Module norm = sequential.child("0", kLayerNorm);
   if (!norm || sequential.child("1")) return false;
   out->weight = norm.parameter("weight");
   out->bias = norm.parameter("bias");
   out->eps = (float)norm.real("eps", -1.0);
-  return out->eps >= 0.f && same(out->weight, x, channels, false) && same(out->bias, x, channels, false);
+  return out->eps >= 0.f && usable(out->weight, x, dtype, channels, false) && usable(out->bias, x, dtype, channels, false);
 }
 
-bool load_linear(const Module &m, const Tensor &x, int64_t in, int64_t out, Tensor *w, Tensor *b) {
+bool load_linear(const Module &m, const Tensor &x, at::ScalarType dtype, int64_t in, int64_t out, Tensor *w, Tensor *b) {
   if (!m) return false;
   *w = m.parameter("weight");
   *b = m.parameter("bias");
-  return same(*w, x, in * out, false) && same(*b, x, out, true);
+  return usable(*w, x, dtype, in * out, false) && usable(*b, x, dtype, out, true);
 }
 
-bool Layer::load(const Module &m, const Tensor &x) {
+}  // namespace
+
+bool Layer::load(const Module &m, const Tensor &x, at::ScalarType params) {
   const int64_t c = channels = x.size(-1);
   if (c % 8 != 0 || c > 4096) return false;
   post_norm = m.truth("post_norm", false);
-  if (!idle(m.child("drop_path"), kDropPath)) return false;
-  if (!load_norm(m.child("norm1", kSequential), x, c, &norm1) || !load_norm(m.child("norm2", kSequential), x, c, &norm2)) return false;
+  const Module path = m.child("drop_path");
+  if (!idle(path, kDropPath)) {
+    if (!path.is(kDropPath) || path.hooked()) return false;
+    drop_path = path.real("p", -1.0);
+    if (drop_path <= 0.0 || drop_path >= 1.0) return false;
+  }
+  if (!load_norm(m.child("norm1", kSequential), x, params, c, &norm1) || !load_norm(m.child("norm2", kSequential), x, params, c, &norm2)) return false;
   if (m.truth("layer_scale", false)) {
     gamma1 = m.parameter("gamma1");
     gamma2 = m.parameter("gamma2");
-    if (!same(gamma1, x, c, false) || !same(gamma2, x, c, false)) return false;
+    if (!usable(gamma1, x, params, c, false) || !usable(gamma2, x, params, c, false)) return false;
   }
   const Module mlp = m.child("mlp", kMlp);
   if (!mlp || !idle(mlp.child("drop"), kDropout)) return false;
@@ -71,8 +59,8 @@ bool Layer::load(const Module &m, const Tensor &x) {
   if (approximate == nullptr || PyUnicode_CompareWithASCIIString(approximate, "none") != 0) return false;
   const Module fc1 = mlp.child("fc1", kLinear);
   hidden = fc1.integer("out_features", 0);
-  if (hidden <= 0 || hidden % 8 != 0 || !load_linear(fc1, x, c, hidden, &fc1_w, &fc1_b) ||
-      !load_linear(mlp.child("fc2", kLinear), x, hidden, c, &fc2_w, &fc2_b))
+  if (hidden <= 0 || hidden % 8 != 0 || !load_linear(fc1, x, params, c, hidden, &fc1_w, &fc1_b) ||
+      !load_linear(mlp.child("fc2", kLinear), x, params, hidden, c, &fc2_w, &fc2_b))
     return false;
 
   const Module dcn = m.child("dcn", kDCNv4);
@@ -87,9 +75,9 @@ bool Layer::load(const Module &m, const Tensor &x) {
   if (kernel <= 0 || dilation <= 0 || 2 * pad != dilation * (kernel - 1) || (int64_t)group * group_channels != c) return false;
   const Module offset = dcn.child("offset_mask", kLinear);
   row = offset.integer("out_features", 0);
-  if (row <= 0 || row % 8 != 0 || !load_linear(offset, x, c, row, &offset_w, &offset_b) ||
-      !load_linear(dcn.child("value_proj", kLinear), x, c, c, &value_w, &value_b) ||
-      !load_linear(dcn.child("output_proj", kLinear), x, c, c, &output_w, &output_b))
+  if (row <= 0 || row % 8 != 0 || !load_linear(offset, x, params, c, row, &offset_w, &offset_b) ||
+      !load_linear(dcn.child("value_proj", kLinear), x, params, c, c, &value_w, &value_b) ||
+      !load_linear(dcn.child("output_proj", kLinear), x, params, c, c, &output_w, &output_b))
     return false;
   PyObject *dw = dcn.attribute("dw_kernel_size");
   if (dw != nullptr && dw != Py_None) {
@@ -99,7 +87,7 @@ bool Layer::load(const Module &m, const Tensor &x) {
     if (!conv) return false;
     dw_w = conv.parameter("weight");
     dw_b = conv.parameter("bias");
-    if (!same(dw_w, x, c * dw_kernel * dw_kernel, false) || !same(dw_b, x, c, true)) return false;
+    if (!usable(dw_w, x, params, c * dw_kernel * dw_kernel, false) || !usable(dw_b, x, params, c, true)) return false;
   }
   return true;
 }
@@ -108,6 +96,13 @@ void launch(int code, const LinearLaunch &l, void *stream) {
   const hipError_t e = launch_linear(code, l, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) raise_runtime("linear layer launch: %s", hipGetErrorString(e));
 }
+
+bool usable_input(const Tensor &x, int h, int w) {
+  return x.is_cuda() && x.dim() == 3 && x.is_contiguous() && x.numel() != 0 && x.size(1) == (int64_t)h * w &&
+         (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15) == 0;
+}
+
+namespace {
 
 Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w) {
   OnDevice guard(x);
@@ -186,8 +181,9 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!linear_fits(code, rows, (int)width, (int)k)) raise_runtime("linear takes 16-bit tensors of a depth and width in multiples of 8");
   auto sizes = in.sizes().vec();
   sizes.back() = width;
-  if (!same(in, in, in.numel(), false) || !same(weight, in, width * k, false) || !same(bias, in, width, true) ||
-      !same(gamma, in, width, true) || !same(residual, in, rows * width, true))
+  const auto dtype = in.scalar_type();
+  if (!usable(in, in, dtype, in.numel(), false) || !usable(weight, in, dtype, width * k, false) || !usable(bias, in, dtype, width, true) ||
+      !usable(gamma, in, dtype, width, true) || !usable(residual, in, dtype, rows * width, true))
     raise_runtime("bias, gamma and residual must be contiguous, 16-byte aligned and of the input's dtype");
   OnDevice guard(in);
   at::AutoGradMode no_grad(false);
@@ -208,11 +204,9 @@ PyObject *py_layer_inference(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Tensor &x = a.tensor();
   const int h = a.integer(), w = a.integer();
   if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks()) Py_RETURN_NONE;
-  if (!x.is_cuda() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) || x.dim() != 3 || !x.is_contiguous() ||
-      x.numel() == 0 || x.size(1) != (int64_t)h * w || (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15) != 0)
-    Py_RETURN_NONE;
+  if (!usable_input(x, h, w) || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) Py_RETURN_NONE;
   Layer layer;
-  if (!layer.load(Module(args[0]), x)) Py_RETURN_NONE;
+  if (!layer.load(Module(args[0]), x, x.scalar_type()) || layer.drop_path != 0.0) Py_RETURN_NONE;
   const int batch = (int)x.size(0);
   Tensor out;
   {

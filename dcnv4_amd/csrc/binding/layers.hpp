@@ -1,0 +1,37 @@
+// A FlashInternImage layer as its kernels see it.
+#pragma once
+#include "../linear.hpp"
+#include "modules.hpp"
+
+namespace dcn::binding {
+
+struct NormParams {
+  Tensor weight, bias;
+  float eps = 0.f;
+};
+
+// What the kernels need of a layer; load() says whether they take it.
+struct Layer {
+  NormParams norm1, norm2;
+  Tensor gamma1, gamma2;
+  Tensor value_w, value_b, offset_w, offset_b, output_w, output_b, dw_w, dw_b;
+  Tensor fc1_w, fc1_b, fc2_w, fc2_b;
+  int kernel = 0, pad = 0, dilation = 0, group = 0, group_channels = 0, remove_center = 0, dw_kernel = 0;
+  float offset_scale = 1.f;
+  bool post_norm = false;
+  int64_t channels = 0, row = 0, hidden = 0;
+
+  double drop_path = 0.0;      // of a layer in training
+  // Reads the module; false where its kernels do not take it.  The parameters must have dtype `params`.
+  bool load(const Module &m, const Tensor &x, at::ScalarType params);
+};
+
+// Contiguous, aligned, on x's device, of that dtype and size.
+bool usable(const Tensor &t, const Tensor &x, at::ScalarType dtype, int64_t elements, bool optional);
+void launch(int code, const LinearLaunch &l, void *stream);
+// The arguments (layer, x, h, w) of a call that takes a layer.
+bool usable_input(const Tensor &x, int h, int w);
+
+extern PyMethodDef training_methods[];
+
+}  // namespace dcn::binding

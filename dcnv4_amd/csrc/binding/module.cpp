@@ -1,7 +1,7 @@
 // The extension module dcnv4_amd._native and the helpers its files share.
 #include <cstdarg>
 
-#include "modules.hpp"
+#include "layers.hpp"
 
 namespace dcn::binding {
 
@@ -87,7 +87,7 @@ static struct PyModuleDef native_module = {PyModuleDef_HEAD_INIT, "_native", "Ho
 PyMODINIT_FUNC PyInit__native(void) {
   PyObject *m = PyModule_Create(&native_module);
   if (m == nullptr) return nullptr;
-  for (PyMethodDef *methods : {dcn::binding::module_methods, dcn::binding::layer_methods})
+  for (PyMethodDef *methods : {dcn::binding::module_methods, dcn::binding::layer_methods, dcn::binding::training_methods})
     if (PyModule_AddFunctions(m, methods) != 0) {
       Py_DECREF(m);
       return nullptr;

@@ -681,6 +681,33 @@ char *at(void *base, size_t elems, int s) { return static_cast<char *>(base) + e
 }  // namespace
 }  // namespace dcn
 
+namespace dcn {
+
+int prepare_layer_norm(LnLaunch *L, int dtype, long long rows, int channels, float eps) {
+  const int s = elem_bytes(dtype);
+  if (s == 0) return fail(DCNV4_ERR_RUNTIME, "unsupported dtype code %d (fp32, fp16, bf16 only)", dtype);
+  if (rows <= 0 || channels <= 0) return fail(DCNV4_ERR_RUNTIME, "empty or negative extent (rows %lld, channels %d)", rows, channels);
+  const int V = 16 / s;
+  if (channels % V != 0) return fail(DCNV4_ERR_INVALID_ARGUMENT, "channels (%d) must be a multiple of %d for this dtype", channels, V);
+  const int nvec = channels / V;
+  if (nvec > 64 * 8) return fail(DCNV4_ERR_INVALID_ARGUMENT, "rows of %d channels are too long (at most %d)", channels, 64 * 8 * V);
+  *L = LnLaunch{};
+  L->rows = rows; L->C = channels; L->eps = eps;
+  L->team = 1;
+  while (L->team < 64 && L->team < nvec) L->team *= 2;
+  L->vpl = 1;
+  while (L->team * L->vpl < nvec) L->vpl *= 2;
+  // backward: about 2048 workgroups at most, each a slab of whole passes; partial sums stay below 32 MB
+  const long long rows_per_pass = 256 / L->team;
+  long long parts = std::min<long long>((rows + rows_per_pass - 1) / rows_per_pass, 2048);
+  while (parts > 1 && (size_t)parts * 3 * channels * sizeof(float) > (size_t(32) << 20)) parts /= 2;
+  L->slab = ((rows + parts - 1) / parts + rows_per_pass - 1) / rows_per_pass * rows_per_pass;
+  L->n_part = (int)((rows + L->slab - 1) / L->slab);
+  return DCNV4_OK;
+}
+
+}  // namespace dcn
+
 using namespace dcn;
 
 extern "C" {
@@ -1168,10 +1195,9 @@ size_t dcnv4_gfx950_depthwise_conv_backward_workspace_bytes(int dtype, int batch
   return round16(pr.total_parts * (size_t)(kernel_size * kernel_size + 1) * channels * sizeof(float));
 }
 
-int dcnv4_gfx950_depthwise_conv_backward(const void *input, const void *weight, const void *grad_output, void *grad_input,
-                                         void *grad_weight, void *grad_bias, void *workspace, size_t workspace_bytes,
-                                         int dtype, int batch, int height, int width, int channels, int kernel_size,
-                                         int pad, void *stream) {
+static int dw_backward_impl(const void *input, const void *weight, const void *grad_output, void *grad_input, void *grad_weight,
+                            void *grad_bias, void *workspace, size_t workspace_bytes, int dtype, int grads_dtype, int batch,
+                            int height, int width, int channels, int kernel_size, int pad, void *stream) {
   DwProblem pr;
   if (int rc = dw_prepare(&pr, dtype, batch, height, width, channels, kernel_size, pad)) return rc;
   if (int rc = check_ptrs({grad_output})) return rc;
@@ -1216,33 +1242,22 @@ int dcnv4_gfx950_depthwise_conv_backward(const void *input, const void *weight, 
     L.n_part = (int)parts_done;
     L.grad_weight = grad_weight;
     L.grad_bias = grad_bias;
-    if (hipError_t e = launch_depthwise_grad_weight_reduce(dtype, L, st)) return hip_fail("depthwise grad_weight reduction launch", e);
+    if (hipError_t e = launch_depthwise_grad_weight_reduce(grads_dtype, L, st)) return hip_fail("depthwise grad_weight reduction launch", e);
   }
   return DCNV4_OK;
 }
 
+int dcnv4_gfx950_depthwise_conv_backward(const void *input, const void *weight, const void *grad_output, void *grad_input,
+                                         void *grad_weight, void *grad_bias, void *workspace, size_t workspace_bytes,
+                                         int dtype, int batch, int height, int width, int channels, int kernel_size,
+                                         int pad, void *stream) {
+  return dw_backward_impl(input, weight, grad_output, grad_input, grad_weight, grad_bias, workspace, workspace_bytes, dtype, dtype,
+                          batch, height, width, channels, kernel_size, pad, stream);
+}
+
 // Row geometry shared by the layer-norm forward and backward: a team of lanes per row, 16-byte vectors per lane.
 static int ln_prepare(LnLaunch *L, int dtype, long long rows, int channels, float eps) {
-  const int s = elem_bytes(dtype);
-  if (s == 0) return fail(DCNV4_ERR_RUNTIME, "unsupported dtype code %d (fp32, fp16, bf16 only)", dtype);
-  if (rows <= 0 || channels <= 0) return fail(DCNV4_ERR_RUNTIME, "empty or negative extent (rows %lld, channels %d)", rows, channels);
-  const int V = 16 / s;
-  if (channels % V != 0) return fail(DCNV4_ERR_INVALID_ARGUMENT, "channels (%d) must be a multiple of %d for this dtype", channels, V);
-  const int nvec = channels / V;
-  if (nvec > 64 * 8) return fail(DCNV4_ERR_INVALID_ARGUMENT, "rows of %d channels are too long (at most %d)", channels, 64 * 8 * V);
-  *L = LnLaunch{};
-  L->rows = rows; L->C = channels; L->eps = eps;
-  L->team = 1;
-  while (L->team < 64 && L->team < nvec) L->team *= 2;
-  L->vpl = 1;
-  while (L->team * L->vpl < nvec) L->vpl *= 2;
-  // backward: about 2048 workgroups at most, each a slab of whole passes; partial sums stay below 32 MB
-  const long long rows_per_pass = 256 / L->team;
-  long long parts = std::min<long long>((rows + rows_per_pass - 1) / rows_per_pass, 2048);
-  while (parts > 1 && (size_t)parts * 3 * channels * sizeof(float) > (size_t(32) << 20)) parts /= 2;
-  L->slab = ((rows + parts - 1) / parts + rows_per_pass - 1) / rows_per_pass * rows_per_pass;
-  L->n_part = (int)((rows + L->slab - 1) / L->slab);
-  return DCNV4_OK;
+  return prepare_layer_norm(L, dtype, rows, channels, eps);
 }
 
 int dcnv4_gfx950_layer_norm_residual_forward(const void *input, const void *residual, const void *weight,
@@ -1359,3 +1374,14 @@ int dcnv4_gfx950_stream_copy(const void *src, void *dst, size_t bytes, void *str
 }
 
 }  // extern "C"
+
+namespace dcn {
+
+int depthwise_backward_fp32_grads(const void *input, const void *weight, const void *grad_output, void *grad_input, float *grad_weight,
+                                  float *grad_bias, void *workspace, size_t workspace_bytes, int dtype, int batch, int height, int width,
+                                  int channels, int kernel_size, int pad, void *stream) {
+  return dw_backward_impl(input, weight, grad_output, grad_input, grad_weight, grad_bias, workspace, workspace_bytes, dtype,
+                          DCNV4_DTYPE_F32, batch, height, width, channels, kernel_size, pad, stream);
+}
+
+}  // namespace dcn

@@ -2,6 +2,7 @@
 // launchers defined next to the kernels.  Everything is plain data passed by value to kernels.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "layer_norm.hpp"
 #include <stdint.h>
 
 #include <mutex>
@@ -214,22 +215,6 @@ struct DwLaunch {
   int slab, n_part;        // grad_weight: row segments (seg columns each) per workgroup, workgroups
 };
 
-// out = residual + gamma * LayerNorm(y) over rows of C channels (residual and gamma may be null).
-struct LnLaunch {
-  const void *y, *residual, *weight, *bias, *gamma;
-  void *out;
-  long long rows;
-  int C;
-  float eps;
-  int team;      // lanes per row: a power of two, <= 64
-  int vpl;       // 16-byte vectors per lane: 1, 2, 4 or 8 (team * vpl * 16 bytes cover a row)
-  // backward
-  const void *grad_out;
-  void *grad_y, *grad_weight, *grad_bias, *grad_gamma;     // the three parameter gradients may be null
-  float *partial;   // [n_part][3][C] column sums of one workgroup each: grad_weight, grad_bias, grad_gamma
-  long long slab;   // consecutive rows per workgroup (a multiple of the rows one pass of the workgroup takes)
-  int n_part;       // workgroups of the backward
-};
 // Centre-feature blend: out = y * (1 - gate) + x * gate, gate[g] = sigmoid(<W[g,:], y> + b[g]) per (row, group).
 struct CfLaunch {
   const void *y, *x, *weight, *bias;      // y, x [rows, C]; weight [G, C]; bias [G]
@@ -242,8 +227,6 @@ struct CfLaunch {
   int team, vpl;                          // as in LnLaunch
 };
 hipError_t launch_center_feature_blend(int dtype, const CfLaunch &p, bool backward, hipStream_t stream);
-hipError_t launch_layer_norm_residual(int dtype, const LnLaunch &p, hipStream_t stream);
-hipError_t launch_layer_norm_residual_backward(int dtype, const LnLaunch &p, hipStream_t stream);
 
 // Each returns hipSuccess or the launch error.  dtype: 0 fp32, 1 fp16, 2 bf16.
 hipError_t launch_depthwise_forward(int dtype, const DwLaunch &p, hipStream_t stream);

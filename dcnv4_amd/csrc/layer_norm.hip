@@ -17,19 +17,57 @@ namespace {
 
 constexpr int kLnThreads = 256;
 
-template <typename Tag, int VPL>
+// V elements of a row as raw words: one word of up to 16 bytes, or two of 16 (fp32 beside eight 16-bit elements).
+template <typename Tag, int V> struct Elems {
+  static constexpr bool kTwo = V * Tag::kBytes > 16;
+  typedef Pack<Tag, kTwo ? V / 2 : V> half_t;
+  struct raw_t { typename half_t::raw_t w[kTwo ? 2 : 1]; };
+  static __device__ __forceinline__ raw_t load(const void *base, size_t i) { return static_cast<const raw_t *>(base)[i]; }
+  static __device__ __forceinline__ void decode(const raw_t &r, float (&f)[V]) {
+    if constexpr (kTwo) {
+      float a[V / 2], b[V / 2];
+      half_t::decode(r.w[0], a);
+      half_t::decode(r.w[1], b);
+#pragma unroll
+      for (int c = 0; c < V / 2; ++c) { f[c] = a[c]; f[V / 2 + c] = b[c]; }
+    } else {
+      half_t::decode(r.w[0], f);
+    }
+  }
+  static __device__ __forceinline__ void store(void *base, size_t i, const float (&f)[V]) {
+    raw_t r;
+    if constexpr (kTwo) {
+      float a[V / 2], b[V / 2];
+#pragma unroll
+      for (int c = 0; c < V / 2; ++c) { a[c] = f[c]; b[c] = f[V / 2 + c]; }
+      r.w[0] = half_t::encode(a);
+      r.w[1] = half_t::encode(b);
+    } else {
+      r.w[0] = half_t::encode(f);
+    }
+    static_cast<raw_t *>(base)[i] = r;
+  }
+};
+
+// What a row's branch is scaled by beside gamma: stochastic depth, one factor per sample.
+__device__ __forceinline__ float row_scale(const LnLaunch &p, size_t row) {
+  return p.row_scale != nullptr ? p.row_scale[row / (size_t)p.scale_rows] : 1.f;
+}
+
+// Y: the normalised tensor (and the copy); R: residual and result; P: weight, bias, gamma.  Mixed-precision training has a
+// 16-bit Y beside fp32 R and P, and takes a 16-bit copy of the result for the next matrix product along.
+template <typename Y, typename R, typename P, int VPL>
 __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_kernel(const LnLaunch p) {
-  constexpr int V = 16 / Tag::kBytes;
-  typedef Pack<Tag, V> pack;
-  typedef typename pack::raw_t raw_t;
+  constexpr int V = 16 / Y::kBytes;
+  typedef Elems<Y, V> ey;
+  typedef Elems<R, V> er;
+  typedef Elems<P, V> ep;
   const int team = p.team, nvec = p.C / V;
   const int teams_per_block = kLnThreads / team;
   const int lane_in_team = threadIdx.x & (team - 1);
   const size_t row = (size_t)blockIdx.x * teams_per_block + threadIdx.x / team;
   const bool row_live = row < (size_t)p.rows;
-  const raw_t *y = reinterpret_cast<const raw_t *>(p.y) + row * nvec;
-  const raw_t *res = reinterpret_cast<const raw_t *>(p.residual) + row * nvec;
-  raw_t *out = reinterpret_cast<raw_t *>(p.out) + row * nvec;
+  const size_t first = row * nvec;
 
   float v[VPL][V];
   bool live[VPL];
@@ -39,7 +77,7 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_kernel(const L
     const int i = lane_in_team + u * team;
     live[u] = row_live && i < nvec;
     if (live[u]) {
-      pack::decode(y[i], v[u]);
+      ey::decode(ey::load(p.y, first + i), v[u]);
 #pragma unroll
       for (int c = 0; c < V; ++c) sum += v[u][c];
     } else {
@@ -58,40 +96,45 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_kernel(const L
   sq = cluster_sum(sq, team);
   const float rstd = rsqrtf(sq / (float)p.C + p.eps);
 
+  const float scale = row_live ? row_scale(p, row) : 1.f;
 #pragma unroll
   for (int u = 0; u < VPL; ++u) {
     if (!live[u]) continue;
     const int i = lane_in_team + u * team;
     float w[V], b[V], r[V];
-    pack::decode(reinterpret_cast<const raw_t *>(p.weight)[i], w);
-    pack::decode(reinterpret_cast<const raw_t *>(p.bias)[i], b);
+    ep::decode(ep::load(p.weight, i), w);
+    ep::decode(ep::load(p.bias, i), b);
 #pragma unroll
     for (int c = 0; c < V; ++c) r[c] = fmaf((v[u][c] - mean) * rstd, w[c], b[c]);
     if (p.gamma != nullptr) {
       float g[V];
-      pack::decode(reinterpret_cast<const raw_t *>(p.gamma)[i], g);
+      ep::decode(ep::load(p.gamma, i), g);
 #pragma unroll
       for (int c = 0; c < V; ++c) r[c] *= g[c];
     }
+    if (p.row_scale != nullptr)
+#pragma unroll
+      for (int c = 0; c < V; ++c) r[c] *= scale;
     if (p.residual != nullptr) {
       float x[V];
-      pack::decode(res[i], x);
+      er::decode(er::load(p.residual, first + i), x);
 #pragma unroll
       for (int c = 0; c < V; ++c) r[c] += x[c];
     }
-    out[i] = pack::encode(r);
+    er::store(p.out, first + i, r);
+    if (p.copy != nullptr) ey::store(p.copy, first + i, r);
   }
 }
 
-template <typename Tag>
+template <typename Y, typename R, typename P>
 hipError_t launch_t(const LnLaunch &p, hipStream_t stream) {
   const int teams_per_block = kLnThreads / p.team;
   const dim3 grid((unsigned)((p.rows + teams_per_block - 1) / teams_per_block)), block(kLnThreads);
   switch (p.vpl) {
-    case 1: hipLaunchKernelGGL((layer_norm_residual_kernel<Tag, 1>), grid, block, 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((layer_norm_residual_kernel<Tag, 2>), grid, block, 0, stream, p); break;
-    case 4: hipLaunchKernelGGL((layer_norm_residual_kernel<Tag, 4>), grid, block, 0, stream, p); break;
-    case 8: hipLaunchKernelGGL((layer_norm_residual_kernel<Tag, 8>), grid, block, 0, stream, p); break;
+    case 1: hipLaunchKernelGGL((layer_norm_residual_kernel<Y, R, P, 1>), grid, block, 0, stream, p); break;
+    case 2: hipLaunchKernelGGL((layer_norm_residual_kernel<Y, R, P, 2>), grid, block, 0, stream, p); break;
+    case 4: hipLaunchKernelGGL((layer_norm_residual_kernel<Y, R, P, 4>), grid, block, 0, stream, p); break;
+    case 8: hipLaunchKernelGGL((layer_norm_residual_kernel<Y, R, P, 8>), grid, block, 0, stream, p); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -109,12 +152,16 @@ hipError_t launch_t(const LnLaunch &p, hipStream_t stream) {
 // consecutive rows and keeps the three column sums of its lanes' channels in registers; at the end the teams
 // of the workgroup are added through LDS in a fixed order and the workgroup writes one row of partial sums;
 // a second kernel adds the partial rows in order.  No atomics: the result does not depend on scheduling.
-template <typename Tag, int VPL>
+// G: grad_out; Y: the normalised tensor; D: grad_y (and an addend to it: the gradient that reaches y around the
+// normalisation); P: the parameters and their gradients.
+template <typename G, typename Y, typename D, typename P, int VPL>
 __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kernel(const LnLaunch p) {
   extern __shared__ float s_cols[];                     // [teams][C]
-  constexpr int V = 16 / Tag::kBytes;
-  typedef Pack<Tag, V> pack;
-  typedef typename pack::raw_t raw_t;
+  constexpr int V = 16 / Y::kBytes;
+  typedef Elems<G, V> eg;
+  typedef Elems<Y, V> ey;
+  typedef Elems<D, V> ed;
+  typedef Elems<P, V> ep;
   const int team = p.team, nvec = p.C / V;
   const int teams_per_block = kLnThreads / team;
   const int lane_in_team = threadIdx.x & (team - 1), team_id = threadIdx.x / team;
@@ -130,10 +177,10 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kerne
 #pragma unroll
     for (int c = 0; c < V; ++c) { w[u][c] = 0.f; gam[u][c] = 1.f; b[u][c] = 0.f; dw[u][c] = db[u][c] = dg[u][c] = 0.f; }
     if (col_live[u]) {
-      pack::decode(reinterpret_cast<const raw_t *>(p.weight)[i], w[u]);
+      ep::decode(ep::load(p.weight, i), w[u]);
       if (p.gamma != nullptr) {
-        pack::decode(reinterpret_cast<const raw_t *>(p.gamma)[i], gam[u]);
-        pack::decode(reinterpret_cast<const raw_t *>(p.bias)[i], b[u]);
+        ep::decode(ep::load(p.gamma, i), gam[u]);
+        ep::decode(ep::load(p.bias, i), b[u]);
       }
     }
   }
@@ -141,18 +188,19 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kerne
   const long long row_begin = (long long)blockIdx.x * p.slab;
   const long long row_end = row_begin + p.slab < p.rows ? row_begin + p.slab : p.rows;
   // the rows of the next pass are requested before the current pass is worked on
-  raw_t next_y[VPL], next_g[VPL];
+  typename ey::raw_t next_y[VPL];
+  typename eg::raw_t next_g[VPL];
   auto request = [&](long long row0) {
     const long long row = row0 + team_id;
 #pragma unroll
     for (int u = 0; u < VPL; ++u) {
       const int i = lane_in_team + u * team;
       if (row < row_end && col_live[u]) {
-        next_y[u] = reinterpret_cast<const raw_t *>(p.y)[row * nvec + i];
-        next_g[u] = reinterpret_cast<const raw_t *>(p.grad_out)[row * nvec + i];
+        next_y[u] = ey::load(p.y, row * nvec + i);
+        next_g[u] = eg::load(p.grad_out, row * nvec + i);
       } else {
-        next_y[u] = raw_t{};
-        next_g[u] = raw_t{};
+        next_y[u] = {};
+        next_g[u] = {};
       }
     }
   };
@@ -164,10 +212,17 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kerne
     float sum = 0.f;
 #pragma unroll
     for (int u = 0; u < VPL; ++u) {
-      pack::decode(next_y[u], v[u]);
-      pack::decode(next_g[u], g[u]);
+      ey::decode(next_y[u], v[u]);
+      eg::decode(next_g[u], g[u]);
 #pragma unroll
       for (int c = 0; c < V; ++c) sum += v[u][c];
+    }
+    if (p.row_scale != nullptr) {
+      const float scale = row_live ? row_scale(p, row) : 1.f;
+#pragma unroll
+      for (int u = 0; u < VPL; ++u)
+#pragma unroll
+        for (int c = 0; c < V; ++c) g[u][c] *= scale;
     }
     request(row0 + teams_per_block);
     sum = cluster_sum(sum, team);
@@ -202,14 +257,20 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kerne
     s2 = cluster_sum(s2, team);
     const float m1 = s1 * inv_c, m2 = s2 * inv_c;
     if (row_live) {
-      raw_t *gy = reinterpret_cast<raw_t *>(p.grad_y) + row * nvec;
 #pragma unroll
       for (int u = 0; u < VPL; ++u) {
         if (!col_live[u]) continue;
+        const size_t at = row * nvec + lane_in_team + u * team;
         float r[V];
 #pragma unroll
         for (int c = 0; c < V; ++c) r[c] = rstd * (g[u][c] - m1 - v[u][c] * m2);
-        gy[lane_in_team + u * team] = pack::encode(r);
+        if (p.addend != nullptr) {
+          float x[V];
+          ed::decode(ed::load(p.addend, at), x);
+#pragma unroll
+          for (int c = 0; c < V; ++c) r[c] += x[c];
+        }
+        ed::store(p.grad_y, at, r);
       }
     }
   }
@@ -260,41 +321,62 @@ __global__ void __launch_bounds__(kPgCols * kPgRows) layer_norm_param_grad_kerne
   reinterpret_cast<typename RawWord<Tag::kBytes>::type *>(dst)[c] = Pack<Tag, 1>::encode(f);
 }
 
-template <typename Tag>
+template <typename G, typename Y, typename D, typename P>
 hipError_t launch_bwd_t(const LnLaunch &p, hipStream_t stream) {
   const int teams_per_block = kLnThreads / p.team;
   const dim3 grid((unsigned)p.n_part), block(kLnThreads);
   const size_t lds = (size_t)teams_per_block * p.C * sizeof(float);
   switch (p.vpl) {
-    case 1: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<Tag, 1>), grid, block, lds, stream, p); break;
-    case 2: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<Tag, 2>), grid, block, lds, stream, p); break;
-    case 4: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<Tag, 4>), grid, block, lds, stream, p); break;
-    case 8: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<Tag, 8>), grid, block, lds, stream, p); break;
+    case 1: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<G, Y, D, P, 1>), grid, block, lds, stream, p); break;
+    case 2: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<G, Y, D, P, 2>), grid, block, lds, stream, p); break;
+    case 4: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<G, Y, D, P, 4>), grid, block, lds, stream, p); break;
+    case 8: hipLaunchKernelGGL((layer_norm_residual_backward_kernel<G, Y, D, P, 8>), grid, block, lds, stream, p); break;
     default: return hipErrorInvalidValue;
   }
   if (hipError_t e = hipGetLastError()) return e;
-  hipLaunchKernelGGL((layer_norm_param_grad_kernel<Tag>), dim3((unsigned)((3 * p.C + kPgCols - 1) / kPgCols)), dim3(kPgCols * kPgRows), 0, stream, p);
+  hipLaunchKernelGGL((layer_norm_param_grad_kernel<P>), dim3((unsigned)((3 * p.C + kPgCols - 1) / kPgCols)), dim3(kPgCols * kPgRows), 0, stream, p);
   return hipGetLastError();
+}
+
+// Mixed precision: parameters in fp32, H the 16-bit type.  Forward: a 16-bit tensor into an fp32 stream (post-norm) or into
+// 16 bits, an fp32 stream into 16 bits (pre-norm).  Backward: the same, from the result's type.
+template <typename H>
+hipError_t launch_mixed_t(const LnLaunch &p, bool y32, bool r32, hipStream_t stream) {
+  if (y32) return r32 ? hipErrorInvalidValue : launch_t<F32, H, F32>(p, stream);
+  return r32 ? launch_t<H, F32, F32>(p, stream) : launch_t<H, H, F32>(p, stream);
+}
+template <typename H>
+hipError_t launch_mixed_bwd_t(const LnLaunch &p, bool g32, bool y32, hipStream_t stream) {
+  if (y32) return g32 ? hipErrorInvalidValue : launch_bwd_t<H, F32, F32, F32>(p, stream);
+  return g32 ? launch_bwd_t<F32, H, H, F32>(p, stream) : launch_bwd_t<H, H, H, F32>(p, stream);
 }
 
 }  // namespace
 
 hipError_t launch_layer_norm_residual(int dtype, const LnLaunch &p, hipStream_t stream) {
   switch (dtype) {
-    case F32::kCode: return launch_t<F32>(p, stream);
-    case F16::kCode: return launch_t<F16>(p, stream);
-    case BF16::kCode: return launch_t<BF16>(p, stream);
+    case F32::kCode: return launch_t<F32, F32, F32>(p, stream);
+    case F16::kCode: return launch_t<F16, F16, F16>(p, stream);
+    case BF16::kCode: return launch_t<BF16, BF16, BF16>(p, stream);
   }
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_layer_norm_residual_backward(int dtype, const LnLaunch &p, hipStream_t stream) {
   switch (dtype) {
-    case F32::kCode: return launch_bwd_t<F32>(p, stream);
-    case F16::kCode: return launch_bwd_t<F16>(p, stream);
-    case BF16::kCode: return launch_bwd_t<BF16>(p, stream);
+    case F32::kCode: return launch_bwd_t<F32, F32, F32, F32>(p, stream);
+    case F16::kCode: return launch_bwd_t<F16, F16, F16, F16>(p, stream);
+    case BF16::kCode: return launch_bwd_t<BF16, BF16, BF16, BF16>(p, stream);
   }
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_layer_norm_mixed(int half_dtype, bool y32, bool r32, const LnLaunch &p, hipStream_t stream) {
+  return half_dtype == F16::kCode ? launch_mixed_t<F16>(p, y32, r32, stream) : launch_mixed_t<BF16>(p, y32, r32, stream);
+}
+
+hipError_t launch_layer_norm_mixed_backward(int half_dtype, bool g32, bool y32, const LnLaunch &p, hipStream_t stream) {
+  return half_dtype == F16::kCode ? launch_mixed_bwd_t<F16>(p, g32, y32, stream) : launch_mixed_bwd_t<BF16>(p, g32, y32, stream);
 }
 
 }  // namespace dcn

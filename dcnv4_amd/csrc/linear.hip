@@ -31,29 +31,55 @@ struct Columns {
   }
 };
 
-// The epilogue for eight consecutive features of one row: 16 bytes in and out.
-template <typename Tag>
+// The epilogue for eight consecutive features of one row: 16 bytes in and out.  EXTRA: with what training adds, which
+// costs the small tiles a third more registers.
+template <typename Tag, bool EXTRA>
 __device__ __forceinline__ void finish(const LinearProblem &q, const Columns<Tag> &col, int gelu, long long row, int n, float (&v)[8]) {
   if (col.has_bias)
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] += col.bias[c];
+  const size_t element = (size_t)row * q.n + n, at = element * 2;
+  auto half_at = [&](const void *base, float (&f)[8]) { Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(base) + at), f); };
+  if (EXTRA && q.pre != nullptr) *reinterpret_cast<u32x4 *>(static_cast<char *>(q.pre) + at) = Pack<Tag, 8>::encode(v);
   if (gelu)
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] = gelu_exact(v[c]);
+  if (EXTRA && q.gelu_grad_at != nullptr) {
+    float x[8];
+    half_at(q.gelu_grad_at, x);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] *= gelu_derivative(x[c]);
+  }
   if (col.has_gamma)
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] *= col.gamma[c];
-  const size_t at = ((size_t)row * q.n + n) * 2;
+  if (EXTRA && q.row_scale != nullptr) {
+    const float s = q.row_scale[row / q.scale_rows];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] *= s;
+  }
   if (q.residual != nullptr) {
     float r[8];
-    Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.residual) + at), r);
+    half_at(q.residual, r);
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] += r[c];
   }
-  *reinterpret_cast<u32x4 *>(static_cast<char *>(q.out) + at) = Pack<Tag, 8>::encode(v);
+  if (EXTRA && q.residual32 != nullptr) {
+    const f32x4 *r = reinterpret_cast<const f32x4 *>(q.residual32 + element);
+    const f32x4 lo = r[0], hi = r[1];
+    v[0] += lo.x; v[1] += lo.y; v[2] += lo.z; v[3] += lo.w;
+    v[4] += hi.x; v[5] += hi.y; v[6] += hi.z; v[7] += hi.w;
+  }
+  if (EXTRA && q.out32 != nullptr) {
+    f32x4 *o = reinterpret_cast<f32x4 *>(q.out32 + element);
+    o[0] = f32x4{v[0], v[1], v[2], v[3]};
+    o[1] = f32x4{v[4], v[5], v[6], v[7]};
+  } else {
+    *reinterpret_cast<u32x4 *>(static_cast<char *>(q.out) + at) = Pack<Tag, 8>::encode(v);
+  }
 }
 
-template <typename Tag, int BM, int BN, int WM, int WN>
+template <typename Tag, int BM, int BN, int WM, int WN, bool EXTRA>
 __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
   static_assert(WM * WN == 4 && BM % (16 * WM) == 0 && BN % (32 * WN) == 0 && BM % 32 == 0, "tile shape");
   constexpr int MF = BM / WM / 16, NF = BN / WN / 16;
@@ -133,7 +159,7 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
       const int r = u * rows_per_pass + lane / lanes_per_row, row = wm * (BM / WM) + j * 16 + r;
       const f32x4 lo = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col), hi = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col + 4);
       float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      if (row < live_m && n < live_n) finish<Tag>(q, columns, p.gelu, m0 + row, n0 + n, v);
+      if (row < live_m && n < live_n) finish<Tag, EXTRA>(q, columns, p.gelu, m0 + row, n0 + n, v);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -141,7 +167,7 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
 
 constexpr int kFewTile = 32;
 
-template <typename Tag>
+template <typename Tag, bool EXTRA>
 __global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
   __shared__ __align__(16) float part[4][kFewTile][kFewTile + 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -190,24 +216,24 @@ __global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch
     for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
     v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
   }
-  if (row < live_m && n < live_n) finish<Tag>(q, columns, p.gelu, m0 + row, n0 + n, v);
+  if (row < live_m && n < live_n) finish<Tag, EXTRA>(q, columns, p.gelu, m0 + row, n0 + n, v);
 }
 
-template <typename Tag, int BM, int BN, int WM, int WN>
+template <typename Tag, bool EXTRA, int BM, int BN, int WM, int WN>
 hipError_t launch_tiled(const LinearLaunch &p, hipStream_t stream) {
   const long long tiles_m = (p.rows + BM - 1) / BM;
   const int tiles_n0 = (p.p[0].n + BN - 1) / BN, tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + BN - 1) / BN : 0);
   if (tiles_m * tiles_n > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((linear_tiled_kernel<Tag, BM, BN, WM, WN>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p,
+  hipLaunchKernelGGL((linear_tiled_kernel<Tag, BM, BN, WM, WN, EXTRA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p,
                      tiles_n0, tiles_n);
   return hipGetLastError();
 }
 
-template <typename Tag>
+template <typename Tag, bool EXTRA>
 hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
   const int tiles_m = (int)((p.rows + kFewTile - 1) / kFewTile), tiles_n0 = (p.p[0].n + kFewTile - 1) / kFewTile;
   const int tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kFewTile - 1) / kFewTile : 0);
-  hipLaunchKernelGGL((linear_few_rows_kernel<Tag>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p, tiles_n0, tiles_n);
+  hipLaunchKernelGGL((linear_few_rows_kernel<Tag, EXTRA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p, tiles_n0, tiles_n);
   return hipGetLastError();
 }
 
@@ -217,19 +243,19 @@ hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
 //   128x64 against 128x128: 25088 x 448 x 448 17.7 / 18.9, 25088 x 1792 x 448 62.5 / 55.5, 6272 x 3584 x 896 59.3 / 51.4,
 //     6272 x 1512 x 896 25.4 / 30.1 (600 against 588 tiles of which the last round is a third full)
 //   256x64 where the width is not a multiple of 128: 401408 x 192 x 112 52.4 against 62.0
-template <typename Tag>
+template <typename Tag, bool EXTRA>
 hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
   auto tiles = [&](int bm, int bn) {
     long long n = 0;
     for (int i = 0; i < p.count; ++i) n += (p.p[i].n + bn - 1) / bn;
     return n * ((p.rows + bm - 1) / bm);
   };
-  if (tiles(64, 64) < 64) return launch_few<Tag>(p, stream);
-  if (tiles(128, 64) < kCus) return launch_tiled<Tag, 64, 64, 2, 2>(p, stream);
+  if (tiles(64, 64) < 64) return launch_few<Tag, EXTRA>(p, stream);
+  if (tiles(128, 64) < kCus) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
   const long long wide = tiles(128, 128), narrow = tiles(128, 64);
-  if (wide < 4 * kCus) return launch_tiled<Tag, 128, 64, 4, 1>(p, stream);
-  if (20 * wide <= 11 * narrow) return launch_tiled<Tag, 128, 128, 2, 2>(p, stream);
-  return launch_tiled<Tag, 256, 64, 4, 1>(p, stream);
+  if (wide < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
+  if (20 * wide <= 11 * narrow) return launch_tiled<Tag, EXTRA, 128, 128, 2, 2>(p, stream);
+  return launch_tiled<Tag, EXTRA, 256, 64, 4, 1>(p, stream);
 }
 
 }  // namespace
@@ -240,7 +266,13 @@ bool linear_fits(int dtype, long long rows, int n, int k) {
 }
 
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream) {
-  return dtype == F16::kCode ? launch_t<F16>(p, stream) : launch_t<BF16>(p, stream);
+  bool extra = false;
+  for (int i = 0; i < p.count; ++i) {
+    const LinearProblem &q = p.p[i];
+    extra |= q.pre != nullptr || q.gelu_grad_at != nullptr || q.residual32 != nullptr || q.out32 != nullptr || q.row_scale != nullptr;
+  }
+  if (dtype == F16::kCode) return extra ? launch_t<F16, true>(p, stream) : launch_t<F16, false>(p, stream);
+  return extra ? launch_t<BF16, true>(p, stream) : launch_t<BF16, false>(p, stream);
 }
 
 }  // namespace dcn

@@ -3,14 +3,22 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace dcn {
 
 // out[m, n] = act(a[m, :] . w[n, :] + bias[n]) * gamma[n] + residual[m, n]; a [rows, k], w [n, k], out and residual
-// [rows, n], all dense.  bias, gamma and residual may be null.
+// [rows, n], all dense.  bias, gamma and residual may be null, and so may what training adds.
 struct LinearProblem {
   const void *a, *w, *bias, *gamma, *residual;
   void *out;
   int n;
+  void *pre;                   // the product before act, as out
+  const void *gelu_grad_at;    // [rows, n]: times the derivative of the GELU there, in place of act
+  const float *residual32;     // another residual, fp32
+  float *out32;                // the result in fp32, in place of out
+  const float *row_scale;      // per sample of scale_rows rows: factor in front of the residuals
+  int scale_rows;
 };
 
 // Up to two products over the same rows and depth in one launch (a layer's value and offset projections).
@@ -25,5 +33,54 @@ struct LinearLaunch {
 // Whether the matrix kernels take a product: 16-bit tensors, depth and width in whole 16-byte vectors.
 bool linear_fits(int dtype, long long rows, int n, int k);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
+
+// grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k] (and grad_bias[n], may be null), several products over the same
+// rows at once.  With splits > 1 grad_w and grad_bias point into partial sums whose splits lie split_stride floats apart.
+constexpr int kMaxWeightGrads = 6;
+struct WeightGradProblem {
+  const void *grad_out, *in;
+  float *grad_w, *grad_bias;
+  int n, k;
+};
+struct WeightGradLaunch {
+  WeightGradProblem p[kMaxWeightGrads];
+  int tile_end[kMaxWeightGrads];      // set by the launcher
+  int count, splits;
+  long long rows, rows_per_split;     // the latter set by the launcher
+  size_t split_stride;
+};
+struct WeightGradPlan { int tile, splits; };
+WeightGradPlan plan_weight_grad(const WeightGradLaunch &p);
+hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &p, int tile, hipStream_t stream);
+
+struct WeightGradSegment {
+  float *grad;
+  size_t offset;                      // of the segment in a split's partial sums, a multiple of 4
+  int count;
+};
+struct WeightGradReduce {
+  WeightGradSegment s[2 * kMaxWeightGrads];
+  int count, splits;
+  const float *partial;
+  size_t split_stride;
+};
+hipError_t launch_weight_grad_reduce(const WeightGradReduce &p, hipStream_t stream);
+
+// 16-bit copies of fp32 matrices [n, k], and turned ones [k, n] (may be null).
+constexpr int kMaxCasts = 16;
+struct CastWeights {
+  const float *from;
+  void *to, *turned;
+  int n, k;
+};
+struct CastWeightsLaunch {
+  CastWeights p[kMaxCasts];
+  int tile_end[kMaxCasts];            // set by the launcher
+  int count;
+};
+hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &p, hipStream_t stream);
+// dst = 16-bit src (fp32, or 16-bit with a factor per sample of scale_elements elements); n and scale_elements multiples of 8
+hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
+                              hipStream_t stream);
 
 }  // namespace dcn

@@ -1,0 +1,267 @@
+// Weight gradients of linear layers, and the 16-bit copies of their weights that mixed-precision training works with.
+//
+// linear_weight_grad_kernel: grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k], for all the linear layers of a
+// block in one launch.  The reduction runs over the slow axis of both operands, so a fragment's eight values lie a row
+// apart: slices of 64 rows come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns them
+// on the way into registers (16 lanes read 4 rows x 16 columns; lane i gets column i).  A row's 32-byte units are stored at
+// unit ^ f(row), f taking each value once over the eight rows that half a wave reads, so those reads fall into different
+// banks.  The rows are split over workgroups until the chip is full, partial sums are fp32 and are added in split order by
+// linear_grad_reduce_kernel: no atomics, the same bits every time.  The bias gradient is one more matrix instruction per
+// fragment, against a vector of ones.
+//   12544 rows, five layers of 448 channels (59 GFLOP): the library's one product at a time left 49 workgroups for each
+//   (82 us, five of them, 412 us) and its column sums took 65 us more.
+#include "linear.hpp"
+#include "mfma.hpp"
+
+namespace dcn {
+namespace {
+
+constexpr int kRows = 64;      // rows of a slice
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ u32x2 read_turned(const char *lds) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)lds));
+}
+
+template <int WIDTH>
+__device__ __forceinline__ int unit_swizzle(int row) {      // 32-byte units of a row of WIDTH 16-bit elements
+  return WIDTH == 128 ? (row & 3) | ((row >> 1) & 4) : ((row >> 1) & 1) | ((row >> 2) & 2);
+}
+
+template <typename Tag, int W>
+__global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGradLaunch p) {
+  static_assert(W == 64 || W == 128, "tile side");
+  constexpr int kRowBytes = W * 2, F = W / 2 / 16;              // a wave takes W/2 x W/2
+  constexpr int kRowsPerLoad = 64 * 16 / kRowBytes, kLoads = kRows / kRowsPerLoad / 4;
+  __shared__ __align__(16) char lds[2][2][kRows * kRowBytes];   // [buffer][grad_out, in]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int split = blockIdx.x % p.splits, tile = blockIdx.x / p.splits;
+  int which = 0;
+  while (which + 1 < p.count && tile >= p.tile_end[which]) ++which;
+  const WeightGradProblem &q = p.p[which];
+  const int local = tile - (which ? p.tile_end[which - 1] : 0), tiles_k = (q.k + W - 1) / W;
+  const int n0 = local / tiles_k * W, k0 = local % tiles_k * W;
+  const long long row_begin = (long long)split * p.rows_per_split;
+  const long long row_end = min(row_begin + p.rows_per_split, p.rows);
+
+  // a wave's load covers kRowsPerLoad rows; a lane's 16 bytes go to position lane, which holds unit (u ^ f) of the row
+  const int load_row = lane * 16 / kRowBytes, load_chunk = lane % (kRowBytes / 16);
+  auto stage = [&](long long row0, char (&buf)[2][kRows * kRowBytes]) {
+    const int live = (int)max(0ll, min((long long)kRows, row_end - row0));
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.n * 2, (uint32_t)live * q.n * 2);
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char *>(q.in) + (size_t)row0 * q.k * 2, (uint32_t)live * q.k * 2);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int base = (i * 4 + wave) * kRowsPerLoad, row = base + load_row;
+      const int col = (((load_chunk >> 1) ^ unit_swizzle<W>(row)) * 2 + (load_chunk & 1)) * 8;
+      // columns beyond the matrix read the next row's values; they only reach results beyond the matrix
+      load_to_lds(rg, buf[0] + base * kRowBytes, (uint32_t)(row * q.n + n0 + col) * 2);
+      load_to_lds(rx, buf[1] + base * kRowBytes, (uint32_t)(row * q.k + k0 + col) * 2);
+    }
+  };
+
+  const int wn = wave >> 1, wk = wave & 1, kb = lane >> 4, i16 = lane & 15;
+  const int frag_row = kb * 8 + (i16 >> 2), f = unit_swizzle<W>(frag_row);
+  int at_n[F], at_k[F];
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    at_n[i] = frag_row * kRowBytes + (((wn * F + i) ^ f) * 32) + (i16 & 3) * 8;
+    at_k[i] = frag_row * kRowBytes + (((wk * F + i) ^ f) * 32) + (i16 & 3) * 8;
+  }
+  auto fragment = [&](const char *base, int at, int s) {
+    const u32x2 lo = read_turned(base + at + s * 32 * kRowBytes), hi = read_turned(base + at + (s * 32 + 4) * kRowBytes);
+    return u32x4{lo.x, lo.y, hi.x, hi.y};
+  };
+  const uint32_t one = Tag::kCode == F16::kCode ? 0x3c003c00u : 0x3f803f80u;
+  const u32x4 ones = {one, one, one, one};
+  const bool with_bias = q.grad_bias != nullptr && k0 == 0 && wk == 0;
+
+  f32x4 acc[F][F], bias[F];
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    bias[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (row_begin < row_end) stage(row_begin, lds[0]);
+  int cur = 0;
+  for (long long row0 = row_begin; row0 < row_end; row0 += kRows, cur ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    u32x4 fn[2][F], fk[2][F];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+        fn[s][i] = fragment(lds[cur][0], at_n[i], s);
+        fk[s][i] = fragment(lds[cur][1], at_k[i], s);
+      }
+    if (row0 + kRows < row_end) stage(row0 + kRows, lds[cur ^ 1]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = mfma_16x16x32<Tag>(fk[s][j], fn[s][i], acc[i][j]);
+        if (with_bias) bias[i] = mfma_16x16x32<Tag>(ones, fn[s][i], bias[i]);
+      }
+  }
+  // results: rows of the fragment are the depth, so a lane stores four consecutive k of one n
+  float *grad_w = q.grad_w + (size_t)split * p.split_stride, *grad_b = q.grad_bias + (size_t)split * p.split_stride;
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    const int n = n0 + (wn * F + i) * 16 + i16;
+    if (n >= q.n) continue;
+    if (with_bias && kb == 0) grad_b[n] = bias[i].x;
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const int k = k0 + (wk * F + j) * 16 + kb * 4;
+      if (k < q.k) *reinterpret_cast<f32x4 *>(grad_w + (size_t)n * q.k + k) = acc[i][j];
+    }
+  }
+}
+
+// partial sums [split][split_stride] -> the gradients; every segment starts on a 16-byte boundary and a whole vector of padding
+// may be read behind it
+__global__ void __launch_bounds__(256) linear_grad_reduce_kernel(const WeightGradReduce p) {
+  const WeightGradSegment &s = p.s[blockIdx.y];
+  const int stride = gridDim.x * 256;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i * 4 < s.count; i += stride) {
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    const float *src = p.partial + s.offset + (size_t)i * 4;
+    int split = 0;
+    for (; split + 4 <= p.splits; split += 4) {
+      f32x4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const f32x4 *>(src + (size_t)(split + u) * p.split_stride);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sum += v[u];
+    }
+    for (; split < p.splits; ++split) sum += *reinterpret_cast<const f32x4 *>(src + (size_t)split * p.split_stride);
+    if (i * 4 + 4 <= s.count) {
+      *reinterpret_cast<f32x4 *>(s.grad + (size_t)i * 4) = sum;
+    } else {
+      for (int c = 0; i * 4 + c < s.count; ++c) s.grad[(size_t)i * 4 + c] = sum[c];
+    }
+  }
+}
+
+// 16-bit copies of fp32 parameters: a matrix [n, k] as it lies and turned [k, n], in tiles of 64 x 64 through LDS; a vector
+// (n = 1, nothing turned) as a row.
+template <typename Tag>
+__global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaunch p) {
+  typedef typename RawWord<2>::type half_t;
+  __shared__ half_t tile[64][66];
+  int which = 0;
+  while (which + 1 < p.count && (int)blockIdx.x >= p.tile_end[which]) ++which;
+  const CastWeights &q = p.p[which];
+  const int local = blockIdx.x - (which ? p.tile_end[which - 1] : 0), tiles_k = (q.k + 63) / 64;
+  const int n0 = local / tiles_k * 64, k0 = local % tiles_k * 64;
+  const int col = threadIdx.x & 63;
+  for (int r = threadIdx.x >> 6; r < 64; r += 4) {
+    const int n = n0 + r, k = k0 + col;
+    if (n >= q.n || k >= q.k) continue;
+    const float v[1] = {q.from[(size_t)n * q.k + k]};
+    const half_t h = Pack<Tag, 1>::encode(v);
+    static_cast<half_t *>(q.to)[(size_t)n * q.k + k] = h;
+    tile[r][col] = h;
+  }
+  if (q.turned == nullptr) return;
+  __syncthreads();
+  for (int r = threadIdx.x >> 6; r < 64; r += 4) {
+    const int k = k0 + r, n = n0 + col;
+    if (n < q.n && k < q.k) static_cast<half_t *>(q.turned)[(size_t)k * q.n + n] = tile[col][r];
+  }
+}
+
+template <typename Tag, bool SRC32>
+__global__ void __launch_bounds__(256) narrow_rows_kernel(const void *src, u32x4 *dst, size_t n8, const float *row_scale, size_t scale8) {
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += stride) {
+    float f[8];
+    if constexpr (SRC32) {
+      const f32x4 a = static_cast<const f32x4 *>(src)[2 * i], b = static_cast<const f32x4 *>(src)[2 * i + 1];
+      f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
+    } else {
+      Pack<Tag, 8>::decode(static_cast<const u32x4 *>(src)[i], f);
+    }
+    if (row_scale != nullptr) {
+      const float s = row_scale[i / scale8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) f[c] *= s;
+    }
+    dst[i] = Pack<Tag, 8>::encode(f);
+  }
+}
+
+template <typename Tag, int W>
+hipError_t launch_grad_t(const WeightGradLaunch &p, hipStream_t stream) {
+  hipLaunchKernelGGL((linear_weight_grad_kernel<Tag, W>), dim3((unsigned)(p.tile_end[p.count - 1] * p.splits)), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// Tile and split.  A split is a power of two: consecutive workgroups go to the eight XCDs in turn, and the tiles that read
+// the same rows then share an L2 (12544 rows, 256 channels: 22 splits 67 us, 16 splits 53).  Measured over five layers of C
+// channels, us, 128 / 64 wide tiles at their best split: 12544 x 448 127 / 119, 12544 x 256 48 / 42, 50176 x 128 50 / 44,
+// 50176 x 224 151 / 185, 200704 x 112 169 / 238, 200704 x 64 106 / 84 - the wide tile is for many rows, where it reads its
+// operands half as often, unless most of it is padding.  Best splits: about 3136 rows each for the small tile (42, 44, 84,
+// 119 us above; 2 to 4 times as many cost 15 to 30 % more), about 400 workgroups for the wide one.
+WeightGradPlan plan_weight_grad(const WeightGradLaunch &p) {
+  auto tiles = [&](int w) {
+    long long n = 0;
+    for (int i = 0; i < p.count; ++i) n += (long long)((p.p[i].n + w - 1) / w) * ((p.p[i].k + w - 1) / w);
+    return n;
+  };
+  WeightGradPlan plan;
+  const long long wide = tiles(128), small = tiles(64);
+  plan.tile = p.rows >= 32768 && wide * 4 * 5 <= small * 6 ? 128 : 64;
+  const double want = plan.tile == 64 ? (double)p.rows / 3136 : std::min(400.0 / (double)wide, (double)p.rows / 1500);
+  plan.splits = 1;
+  while (plan.splits < 64 && want >= 1.5 * plan.splits) plan.splits *= 2;
+  return plan;
+}
+
+hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &launch, int tile, hipStream_t stream) {
+  WeightGradLaunch p = launch;
+  p.rows_per_split = ((p.rows + p.splits - 1) / p.splits + kRows - 1) / kRows * kRows;
+  int end = 0;
+  for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + tile - 1) / tile) * ((p.p[i].k + tile - 1) / tile);
+  if (dtype == F16::kCode) return tile == 128 ? launch_grad_t<F16, 128>(p, stream) : launch_grad_t<F16, 64>(p, stream);
+  return tile == 128 ? launch_grad_t<BF16, 128>(p, stream) : launch_grad_t<BF16, 64>(p, stream);
+}
+
+hipError_t launch_weight_grad_reduce(const WeightGradReduce &p, hipStream_t stream) {
+  int most = 1;
+  for (int i = 0; i < p.count; ++i) most = std::max(most, p.s[i].count);
+  hipLaunchKernelGGL(linear_grad_reduce_kernel, dim3((unsigned)std::min(512, (most / 4 + 255) / 256 + 1), (unsigned)p.count), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &launch, hipStream_t stream) {
+  CastWeightsLaunch p = launch;
+  int end = 0;
+  for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + 63) / 64) * ((p.p[i].k + 63) / 64);
+  if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3(end), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(cast_weights_kernel<BF16>, dim3(end), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
+                              hipStream_t stream) {
+  const size_t n8 = n / 8, scale8 = std::max<size_t>(1, scale_elements / 8);
+  const dim3 grid((unsigned)std::max<size_t>(1, std::min<size_t>((n8 + 255) / 256, 4096)));
+  u32x4 *out = static_cast<u32x4 *>(dst);
+  if (dtype == F16::kCode) {
+    if (src32) hipLaunchKernelGGL((narrow_rows_kernel<F16, true>), grid, dim3(256), 0, stream, src, out, n8, row_scale, scale8);
+    else hipLaunchKernelGGL((narrow_rows_kernel<F16, false>), grid, dim3(256), 0, stream, src, out, n8, row_scale, scale8);
+  } else {
+    if (src32) hipLaunchKernelGGL((narrow_rows_kernel<BF16, true>), grid, dim3(256), 0, stream, src, out, n8, row_scale, scale8);
+    else hipLaunchKernelGGL((narrow_rows_kernel<BF16, false>), grid, dim3(256), 0, stream, src, out, n8, row_scale, scale8);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace dcn

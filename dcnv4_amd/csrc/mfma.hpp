@@ -21,17 +21,27 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
 // polynomial in 1 / (1 + 0.35 |x|), fitted by weighted least squares to a relative error of 5e-6 on |x| <= 8.5 (the rounding of a
 // 16-bit result is a hundred times that), so the far negative tail keeps its relative precision too.  13 instructions, two of
 // them transcendental.
-__device__ __forceinline__ float gelu_exact(float x) {
-  const float a = fabsf(x);
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.35f, a, 1.f));
+struct NormalTail {
+  float tail, bell;      // Phi(-|x|) and exp(-x^2 / 2)
+};
+__device__ __forceinline__ NormalTail normal_tail(float x) {
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.35f, fabsf(x), 1.f));
   float p = -0.104951305f;
   p = fmaf(p, t, 0.299319575f);
   p = fmaf(p, t, -0.0110993107f);
   p = fmaf(p, t, 0.184176963f);
   p = fmaf(p, t, 0.132029197f);
   p = fmaf(p, t, 0.000522414528f);
-  const float tail = p * __builtin_amdgcn_exp2f(x * -0.72134752f * x);
-  return fmaf(-a, tail, fmaxf(x, 0.f));
+  NormalTail r;
+  r.bell = __builtin_amdgcn_exp2f(x * -0.72134752f * x);
+  r.tail = p * r.bell;
+  return r;
+}
+__device__ __forceinline__ float gelu_exact(float x) { return fmaf(-fabsf(x), normal_tail(x).tail, fmaxf(x, 0.f)); }
+// Phi(x) + x phi(x)
+__device__ __forceinline__ float gelu_derivative(float x) {
+  const NormalTail n = normal_tail(x);
+  return fmaf(x * 0.39894228f, n.bell, x >= 0.f ? 1.f - n.tail : n.tail);
 }
 
 // 16 bytes per lane from a range-checked buffer straight into LDS: lane l's vector lands at lds + 16 * l.

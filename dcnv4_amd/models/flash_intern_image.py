@@ -130,9 +130,11 @@ class InternImageLayer(nn.Module):
         return residual + self.drop_path(layer_norm_residual(y, ln, gamma))
 
     def forward(self, x, shape):
-        if not torch.is_grad_enabled() and not GFX950_TABLE and ext.dcnv4_forward is _ext_forward:
-            # inference in one call (csrc/binding/layers.cpp) where the kernels take the layer as it is
-            y = ext._native.layer_inference(self, x, *shape)
+        if x.is_cuda and not GFX950_TABLE and ext.dcnv4_forward is _ext_forward:
+            # one call where the kernels take the layer as it is: under autocast csrc/binding/training.cpp, else without
+            # gradients csrc/binding/layers.cpp
+            call = ext._native.layer_training if torch.is_autocast_enabled("cuda") else ext._native.layer_inference
+            y = call(self, x, *shape)
             if y is not None:
                 return y
         g1, g2 = (self.gamma1, self.gamma2) if self.layer_scale else (None, None)

@@ -68,3 +68,65 @@ def test_layer_inference_matches_the_modules_in_fp32(channels, groups, post_norm
     assert seen == [1] and got.dtype == dtype
     tol = 2e-3 if dtype == torch.float16 else 1.5e-2
     assert _rel(got, want) < tol and _rel(composed, want) < tol
+
+
+def _composed(layer, x, shape):
+    """The layer run module by module: a forward hook on a child keeps the one-call path away."""
+    handle = layer.mlp.register_forward_hook(lambda *a: None)
+    try:
+        return layer(x, shape)
+    finally:
+        handle.remove()
+
+
+# channels, groups, post-norm, depthwise kernel, layer scale, (N, H, W), fp32 residual stream; 64- and 128-wide weight-gradient
+# tiles with one split and several, rows that are no whole slice
+TRAINING = [(64, 4, False, None, None, (3, 9, 7), False), (64, 4, False, 3, None, (2, 14, 11), True),
+            (112, 7, True, 3, 0.3, (2, 17, 13), True), (160, 10, True, 5, None, (5, 7, 7), True),
+            (112, 7, True, 3, 0.3, (13, 52, 50), True), (64, 4, False, None, None, (12, 28, 28), False)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("drop_path", [0.0, 0.4], ids=["no-drop", "drop-path"])
+@pytest.mark.parametrize("channels,groups,post_norm,dw,scale,size,stream32", TRAINING, ids=[f"{c[0]}-{c[5][0]}x{c[5][1]}" for c in TRAINING])
+def test_layer_training_under_autocast_matches_the_composition(channels, groups, post_norm, dw, scale, size, stream32, drop_path, dtype):
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    torch.manual_seed(channels + size[1])
+    layer = InternImageLayer(channels, groups, post_norm=post_norm, layer_scale=scale, dw_kernel_size=dw, drop_path=drop_path,
+                             dcn_output_bias=True, mlp_fc2_bias=True).cuda()
+    with torch.no_grad():
+        layer.dcn.offset_mask.weight.normal_(0, 0.02)
+        layer.dcn.offset_mask.bias.normal_(0, 0.5)
+        for name in ("gamma1", "gamma2"):
+            if scale is not None:
+                getattr(layer, name).uniform_(0.1, 0.5)
+    n, h, w = size
+    x = torch.randn(n, h * w, channels, device="cuda").to(torch.float32 if stream32 else dtype)
+    grad = torch.randn_like(x)
+    results = []
+    for run in (layer, lambda *a: _composed(layer, *a)):
+        torch.manual_seed(7)
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=dtype):
+            out = run(xi, (h, w))
+        grads = torch.autograd.grad(out, [xi, *layer.parameters()], grad)
+        results.append([out.detach(), *grads])
+    assert type(results[0]) is list and results[0][0].dtype == results[1][0].dtype
+    tol = 3e-3 if dtype == torch.float16 else 2e-2
+    names = ["output", "x"] + [k for k, _ in layer.named_parameters()]
+    for name, got, want in zip(names, *results):
+        assert got.dtype == want.dtype and got.shape == want.shape, name
+        assert _rel(got, want) < tol, (name, _rel(got, want))
+
+
+def test_layer_training_takes_one_node_and_reports_a_second_backward():
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    layer = InternImageLayer(64, 4).cuda()
+    x = torch.randn(1, 64, 64, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = layer(x, (8, 8))
+    assert out.grad_fn.name() == "InternImageLayerBackward"
+    first = torch.autograd.grad(out.sum(), x, retain_graph=True)[0]
+    assert torch.equal(first, torch.autograd.grad(out.sum(), x)[0])
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out.sum(), x)
