@@ -24,7 +24,7 @@ HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "mfma.hpp"), os.
            os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]
 
 BINDING = os.path.join(CSRC, "binding")
-BINDING_SOURCES = ["module.cpp", "operators.cpp", "modules.cpp", "layers.cpp", "training.cpp"]
+BINDING_SOURCES = ["module.cpp", "operators.cpp", "modules.cpp", "layers.cpp", "training.cpp", "attention.cpp"]
 BINDING_HEADERS = [os.path.join(BINDING, "binding.hpp"), os.path.join(BINDING, "modules.hpp"), os.path.join(BINDING, "layers.hpp"),
                    os.path.join(CSRC, "linear.hpp"), os.path.join(CSRC, "layer_norm.hpp"),
                    os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]

@@ -1,0 +1,311 @@
+// The FlashDeformAttn module (dcnv4_amd/modules/flash_deform_attn.py) as one autograd node: fp32 without autocast, or 16-bit
+// products under it with fp32 parameters.
+//
+// Composed of its operators a decoder layer of 300 queries took 0.92-1.04 ms forward and backward, 59 launches whose
+// kernels run 0.56 ms; an encoder layer over two 100x152 pyramids in fp32 1.90 ms, of which 520 us were four weight gradients
+// on 77 workgroups, 103 us bias sums and 210 us elementwise passes around the sampling locations and the padding.  Here the
+// offsets' product writes locations, the value product clears padded rows, the operator takes its rows un-packed, and the
+// parameter gradients are one product (two when queries and features differ in number).
+#include <ATen/autocast_mode.h>
+#include <torch/csrc/autograd/functions/utils.h>
+
+#include "layers.hpp"
+
+namespace dcn::binding {
+namespace {
+
+enum Input { kQuery, kFeatures, kValueW, kValueB, kOffsetsW, kOffsetsB, kLogitsW, kLogitsB, kOutputW, kOutputB, kInputs };
+
+struct AttentionSaved {
+  Arena arena;
+  size_t query, features, value, locations, logits, sampled;      // query, features: their 16-bit copies under autocast
+  size_t value_wt, offsets_wt, logits_wt, output_wt;
+};
+
+struct Attention {
+  Tensor params[kInputs];           // parameters by their Input
+  int code;                         // of the products: fp32, or the autocast type
+  int heads, levels, points, batch;
+  int64_t width, pixels, queries;
+  bool query32, features32;         // inputs in fp32 (always, without autocast)
+
+  int bytes() const { return code == DCNV4_DTYPE_F32 ? 4 : 2; }
+  int64_t query_rows() const { return batch * queries; }
+  int64_t feature_rows() const { return batch * pixels; }
+  int64_t logits() const { return (int64_t)heads * levels * points; }
+  // locations are rounded through fp16 by the operator: fp16 tensors hold them as they are used
+  int location_code() const { return code == DCNV4_DTYPE_F16 ? DCNV4_DTYPE_F16 : DCNV4_DTYPE_F32; }
+  int location_bytes() const { return code == DCNV4_DTYPE_F16 ? 2 : 4; }
+
+  SamplingLocations sampling(const Tensor &reference, const Tensor &shapes) const {
+    return {static_cast<const float *>(reference.const_data_ptr()), shapes.const_data_ptr<int64_t>(), (int)reference.size(-1), levels, points};
+  }
+  LinearLaunch product(const void *a, const void *w, const void *bias, int64_t rows, int64_t k, int64_t n, void *out) const {
+    LinearLaunch p = {};
+    p.p[0].a = a; p.p[0].w = w; p.p[0].bias = bias; p.p[0].out = out; p.p[0].n = (int)n;
+    p.count = 1; p.rows = rows; p.k = (int)k;
+    return p;
+  }
+  Tensor forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
+                 const Tensor &padding, AttentionSaved *s) const;
+  variable_list backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
+                         const Tensor &padding, const Tensor &grad, const AttentionSaved &s, bool want_query, bool want_features) const;
+};
+
+Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
+                          const Tensor &starts, const Tensor &padding, AttentionSaved *s) const {
+  OnDevice guard(query);
+  void *stream = stream_of(query);
+  const bool half = code != DCNV4_DTYPE_F32;
+  const int64_t n_loc = 2 * logits(), n_log = logits();
+  Arena &a = s->arena;
+  s->query = half && query32 ? a.take((size_t)(query_rows() * width) * 2) : 0;
+  s->features = half && features32 ? a.take((size_t)(feature_rows() * width) * 2) : 0;
+  s->value = a.take((size_t)(feature_rows() * width) * bytes());
+  s->locations = a.take((size_t)(query_rows() * n_loc) * location_bytes());
+  s->logits = a.take((size_t)(query_rows() * n_log) * bytes());
+  s->sampled = a.take((size_t)(query_rows() * width) * bytes());
+
+  // parameters in the products' type, and their matrices turned for the backward
+  CastWeightsLaunch cast = {};
+  size_t as_is[kInputs], turned[kInputs];
+  auto narrowed = [&](Input i, int64_t n, int64_t k) {
+    as_is[i] = half ? a.take((size_t)(n * k) * 2) : 0;
+    turned[i] = n > 1 ? a.take((size_t)(n * k) * bytes()) : 0;
+  };
+  narrowed(kValueW, width, width);
+  narrowed(kOffsetsW, n_loc, width);
+  narrowed(kLogitsW, n_log, width);
+  narrowed(kOutputW, width, width);
+  for (Input i : {kValueB, kOffsetsB, kLogitsB, kOutputB})
+    if (params[i].defined()) narrowed(i, 1, params[i].numel());
+  a.allocate(query);
+  s->value_wt = turned[kValueW]; s->offsets_wt = turned[kOffsetsW]; s->logits_wt = turned[kLogitsW]; s->output_wt = turned[kOutputW];
+  for (int i = kValueW; i < kInputs; ++i) {
+    const Tensor &t = params[i];
+    const bool matrix = t.defined() && t.dim() == 2;
+    if (!t.defined() || (!half && !matrix)) continue;
+    CastWeights &q = cast.p[cast.count++];
+    q.from = static_cast<const float *>(t.const_data_ptr());
+    q.to = half ? a.at(as_is[i]) : nullptr;
+    q.turned = matrix ? a.at(turned[i]) : nullptr;
+    q.n = matrix ? (int)t.size(0) : 1;
+    q.k = matrix ? (int)t.size(1) : (int)t.numel();
+  }
+  hip_check(launch_cast_weights(code, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
+  auto param = [&](Input i) -> const void * { return !params[i].defined() ? nullptr : half ? a.at(as_is[i]) : params[i].const_data_ptr(); };
+  auto input = [&](const Tensor &t, bool is32, size_t at, int64_t rows) -> const void * {
+    if (!half || !is32) return t.const_data_ptr();
+    hip_check(launch_narrow_rows(code, t.const_data_ptr(), true, a.at(at), (size_t)(rows * width), nullptr, 0, static_cast<hipStream_t>(stream)),
+              "conversion launch");
+    return a.at(at);
+  };
+
+  LinearLaunch value = product(input(features, features32, s->features, feature_rows()), param(kValueW), param(kValueB), feature_rows(),
+                               width, width, a.at(s->value));
+  value.p[0].zero_rows = static_cast<const uint8_t *>(ptr(padding));
+  launch(code, value, stream);
+  LinearLaunch rows = product(input(query, query32, s->query, query_rows()), param(kOffsetsW), param(kOffsetsB), query_rows(), width, n_loc,
+                              a.at(s->locations));
+  if (half && location_code() == DCNV4_DTYPE_F32) rows.p[0].out32 = static_cast<float *>(a.at(s->locations));
+  rows.p[1].a = rows.p[0].a; rows.p[1].w = param(kLogitsW); rows.p[1].bias = param(kLogitsB);
+  rows.p[1].out = a.at(s->logits); rows.p[1].n = (int)n_log;
+  rows.count = 2;
+  rows.locations = sampling(reference, shapes);
+  launch(code, rows, stream);
+  check(flash_deform_attn_gfx950_forward_split(a.at(s->value), shapes.const_data_ptr<int64_t>(), starts.const_data_ptr<int64_t>(),
+                                               a.at(s->locations), a.at(s->logits), a.at(s->sampled), code, location_code(), batch,
+                                               (int)pixels, heads, (int)width / heads, levels, (int)queries, points, 64, 0, 0, stream));
+  Tensor out = at::empty({batch, queries, width}, query.options().dtype(code == DCNV4_DTYPE_F32   ? at::kFloat
+                                                                        : code == DCNV4_DTYPE_F16 ? at::kHalf
+                                                                                                  : at::kBFloat16));
+  launch(code, product(a.at(s->sampled), param(kOutputW), param(kOutputB), query_rows(), width, width, out.data_ptr()), stream);
+  return out;
+}
+
+variable_list Attention::backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
+                                  const Tensor &starts, const Tensor &padding, const Tensor &grad, const AttentionSaved &s,
+                                  bool want_query, bool want_features) const {
+  OnDevice guard(query);
+  void *stream = stream_of(query);
+  hipStream_t hip = static_cast<hipStream_t>(stream);
+  const bool half = code != DCNV4_DTYPE_F32;
+  const int64_t n_loc = 2 * logits(), n_log = logits();
+  const Arena &a = s.arena;
+  variable_list g(kInputs);
+
+  Arena t;
+  const size_t d_sampled = t.take((size_t)(query_rows() * width) * bytes()), d_value = t.take((size_t)(feature_rows() * width) * bytes()),
+               d_locations = t.take((size_t)(query_rows() * n_loc) * location_bytes()), d_logits = t.take((size_t)(query_rows() * n_log) * bytes()),
+               d_offsets = t.take((size_t)(query_rows() * n_loc) * bytes());
+  const size_t ws_bytes = flash_deform_attn_gfx950_backward_workspace_bytes(code, batch, (int)pixels, heads, (int)width / heads, levels,
+                                                                            (int)queries, points);
+  const size_t ws = t.take(ws_bytes);
+  t.allocate(query);
+
+  launch(code, product(grad.const_data_ptr(), a.at(s.output_wt), nullptr, query_rows(), width, width, t.at(d_sampled)), stream);
+  check(flash_deform_attn_gfx950_backward_split(a.at(s.value), shapes.const_data_ptr<int64_t>(), starts.const_data_ptr<int64_t>(),
+                                                a.at(s.locations), a.at(s.logits), t.at(d_sampled), t.at(d_value), t.at(d_locations),
+                                                t.at(d_logits), t.at(ws), ws_bytes, code, location_code(), batch, (int)pixels, heads,
+                                                (int)width / heads, levels, (int)queries, points, 64, 0, 0, stream));
+  if (padding.defined())
+    hip_check(launch_zero_rows(bytes(), t.at(d_value), static_cast<const uint8_t *>(padding.const_data_ptr()), feature_rows(), (int)width, hip),
+              "padding launch");
+  hip_check(launch_location_grad(code, sampling(reference, shapes), t.at(d_locations), location_code() == DCNV4_DTYPE_F32, t.at(d_offsets),
+                                 query_rows(), (int)n_loc, hip),
+            "location gradient launch");
+  // results in the type of the input: fp32 beside 16-bit products
+  auto result = [&](LinearLaunch p, const Tensor &out, bool is32, bool add) {
+    LinearProblem &q = p.p[0];
+    if (half && is32) {
+      q.out32 = static_cast<float *>(out.data_ptr());
+      if (add) q.residual32 = q.out32;
+    } else {
+      q.out = out.data_ptr();
+      if (add) q.residual = q.out;
+    }
+    launch(code, p, stream);
+  };
+  if (want_features) {
+    g[kFeatures] = at::empty(features.sizes(), features.options());
+    result(product(t.at(d_value), a.at(s.value_wt), nullptr, feature_rows(), width, width, nullptr), g[kFeatures], features32, false);
+  }
+  if (want_query) {
+    g[kQuery] = at::empty(query.sizes(), query.options());
+    result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc, width, nullptr), g[kQuery], query32, false);
+    result(product(t.at(d_logits), a.at(s.logits_wt), nullptr, query_rows(), n_log, width, nullptr), g[kQuery], query32, true);
+  }
+  const void *q_in = half && query32 ? a.at(s.query) : query.const_data_ptr();
+  const void *f_in = half && features32 ? a.at(s.features) : features.const_data_ptr();
+  const auto fp32 = params[kValueW].options();
+  const WeightGradient value = {t.at(d_value), f_in, width, width, &params[kValueW], &params[kValueB], &g[kValueW], &g[kValueB]},
+                       offsets = {t.at(d_offsets), q_in, n_loc, width, &params[kOffsetsW], &params[kOffsetsB], &g[kOffsetsW], &g[kOffsetsB]},
+                       logit = {t.at(d_logits), q_in, n_log, width, &params[kLogitsW], &params[kLogitsB], &g[kLogitsW], &g[kLogitsB]},
+                       output = {grad.const_data_ptr(), a.at(s.sampled), width, width, &params[kOutputW], &params[kOutputB], &g[kOutputW],
+                                 &g[kOutputB]};
+  if (query_rows() == feature_rows()) {
+    weight_gradients(code, query_rows(), fp32, {output, offsets, value, logit}, stream);
+  } else {
+    weight_gradients(code, query_rows(), fp32, {output, offsets, logit}, stream);
+    weight_gradients(code, feature_rows(), fp32, {value}, stream);
+  }
+  return g;
+}
+
+struct FlashDeformAttnBackward final : torch::autograd::Node {
+  Attention layer;
+  AttentionSaved saved;
+  SavedVariable inputs[6];          // query, reference, features, shapes, starts, padding
+  std::string name() const override { return "FlashDeformAttnBackward"; }
+  void release_variables() override {
+    for (SavedVariable &v : inputs) v.reset_data();
+    saved.arena.release();
+    released_ = true;
+  }
+  variable_list apply(variable_list &&grads) override {
+    if (!grads[0].defined()) return variable_list(kInputs);
+    TORCH_CHECK(!released_, "Trying to backward through the graph a second time (or directly access saved tensors after they have already "
+                            "been freed). Specify retain_graph=True if you need to backward through the graph a second time.");
+    variable_list out;
+    {
+      at::AutoGradMode no_grad(false);
+      Tensor v[6];
+      for (int i = 0; i < 6; ++i) v[i] = inputs[i].unpack();
+      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], grads[0].contiguous(), saved, task_should_compute_output(kQuery),
+                           task_should_compute_output(kFeatures));
+    }
+    return once_differentiable(std::move(out));
+  }
+
+ private:
+  bool released_ = false;
+};
+
+bool dense(const Tensor &t, const Tensor &like, at::ScalarType dtype) {
+  return t.device() == like.device() && t.scalar_type() == dtype && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
+}
+
+bool load(const Module &m, Attention *a, Input weight, int64_t in, int64_t out, const Tensor &like) {
+  if (!m) return false;
+  a->params[weight] = m.parameter("weight");
+  a->params[weight + 1] = m.parameter("bias");
+  return usable(a->params[weight], like, at::kFloat, in * out, false) && usable(a->params[weight + 1], like, at::kFloat, out, true);
+}
+
+// attention_layer(module, query, reference_points, input_flatten, spatial_shapes, level_start_index, padding or None): the
+// module's output, or None where the composition of its operators has to run.
+PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args arg("attention_layer", args + 1, n - 1, 6);
+  const Tensor &query = arg.tensor(), &reference = arg.tensor(), &features = arg.tensor(), &shapes = arg.tensor(), &starts = arg.tensor();
+  const Tensor padding = arg.optional_tensor();
+  const Module m(args[0]);
+  if (!query.is_cuda() || global_module_hooks()) Py_RETURN_NONE;
+  Attention a;
+  at::ScalarType type = at::kFloat;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) {
+    type = at::autocast::get_autocast_dtype(at::kCUDA);
+    if (type != at::kHalf && type != at::kBFloat16) Py_RETURN_NONE;
+  }
+  auto accepts = [&](const Tensor &t) { return dense(t, query, at::kFloat) || (type != at::kFloat && dense(t, query, type)); };
+  if (query.dim() != 3 || features.dim() != 3 || query.numel() == 0 || features.numel() == 0 || !accepts(query) || !accepts(features)) Py_RETURN_NONE;
+  a.code = type == at::kFloat ? DCNV4_DTYPE_F32 : type == at::kHalf ? DCNV4_DTYPE_F16 : DCNV4_DTYPE_BF16;
+  a.query32 = query.scalar_type() == at::kFloat;
+  a.features32 = features.scalar_type() == at::kFloat;
+  a.heads = (int)m.integer("n_heads", 0);
+  a.levels = (int)m.integer("n_levels", 0);
+  a.points = (int)m.integer("n_points", 0);
+  a.width = query.size(2);
+  a.batch = (int)query.size(0);
+  a.queries = query.size(1);
+  a.pixels = features.size(1);
+  if (a.heads <= 0 || a.levels <= 0 || a.points <= 0 || a.points % 4 != 0 || a.width % 8 != 0 || a.logits() % 8 != 0 ||
+      a.width % a.heads != 0 || features.size(2) != a.width || features.size(0) != a.batch || m.integer("d_model", 0) != a.width)
+    Py_RETURN_NONE;
+  if (!dense(reference, query, at::kFloat) || reference.requires_grad() || reference.dim() != 4 || reference.size(0) != a.batch ||
+      reference.size(1) != a.queries || reference.size(2) != a.levels || (reference.size(3) != 2 && reference.size(3) != 4))
+    Py_RETURN_NONE;
+  if (!dense(shapes, query, at::kLong) || !dense(starts, query, at::kLong) || shapes.numel() != 2 * a.levels || starts.numel() != a.levels)
+    Py_RETURN_NONE;
+  if (padding.defined() && (padding.device() != query.device() || padding.scalar_type() != at::kBool || !padding.is_contiguous() ||
+                            padding.numel() != a.feature_rows()))
+    Py_RETURN_NONE;
+  if (!load(m.child("value_proj", kLinear), &a, kValueW, a.width, a.width, query) ||
+      !load(m.child("sampling_offsets", kLinear), &a, kOffsetsW, a.width, 2 * a.logits(), query) ||
+      !load(m.child("attention_weights", kLinear), &a, kLogitsW, a.width, a.logits(), query) ||
+      !load(m.child("output_proj", kLinear), &a, kOutputW, a.width, a.width, query))
+    Py_RETURN_NONE;
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    variable_list inputs = {query, features};
+    for (int i = kValueW; i < kInputs; ++i) inputs.push_back(a.params[i]);
+    bool wanted = false;
+    if (at::GradMode::is_enabled())
+      for (const Tensor &i : inputs) wanted |= i.defined() && i.requires_grad();
+    AttentionSaved saved;
+    {
+      at::AutoGradMode no_grad(false);
+      out = a.forward(query, reference, features, shapes, starts, padding, &saved);
+    }
+    if (wanted) {
+      std::shared_ptr<FlashDeformAttnBackward> node(new FlashDeformAttnBackward(), torch::autograd::deleteNode);
+      node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+      node->layer = a;
+      node->saved = std::move(saved);
+      int i = 0;
+      for (const Tensor *t : {&query, &reference, &features, &shapes, &starts, &padding}) node->inputs[i++] = SavedVariable(*t, false);
+      record(node, out);
+    }
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+}  // namespace
+
+PyMethodDef attention_methods[] = {
+    {"attention_layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_attention_layer)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+}  // namespace dcn::binding

@@ -97,6 +97,52 @@ void launch(int code, const LinearLaunch &l, void *stream) {
   if (e != hipSuccess) raise_runtime("linear layer launch: %s", hipGetErrorString(e));
 }
 
+void hip_check(hipError_t e, const char *what) {
+  if (e != hipSuccess) raise_runtime("%s: %s", what, hipGetErrorString(e));
+}
+
+void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream) {
+  WeightGradLaunch launch = {};
+  launch.rows = rows;
+  for (const WeightGradient &l : layers) {
+    *l.grad_w = at::empty(l.weight->sizes(), fp32);
+    if (l.bias->defined()) *l.grad_b = at::empty(l.bias->sizes(), fp32);
+    WeightGradProblem &q = launch.p[launch.count++];
+    q.grad_out = l.grad_out; q.in = l.in; q.n = (int)l.n; q.k = (int)l.k;
+  }
+  const WeightGradPlan plan = plan_weight_grad(code, launch);
+  launch.splits = plan.splits;
+  // one split writes the gradients themselves, several their partial sums
+  WeightGradReduce reduce = {};
+  reduce.splits = plan.splits;
+  size_t floats = 0;
+  auto place = [&](const Tensor &grad) {
+    reduce.s[reduce.count++] = {static_cast<float *>(grad.data_ptr()), floats, (int)grad.numel()};
+    floats += (size_t)(grad.numel() + 3) / 4 * 4;
+  };
+  for (const WeightGradient &l : layers) {
+    place(*l.grad_w);
+    if (l.bias->defined()) place(*l.grad_b);
+  }
+  Tensor partial;
+  if (plan.splits > 1) partial = at::empty({(int64_t)(floats * plan.splits)}, fp32);
+  float *base = plan.splits > 1 ? static_cast<float *>(partial.data_ptr()) : nullptr;
+  reduce.partial = base;
+  reduce.split_stride = launch.split_stride = floats;
+  int segment = 0, i = 0;
+  auto target = [&] {
+    const WeightGradSegment &s = reduce.s[segment++];
+    return base != nullptr ? base + s.offset : s.grad;
+  };
+  for (const WeightGradient &l : layers) {
+    launch.p[i].grad_w = target();
+    if (l.bias->defined()) launch.p[i].grad_bias = target();
+    ++i;
+  }
+  hip_check(launch_weight_grad(code, launch, plan.tile, static_cast<hipStream_t>(stream)), "weight gradient launch");
+  if (plan.splits > 1) hip_check(launch_weight_grad_reduce(reduce, static_cast<hipStream_t>(stream)), "weight gradient sum launch");
+}
+
 bool usable_input(const Tensor &x, int h, int w) {
   return x.is_cuda() && x.dim() == 3 && x.is_contiguous() && x.numel() != 0 && x.size(1) == (int64_t)h * w &&
          (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15) == 0;
@@ -178,7 +224,7 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (in.dim() < 1 || weight.dim() != 2 || weight.size(1) != in.size(-1)) raise_runtime("weight must be (N, K) for an input (..., K)");
   const int64_t k = weight.size(1), width = weight.size(0), rows = k ? in.numel() / k : 0;
   const int code = dtype_code(in, "input");
-  if (!linear_fits(code, rows, (int)width, (int)k)) raise_runtime("linear takes 16-bit tensors of a depth and width in multiples of 8");
+  if (!linear_fits(code, rows, (int)width, (int)k)) raise_runtime("linear takes a depth and width in multiples of 8");
   auto sizes = in.sizes().vec();
   sizes.back() = width;
   const auto dtype = in.scalar_type();

@@ -32,6 +32,35 @@ void launch(int code, const LinearLaunch &l, void *stream);
 // The arguments (layer, x, h, w) of a call that takes a layer.
 bool usable_input(const Tensor &x, int h, int w);
 
+void hip_check(hipError_t e, const char *what);
+
+// Sub-tensors of one allocation, each on a 256-byte boundary.
+class Arena {
+ public:
+  size_t take(size_t bytes) {
+    const size_t at = total_;
+    total_ += (bytes + 255) / 256 * 256;
+    return at;
+  }
+  void allocate(const Tensor &like) { storage_ = workspace(std::max<size_t>(total_, 256), like); }
+  void *at(size_t offset) const { return static_cast<char *>(storage_.data_ptr()) + offset; }
+  void release() { storage_ = Tensor(); }
+
+ private:
+  size_t total_ = 0;
+  Tensor storage_;
+};
+
+// A linear layer's parameter gradients: grad_out [rows, n], in [rows, k]; *grad_w and *grad_b are allocated in fp32.
+struct WeightGradient {
+  const void *grad_out, *in;
+  int64_t n, k;
+  const Tensor *weight, *bias;
+  Tensor *grad_w, *grad_b;
+};
+void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream);
+
 extern PyMethodDef training_methods[];
+extern PyMethodDef attention_methods[];
 
 }  // namespace dcn::binding

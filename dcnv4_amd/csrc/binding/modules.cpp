@@ -84,13 +84,21 @@ bool idle(const Module &m, ModuleKind kind) {
 
 namespace {
 
-// register_modules(*classes in the order of ModuleKind)
+constexpr const char *kKindNames[kModuleKinds] = {"Linear", "LayerNorm", "GELU", "Dropout", "Identity", "Conv2d", "Sequential", "DropPath",
+                                                   "DCNv4", "MLPLayer"};
+
+// register_modules(*classes): each fills the kind of its name
 PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != kModuleKinds) raise_runtime("register_modules takes %d classes, got %zd", (int)kModuleKinds, n);
-  for (int i = 0; i < kModuleKinds; ++i) {
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject *name = PyObject_GetAttrString(args[i], "__name__");
+    if (name == nullptr) throw python_error();
+    int kind = 0;
+    while (kind < kModuleKinds && PyUnicode_CompareWithASCIIString(name, kKindNames[kind]) != 0) ++kind;
+    Py_DECREF(name);
+    if (kind == kModuleKinds) raise_runtime("register_modules: no kind for argument %zd", i);
     Py_INCREF(args[i]);
-    Py_XSETREF(g_kinds[i], args[i]);
+    Py_XSETREF(g_kinds[kind], args[i]);
   }
   PyObject *m = PyImport_ImportModule("torch.nn.modules.module");
   if (m == nullptr) throw python_error();

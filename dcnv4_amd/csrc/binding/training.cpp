@@ -22,27 +22,6 @@ namespace {
 enum Input { kX, kNorm1W, kNorm1B, kGamma1, kNorm2W, kNorm2B, kGamma2, kValueW, kValueB, kOffsetW, kOffsetB, kOutputW, kOutputB, kDwW,
              kDwB, kFc1W, kFc1B, kFc2W, kFc2B, kInputs };
 
-void hip_check(hipError_t e, const char *what) {
-  if (e != hipSuccess) raise_runtime("%s: %s", what, hipGetErrorString(e));
-}
-
-// Sub-tensors of one allocation, each on a 256-byte boundary.
-class Arena {
- public:
-  size_t take(size_t bytes) {
-    const size_t at = total_;
-    total_ += (bytes + 255) / 256 * 256;
-    return at;
-  }
-  void allocate(const Tensor &like) { storage_ = workspace(std::max<size_t>(total_, 256), like); }
-  void *at(size_t offset) const { return static_cast<char *>(storage_.data_ptr()) + offset; }
-  void release() { storage_ = Tensor(); }
-
- private:
-  size_t total_ = 0;
-  Tensor storage_;
-};
-
 struct Saved {
   Arena arena;
   // offsets into the arena
@@ -293,50 +272,13 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   }
 
   // all weight and bias gradients
-  WeightGradLaunch wg = {};
-  struct Target { Input w, b; };
-  Target target[kMaxWeightGrads];
-  auto add = [&](const void *grad_out, const void *in, int64_t n, int64_t k, Input wi, const Tensor &wt, Input bi, const Tensor &bt) {
-    g[wi] = at::empty(wt.sizes(), f32);
-    if (bt.defined()) g[bi] = at::empty(bt.sizes(), f32);
-    target[wg.count] = {wi, bi};
-    WeightGradProblem &q = wg.p[wg.count++];
-    q.grad_out = grad_out; q.in = in; q.n = (int)n; q.k = (int)k;
-  };
-  add(last, a.at(s.hidden), c, l.hidden, kFc2W, l.fc2_w, kFc2B, l.fc2_b);
-  add(t.at(d_hidden), a.at(s.half_mid), l.hidden, c, kFc1W, l.fc1_w, kFc1B, l.fc1_b);
-  add(projected, a.at(s.sampled), c, c, kOutputW, l.output_w, kOutputB, l.output_b);
-  add(t.at(d_value), a.at(s.half_x), c, c, kValueW, l.value_w, kValueB, l.value_b);
-  add(t.at(d_offsets), a.at(s.pre), l.row, c, kOffsetW, l.offset_w, kOffsetB, l.offset_b);
-  wg.rows = rows;
-  const WeightGradPlan plan = plan_weight_grad(wg);
-  wg.splits = plan.splits;
-  WeightGradReduce reduce = {};
-  reduce.splits = plan.splits;
-  size_t floats = 0;
-  Tensor partial;
-  if (plan.splits > 1) {
-    for (int i = 0; i < wg.count; ++i) {
-      for (const bool weight : {true, false}) {
-        const Tensor &out = g[weight ? target[i].w : target[i].b];
-        if (!out.defined()) continue;
-        reduce.s[reduce.count++] = {static_cast<float *>(out.data_ptr()), floats, (int)out.numel()};
-        floats += (size_t)(out.numel() + 3) / 4 * 4;
-      }
-    }
-    partial = at::empty({(int64_t)(floats * plan.splits)}, f32);
-    reduce.partial = static_cast<const float *>(partial.data_ptr());
-    reduce.split_stride = wg.split_stride = floats;
-  }
-  int segment = 0;
-  for (int i = 0; i < wg.count; ++i) {
-    const Tensor &gw = g[target[i].w], &gb = g[target[i].b];
-    float *base = plan.splits > 1 ? static_cast<float *>(partial.data_ptr()) : nullptr;
-    wg.p[i].grad_w = base ? base + reduce.s[segment++].offset : static_cast<float *>(gw.data_ptr());
-    if (gb.defined()) wg.p[i].grad_bias = base ? base + reduce.s[segment++].offset : static_cast<float *>(gb.data_ptr());
-  }
-  hip_check(launch_weight_grad(c16, wg, plan.tile, static_cast<hipStream_t>(stream)), "weight gradient launch");
-  if (plan.splits > 1) hip_check(launch_weight_grad_reduce(reduce, static_cast<hipStream_t>(stream)), "weight gradient sum launch");
+  weight_gradients(c16, rows, f32,
+                   {{last, a.at(s.hidden), c, l.hidden, &l.fc2_w, &l.fc2_b, &g[kFc2W], &g[kFc2B]},
+                    {t.at(d_hidden), a.at(s.half_mid), l.hidden, c, &l.fc1_w, &l.fc1_b, &g[kFc1W], &g[kFc1B]},
+                    {projected, a.at(s.sampled), c, c, &l.output_w, &l.output_b, &g[kOutputW], &g[kOutputB]},
+                    {t.at(d_value), a.at(s.half_x), c, c, &l.value_w, &l.value_b, &g[kValueW], &g[kValueB]},
+                    {t.at(d_offsets), a.at(s.pre), l.row, c, &l.offset_w, &l.offset_b, &g[kOffsetW], &g[kOffsetB]}},
+                   stream);
   return g;
 }
 

@@ -1,8 +1,8 @@
-// Linear layers on the matrix cores for 16-bit tensors, with what follows the product fused into its epilogue: bias, GELU,
+// Linear layers on the matrix cores, with what follows the product fused into its epilogue: bias, GELU,
 // layer scale, residual.  Two kernels:
 //
-//  linear_tiled_kernel: many rows.  A workgroup of four waves owns BM rows x BN features; both operands come in slices of 64
-//    along the depth, 16 bytes a lane, straight into LDS (two buffers, one barrier a slice: the next slice's loads are in
+//  linear_tiled_kernel: many rows.  A workgroup of four waves owns BM rows x BN features; both operands come in slices of
+//    128 bytes along the depth, 16 bytes a lane, straight into LDS (two buffers, one barrier a slice: the next slice's loads are in
 //    flight while the matrix cores work on this one).  The 16-byte vectors of a row are stored at position
 //    vector ^ (row / 2 & 7), so the 16 rows that a fragment read touches fall into 16 different slots of 256 bytes and the
 //    read has no bank conflicts.  The features are the rows of the matrix instruction's result, so a lane ends up with
@@ -17,8 +17,8 @@ namespace dcn {
 namespace {
 
 constexpr int kCus = 256;                        // MI355X
-constexpr int kSlice = 64;                       // depth of a slice: 128 bytes of a row
-constexpr int kRowVectors = kSlice * 2 / 16;     // 16-byte vectors of a row's slice
+constexpr int kSliceBytes = 128;                 // of a row
+constexpr int kRowVectors = kSliceBytes / 16;
 
 // What a lane needs of a feature vector for its eight columns, read once.
 template <typename Tag>
@@ -26,27 +26,49 @@ struct Columns {
   float bias[8], gamma[8];
   bool has_bias, has_gamma;
   __device__ __forceinline__ Columns(const LinearProblem &q, int n, bool live) : has_bias(q.bias != nullptr), has_gamma(q.gamma != nullptr) {
-    if (has_bias && live) Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.bias) + n * 2), bias);
-    if (has_gamma && live) Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(q.gamma) + n * 2), gamma);
+    if (has_bias && live) load8<Tag>(q.bias, n, bias);
+    if (has_gamma && live) load8<Tag>(q.gamma, n, gamma);
   }
 };
 
-// The epilogue for eight consecutive features of one row: 16 bytes in and out.  EXTRA: with what training adds, which
-// costs the small tiles a third more registers.
+template <typename Tag>
+__device__ __forceinline__ void to_locations(const SamplingLocations &l, long long row, int n, float (&v)[8]) {
+  const int level = n / (2 * l.points) % l.levels;
+  const float *ref = l.reference + (row * l.levels + level) * l.kind;
+  round8<Tag>(v);
+  if (l.kind == 2) {
+    const float w = (float)l.shapes[2 * level + 1], h = (float)l.shapes[2 * level];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] /= (c & 1) ? h : w;
+    round8<Tag>(v);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = add_rn(ref[c & 1], v[c]);
+  } else {
+    const float points = (float)l.points;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] /= points;
+    round8<Tag>(v);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = add_rn(ref[c & 1], mul_rn(mul_rn(v[c], ref[2 + (c & 1)]), 0.5f));
+  }
+}
+
+// The epilogue for eight consecutive features of one row: 16 bytes in and out (32 of fp32).  EXTRA: with what training adds,
+// which costs the small tiles a third more registers.
 template <typename Tag, bool EXTRA>
-__device__ __forceinline__ void finish(const LinearProblem &q, const Columns<Tag> &col, int gelu, long long row, int n, float (&v)[8]) {
+__device__ __forceinline__ void finish(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8]) {
+  const LinearProblem &q = p.p[which];
   if (col.has_bias)
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] += col.bias[c];
-  const size_t element = (size_t)row * q.n + n, at = element * 2;
-  auto half_at = [&](const void *base, float (&f)[8]) { Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(base) + at), f); };
-  if (EXTRA && q.pre != nullptr) *reinterpret_cast<u32x4 *>(static_cast<char *>(q.pre) + at) = Pack<Tag, 8>::encode(v);
-  if (gelu)
+  const size_t at = (size_t)row * q.n + n;
+  if (EXTRA && q.pre != nullptr) store8<Tag>(q.pre, at, v);
+  if (p.gelu)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = gelu_exact(v[c]);
+    for (int c = 0; c < 8; ++c) v[c] = gelu_exact<Tag>(v[c]);
   if (EXTRA && q.gelu_grad_at != nullptr) {
     float x[8];
-    half_at(q.gelu_grad_at, x);
+    load8<Tag>(q.gelu_grad_at, at, x);
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] *= gelu_derivative(x[c]);
   }
@@ -60,28 +82,28 @@ __device__ __forceinline__ void finish(const LinearProblem &q, const Columns<Tag
   }
   if (q.residual != nullptr) {
     float r[8];
-    half_at(q.residual, r);
+    load8<Tag>(q.residual, at, r);
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] += r[c];
   }
   if (EXTRA && q.residual32 != nullptr) {
-    const f32x4 *r = reinterpret_cast<const f32x4 *>(q.residual32 + element);
-    const f32x4 lo = r[0], hi = r[1];
-    v[0] += lo.x; v[1] += lo.y; v[2] += lo.z; v[3] += lo.w;
-    v[4] += hi.x; v[5] += hi.y; v[6] += hi.z; v[7] += hi.w;
+    float r[8];
+    load8<F32>(q.residual32, at, r);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += r[c];
   }
-  if (EXTRA && q.out32 != nullptr) {
-    f32x4 *o = reinterpret_cast<f32x4 *>(q.out32 + element);
-    o[0] = f32x4{v[0], v[1], v[2], v[3]};
-    o[1] = f32x4{v[4], v[5], v[6], v[7]};
-  } else {
-    *reinterpret_cast<u32x4 *>(static_cast<char *>(q.out) + at) = Pack<Tag, 8>::encode(v);
-  }
+  if (EXTRA && which == 0 && p.locations.kind != 0) to_locations<Tag>(p.locations, row, n, v);
+  if (EXTRA && q.zero_rows != nullptr && q.zero_rows[row] != 0)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = 0.f;
+  if (EXTRA && q.out32 != nullptr) store8<F32>(q.out32, at, v);
+  else store8<Tag>(q.out, at, v);
 }
 
 template <typename Tag, int BM, int BN, int WM, int WN, bool EXTRA>
 __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
   static_assert(WM * WN == 4 && BM % (16 * WM) == 0 && BN % (32 * WN) == 0 && BM % 32 == 0, "tile shape");
+  constexpr int kBytes = Tag::kBytes, kSlice = kSliceBytes / kBytes;
   constexpr int MF = BM / WM / 16, NF = BN / WN / 16;
   __shared__ u32x4 lds[2][(BM + BN) * kRowVectors];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -94,8 +116,8 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
   const long long m0 = (long long)tm * BM;
   const int n0 = tn * BN, k = p.k;
   const int live_m = (int)min((long long)BM, p.rows - m0), live_n = min(BN, q.n - n0);
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * 2, (uint32_t)live_m * k * 2);
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * 2, (uint32_t)live_n * k * 2);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * kBytes, (uint32_t)live_m * k * kBytes);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * kBytes, (uint32_t)live_n * k * kBytes);
 
   // a wave's load covers eight rows of a tile: lane l takes row l / 8, position l & 7
   const int row8 = lane >> 3, pos = lane & 7;
@@ -104,8 +126,8 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
     for (int i = 0; i < (BM + BN) / 32; ++i) {
       const bool act = i < BM / 32;
       const int base = (i * 4 + wave) * 8, row = base + row8;             // rows of the row tile, then of the feature tile
-      const int kk = k0 + (pos ^ ((row >> 1) & 7)) * 8;
-      const uint32_t off = (uint32_t)((act ? row : row - BM) * k + kk) * 2;
+      const int kk = k0 + (pos ^ ((row >> 1) & 7)) * (16 / kBytes);
+      const uint32_t off = (uint32_t)((act ? row : row - BM) * k + kk) * kBytes;
       load_to_lds(act ? ra : rw, buf + base * kRowVectors, kk < k ? off : kDropOffset);
     }
   };
@@ -137,7 +159,7 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
 #pragma unroll
       for (int i = 0; i < NF; ++i)
 #pragma unroll
-        for (int j = 0; j < MF; ++j) acc[i][j] = mfma_16x16x32<Tag>(fn[s][i], fm[s][j], acc[i][j]);
+        for (int j = 0; j < MF; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[s][i], fm[s][j], acc[i][j]);
   }
   // Epilogue, sixteen rows of the wave at a time: the fragments are turned through the buffer that the last slice did not
   // use (the wave's own part of it, so no barrier), each lane then holds eight consecutive features of a row, and a row's
@@ -159,7 +181,7 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
       const int r = u * rows_per_pass + lane / lanes_per_row, row = wm * (BM / WM) + j * 16 + r;
       const f32x4 lo = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col), hi = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col + 4);
       float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      if (row < live_m && n < live_n) finish<Tag, EXTRA>(q, columns, p.gelu, m0 + row, n0 + n, v);
+      if (row < live_m && n < live_n) finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -169,6 +191,7 @@ constexpr int kFewTile = 32;
 
 template <typename Tag, bool EXTRA>
 __global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
+  constexpr int kBytes = Tag::kBytes;
   __shared__ __align__(16) float part[4][kFewTile][kFewTile + 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tm = blockIdx.x / tiles_n;
@@ -178,27 +201,28 @@ __global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch
   if (which) tn -= tiles_n0;
   const int m0 = tm * kFewTile, n0 = tn * kFewTile, k = p.k;
   const int live_m = (int)min((long long)kFewTile, p.rows - m0), live_n = min(kFewTile, q.n - n0);
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * 2, (uint32_t)live_m * k * 2);
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * 2, (uint32_t)live_n * k * 2);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * kBytes, (uint32_t)live_m * k * kBytes);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * kBytes, (uint32_t)live_n * k * kBytes);
   const int r16 = lane & 15, kb = lane >> 4;
-  const int steps = (k + 31) / 32;
+  constexpr int kStep = 64 / kBytes;
+  const int steps = (k + kStep - 1) / kStep;
 
   f32x4 acc[2][2] = {};
-  // wave w takes every fourth step of 32 along the depth
+  // wave w takes every fourth 64 bytes of the depth
 #pragma unroll 4
   for (int s = wave; s < steps; s += 4) {
-    const int kk = s * 32 + kb * 8;
+    const int kk = s * kStep + kb * (16 / kBytes);
     u32x4 fm[2], fn[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const uint32_t off = (uint32_t)((j * 16 + r16) * k + kk) * 2;
+      const uint32_t off = (uint32_t)((j * 16 + r16) * k + kk) * kBytes;
       fm[j] = buffer_load<16>(ra, kk < k ? off : kDropOffset);
       fn[j] = buffer_load<16>(rw, kk < k ? off : kDropOffset);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_16x16x32<Tag>(fn[i], fm[j], acc[i][j]);
+      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[i], fm[j], acc[i][j]);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -216,7 +240,7 @@ __global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch
     for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
     v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
   }
-  if (row < live_m && n < live_n) finish<Tag, EXTRA>(q, columns, p.gelu, m0 + row, n0 + n, v);
+  if (row < live_m && n < live_n) finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v);
 }
 
 template <typename Tag, bool EXTRA, int BM, int BN, int WM, int WN>
@@ -250,18 +274,23 @@ hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
     for (int i = 0; i < p.count; ++i) n += (p.p[i].n + bn - 1) / bn;
     return n * ((p.rows + bm - 1) / bm);
   };
+  // fp32 is bound by the matrix cores (157 TFLOP/s): the tile that spreads most evenly
   if (tiles(64, 64) < 64) return launch_few<Tag, EXTRA>(p, stream);
-  if (tiles(128, 64) < kCus) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
-  const long long wide = tiles(128, 128), narrow = tiles(128, 64);
-  if (wide < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
-  if (20 * wide <= 11 * narrow) return launch_tiled<Tag, EXTRA, 128, 128, 2, 2>(p, stream);
-  return launch_tiled<Tag, EXTRA, 256, 64, 4, 1>(p, stream);
+  if constexpr (Tag::kBytes == 4) {
+    return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
+  } else {
+    if (tiles(128, 64) < kCus) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
+    const long long wide = tiles(128, 128), narrow = tiles(128, 64);
+    if (wide < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
+    if (20 * wide <= 11 * narrow) return launch_tiled<Tag, EXTRA, 128, 128, 2, 2>(p, stream);
+    return launch_tiled<Tag, EXTRA, 256, 64, 4, 1>(p, stream);
+  }
 }
 
 }  // namespace
 
 bool linear_fits(int dtype, long long rows, int n, int k) {
-  return (dtype == F16::kCode || dtype == BF16::kCode) && rows > 0 && n > 0 && k > 0 && n % 8 == 0 && k % 8 == 0 && k <= (1 << 20) &&
+  return (dtype == F32::kCode || dtype == F16::kCode || dtype == BF16::kCode) && rows > 0 && n > 0 && k > 0 && n % 8 == 0 && k % 8 == 0 && k <= (1 << 20) &&
          rows * (long long)n < (1ll << 42) && (rows + 63) / 64 * ((n + 63) / 64) < (1ll << 30);
 }
 
@@ -269,8 +298,11 @@ hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream) {
   bool extra = false;
   for (int i = 0; i < p.count; ++i) {
     const LinearProblem &q = p.p[i];
-    extra |= q.pre != nullptr || q.gelu_grad_at != nullptr || q.residual32 != nullptr || q.out32 != nullptr || q.row_scale != nullptr;
+    extra |= q.pre != nullptr || q.gelu_grad_at != nullptr || q.residual32 != nullptr || q.out32 != nullptr || q.row_scale != nullptr ||
+             q.zero_rows != nullptr;
   }
+  extra |= p.locations.kind != 0;
+  if (dtype == F32::kCode) return extra ? launch_t<F32, true>(p, stream) : launch_t<F32, false>(p, stream);
   if (dtype == F16::kCode) return extra ? launch_t<F16, true>(p, stream) : launch_t<F16, false>(p, stream);
   return extra ? launch_t<BF16, true>(p, stream) : launch_t<BF16, false>(p, stream);
 }

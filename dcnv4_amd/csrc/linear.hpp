@@ -19,6 +19,16 @@ struct LinearProblem {
   float *out32;                // the result in fp32, in place of out
   const float *row_scale;      // per sample of scale_rows rows: factor in front of the residuals
   int scale_rows;
+  const uint8_t *zero_rows;    // per row: non-zero where the result is zero (padding)
+};
+
+// Sampling locations of deformable attention in place of the offsets that the first product gives, features ordered
+// [head][level][point][x, y]: reference + offset / (width, height) of the level for reference points (kind 2), reference +
+// offset / points * size / 2 for boxes (kind 4); every step rounded as the framework's operators round it.
+struct SamplingLocations {
+  const float *reference;      // [rows][levels][kind]
+  const int64_t *shapes;       // [levels][height, width]
+  int kind, levels, points;    // kind 0: no locations; points a multiple of 4
 };
 
 // Up to two products over the same rows and depth in one launch (a layer's value and offset projections).
@@ -28,9 +38,10 @@ struct LinearLaunch {
   long long rows;
   int k;
   int gelu;              // act: the exact GELU, else none
+  SamplingLocations locations;
 };
 
-// Whether the matrix kernels take a product: 16-bit tensors, depth and width in whole 16-byte vectors.
+// Whether the matrix kernels take a product: depth and width in multiples of 8.
 bool linear_fits(int dtype, long long rows, int n, int k);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
 
@@ -50,7 +61,7 @@ struct WeightGradLaunch {
   size_t split_stride;
 };
 struct WeightGradPlan { int tile, splits; };
-WeightGradPlan plan_weight_grad(const WeightGradLaunch &p);
+WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p);
 hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &p, int tile, hipStream_t stream);
 
 struct WeightGradSegment {
@@ -66,7 +77,7 @@ struct WeightGradReduce {
 };
 hipError_t launch_weight_grad_reduce(const WeightGradReduce &p, hipStream_t stream);
 
-// 16-bit copies of fp32 matrices [n, k], and turned ones [k, n] (may be null).
+// Copies of fp32 matrices [n, k] in the dtype, as they lie and turned [k, n] (either may be null).
 constexpr int kMaxCasts = 16;
 struct CastWeights {
   const float *from;
@@ -80,6 +91,11 @@ struct CastWeightsLaunch {
 };
 hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &p, hipStream_t stream);
 // dst = 16-bit src (fp32, or 16-bit with a factor per sample of scale_elements elements); n and scale_elements multiples of 8
+// grad_offsets (dtype) from the gradients of the locations (fp32, or the dtype): the backward of SamplingLocations.
+hipError_t launch_location_grad(int dtype, const SamplingLocations &l, const void *grad_locations, bool locations32, void *grad_offsets,
+                                long long rows, int n, hipStream_t stream);
+// Clears the rows of n elements whose byte is not zero.
+hipError_t launch_zero_rows(int elem_bytes, void *rows_of, const uint8_t *zero, long long rows, int n, hipStream_t stream);
 hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
                               hipStream_t stream);
 

@@ -2,7 +2,7 @@
 //
 // linear_weight_grad_kernel: grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k], for all the linear layers of a
 // block in one launch.  The reduction runs over the slow axis of both operands, so a fragment's eight values lie a row
-// apart: slices of 64 rows come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns them
+// apart: slices of 64 rows (32 in fp32) come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns them
 // on the way into registers (16 lanes read 4 rows x 16 columns; lane i gets column i).  A row's 32-byte units are stored at
 // unit ^ f(row), f taking each value once over the eight rows that half a wave reads, so those reads fall into different
 // banks.  The rows are split over workgroups until the chip is full, partial sums are fp32 and are added in split order by
@@ -10,13 +10,15 @@
 // fragment, against a vector of ones.
 //   12544 rows, five layers of 448 channels (59 GFLOP): the library's one product at a time left 49 workgroups for each
 //   (82 us, five of them, 412 us) and its column sums took 65 us more.
+#include <type_traits>
+
 #include "linear.hpp"
 #include "mfma.hpp"
 
 namespace dcn {
 namespace {
 
-constexpr int kRows = 64;      // rows of a slice
+template <typename Tag> constexpr int kRowsOf = 128 / Tag::kBytes;      // rows of a slice
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -24,15 +26,18 @@ __device__ __forceinline__ u32x2 read_turned(const char *lds) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)lds));
 }
 
-template <int WIDTH>
-__device__ __forceinline__ int unit_swizzle(int row) {      // 32-byte units of a row of WIDTH 16-bit elements
-  return WIDTH == 128 ? (row & 3) | ((row >> 1) & 4) : ((row >> 1) & 1) | ((row >> 2) & 2);
+// Sixteen columns of a row - 32 bytes, or 64 of fp32 - are a unit, stored at unit ^ swizzle(row).
+template <typename Tag, int WIDTH>
+__device__ __forceinline__ int unit_swizzle(int row) {
+  if constexpr (Tag::kBytes == 4) return row & 3;
+  else return WIDTH == 128 ? (row & 3) | ((row >> 1) & 4) : ((row >> 1) & 1) | ((row >> 2) & 2);
 }
 
 template <typename Tag, int W>
 __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGradLaunch p) {
   static_assert(W == 64 || W == 128, "tile side");
-  constexpr int kRowBytes = W * 2, F = W / 2 / 16;              // a wave takes W/2 x W/2
+  constexpr int kBytes = Tag::kBytes, kRows = kRowsOf<Tag>, kRowBytes = W * kBytes, kUnit = 16 * kBytes;
+  constexpr int F = W / 2 / 16;                                 // a wave takes W/2 x W/2
   constexpr int kRowsPerLoad = 64 * 16 / kRowBytes, kLoads = kRows / kRowsPerLoad / 4;
   __shared__ __align__(16) char lds[2][2][kRows * kRowBytes];   // [buffer][grad_out, in]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -45,36 +50,54 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   const long long row_begin = (long long)split * p.rows_per_split;
   const long long row_end = min(row_begin + p.rows_per_split, p.rows);
 
-  // a wave's load covers kRowsPerLoad rows; a lane's 16 bytes go to position lane, which holds unit (u ^ f) of the row
+  // a wave's load covers kRowsPerLoad rows; a lane's 16 bytes go to position lane, which holds a unit's piece of the row
   const int load_row = lane * 16 / kRowBytes, load_chunk = lane % (kRowBytes / 16);
   auto stage = [&](long long row0, char (&buf)[2][kRows * kRowBytes]) {
     const int live = (int)max(0ll, min((long long)kRows, row_end - row0));
-    const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.n * 2, (uint32_t)live * q.n * 2);
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char *>(q.in) + (size_t)row0 * q.k * 2, (uint32_t)live * q.k * 2);
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.n * kBytes, (uint32_t)live * q.n * kBytes);
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char *>(q.in) + (size_t)row0 * q.k * kBytes, (uint32_t)live * q.k * kBytes);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int base = (i * 4 + wave) * kRowsPerLoad, row = base + load_row;
-      const int col = (((load_chunk >> 1) ^ unit_swizzle<W>(row)) * 2 + (load_chunk & 1)) * 8;
+      const int col = ((load_chunk * 16 / kUnit) ^ unit_swizzle<Tag, W>(row)) * 16 + load_chunk * 16 % kUnit / kBytes;
       // columns beyond the matrix read the next row's values; they only reach results beyond the matrix
-      load_to_lds(rg, buf[0] + base * kRowBytes, (uint32_t)(row * q.n + n0 + col) * 2);
-      load_to_lds(rx, buf[1] + base * kRowBytes, (uint32_t)(row * q.k + k0 + col) * 2);
+      load_to_lds(rg, buf[0] + base * kRowBytes, (uint32_t)(row * q.n + n0 + col) * kBytes);
+      load_to_lds(rx, buf[1] + base * kRowBytes, (uint32_t)(row * q.k + k0 + col) * kBytes);
     }
   };
 
+  // Fragments of a slice: for 16-bit types two steps of 32 rows, a lane's eight values by two turned reads; for fp32 eight
+  // steps of four rows, a lane's value as it lies.
+  typedef typename std::conditional<kBytes == 2, u32x4, float>::type frag_t;
+  constexpr int kSteps = kBytes == 2 ? 2 : kRows / 4;
   const int wn = wave >> 1, wk = wave & 1, kb = lane >> 4, i16 = lane & 15;
-  const int frag_row = kb * 8 + (i16 >> 2), f = unit_swizzle<W>(frag_row);
+  const int frag_row = kBytes == 2 ? kb * 8 + (i16 >> 2) : kb, f = unit_swizzle<Tag, W>(frag_row);
+  const int in_unit = kBytes == 2 ? (i16 & 3) * 8 : i16 * 4;
   int at_n[F], at_k[F];
 #pragma unroll
   for (int i = 0; i < F; ++i) {
-    at_n[i] = frag_row * kRowBytes + (((wn * F + i) ^ f) * 32) + (i16 & 3) * 8;
-    at_k[i] = frag_row * kRowBytes + (((wk * F + i) ^ f) * 32) + (i16 & 3) * 8;
+    at_n[i] = frag_row * kRowBytes + ((wn * F + i) ^ f) * kUnit + in_unit;
+    at_k[i] = frag_row * kRowBytes + ((wk * F + i) ^ f) * kUnit + in_unit;
   }
-  auto fragment = [&](const char *base, int at, int s) {
-    const u32x2 lo = read_turned(base + at + s * 32 * kRowBytes), hi = read_turned(base + at + (s * 32 + 4) * kRowBytes);
-    return u32x4{lo.x, lo.y, hi.x, hi.y};
+  auto fragment = [&](const char *base, int at, int s) -> frag_t {
+    if constexpr (kBytes == 2) {
+      const u32x2 lo = read_turned(base + at + s * 32 * kRowBytes), hi = read_turned(base + at + (s * 32 + 4) * kRowBytes);
+      return u32x4{lo.x, lo.y, hi.x, hi.y};
+    } else {
+      return *reinterpret_cast<const float *>(base + at + s * 4 * kRowBytes);
+    }
   };
-  const uint32_t one = Tag::kCode == F16::kCode ? 0x3c003c00u : 0x3f803f80u;
-  const u32x4 ones = {one, one, one, one};
+  auto multiply = [](frag_t a, frag_t b, f32x4 c) {
+    if constexpr (kBytes == 2) return mfma_64_bytes<Tag>(a, b, c);
+    else return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  };
+  frag_t ones;
+  if constexpr (kBytes == 2) {
+    constexpr uint32_t one = Tag::kCode == F16::kCode ? 0x3c003c00u : 0x3f803f80u;
+    ones = u32x4{one, one, one, one};
+  } else {
+    ones = 1.f;
+  }
   const bool with_bias = q.grad_bias != nullptr && k0 == 0 && wk == 0;
 
   f32x4 acc[F][F], bias[F];
@@ -89,9 +112,9 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   for (long long row0 = row_begin; row0 < row_end; row0 += kRows, cur ^= 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    u32x4 fn[2][F], fk[2][F];
+    frag_t fn[kSteps][F], fk[kSteps][F];
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < kSteps; ++s)
 #pragma unroll
       for (int i = 0; i < F; ++i) {
         fn[s][i] = fragment(lds[cur][0], at_n[i], s);
@@ -99,12 +122,12 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
       }
     if (row0 + kRows < row_end) stage(row0 + kRows, lds[cur ^ 1]);
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < kSteps; ++s)
 #pragma unroll
       for (int i = 0; i < F; ++i) {
 #pragma unroll
-        for (int j = 0; j < F; ++j) acc[i][j] = mfma_16x16x32<Tag>(fk[s][j], fn[s][i], acc[i][j]);
-        if (with_bias) bias[i] = mfma_16x16x32<Tag>(ones, fn[s][i], bias[i]);
+        for (int j = 0; j < F; ++j) acc[i][j] = multiply(fk[s][j], fn[s][i], acc[i][j]);
+        if (with_bias) bias[i] = multiply(ones, fn[s][i], bias[i]);
       }
   }
   // results: rows of the fragment are the depth, so a lane stores four consecutive k of one n
@@ -147,32 +170,68 @@ __global__ void __launch_bounds__(256) linear_grad_reduce_kernel(const WeightGra
   }
 }
 
-// 16-bit copies of fp32 parameters: a matrix [n, k] as it lies and turned [k, n], in tiles of 64 x 64 through LDS; a vector
-// (n = 1, nothing turned) as a row.
+// Copies of fp32 parameters in the type: a matrix [n, k] as it lies and turned [k, n], in tiles of 64 x 64 through LDS; a
+// vector (n = 1, nothing turned) as a row.
 template <typename Tag>
 __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaunch p) {
-  typedef typename RawWord<2>::type half_t;
-  __shared__ half_t tile[64][66];
+  typedef typename RawWord<Tag::kBytes>::type elem_t;
+  __shared__ elem_t tile[64][64 + 4 / Tag::kBytes];
   int which = 0;
   while (which + 1 < p.count && (int)blockIdx.x >= p.tile_end[which]) ++which;
   const CastWeights &q = p.p[which];
   const int local = blockIdx.x - (which ? p.tile_end[which - 1] : 0), tiles_k = (q.k + 63) / 64;
   const int n0 = local / tiles_k * 64, k0 = local % tiles_k * 64;
   const int col = threadIdx.x & 63;
+#pragma unroll 4
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
     const int n = n0 + r, k = k0 + col;
     if (n >= q.n || k >= q.k) continue;
     const float v[1] = {q.from[(size_t)n * q.k + k]};
-    const half_t h = Pack<Tag, 1>::encode(v);
-    static_cast<half_t *>(q.to)[(size_t)n * q.k + k] = h;
+    const elem_t h = Pack<Tag, 1>::encode(v);
+    if (q.to != nullptr) static_cast<elem_t *>(q.to)[(size_t)n * q.k + k] = h;
     tile[r][col] = h;
   }
   if (q.turned == nullptr) return;
   __syncthreads();
+#pragma unroll 4
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
     const int k = k0 + r, n = n0 + col;
-    if (n < q.n && k < q.k) static_cast<half_t *>(q.turned)[(size_t)k * q.n + n] = tile[col][r];
+    if (n < q.n && k < q.k) static_cast<elem_t *>(q.turned)[(size_t)k * q.n + n] = tile[col][r];
   }
+}
+
+// Eight gradients of one (head, level) at a time: the backward of SamplingLocations, rounded where the framework rounds.
+template <typename Tag, typename LocTag>
+__global__ void __launch_bounds__(256) location_grad_kernel(const SamplingLocations l, const void *grad_locations, void *grad_offsets,
+                                                            size_t vectors, int vectors_per_row) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= vectors) return;
+  const size_t row = i / (size_t)vectors_per_row;
+  const int n = (int)(i - row * vectors_per_row) * 8, level = n / (2 * l.points) % l.levels;
+  float g[8];
+  load8<LocTag>(grad_locations, i * 8, g);
+  if (l.kind == 2) {
+    const float w = (float)l.shapes[2 * level + 1], h = (float)l.shapes[2 * level];
+    round8<Tag>(g);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) g[c] /= (c & 1) ? h : w;
+  } else {
+    const float *size = l.reference + (row * l.levels + level) * 4 + 2;
+    const float points = (float)l.points;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) g[c] = mul_rn(mul_rn(g[c], 0.5f), size[c & 1]);
+    round8<Tag>(g);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) g[c] /= points;
+  }
+  store8<Tag>(grad_offsets, i * 8, g);
+}
+
+// A wave per row.
+__global__ void __launch_bounds__(256) zero_rows_kernel(u32x4 *out, const uint8_t *zero, long long rows, int vectors) {
+  const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows || zero[row] == 0) return;
+  for (int i = threadIdx.x & 63; i < vectors; i += 64) out[row * vectors + i] = u32x4{0, 0, 0, 0};
 }
 
 template <typename Tag, bool SRC32>
@@ -209,7 +268,7 @@ hipError_t launch_grad_t(const WeightGradLaunch &p, hipStream_t stream) {
 // 50176 x 224 151 / 185, 200704 x 112 169 / 238, 200704 x 64 106 / 84 - the wide tile is for many rows, where it reads its
 // operands half as often, unless most of it is padding.  Best splits: about 3136 rows each for the small tile (42, 44, 84,
 // 119 us above; 2 to 4 times as many cost 15 to 30 % more), about 400 workgroups for the wide one.
-WeightGradPlan plan_weight_grad(const WeightGradLaunch &p) {
+WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p) {
   auto tiles = [&](int w) {
     long long n = 0;
     for (int i = 0; i < p.count; ++i) n += (long long)((p.p[i].n + w - 1) / w) * ((p.p[i].k + w - 1) / w);
@@ -218,7 +277,9 @@ WeightGradPlan plan_weight_grad(const WeightGradLaunch &p) {
   WeightGradPlan plan;
   const long long wide = tiles(128), small = tiles(64);
   plan.tile = p.rows >= 32768 && wide * 4 * 5 <= small * 6 ? 128 : 64;
-  const double want = plan.tile == 64 ? (double)p.rows / 3136 : std::min(400.0 / (double)wide, (double)p.rows / 1500);
+  // fp32 is bound by the matrix cores: even shares of the chip count
+  if (dtype == F32::kCode) plan.tile = 64;
+  const double want = dtype == F32::kCode ? (double)p.rows / 1300 : plan.tile == 64 ? (double)p.rows / 3136 : std::min(400.0 / (double)wide, (double)p.rows / 1500);
   plan.splits = 1;
   while (plan.splits < 64 && want >= 1.5 * plan.splits) plan.splits *= 2;
   return plan;
@@ -226,9 +287,11 @@ WeightGradPlan plan_weight_grad(const WeightGradLaunch &p) {
 
 hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &launch, int tile, hipStream_t stream) {
   WeightGradLaunch p = launch;
-  p.rows_per_split = ((p.rows + p.splits - 1) / p.splits + kRows - 1) / kRows * kRows;
+  const int slice = dtype == F32::kCode ? kRowsOf<F32> : kRowsOf<F16>;
+  p.rows_per_split = ((p.rows + p.splits - 1) / p.splits + slice - 1) / slice * slice;
   int end = 0;
   for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + tile - 1) / tile) * ((p.p[i].k + tile - 1) / tile);
+  if (dtype == F32::kCode) return launch_grad_t<F32, 64>(p, stream);
   if (dtype == F16::kCode) return tile == 128 ? launch_grad_t<F16, 128>(p, stream) : launch_grad_t<F16, 64>(p, stream);
   return tile == 128 ? launch_grad_t<BF16, 128>(p, stream) : launch_grad_t<BF16, 64>(p, stream);
 }
@@ -244,8 +307,28 @@ hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &launch, hipSt
   CastWeightsLaunch p = launch;
   int end = 0;
   for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + 63) / 64) * ((p.p[i].k + 63) / 64);
-  if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3(end), dim3(256), 0, stream, p);
+  if (dtype == F32::kCode) hipLaunchKernelGGL(cast_weights_kernel<F32>, dim3(end), dim3(256), 0, stream, p);
+  else if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3(end), dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(cast_weights_kernel<BF16>, dim3(end), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_location_grad(int dtype, const SamplingLocations &l, const void *grad_locations, bool locations32, void *grad_offsets,
+                                long long rows, int n, hipStream_t stream) {
+  const size_t vectors = (size_t)rows * (n / 8);
+  const dim3 grid((unsigned)((vectors + 255) / 256)), block(256);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, l, grad_locations, grad_offsets, vectors, n / 8);
+    return hipGetLastError();
+  };
+  if (dtype == F32::kCode) return run(location_grad_kernel<F32, F32>);
+  if (dtype == F16::kCode) return locations32 ? run(location_grad_kernel<F16, F32>) : run(location_grad_kernel<F16, F16>);
+  return locations32 ? run(location_grad_kernel<BF16, F32>) : run(location_grad_kernel<BF16, BF16>);
+}
+
+hipError_t launch_zero_rows(int elem_bytes, void *rows_of, const uint8_t *zero, long long rows, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, static_cast<u32x4 *>(rows_of), zero, rows,
+                     n * elem_bytes / 16);
   return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-// Matrix-core helpers for 16-bit tensors: fragments of v_mfma_f32_16x16x32, the exact GELU, 16-byte loads into LDS.
+// Matrix-core helpers: fragments of the 16 x 16 instructions, the exact GELU, 16-byte loads into LDS.
 #pragma once
 #include "common.hpp"
 
@@ -7,14 +7,49 @@ namespace dcn {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// d[i][j] += sum over k of a[i][k] * b[j][k], 16 x 16 x 32.  A lane holds 8 consecutive k of row (lane & 15) of each
-// operand, k block lane >> 4; of the result it holds rows 4 * (lane >> 4) .. + 3 of column (lane & 15).
+// d[i][j] += sum over 64 bytes of depth of a[i][k] * b[j][k], 16 x 16: one 16x16x32 instruction for 16-bit types, four 16x16x4
+// for fp32.  A lane holds 16 bytes of row (lane & 15) of each operand, those at depth block lane >> 4 (an fp32 instruction
+// takes one of a lane's four values, the same one of both operands, so the order of the depth does not matter); of the result it
+// holds rows 4 * (lane >> 4) .. + 3 of column (lane & 15).
 template <typename Tag>
-__device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (Tag::kCode == F16::kCode)
+__device__ __forceinline__ f32x4 mfma_64_bytes(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (Tag::kCode == F16::kCode) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
+  } else if constexpr (Tag::kCode == BF16::kCode) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  } else {
+    const f32x4 x = __builtin_bit_cast(f32x4, a), y = __builtin_bit_cast(f32x4, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], c, 0, 0, 0);
+    return c;
+  }
+}
+
+// Eight consecutive elements: 16 bytes, or 32 of fp32.
+template <typename Tag>
+__device__ __forceinline__ void load8(const void *base, size_t element, float (&f)[8]) {
+  if constexpr (Tag::kBytes == 2) {
+    Pack<Tag, 8>::decode(*reinterpret_cast<const u32x4 *>(static_cast<const char *>(base) + element * 2), f);
+  } else {
+    const f32x4 *v = reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + element);
+    const f32x4 lo = v[0], hi = v[1];
+    f[0] = lo.x; f[1] = lo.y; f[2] = lo.z; f[3] = lo.w; f[4] = hi.x; f[5] = hi.y; f[6] = hi.z; f[7] = hi.w;
+  }
+}
+template <typename Tag>
+__device__ __forceinline__ void store8(void *base, size_t element, const float (&f)[8]) {
+  if constexpr (Tag::kBytes == 2) {
+    *reinterpret_cast<u32x4 *>(static_cast<char *>(base) + element * 2) = Pack<Tag, 8>::encode(f);
+  } else {
+    f32x4 *v = reinterpret_cast<f32x4 *>(static_cast<float *>(base) + element);
+    v[0] = f32x4{f[0], f[1], f[2], f[3]};
+    v[1] = f32x4{f[4], f[5], f[6], f[7]};
+  }
+}
+// Rounded to the type and back.
+template <typename Tag>
+__device__ __forceinline__ void round8(float (&f)[8]) {
+  if constexpr (Tag::kBytes == 2) Pack<Tag, 8>::decode(Pack<Tag, 8>::encode(f), f);
 }
 
 // x * Phi(x) = max(x, 0) - |x| Phi(-|x|), with Phi(-|x|) = exp(-x^2 / 2) * erfcx(|x| / sqrt 2) / 2 and the scaled function as a
@@ -37,7 +72,11 @@ __device__ __forceinline__ NormalTail normal_tail(float x) {
   r.tail = p * r.bell;
   return r;
 }
-__device__ __forceinline__ float gelu_exact(float x) { return fmaf(-fabsf(x), normal_tail(x).tail, fmaxf(x, 0.f)); }
+template <typename Tag>
+__device__ __forceinline__ float gelu_exact(float x) {
+  if constexpr (Tag::kBytes == 4) return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));      // an fp32 result keeps fp32 precision
+  else return fmaf(-fabsf(x), normal_tail(x).tail, fmaxf(x, 0.f));
+}
 // Phi(x) + x phi(x)
 __device__ __forceinline__ float gelu_derivative(float x) {
   const NormalTail n = normal_tail(x);

@@ -8,11 +8,13 @@ plus torch's current HIP stream to the C ABI; for the two sampling operators tha
 them.
 """
 import torch
+from torch import nn
 
 from . import _lib
 
 _L = _lib.load()
 _native = _lib.load_native()
+_native.register_modules(nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Identity, nn.Conv2d, nn.Sequential)
 
 _DTYPES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
 
@@ -140,7 +142,7 @@ def flash_deform_attn_backward(value, spatial_shapes, level_start_index, samplin
 
 
 def linear_forward(input, weight, bias=None, gamma=None, residual=None, gelu=False):
-    """``act(input @ weight.T + bias) * gamma + residual`` for 16-bit tensors, ``act`` the exact GELU or nothing: the linear
+    """``act(input @ weight.T + bias) * gamma + residual``, ``act`` the exact GELU or nothing: the linear
     layers of a FlashInternImage layer with what follows them, as one matrix-core kernel."""
     return _native.linear(input, weight, bias, gamma, residual, bool(gelu))
 

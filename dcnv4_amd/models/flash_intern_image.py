@@ -150,8 +150,7 @@ class InternImageLayer(nn.Module):
 
 
 _ext_forward = ext.dcnv4_forward
-ext._native.register_modules(nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Identity, nn.Conv2d, nn.Sequential, DropPath, DCNv4,
-                             MLPLayer)
+ext._native.register_modules(DropPath, DCNv4, MLPLayer)
 
 
 class InternImageBlock(nn.Module):

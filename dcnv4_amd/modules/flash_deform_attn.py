@@ -12,7 +12,9 @@ import warnings
 import torch
 from torch import nn
 
+from .. import ext
 from ..functions import FlashDeformAttnFunction, FlashDeformAttnSplitFunction
+from ..functions.flash_deform_attn_func import _interpreted
 
 
 def _ring_directions(n_heads):
@@ -20,6 +22,18 @@ def _ring_directions(n_heads):
     angle = torch.arange(n_heads, dtype=torch.float32) * (2.0 * math.pi / n_heads)
     xy = torch.stack((angle.cos(), angle.sin()), dim=-1)
     return xy / xy.abs().amax(dim=-1, keepdim=True)
+
+
+def _pixels(spatial_shapes):
+    """Pixels of all levels together.  Reading them waits for the GPU, so a tensor of shapes is read once: the encoder and
+    decoder layers of a pass share it.  What was read is kept with the tensor's version and read again after a change."""
+    known = getattr(spatial_shapes, "_dcnv4_pixels", None)      # (inference tensors have no version and are never kept)
+    if known is not None and known[0] == spatial_shapes._version:
+        return known[1]
+    n = int(spatial_shapes.prod(-1).sum())
+    if not spatial_shapes.is_inference():
+        spatial_shapes._dcnv4_pixels = (spatial_shapes._version, n)
+    return n
 
 
 class FlashDeformAttn(nn.Module):
@@ -72,7 +86,14 @@ class FlashDeformAttn(nn.Module):
         input_padding_mask (N, sum H_l W_l) bool, True where the input is padding.  Returns (N, Lq, C)."""
         n, n_query, _ = query.shape
         n_in = input_flatten.shape[1]
-        assert int(input_spatial_shapes.prod(-1).sum()) == n_in, "the levels do not add up to the flattened input"
+        assert _pixels(input_spatial_shapes) == n_in, "the levels do not add up to the flattened input"
+
+        if query.is_cuda and not _interpreted():
+            # one call where the kernels take the layer as it is (csrc/binding/attention.cpp)
+            out = ext._native.attention_layer(self, query, reference_points, input_flatten, input_spatial_shapes,
+                                              input_level_start_index, input_padding_mask)
+            if out is not None:
+                return out
 
         value = self.value_proj(input_flatten)
         if input_padding_mask is not None:

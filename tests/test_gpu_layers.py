@@ -130,3 +130,66 @@ def test_layer_training_takes_one_node_and_reports_a_second_backward():
     assert torch.equal(first, torch.autograd.grad(out.sum(), x)[0])
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(out.sum(), x)
+
+
+# levels, queries (0: every pixel), reference coordinates, batch, padding, model width, points: few-row and tiled products, rows
+# that fill no tile, feature rows that differ from query rows and do not
+ATTENTION = [([(7, 9), (4, 5), (2, 3), (1, 2)], 0, 2, 3, True, 256, 4), ([(25, 31), (13, 16), (7, 8), (4, 4)], 77, 4, 2, True, 256, 4),
+             ([(12, 10), (6, 5)], 33, 2, 1, False, 64, 8), ([(40, 52), (20, 26), (10, 13), (5, 7)], 0, 4, 2, False, 128, 4)]
+
+
+@pytest.mark.parametrize("amp", [None, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("levels,queries,kind,batch,padded,width,points", ATTENTION, ids=[f"L{len(c[0])}-q{c[1]}-ref{c[2]}" for c in ATTENTION])
+def test_attention_layer_in_one_call_matches_the_composition(levels, queries, kind, batch, padded, width, points, amp):
+    import dcnv4_amd
+    torch.manual_seed(queries + kind)
+    m = dcnv4_amd.FlashDeformAttn(width, len(levels), 4, points).cuda()
+    with torch.no_grad():
+        m.sampling_offsets.weight.normal_(0, 0.05)
+        m.attention_weights.weight.normal_(0, 0.05)
+    pixels = sum(h * w for h, w in levels)
+    q = queries or pixels
+    shapes = torch.tensor(levels, device="cuda")
+    starts = torch.tensor([sum(h * w for h, w in levels[:i]) for i in range(len(levels))], device="cuda")
+    query, features = torch.randn(batch, q, width, device="cuda"), torch.randn(batch, pixels, width, device="cuda")
+    reference = torch.rand(batch, q, len(levels), kind, device="cuda")
+    mask = torch.rand(batch, pixels, device="cuda") < 0.2 if padded else None
+    grad = torch.randn(batch, q, width, device="cuda").to(amp or torch.float32)
+    results = []
+    for composed in (False, True):
+        handle = m.output_proj.register_forward_hook(lambda *a: None) if composed else None
+        qi, fi = query.clone().requires_grad_(), features.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            out = m(qi, reference, fi, shapes, starts, mask)
+        assert (out.grad_fn.name() == "FlashDeformAttnBackward") != composed
+        results.append([out.detach(), *torch.autograd.grad(out, [qi, fi, *m.parameters()], grad)])
+        if composed:
+            handle.remove()
+    # fp32: a location that rounds to the other side in fp16 moves its sample
+    tol = {None: 2e-3, torch.float16: 4e-3, torch.bfloat16: 2e-2}[amp]
+    for name, got, want in zip(["output", "query", "features"] + [k for k, _ in m.named_parameters()], *results):
+        assert got.dtype == want.dtype and got.shape == want.shape, name
+        assert _rel(got, want) < tol, (name, _rel(got, want))
+    if padded:
+        assert not results[0][2][mask].any()
+
+
+def test_attention_layer_reads_changed_level_shapes_again():
+    import dcnv4_amd
+    m = dcnv4_amd.FlashDeformAttn(64, 1, 4, 4).cuda()
+    shapes, starts = torch.tensor([[4, 6]], device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    x, ref = torch.randn(1, 24, 64, device="cuda"), torch.rand(1, 24, 1, 2, device="cuda")
+    with torch.no_grad():
+        m(x, ref, x, shapes, starts)
+        shapes[0, 0] = 5
+        with pytest.raises(AssertionError, match="levels"):
+            m(x, ref, x, shapes, starts)
+
+
+@pytest.mark.parametrize("rows,depth,width", [(5, 16, 8), (129, 72, 104), (6000, 256, 384)])
+def test_fp32_linear_matches_fp64(rows, depth, width):
+    from dcnv4_amd import ext
+    a, w, b = torch.randn(rows, depth, device="cuda"), torch.randn(width, depth, device="cuda"), torch.randn(width, device="cuda")
+    product = a.double() @ w.double().t() + b.double()
+    assert _rel(ext.linear_forward(a, w, b), product) < 1e-6
+    assert _rel(ext.linear_forward(a, w, b, gelu=True), torch.nn.functional.gelu(product)) < 1e-6
