@@ -361,6 +361,48 @@ bool plan_gather_tiles(DcnLaunch *L, int s, bool backward) {
   return false;
 }
 
+// Window gathers (dcnv4_window.hip): 3x3 kernels with their centre, stride and dilation 1, groups of 32, 64 or 128 bytes.
+// Returns the 32-byte units per workgroup and sets the output tile, or 0.
+//
+// A workgroup's 256 lanes take `units` units of 256 / units pixels.  One group at a time is best wherever the image fills the
+// tile (64x56x56, 4 groups of 16, fp16: 32 us, 36 with two, 41 with four: more pixels share a window), two where it fills
+// less than a quarter of it (64x7x7, 32 groups: 9.7 us with one, 8.4 with two).  The tile is the one with the least work:
+// workgroups times their lanes and window; of equals the taller one, whose window rows are shorter than they are many (28x8
+// 32.3 us, 8x28 35.0).  Tiles for the backward stay within 16 x 16, because every point that a window serves counts for the
+// distance the grad_value kernel looks at.  The reach is 5 pixels, and 4 for groups of 128 bytes, whose window then lets a CU
+// hold four workgroups instead of three (64x56x56, 4 groups of 32 fp32: 84 against 99 us).
+int plan_window_gather(DcnLaunch *L, int s, int batch, bool backward) {
+  const int unit_bytes = L->D * s;
+  if (g_opt.gather != kOptAuto || g_opt.gather_tile != 0 || L->kh != 3 || L->kw != 3 || L->remove_center || L->softmax || L->sh != 1 ||
+      L->sw != 1 || L->dh != 1 || L->dw != 1 || (unit_bytes != 32 && unit_bytes != 64 && unit_bytes != 128) || (s == 4 && unit_bytes == 32))
+    return 0;
+  const int lpg = unit_bytes / 32, Ho = L->Q / L->Wo, Wo = L->Wo;
+  const int reach = g_opt.reach >= 0 ? std::min(g_opt.reach, 12) : lpg == 4 ? 4 : kDefaultReach;
+  int units = lpg;
+  while (units < 4 && L->Q <= 256 / units / 4) units *= 2;
+  const int most = backward ? 16 : 32, pixels = 256 / units;
+  const double chunks = (L->G + units / lpg - 1) / (units / lpg);
+  auto parts = [](int extent, int size) { return (extent + size - 1) / size; };
+  double best = 0.;
+  for (int h = 4; h <= std::min(most, pixels); ++h) {
+    const int nty = parts(Ho, h), th = parts(Ho, nty);
+    const int ntx = parts(Wo, std::min(most, pixels / th)), tw = parts(Wo, ntx);
+    const int wh = std::min(th + 2 * reach, L->H + 2), ww = std::min(tw + 2 * reach, L->W + 2);
+    const size_t window = (size_t)wh * ww * units * 32;
+    if (window > kMaxLdsPerWorkgroup / 2) continue;
+    const double cost = std::max(batch * chunks * nty * ntx, 2. * kCusPerDevice) * (1. + (double)window / (64 * 1024));
+    if (best == 0. || cost <= best) {
+      best = cost;
+      L->gt_h = th; L->gt_w = tw;
+      L->gt_wh = wh; L->gt_ww = ww;
+    }
+    if (th >= Ho) break;
+  }
+  if (best == 0.) return 0;
+  L->gt_reach = reach;
+  return units;
+}
+
 // ---------------------------------------------------------------- DCNv4
 // Output pixels per workgroup: about block_thread (default 256) lanes of whole pixels, capped by
 // the LDS that the staged offset_mask rows (and, backward, their gradients) take.
@@ -763,13 +805,14 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
     return rc;
   if (int rc = check_ptrs({value, offset_mask, output})) return rc;
   const int per = images_per_launch(pr, false);
-  // A small call is a chain of latencies: the direct kernel's lanes go to memory at once, where the tiled one first stages
-  // its window behind a barrier.  Measured (fp16 / fp32, us, direct against tiled): 1x7x7x512 5.6 / 5.3 against 10.8 / 9.3,
-  // 2x56x56x112 6.7 / 7.6 against 9.8 / 8.3, 8x28x28x128 6.6 / 8.7 against 9.8 / 8.3; at 8x56x56x64 they meet in fp16
-  // (10.6 / 14.5 against 10.2 / 11.5), at 1x100x152x160 the tiled one is ahead (15.9 / 23.1 against 14.2 / 17.8).
+  // A small call is a chain of latencies: the direct kernel's lanes go to memory at once, where the others first stage a window
+  // behind a barrier.  Measured (fp16, us, direct against window): 4x56x56x64 (1.6 MB) 6.5 against 7.4, 1x100x152x64 (1.9 MB)
+  // 6.9 against 7.6, 6x56x56x64 (2.4 MB) 8.3 against 7.9, 4x64x64x128 (4.2 MB) 9.5 against 8.8; against the tiled kernel, which
+  // takes the other kernel shapes, they meet at about 3 MB.
   const bool small = g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 &&
                      (uint64_t)batch * pr.img_out_elems * pr.s <= kDirectForwardBytes;
-  const bool tiled = !small && plan_gather_tiles(&pr.launch, pr.s, false);
+  const int window = small ? 0 : plan_window_gather(&pr.launch, pr.s, batch, false);
+  const bool tiled = !small && window == 0 && plan_gather_tiles(&pr.launch, pr.s, false);
   for (int b0 = 0; b0 < batch; b0 += per) {
     const int nb = std::min(per, batch - b0);
     DcnLaunch L = pr.launch;
@@ -778,8 +821,9 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
     L.out = at(output, b0 * pr.img_out_elems, pr.s);
     L.value_bytes = (uint32_t)(nb * pr.img_elems * pr.s);
     L.n_pix = nb * L.Q;
-    const hipError_t e = tiled ? launch_dcnv4_forward_tiled(dtype, L, static_cast<hipStream_t>(stream))
-                               : launch_dcnv4_forward(dtype, L, static_cast<hipStream_t>(stream));
+    const hipError_t e = window  ? launch_dcnv4_forward_window(dtype, L, window, static_cast<hipStream_t>(stream))
+                         : tiled ? launch_dcnv4_forward_tiled(dtype, L, static_cast<hipStream_t>(stream))
+                                 : launch_dcnv4_forward(dtype, L, static_cast<hipStream_t>(stream));
     if (e) return hip_fail("dcnv4 forward launch", e);
   }
   return DCNV4_OK;
@@ -818,7 +862,7 @@ static int dcn_backward_impl(const void *value, const void *offset_mask, const v
   if (base.Q >= (1 << 24) || (uint64_t)base.Q * (uint64_t)base.P_pad >= (1ull << 31) ||
       (uint64_t)base.Q * (uint64_t)(base.G * base.D) >= (1ull << 31))
     return fail(DCNV4_ERR_RUNTIME, "one image of %d output pixels is too large for the backward", base.Q);
-  const bool gather_tiled = plan_gather_tiles(&base, pr.s, true);
+  bool gather_tiled = plan_gather_tiles(&base, pr.s, true);
   base.state = static_cast<GradState *>(workspace);
   // When a grad_value tile is a whole image its workgroups visit every output pixel whatever the reach: nobody reads
   // the statistic that the first kernel folds into the state, and the launch that resets it is left out.
@@ -829,6 +873,12 @@ static int dcn_backward_impl(const void *value, const void *offset_mask, const v
   // learn how far to look for them (GradState::far_reach) and only their workgroups visit the pixels in between.
   // The cap exceeds what a staged window of the first kernel spans, so that a point beyond it is always one of the
   // points that kernel serves from memory - where it is folded.
+  const int per = images_per_launch(pr, false);
+  // both kernels in one launch when they do not depend on each other and the shape suits the two-role kernel
+  const bool dual = g_opt.dual != kOptPlain && dcnv4_backward_dual_fits(base, pr.s);
+  if (dual) base.dual_interleave = dcnv4_backward_dual_workgroups(base, std::min(per, batch)) <= 3u * kCusPerDevice ? 1 : 0;
+  const int window = dual ? 0 : plan_window_gather(&base, pr.s, batch, true);
+  if (window) gather_tiled = true;
   base.gv_reach_cap = 3.0e38f;
   if (!base.gv_whole) {
     int cap = kReachCap;
@@ -839,10 +889,6 @@ static int dcn_backward_impl(const void *value, const void *offset_mask, const v
     hipLaunchKernelGGL(init_state_kernel, dim3(1), dim3(64), 0, st, base.state);
     if (hipError_t e = hipGetLastError()) return hip_fail("state init launch", e);
   }
-  const int per = images_per_launch(pr, false);
-  // both kernels in one launch when they do not depend on each other and the shape suits the two-role kernel
-  const bool dual = g_opt.dual != kOptPlain && dcnv4_backward_dual_fits(base, pr.s);
-  if (dual) base.dual_interleave = dcnv4_backward_dual_workgroups(base, std::min(per, batch)) <= 3u * kCusPerDevice ? 1 : 0;
   for (int pass = 0; pass < (dual ? 1 : 2); ++pass) {
     for (int b0 = 0; b0 < batch; b0 += per) {
       const int nb = std::min(per, batch - b0);
@@ -857,6 +903,7 @@ static int dcn_backward_impl(const void *value, const void *offset_mask, const v
       L.n_img = nb;
       hipError_t e = hipSuccess;
       if (dual) e = launch_dcnv4_backward_dual(dtype, L, st);
+      else if (pass == 0 && window) e = launch_dcnv4_offset_mask_grad_window(dtype, L, window, st);
       else if (pass == 0 && gather_tiled) e = launch_dcnv4_offset_mask_grad_tiled(dtype, L, st);
       else if (pass == 0) e = launch_dcnv4_offset_mask_grad(dtype, L, st);
       else e = launch_dcnv4_grad_value(dtype, L, st);

@@ -112,6 +112,13 @@ template <typename Tag, int N> struct Pack {
   }
 };
 
+// a.lo * b.lo + a.hi * b.hi + c for two packed 16-bit elements per word, products and sum in fp32
+template <typename Tag>
+__device__ __forceinline__ float dot2_pair(uint32_t a, uint32_t b, float c) {
+  if constexpr (Tag::kCode == F16::kCode) return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
+  else return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
+}
+
 // ---------------------------------------------------------------- coordinate arithmetic
 // Sampling coordinates are formed in fp32 one rounded operation at a time, in the reference's
 // source order (dcnv4_im2col_cuda.cuh:203-224, flash_deform_im2col_cuda.cuh:188-189), never

@@ -39,13 +39,6 @@ constexpr int kTiledThreads = 512;      // lanes per workgroup at most: leaves e
 __device__ __forceinline__ float rcp(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ int fdiv(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
 
-// a.lo * b.lo + a.hi * b.hi + c for two packed 16-bit elements per word, products and sum in fp32
-template <typename Tag>
-__device__ __forceinline__ float dot2_pair(uint32_t a, uint32_t b, float c) {
-  if constexpr (Tag::kCode == F16::kCode) return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
-  else return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
-}
-
 template <typename Tag>
 __device__ __forceinline__ float lds_elem(const typename RawWord<Tag::kBytes>::type *p, int i) {
   float f[1];

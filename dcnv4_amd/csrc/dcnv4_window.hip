@@ -1,0 +1,389 @@
+// DCNv4 forward for 3x3 kernels of stride and dilation 1 over groups of 32, 64 or 128 bytes (dcnv4_window.hpp).
+#include "dcnv4_window.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace dcn {
+namespace {
+
+template <typename Tag, int LPG, int UNITS>
+__global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel(const DcnLaunch p) {
+  extern __shared__ u32x4 lds128[];
+  constexpr int kGroups = UNITS / LPG, EPV = 16 / Tag::kBytes, kCell = UNITS * 32;
+  typedef Pack<Tag, EPV> pack;
+  char *lds = reinterpret_cast<char *>(lds128);
+  const WindowTile t = window_tile<kGroups>(p, blockIdx.x, gridDim.x);
+  const WindowFrame<UNITS> frame(t);
+
+  // lane -> (pixel of the tile, group of the workgroup, part of the group): a wave stays within one group
+  constexpr int kPixels = kWindowThreads / UNITS, kPerGroup = kPixels * LPG;
+  const int gl = threadIdx.x / kPerGroup, part = threadIdx.x & (LPG - 1), q = threadIdx.x % kPerGroup / LPG;
+  const int py = exact_div(q, __builtin_amdgcn_rcpf((float)p.gt_w)), px = q - py * p.gt_w;
+  const bool active = py < t.th && px < t.tw && t.g0 + gl < p.G;
+  const int ho = t.oy0 + py, wo = t.ox0 + px;
+  const size_t pixel = active ? (size_t)t.b * p.Q + (size_t)ho * p.Wo + wo : 0;
+  const int g = active ? t.g0 + gl : 0;
+  PointRows<Tag, LPG> rows;
+  const void *row = static_cast<const char *>(p.offset_mask) + (pixel * p.P_pad + (size_t)g * 27) * Tag::kBytes;
+  rows.load(row, part);
+  stage_window<Tag, UNITS>(p, t, lds);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (!active) return;
+
+  const float x_base = sub_rn((float)(1 - p.pw + wo), p.offset_scale), y_base = sub_rn((float)(1 - p.ph + ho), p.offset_scale);
+  auto position = [&](int own, int k, float &y, float &x, float &m) {
+    float ox, oy;
+    rows.get(own, ox, oy, m);
+    const int i = LPG == 1 ? k / 3 : exact_div(k, 1.f / 3.f), j = k - 3 * i;
+    x = add_rn(x_base, mul_rn(add_rn((float)i, ox), p.offset_scale));
+    y = add_rn(y_base, mul_rn(add_rn((float)j, oy), p.offset_scale));
+  };
+  const int lane_bytes = (gl * LPG + part) * 32;
+  float acc[2][EPV];
+#pragma unroll
+  for (int v = 0; v < 2; ++v)
+#pragma unroll
+    for (int c = 0; c < EPV; ++c) acc[v][c] = 0.f;
+  uint32_t far = 0;      // a bit for each point this lane prepares that is inside the image but outside the window
+  auto gather = [&](int addr, const float (&w)[4]) {
+    const char *src = lds + addr;
+    u32x4 raw[4][2];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) raw[cn][v] = *reinterpret_cast<const u32x4 *>(src + (cn & 1) * kCell + (cn >> 1) * frame.row_bytes + 16 * v);
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        float f[EPV];
+        pack::decode(raw[cn][v], f);
+#pragma unroll
+        for (int c = 0; c < EPV; ++c) acc[v][c] = fmaf(w[cn], f[c], acc[v][c]);
+      }
+  };
+  constexpr int kOwn = PointRows<Tag, LPG>::kOwn;
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    const int k = LPG == 1 ? i : min(part + i * LPG, 8);
+    float y, x, m;
+    position(i, k, y, x, m);
+    const WindowPoint pt = window_point<UNITS>(frame, y, x, m);
+    if (!__all(pt.ok)) {
+      const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
+      far |= (uint32_t)(inside && !pt.ok) << k;
+    }
+    auto one = [&](auto jj) {
+      constexpr int J = decltype(jj)::value;
+      if constexpr (J < LPG) {
+        if (i * LPG + J < 9) {
+          const float w[4] = {share<LPG, J>(pt.w[0]), share<LPG, J>(pt.w[1]), share<LPG, J>(pt.w[2]), share<LPG, J>(pt.w[3])};
+          gather(share<LPG, J>(pt.addr) + lane_bytes, w);
+        }
+      }
+    };
+    one(std::integral_constant<int, 0>{});
+    one(std::integral_constant<int, 1>{});
+    one(std::integral_constant<int, 2>{});
+    one(std::integral_constant<int, 3>{});
+    // one point at a time: left alone the compiler puts the sums off until all 72 vectors are in registers, and spills
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int c = 0; c < EPV; ++c) asm volatile("" : "+v"(acc[v][c]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // points outside the window, from memory: all lanes of a group take part, and read the point's offsets again
+  if constexpr (LPG >= 2) far |= (uint32_t)dpp_quad_xor1((int)far);
+  if constexpr (LPG >= 4) far |= (uint32_t)dpp_quad_xor2((int)far);
+  if (__any(far != 0)) {
+    const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
+    const uint32_t pix_bytes = (uint32_t)(p.G * p.D) * Tag::kBytes;
+    const uint32_t base = (uint32_t)t.b * (uint32_t)(p.H * p.W) * pix_bytes + (uint32_t)(g * p.D) * Tag::kBytes + (uint32_t)part * 32u;
+#pragma unroll 1
+    for (int k = 0; k < 9; ++k) {
+      if (((far >> k) & 1) == 0) continue;
+      float f3[3];
+      point_of_row<Tag>(row, k, f3);
+      const int i = exact_div(k, 1.f / 3.f), j = k - 3 * i;
+      const float x = add_rn(x_base, mul_rn(add_rn((float)i, f3[0]), p.offset_scale));
+      const float y = add_rn(y_base, mul_rn(add_rn((float)j, f3[1]), p.offset_scale));
+      const Tap tp = make_tap(y, x, p.H, p.W, base, pix_bytes);
+#pragma unroll
+      for (int cn = 0; cn < 4; ++cn)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          float f[EPV];
+          pack::decode(buffer_load<16>(value, tp.off[cn] + 16u * v), f);      // a dropped corner stays out of range
+          const float w = f3[2] * tp.w[cn];
+#pragma unroll
+          for (int c = 0; c < EPV; ++c) acc[v][c] = fmaf(w, f[c], acc[v][c]);
+        }
+    }
+  }
+  char *dst = static_cast<char *>(p.out) + (pixel * (size_t)(p.G * p.D) + (size_t)g * p.D) * Tag::kBytes + part * 32;
+#pragma unroll
+  for (int v = 0; v < 2; ++v) *reinterpret_cast<u32x4 *>(dst + 16 * v) = pack::encode(acc[v]);
+}
+
+// ------------------------------------------------------------------------------- backward
+// grad_offset_mask (the part of dcnv4_col2im_cuda.cuh:280-350 and common.h:188-211 that does not scatter): the four
+// corner . grad_out products of a point give d/dx, d/dy and d/dmask.  Where lanes share a group each forms the gradients of the
+// points it prepared.  The rows then go through LDS, in the window's place, so that they leave as whole runs; points outside the
+// window are served in between.  Also folds the reach that the grad_value kernel has to cover into GradState.
+template <typename Tag, int LPG, int UNITS>
+__global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_window_kernel(const DcnLaunch p) {
+  extern __shared__ u32x4 lds128[];
+  __shared__ uint32_t s_reach;
+  typedef typename RawWord<Tag::kBytes>::type elem_t;
+  constexpr int kGroups = UNITS / LPG, kCell = UNITS * 32;
+  char *lds = reinterpret_cast<char *>(lds128);
+  const WindowTile t = window_tile<kGroups>(p, blockIdx.x, gridDim.x);
+  const WindowFrame<UNITS> frame(t);
+  if (threadIdx.x == 0) s_reach = 0u;
+
+  constexpr int kPixels = kWindowThreads / UNITS, kPerGroup = kPixels * LPG;
+  const int gl = threadIdx.x / kPerGroup, part = threadIdx.x & (LPG - 1), q = threadIdx.x % kPerGroup / LPG;
+  const int py = exact_div(q, __builtin_amdgcn_rcpf((float)p.gt_w)), px = q - py * p.gt_w;
+  const bool active = py < t.th && px < t.tw && t.g0 + gl < p.G;
+  const int ho = t.oy0 + py, wo = t.ox0 + px;
+  const size_t pixel = active ? (size_t)t.b * p.Q + (size_t)ho * p.Wo + wo : 0;
+  const int g = active ? t.g0 + gl : 0;
+  const void *row = static_cast<const char *>(p.offset_mask) + (pixel * p.P_pad + (size_t)g * 27) * Tag::kBytes;
+  PointRows<Tag, LPG> rows;
+  rows.load(row, part);
+  u32x4 go_raw[2];
+  const char *go_src = static_cast<const char *>(p.grad_out) + (pixel * (size_t)(p.G * p.D) + (size_t)g * p.D) * Tag::kBytes + part * 32;
+#pragma unroll
+  for (int v = 0; v < 2; ++v) go_raw[v] = *reinterpret_cast<const u32x4 *>(go_src + 16 * v);
+  stage_window<Tag, UNITS>(p, t, lds);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  const int p0x = 1 - p.pw + wo, p0y = 1 - p.ph + ho;      // reference point
+  const float p0xf = (float)p0x, p0yf = (float)p0y;
+  const float x_base = sub_rn(p0xf, p.offset_scale), y_base = sub_rn(p0yf, p.offset_scale);
+  auto at = [&](int k, float ox, float oy, float &y, float &x) {
+    const int i = LPG == 1 ? k / 3 : exact_div(k, 1.f / 3.f), j = k - 3 * i;
+    x = add_rn(x_base, mul_rn(add_rn((float)i, ox), p.offset_scale));
+    y = add_rn(y_base, mul_rn(add_rn((float)j, oy), p.offset_scale));
+  };
+  // corner . grad_out over this lane's channels
+  auto dots = [&](auto fetch, float (&d)[4]) {
+    u32x4 raw[4][2];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) raw[cn][v] = fetch(cn, v);
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      float sum[2] = {0.f, 0.f};      // two running sums: consecutive instructions do not wait for each other
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const u32x4 a = raw[cn][v], b = go_raw[v];
+        if constexpr (Tag::kBytes == 2) {      // two channels per instruction, products and sums in fp32
+#pragma unroll
+          for (int c = 0; c < 4; ++c) sum[c & 1] = dot2_pair<Tag>(a[c], b[c], sum[c & 1]);
+        } else {
+          float fa[4], fb[4];
+          Pack<Tag, 4>::decode(a, fa);
+          Pack<Tag, 4>::decode(b, fb);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) sum[c & 1] = fmaf(fa[c], fb[c], sum[c & 1]);
+        }
+      }
+      d[cn] = sum[0] + sum[1];
+      if constexpr (LPG >= 2) d[cn] += dcn::dpp_quad_xor1(d[cn]);
+      if constexpr (LPG >= 4) d[cn] += dcn::dpp_quad_xor2(d[cn]);
+    }
+  };
+  auto gradients = [&](const float (&d)[4], float ly, float lx, float m, float (&r)[3]) {
+    const float hy = 1.f - ly, hx = 1.f - lx;
+    r[0] = (hy * (d[1] - d[0]) + ly * (d[3] - d[2])) * p.offset_scale * m;      // common.h:188-201
+    r[1] = (hx * (d[2] - d[0]) + lx * (d[3] - d[1])) * p.offset_scale * m;
+    r[2] = hy * hx * d[0] + hy * lx * d[1] + ly * hx * d[2] + ly * lx * d[3];
+  };
+
+  const int lane_bytes = (gl * LPG + part) * 32;
+  constexpr int kOwn = PointRows<Tag, LPG>::kOwn;
+  float result[kOwn][3];
+  uint32_t far = 0;
+  uint32_t reach_bits = 0;      // bits of the largest distance so far: non-negative floats order like their bits
+  if (active) {
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      const int k = LPG == 1 ? i : min(part + i * LPG, 8);
+      float ox, oy, y, x, m;
+      rows.get(i, ox, oy, m);
+      at(k, ox, oy, y, x);
+      const WindowPoint pt = window_point<UNITS>(frame, y, x, 1.f);
+      // Chebyshev distance of the point from its reference point: its ceiling is how far the weighted corners of its 2x2 block
+      // lie from it at most.  Points beyond the cap - which exceeds what a window covers - are folded where they are served.
+      bool counts = pt.ok;
+      if (!__all(pt.ok)) {
+        const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
+        far |= (uint32_t)(inside && !pt.ok) << k;
+        counts = inside;
+      }
+      const float dist = fmaxf(fabsf(x - p0xf), fabsf(y - p0yf));
+      reach_bits = max(reach_bits, (counts && dist <= p.gv_reach_cap) ? __builtin_bit_cast(uint32_t, dist) : 0u);
+      float d[4] = {0.f, 0.f, 0.f, 0.f};
+      auto one = [&](auto jj) {
+        constexpr int J = decltype(jj)::value;
+        if constexpr (J < LPG) {
+          if (i * LPG + J < 9) {
+            const char *src = lds + share<LPG, J>(pt.addr) + lane_bytes;
+            float dj[4];
+            dots([&](int cn, int v) { return *reinterpret_cast<const u32x4 *>(src + (cn & 1) * kCell + (cn >> 1) * frame.row_bytes + 16 * v); }, dj);
+#pragma unroll
+            for (int cn = 0; cn < 4; ++cn) d[cn] = LPG == 1 || part == J ? dj[cn] : d[cn];
+          }
+        }
+      };
+      one(std::integral_constant<int, 0>{});
+      one(std::integral_constant<int, 1>{});
+      one(std::integral_constant<int, 2>{});
+      one(std::integral_constant<int, 3>{});
+      gradients(d, pt.ly, pt.lx, m, result[i]);      // all zeros for a point outside the image or the window
+      // one point at a time, as in the forward
+#pragma unroll
+      for (int c = 0; c < 3; ++c) asm volatile("" : "+v"(result[i][c]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();      // nobody reads the window any more
+
+  // rows of 27 gradients in LDS, a run of kGroups of them per pixel
+  constexpr int kRun = kGroups * 27, kPitch = Tag::kBytes == 2 ? (kRun + 1) / 2 * 2 : kRun;      // elements: runs start on a word
+  elem_t *out = reinterpret_cast<elem_t *>(lds) + (size_t)q * kPitch + gl * 27;
+  auto put = [&](int k, const float (&r)[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const float f[1] = {r[c]};
+      out[c == 2 ? 18 + k : 2 * k + c] = Pack<Tag, 1>::encode(f);
+    }
+  };
+  if (active) {
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      const int k = part + i * LPG;
+      if (LPG == 1 || k < 9) put(k, result[i]);
+    }
+    if constexpr (LPG >= 2) far |= (uint32_t)dpp_quad_xor1((int)far);
+    if constexpr (LPG >= 4) far |= (uint32_t)dpp_quad_xor2((int)far);
+    if (__any(far != 0)) {
+      const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
+      const uint32_t pix_bytes = (uint32_t)(p.G * p.D) * Tag::kBytes;
+      const uint32_t base = (uint32_t)t.b * (uint32_t)(p.H * p.W) * pix_bytes + (uint32_t)(g * p.D) * Tag::kBytes + (uint32_t)part * 32u;
+#pragma unroll 1
+      for (int k = 0; k < 9; ++k) {
+        if (((far >> k) & 1) == 0) continue;
+        float f3[3], y, x, d[4], r[3];
+        point_of_row<Tag>(row, k, f3);
+        const int i = exact_div(k, 1.f / 3.f);
+        x = add_rn(x_base, mul_rn(add_rn((float)i, f3[0]), p.offset_scale));
+        y = add_rn(y_base, mul_rn(add_rn((float)(k - 3 * i), f3[1]), p.offset_scale));
+        const Tap tp = make_tap(y, x, p.H, p.W, base, pix_bytes);
+        if (tp.valid != 0 && fmaxf(fabsf(x - p0xf), fabsf(y - p0yf)) > p.gv_reach_cap) dcnv4_fold_far_point(p, t.b, g, tp.y0, tp.x0, p0y, p0x);
+        dots([&](int cn, int v) { return buffer_load<16>(value, tp.off[cn] + 16u * v); }, d);
+        gradients(d, tp.ly, tp.lx, f3[2], r);
+        if (part == k % LPG) put(k, r);
+      }
+    }
+  }
+  // the reach: fold in LDS, touch the global word only when it would grow
+  const uint32_t reach = wave_max_u32((uint32_t)min(ceilf(__builtin_bit_cast(float, reach_bits)), 1048576.f));
+  if ((threadIdx.x & (kWave - 1)) == 0 && reach != 0) atomicMax(&s_reach, reach);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t *dst = &p.state->reach_needed;
+    const uint32_t mine = s_reach;
+    if (mine > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, mine);
+  }
+  // runs to memory, a word a lane whatever the alignment, the last element of an odd run alone
+  const int groups = min(kGroups, p.G - t.g0), run = groups * 27;
+  char *gom = static_cast<char *>(p.grad_offset_mask) + (((size_t)t.b * p.Q + (size_t)t.oy0 * p.Wo + t.ox0) * p.P_pad + (size_t)t.g0 * 27) * Tag::kBytes;
+  constexpr int kPerWord = 4 / Tag::kBytes;
+  const int words = (run + kPerWord - 1) / kPerWord, total = t.th * t.tw * words;
+  const float inv_words = __builtin_amdgcn_rcpf((float)words), inv_tw = __builtin_amdgcn_rcpf((float)t.tw);
+  for (int idx = threadIdx.x; idx < total; idx += kWindowThreads) {
+    const int pix = exact_div(idx, inv_words), w = idx - pix * words;
+    const int y = exact_div(pix, inv_tw), x = pix - y * t.tw;
+    const elem_t *src = reinterpret_cast<const elem_t *>(lds) + (size_t)(y * p.gt_w + x) * kPitch + w * kPerWord;
+    char *dst = gom + (((size_t)y * p.Wo + x) * p.P_pad + (size_t)w * kPerWord) * Tag::kBytes;
+    if (w * kPerWord + kPerWord <= run) {
+      const uint32_t word = *reinterpret_cast<const uint32_t *>(src);
+      if constexpr (Tag::kBytes == 4) __builtin_nontemporal_store(word, reinterpret_cast<uint32_t *>(dst));
+      else __builtin_memcpy(dst, &word, 4);
+    } else {
+      *reinterpret_cast<elem_t *>(dst) = *src;
+    }
+  }
+  const int tail = p.P_pad - p.G * 27;
+  if (tail > 0 && t.g0 + groups == p.G) {
+    const float inv_tail = __builtin_amdgcn_rcpf((float)tail);
+    for (int idx = threadIdx.x; idx < t.th * t.tw * tail; idx += kWindowThreads) {
+      const int pix = exact_div(idx, inv_tail), e = idx - pix * tail;
+      const int y = exact_div(pix, inv_tw), x = pix - y * t.tw;
+      reinterpret_cast<elem_t *>(gom)[((size_t)y * p.Wo + x) * p.P_pad + run + e] = elem_t(0);
+    }
+  }
+}
+
+template <typename Tag, int LPG, int UNITS, bool BWD>
+hipError_t launch_units(const DcnLaunch &p, hipStream_t stream) {
+  constexpr int kGroups = UNITS / LPG;
+  const int Ho = p.Q / p.Wo;
+  const unsigned tiles = (unsigned)(p.n_pix / p.Q) * ((Ho + p.gt_h - 1) / p.gt_h) * ((p.Wo + p.gt_w - 1) / p.gt_w) * ((p.G + kGroups - 1) / kGroups);
+  auto go = [&](auto kernel) {
+    if (hipError_t e = ensure_dynamic_lds_limit(reinterpret_cast<const void *>(kernel), kMaxLdsPerWorkgroup - 1024)) return e;
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kWindowThreads), dcnv4_window_lds_bytes(p, UNITS), stream, p);
+    return hipGetLastError();
+  };
+  if constexpr (BWD) return go(dcnv4_offset_mask_grad_window_kernel<Tag, LPG, UNITS>);
+  else return go(dcnv4_forward_window_kernel<Tag, LPG, UNITS>);
+}
+
+template <typename Tag, int LPG, bool BWD>
+hipError_t launch_lpg(const DcnLaunch &p, int units, hipStream_t stream) {
+  if constexpr (LPG <= 1) if (units == 1) return launch_units<Tag, LPG, 1, BWD>(p, stream);
+  if constexpr (LPG <= 2) if (units == 2) return launch_units<Tag, LPG, 2, BWD>(p, stream);
+  if (units == 4) return launch_units<Tag, LPG, 4, BWD>(p, stream);
+  return hipErrorInvalidValue;
+}
+
+template <bool BWD>
+hipError_t launch_any(int dtype, const DcnLaunch &p, int units, hipStream_t stream) {
+  const int lpg = p.D * (dtype == F32::kCode ? 4 : 2) / 32;
+  if (dtype == F32::kCode) return lpg == 2 ? launch_lpg<F32, 2, BWD>(p, units, stream) : lpg == 4 ? launch_lpg<F32, 4, BWD>(p, units, stream) : hipErrorInvalidValue;
+  auto half = [&](auto tag) -> hipError_t {
+    typedef decltype(tag) T;
+    if (lpg == 1) return launch_lpg<T, 1, BWD>(p, units, stream);
+    if (lpg == 2) return launch_lpg<T, 2, BWD>(p, units, stream);
+    if (lpg == 4) return launch_lpg<T, 4, BWD>(p, units, stream);
+    return hipErrorInvalidValue;
+  };
+  return dtype == F16::kCode ? half(F16{}) : half(BF16{});
+}
+
+}  // namespace
+
+// LDS of a workgroup: the window and its zeros, in whole rounds of the loads that fill it, or the gradient rows that take its place
+// (28 16-bit or 27 fp32 elements of each pixel and group at most).
+size_t dcnv4_window_lds_bytes(const DcnLaunch &p, int units) {
+  const size_t pieces = (size_t)(p.gt_wh * p.gt_ww + p.gt_ww + 2) * units * 2;
+  return std::max((pieces + 63) / 64 * 64 * 16, (size_t)kWindowThreads * 56);
+}
+
+hipError_t launch_dcnv4_forward_window(int dtype, const DcnLaunch &p, int units, hipStream_t stream) {
+  return launch_any<false>(dtype, p, units, stream);
+}
+
+hipError_t launch_dcnv4_offset_mask_grad_window(int dtype, const DcnLaunch &p, int units, hipStream_t stream) {
+  return launch_any<true>(dtype, p, units, stream);
+}
+
+}  // namespace dcn

@@ -254,6 +254,10 @@ size_t dcnv4_grad_value_lds_bytes(const DcnLaunch &p);
 hipError_t launch_dcnv4_forward_tiled(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_offset_mask_grad_tiled(int dtype, const DcnLaunch &p, hipStream_t stream);
 size_t dcnv4_tiled_gather_lds_bytes(const DcnLaunch &p, int elem_bytes);
+// Window gathers (dcnv4_window.hip): workgroups of gt_h x gt_w pixels for `units` 32-byte units of a pixel's channels.
+hipError_t launch_dcnv4_forward_window(int dtype, const DcnLaunch &p, int units, hipStream_t stream);
+hipError_t launch_dcnv4_offset_mask_grad_window(int dtype, const DcnLaunch &p, int units, hipStream_t stream);
+size_t dcnv4_window_lds_bytes(const DcnLaunch &p, int units);
 hipError_t launch_fda_forward(int dtype, const FdaLaunch &p, hipStream_t stream);
 // Lanes of a workgroup that takes one head (measured on the 128x128 pyramid against 256: the first backward pass is
 // 2 % faster with 512 and slower with 1024; the forward 6 % faster with 1024 on 128-byte heads, unchanged on 64-byte ones)
