@@ -62,5 +62,6 @@ void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std
 
 extern PyMethodDef training_methods[];
 extern PyMethodDef attention_methods[];
+extern PyMethodDef convolution_methods[];
 
 }  // namespace dcn::binding

@@ -87,7 +87,8 @@ static struct PyModuleDef native_module = {PyModuleDef_HEAD_INIT, "_native", "Ho
 PyMODINIT_FUNC PyInit__native(void) {
   PyObject *m = PyModule_Create(&native_module);
   if (m == nullptr) return nullptr;
-  for (PyMethodDef *methods : {dcn::binding::module_methods, dcn::binding::layer_methods, dcn::binding::training_methods, dcn::binding::attention_methods})
+  for (PyMethodDef *methods : {dcn::binding::module_methods, dcn::binding::layer_methods, dcn::binding::training_methods, dcn::binding::attention_methods,
+                               dcn::binding::convolution_methods})
     if (PyModule_AddFunctions(m, methods) != 0) {
       Py_DECREF(m);
       return nullptr;

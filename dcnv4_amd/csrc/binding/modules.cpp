@@ -44,6 +44,11 @@ Tensor Module::parameter(const char *name) const {
   return p != nullptr && THPVariable_Check(p) ? THPVariable_Unpack(p) : Tensor();
 }
 
+Tensor Module::buffer(const char *name) const {
+  PyObject *b = o_ != nullptr ? item(item(dict_of(o_), "_buffers"), name) : nullptr;
+  return b != nullptr && THPVariable_Check(b) ? THPVariable_Unpack(b) : Tensor();
+}
+
 PyObject *Module::attribute(const char *name) const { return o_ != nullptr ? item(dict_of(o_), name) : nullptr; }
 
 long Module::integer(const char *name, long otherwise) const {
@@ -85,7 +90,7 @@ bool idle(const Module &m, ModuleKind kind) {
 namespace {
 
 constexpr const char *kKindNames[kModuleKinds] = {"Linear", "LayerNorm", "GELU", "Dropout", "Identity", "Conv2d", "Sequential", "DropPath",
-                                                   "DCNv4", "MLPLayer"};
+                                                   "DCNv4", "MLPLayer", "BatchNorm2d", "_ToChannelsFirst", "_ToChannelsLast"};
 
 // register_modules(*classes): each fills the kind of its name
 PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {

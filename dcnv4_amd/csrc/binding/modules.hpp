@@ -6,7 +6,8 @@
 namespace dcn::binding {
 
 // The classes that a layer is made of; a module of another class (a subclass, a wrapper) is left to Python.
-enum ModuleKind { kLinear, kLayerNorm, kGelu, kDropout, kIdentity, kConv2d, kSequential, kDropPath, kDCNv4, kMlp, kModuleKinds };
+enum ModuleKind { kLinear, kLayerNorm, kGelu, kDropout, kIdentity, kConv2d, kSequential, kDropPath, kDCNv4, kMlp, kBatchNorm2d, kToChannelsFirst,
+                  kToChannelsLast, kModuleKinds };
 
 class Module {
  public:
@@ -16,6 +17,7 @@ class Module {
   Module child(const char *name, ModuleKind kind) const;      // null unless there is one of exactly that class
   Module child(const char *name) const;
   Tensor parameter(const char *name) const;                   // undefined: absent or None
+  Tensor buffer(const char *name) const;
   PyObject *attribute(const char *name) const;                // borrowed; null: absent
   long integer(const char *name, long otherwise) const;
   double real(const char *name, double otherwise) const;

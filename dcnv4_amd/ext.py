@@ -14,7 +14,7 @@ from . import _lib
 
 _L = _lib.load()
 _native = _lib.load_native()
-_native.register_modules(nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Identity, nn.Conv2d, nn.Sequential)
+_native.register_modules(nn.Linear, nn.LayerNorm, nn.GELU, nn.Dropout, nn.Identity, nn.Conv2d, nn.Sequential, nn.BatchNorm2d)
 
 _DTYPES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
 

@@ -72,6 +72,10 @@ class StemLayer(nn.Module):
         self.norm2 = _norm(out_chans, norm_layer, "channels_first", "channels_last")
 
     def forward(self, x):
+        if x.is_cuda and not torch.is_grad_enabled():
+            y = ext._native.stem_inference(self, x)      # csrc/binding/convolutions.cpp
+            if y is not None:
+                return y
         # channels-last memory from the first convolution on: the NHWC view the blocks work on is then dense, so
         # every kernel after the stem sees contiguous rows of channels (no strided elementwise kernels, no copies)
         x = x.contiguous(memory_format=torch.channels_last)
@@ -87,6 +91,10 @@ class DownsampleLayer(nn.Module):
     def forward(self, x, shape):
         H, W = shape
         N, _, C = x.shape
+        if x.is_cuda and not torch.is_grad_enabled():
+            y = ext._native.downsample_inference(self, x, H, W)
+            if y is not None:
+                return y, ((H + 1) // 2, (W + 1) // 2)
         x = self.norm(self.conv(x.view(N, H, W, C).permute(0, 3, 1, 2)))
         H, W = x.size(2), x.size(3)
         return x.flatten(2).permute(0, 2, 1), (H, W)
@@ -150,7 +158,7 @@ class InternImageLayer(nn.Module):
 
 
 _ext_forward = ext.dcnv4_forward
-ext._native.register_modules(DropPath, DCNv4, MLPLayer)
+ext._native.register_modules(DropPath, DCNv4, MLPLayer, _ToChannelsFirst, _ToChannelsLast)
 
 
 class InternImageBlock(nn.Module):
@@ -245,7 +253,8 @@ class FlashInternImage(nn.Module):
         for level in self.levels:
             x, shape = level(x, shape)
         h, w = shape
-        x = self.conv_head(x.view(N, h, w, -1).permute(0, 3, 1, 2))
+        y = ext._native.head_inference(self.conv_head, x, h, w) if x.is_cuda and not torch.is_grad_enabled() else None
+        x = self.conv_head(x.view(N, h, w, -1).permute(0, 3, 1, 2)) if y is None else y.permute(0, 3, 1, 2)
         return torch.flatten(self.avgpool(x), 1)
 
     def forward(self, x):
