@@ -805,12 +805,13 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
     return rc;
   if (int rc = check_ptrs({value, offset_mask, output})) return rc;
   const int per = images_per_launch(pr, false);
-  // A small call is a chain of latencies: the direct kernel's lanes go to memory at once, where the others first stage a window
-  // behind a barrier.  Measured (fp16, us, direct against window): 4x56x56x64 (1.6 MB) 6.5 against 7.4, 1x100x152x64 (1.9 MB)
-  // 6.9 against 7.6, 6x56x56x64 (2.4 MB) 8.3 against 7.9, 4x64x64x128 (4.2 MB) 9.5 against 8.8; against the tiled kernel, which
-  // takes the other kernel shapes, they meet at about 3 MB.
+  // A small call is a chain of latencies: the small kernel asks for everything it needs at once (other kernel shapes and lanes:
+  // the direct one), where the others first stage a window behind a barrier.  Measured (fp16, us, small against window):
+  // 1x56x56x64 4.3 against 5.7, 4x56x56x64 (1.6 MB) 6.1 against 7.3, 2x64x64x128 (2.1 MB) 5.4 against 8.1, 6x56x56x64 (2.4 MB)
+  // 8.3 against 8.0, 4x64x64x128 (4.2 MB) 9.3 against 8.9.
   const bool small = g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 &&
                      (uint64_t)batch * pr.img_out_elems * pr.s <= kDirectForwardBytes;
+  const bool at_once = small && kernel_h == 3 && kernel_w == 3 && !remove_center && !softmax && pr.launch.lanes.cpt * pr.s == 16;
   const int window = small ? 0 : plan_window_gather(&pr.launch, pr.s, batch, false);
   const bool tiled = !small && window == 0 && plan_gather_tiles(&pr.launch, pr.s, false);
   for (int b0 = 0; b0 < batch; b0 += per) {
@@ -821,9 +822,10 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
     L.out = at(output, b0 * pr.img_out_elems, pr.s);
     L.value_bytes = (uint32_t)(nb * pr.img_elems * pr.s);
     L.n_pix = nb * L.Q;
-    const hipError_t e = window  ? launch_dcnv4_forward_window(dtype, L, window, static_cast<hipStream_t>(stream))
-                         : tiled ? launch_dcnv4_forward_tiled(dtype, L, static_cast<hipStream_t>(stream))
-                                 : launch_dcnv4_forward(dtype, L, static_cast<hipStream_t>(stream));
+    const hipError_t e = at_once ? launch_dcnv4_forward_small(dtype, L, static_cast<hipStream_t>(stream))
+                         : window ? launch_dcnv4_forward_window(dtype, L, window, static_cast<hipStream_t>(stream))
+                         : tiled  ? launch_dcnv4_forward_tiled(dtype, L, static_cast<hipStream_t>(stream))
+                                  : launch_dcnv4_forward(dtype, L, static_cast<hipStream_t>(stream));
     if (e) return hip_fail("dcnv4 forward launch", e);
   }
   return DCNV4_OK;

@@ -235,6 +235,7 @@ int depthwise_grad_weight_vector(int elem_bytes, int C, int k);
 int depthwise_grad_weight_pixel_lanes(int elem_bytes, int C, int k);
 hipError_t launch_depthwise_grad_weight_partials(int dtype, const DwLaunch &p, hipStream_t stream);
 hipError_t launch_depthwise_grad_weight_reduce(int dtype, const DwLaunch &p, hipStream_t stream);
+hipError_t launch_dcnv4_forward_small(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_forward(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_offset_mask_grad(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_grad_value(int dtype, const DcnLaunch &p, hipStream_t stream);
