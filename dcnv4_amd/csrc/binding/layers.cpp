@@ -156,14 +156,14 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
   void *stream = stream_of(x);
   const int64_t rows = (int64_t)batch * h * w, c = l.channels;
   Tensor out = at::empty(x.sizes(), x.options());
-  // intermediates, each on a 256-byte boundary: the depthwise output (or a normalised input), value and the operator's output,
-  // offset rows, a projection's output, the stream between the two halves; the MLP's hidden tensor takes the place of the first four
+  // intermediates, each on a 256-byte boundary: the depthwise output, value and the operator's output, offset rows, the stream
+  // between the two halves, a projection's output; the MLP's hidden tensor takes the place of the first four
   auto span = [](int64_t elements) { return (elements * 2 + 255) / 256 * 256; };
   const int64_t act = span(rows * c), om = span(rows * l.row), hid = span(rows * l.hidden);
-  const int64_t front = std::max(4 * act + om, hid);
+  const int64_t front = std::max(3 * act + om, hid);
   const Tensor ws = workspace((size_t)(front + 2 * act), x);
   char *base = static_cast<char *>(ws.data_ptr());
-  char *pre = base, *value = base + act, *sampled = base + 2 * act, *projected = base + 3 * act, *offsets = base + 4 * act;
+  char *pre = base, *value = base + act, *sampled = base + 2 * act, *offsets = base + 3 * act;
   char *hidden = base, *middle = base + front, *last = base + front + act;
   const void *in = x.const_data_ptr();
 
@@ -178,9 +178,21 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
     launch(code, p, stream);
   };
 
+  // a normalisation in front of a product, by the product's own kernel where that pays: launches are what a picture or two wait for
+  auto normed = [&](LinearLaunch &p, const NormParams &n, const Tensor &gamma, const void *residual, void *o) {
+    if (linear_takes_norm(p)) {
+      p.norm = {ptr(n.weight), ptr(n.bias), n.eps, residual, ptr(gamma), residual != nullptr ? o : nullptr};
+    } else {
+      norm(p.p[0].a, n, gamma, residual, o);
+      for (int i = 0; i < p.count; ++i) p.p[i].a = o;
+    }
+    launch(code, p, stream);
+  };
+
   // DCNv4 half
+  const bool norm_first = !l.post_norm && l.dw_kernel == 0;      // the normalised rows go into the projections alone
   const void *source = in;
-  if (!l.post_norm) {
+  if (!l.post_norm && !norm_first) {
     norm(in, l.norm1, Tensor(), nullptr, middle);
     source = middle;
   }
@@ -194,19 +206,21 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
   both.p[0] = {source, ptr(l.value_w), ptr(l.value_b), nullptr, nullptr, value, (int)c};
   both.p[1] = {offset_source, ptr(l.offset_w), ptr(l.offset_b), nullptr, nullptr, offsets, (int)l.row};
   both.count = 2; both.rows = rows; both.k = (int)c;
-  launch(code, both, stream);
+  if (norm_first) normed(both, l.norm1, Tensor(), nullptr, middle);
+  else launch(code, both, stream);
   check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
                              l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
+  LinearLaunch fc1 = {};
+  fc1.p[0] = {last, ptr(l.fc1_w), ptr(l.fc1_b), nullptr, nullptr, hidden, (int)l.hidden};
+  fc1.count = 1; fc1.rows = rows; fc1.k = (int)c; fc1.gelu = 1;
   if (l.post_norm) {
-    linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, projected);
-    norm(projected, l.norm1, l.gamma1, in, middle);
-    linear(middle, l.fc1_w, l.fc1_b, c, l.hidden, true, Tensor(), nullptr, hidden);
+    linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
+    normed(fc1, l.norm1, l.gamma1, in, middle);
     linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
     norm(last, l.norm2, l.gamma2, middle, out.data_ptr());
   } else {
     linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
-    norm(last, l.norm2, Tensor(), nullptr, middle);
-    linear(middle, l.fc1_w, l.fc1_b, c, l.hidden, true, Tensor(), nullptr, hidden);
+    normed(fc1, l.norm2, Tensor(), nullptr, middle);
     linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, l.gamma2, last, out.data_ptr());
   }
   return out;

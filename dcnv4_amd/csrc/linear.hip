@@ -8,9 +8,12 @@
 //    read has no bank conflicts.  The features are the rows of the matrix instruction's result, so a lane ends up with
 //    four consecutive features of one row and stores 8 bytes.
 //  linear_few_rows_kernel: a picture or two at the later stages, where a launch has a handful of tiles and its time is load
-//    latency.  A workgroup owns 32 rows x 32 features; its four waves share the depth between them, take their fragments
-//    straight from memory and meet in LDS once.
+//    latency.  A workgroup owns 32 rows x 32 features; its four or eight waves share the depth between them, take their fragments
+//    straight from memory and meet in LDS once.  What the epilogue reads is requested first.  With a layer normalisation in
+//    front the workgroup normalises its 32 rows itself, into LDS: each does so again for every 32 features, but a launch less
+//    is 3 us less for the device and as much for the host.
 #include "linear.hpp"
+#include "launch.hpp"
 #include "mfma.hpp"
 
 namespace dcn {
@@ -56,7 +59,8 @@ __device__ __forceinline__ void to_locations(const SamplingLocations &l, long lo
 // The epilogue for eight consecutive features of one row: 16 bytes in and out (32 of fp32).  EXTRA: with what training adds,
 // which costs the small tiles a third more registers.
 template <typename Tag, bool EXTRA>
-__device__ __forceinline__ void finish(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8]) {
+__device__ __forceinline__ void finish(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8],
+                                       const float *residual = nullptr) {      // residual: q.residual's values, where they are at hand
   const LinearProblem &q = p.p[which];
   if (col.has_bias)
 #pragma unroll
@@ -80,7 +84,10 @@ __device__ __forceinline__ void finish(const LinearLaunch &p, int which, const C
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] *= s;
   }
-  if (q.residual != nullptr) {
+  if (residual != nullptr) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += residual[c];
+  } else if (q.residual != nullptr) {
     float r[8];
     load8<Tag>(q.residual, at, r);
 #pragma unroll
@@ -188,59 +195,169 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
 }
 
 constexpr int kFewTile = 32;
+// Longest row that is normalised on its way in, and most 32 x 32 tiles.  FlashInternImage-T, 1 / 8 pictures of 224: at most 256
+// tiles 893 / 1366 us, 512 883 / 1367, 1024 893 / 1421, separate normalisations 1097 / 1417.
+constexpr int kNormTiles = 512;
+constexpr int kNormDepth = 512;
 
-template <typename Tag, bool EXTRA>
-__global__ void __launch_bounds__(256) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
+// bytes of a normalised row in LDS: an odd number of 16-byte units
+__host__ __device__ constexpr int norm_row_bytes(int k) { return k * 2 + 16; }
+
+__device__ __forceinline__ float sum_of_sixteen(float v) {      // aligned lanes of a wave
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));       // one away
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));       // two away
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));      // mirrored in eight
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, true));      // and in sixteen
+  return v;
+}
+
+// The tile's rows, normalised, into LDS: sixteen lanes a row, MOST vectors of it in each, everything requested at once.
+constexpr int kNormWaves = 8;
+template <typename Tag, int MOST>
+__device__ __forceinline__ void normalise_rows(const LinearLaunch &p, long long m0, int live_m, bool write_out, char *lds) {
+  const RowNorm &n = p.norm;
+  const int row = threadIdx.x / 16, part = threadIdx.x % 16, vectors = p.k / 8;
+  const size_t at = ((size_t)m0 + min(row, live_m - 1)) * p.k;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 raw[MOST], res[MOST], w[MOST], b[MOST], g[MOST];
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) {
+    const int i = part + u * 16;
+    raw[u] = res[u] = w[u] = b[u] = g[u] = zero;
+    if (i >= vectors) continue;
+    raw[u] = reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(p.p[0].a) + at)[i];
+    if (n.residual != nullptr) res[u] = reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(n.residual) + at)[i];
+    w[u] = static_cast<const u32x4 *>(n.weight)[i];
+    b[u] = static_cast<const u32x4 *>(n.bias)[i];
+    if (n.gamma != nullptr) g[u] = static_cast<const u32x4 *>(n.gamma)[i];
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) {
+    float f[8];
+    Pack<Tag, 8>::decode(raw[u], f);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) sum += f[c];
+  }
+  const float mean = sum_of_sixteen(sum) / (float)p.k;
+  float squares = 0.f;
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) {
+    if (part + u * 16 >= vectors) continue;
+    float f[8];
+    Pack<Tag, 8>::decode(raw[u], f);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) squares = fmaf(f[c] - mean, f[c] - mean, squares);
+  }
+  const float rstd = rsqrtf(sum_of_sixteen(squares) / (float)p.k + n.eps);
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) {
+    const int i = part + u * 16;
+    if (i >= vectors) continue;
+    float f[8], x[8];
+    Pack<Tag, 8>::decode(raw[u], f);
+    Pack<Tag, 8>::decode(w[u], x);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] = (f[c] - mean) * rstd * x[c];
+    Pack<Tag, 8>::decode(b[u], x);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] += x[c];
+    if (n.gamma != nullptr) {
+      Pack<Tag, 8>::decode(g[u], x);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) f[c] *= x[c];
+    }
+    Pack<Tag, 8>::decode(res[u], x);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] += x[c];
+    const u32x4 out = Pack<Tag, 8>::encode(f);
+    *reinterpret_cast<u32x4 *>(lds + row * norm_row_bytes(p.k) + i * 16) = out;
+    if (write_out && n.out != nullptr && row < live_m) reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(n.out) + at)[i] = out;
+  }
+}
+
+// NORM: vectors of a normalised row in a lane, 0 without normalisation
+template <typename Tag, int WAVES, bool EXTRA, int NORM>
+__global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
   constexpr int kBytes = Tag::kBytes;
-  __shared__ __align__(16) float part[4][kFewTile][kFewTile + 4];
+  extern __shared__ u32x4 lds[];
+  float (*part)[kFewTile][kFewTile + 4] = reinterpret_cast<float (*)[kFewTile][kFewTile + 4]>(lds);
+  char *rows = reinterpret_cast<char *>(part + WAVES);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tm = blockIdx.x / tiles_n;
   int tn = blockIdx.x % tiles_n;
   const int which = tn >= tiles_n0;
   const LinearProblem &q = p.p[which];
+  const int m0 = tm * kFewTile, k = p.k;
+  const int live_m = (int)min((long long)kFewTile, p.rows - m0);
+  const bool first_tile = tn == 0;
   if (which) tn -= tiles_n0;
-  const int m0 = tm * kFewTile, n0 = tn * kFewTile, k = p.k;
-  const int live_m = (int)min((long long)kFewTile, p.rows - m0), live_n = min(kFewTile, q.n - n0);
+  const int n0 = tn * kFewTile, live_n = min(kFewTile, q.n - n0);
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * kBytes, (uint32_t)live_m * k * kBytes);
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * kBytes, (uint32_t)live_n * k * kBytes);
   const int r16 = lane & 15, kb = lane >> 4;
   constexpr int kStep = 64 / kBytes;
   const int steps = (k + kStep - 1) / kStep;
 
-  f32x4 acc[2][2] = {};
-  // wave w takes every fourth 64 bytes of the depth
-#pragma unroll 4
-  for (int s = wave; s < steps; s += 4) {
-    const int kk = s * kStep + kb * (16 / kBytes);
-    u32x4 fm[2], fn[2];
+  // wave w takes every WAVES-th 64 bytes of the depth, two of them requested together (four: 1 % slower)
+  constexpr int kTogether = 2;
+  u32x4 fm[kTogether][2], fn[kTogether][2];
+  auto request = [&](int s0, const __amdgpu_buffer_rsrc_t &r, u32x4 (&f)[kTogether][2]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t off = (uint32_t)((j * 16 + r16) * k + kk) * kBytes;
-      fm[j] = buffer_load<16>(ra, kk < k ? off : kDropOffset);
-      fn[j] = buffer_load<16>(rw, kk < k ? off : kDropOffset);
+    for (int u = 0; u < kTogether; ++u) {
+      const int kk = (s0 + u * WAVES) * kStep + kb * (16 / kBytes);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) f[u][j] = buffer_load<16>(r, kk < k ? (uint32_t)((j * 16 + r16) * k + kk) * kBytes : kDropOffset);
+    }
+  };
+  request(wave, rw, fn);
+  if constexpr (NORM == 0) request(wave, ra, fm);
+  // what the epilogue needs, by the lanes that run it
+  const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
+  const bool finishes = threadIdx.x < 128 && row < live_m && n < live_n;
+  const Columns<Tag> columns(q, n0 + n, finishes);
+  float residual[8];
+  if (finishes && q.residual != nullptr) load8<Tag>(q.residual, (size_t)(m0 + row) * q.n + n0 + n, residual);
+  if constexpr (NORM > 0) {
+    normalise_rows<Tag, NORM>(p, m0, live_m, first_tile, rows);
+    __syncthreads();
+  }
+
+  f32x4 acc[2][2] = {};
+  for (int s0 = wave; s0 < steps; s0 += kTogether * WAVES) {
+    if (s0 != wave) {
+      request(s0, rw, fn);
+      if constexpr (NORM == 0) request(s0, ra, fm);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int u = 0; u < kTogether; ++u) {
+      if (s0 + u * WAVES >= steps) break;
+      if constexpr (NORM > 0) {
+        const int kk = (s0 + u * WAVES) * kStep + kb * (16 / kBytes);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[i], fm[j], acc[i][j]);
+        for (int j = 0; j < 2; ++j) fm[u][j] = kk < k ? *reinterpret_cast<const u32x4 *>(rows + (j * 16 + r16) * norm_row_bytes(k) + kk * 2) : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[u][i], fm[u][j], acc[i][j]);
+    }
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
   __syncthreads();
-  if (threadIdx.x >= 128) return;
-  const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
-  const Columns<Tag> columns(q, n0 + n, n < live_n);
+  if (!finishes) return;
   float v[8];
 #pragma unroll
   for (int c = 0; c < 8; c += 4) {
     f32x4 sum = *reinterpret_cast<const f32x4 *>(&part[0][row][n + c]);
 #pragma unroll
-    for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
+    for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
     v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
   }
-  if (row < live_m && n < live_n) finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v);
+  finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v, q.residual != nullptr ? residual : nullptr);
 }
 
 template <typename Tag, bool EXTRA, int BM, int BN, int WM, int WN>
@@ -253,12 +370,27 @@ hipError_t launch_tiled(const LinearLaunch &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename Tag, bool EXTRA>
-hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
+template <typename Tag, bool EXTRA, int WAVES, int NORM>
+hipError_t launch_few_waves(const LinearLaunch &p, hipStream_t stream) {
   const int tiles_m = (int)((p.rows + kFewTile - 1) / kFewTile), tiles_n0 = (p.p[0].n + kFewTile - 1) / kFewTile;
   const int tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kFewTile - 1) / kFewTile : 0);
-  hipLaunchKernelGGL((linear_few_rows_kernel<Tag, EXTRA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p, tiles_n0, tiles_n);
+  const auto kernel = linear_few_rows_kernel<Tag, WAVES, EXTRA, NORM>;
+  const size_t lds = (size_t)WAVES * kFewTile * (kFewTile + 4) * 4 + (NORM > 0 ? (size_t)kFewTile * norm_row_bytes(p.k) : 0);
+  if (NORM > 0)
+    if (hipError_t e = ensure_dynamic_lds_limit(reinterpret_cast<const void *>(kernel), 112 * 1024)) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(WAVES * 64), lds, stream, p, tiles_n0, tiles_n);
   return hipGetLastError();
+}
+
+// Eight waves where four would take more than four turns each (196 x 256 x 1024 8.4 -> 7.0 us; sixteen gain nothing further, the
+// bytes that a CU reads then bound it).
+template <typename Tag, bool EXTRA>
+hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
+  if constexpr (!EXTRA && Tag::kBytes == 2) {
+    if (p.norm.weight != nullptr) return p.k <= 256 ? launch_few_waves<Tag, false, kNormWaves, 2>(p, stream) : launch_few_waves<Tag, false, kNormWaves, 4>(p, stream);
+  }
+  const long long steps = (long long)p.k * Tag::kBytes / 64;
+  return steps <= 16 ? launch_few_waves<Tag, EXTRA, 4, 0>(p, stream) : launch_few_waves<Tag, EXTRA, 8, 0>(p, stream);
 }
 
 // Which kernel and tile: enough workgroups for the 256 CUs first, then the widest tile whose padding does not cost more
@@ -275,7 +407,7 @@ hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
     return n * ((p.rows + bm - 1) / bm);
   };
   // fp32 is bound by the matrix cores (157 TFLOP/s): the tile that spreads most evenly
-  if (tiles(64, 64) < 64) return launch_few<Tag, EXTRA>(p, stream);
+  if (tiles(64, 64) < 64 || p.norm.weight != nullptr) return launch_few<Tag, EXTRA>(p, stream);
   if constexpr (Tag::kBytes == 4) {
     return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
   } else {
@@ -292,6 +424,12 @@ hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
 bool linear_fits(int dtype, long long rows, int n, int k) {
   return (dtype == F32::kCode || dtype == F16::kCode || dtype == BF16::kCode) && rows > 0 && n > 0 && k > 0 && n % 8 == 0 && k % 8 == 0 && k <= (1 << 20) &&
          rows * (long long)n < (1ll << 42) && (rows + 63) / 64 * ((n + 63) / 64) < (1ll << 30);
+}
+
+bool linear_takes_norm(const LinearLaunch &p) {
+  long long tiles = 0;
+  for (int i = 0; i < p.count; ++i) tiles += (p.p[i].n + kFewTile - 1) / kFewTile;
+  return p.k <= kNormDepth && tiles * ((p.rows + kFewTile - 1) / kFewTile) <= kNormTiles;
 }
 
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream) {

@@ -31,6 +31,15 @@ struct SamplingLocations {
   int kind, levels, points;    // kind 0: no locations; points a multiple of 4
 };
 
+// A layer normalisation of the products' rows on their way in, each rounded to the type: norm(a), or residual + gamma * norm(a),
+// which also goes to out.  Few rows only (linear_takes_norm), 16-bit types.
+struct RowNorm {
+  const void *weight, *bias;      // null: no normalisation
+  float eps;
+  const void *residual, *gamma;   // gamma may be null
+  void *out;
+};
+
 // Up to two products over the same rows and depth in one launch (a layer's value and offset projections).
 struct LinearLaunch {
   LinearProblem p[2];
@@ -38,11 +47,14 @@ struct LinearLaunch {
   long long rows;
   int k;
   int gelu;              // act: the exact GELU, else none
+  RowNorm norm;          // of p[0].a, which is p[1].a too
   SamplingLocations locations;
 };
 
 // Whether the matrix kernels take a product: depth and width in multiples of 8.
 bool linear_fits(int dtype, long long rows, int n, int k);
+// Whether the rows may come normalised: few enough that a workgroup normalising its own costs less than a launch.
+bool linear_takes_norm(const LinearLaunch &p);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
 
 // grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k] (and grad_bias[n], may be null), several products over the same
