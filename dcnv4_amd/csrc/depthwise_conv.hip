@@ -242,11 +242,11 @@ __global__ void __launch_bounds__(kDwThreads) dwconv_grad_weight_kernel(const Dw
   }
 }
 
-// grad_weight[c][tap] and grad_bias[c] from the partial sums.  A workgroup takes 16 consecutive
-// (tap, channel) entries; THREADS / 16 lanes per entry each add every so-manieth partial sum, then the first lane
-// adds the lane sums in index order: a fixed order whatever the schedule.  64 lanes per entry when there are few
-// entries (112 channels: 0.110 -> 0.103 ms for the whole backward), 16 otherwise.
-constexpr int kReduceEntries = 16;
+// grad_weight[c][tap] and grad_bias[c] from the partial sums.  A workgroup takes 32 consecutive
+// (tap, channel) entries - a line of memory a partial sum: half lines took 13.0 us at 12544 x 448, lines 8.1 -; THREADS / 32
+// lanes per entry each add every so-manieth partial sum, then the first lane adds the lane sums in index order: a fixed order
+// whatever the schedule.  32 lanes per entry when there are few entries, 8 otherwise.
+constexpr int kReduceEntries = 32;
 
 template <typename Tag, int THREADS>
 __global__ void __launch_bounds__(THREADS) dwconv_reduce_kernel(const DwLaunch p, int taps, int n_part) {
@@ -321,7 +321,7 @@ template <typename Tag>
 hipError_t reduce_t(const DwLaunch &p, hipStream_t stream) {
   const int taps = p.kh * p.kw, n = (taps + 1) * p.C;
   const dim3 grid((unsigned)((n + kReduceEntries - 1) / kReduceEntries));
-  if (n <= 3072) hipLaunchKernelGGL((dwconv_reduce_kernel<Tag, 1024>), grid, dim3(1024), 0, stream, p, taps, p.n_part);
+  if (n <= 6144) hipLaunchKernelGGL((dwconv_reduce_kernel<Tag, 1024>), grid, dim3(1024), 0, stream, p, taps, p.n_part);
   else hipLaunchKernelGGL((dwconv_reduce_kernel<Tag, 256>), grid, dim3(256), 0, stream, p, taps, p.n_part);
   return hipGetLastError();
 }

@@ -296,19 +296,26 @@ __global__ void __launch_bounds__(kLnThreads) layer_norm_residual_backward_kerne
   }
 }
 
-// partial [n_part][3][C] -> grad_weight, grad_bias, grad_gamma.  A workgroup takes 8 columns; its 128 row lanes each add
-// every 128th partial row (independent loads, many in flight), then the row lanes meet through LDS in lane order: a fixed
+// partial [n_part][3][C] -> grad_weight, grad_bias, grad_gamma.  A workgroup takes 32 columns, a line of memory of each
+// row; its 32 row lanes each add every 32nd partial row (independent loads, four in flight), then the row lanes meet through LDS in lane order: a fixed
 // summation tree, so the result does not depend on scheduling.
-constexpr int kPgCols = 8, kPgRows = 128;
+constexpr int kPgCols = 32, kPgRows = 32;
 template <typename Tag>
 __global__ void __launch_bounds__(kPgCols * kPgRows) layer_norm_param_grad_kernel(const LnLaunch p) {
   __shared__ float s_part[kPgRows][kPgCols + 1];
   const int col = threadIdx.x % kPgCols, rl = threadIdx.x / kPgCols;
   const int idx = blockIdx.x * kPgCols + col;                   // column of the [3][C] row
-  float acc = 0.f;
-  if (idx < 3 * p.C)
-    for (int w = rl; w < p.n_part; w += kPgRows) acc += p.partial[(size_t)w * 3 * p.C + idx];
-  s_part[rl][col] = acc;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  if (idx < 3 * p.C) {
+    const float *src = p.partial + idx;
+    const size_t step = (size_t)3 * p.C;
+    int w = rl;
+    for (; w + 3 * kPgRows < p.n_part; w += 4 * kPgRows)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] += src[(size_t)(w + u * kPgRows) * step];
+    for (; w < p.n_part; w += kPgRows) acc[0] += src[(size_t)w * step];
+  }
+  s_part[rl][col] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   __syncthreads();
   if (rl != 0 || idx >= 3 * p.C) return;
   float total = 0.f;

@@ -181,6 +181,37 @@ __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaun
   const CastWeights &q = p.p[which];
   const int local = blockIdx.x - (which ? p.tile_end[which - 1] : 0), tiles_k = (q.k + 63) / 64;
   const int n0 = local / tiles_k * 64, k0 = local % tiles_k * 64;
+  if (q.k % 4 == 0 && (q.turned == nullptr || q.n % 4 == 0)) {      // four columns a lane: 16 bytes in, a row's piece or a turned one out
+    const int c4 = (threadIdx.x & 15) * 4;
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int n = n0 + u * 16 + (threadIdx.x >> 4);
+      v[u] = n < q.n && k0 + c4 < q.k ? *reinterpret_cast<const f32x4 *>(q.from + (size_t)n * q.k + k0 + c4) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    typedef typename Pack<Tag, 4>::raw_t raw_t;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = u * 16 + (threadIdx.x >> 4), n = n0 + r;
+      const float f[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      const raw_t h = Pack<Tag, 4>::encode(f);
+      if (q.to != nullptr && n < q.n && k0 + c4 < q.k) *reinterpret_cast<raw_t *>(static_cast<elem_t *>(q.to) + (size_t)n * q.k + k0 + c4) = h;
+      __builtin_memcpy(&tile[r][c4], &h, sizeof(h));
+    }
+    if (q.turned == nullptr) return;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = u * 16 + (threadIdx.x >> 4), k = k0 + r;
+      elem_t e[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) e[c] = tile[c4 + c][r];
+      raw_t h;
+      __builtin_memcpy(&h, e, sizeof(h));
+      if (k < q.k && n0 + c4 < q.n) *reinterpret_cast<raw_t *>(static_cast<elem_t *>(q.turned) + (size_t)k * q.n + n0 + c4) = h;
+    }
+    return;
+  }
   const int col = threadIdx.x & 63;
 #pragma unroll 4
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
