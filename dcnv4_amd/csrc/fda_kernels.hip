@@ -173,58 +173,125 @@ __device__ __forceinline__ void quad_softmax_stats(const float *m, int n, int my
   inv = 1.f / sum;
 }
 
-// The K points of level l for one lane.  base: byte offset of the level's pixel 0 for this (image, head), without
+// The softmax and sampling points of a (query, head) with four levels of four points, a lane's share of them - point my_k of every
+// level - from memory straight into its registers: no staging of rows, and every exponential once.  The staged forward, which is
+// bound by its vector instructions (277 -> 225 for 64 points), took 146 -> 140 us with it for 4 images of 128x128.., 8 heads of
+// 32, fp16, inputs not in a cache.
+constexpr int kFour = 4;
+template <typename Tag>
+struct QuadRow {
+  typedef typename RawWord<Tag::kBytes>::type elem_t;
+  uint32_t xy[kFour][2];      // raw: one word of 16-bit pairs, two of fp32
+  uint32_t logit[kFour];
+
+  __device__ __forceinline__ void request(const FdaLaunch &p, size_t row, int g, int my_k) {
+    const size_t at = row * p.G + g;
+    const bool packed = p.loc == nullptr, wide = packed ? Tag::kBytes == 4 : p.loc_f32 != 0;
+    const char *loc = packed ? static_cast<const char *>(p.sla) + (at * 48 + 2 * my_k) * Tag::kBytes
+                             : static_cast<const char *>(p.loc) + (at * 32 + 2 * my_k) * (wide ? 4 : Tag::kBytes);
+    const elem_t *w = packed ? static_cast<const elem_t *>(p.sla) + at * 48 + 32 + my_k : static_cast<const elem_t *>(p.logits) + at * 16 + my_k;
+#pragma unroll
+    for (int l = 0; l < kFour; ++l) {
+      if (wide) {
+        const u32x2 v = *reinterpret_cast<const u32x2 *>(loc + l * 32);
+        xy[l][0] = v.x; xy[l][1] = v.y;
+      } else {
+        xy[l][0] = *reinterpret_cast<const uint32_t *>(loc + l * 16);
+      }
+      logit[l] = w[4 * l];
+    }
+  }
+  // locations and probabilities
+  __device__ __forceinline__ void unpack(const FdaLaunch &p, float (&x)[kFour], float (&y)[kFour], float (&pr)[kFour]) const {
+    const bool packed = p.loc == nullptr, wide = packed ? Tag::kBytes == 4 : p.loc_f32 != 0;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int l = 0; l < kFour; ++l) {
+      if (wide) {
+        x[l] = __builtin_bit_cast(float, xy[l][0]); y[l] = __builtin_bit_cast(float, xy[l][1]);
+      } else if constexpr (Tag::kBytes == 2) {
+        float f[2];
+        Pack<Tag, 2>::decode(xy[l][0], f);
+        x[l] = f[0]; y[l] = f[1];
+      }
+      if (!packed) { x[l] = (float)(_Float16)x[l]; y[l] = (float)(_Float16)y[l]; }      // as fda_stage_rows
+      float one[1];
+      Pack<Tag, 1>::decode((elem_t)logit[l], one);
+      pr[l] = one[0];
+      mx = fmaxf(mx, one[0]);
+    }
+    mx = fmaxf(mx, dpp_quad_xor1(mx));
+    mx = fmaxf(mx, dpp_quad_xor2(mx));
+    float sum = 0.f;
+#pragma unroll
+    for (int l = 0; l < kFour; ++l) sum += pr[l] = __expf(pr[l] - mx);
+    sum += dpp_quad_xor1(sum);
+    sum += dpp_quad_xor2(sum);
+    const float inv = 1.f / sum;
+#pragma unroll
+    for (int l = 0; l < kFour; ++l) pr[l] *= inv;
+  }
+};
+
+// Four points, one prepared by each lane of the quad.  base: byte offset of the level's pixel 0 for this (image, head), without
 // the lane's channels; staged: the level lies in LDS at s_stage + base, with one head's width of zero bytes at s_stage
 // for corners outside the level (a lane's channel offset stays inside them).
+template <typename Tag, int CPT>
+__device__ __forceinline__ void fda_quad_points(float (&acc)[CPT], float loc_x, float loc_y, float pr, const Level &lv, uint32_t base,
+                                                uint32_t step, uint32_t lane_off, bool staged, const char *s_stage,
+                                                const __amdgpu_buffer_rsrc_t &value) {
+  typedef Pack<Tag, CPT> pack;
+  typedef typename pack::raw_t raw_t;
+  const float x = sub_rn(mul_rn(loc_x, (float)lv.W), 0.5f);       // flash_deform_im2col_cuda.cuh:188-189
+  const float y = sub_rn(mul_rn(loc_y, (float)lv.H), 0.5f);
+  const Tap tp = make_tap(y, x, lv.H, lv.W, base, step);
+  int wq[4], oq[4];
+#pragma unroll
+  for (int cn = 0; cn < 4; ++cn) {
+    wq[cn] = __builtin_bit_cast(int, pr * tp.w[cn]);
+    oq[cn] = (int)((staged && !((tp.valid >> cn) & 1u)) ? 0u : tp.off[cn]);
+  }
+  raw_t raw[4][4];
+  float w[4][4];
+  if (staged) {
+    static_for(std::make_integer_sequence<int, 4>{}, [&](auto j) {
+      constexpr int J = decltype(j)::value;
+#pragma unroll
+      for (int cn = 0; cn < 4; ++cn) {
+        w[J][cn] = __builtin_bit_cast(float, quad_pick<J>(wq[cn]));
+        raw[J][cn] = *reinterpret_cast<const raw_t *>(s_stage + ((uint32_t)quad_pick<J>(oq[cn]) + lane_off));
+      }
+    });
+  } else {
+    static_for(std::make_integer_sequence<int, 4>{}, [&](auto j) {
+      constexpr int J = decltype(j)::value;
+#pragma unroll
+      for (int cn = 0; cn < 4; ++cn) {
+        w[J][cn] = __builtin_bit_cast(float, quad_pick<J>(wq[cn]));
+        raw[J][cn] = buffer_load<pack::kBytes>(value, (uint32_t)quad_pick<J>(oq[cn]) + lane_off);
+      }
+    });
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      float v[CPT];
+      pack::decode(raw[j][cn], v);
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) acc[c] = fmaf(w[j][cn], v[c], acc[c]);
+    }
+}
+
+// The K points of level l for one lane, from its row in LDS.
 template <typename Tag, int CPT>
 __device__ __forceinline__ void fda_quad_level(float (&acc)[CPT], const float *s, int LK, int K, int l, const Level &lv,
                                                float mx, float inv, uint32_t base, uint32_t step, uint32_t lane_off,
                                                int my_k, bool staged, const char *s_stage,
                                                const __amdgpu_buffer_rsrc_t &value) {
-  typedef Pack<Tag, CPT> pack;
-  typedef typename pack::raw_t raw_t;
   for (int k0 = 0; k0 < K; k0 += 4) {
     const int t = l * K + k0 + my_k;
-    const float x = sub_rn(mul_rn(s[2 * t], (float)lv.W), 0.5f);       // flash_deform_im2col_cuda.cuh:188-189
-    const float y = sub_rn(mul_rn(s[2 * t + 1], (float)lv.H), 0.5f);
-    const float pr = __expf(s[2 * LK + t] - mx) * inv;
-    const Tap tp = make_tap(y, x, lv.H, lv.W, base, step);
-    int wq[4], oq[4];
-#pragma unroll
-    for (int cn = 0; cn < 4; ++cn) {
-      wq[cn] = __builtin_bit_cast(int, pr * tp.w[cn]);
-      oq[cn] = (int)((staged && !((tp.valid >> cn) & 1u)) ? 0u : tp.off[cn]);
-    }
-    raw_t raw[4][4];
-    float w[4][4];
-    if (staged) {
-      static_for(std::make_integer_sequence<int, 4>{}, [&](auto j) {
-        constexpr int J = decltype(j)::value;
-#pragma unroll
-        for (int cn = 0; cn < 4; ++cn) {
-          w[J][cn] = __builtin_bit_cast(float, quad_pick<J>(wq[cn]));
-          raw[J][cn] = *reinterpret_cast<const raw_t *>(s_stage + ((uint32_t)quad_pick<J>(oq[cn]) + lane_off));
-        }
-      });
-    } else {
-      static_for(std::make_integer_sequence<int, 4>{}, [&](auto j) {
-        constexpr int J = decltype(j)::value;
-#pragma unroll
-        for (int cn = 0; cn < 4; ++cn) {
-          w[J][cn] = __builtin_bit_cast(float, quad_pick<J>(wq[cn]));
-          raw[J][cn] = buffer_load<pack::kBytes>(value, (uint32_t)quad_pick<J>(oq[cn]) + lane_off);
-        }
-      });
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int cn = 0; cn < 4; ++cn) {
-        float v[CPT];
-        pack::decode(raw[j][cn], v);
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) acc[c] = fmaf(w[j][cn], v[c], acc[c]);
-      }
+    fda_quad_points<Tag, CPT>(acc, s[2 * t], s[2 * t + 1], __expf(s[2 * LK + t] - mx) * inv, lv, base, step, lane_off, staged, s_stage, value);
   }
 }
 
@@ -304,7 +371,7 @@ __device__ __forceinline__ float fda_quad_level_backward(const float (&go)[CPT],
 }
 
 // ------------------------------------------------------------------------------- forward
-template <typename Tag, int CPT, int KT, bool QUAD>
+template <typename Tag, int CPT, int KT, bool QUAD, bool FOUR>      // FOUR: QUAD, four levels of four points
 __global__ void __launch_bounds__(kFdaForwardThreads) fda_forward_kernel(const FdaLaunch p) {
   extern __shared__ float lds[];
   typedef Pack<Tag, CPT> pack;
@@ -327,8 +394,10 @@ __global__ void __launch_bounds__(kFdaForwardThreads) fda_forward_kernel(const F
     row0 = (int)blk * p.nq_block;
     nrow = min(p.nq_block, p.n_row - row0);
   }
-  fda_stage_rows<Tag>(lds, p, row0, nrow, g_fixed, heads_here);
-  __syncthreads();
+  if constexpr (!FOUR) {
+    fda_stage_rows<Tag>(lds, p, row0, nrow, g_fixed, heads_here);
+    __syncthreads();
+  }
 
   const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
   const int tpgp_log2 = p.lanes.tpgp_log2;
@@ -347,7 +416,22 @@ __global__ void __launch_bounds__(kFdaForwardThreads) fda_forward_kernel(const F
 #pragma unroll
     for (int c = 0; c < CPT; ++c) acc[c] = 0.f;
     float mx, inv;
-    if constexpr (QUAD) {
+    if constexpr (FOUR) {
+      const uint32_t lane_off = (uint32_t)(chunk * CPT) * Tag::kBytes;
+      QuadRow<Tag> row;
+      float x[kFour], y[kFour], pr[kFour];
+      row.request(p, (size_t)(row0 + lr), g, chunk & 3);
+      row.unpack(p, x, y, pr);
+#pragma unroll
+      for (int l = 0; l < kFour; ++l) {
+        const Level lv = load_level(p, l);
+        const uint32_t base = (uint32_t)(b * p.N + lv.start) * pix_bytes + (uint32_t)(g * p.D) * Tag::kBytes;
+        fda_quad_points<Tag, CPT>(acc, x[l], y[l], pr[l], lv, base, pix_bytes, lane_off, false, nullptr, value);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) asm volatile("" : "+v"(acc[c]));      // as in the staged kernel
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else if constexpr (QUAD) {
       const int my_k = chunk & 3;
       quad_softmax_stats(s + 2 * LK, LK, my_k, mx, inv);
       const uint32_t lane_off = (uint32_t)(chunk * CPT) * Tag::kBytes;
@@ -396,7 +480,7 @@ __global__ void __launch_bounds__(kFdaForwardThreads) fda_forward_kernel(const F
 // own 64 lanes' queries (no workgroup barriers); sampling points on a staged level are served from LDS, the others from
 // memory as in fda_forward_kernel.  Same arithmetic in the same order per
 // (query, head): identical results.  Which levels fit is decided on the device from spatial_shapes.
-template <typename Tag, int CPT, int KT, bool QUAD>
+template <typename Tag, int CPT, int KT, bool QUAD, bool FOUR>      // FOUR: QUAD, four levels of four points
 __global__ void __launch_bounds__(kFdaStagedThreads) fda_forward_staged_kernel(const FdaLaunch p) {
   extern __shared__ float lds[];
   __shared__ int s_level_off[kMaxLevels];       // byte offset of a staged level in the stage area, -1: not staged
@@ -452,6 +536,43 @@ __global__ void __launch_bounds__(kFdaStagedThreads) fda_forward_staged_kernel(c
   const int qpw = kWave >> tpgp_log2;
   const int chunk = lane & ((1 << tpgp_log2) - 1), lr = lane >> tpgp_log2;
   const uint32_t lane_off = (uint32_t)(chunk * CPT) * Tag::kBytes;
+  constexpr int kQueryStep = kFdaStagedThreads / kWave;
+  if constexpr (FOUR) {
+    if (chunk >= p.lanes.tpg) return;
+    Level level[kFour];
+    int stage_off[kFour];
+#pragma unroll
+    for (int l = 0; l < kFour; ++l) {
+      const Level lv = load_level(p, l);
+      level[l] = {__builtin_amdgcn_readfirstlane(lv.H), __builtin_amdgcn_readfirstlane(lv.W), __builtin_amdgcn_readfirstlane(lv.start)};
+      stage_off[l] = __builtin_amdgcn_readfirstlane(s_level_off[l]);
+    }
+    QuadRow<Tag> row;
+    int q = q_begin + wave * qpw + lr;
+    row.request(p, (size_t)b * p.Q + min(q, q_end - 1), g, chunk & 3);
+    for (int q0 = q_begin + wave * qpw; q0 < q_end; q0 += kQueryStep * qpw, q += kQueryStep * qpw) {
+      float x[kFour], y[kFour], pr[kFour], acc[CPT];
+      row.unpack(p, x, y, pr);
+      row.request(p, (size_t)b * p.Q + min(q + kQueryStep * qpw, q_end - 1), g, chunk & 3);      // the next query's, while this one is sampled
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) acc[c] = 0.f;
+#pragma unroll
+      for (int l = 0; l < kFour; ++l) {
+        const bool staged = stage_off[l] >= 0;
+        const uint32_t base = staged ? (uint32_t)stage_off[l] : (uint32_t)(b * p.N + level[l].start) * pix_bytes + (uint32_t)g * head_bytes;
+        fda_quad_points<Tag, CPT>(acc, x[l], y[l], pr[l], level[l], base, staged ? head_bytes : pix_bytes, lane_off, staged, s_stage, value);
+        // a level at a time: left alone the compiler puts the sums off to the end, and spills
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) asm volatile("" : "+v"(acc[c]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (q < q_end) {
+        char *dst = (char *)p.out + ((size_t)(b * p.Q + q) * (p.G * p.D) + g * p.D + chunk * CPT) * Tag::kBytes;
+        *reinterpret_cast<typename pack::raw_t *>(dst) = pack::encode(acc);
+      }
+    }
+    return;
+  }
   float *rows = lds + (size_t)wave * qpw * row_len;
   constexpr int EPV = 16 / Tag::kBytes;
   const bool vec_rows = p.loc == nullptr && (row_len % EPV) == 0;
@@ -760,9 +881,10 @@ hipError_t launch_staged(const FdaLaunch &p, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
     return hipGetLastError();
   };
-  if (fda_quad_setup(p)) return go(fda_forward_staged_kernel<Tag, CPT, 0, true>);
-  if (p.K == 4) return go(fda_forward_staged_kernel<Tag, CPT, 4, false>);
-  return go(fda_forward_staged_kernel<Tag, CPT, 0, false>);      // (unrolled for 8 points the kernel spills a hundred registers)
+  if (fda_quad_setup(p) && p.L == kFour && p.K == kFour) return go(fda_forward_staged_kernel<Tag, CPT, 0, true, true>);
+  if (fda_quad_setup(p)) return go(fda_forward_staged_kernel<Tag, CPT, 0, true, false>);
+  if (p.K == 4) return go(fda_forward_staged_kernel<Tag, CPT, 4, false, false>);
+  return go(fda_forward_staged_kernel<Tag, CPT, 0, false, false>);      // (unrolled for 8 points the kernel spills a hundred registers)
 }
 
 template <typename Tag, int CPT, int MODE>      // MODE -1: forward
@@ -773,11 +895,18 @@ hipError_t launch_k(const FdaLaunch &p, hipStream_t stream, dim3 grid, dim3 bloc
 #define FDA_LAUNCH(KT)                                                                                     \
   do {                                                                                                     \
     if constexpr (MODE >= 0) hipLaunchKernelGGL((fda_backward_kernel<Tag, CPT, KT, MODE, false>), grid, block, lds, stream, p); \
-    else hipLaunchKernelGGL((fda_forward_kernel<Tag, CPT, KT, false>), grid, block, lds, stream, p);       \
+    else hipLaunchKernelGGL((fda_forward_kernel<Tag, CPT, KT, false, false>), grid, block, lds, stream, p);       \
   } while (0)
   if constexpr (MODE < 0) {
+    // Calls that leave the chip half empty: a chain of latencies, one fewer.  Larger ones are bound by the answers of the L2 and want
+    // the waves that fewer registers leave room for: 2 images of 100x152.., 8 heads of 32, four levels of four points, fp32, 300
+    // queries 11.4 -> 7.6 us, 3000 queries 25.7 -> 29.9, every pixel 116 -> 130.
+    if (fda_quad_setup(p) && p.L == kFour && p.K == kFour && ((long long)p.n_row * p.G << p.lanes.tpgp_log2) <= 128 * 1024) {
+      hipLaunchKernelGGL((fda_forward_kernel<Tag, CPT, 0, true, true>), grid, block, 0, stream, p);
+      return hipGetLastError();
+    }
     if (fda_quad_setup(p)) {
-      hipLaunchKernelGGL((fda_forward_kernel<Tag, CPT, 0, true>), grid, block, lds, stream, p);
+      hipLaunchKernelGGL((fda_forward_kernel<Tag, CPT, 0, true, false>), grid, block, lds, stream, p);
       return hipGetLastError();
     }
   }
