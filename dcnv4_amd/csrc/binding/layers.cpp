@@ -210,18 +210,33 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
   else launch(code, both, stream);
   check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
                              l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
+  const bool fused = mlp_fits(code, rows, (int)c, (int)l.hidden);      // the MLP in one kernel
+  auto mlp = [&](const Tensor &gamma, const void *residual, void *o) {
+    const MlpLaunch m = {middle, ptr(l.fc1_w), ptr(l.fc1_b), ptr(l.fc2_w), ptr(l.fc2_b), ptr(gamma), residual, o, rows, (int)c, (int)l.hidden};
+    hip_check(launch_mlp(code, m, static_cast<hipStream_t>(stream)), "MLP launch");
+  };
   LinearLaunch fc1 = {};
   fc1.p[0] = {last, ptr(l.fc1_w), ptr(l.fc1_b), nullptr, nullptr, hidden, (int)l.hidden};
   fc1.count = 1; fc1.rows = rows; fc1.k = (int)c; fc1.gelu = 1;
   if (l.post_norm) {
     linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
-    normed(fc1, l.norm1, l.gamma1, in, middle);
-    linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
+    if (fused) {
+      norm(last, l.norm1, l.gamma1, in, middle);
+      mlp(Tensor(), nullptr, last);
+    } else {
+      normed(fc1, l.norm1, l.gamma1, in, middle);
+      linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
+    }
     norm(last, l.norm2, l.gamma2, middle, out.data_ptr());
   } else {
     linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
-    normed(fc1, l.norm2, Tensor(), nullptr, middle);
-    linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, l.gamma2, last, out.data_ptr());
+    if (fused) {
+      norm(last, l.norm2, Tensor(), nullptr, middle);
+      mlp(l.gamma2, last, out.data_ptr());
+    } else {
+      normed(fc1, l.norm2, Tensor(), nullptr, middle);
+      linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, l.gamma2, last, out.data_ptr());
+    }
   }
   return out;
 }

@@ -57,6 +57,18 @@ bool linear_fits(int dtype, long long rows, int n, int k);
 bool linear_takes_norm(const LinearLaunch &p);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
 
+// (gelu(a w1' + b1) w2' + b2) * gamma + residual over [rows, c], w1 [hidden, c], w2 [c, hidden]; b1, b2, gamma, residual may be null.
+struct MlpLaunch {
+  const void *a, *w1, *b1, *w2, *b2, *gamma, *residual;
+  void *out;
+  long long rows;
+  int c, hidden;
+};
+constexpr long long kMlpLeastRows = 32768;      // a workgroup of 128 rows for every CU
+// 16-bit types, up to 224 channels (more do not fit a wave's registers), hidden features in whole steps.
+bool mlp_fits(int dtype, long long rows, int c, int hidden);
+hipError_t launch_mlp(int dtype, const MlpLaunch &p, hipStream_t stream);
+
 // grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k] (and grad_bias[n], may be null), several products over the same
 // rows at once.  With splits > 1 grad_w and grad_bias point into partial sums whose splits lie split_stride floats apart.
 constexpr int kMaxWeightGrads = 6;

@@ -75,7 +75,8 @@ __device__ __forceinline__ NormalTail normal_tail(float x) {
 template <typename Tag>
 __device__ __forceinline__ float gelu_exact(float x) {
   if constexpr (Tag::kBytes == 4) return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));      // an fp32 result keeps fp32 precision
-  else return fmaf(-fabsf(x), normal_tail(x).tail, fmaxf(x, 0.f));
+  // max(x, 0) as integers, one instruction (fmaxf costs another to quiet a NaN, which the product carries through here)
+  else return fmaf(-fabsf(x), normal_tail(x).tail, __builtin_bit_cast(float, max(__builtin_bit_cast(int, x), 0)));
 }
 // Phi(x) + x phi(x)
 __device__ __forceinline__ float gelu_derivative(float x) {
@@ -84,8 +85,8 @@ __device__ __forceinline__ float gelu_derivative(float x) {
 }
 
 // 16 bytes per lane from a range-checked buffer straight into LDS: lane l's vector lands at lds + 16 * l.
-__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, void *lds, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 16, (int)off, 0, 0, 0);
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, void *lds, uint32_t off, uint32_t uniform_off = 0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 16, (int)off, (int)uniform_off, 0, 0);
 }
 
 }  // namespace dcn

@@ -47,7 +47,8 @@ def test_gelu_epilogue_keeps_its_relative_precision_in_the_tails():
 @pytest.mark.parametrize("channels,groups,post_norm,dw,scale,size", [
     (64, 4, False, None, None, (3, 13, 9)), (112, 7, True, 3, 0.3, (2, 14, 11)), (160, 10, True, 5, None, (1, 7, 7)),
     (64, 4, False, 3, 0.5, (40, 28, 28)), (512, 32, False, None, None, (1, 5, 7)), (272, 17, True, 3, 0.3, (1, 3, 11)),
-    (640, 40, True, 3, 0.3, (1, 7, 7))])
+    (640, 40, True, 3, 0.3, (1, 7, 7)), (48, 3, False, None, None, (42, 28, 29)), (112, 7, False, None, 0.5, (41, 28, 29)),
+    (224, 14, True, 3, 0.3, (33, 32, 32))])
 def test_layer_inference_matches_the_modules_in_fp32(channels, groups, post_norm, dw, scale, size, dtype):
     from dcnv4_amd.models.flash_intern_image import InternImageLayer
     torch.manual_seed(channels)
