@@ -8,6 +8,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -88,6 +89,10 @@ inline bool wants_grad(std::initializer_list<const Tensor *> inputs) {
     if (t->defined() && t->requires_grad()) return true;
   return false;
 }
+
+// Whether a tracer records torch's operators on this thread.  The kernels write through raw pointers, which it does not see: a
+// trace would hold the allocation of a result and nothing that fills it.  The Python path is a node of the trace.
+bool observed();
 
 extern PyMethodDef operator_methods[];
 

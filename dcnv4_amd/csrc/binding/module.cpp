@@ -69,6 +69,8 @@ float Args::real() {
   return (float)v;
 }
 
+bool observed() { return at::tracer::impl::is_dispatch_enabled(); }
+
 variable_list once_differentiable(variable_list grads) {
   if (!at::GradMode::is_enabled()) return grads;
   const auto error = std::make_shared<torch::autograd::DelayedError>(

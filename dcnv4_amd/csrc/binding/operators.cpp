@@ -97,13 +97,14 @@ struct DCNv4FunctionBackward final : torch::autograd::Node {
   }
 };
 
-// dcnv4(input, offset_mask, 12 x geometry, remove_center): what DCNv4Function.apply takes
+// dcnv4(input, offset_mask, 12 x geometry, remove_center): what DCNv4Function.apply takes; None where its methods have to run
 PyObject *py_dcnv4(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Args a("dcnv4", args, n, 15);
   const Tensor &value = a.tensor(), &offset = a.tensor();
   const DcnGeometry g(a);
   const int remove_center = a.integer();
+  if (observed()) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
@@ -291,7 +292,7 @@ Tensor fda_apply(const Tensor &value, const Tensor &shapes, const Tensor &starts
   return out;
 }
 
-// flash_deform_attn(value, spatial_shapes, level_start_index, sampling_loc_attn, im2col_step, K)
+// flash_deform_attn(value, spatial_shapes, level_start_index, sampling_loc_attn, im2col_step, K), or None as above
 PyObject *py_fda(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Args a("flash_deform_attn", args, n, 6);
@@ -299,6 +300,7 @@ PyObject *py_fda(PyObject *, PyObject *const *args, Py_ssize_t n) {
   FdaRows r;
   r.packed = a.tensor();
   const int step = a.integer(), points = a.integer();
+  if (observed()) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
@@ -317,6 +319,7 @@ PyObject *py_fda_split(PyObject *, PyObject *const *args, Py_ssize_t n) {
   r.locations = a.tensor();
   r.logits = a.tensor();
   const int step = a.integer(), points = a.integer();
+  if (observed()) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;

@@ -19,10 +19,13 @@ class DCNv4Function(Function):
     def apply(*args):
         # The C++ path (csrc/binding/operators.cpp) does what the two methods below do when the library is to choose the
         # launch: host time of a small forward 15 -> 6 us, of forward + backward 65-130 -> 40-60 us.  They run for tuned
-        # table entries, whose options are set around the calls, and for programs that wrap ext's functions.
-        if GFX950_TABLE or ext.dcnv4_forward is not _ext_functions[0] or ext.dcnv4_backward is not _ext_functions[1]:
-            return super(DCNv4Function, DCNv4Function).apply(*args)
-        return _native_dcnv4(*args)
+        # table entries, whose options are set around the calls, for programs that wrap ext's functions, and where the C++
+        # path declines: under a tracer.
+        if not GFX950_TABLE and ext.dcnv4_forward is _ext_functions[0] and ext.dcnv4_backward is _ext_functions[1]:
+            output = _native_dcnv4(*args)
+            if output is not None:
+                return output
+        return super(DCNv4Function, DCNv4Function).apply(*args)
 
     @staticmethod
     @custom_fwd(device_type="cuda")

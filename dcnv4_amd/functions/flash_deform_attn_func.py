@@ -25,10 +25,9 @@ def _interpreted():
 class FlashDeformAttnFunction(Function):
     @staticmethod
     def apply(value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K=8):
-        if _interpreted():
-            return super(FlashDeformAttnFunction, FlashDeformAttnFunction).apply(
-                value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K)
-        return _native.flash_deform_attn(value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K)
+        args = (value, value_spatial_shapes, value_level_start_index, sampling_loc_attn, im2col_step, K)
+        output = None if _interpreted() else _native.flash_deform_attn(*args)      # None: declined, as under a tracer
+        return super(FlashDeformAttnFunction, FlashDeformAttnFunction).apply(*args) if output is None else output
 
     @staticmethod
     @torch.autocast("cuda", enabled=True, dtype=torch.float16)
@@ -69,9 +68,8 @@ class FlashDeformAttnSplitFunction(Function):
     @staticmethod
     def apply(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_logits, im2col_step, K=8):
         args = (value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_logits, im2col_step, K)
-        if _interpreted():
-            return super(FlashDeformAttnSplitFunction, FlashDeformAttnSplitFunction).apply(*args)
-        return _native.flash_deform_attn_split(*args)
+        output = None if _interpreted() else _native.flash_deform_attn_split(*args)
+        return super(FlashDeformAttnSplitFunction, FlashDeformAttnSplitFunction).apply(*args) if output is None else output
 
     @staticmethod
     @torch.autocast("cuda", enabled=True, dtype=torch.float16)

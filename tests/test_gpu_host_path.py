@@ -1,0 +1,110 @@
+"""What a call through the extension module must not pass by: what torch's autograd Functions and modules refuse, record or let a
+program replace, on the paths that run a whole operator or layer in one call."""
+import types
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+
+pytestmark = pytest.mark.gpu
+
+GEOMETRY = (3, 3, 1, 1, 1, 1, 1, 1)
+
+
+def _rel(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm()).item()
+
+
+def _layer(channels=64, dtype=torch.float16, **kw):
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    torch.manual_seed(channels)
+    layer = InternImageLayer(channels, channels // 16, **kw).cuda()
+    with torch.no_grad():
+        layer.dcn.offset_mask.weight.normal_(0, 0.02)
+        layer.dcn.offset_mask.bias.normal_(0, 0.5)
+    return layer.to(dtype)
+
+
+def _attention(width=64, levels=((6, 7), (3, 4)), queries=33, batch=2, module=None):
+    import dcnv4_amd
+    torch.manual_seed(queries)
+    m = (module or dcnv4_amd.FlashDeformAttn)(width, len(levels), 4, 4).cuda()
+    with torch.no_grad():
+        m.sampling_offsets.weight.normal_(0, 0.05)
+        m.attention_weights.weight.normal_(0, 0.05)
+    pixels = sum(h * w for h, w in levels)
+    shapes = torch.tensor(levels, device="cuda")
+    starts = torch.tensor([sum(h * w for h, w in levels[:i]) for i in range(len(levels))], device="cuda")
+    query, features = torch.randn(batch, queries, width, device="cuda"), torch.randn(batch, pixels, width, device="cuda")
+    reference = torch.rand(batch, queries, len(levels), 2, device="cuda")
+    return m, (query, reference, features, shapes, starts)
+
+
+def _operators():
+    """name -> (function of two float tensors, those tensors)"""
+    from dcnv4_amd import DCNv4Function, FlashDeformAttnFunction
+    from dcnv4_amd.functions import FlashDeformAttnSplitFunction
+    rand = lambda *s: torch.randn(s, device="cuda")
+    shapes, starts = torch.tensor([[5, 6], [3, 3]], device="cuda"), torch.tensor([0, 30], device="cuda")
+    rows = torch.rand(1, 7, 2, 8 * 3, device="cuda")
+    return {
+        "dcnv4": (lambda v, o: DCNv4Function.apply(v, o, *GEOMETRY, 2, 16, 1.0, 256, 0), (rand(1, 6, 7, 32), rand(1, 6, 7, 56))),
+        "attention": (lambda v, r: FlashDeformAttnFunction.apply(v, shapes, starts, r, 64, 4), (rand(1, 39, 2, 16), rows)),
+        "attention split": (lambda v, r: FlashDeformAttnSplitFunction.apply(v, shapes, starts, r[..., :16].contiguous(), r[..., 16:].contiguous(), 64, 4),
+                            (rand(1, 39, 2, 16), rows)),
+    }
+
+
+OPERATORS = ("dcnv4", "attention", "attention split")
+
+
+def _poison():
+    """Blocks that the allocator hands out next hold NaN."""
+    torch.cuda.empty_cache()
+    held = [torch.full((n,), float("nan"), device="cuda") for n in (64, 512, 4096, 65536, 1 << 20) for _ in range(32)]
+    del held
+
+
+@pytest.mark.parametrize("name", OPERATORS)
+def test_a_traced_operator_computes_its_result(name):
+    f, inputs = _operators()[name]
+    traced = torch.jit.trace(f, inputs, check_trace=False)
+    again = tuple(torch.rand_like(t) for t in inputs)
+    _poison()
+    assert torch.equal(traced(*again), f(*again))
+
+
+@pytest.mark.parametrize("kind", ["inference", "autocast"])
+def test_a_traced_layer_computes_its_result(kind):
+    layer = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval().requires_grad_(False)
+    x, other = (torch.randn(2, 42, 64, device="cuda", dtype=layer.norm1[0].weight.dtype) for _ in range(2))
+
+    def run(y):
+        with torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+            return layer(y, (6, 7))
+
+    with torch.no_grad():
+        traced = torch.jit.trace(run, x, check_trace=False)
+        _poison()
+        assert _rel(traced(other), run(other)) < 3e-3
+
+
+def test_a_traced_attention_layer_computes_its_result():
+    m, (query, reference, features, shapes, starts) = _attention()
+    m.requires_grad_(False)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda q, f: m(q, reference, f, shapes, starts), (query, features), check_trace=False)
+        other = torch.randn_like(query), torch.randn_like(features)
+        _poison()
+        assert _rel(traced(*other), m(other[0], reference, other[1], shapes, starts)) < 2e-3
+
+
+def test_a_traced_model_computes_its_result():
+    from dcnv4_amd.models import flash_intern_image
+    torch.manual_seed(1)
+    model = flash_intern_image("t", depths=(1, 1, 1, 1)).cuda().half().eval()
+    x, other = (torch.randn(1, 3, 64, 64, device="cuda").half() for _ in range(2))
+    with torch.no_grad():
+        traced = torch.jit.trace(model, x, check_trace=False)
+        _poison()
+        assert _rel(traced(other), model(other)) < 3e-3
