@@ -211,7 +211,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
       at::AutoGradMode no_grad(false);
       Tensor v[6];
       for (int i = 0; i < 6; ++i) v[i] = inputs[i].unpack();
-      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], grads[0].contiguous(), saved, task_should_compute_output(kQuery),
+      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0]), saved, task_should_compute_output(kQuery),
                            task_should_compute_output(kFeatures));
     }
     return once_differentiable(std::move(out));
@@ -222,7 +222,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
 };
 
 bool dense(const Tensor &t, const Tensor &like, at::ScalarType dtype) {
-  return t.device() == like.device() && t.scalar_type() == dtype && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
+  return t.device() == like.device() && t.scalar_type() == dtype && t.is_contiguous() && in_memory(t) && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
 }
 
 bool load(const Module &m, Attention *a, Input weight, int64_t in, int64_t out, const Tensor &like) {
@@ -267,7 +267,7 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Py_RETURN_NONE;
   if (!dense(shapes, query, at::kLong) || !dense(starts, query, at::kLong) || shapes.numel() != 2 * a.levels || starts.numel() != a.levels)
     Py_RETURN_NONE;
-  if (padding.defined() && (padding.device() != query.device() || padding.scalar_type() != at::kBool || !padding.is_contiguous() ||
+  if (padding.defined() && (padding.device() != query.device() || padding.scalar_type() != at::kBool || !padding.is_contiguous() || !in_memory(padding) ||
                             padding.numel() != a.feature_rows()))
     Py_RETURN_NONE;
   if (!load(m.child("value_proj", kLinear), &a, kValueW, a.width, a.width, query) ||

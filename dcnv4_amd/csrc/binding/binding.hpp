@@ -94,6 +94,13 @@ inline bool wants_grad(std::initializer_list<const Tensor *> inputs) {
 // trace would hold the allocation of a result and nothing that fills it.  The Python path is a node of the trace.
 bool observed();
 
+// Whether a tensor's elements lie in memory that it points to: not so for wrappers around other tensors, fake tensors and the
+// zeros of autograd, whose pointer is null.
+bool in_memory(const Tensor &t);
+
+// A gradient that arrives at a node, as the kernels read it.
+Tensor incoming(const Tensor &grad);
+
 extern PyMethodDef operator_methods[];
 
 }  // namespace dcn::binding

@@ -33,6 +33,7 @@ int dtype_code(const Tensor &t, const char *name) {
 void check_tensor(const Tensor &t, const char *name) {
   if (!t.is_contiguous()) raise_runtime("%s tensor has to be contiguous", name);
   if (!t.is_cuda()) raise_runtime("%s must be a CUDA tensor (Not implemented on the CPU)", name);
+  if (!in_memory(t)) raise_runtime("%s has no memory of its own", name);
 }
 
 void check_tensor(const Tensor &t, const char *name, at::ScalarType dtype) {
@@ -70,6 +71,14 @@ float Args::real() {
 }
 
 bool observed() { return at::tracer::impl::is_dispatch_enabled(); }
+
+bool in_memory(const Tensor &t) { return t.has_storage() && (t.numel() == 0 || t.const_data_ptr() != nullptr); }
+
+Tensor incoming(const Tensor &grad) {
+  const Tensor g = grad._is_zerotensor() ? at::zeros(grad.sizes(), grad.options()) : grad.contiguous();
+  if (!in_memory(g)) raise_runtime("the gradient of the output has no memory of its own");
+  return g;
+}
 
 variable_list once_differentiable(variable_list grads) {
   if (!at::GradMode::is_enabled()) return grads;

@@ -108,3 +108,55 @@ def test_a_traced_model_computes_its_result():
         traced = torch.jit.trace(model, x, check_trace=False)
         _poison()
         assert _rel(traced(other), model(other)) < 3e-3
+
+
+class Wrapper(torch.Tensor):
+    """Holds another tensor and has no storage of its own, as quantised or sharded parameters do."""
+
+    @staticmethod
+    def __new__(cls, held):
+        return torch.Tensor._make_wrapper_subclass(cls, held.shape, dtype=held.dtype, device=held.device, requires_grad=False)
+
+    def __init__(self, held):
+        self.held = held
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        open_ = lambda t: t.held if isinstance(t, Wrapper) else t
+        return func(*torch.utils._pytree.tree_map(open_, args), **torch.utils._pytree.tree_map(open_, kwargs or {}))
+
+
+@pytest.mark.parametrize("kind", ["inference", "autocast", "attention"])
+def test_parameters_without_storage_run_the_modules(kind):
+    if kind == "attention":
+        m, inputs = _attention()
+        run, linear = lambda: m(*inputs), m.output_proj
+    else:
+        m = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval()
+        x = torch.randn(2, 42, 64, device="cuda", dtype=m.norm1[0].weight.dtype)
+        run, linear = lambda: m(x, (6, 7)), m.mlp.fc1
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+        want = run()
+        linear._parameters["weight"] = Wrapper(linear.weight.detach())
+        assert _rel(run(), want) < 3e-3
+
+
+@pytest.mark.parametrize("kind", ["dcnv4", "layer", "attention"])
+def test_gradients_without_storage_are_refused_and_zeros_are_zeros(kind):
+    def forward():
+        if kind == "dcnv4":
+            f, (v, o) = _operators()["dcnv4"]
+            return v.requires_grad_(), f(v, o)
+        if kind == "attention":
+            m, (x, *rest) = _attention()
+            return x.requires_grad_(), m(x, *rest)
+        x = torch.randn(2, 42, 64, device="cuda", requires_grad=True)
+        with torch.autocast("cuda", dtype=torch.float16):
+            return x, _layer(dtype=torch.float32)(x, (6, 7))
+
+    x, out = forward()
+    with pytest.raises(RuntimeError, match="memory"):
+        torch.autograd.grad(out, x, Wrapper(torch.ones_like(out)))
+    x, out = forward()
+    zeros = torch._efficientzerotensor(out.shape, dtype=out.dtype, device="cuda")
+    assert not torch.autograd.grad(out, x, zeros)[0].any()
