@@ -211,7 +211,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
       at::AutoGradMode no_grad(false);
       Tensor v[6];
       for (int i = 0; i < 6; ++i) v[i] = inputs[i].unpack();
-      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0]), saved, task_should_compute_output(kQuery),
+      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0], true), saved, task_should_compute_output(kQuery),
                            task_should_compute_output(kFeatures));
     }
     return once_differentiable(std::move(out));

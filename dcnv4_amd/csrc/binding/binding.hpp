@@ -98,8 +98,9 @@ bool observed();
 // zeros of autograd, whose pointer is null.
 bool in_memory(const Tensor &t);
 
-// A gradient that arrives at a node, as the kernels read it.
-Tensor incoming(const Tensor &grad);
+// A gradient that arrives at a node, as the kernels read it: dense, and where a layer's kernels take it in 16-byte vectors with no
+// further check, on a 16-byte boundary (a contiguous slice of a larger tensor may begin at any element).
+Tensor incoming(const Tensor &grad, bool aligned);
 
 extern PyMethodDef operator_methods[];
 

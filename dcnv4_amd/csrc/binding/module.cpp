@@ -74,9 +74,10 @@ bool observed() { return at::tracer::impl::is_dispatch_enabled(); }
 
 bool in_memory(const Tensor &t) { return t.has_storage() && (t.numel() == 0 || t.const_data_ptr() != nullptr); }
 
-Tensor incoming(const Tensor &grad) {
-  const Tensor g = grad._is_zerotensor() ? at::zeros(grad.sizes(), grad.options()) : grad.contiguous();
+Tensor incoming(const Tensor &grad, bool aligned) {
+  Tensor g = grad._is_zerotensor() ? at::zeros(grad.sizes(), grad.options()) : grad.contiguous();
   if (!in_memory(g)) raise_runtime("the gradient of the output has no memory of its own");
+  if (aligned && (reinterpret_cast<uintptr_t>(g.const_data_ptr()) & 15) != 0) g = g.clone(at::MemoryFormat::Contiguous);
   return g;
 }
 

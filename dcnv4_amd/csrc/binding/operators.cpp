@@ -91,7 +91,7 @@ struct DCNv4FunctionBackward final : torch::autograd::Node {
     variable_list out(2);
     {
       at::AutoGradMode no_grad(false);
-      std::tie(out[0], out[1]) = dcn_backward(value.unpack(), offset.unpack(), incoming(grads[0]), geometry, remove_center, 0, 0, 0);
+      std::tie(out[0], out[1]) = dcn_backward(value.unpack(), offset.unpack(), incoming(grads[0], false), geometry, remove_center, 0, 0, 0);
     }
     return once_differentiable(std::move(out));
   }
@@ -273,7 +273,7 @@ struct FlashDeformAttnFunctionBackward final : torch::autograd::Node {
       FdaRows r;
       (split ? r.locations : r.packed) = first.unpack();
       if (split) r.logits = logits.unpack();
-      out = fda_backward(value.unpack(), shapes.unpack(), starts.unpack(), r, incoming(grads[0]), step, points, 0, 0);
+      out = fda_backward(value.unpack(), shapes.unpack(), starts.unpack(), r, incoming(grads[0], false), step, points, 0, 0);
     }
     return once_differentiable(std::move(out));
   }

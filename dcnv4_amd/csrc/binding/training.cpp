@@ -317,7 +317,7 @@ struct InternImageLayerBackward final : torch::autograd::Node {
       std::array<Tensor *, 6> into = {&now.l.norm1.weight, &now.l.norm1.bias, &now.l.gamma1, &now.l.norm2.weight, &now.l.norm2.bias,
                                       &now.l.gamma2};
       for (int i = 0; i < 6; ++i) *into[i] = params[i].unpack();
-      out = now.backward(x.unpack(), incoming(grads[0]), saved);
+      out = now.backward(x.unpack(), incoming(grads[0], true), saved);
     }
     return once_differentiable(std::move(out));
   }

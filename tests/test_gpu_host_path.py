@@ -160,3 +160,23 @@ def test_gradients_without_storage_are_refused_and_zeros_are_zeros(kind):
     x, out = forward()
     zeros = torch._efficientzerotensor(out.shape, dtype=out.dtype, device="cuda")
     assert not torch.autograd.grad(out, x, zeros)[0].any()
+
+
+@pytest.mark.parametrize("kind", ["post-norm", "pre-norm", "attention", "attention fp32"])
+def test_a_gradient_may_begin_at_any_element(kind):
+    if kind.startswith("attention"):
+        m, (x, *rest) = _attention()
+        run = lambda: m(x, *rest)
+    else:
+        m, x = _layer(dtype=torch.float32, post_norm=kind == "post-norm"), torch.randn(2, 42, 64, device="cuda")
+        run = lambda: m(x, (6, 7))
+    x.requires_grad_()
+    with torch.autocast("cuda", dtype=torch.float16, enabled=kind != "attention fp32"):
+        out = run()
+    # as the split of a flattened cat hands it out
+    shifted = torch.randn(out.numel() + 1, device="cuda").to(out.dtype)[1:].view(out.shape)
+    assert shifted.is_contiguous() and shifted.data_ptr() % 16 != 0
+    wanted = [x, *m.parameters()]
+    got = torch.autograd.grad(out, wanted, shifted, retain_graph=True)
+    for a, b in zip(got, torch.autograd.grad(out, wanted, shifted.clone())):
+        assert _rel(a, b) < 1e-5
