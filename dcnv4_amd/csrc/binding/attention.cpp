@@ -222,7 +222,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
 };
 
 bool dense(const Tensor &t, const Tensor &like, at::ScalarType dtype) {
-  return t.device() == like.device() && t.scalar_type() == dtype && t.is_contiguous() && in_memory(t) && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
+  return t.device() == like.device() && t.scalar_type() == dtype && t.is_contiguous() && plain(t) && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
 }
 
 bool load(const Module &m, Attention *a, Input weight, int64_t in, int64_t out, const Tensor &like) {

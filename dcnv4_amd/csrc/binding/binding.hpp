@@ -98,6 +98,10 @@ bool observed();
 // zeros of autograd, whose pointer is null.
 bool in_memory(const Tensor &t);
 
+// Whether a tensor is its elements and nothing else: in memory, without a tangent of forward-mode differentiation, which the
+// nodes here would drop without a word (an autograd Function without a jvp refuses it, torch's operators carry it on).
+bool plain(const Tensor &t);
+
 // A gradient that arrives at a node, as the kernels read it: dense, and where a layer's kernels take it in 16-byte vectors with no
 // further check, on a 16-byte boundary (a contiguous slice of a larger tensor may begin at any element).
 Tensor incoming(const Tensor &grad, bool aligned);

@@ -68,7 +68,7 @@ bool exact_gelu(const Module &act) {
 }
 
 bool inference(const Tensor &x) {
-  return !observed() && !at::GradMode::is_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA) && !global_module_hooks() && x.is_cuda() && in_memory(x) && x.numel() != 0 &&
+  return !observed() && !at::GradMode::is_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA) && !global_module_hooks() && x.is_cuda() && plain(x) && x.numel() != 0 &&
          x.dtype() != at::kFloat && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16);
 }
 

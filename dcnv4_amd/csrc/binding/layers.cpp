@@ -12,7 +12,7 @@ namespace dcn::binding {
 
 bool usable(const Tensor &t, const Tensor &x, at::ScalarType dtype, int64_t elements, bool optional) {
   if (!t.defined()) return optional;
-  return t.scalar_type() == dtype && t.device() == x.device() && t.numel() == elements && t.is_contiguous() && in_memory(t) &&
+  return t.scalar_type() == dtype && t.device() == x.device() && t.numel() == elements && t.is_contiguous() && plain(t) &&
          (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0;
 }
 
@@ -144,7 +144,7 @@ void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std
 }
 
 bool usable_input(const Tensor &x, int h, int w) {
-  return x.is_cuda() && x.dim() == 3 && x.is_contiguous() && in_memory(x) && x.numel() != 0 && x.size(1) == (int64_t)h * w &&
+  return x.is_cuda() && x.dim() == 3 && x.is_contiguous() && plain(x) && x.numel() != 0 && x.size(1) == (int64_t)h * w &&
          (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15) == 0;
 }
 

@@ -74,6 +74,8 @@ bool observed() { return at::tracer::impl::is_dispatch_enabled(); }
 
 bool in_memory(const Tensor &t) { return t.has_storage() && (t.numel() == 0 || t.const_data_ptr() != nullptr); }
 
+bool plain(const Tensor &t) { return in_memory(t) && !torch::autograd::isFwGradDefined(t); }
+
 Tensor incoming(const Tensor &grad, bool aligned) {
   Tensor g = grad._is_zerotensor() ? at::zeros(grad.sizes(), grad.options()) : grad.contiguous();
   if (!in_memory(g)) raise_runtime("the gradient of the output has no memory of its own");

@@ -104,7 +104,7 @@ PyObject *py_dcnv4(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Tensor &value = a.tensor(), &offset = a.tensor();
   const DcnGeometry g(a);
   const int remove_center = a.integer();
-  if (observed()) Py_RETURN_NONE;
+  if (observed() || !plain(value) || !plain(offset)) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
@@ -300,7 +300,7 @@ PyObject *py_fda(PyObject *, PyObject *const *args, Py_ssize_t n) {
   FdaRows r;
   r.packed = a.tensor();
   const int step = a.integer(), points = a.integer();
-  if (observed()) Py_RETURN_NONE;
+  if (observed() || !plain(value) || !plain(r.packed)) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
@@ -319,7 +319,7 @@ PyObject *py_fda_split(PyObject *, PyObject *const *args, Py_ssize_t n) {
   r.locations = a.tensor();
   r.logits = a.tensor();
   const int step = a.integer(), points = a.integer();
-  if (observed()) Py_RETURN_NONE;
+  if (observed() || !plain(value) || !plain(r.locations) || !plain(r.logits)) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;

@@ -20,7 +20,7 @@ class DCNv4Function(Function):
         # The C++ path (csrc/binding/operators.cpp) does what the two methods below do when the library is to choose the
         # launch: host time of a small forward 15 -> 6 us, of forward + backward 65-130 -> 40-60 us.  They run for tuned
         # table entries, whose options are set around the calls, for programs that wrap ext's functions, and where the C++
-        # path declines: under a tracer.
+        # path declines: under a tracer, or for a tensor that carries a tangent.
         if not GFX950_TABLE and ext.dcnv4_forward is _ext_functions[0] and ext.dcnv4_backward is _ext_functions[1]:
             output = _native_dcnv4(*args)
             if output is not None:

@@ -180,3 +180,49 @@ def test_a_gradient_may_begin_at_any_element(kind):
     got = torch.autograd.grad(out, wanted, shifted, retain_graph=True)
     for a, b in zip(got, torch.autograd.grad(out, wanted, shifted.clone())):
         assert _rel(a, b) < 1e-5
+
+
+@pytest.mark.parametrize("grad", [True, False], ids=["grad", "no-grad"])
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("name", OPERATORS)
+def test_an_operator_refuses_forward_mode(name, which, grad):
+    f, inputs = _operators()[name]
+    with fwAD.dual_level(), torch.set_grad_enabled(grad):
+        inputs = list(inputs)
+        inputs[which] = fwAD.make_dual(inputs[which], torch.ones_like(inputs[which]))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            f(*inputs)
+
+
+@pytest.mark.parametrize("where", ["input", "parameter"])
+@pytest.mark.parametrize("kind", ["inference", "autocast", "attention"])
+def test_a_layer_refuses_forward_mode(kind, where):
+    if kind == "attention":
+        m, (query, reference, features, shapes, starts) = _attention()
+        run, x, weight = lambda q: m(q, reference, features, shapes, starts), query, m.value_proj
+    else:
+        m = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval()
+        x, weight = torch.randn(2, 42, 64, device="cuda", dtype=m.norm1[0].weight.dtype), m.dcn.value_proj
+        run = lambda y: m(y, (6, 7))
+    with fwAD.dual_level(), torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+        if where == "input":
+            x = fwAD.make_dual(x, torch.ones_like(x))
+        else:
+            w = weight.weight
+            del weight.weight
+            weight.register_parameter("weight", None)
+            weight._parameters["weight"] = fwAD.make_dual(w.detach(), torch.ones_like(w))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            run(x)
+
+
+def test_the_convolutions_around_the_layers_carry_tangents():
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer
+    torch.manual_seed(2)
+    stem, down = StemLayer(3, 64).cuda().half().eval(), DownsampleLayer(64).cuda().half().eval()
+    x = torch.randn(1, 3, 32, 32, device="cuda").half()
+    with torch.no_grad(), fwAD.dual_level():
+        y = stem(fwAD.make_dual(x, torch.ones_like(x)))
+        assert fwAD.unpack_dual(y).tangent is not None
+        z, _ = down(y.reshape(1, 64, 64), (8, 8))
+        assert fwAD.unpack_dual(z).tangent is not None
