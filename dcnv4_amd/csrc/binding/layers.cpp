@@ -4,6 +4,7 @@
 // A picture or a few are bound by the host: 415 launches through Python took 6.5 ms for a T variant whose kernels run
 // 2.2 ms.  Here a layer is seven (pre-norm) or eight launches: the two projections in front of the operator share one,
 // bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 
 #include "layers.hpp"
@@ -96,6 +97,8 @@ void launch(int code, const LinearLaunch &l, void *stream) {
   const hipError_t e = launch_linear(code, l, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) raise_runtime("linear layer launch: %s", hipGetErrorString(e));
 }
+
+bool saves_under_hooks() { return at::GradMode::is_enabled() && at::SavedTensorDefaultHooks::get_hooks().has_value(); }
 
 void hip_check(hipError_t e, const char *what) {
   if (e != hipSuccess) raise_runtime("%s: %s", what, hipGetErrorString(e));

@@ -32,6 +32,10 @@ void launch(int code, const LinearLaunch &l, void *stream);
 // The arguments (layer, x, h, w) of a call that takes a layer.
 bool usable_input(const Tensor &x, int h, int w);
 
+// Whether the call is to keep its activations under hooks that pack what a backward needs (checkpointing, save_on_cpu).  They see
+// what torch's operators save; a layer's node keeps one block of all its activations, which is nothing to hand to them.
+bool saves_under_hooks();
+
 void hip_check(hipError_t e, const char *what);
 
 // Sub-tensors of one allocation, each on a 256-byte boundary.

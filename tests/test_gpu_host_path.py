@@ -226,3 +226,49 @@ def test_the_convolutions_around_the_layers_carry_tangents():
         assert fwAD.unpack_dual(y).tangent is not None
         z, _ = down(y.reshape(1, 64, 64), (8, 8))
         assert fwAD.unpack_dual(z).tangent is not None
+
+
+@pytest.mark.parametrize("kind", ["layer", "attention"])
+def test_saved_tensor_hooks_see_the_activations(kind):
+    if kind == "layer":
+        m, x = _layer(dtype=torch.float32), torch.randn(2, 42, 64, device="cuda", requires_grad=True)
+        run, least = lambda: m(x, (6, 7)), 2 * 42 * 64 * 8       # the hidden tensor before and after its activation
+    else:
+        m, (x, reference, features, shapes, starts) = _attention()
+        x.requires_grad_()
+        run, least = lambda: m(x, reference, features, shapes, starts), x.numel()
+    wanted = [x, *m.parameters()]
+
+    def grads():
+        with torch.autocast("cuda", dtype=torch.float16, enabled=kind == "layer"):
+            out = run()
+        return torch.autograd.grad(out, wanted, torch.ones_like(out))
+
+    seen = []
+    plain = grads()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append((t.numel(), t.is_floating_point())) or t.cpu(), lambda t: t.cuda()):
+        hooked = grads()
+    assert sum(n for n, floating in seen if floating) > least + sum(p.numel() for p in m.parameters())
+    for a, b in zip(plain, hooked):
+        assert _rel(a, b) < 3e-3
+
+
+def test_checkpointing_a_layer_frees_its_activations():
+    from torch.utils.checkpoint import checkpoint
+    layer, shape = _layer(dtype=torch.float32), (56, 56)
+    x = torch.randn(4, 56 * 56, 64, device="cuda", requires_grad=True)
+
+    def step(run):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = run()
+        kept = torch.cuda.memory_allocated() - before
+        return kept, torch.autograd.grad(out, [x, *layer.parameters()], torch.ones_like(out))
+
+    step(lambda: layer(x, shape))       # caches of the first call
+    kept, want = step(lambda: layer(x, shape))
+    held, got = step(lambda: checkpoint(layer, x, shape, use_reentrant=False))
+    assert held < 2 * x.numel() * x.element_size() < kept       # the output and what torch keeps of small things
+    for a, b in zip(want, got):
+        assert _rel(b, a) < 3e-3
