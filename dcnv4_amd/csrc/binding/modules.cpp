@@ -5,7 +5,15 @@
 namespace dcn::binding {
 namespace {
 
-PyObject *g_kinds[kModuleKinds] = {};
+// A class and the methods that a call of its modules goes through, looked up again for each module: a program may replace them on
+// the class (or on nn.Module, whose methods they mostly are).
+constexpr const char *kMethods[] = {"forward", "__call__", "_call_impl"};
+constexpr int kMethodCount = sizeof(kMethods) / sizeof(kMethods[0]);
+struct Kind {
+  PyTypeObject *type = nullptr;
+  PyObject *methods[kMethodCount] = {};
+};
+Kind g_kinds[kModuleKinds];
 PyObject *g_global_hooks[4] = {};
 
 // Interned attribute names, looked up by the address of the literal.
@@ -27,7 +35,13 @@ PyObject *item(PyObject *dict, const char *name) {
 
 }  // namespace
 
-bool Module::is(ModuleKind kind) const { return o_ != nullptr && (PyObject *)Py_TYPE(o_) == g_kinds[kind]; }
+bool Module::is(ModuleKind kind) const {
+  const Kind &k = g_kinds[kind];
+  if (o_ == nullptr || Py_TYPE(o_) != k.type) return false;
+  for (int i = 0; i < kMethodCount; ++i)
+    if (_PyType_Lookup(k.type, name_object(kMethods[i])) != k.methods[i]) return false;
+  return true;
+}
 
 Module Module::child(const char *name) const {
   PyObject *c = o_ != nullptr ? item(item(dict_of(o_), "_modules"), name) : nullptr;
@@ -72,6 +86,10 @@ bool Module::hooked() const {
     PyObject *hooks = item(d, name);
     if (hooks != nullptr && PyDict_Check(hooks) && PyDict_GET_SIZE(hooks) != 0) return true;
   }
+  for (const char *name : {"forward", "_call_impl", "_compiled_call_impl"}) {
+    PyObject *replaced = item(d, name);
+    if (replaced != nullptr && replaced != Py_None) return true;
+  }
   return false;
 }
 
@@ -102,8 +120,15 @@ PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
     while (kind < kModuleKinds && PyUnicode_CompareWithASCIIString(name, kKindNames[kind]) != 0) ++kind;
     Py_DECREF(name);
     if (kind == kModuleKinds) raise_runtime("register_modules: no kind for argument %zd", i);
+    if (!PyType_Check(args[i])) raise_runtime("register_modules: argument %zd is no class", i);
+    Kind &k = g_kinds[kind];
     Py_INCREF(args[i]);
-    Py_XSETREF(g_kinds[kind], args[i]);
+    Py_XSETREF(k.type, reinterpret_cast<PyTypeObject *>(args[i]));
+    for (int m = 0; m < kMethodCount; ++m) {
+      PyObject *method = _PyType_Lookup(k.type, name_object(kMethods[m]));
+      Py_XINCREF(method);
+      Py_XSETREF(k.methods[m], method);
+    }
   }
   PyObject *m = PyImport_ImportModule("torch.nn.modules.module");
   if (m == nullptr) throw python_error();

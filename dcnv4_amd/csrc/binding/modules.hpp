@@ -22,8 +22,8 @@ class Module {
   long integer(const char *name, long otherwise) const;
   double real(const char *name, double otherwise) const;
   bool truth(const char *name, bool otherwise) const;
-  bool is(ModuleKind kind) const;
-  bool hooked() const;                                        // a hook that a direct call of the kernels would miss
+  bool is(ModuleKind kind) const;                             // exactly that class, its methods as they were registered
+  bool hooked() const;                                        // a hook or replaced method that a direct call of the kernels would miss
 
  private:
   PyObject *o_ = nullptr;

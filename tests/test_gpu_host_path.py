@@ -1,7 +1,5 @@
 """What a call through the extension module must not pass by: what torch's autograd Functions and modules refuse, record or let a
 program replace, on the paths that run a whole operator or layer in one call."""
-import types
-
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -272,3 +270,51 @@ def test_checkpointing_a_layer_frees_its_activations():
     assert held < 2 * x.numel() * x.element_size() < kept       # the output and what torch keeps of small things
     for a, b in zip(want, got):
         assert _rel(b, a) < 3e-3
+
+
+# the fused block tail takes a normalisation's parameters and calls its forward under autocast alone
+@pytest.mark.parametrize("kind,child", [(k, c) for k in ("inference", "autocast") for c in ("mlp", "mlp.fc1", "mlp.act", "dcn", "dcn.value_proj")] +
+                         [("autocast", "norm1.0")])
+def test_a_replaced_forward_is_called(kind, child):
+    layer = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval()
+    x = torch.randn(2, 42, 64, device="cuda", dtype=layer.norm1[0].weight.dtype)
+    calls = []
+    target = layer.get_submodule(child)
+    forward = target.forward
+    target.forward = lambda *a, **kw: calls.append(1) or forward(*a, **kw)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+        layer(x, (6, 7))
+    assert calls == [1]
+
+
+@pytest.mark.parametrize("child", ["value_proj", "output_proj"])
+def test_a_replaced_forward_in_attention_is_called(child):
+    m, inputs = _attention()
+    calls, target = [], m.get_submodule(child)
+    forward = target.forward
+    target.forward = lambda *a: calls.append(1) or forward(*a)
+    m(*inputs)
+    assert calls == [1]
+
+
+def test_replaced_forwards_around_the_layers_are_called():
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer
+    stem, down = StemLayer(3, 64).cuda().half().eval(), DownsampleLayer(64).cuda().half().eval()
+    calls = []
+    for m in (stem.conv1, stem.norm2, stem.norm2[0], down.norm, down.conv):
+        m.forward = (lambda f: lambda *a: calls.append(1) or f(*a))(m.forward)
+    with torch.no_grad():
+        y = stem(torch.randn(1, 3, 32, 32, device="cuda").half())
+        down(y.reshape(1, 64, 64), (8, 8))
+    assert len(calls) == 5
+
+
+@pytest.mark.parametrize("name", ["forward", "__call__"])
+@pytest.mark.parametrize("cls", [torch.nn.GELU, torch.nn.Linear], ids=lambda c: c.__name__)
+def test_a_class_with_a_replaced_method_is_called(cls, name, monkeypatch):
+    layer, calls = _layer().eval(), []
+    method = getattr(cls, name)
+    monkeypatch.setattr(cls, name, lambda self, *a: calls.append(1) or method(self, *a))
+    with torch.no_grad():
+        layer(torch.randn(1, 42, 64, device="cuda").half(), (6, 7))
+    assert len(calls) == (1 if cls is torch.nn.GELU else 5)
