@@ -38,6 +38,7 @@ bool load_linear(const Module &m, const Tensor &x, at::ScalarType dtype, int64_t
 }  // namespace
 
 bool Layer::load(const Module &m, const Tensor &x, at::ScalarType params) {
+  if (!m.computes(kInternImageLayer)) return false;
   const int64_t c = channels = x.size(-1);
   if (c % 8 != 0 || c > 4096) return false;
   post_norm = m.truth("post_norm", false);
@@ -65,7 +66,7 @@ bool Layer::load(const Module &m, const Tensor &x, at::ScalarType params) {
     return false;
 
   const Module dcn = m.child("dcn", kDCNv4);
-  if (!dcn || dcn.truth("without_pointwise", true) || dcn.truth("center_feature_scale", true) || dcn.integer("stride", 0) != 1) return false;
+  if (!dcn || !dcn.computes(kDCNv4) || dcn.truth("without_pointwise", true) || dcn.truth("center_feature_scale", true) || dcn.integer("stride", 0) != 1) return false;
   kernel = (int)dcn.integer("kernel_size", 0);
   pad = (int)dcn.integer("pad", -1);
   dilation = (int)dcn.integer("dilation", 0);

@@ -7,7 +7,9 @@ namespace {
 
 // A class and the methods that a call of its modules goes through, looked up again for each module: a program may replace them on
 // the class (or on nn.Module, whose methods they mostly are).
-constexpr const char *kMethods[] = {"forward", "__call__", "_call_impl"};
+// The last ones are the parts of a forward: of DCNv4, InternImageLayer and FlashDeformAttn.
+constexpr const char *kMethods[] = {"forward", "__call__", "_call_impl", "_offset_mask_rows", "_scaled_norm", "_sampling_locations"};
+constexpr int kParts = 3;
 constexpr int kMethodCount = sizeof(kMethods) / sizeof(kMethods[0]);
 struct Kind {
   PyTypeObject *type = nullptr;
@@ -38,8 +40,17 @@ PyObject *item(PyObject *dict, const char *name) {
 bool Module::is(ModuleKind kind) const {
   const Kind &k = g_kinds[kind];
   if (o_ == nullptr || Py_TYPE(o_) != k.type) return false;
-  for (int i = 0; i < kMethodCount; ++i)
+  for (int i = 0; i < kParts; ++i)
     if (_PyType_Lookup(k.type, name_object(kMethods[i])) != k.methods[i]) return false;
+  return true;
+}
+
+bool Module::computes(ModuleKind kind) const {
+  const Kind &k = g_kinds[kind];
+  if (o_ == nullptr || k.type == nullptr || !PyType_IsSubtype(Py_TYPE(o_), k.type)) return false;
+  PyObject *d = dict_of(o_);
+  for (int i = kParts; i < kMethodCount; ++i)
+    if (item(d, kMethods[i]) != nullptr || _PyType_Lookup(Py_TYPE(o_), name_object(kMethods[i])) != k.methods[i]) return false;
   return true;
 }
 
@@ -108,7 +119,8 @@ bool idle(const Module &m, ModuleKind kind) {
 namespace {
 
 constexpr const char *kKindNames[kModuleKinds] = {"Linear", "LayerNorm", "GELU", "Dropout", "Identity", "Conv2d", "Sequential", "DropPath",
-                                                   "DCNv4", "MLPLayer", "BatchNorm2d", "_ToChannelsFirst", "_ToChannelsLast"};
+                                                   "DCNv4", "MLPLayer", "BatchNorm2d", "_ToChannelsFirst", "_ToChannelsLast",
+                                                   "InternImageLayer", "StemLayer", "DownsampleLayer", "FlashDeformAttn"};
 
 // register_modules(*classes): each fills the kind of its name
 PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {

@@ -7,7 +7,7 @@ namespace dcn::binding {
 
 // The classes that a layer is made of; a module of another class (a subclass, a wrapper) is left to Python.
 enum ModuleKind { kLinear, kLayerNorm, kGelu, kDropout, kIdentity, kConv2d, kSequential, kDropPath, kDCNv4, kMlp, kBatchNorm2d, kToChannelsFirst,
-                  kToChannelsLast, kModuleKinds };
+                  kToChannelsLast, kInternImageLayer, kStemLayer, kDownsampleLayer, kFlashDeformAttn, kModuleKinds };
 
 class Module {
  public:
@@ -23,6 +23,7 @@ class Module {
   double real(const char *name, double otherwise) const;
   bool truth(const char *name, bool otherwise) const;
   bool is(ModuleKind kind) const;                             // exactly that class, its methods as they were registered
+  bool computes(ModuleKind kind) const;                       // that class or a subclass that overrides no part of its forward
   bool hooked() const;                                        // a hook or replaced method that a direct call of the kernels would miss
 
  private:

@@ -158,7 +158,7 @@ class InternImageLayer(nn.Module):
 
 
 _ext_forward = ext.dcnv4_forward
-ext._native.register_modules(DropPath, DCNv4, MLPLayer, _ToChannelsFirst, _ToChannelsLast)
+ext._native.register_modules(DropPath, DCNv4, MLPLayer, _ToChannelsFirst, _ToChannelsLast, InternImageLayer, StemLayer, DownsampleLayer)
 
 
 class InternImageBlock(nn.Module):

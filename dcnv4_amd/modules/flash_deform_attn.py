@@ -117,3 +117,6 @@ class FlashDeformAttn(nn.Module):
             sampled = FlashDeformAttnFunction.apply(value, input_spatial_shapes, input_level_start_index, packed,
                                                     self.im2col_step, self.n_points)
         return self.output_proj(sampled)
+
+
+ext._native.register_modules(FlashDeformAttn)

@@ -318,3 +318,27 @@ def test_a_class_with_a_replaced_method_is_called(cls, name, monkeypatch):
     with torch.no_grad():
         layer(torch.randn(1, 42, 64, device="cuda").half(), (6, 7))
     assert len(calls) == (1 if cls is torch.nn.GELU else 5)
+
+
+def test_subclasses_keep_what_they_override():
+    import dcnv4_amd
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    calls = []
+
+    class Centred(dcnv4_amd.FlashDeformAttn):
+        def _sampling_locations(self, offsets, reference_points, spatial_shapes):
+            calls.append("locations")
+            return super()._sampling_locations(offsets, reference_points, spatial_shapes)
+
+    m, inputs = _attention(module=Centred)
+    m(*inputs)
+
+    class Layer(InternImageLayer):
+        def _scaled_norm(self, *a):
+            calls.append("norm")
+            return super()._scaled_norm(*a)
+
+    layer = Layer(64, 4, post_norm=True).cuda().half().eval()
+    with torch.no_grad():
+        layer(torch.randn(1, 42, 64, device="cuda").half(), (6, 7))
+    assert calls == ["locations", "norm", "norm"]
