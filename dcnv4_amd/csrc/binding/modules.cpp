@@ -17,6 +17,10 @@ struct Kind {
 };
 Kind g_kinds[kModuleKinds];
 PyObject *g_global_hooks[4] = {};
+constexpr const char *kFunctions[] = {"dcnv4_forward", "dcnv4_backward", "depthwise_conv_forward", "depthwise_conv_backward",
+                                      "layer_norm_residual_forward", "layer_norm_residual_backward"};
+constexpr int kFunctionCount = sizeof(kFunctions) / sizeof(kFunctions[0]);
+PyObject *g_namespace = nullptr, *g_functions[kFunctionCount] = {};      // ext's, and what it held when it was loaded
 
 // Interned attribute names, looked up by the address of the literal.
 PyObject *name_object(const char *name) {
@@ -110,6 +114,12 @@ bool global_module_hooks() {
   return false;
 }
 
+bool functions_replaced() {
+  for (int i = 0; i < kFunctionCount; ++i)
+    if (item(g_namespace, kFunctions[i]) != g_functions[i]) return true;
+  return false;
+}
+
 bool idle(const Module &m, ModuleKind kind) {
   if (!m || m.hooked()) return false;
   if (m.is(kIdentity)) return true;
@@ -155,9 +165,26 @@ PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// register_functions(namespace): ext's, once its functions are defined
+PyObject *py_register_functions(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 1 || !PyDict_Check(args[0])) raise_runtime("register_functions takes a module's namespace");
+  Py_INCREF(args[0]);
+  Py_XSETREF(g_namespace, args[0]);
+  for (int i = 0; i < kFunctionCount; ++i) {
+    PyObject *f = item(g_namespace, kFunctions[i]);
+    if (f == nullptr) raise_runtime("register_functions: no %s", kFunctions[i]);
+    Py_INCREF(f);
+    Py_XSETREF(g_functions[i], f);
+  }
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 }  // namespace
 
-PyMethodDef module_methods[] = {{"register_modules", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_register)), METH_FASTCALL, nullptr},
+PyMethodDef module_methods[] = {{"register_functions", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_register_functions)), METH_FASTCALL, nullptr},
+                                {"register_modules", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_register)), METH_FASTCALL, nullptr},
                                 {nullptr, nullptr, 0, nullptr}};
 
 }  // namespace dcn::binding

@@ -32,6 +32,9 @@ class Module {
 
 bool global_module_hooks();
 
+// Whether a program has put a function of its own in place of one of ext's that a FlashInternImage layer calls.
+bool functions_replaced();
+
 // A dropout or stochastic-depth module that does nothing here: identity, probability 0, or in eval mode.
 bool idle(const Module &m, ModuleKind kind);
 

@@ -349,3 +349,6 @@ def lds_read_probe(pattern, iters=4000, device=None):
         out = torch.zeros(1, dtype=torch.int32, device=device)
         _lib.check(_L.dcnv4_gfx950_lds_read_probe(int(pattern), int(iters), out.data_ptr(), _stream()))
         return out.item() / 1000.0
+
+
+_native.register_functions(globals())

@@ -138,7 +138,7 @@ class InternImageLayer(nn.Module):
         return residual + self.drop_path(layer_norm_residual(y, ln, gamma))
 
     def forward(self, x, shape):
-        if x.is_cuda and not GFX950_TABLE and ext.dcnv4_forward is _ext_forward:
+        if x.is_cuda and not GFX950_TABLE:
             # one call where the kernels take the layer as it is: under autocast csrc/binding/training.cpp, else without
             # gradients csrc/binding/layers.cpp
             call = ext._native.layer_training if torch.is_autocast_enabled("cuda") else ext._native.layer_inference
@@ -157,7 +157,6 @@ class InternImageLayer(nn.Module):
         return x
 
 
-_ext_forward = ext.dcnv4_forward
 ext._native.register_modules(DropPath, DCNv4, MLPLayer, _ToChannelsFirst, _ToChannelsLast, InternImageLayer, StemLayer, DownsampleLayer)
 
 

@@ -342,3 +342,21 @@ def test_subclasses_keep_what_they_override():
     with torch.no_grad():
         layer(torch.randn(1, 42, 64, device="cuda").half(), (6, 7))
     assert calls == ["locations", "norm", "norm"]
+
+
+def test_wrapped_extension_functions_are_called(monkeypatch):
+    from dcnv4_amd import ext
+    calls = []
+    for name in ("dcnv4_backward", "layer_norm_residual_forward", "depthwise_conv_forward"):
+        f = getattr(ext, name)
+        with monkeypatch.context() as patch:
+            patch.setattr(ext, name, lambda *a, f=f, name=name, **kw: calls.append(name) or f(*a, **kw))
+            layer = _layer(post_norm=True, dw_kernel_size=3, dtype=torch.float32 if name == "dcnv4_backward" else torch.float16)
+            x = torch.randn(1, 42, 64, device="cuda", dtype=layer.norm1[0].weight.dtype)
+            if name == "dcnv4_backward":
+                with torch.autocast("cuda", dtype=torch.float16):
+                    layer(x, (6, 7)).sum().backward()
+            else:
+                with torch.no_grad():
+                    layer.eval()(x, (6, 7))
+    assert set(calls) == {"dcnv4_backward", "layer_norm_residual_forward", "depthwise_conv_forward"}
