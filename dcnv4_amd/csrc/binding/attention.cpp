@@ -240,7 +240,7 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Tensor &query = arg.tensor(), &reference = arg.tensor(), &features = arg.tensor(), &shapes = arg.tensor(), &starts = arg.tensor();
   const Tensor padding = arg.optional_tensor();
   const Module m(args[0]);
-  if (!m.computes(kFlashDeformAttn) || !query.is_cuda() || observed() || global_module_hooks() || saves_under_hooks()) Py_RETURN_NONE;
+  if (!m.computes(kFlashDeformAttn) || !query.is_cuda() || arg.overridden({0, 1, 2, 3, 4, 5}) || observed() || global_module_hooks() || saves_under_hooks()) Py_RETURN_NONE;
   Attention a;
   at::ScalarType type = at::kFloat;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) {

@@ -62,7 +62,7 @@ inline Tensor workspace(size_t bytes, const Tensor &like) {
 // Arguments of a METH_FASTCALL function, taken in order.
 class Args {
  public:
-  Args(const char *name, PyObject *const *args, Py_ssize_t n, Py_ssize_t want) : args_(args) {
+  Args(const char *name, PyObject *const *args, Py_ssize_t n, Py_ssize_t want) : args_(args), first_(args) {
     if (n != want) throw c10::TypeError({__func__, __FILE__, (uint32_t)__LINE__},
                                         std::string(name) + " takes " + std::to_string(want) + " arguments, got " + std::to_string(n));
   }
@@ -70,9 +70,11 @@ class Args {
   Tensor optional_tensor();      // None: an undefined tensor
   int integer();                 // None: 0
   float real();
+  // whether one of these arguments is of a class of its own, which torch's functions call and give their result
+  bool overridden(std::initializer_list<Py_ssize_t> which) const;
 
  private:
-  PyObject *const *args_;
+  PyObject *const *args_, *const *first_;
 };
 
 // Gradient outputs of a node whose formula is not differentiable itself: with create_graph they carry an error.
@@ -90,8 +92,10 @@ inline bool wants_grad(std::initializer_list<const Tensor *> inputs) {
   return false;
 }
 
-// Whether a tracer records torch's operators on this thread.  The kernels write through raw pointers, which it does not see: a
-// trace would hold the allocation of a result and nothing that fills it.  The Python path is a node of the trace.
+// Whether something records or changes torch's operators on this thread: a tracer, a dispatch or function mode (but the one that
+// stands for a default device), a functorch transform.  The kernels write through raw pointers, which none of them sees: a
+// trace would hold the allocation of a result and nothing that fills it.  The Python path is a node of the trace, and a layer's
+// modules call the operators that a mode counts or replaces.
 bool observed();
 
 // Whether a tensor's elements lie in memory that it points to: not so for wrappers around other tensors, fake tensors and the

@@ -90,7 +90,7 @@ PyObject *py_stem(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Args a("stem_inference", args + 1, n - 1, 1);
   const Tensor &x = a.tensor();
   const Module stem(args[0]);
-  if (!stem.computes(kStemLayer) || !inference(x) || x.dim() != 4 || x.size(0) * x.size(2) * x.size(3) >= (1ll << 31)) Py_RETURN_NONE;
+  if (!stem.computes(kStemLayer) || a.overridden({0}) || !inference(x) || x.dim() != 4 || x.size(0) * x.size(2) * x.size(3) >= (1ll << 31)) Py_RETURN_NONE;
   const Module norm1 = stem.child("norm1", kSequential), norm2 = stem.child("norm2", kSequential), act = stem.child("act", kGelu);
   Convolution c1, c2;
   if (!norm1 || norm1.child("1") || !norm2.child("1", kToChannelsLast) || norm2.child("2") || !act || !exact_gelu(act) ||
@@ -127,7 +127,7 @@ PyObject *py_downsample(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Tensor &x = a.tensor();
   const int h = a.integer(), w = a.integer();
   const Module m(args[0]);
-  if (!m.computes(kDownsampleLayer) || !inference(x) || !usable_input(x, h, w)) Py_RETURN_NONE;
+  if (!m.computes(kDownsampleLayer) || a.overridden({0}) || !inference(x) || !usable_input(x, h, w)) Py_RETURN_NONE;
   const Module norm = m.child("norm", kSequential);
   Convolution conv;
   if (!norm || !norm.child("0", kToChannelsLast) || !norm.child("2", kToChannelsFirst) || norm.child("3") ||
@@ -165,7 +165,7 @@ PyObject *py_head(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Tensor &x = a.tensor();
   const int h = a.integer(), w = a.integer();
   const Module head(args[0]);
-  if (!inference(x) || !usable_input(x, h, w) || !head.is(kSequential) || head.hooked()) Py_RETURN_NONE;
+  if (a.overridden({0}) || !inference(x) || !usable_input(x, h, w) || !head.is(kSequential) || head.hooked()) Py_RETURN_NONE;
   const Module norm = head.child("1", kSequential), act = head.child("2", kGelu);
   Convolution conv;
   if (!norm || norm.child("1") || !act || !exact_gelu(act) || head.child("3") || !conv.load(head.child("0", kConv2d), x, x.size(2), 1, 1, 0) ||

@@ -282,7 +282,7 @@ PyObject *py_layer_inference(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Args a("layer_inference", args + 1, n - 1, 3);
   const Tensor &x = a.tensor();
   const int h = a.integer(), w = a.integer();
-  if (observed() || functions_replaced() || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks()) Py_RETURN_NONE;
+  if (a.overridden({0}) || observed() || functions_replaced() || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks()) Py_RETURN_NONE;
   if (!usable_input(x, h, w) || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) Py_RETURN_NONE;
   Layer layer;
   if (!layer.load(Module(args[0]), x, x.scalar_type()) || layer.drop_path != 0.0) Py_RETURN_NONE;

@@ -1,6 +1,11 @@
 // The extension module dcnv4_amd._native and the helpers its files share.
 #include <cstdarg>
 
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/PyInterpreter.h>
+
 #include "layers.hpp"
 
 namespace dcn::binding {
@@ -41,6 +46,12 @@ void check_tensor(const Tensor &t, const char *name, at::ScalarType dtype) {
   if (t.scalar_type() != dtype) raise_runtime("%s has dtype %s, expected %s", name, c10::toString(t.scalar_type()), c10::toString(dtype));
 }
 
+bool Args::overridden(std::initializer_list<Py_ssize_t> which) const {
+  for (Py_ssize_t i : which)
+    if (THPVariable_Check(first_[i]) && !THPVariable_CheckExact(first_[i])) return true;
+  return false;
+}
+
 const Tensor &Args::tensor() {
   PyObject *o = *args_++;
   if (!THPVariable_Check(o)) throw c10::TypeError({__func__, __FILE__, (uint32_t)__LINE__}, std::string("expected a Tensor, got ") + Py_TYPE(o)->tp_name);
@@ -70,7 +81,23 @@ float Args::real() {
   return (float)v;
 }
 
-bool observed() { return at::tracer::impl::is_dispatch_enabled(); }
+namespace {
+
+bool function_mode() {
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); ++i) {
+    PyObject *mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+    if (!is_device_context(mode)) return true;
+  }
+  return false;
+}
+
+}  // namespace
+
+bool observed() {
+  return at::tracer::impl::is_dispatch_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || function_mode();
+}
 
 bool in_memory(const Tensor &t) { return t.has_storage() && (t.numel() == 0 || t.const_data_ptr() != nullptr); }
 

@@ -17,6 +17,7 @@ struct Kind {
 };
 Kind g_kinds[kModuleKinds];
 PyObject *g_global_hooks[4] = {};
+PyObject *g_device_context = nullptr;
 constexpr const char *kFunctions[] = {"dcnv4_forward", "dcnv4_backward", "depthwise_conv_forward", "depthwise_conv_backward",
                                       "layer_norm_residual_forward", "layer_norm_residual_backward"};
 constexpr int kFunctionCount = sizeof(kFunctions) / sizeof(kFunctions[0]);
@@ -38,6 +39,9 @@ PyObject *dict_of(PyObject *o) {
 PyObject *item(PyObject *dict, const char *name) {
   return dict != nullptr && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, name_object(name)) : nullptr;
 }
+
+// A tensor that no kernel takes: on another device than any input of theirs.
+Tensor unusable() { return at::empty({0}, at::TensorOptions().device(at::kCPU)); }
 
 }  // namespace
 
@@ -70,12 +74,15 @@ Module Module::child(const char *name, ModuleKind kind) const {
 
 Tensor Module::parameter(const char *name) const {
   PyObject *p = o_ != nullptr ? item(item(dict_of(o_), "_parameters"), name) : nullptr;
-  return p != nullptr && THPVariable_Check(p) ? THPVariable_Unpack(p) : Tensor();
+  if (p == nullptr || !THPVariable_Check(p)) return Tensor();
+  // a parameter of a class of its own (torch's functions call that class) is nothing for the kernels
+  return THPVariable_CheckTypeExact(Py_TYPE(p)) ? THPVariable_Unpack(p) : unusable();
 }
 
 Tensor Module::buffer(const char *name) const {
   PyObject *b = o_ != nullptr ? item(item(dict_of(o_), "_buffers"), name) : nullptr;
-  return b != nullptr && THPVariable_Check(b) ? THPVariable_Unpack(b) : Tensor();
+  if (b == nullptr || !THPVariable_Check(b)) return Tensor();
+  return THPVariable_CheckTypeExact(Py_TYPE(b)) ? THPVariable_Unpack(b) : unusable();
 }
 
 PyObject *Module::attribute(const char *name) const { return o_ != nullptr ? item(dict_of(o_), name) : nullptr; }
@@ -113,6 +120,8 @@ bool global_module_hooks() {
     if (hooks != nullptr && PyDict_Check(hooks) && PyDict_GET_SIZE(hooks) != 0) return true;
   return false;
 }
+
+bool is_device_context(PyObject *mode) { return (PyObject *)Py_TYPE(mode) == g_device_context; }
 
 bool functions_replaced() {
   for (int i = 0; i < kFunctionCount; ++i)
@@ -152,6 +161,11 @@ PyObject *py_register(PyObject *, PyObject *const *args, Py_ssize_t n) {
       Py_XSETREF(k.methods[m], method);
     }
   }
+  PyObject *device = PyImport_ImportModule("torch.utils._device");
+  if (device == nullptr) throw python_error();
+  Py_XSETREF(g_device_context, PyObject_GetAttrString(device, "DeviceContext"));
+  Py_DECREF(device);
+  if (g_device_context == nullptr) throw python_error();
   PyObject *m = PyImport_ImportModule("torch.nn.modules.module");
   if (m == nullptr) throw python_error();
   int i = 0;

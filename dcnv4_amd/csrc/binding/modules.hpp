@@ -31,6 +31,7 @@ class Module {
 };
 
 bool global_module_hooks();
+bool is_device_context(PyObject *mode);
 
 // Whether a program has put a function of its own in place of one of ext's that a FlashInternImage layer calls.
 bool functions_replaced();

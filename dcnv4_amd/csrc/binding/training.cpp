@@ -332,7 +332,7 @@ PyObject *py_layer_training(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Args arg("layer_training", args + 1, n - 1, 3);
   Tensor x = arg.tensor();
   const int h = arg.integer(), w = arg.integer();
-  if (observed() || functions_replaced() || !at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks() || saves_under_hooks() ||
+  if (arg.overridden({0}) || observed() || functions_replaced() || !at::autocast::is_autocast_enabled(at::kCUDA) || global_module_hooks() || saves_under_hooks() ||
       !usable_input(x, h, w))
     Py_RETURN_NONE;
   LayerTraining t;

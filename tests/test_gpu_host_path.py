@@ -360,3 +360,35 @@ def test_wrapped_extension_functions_are_called(monkeypatch):
                 with torch.no_grad():
                     layer.eval()(x, (6, 7))
     assert set(calls) == {"dcnv4_backward", "layer_norm_residual_forward", "depthwise_conv_forward"}
+
+
+def test_modes_and_subclasses_see_a_layers_operators():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    layer, x = _layer().eval(), torch.randn(1, 42, 64, device="cuda").half()
+    products = 2 * 42 * 64 * (64 + 112 + 64 + 8 * 64)
+    with torch.no_grad():
+        with FlopCounterMode(display=False) as counter:
+            layer(x, (6, 7))
+        assert counter.get_total_flops() == products
+        seen = []
+
+        class Watch(TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                seen.append(func)
+                return func(*args, **(kwargs or {}))
+
+        with Watch():
+            layer(x, (6, 7))
+        assert torch.nn.functional.linear in seen
+
+        class Named(torch.Tensor):
+            pass
+
+        assert type(layer(x.as_subclass(Named), (6, 7))) is Named
+
+
+def test_a_default_device_keeps_the_one_call_path():
+    layer, x = _layer(dtype=torch.float32), torch.randn(1, 42, 64, device="cuda")
+    with torch.device("cuda"), torch.autocast("cuda", dtype=torch.float16):
+        assert layer(x, (6, 7)).grad_fn.name() == "InternImageLayerBackward"
