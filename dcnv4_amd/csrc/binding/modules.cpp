@@ -73,9 +73,12 @@ Module Module::child(const char *name, ModuleKind kind) const {
 }
 
 Tensor Module::parameter(const char *name) const {
-  PyObject *p = o_ != nullptr ? item(item(dict_of(o_), "_parameters"), name) : nullptr;
-  if (p == nullptr || !THPVariable_Check(p)) return Tensor();
-  // a parameter of a class of its own (torch's functions call that class) is nothing for the kernels
+  if (o_ == nullptr) return Tensor();
+  PyObject *d = dict_of(o_), *p = item(item(d, "_parameters"), name);
+  if (p == Py_None && item(d, name) == nullptr) return Tensor();
+  // what a program has put in a parameter's place - a plain attribute - is nothing for the kernels, nor is a parameter of a class
+  // of its own, which torch's functions call
+  if (p == nullptr || !THPVariable_Check(p) || item(d, name) != nullptr) return unusable();
   return THPVariable_CheckTypeExact(Py_TYPE(p)) ? THPVariable_Unpack(p) : unusable();
 }
 

@@ -392,3 +392,21 @@ def test_a_default_device_keeps_the_one_call_path():
     layer, x = _layer(dtype=torch.float32), torch.randn(1, 42, 64, device="cuda")
     with torch.device("cuda"), torch.autocast("cuda", dtype=torch.float16):
         assert layer(x, (6, 7)).grad_fn.name() == "InternImageLayerBackward"
+
+
+@pytest.mark.parametrize("kind", ["inference", "autocast", "attention"])
+def test_a_plain_attribute_in_a_parameters_place_is_used(kind):
+    if kind == "attention":
+        m, inputs = _attention()
+        run, linear = lambda: m(*inputs), m.output_proj
+    else:
+        m = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval()
+        x = torch.randn(2, 42, 64, device="cuda", dtype=m.norm1[0].weight.dtype)
+        run, linear = lambda: m(x, (6, 7)), m.mlp.fc1
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+        bias = torch.randn_like(linear.bias)
+        linear.bias.copy_(bias)
+        want = run()
+        del linear.bias
+        linear.bias = bias
+        assert _rel(run(), want) < 3e-3
