@@ -49,7 +49,7 @@ struct Attention {
   Tensor forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
                  const Tensor &padding, AttentionSaved *s) const;
   variable_list backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
-                         const Tensor &padding, const Tensor &grad, const AttentionSaved &s, bool want_query, bool want_features) const;
+                         const Tensor &padding, const Tensor &grad, const AttentionSaved &s, const std::array<bool, kInputs> &want) const;
 };
 
 Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
@@ -125,7 +125,7 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
 
 variable_list Attention::backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
                                   const Tensor &starts, const Tensor &padding, const Tensor &grad, const AttentionSaved &s,
-                                  bool want_query, bool want_features) const {
+                                  const std::array<bool, kInputs> &want) const {
   OnDevice guard(query);
   void *stream = stream_of(query);
   hipStream_t hip = static_cast<hipStream_t>(stream);
@@ -133,6 +133,10 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
   const int64_t n_loc = 2 * logits(), n_log = logits();
   const Arena &a = s.arena;
   variable_list g(kInputs);
+  auto wants = [&](Input weight) { return want[weight] || want[weight + 1]; };
+  // what has to be known of the way back: the gradients of the values, of the offsets, and of anything the operator took
+  const bool into_value = want[kFeatures] || wants(kValueW), into_offsets = want[kQuery] || wants(kOffsetsW);
+  const bool through = into_value || into_offsets || wants(kLogitsW);
 
   Arena t;
   const size_t d_sampled = t.take((size_t)(query_rows() * width) * bytes()), d_value = t.take((size_t)(feature_rows() * width) * bytes()),
@@ -143,17 +147,20 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
   const size_t ws = t.take(ws_bytes);
   t.allocate(query);
 
-  launch(code, product(grad.const_data_ptr(), a.at(s.output_wt), nullptr, query_rows(), width, width, t.at(d_sampled)), stream);
-  check(flash_deform_attn_gfx950_backward_split(a.at(s.value), shapes.const_data_ptr<int64_t>(), starts.const_data_ptr<int64_t>(),
-                                                a.at(s.locations), a.at(s.logits), t.at(d_sampled), t.at(d_value), t.at(d_locations),
-                                                t.at(d_logits), t.at(ws), ws_bytes, code, location_code(), batch, (int)pixels, heads,
-                                                (int)width / heads, levels, (int)queries, points, 64, 0, 0, stream));
-  if (padding.defined())
+  if (through) {
+    launch(code, product(grad.const_data_ptr(), a.at(s.output_wt), nullptr, query_rows(), width, width, t.at(d_sampled)), stream);
+    check(flash_deform_attn_gfx950_backward_split(a.at(s.value), shapes.const_data_ptr<int64_t>(), starts.const_data_ptr<int64_t>(),
+                                                  a.at(s.locations), a.at(s.logits), t.at(d_sampled), t.at(d_value), t.at(d_locations),
+                                                  t.at(d_logits), t.at(ws), ws_bytes, code, location_code(), batch, (int)pixels, heads,
+                                                  (int)width / heads, levels, (int)queries, points, 64, 0, 0, stream));
+  }
+  if (into_value && padding.defined())
     hip_check(launch_zero_rows(bytes(), t.at(d_value), static_cast<const uint8_t *>(padding.const_data_ptr()), feature_rows(), (int)width, hip),
               "padding launch");
-  hip_check(launch_location_grad(code, sampling(reference, shapes), t.at(d_locations), location_code() == DCNV4_DTYPE_F32, t.at(d_offsets),
-                                 query_rows(), (int)n_loc, hip),
-            "location gradient launch");
+  if (into_offsets)
+    hip_check(launch_location_grad(code, sampling(reference, shapes), t.at(d_locations), location_code() == DCNV4_DTYPE_F32, t.at(d_offsets),
+                                   query_rows(), (int)n_loc, hip),
+              "location gradient launch");
   // results in the type of the input: fp32 beside 16-bit products
   auto result = [&](LinearLaunch p, const Tensor &out, bool is32, bool add) {
     LinearProblem &q = p.p[0];
@@ -166,11 +173,11 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
     }
     launch(code, p, stream);
   };
-  if (want_features) {
+  if (want[kFeatures]) {
     g[kFeatures] = at::empty(features.sizes(), features.options());
     result(product(t.at(d_value), a.at(s.value_wt), nullptr, feature_rows(), width, width, nullptr), g[kFeatures], features32, false);
   }
-  if (want_query) {
+  if (want[kQuery]) {
     g[kQuery] = at::empty(query.sizes(), query.options());
     result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc, width, nullptr), g[kQuery], query32, false);
     result(product(t.at(d_logits), a.at(s.logits_wt), nullptr, query_rows(), n_log, width, nullptr), g[kQuery], query32, true);
@@ -178,11 +185,12 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
   const void *q_in = half && query32 ? a.at(s.query) : query.const_data_ptr();
   const void *f_in = half && features32 ? a.at(s.features) : features.const_data_ptr();
   const auto fp32 = params[kValueW].options();
-  const WeightGradient value = {t.at(d_value), f_in, width, width, &params[kValueW], &params[kValueB], &g[kValueW], &g[kValueB]},
-                       offsets = {t.at(d_offsets), q_in, n_loc, width, &params[kOffsetsW], &params[kOffsetsB], &g[kOffsetsW], &g[kOffsetsB]},
-                       logit = {t.at(d_logits), q_in, n_log, width, &params[kLogitsW], &params[kLogitsB], &g[kLogitsW], &g[kLogitsB]},
-                       output = {grad.const_data_ptr(), a.at(s.sampled), width, width, &params[kOutputW], &params[kOutputB], &g[kOutputW],
-                                 &g[kOutputB]};
+  auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n) -> WeightGradient {
+    return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1]};
+  };
+  const WeightGradient value = gradient(kValueW, t.at(d_value), f_in, width), offsets = gradient(kOffsetsW, t.at(d_offsets), q_in, n_loc),
+                       logit = gradient(kLogitsW, t.at(d_logits), q_in, n_log),
+                       output = gradient(kOutputW, grad.const_data_ptr(), a.at(s.sampled), width);
   if (query_rows() == feature_rows()) {
     weight_gradients(code, query_rows(), fp32, {output, offsets, value, logit}, stream);
   } else {
@@ -211,8 +219,9 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
       at::AutoGradMode no_grad(false);
       Tensor v[6];
       for (int i = 0; i < 6; ++i) v[i] = inputs[i].unpack();
-      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0], true), saved, task_should_compute_output(kQuery),
-                           task_should_compute_output(kFeatures));
+      std::array<bool, kInputs> want;
+      for (size_t i = 0; i < kInputs; ++i) want[i] = task_should_compute_output(i);
+      out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0], true), saved, want);
     }
     return once_differentiable(std::move(out));
   }
@@ -229,7 +238,9 @@ bool load(const Module &m, Attention *a, Input weight, int64_t in, int64_t out, 
   if (!m) return false;
   a->params[weight] = m.parameter("weight");
   a->params[weight + 1] = m.parameter("bias");
-  return usable(a->params[weight], like, at::kFloat, in * out, false) && usable(a->params[weight + 1], like, at::kFloat, out, true);
+  const Tensor &w = a->params[weight], &b = a->params[weight + 1];
+  return w.defined() && w.dim() == 2 && w.size(1) == in && (!b.defined() || b.dim() == 1) && usable(w, like, at::kFloat, in * out, false) &&
+         usable(b, like, at::kFloat, out, true);
 }
 
 // attention_layer(module, query, reference_points, input_flatten, spatial_shapes, level_start_index, padding or None): the

@@ -32,7 +32,7 @@ bool load_linear(const Module &m, const Tensor &x, at::ScalarType dtype, int64_t
   if (!m) return false;
   *w = m.parameter("weight");
   *b = m.parameter("bias");
-  return usable(*w, x, dtype, in * out, false) && usable(*b, x, dtype, out, true);
+  return w->defined() && w->dim() == 2 && w->size(1) == in && usable(*w, x, dtype, in * out, false) && usable(*b, x, dtype, out, true);
 }
 
 }  // namespace
@@ -108,12 +108,17 @@ void hip_check(hipError_t e, const char *what) {
 void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream) {
   WeightGradLaunch launch = {};
   launch.rows = rows;
+  struct { Tensor weight, bias; } grads[kMaxWeightGrads];
   for (const WeightGradient &l : layers) {
-    *l.grad_w = at::empty(l.weight->sizes(), fp32);
-    if (l.bias->defined()) *l.grad_b = at::empty(l.bias->sizes(), fp32);
+    if (!l.want_w && !l.want_b) continue;
+    auto &g = grads[launch.count];
+    g.weight = at::empty(l.weight->sizes(), fp32);
+    if (l.want_w) *l.grad_w = g.weight;
+    if (l.want_b) *l.grad_b = g.bias = at::empty(l.bias->sizes(), fp32);
     WeightGradProblem &q = launch.p[launch.count++];
     q.grad_out = l.grad_out; q.in = l.in; q.n = (int)l.n; q.k = (int)l.k;
   }
+  if (launch.count == 0) return;
   const WeightGradPlan plan = plan_weight_grad(code, launch);
   launch.splits = plan.splits;
   // one split writes the gradients themselves, several their partial sums
@@ -124,24 +129,23 @@ void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std
     reduce.s[reduce.count++] = {static_cast<float *>(grad.data_ptr()), floats, (int)grad.numel()};
     floats += (size_t)(grad.numel() + 3) / 4 * 4;
   };
-  for (const WeightGradient &l : layers) {
-    place(*l.grad_w);
-    if (l.bias->defined()) place(*l.grad_b);
+  for (int i = 0; i < launch.count; ++i) {
+    place(grads[i].weight);
+    if (grads[i].bias.defined()) place(grads[i].bias);
   }
   Tensor partial;
   if (plan.splits > 1) partial = at::empty({(int64_t)(floats * plan.splits)}, fp32);
   float *base = plan.splits > 1 ? static_cast<float *>(partial.data_ptr()) : nullptr;
   reduce.partial = base;
   reduce.split_stride = launch.split_stride = floats;
-  int segment = 0, i = 0;
+  int segment = 0;
   auto target = [&] {
     const WeightGradSegment &s = reduce.s[segment++];
     return base != nullptr ? base + s.offset : s.grad;
   };
-  for (const WeightGradient &l : layers) {
+  for (int i = 0; i < launch.count; ++i) {
     launch.p[i].grad_w = target();
-    if (l.bias->defined()) launch.p[i].grad_bias = target();
-    ++i;
+    if (grads[i].bias.defined()) launch.p[i].grad_bias = target();
   }
   hip_check(launch_weight_grad(code, launch, plan.tile, static_cast<hipStream_t>(stream)), "weight gradient launch");
   if (plan.splits > 1) hip_check(launch_weight_grad_reduce(reduce, static_cast<hipStream_t>(stream)), "weight gradient sum launch");

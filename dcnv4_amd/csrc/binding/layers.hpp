@@ -55,12 +55,14 @@ class Arena {
   Tensor storage_;
 };
 
-// A linear layer's parameter gradients: grad_out [rows, n], in [rows, k]; *grad_w and *grad_b are allocated in fp32.
+// A linear layer's parameter gradients: grad_out [rows, n], in [rows, k]; *grad_w and *grad_b are allocated in fp32 where wanted.
+// (A bias alone is summed beside the product as the two are, the product is dropped.)
 struct WeightGradient {
   const void *grad_out, *in;
   int64_t n, k;
   const Tensor *weight, *bias;
   Tensor *grad_w, *grad_b;
+  bool want_w, want_b;
 };
 void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream);
 

@@ -22,6 +22,8 @@ namespace {
 enum Input { kX, kNorm1W, kNorm1B, kGamma1, kNorm2W, kNorm2B, kGamma2, kValueW, kValueB, kOffsetW, kOffsetB, kOutputW, kOutputB, kDwW,
              kDwB, kFc1W, kFc1B, kFc2W, kFc2B, kInputs };
 
+typedef std::array<bool, kInputs> Wanted;      // the gradients that the backward is asked for
+
 struct Saved {
   Arena arena;
   // offsets into the arena
@@ -64,17 +66,17 @@ struct LayerTraining {
     hip_check(launch_layer_norm_mixed(code(), y32, out32, p, static_cast<hipStream_t>(stream)), "layer norm launch");
   }
 
-  // grad_y in y's type, parameter gradients in fp32
+  // grad_y in y's type, the wanted parameter gradients in fp32: of weight, of the bias behind it and of gamma
   void normalise_backward(const NormParams &n, const void *grad, bool grad32, const void *y, bool y32, void *grad_y, const void *addend,
-                          const Tensor &gamma, const Tensor &scale, Tensor &grad_w, Tensor &grad_b, Tensor *grad_gamma, void *stream) const {
+                          const Tensor &gamma, const Tensor &scale, variable_list &g, const Wanted &want, Input weight, Input gamma_input,
+                          void *stream) const {
     LnLaunch p = norm(n, y32);
     const Tensor partial = at::empty({(int64_t)p.n_part * 3 * l.channels}, n.weight.options());
-    grad_w = at::empty({l.channels}, n.weight.options());
-    grad_b = at::empty({l.channels}, n.weight.options());
-    if (gamma.defined()) *grad_gamma = at::empty({l.channels}, n.weight.options());
+    for (Input i : {weight, Input(weight + 1), gamma_input})
+      if (want[i]) g[i] = at::empty({l.channels}, n.weight.options());
     p.grad_out = grad; p.y = y; p.grad_y = grad_y; p.addend = addend; p.gamma = ptr(gamma);
     p.row_scale = static_cast<const float *>(ptr(scale));
-    p.grad_weight = ptr(grad_w); p.grad_bias = ptr(grad_b); p.grad_gamma = gamma.defined() ? ptr(*grad_gamma) : nullptr;
+    p.grad_weight = ptr(g[weight]); p.grad_bias = ptr(g[weight + 1]); p.grad_gamma = ptr(g[gamma_input]);
     p.partial = static_cast<float *>(partial.data_ptr());
     hip_check(launch_layer_norm_mixed_backward(code(), grad32, y32, p, static_cast<hipStream_t>(stream)), "layer norm backward launch");
   }
@@ -87,7 +89,7 @@ struct LayerTraining {
   }
 
   Tensor forward(const Tensor &x, Saved *s) const;
-  variable_list backward(const Tensor &x, const Tensor &grad, const Saved &s) const;
+  variable_list backward(const Tensor &x, const Tensor &grad, const Saved &s, const Wanted &want) const;
 };
 
 Tensor LayerTraining::forward(const Tensor &x, Saved *s) const {
@@ -192,7 +194,7 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s) const {
   return out;
 }
 
-variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const Saved &s) const {
+variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const Saved &s, const Wanted &want) const {
   OnDevice guard(x);
   void *stream = stream_of(x);
   const int c16 = code();
@@ -201,6 +203,13 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   const size_t act = (size_t)(rows * c) * 2, om = (size_t)(rows * l.row) * 2, hid = (size_t)(rows * l.hidden) * 2;
   const Arena &a = s.arena;
   variable_list g(kInputs);
+  auto wants = [&](Input weight) { return want[weight] || want[weight + 1]; };
+  // how far back the gradient has to go: to the input of the DCNv4 half, of its depthwise layer, through the operator, to the
+  // projection behind it, to the MLP's input and to its hidden tensor
+  const bool into_x = want[kX] || (!l.post_norm && wants(kNorm1W)), into_pre = into_x || wants(kDwW);
+  const bool through = into_pre || wants(kValueW) || wants(kOffsetW);
+  const bool into_mid = through || wants(kOutputW) || (l.post_norm && (wants(kNorm1W) || want[kGamma1]));
+  const bool into_mlp = into_mid || (!l.post_norm && wants(kNorm2W)), into_hidden = into_mlp || wants(kFc1W);
 
   Arena t;
   const bool alias_last = !l.post_norm && !stream32 && !s.scale2.defined();      // the half gradient is grad itself
@@ -212,72 +221,86 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   // MLP half
   const void *last = alias_last ? grad.const_data_ptr() : t.at(d_last);
   if (l.post_norm)
-    normalise_backward(l.norm2, grad.const_data_ptr(), true, a.at(s.last), false, t.at(d_last), nullptr, l.gamma2, s.scale2, g[kNorm2W],
-                       g[kNorm2B], &g[kGamma2], stream);
+    normalise_backward(l.norm2, grad.const_data_ptr(), true, a.at(s.last), false, t.at(d_last), nullptr, l.gamma2, s.scale2, g, want,
+                       kNorm2W, kGamma2, stream);
   else if (!alias_last)
     narrow(grad.const_data_ptr(), stream32, t.at(d_last), s.scale2, stream);
-  LinearLaunch p = product(last, a.at(s.w_fc2_t), nullptr, c, l.hidden, t.at(d_hidden));
-  p.p[0].gelu_grad_at = a.at(s.hidden_pre);
-  launch(c16, p, stream);
-  p = product(t.at(d_hidden), a.at(s.w_fc1_t), nullptr, l.hidden, c, nullptr);
-  if (l.post_norm) {
-    p.p[0].residual32 = static_cast<const float *>(grad.const_data_ptr());
-    p.p[0].out32 = static_cast<float *>(t.at(d_mid));
+  if (into_hidden) {
+    LinearLaunch p = product(last, a.at(s.w_fc2_t), nullptr, c, l.hidden, t.at(d_hidden));
+    p.p[0].gelu_grad_at = a.at(s.hidden_pre);
     launch(c16, p, stream);
-    normalise_backward(l.norm1, t.at(d_mid), true, a.at(s.projected), false, t.at(d_projected), nullptr, l.gamma1, s.scale1, g[kNorm1W],
-                       g[kNorm1B], &g[kGamma1], stream);
-  } else {
-    p.p[0].out = t.at(d_half);
-    launch(c16, p, stream);
-    normalise_backward(l.norm2, t.at(d_half), false, s.mid.const_data_ptr(), stream32, t.at(d_mid), grad.const_data_ptr(), Tensor(),
-                       Tensor(), g[kNorm2W], g[kNorm2B], nullptr, stream);
+  }
+  if (into_mlp) {
+    LinearLaunch p = product(t.at(d_hidden), a.at(s.w_fc1_t), nullptr, l.hidden, c, nullptr);
+    if (l.post_norm) {
+      p.p[0].residual32 = static_cast<const float *>(grad.const_data_ptr());
+      p.p[0].out32 = static_cast<float *>(t.at(d_mid));
+      launch(c16, p, stream);
+      normalise_backward(l.norm1, t.at(d_mid), true, a.at(s.projected), false, t.at(d_projected), nullptr, l.gamma1, s.scale1, g, want,
+                         kNorm1W, kGamma1, stream);
+    } else {
+      p.p[0].out = t.at(d_half);
+      launch(c16, p, stream);
+      normalise_backward(l.norm2, t.at(d_half), false, s.mid.const_data_ptr(), stream32, t.at(d_mid), grad.const_data_ptr(), Tensor(),
+                         Tensor(), g, want, kNorm2W, kGamma2, stream);
+    }
   }
   // DCNv4 half
   const void *projected = t.at(d_projected);
-  if (!l.post_norm) {
+  if (!l.post_norm && into_mid) {
     if (!stream32 && !s.scale1.defined()) projected = t.at(d_mid);
     else narrow(t.at(d_mid), stream32, t.at(d_projected), s.scale1, stream);
   }
-  launch(c16, product(projected, a.at(s.w_output_t), nullptr, c, c, t.at(d_sampled)), stream);
-  const size_t ws_bytes = dcnv4_gfx950_backward_workspace_bytes(c16, batch, h, w, l.group, l.group_channels);
-  const Tensor ws = workspace(ws_bytes, x);
-  check(dcnv4_gfx950_backward(a.at(s.value), a.at(s.offsets), t.at(d_sampled), t.at(d_value), t.at(d_offsets), ptr(ws), ws_bytes, c16,
-                              batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad, l.pad, l.dilation, l.dilation,
-                              l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
-  launch(c16, product(t.at(d_offsets), a.at(s.w_offset_t), nullptr, l.row, c, t.at(d_pre)), stream);
-  const void *into_x = t.at(d_pre);
-  if (l.dw_kernel) {
+  if (through) {
+    launch(c16, product(projected, a.at(s.w_output_t), nullptr, c, c, t.at(d_sampled)), stream);
+    const size_t ws_bytes = dcnv4_gfx950_backward_workspace_bytes(c16, batch, h, w, l.group, l.group_channels);
+    const Tensor ws = workspace(ws_bytes, x);
+    check(dcnv4_gfx950_backward(a.at(s.value), a.at(s.offsets), t.at(d_sampled), t.at(d_value), t.at(d_offsets), ptr(ws), ws_bytes, c16,
+                                batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad, l.pad, l.dilation, l.dilation,
+                                l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
+  }
+  const void *side = t.at(d_pre);      // what reaches x through the offsets
+  if (into_pre) launch(c16, product(t.at(d_offsets), a.at(s.w_offset_t), nullptr, l.row, c, t.at(d_pre)), stream);
+  if (into_pre && l.dw_kernel) {
     const int pad = (l.dw_kernel - 1) / 2;
     const size_t dw_bytes = dcnv4_gfx950_depthwise_conv_backward_workspace_bytes(c16, batch, h, w, (int)c, l.dw_kernel, pad);
     const Tensor dw_ws = workspace(dw_bytes, x);
-    g[kDwW] = at::empty(l.dw_w.sizes(), f32);
-    if (l.dw_b.defined()) g[kDwB] = at::empty({c}, f32);
-    check(depthwise_backward_fp32_grads(a.at(s.half_x), a.at(s.w_dw), t.at(d_pre), t.at(d_dw), static_cast<float *>(ptr(g[kDwW])),
-                                        static_cast<float *>(ptr(g[kDwB])), ptr(dw_ws), dw_bytes, c16, batch, h, w, (int)c, l.dw_kernel,
-                                        pad, stream));
-    into_x = t.at(d_dw);
+    // the kernel gives the bias's gradient beside the weight's
+    Tensor grad_w;
+    if (wants(kDwW)) grad_w = at::empty(l.dw_w.sizes(), f32);
+    if (want[kDwW]) g[kDwW] = grad_w;
+    if (want[kDwB]) g[kDwB] = at::empty({c}, f32);
+    check(depthwise_backward_fp32_grads(a.at(s.half_x), a.at(s.w_dw), t.at(d_pre), into_x ? t.at(d_dw) : nullptr,
+                                        static_cast<float *>(ptr(grad_w)), static_cast<float *>(ptr(g[kDwB])), ptr(dw_ws), dw_bytes, c16,
+                                        batch, h, w, (int)c, l.dw_kernel, pad, stream));
+    side = t.at(d_dw);
   }
-  g[kX] = at::empty(x.sizes(), x.options());
-  p = product(t.at(d_value), a.at(s.w_value_t), nullptr, c, c, nullptr);
-  p.p[0].residual = into_x;
-  if (l.post_norm) {
-    p.p[0].residual32 = static_cast<const float *>(t.at(d_mid));
-    p.p[0].out32 = static_cast<float *>(g[kX].data_ptr());
-    launch(c16, p, stream);
-  } else {
-    p.p[0].out = t.at(d_half);
-    launch(c16, p, stream);
-    normalise_backward(l.norm1, t.at(d_half), false, x.const_data_ptr(), stream32, g[kX].data_ptr(), t.at(d_mid), Tensor(), Tensor(),
-                       g[kNorm1W], g[kNorm1B], nullptr, stream);
+  if (into_x) {
+    g[kX] = at::empty(x.sizes(), x.options());
+    LinearLaunch p = product(t.at(d_value), a.at(s.w_value_t), nullptr, c, c, nullptr);
+    p.p[0].residual = side;
+    if (l.post_norm) {
+      p.p[0].residual32 = static_cast<const float *>(t.at(d_mid));
+      p.p[0].out32 = static_cast<float *>(g[kX].data_ptr());
+      launch(c16, p, stream);
+    } else {
+      p.p[0].out = t.at(d_half);
+      launch(c16, p, stream);
+      normalise_backward(l.norm1, t.at(d_half), false, x.const_data_ptr(), stream32, g[kX].data_ptr(), t.at(d_mid), Tensor(), Tensor(), g,
+                         want, kNorm1W, kGamma1, stream);
+    }
   }
 
-  // all weight and bias gradients
+  // the weight and bias gradients, all in one
+  auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n, int64_t k, const Tensor &wt, const Tensor &b) -> WeightGradient {
+    return {grad_out, in, n, k, &wt, &b, &g[weight], &g[weight + 1], want[weight], want[weight + 1]};
+  };
   weight_gradients(c16, rows, f32,
-                   {{last, a.at(s.hidden), c, l.hidden, &l.fc2_w, &l.fc2_b, &g[kFc2W], &g[kFc2B]},
-                    {t.at(d_hidden), a.at(s.half_mid), l.hidden, c, &l.fc1_w, &l.fc1_b, &g[kFc1W], &g[kFc1B]},
-                    {projected, a.at(s.sampled), c, c, &l.output_w, &l.output_b, &g[kOutputW], &g[kOutputB]},
-                    {t.at(d_value), a.at(s.half_x), c, c, &l.value_w, &l.value_b, &g[kValueW], &g[kValueB]},
-                    {t.at(d_offsets), a.at(s.pre), l.row, c, &l.offset_w, &l.offset_b, &g[kOffsetW], &g[kOffsetB]}},
+                   {gradient(kFc2W, last, a.at(s.hidden), c, l.hidden, l.fc2_w, l.fc2_b),
+                    gradient(kFc1W, t.at(d_hidden), a.at(s.half_mid), l.hidden, c, l.fc1_w, l.fc1_b),
+                    gradient(kOutputW, projected, a.at(s.sampled), c, c, l.output_w, l.output_b),
+                    gradient(kValueW, t.at(d_value), a.at(s.half_x), c, c, l.value_w, l.value_b),
+                    gradient(kOffsetW, t.at(d_offsets), a.at(s.pre), l.row, c, l.offset_w, l.offset_b)},
                    stream);
   return g;
 }
@@ -317,7 +340,9 @@ struct InternImageLayerBackward final : torch::autograd::Node {
       std::array<Tensor *, 6> into = {&now.l.norm1.weight, &now.l.norm1.bias, &now.l.gamma1, &now.l.norm2.weight, &now.l.norm2.bias,
                                       &now.l.gamma2};
       for (int i = 0; i < 6; ++i) *into[i] = params[i].unpack();
-      out = now.backward(x.unpack(), incoming(grads[0], true), saved);
+      Wanted want;
+      for (size_t i = 0; i < kInputs; ++i) want[i] = task_should_compute_output(i);
+      out = now.backward(x.unpack(), incoming(grads[0], true), saved, want);
     }
     return once_differentiable(std::move(out));
   }

@@ -341,6 +341,7 @@ hipError_t launch_bwd_t(const LnLaunch &p, hipStream_t stream) {
     default: return hipErrorInvalidValue;
   }
   if (hipError_t e = hipGetLastError()) return e;
+  if (p.grad_weight == nullptr && p.grad_bias == nullptr && p.grad_gamma == nullptr) return hipSuccess;
   hipLaunchKernelGGL((layer_norm_param_grad_kernel<P>), dim3((unsigned)((3 * p.C + kPgCols - 1) / kPgCols)), dim3(kPgCols * kPgRows), 0, stream, p);
   return hipGetLastError();
 }
