@@ -47,13 +47,13 @@ struct Attention {
     return p;
   }
   Tensor forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
-                 const Tensor &padding, AttentionSaved *s) const;
+                 const Tensor &padding, AttentionSaved *s, bool keep) const;      // keep: a backward will follow
   variable_list backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes, const Tensor &starts,
                          const Tensor &padding, const Tensor &grad, const AttentionSaved &s, const std::array<bool, kInputs> &want) const;
 };
 
 Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
-                          const Tensor &starts, const Tensor &padding, AttentionSaved *s) const {
+                          const Tensor &starts, const Tensor &padding, AttentionSaved *s, bool keep) const {
   OnDevice guard(query);
   void *stream = stream_of(query);
   const bool half = code != DCNV4_DTYPE_F32;
@@ -66,12 +66,12 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
   s->logits = a.take((size_t)(query_rows() * n_log) * bytes());
   s->sampled = a.take((size_t)(query_rows() * width) * bytes());
 
-  // parameters in the products' type, and their matrices turned for the backward
+  // parameters in the products' type, and their matrices turned for a backward
   CastWeightsLaunch cast = {};
   size_t as_is[kInputs], turned[kInputs];
   auto narrowed = [&](Input i, int64_t n, int64_t k) {
     as_is[i] = half ? a.take((size_t)(n * k) * 2) : 0;
-    turned[i] = n > 1 ? a.take((size_t)(n * k) * bytes()) : 0;
+    turned[i] = n > 1 && keep ? a.take((size_t)(n * k) * bytes()) : 0;
   };
   narrowed(kValueW, width, width);
   narrowed(kOffsetsW, n_loc, width);
@@ -83,16 +83,16 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
   s->value_wt = turned[kValueW]; s->offsets_wt = turned[kOffsetsW]; s->logits_wt = turned[kLogitsW]; s->output_wt = turned[kOutputW];
   for (int i = kValueW; i < kInputs; ++i) {
     const Tensor &t = params[i];
-    const bool matrix = t.defined() && t.dim() == 2;
-    if (!t.defined() || (!half && !matrix)) continue;
+    const bool matrix = t.defined() && t.dim() == 2, turn = matrix && keep;
+    if (!t.defined() || (!half && !turn)) continue;
     CastWeights &q = cast.p[cast.count++];
     q.from = static_cast<const float *>(t.const_data_ptr());
     q.to = half ? a.at(as_is[i]) : nullptr;
-    q.turned = matrix ? a.at(turned[i]) : nullptr;
+    q.turned = turn ? a.at(turned[i]) : nullptr;
     q.n = matrix ? (int)t.size(0) : 1;
     q.k = matrix ? (int)t.size(1) : (int)t.numel();
   }
-  hip_check(launch_cast_weights(code, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
+  if (cast.count > 0) hip_check(launch_cast_weights(code, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
   auto param = [&](Input i) -> const void * { return !params[i].defined() ? nullptr : half ? a.at(as_is[i]) : params[i].const_data_ptr(); };
   auto input = [&](const Tensor &t, bool is32, size_t at, int64_t rows) -> const void * {
     if (!half || !is32) return t.const_data_ptr();
@@ -297,7 +297,7 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     AttentionSaved saved;
     {
       at::AutoGradMode no_grad(false);
-      out = a.forward(query, reference, features, shapes, starts, padding, &saved);
+      out = a.forward(query, reference, features, shapes, starts, padding, &saved, wanted);
     }
     if (wanted) {
       std::shared_ptr<FlashDeformAttnBackward> node(new FlashDeformAttnBackward(), torch::autograd::deleteNode);

@@ -88,11 +88,11 @@ struct LayerTraining {
               "conversion launch");
   }
 
-  Tensor forward(const Tensor &x, Saved *s) const;
+  Tensor forward(const Tensor &x, Saved *s, bool keep) const;      // keep: a backward will follow
   variable_list backward(const Tensor &x, const Tensor &grad, const Saved &s, const Wanted &want) const;
 };
 
-Tensor LayerTraining::forward(const Tensor &x, Saved *s) const {
+Tensor LayerTraining::forward(const Tensor &x, Saved *s, bool keep) const {
   OnDevice guard(x);
   void *stream = stream_of(x);
   const int c16 = code();
@@ -106,15 +106,16 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s) const {
   s->sampled = a.take(act);
   s->projected = l.post_norm ? a.take(act) : 0;
   s->half_mid = a.take(act);
-  s->hidden_pre = a.take(hid);
+  s->hidden_pre = keep ? a.take(hid) : 0;
   s->hidden = a.take(hid);
   s->last = l.post_norm ? a.take(act) : 0;
 
-  // 16-bit parameters: as they lie for the forward, turned for the backward
+  // 16-bit parameters: as they lie for the forward, turned for a backward
   CastWeightsLaunch cast = {};
   struct Narrowed { size_t as_is, turned; };
   std::vector<std::pair<int, Narrowed>> placed;
   auto matrix = [&](const Tensor &t, int64_t n, int64_t k, bool turned) {
+    turned = turned && keep;
     const Narrowed at = {a.take((size_t)(n * k) * 2), turned ? a.take((size_t)(n * k) * 2) : 0};
     CastWeights &q = cast.p[cast.count];
     q.from = static_cast<const float *>(t.const_data_ptr()); q.n = (int)n; q.k = (int)k;
@@ -182,7 +183,7 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s) const {
   // MLP half
   LinearLaunch fc1 = product(a.at(s->half_mid), a.at(fc1_w.as_is), bias(fc1_b), c, l.hidden, a.at(s->hidden));
   fc1.gelu = 1;
-  fc1.p[0].pre = a.at(s->hidden_pre);
+  fc1.p[0].pre = keep ? a.at(s->hidden_pre) : nullptr;
   launch(c16, fc1, stream);
   const LinearLaunch fc2 = product(a.at(s->hidden), a.at(fc2_w.as_is), bias(fc2_b), l.hidden, c, l.post_norm ? a.at(s->last) : nullptr);
   if (l.post_norm) {
@@ -388,7 +389,7 @@ PyObject *py_layer_training(PyObject *, PyObject *const *args, Py_ssize_t n) {
         saved.scale1 = factors();
         saved.scale2 = factors();
       }
-      out = t.forward(x, &saved);
+      out = t.forward(x, &saved, wanted);
     }
     if (wanted) {
       std::shared_ptr<InternImageLayerBackward> node(new InternImageLayerBackward(), torch::autograd::deleteNode);

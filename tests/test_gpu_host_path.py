@@ -464,3 +464,24 @@ def test_each_gradient_alone_is_what_it_is_among_all(kind):
     every = torch.autograd.grad(out, wanted, grad, retain_graph=True)
     for t, want in zip(wanted, every):
         assert _rel(torch.autograd.grad(out, t, grad, retain_graph=True)[0], want) < HALF_ULP
+
+
+@pytest.mark.parametrize("kind", ["layer", "attention", "attention fp32"])
+def test_a_forward_without_gradients_keeps_nothing_for_a_backward(kind):
+    if kind == "layer":
+        m, x = _layer(channels=256, dtype=torch.float32).eval(), torch.randn(2, 1024, 256, device="cuda")
+        run, hidden = lambda: m(x, (32, 32)), 2 * 2 * 1024 * 1024
+    else:
+        m, inputs = _attention(width=512)
+        run, hidden = lambda: m(*inputs), 0
+
+    def forward():
+        with torch.autocast("cuda", dtype=torch.float16, enabled=kind != "attention fp32"):
+            return run()
+
+    forward()
+    with torch.no_grad():
+        peak, got = _peak(forward)
+    trained, want = _peak(forward)
+    turned = (4 if kind == "attention fp32" else 2) * sum(p.numel() for p in m.parameters() if p.dim() == 2)
+    assert peak <= trained - turned - hidden and torch.equal(got, want)
