@@ -75,8 +75,12 @@ __device__ __forceinline__ NormalTail normal_tail(float x) {
 template <typename Tag>
 __device__ __forceinline__ float gelu_exact(float x) {
   if constexpr (Tag::kBytes == 4) return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));      // an fp32 result keeps fp32 precision
-  // max(x, 0) as integers, one instruction (fmaxf costs another to quiet a NaN, which the product carries through here)
-  else return fmaf(-fabsf(x), normal_tail(x).tail, __builtin_bit_cast(float, max(__builtin_bit_cast(int, x), 0)));
+  // max(x, 0) as integers, one instruction (fmaxf costs another to quiet a NaN, which the product carries through here), and so is
+  // the largest finite number in the place of an infinite x, whose tail of zero would give NaN
+  else {
+    const int bits = __builtin_bit_cast(int, x);
+    return fmaf(-fabsf(__builtin_bit_cast(float, min(bits, 0x7f7fffff))), normal_tail(x).tail, __builtin_bit_cast(float, max(bits, 0)));
+  }
 }
 // Phi(x) + x phi(x)
 __device__ __forceinline__ float gelu_derivative(float x) {

@@ -195,3 +195,15 @@ def test_fp32_linear_matches_fp64(rows, depth, width):
     product = a.double() @ w.double().t() + b.double()
     assert _rel(ext.linear_forward(a, w, b), product) < 1e-6
     assert _rel(ext.linear_forward(a, w, b, gelu=True), torch.nn.functional.gelu(product)) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["fp16", "bf16", "fp32"])
+@pytest.mark.parametrize("rows", [3, 9000], ids=["few", "tiled"])
+def test_gelu_epilogue_of_infinities_and_nan_is_the_frameworks(rows, dtype):
+    from dcnv4_amd import ext
+    a = torch.zeros(rows, 8, device="cuda", dtype=dtype)
+    a[:3, 0] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    w = torch.ones(64, 8, device="cuda", dtype=dtype)
+    got = ext.linear_forward(a, w, gelu=True)[:3, 0]
+    assert got.isnan().tolist() == [False, True, True] and got[0] == float("inf")
+    assert torch.equal(got.isnan(), torch.nn.functional.gelu(a[:3, 0]).isnan())
