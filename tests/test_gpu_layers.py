@@ -207,3 +207,21 @@ def test_gelu_epilogue_of_infinities_and_nan_is_the_frameworks(rows, dtype):
     got = ext.linear_forward(a, w, gelu=True)[:3, 0]
     assert got.isnan().tolist() == [False, True, True] and got[0] == float("inf")
     assert torch.equal(got.isnan(), torch.nn.functional.gelu(a[:3, 0]).isnan())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_gelu_epilogue_is_as_exact_as_the_fp32_function(dtype):
+    """Every input of the type up to the end of its negative tail: the results' distance from 64 bits is no larger than that of the
+    framework's function, which evaluates erf in fp32 and rounds once."""
+    from dcnv4_amd import ext
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype).cuda()
+    x = x[(x.abs() < 13) & (x != 0)]
+    a = torch.zeros(x.numel(), 8, device="cuda", dtype=dtype)
+    a[:, 0] = x
+    w = torch.zeros(8, 8, device="cuda", dtype=dtype)
+    w[0, 0] = 1.0
+    got = ext.linear_forward(a, w, gelu=True)[:, 0]
+    exact = x.double() * torch.special.ndtr(x.double())
+    framework = torch.nn.functional.gelu(x)
+    assert _rel(got, exact) <= _rel(framework, exact)
+    assert (got != exact.to(dtype)).sum() <= (framework != exact.to(dtype)).sum()
