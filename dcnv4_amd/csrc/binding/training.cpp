@@ -216,7 +216,7 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   const bool alias_last = !l.post_norm && !stream32 && !s.scale2.defined();      // the half gradient is grad itself
   const size_t d_last = alias_last ? 0 : t.take(act), d_hidden = t.take(hid), d_projected = t.take(act), d_sampled = t.take(act),
                d_value = t.take(act), d_offsets = t.take(om), d_pre = t.take(act), d_dw = l.dw_kernel ? t.take(act) : 0,
-               d_half = l.post_norm ? 0 : t.take(act), d_mid = t.take(stream32 ? 2 * act : act);
+               d_half = l.post_norm ? 0 : t.take(2 * act), d_mid = t.take(stream32 ? 2 * act : act);
   t.allocate(x);
 
   // MLP half
@@ -285,9 +285,10 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
       p.p[0].out32 = static_cast<float *>(g[kX].data_ptr());
       launch(c16, p, stream);
     } else {
-      p.p[0].out = t.at(d_half);
+      // two gradients meet here, as in the composition in fp32
+      p.p[0].out32 = static_cast<float *>(t.at(d_half));
       launch(c16, p, stream);
-      normalise_backward(l.norm1, t.at(d_half), false, x.const_data_ptr(), stream32, g[kX].data_ptr(), t.at(d_mid), Tensor(), Tensor(), g,
+      normalise_backward(l.norm1, t.at(d_half), true, x.const_data_ptr(), stream32, g[kX].data_ptr(), t.at(d_mid), Tensor(), Tensor(), g,
                          want, kNorm1W, kGamma1, stream);
     }
   }

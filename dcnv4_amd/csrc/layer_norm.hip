@@ -347,7 +347,7 @@ hipError_t launch_bwd_t(const LnLaunch &p, hipStream_t stream) {
 }
 
 // Mixed precision: parameters in fp32, H the 16-bit type.  Forward: a 16-bit tensor into an fp32 stream (post-norm) or into
-// 16 bits, an fp32 stream into 16 bits (pre-norm).  Backward: the same, from the result's type.
+// 16 bits, an fp32 stream into 16 bits (pre-norm).  Backward: the same, from a gradient of either type (in fp32 where it is a sum).
 template <typename H>
 hipError_t launch_mixed_t(const LnLaunch &p, bool y32, bool r32, hipStream_t stream) {
   if (y32) return r32 ? hipErrorInvalidValue : launch_t<F32, H, F32>(p, stream);
@@ -355,7 +355,7 @@ hipError_t launch_mixed_t(const LnLaunch &p, bool y32, bool r32, hipStream_t str
 }
 template <typename H>
 hipError_t launch_mixed_bwd_t(const LnLaunch &p, bool g32, bool y32, hipStream_t stream) {
-  if (y32) return g32 ? hipErrorInvalidValue : launch_bwd_t<H, F32, F32, F32>(p, stream);
+  if (y32) return g32 ? launch_bwd_t<F32, F32, F32, F32>(p, stream) : launch_bwd_t<H, F32, F32, F32>(p, stream);
   return g32 ? launch_bwd_t<F32, H, H, F32>(p, stream) : launch_bwd_t<H, H, H, F32>(p, stream);
 }
 
