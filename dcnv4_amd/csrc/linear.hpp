@@ -114,12 +114,14 @@ struct CastWeightsLaunch {
   int count;
 };
 hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &p, hipStream_t stream);
-// dst = 16-bit src (fp32, or 16-bit with a factor per sample of scale_elements elements); n and scale_elements multiples of 8
 // grad_offsets (dtype) from the gradients of the locations (fp32, or the dtype): the backward of SamplingLocations.
 hipError_t launch_location_grad(int dtype, const SamplingLocations &l, const void *grad_locations, bool locations32, void *grad_offsets,
                                 long long rows, int n, hipStream_t stream);
 // Clears the rows of n elements whose byte is not zero.
 hipError_t launch_zero_rows(int elem_bytes, void *rows_of, const uint8_t *zero, long long rows, int n, hipStream_t stream);
+// Writes the n (up to 64) numbers to pinned host memory.
+hipError_t launch_read_back(const int64_t *numbers, int n, int64_t *host, hipStream_t stream);
+// dst = 16-bit src (fp32, or 16-bit with a factor per sample of scale_elements elements); n and scale_elements multiples of 8
 hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
                               hipStream_t stream);
 

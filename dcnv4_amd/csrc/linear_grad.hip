@@ -231,6 +231,10 @@ __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaun
   }
 }
 
+__global__ void __launch_bounds__(64) read_back_kernel(const int64_t *numbers, int n, int64_t *host) {
+  if ((int)threadIdx.x < n) host[threadIdx.x] = numbers[threadIdx.x];
+}
+
 // Eight gradients of one (head, level) at a time: the backward of SamplingLocations, rounded where the framework rounds.
 template <typename Tag, typename LocTag>
 __global__ void __launch_bounds__(256) location_grad_kernel(const SamplingLocations l, const void *grad_locations, void *grad_offsets,
@@ -341,6 +345,12 @@ hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &launch, hipSt
   if (dtype == F32::kCode) hipLaunchKernelGGL(cast_weights_kernel<F32>, dim3(end), dim3(256), 0, stream, p);
   else if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3(end), dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(cast_weights_kernel<BF16>, dim3(end), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_read_back(const int64_t *numbers, int n, int64_t *host, hipStream_t stream) {
+  if (n < 0 || n > 64) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, numbers, n, host);
   return hipGetLastError();
 }
 

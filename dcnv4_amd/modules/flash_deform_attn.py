@@ -24,18 +24,6 @@ def _ring_directions(n_heads):
     return xy / xy.abs().amax(dim=-1, keepdim=True)
 
 
-def _pixels(spatial_shapes):
-    """Pixels of all levels together.  Reading them waits for the GPU, so a tensor of shapes is read once: the encoder and
-    decoder layers of a pass share it.  What was read is kept with the tensor's version and read again after a change."""
-    known = getattr(spatial_shapes, "_dcnv4_pixels", None)      # (inference tensors have no version and are never kept)
-    if known is not None and known[0] == spatial_shapes._version:
-        return known[1]
-    n = int(spatial_shapes.prod(-1).sum())
-    if not spatial_shapes.is_inference():
-        spatial_shapes._dcnv4_pixels = (spatial_shapes._version, n)
-    return n
-
-
 class FlashDeformAttn(nn.Module):
     def __init__(self, d_model=256, n_levels=4, n_heads=8, n_points=4):
         super().__init__()
@@ -84,16 +72,18 @@ class FlashDeformAttn(nn.Module):
         """query (N, Lq, C); reference_points (N, Lq, n_levels, 2 or 4) in [0, 1]; input_flatten (N, sum H_l W_l, C);
         input_spatial_shapes (n_levels, 2) int64 rows (H_l, W_l); input_level_start_index (n_levels,) int64;
         input_padding_mask (N, sum H_l W_l) bool, True where the input is padding.  Returns (N, Lq, C)."""
-        n, n_query, _ = query.shape
-        n_in = input_flatten.shape[1]
-        assert _pixels(input_spatial_shapes) == n_in, "the levels do not add up to the flattened input"
-
         if query.is_cuda and not _interpreted():
-            # one call where the kernels take the layer as it is (csrc/binding/attention.cpp)
+            # one call where the kernels take the layer as it is, checks included (csrc/binding/attention.cpp)
             out = ext._native.attention_layer(self, query, reference_points, input_flatten, input_spatial_shapes,
                                               input_level_start_index, input_padding_mask)
             if out is not None:
                 return out
+
+        n, n_query, _ = query.shape
+        n_in = input_flatten.shape[1]
+        # the shapes cannot be read while a graph records them
+        if not (query.is_cuda and torch.cuda.is_current_stream_capturing()):
+            assert input_spatial_shapes.prod(-1).sum() == n_in, "the levels do not add up to the flattened input"
 
         value = self.value_proj(input_flatten)
         if input_padding_mask is not None:

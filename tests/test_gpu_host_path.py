@@ -512,3 +512,31 @@ def test_the_gradient_of_a_pre_norm_layers_projections_meets_in_fp32():
     composed = branch(True)
     handle.remove()
     assert _rel(got, want) < 1.5 * _rel(composed, want)
+
+
+def test_attention_layer_checks_shapes_written_past_the_version_counter():
+    m, (query, reference, features, shapes, starts) = _attention()
+    m(query, reference, features, shapes, starts)
+    shapes.data[0, 0] = 7
+    with pytest.raises(AssertionError, match="levels"):
+        m(query, reference, features, shapes, starts)
+
+
+def test_attention_layer_replays_from_a_graph():
+    """The level check waits for the GPU and is left out of what a graph records; every replay reads the inputs as they are then."""
+    m, (query, reference, features, shapes, starts) = _attention()
+    m.requires_grad_(False)
+    run = lambda: m(query, reference, features, shapes, starts)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run()
+    for _ in range(3):
+        features.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _rel(captured, run()) < 1e-6
