@@ -62,6 +62,8 @@ struct Attention {
   int heads, levels, points, batch;
   int64_t width, pixels, queries;
   bool query32, features32;         // inputs in fp32 (always, without autocast)
+  int kind;                         // coordinates of a reference: 2, a point, or 4, a box
+  at::TensorOptions query_options, features_options;
 
   int bytes() const { return code == DCNV4_DTYPE_F32 ? 4 : 2; }
   int64_t query_rows() const { return batch * queries; }
@@ -72,7 +74,7 @@ struct Attention {
   int location_bytes() const { return code == DCNV4_DTYPE_F16 ? 2 : 4; }
 
   SamplingLocations sampling(const Tensor &reference, const Tensor &shapes) const {
-    return {static_cast<const float *>(reference.const_data_ptr()), shapes.const_data_ptr<int64_t>(), (int)reference.size(-1), levels, points};
+    return {static_cast<const float *>(ptr(reference)), shapes.const_data_ptr<int64_t>(), kind, levels, points};
   }
   LinearLaunch product(const void *a, const void *w, const void *bias, int64_t rows, int64_t k, int64_t n, void *out) const {
     LinearLaunch p = {};
@@ -167,8 +169,8 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
 variable_list Attention::backward(const Tensor &query, const Tensor &reference, const Tensor &features, const Tensor &shapes,
                                   const Tensor &starts, const Tensor &padding, const Tensor &grad, const AttentionSaved &s,
                                   const std::array<bool, kInputs> &want) const {
-  OnDevice guard(query);
-  void *stream = stream_of(query);
+  OnDevice guard(grad);
+  void *stream = stream_of(grad);
   hipStream_t hip = static_cast<hipStream_t>(stream);
   const bool half = code != DCNV4_DTYPE_F32;
   const int64_t n_loc = 2 * logits(), n_log = logits();
@@ -186,7 +188,7 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
   const size_t ws_bytes = flash_deform_attn_gfx950_backward_workspace_bytes(code, batch, (int)pixels, heads, (int)width / heads, levels,
                                                                             (int)queries, points);
   const size_t ws = t.take(ws_bytes);
-  t.allocate(query);
+  t.allocate(grad);
 
   if (through) {
     launch(code, product(grad.const_data_ptr(), a.at(s.output_wt), nullptr, query_rows(), width, width, t.at(d_sampled)), stream);
@@ -215,16 +217,15 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
     launch(code, p, stream);
   };
   if (want[kFeatures]) {
-    g[kFeatures] = at::empty(features.sizes(), features.options());
+    g[kFeatures] = at::empty({batch, pixels, width}, features_options);
     result(product(t.at(d_value), a.at(s.value_wt), nullptr, feature_rows(), width, width, nullptr), g[kFeatures], features32, false);
   }
   if (want[kQuery]) {
-    g[kQuery] = at::empty(query.sizes(), query.options());
+    g[kQuery] = at::empty({batch, queries, width}, query_options);
     result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc, width, nullptr), g[kQuery], query32, false);
     result(product(t.at(d_logits), a.at(s.logits_wt), nullptr, query_rows(), n_log, width, nullptr), g[kQuery], query32, true);
   }
-  const void *q_in = half && query32 ? a.at(s.query) : query.const_data_ptr();
-  const void *f_in = half && features32 ? a.at(s.features) : features.const_data_ptr();
+  const void *q_in = half && query32 ? a.at(s.query) : ptr(query), *f_in = half && features32 ? a.at(s.features) : ptr(features);
   const auto fp32 = params[kValueW].options();
   auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n) -> WeightGradient {
     return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1]};
@@ -244,10 +245,12 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
 struct FlashDeformAttnBackward final : torch::autograd::Node {
   Attention layer;
   AttentionSaved saved;
-  SavedVariable inputs[6];          // query, reference, features, shapes, starts, padding
+  SavedVariable inputs[6];          // query, reference, features, shapes, starts, padding: those that the backward reads
+  SavedVariable weights[4];         // in fp32, where the composition's products would hold them: a change in place is reported
   std::string name() const override { return "FlashDeformAttnBackward"; }
   void release_variables() override {
     for (SavedVariable &v : inputs) v.reset_data();
+    for (SavedVariable &v : weights) v.reset_data();
     saved.arena.release();
     released_ = true;
   }
@@ -260,6 +263,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
       at::AutoGradMode no_grad(false);
       Tensor v[6];
       for (int i = 0; i < 6; ++i) v[i] = inputs[i].unpack();
+      for (SavedVariable &w : weights) w.unpack();
       std::array<bool, kInputs> want;
       for (size_t i = 0; i < kInputs; ++i) want[i] = task_should_compute_output(i);
       out = layer.backward(v[0], v[1], v[2], v[3], v[4], v[5], incoming(grads[0], true), saved, want);
@@ -317,6 +321,9 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!dense(reference, query, at::kFloat) || reference.requires_grad() || reference.dim() != 4 || reference.size(0) != a.batch ||
       reference.size(1) != a.queries || reference.size(2) != a.levels || (reference.size(3) != 2 && reference.size(3) != 4))
     Py_RETURN_NONE;
+  a.kind = (int)reference.size(3);
+  a.query_options = query.options();
+  a.features_options = features.options();
   if (!dense(shapes, query, at::kLong) || !dense(starts, query, at::kLong) || shapes.numel() != 2 * a.levels || a.levels > 32 || starts.numel() != a.levels)
     Py_RETURN_NONE;
   if (padding.defined() && (padding.device() != query.device() || padding.scalar_type() != at::kBool || !padding.is_contiguous() || !in_memory(padding) ||
@@ -345,8 +352,24 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
       node->set_next_edges(torch::autograd::collect_next_edges(inputs));
       node->layer = a;
       node->saved = std::move(saved);
+      // What torch's products would save, no less (a change in place is reported) and no more (it stays allowed, and memory free).
+      auto learns = [&](Input weight) { return a.params[weight].requires_grad(); };
+      auto learn = [&](Input weight) { return learns(weight) || (a.params[weight + 1].defined() && a.params[weight + 1].requires_grad()); };
+      const bool half = a.code != DCNV4_DTYPE_F32;
+      const bool keep_query = !(half && a.query32) && (learns(kOffsetsW) || learns(kLogitsW));
+      const bool keep_features = !(half && a.features32) && learns(kValueW);
+      const Tensor none;
       int i = 0;
-      for (const Tensor *t : {&query, &reference, &features, &shapes, &starts, &padding}) node->inputs[i++] = SavedVariable(*t, false);
+      for (const Tensor *t : {keep_query ? &query : &none, a.kind == 4 ? &reference : &none, keep_features ? &features : &none, &shapes, &starts, &padding})
+        node->inputs[i++] = SavedVariable(*t, false);
+      if (!half) {
+        const bool by_query = query.requires_grad(), by_features = features.requires_grad();
+        if (by_features) node->weights[0] = SavedVariable(a.params[kValueW], false);
+        if (by_query) node->weights[1] = SavedVariable(a.params[kOffsetsW], false);
+        if (by_query) node->weights[2] = SavedVariable(a.params[kLogitsW], false);
+        if (by_query || by_features || learn(kValueW) || learn(kOffsetsW) || learn(kLogitsW))
+          node->weights[3] = SavedVariable(a.params[kOutputW], false);
+      }
       record(node, out);
     }
   } catch (const LevelCheck::Mismatch &) {

@@ -196,8 +196,8 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s, bool keep) const {
 }
 
 variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const Saved &s, const Wanted &want) const {
-  OnDevice guard(x);
-  void *stream = stream_of(x);
+  OnDevice guard(grad);
+  void *stream = stream_of(grad);
   const int c16 = code();
   const int64_t c = l.channels;
   const auto f32 = l.norm1.weight.options();
@@ -217,7 +217,7 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   const size_t d_last = alias_last ? 0 : t.take(act), d_hidden = t.take(hid), d_projected = t.take(act), d_sampled = t.take(act),
                d_value = t.take(act), d_offsets = t.take(om), d_pre = t.take(act), d_dw = l.dw_kernel ? t.take(act) : 0,
                d_half = l.post_norm ? 0 : t.take(2 * act), d_mid = t.take(stream32 ? 2 * act : act);
-  t.allocate(x);
+  t.allocate(grad);
 
   // MLP half
   const void *last = alias_last ? grad.const_data_ptr() : t.at(d_last);
@@ -255,7 +255,7 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   if (through) {
     launch(c16, product(projected, a.at(s.w_output_t), nullptr, c, c, t.at(d_sampled)), stream);
     const size_t ws_bytes = dcnv4_gfx950_backward_workspace_bytes(c16, batch, h, w, l.group, l.group_channels);
-    const Tensor ws = workspace(ws_bytes, x);
+    const Tensor ws = workspace(ws_bytes, grad);
     check(dcnv4_gfx950_backward(a.at(s.value), a.at(s.offsets), t.at(d_sampled), t.at(d_value), t.at(d_offsets), ptr(ws), ws_bytes, c16,
                                 batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad, l.pad, l.dilation, l.dilation,
                                 l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
@@ -265,7 +265,7 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   if (into_pre && l.dw_kernel) {
     const int pad = (l.dw_kernel - 1) / 2;
     const size_t dw_bytes = dcnv4_gfx950_depthwise_conv_backward_workspace_bytes(c16, batch, h, w, (int)c, l.dw_kernel, pad);
-    const Tensor dw_ws = workspace(dw_bytes, x);
+    const Tensor dw_ws = workspace(dw_bytes, grad);
     // the kernel gives the bias's gradient beside the weight's
     Tensor grad_w;
     if (wants(kDwW)) grad_w = at::empty(l.dw_w.sizes(), f32);
@@ -277,7 +277,7 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
     side = t.at(d_dw);
   }
   if (into_x) {
-    g[kX] = at::empty(x.sizes(), x.options());
+    g[kX] = at::empty(s.mid.sizes(), s.mid.options());
     LinearLaunch p = product(t.at(d_value), a.at(s.w_value_t), nullptr, c, c, nullptr);
     p.p[0].residual = side;
     if (l.post_norm) {
@@ -317,7 +317,8 @@ struct InternImageLayerBackward final : torch::autograd::Node {
   }
   std::string name() const override { return "InternImageLayerBackward"; }
   void keep(const Tensor &input) {
-    x = SavedVariable(input, false);
+    // a post-norm layer's backward does not read the input (its products saved 16-bit copies): it may change
+    if (!layer.l.post_norm) x = SavedVariable(input, false);
     int i = 0;
     for (Tensor *p : kept()) {
       params[i++] = SavedVariable(*p, false);

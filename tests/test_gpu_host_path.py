@@ -540,3 +540,24 @@ def test_attention_layer_replays_from_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert _rel(captured, run()) < 1e-6
+
+
+def test_in_place_changes_after_a_layer_are_as_before():
+    """What the composition does not save may change before the backward; what it saves may not."""
+    layer = _layer(dtype=torch.float32, post_norm=True)
+    x = torch.randn(1, 42, 64, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.float16):
+        stream = x * 1.0
+        out = layer(stream, (6, 7))
+        stream += 1.0
+    want = torch.autograd.grad(out.sum(), x)
+    m, (query, reference, features, shapes, starts) = _attention()
+    q = query.clone().requires_grad_()
+    out = m(q, reference, features, shapes, starts)
+    reference.add_(1.0)
+    torch.autograd.grad(out.sum(), q)
+    out = m(q, reference, features, shapes, starts)
+    with torch.no_grad():
+        m.sampling_offsets.weight.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out.sum(), q)
