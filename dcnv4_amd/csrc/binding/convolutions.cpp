@@ -24,6 +24,7 @@ struct Convolution {
   Tensor weight, bias, norm_weight, norm_bias, norm_mean, norm_var;
   int64_t n = 0;
   float eps = 0.f;
+  bool channels_last = false;      // the weights lie in the order that the kernels want, as a channels-last model keeps them
 
   bool load(const Module &m, const Tensor &x, int64_t cin, int kernel, int stride, int pad) {
     if (!m || !is_pair(m, "kernel_size", kernel) || !is_pair(m, "stride", stride) || !is_pair(m, "padding", pad) || !is_pair(m, "dilation", 1) ||
@@ -35,6 +36,8 @@ struct Convolution {
     bias = m.parameter("bias");
     if (!weight.defined() || weight.dim() != 4 || weight.size(1) != cin) return false;
     n = weight.size(0);
+    channels_last = !weight.is_contiguous() && weight.is_contiguous(at::MemoryFormat::ChannelsLast);
+    if (channels_last) weight = weight.permute({0, 2, 3, 1});
     return usable(weight, x, x.scalar_type(), n * cin * kernel * kernel, false) && usable(bias, x, x.scalar_type(), n, true);
   }
   bool load_norm(const Module &m, const Tensor &x) {
@@ -51,6 +54,7 @@ struct Convolution {
   ConvLaunch launch(int batch, int h, int w, int64_t cin, int kernel, int stride, int pad, bool gelu) const {
     ConvLaunch p = {};
     p.weight = weight.const_data_ptr();
+    p.channels_last = channels_last;
     p.bias = ptr(bias);
     p.norm_weight = ptr(norm_weight); p.norm_bias = ptr(norm_bias); p.norm_mean = ptr(norm_mean); p.norm_var = ptr(norm_var);
     p.norm_eps = eps;
@@ -77,7 +81,7 @@ void run(int code, ConvLaunch p, const void *in, void *turned, void *out, void *
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.in = in;
   p.out = out;
-  if (p.kernel != 1) {
+  if (p.kernel != 1 && !p.channels_last) {
     hip_check(launch_turn_conv_weight(p.weight, turned, p.n, p.cin, p.kernel * p.kernel, st), "convolution weight launch");
     p.weight = turned;
   }
@@ -109,7 +113,7 @@ PyObject *py_stem(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const int code = dtype_code(x, "input");
     void *stream = stream_of(x);
     Arena arena;
-    const size_t between = arena.take((size_t)first.batch * first.ho * first.wo * c1.n * 2), turned = arena.take(c2.weight.numel() * 2);
+    const size_t between = arena.take((size_t)first.batch * first.ho * first.wo * c1.n * 2), turned = arena.take(c2.channels_last ? 0 : c2.weight.numel() * 2);
     arena.allocate(x);
     out = at::empty({second.batch, second.ho, second.wo, c2.n}, x.options().memory_format(at::MemoryFormat::Contiguous));
     first.out = arena.at(between);
@@ -147,7 +151,7 @@ PyObject *py_downsample(PyObject *, PyObject *const *args, Py_ssize_t n) {
     void *stream = stream_of(x);
     const int64_t rows = (int64_t)p.batch * p.ho * p.wo;
     Arena arena;
-    const size_t between = arena.take((size_t)rows * conv.n * 2), turned = arena.take(conv.weight.numel() * 2);
+    const size_t between = arena.take((size_t)rows * conv.n * 2), turned = arena.take(conv.channels_last ? 0 : conv.weight.numel() * 2);
     arena.allocate(x);
     out = at::empty({p.batch, (int64_t)p.ho * p.wo, conv.n}, x.options());
     run(code, p, x.const_data_ptr(), arena.at(turned), arena.at(between), stream);

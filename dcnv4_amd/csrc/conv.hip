@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(kPictureWaves * 64) picture_conv_kernel(const 
     tap_x[e] = t % 3;
     tap_off[e] = k < depth ? (int)(c * p.stride_c + tap_y[e] * p.stride_h + tap_x[e] * p.stride_w) : 0;
 #pragma unroll
-    for (int i = 0; i < NF; ++i) fn[i].e[e] = k < depth && i * 16 + r16 < p.n ? weight[(i * 16 + r16) * depth + k] : elem_t(0);
+    for (int i = 0; i < NF; ++i) fn[i].e[e] = k < depth && i * 16 + r16 < p.n ? weight[(i * 16 + r16) * depth + (p.channels_last ? t * p.cin + c : k)] : elem_t(0);
   }
   float scale[NF][4], shift[NF][4];
 #pragma unroll

@@ -7,7 +7,8 @@ namespace dcn {
 // out = act(norm(conv(in) + bias)), norm a batch normalisation by its running statistics.
 struct ConvLaunch {
   const void *in;                  // [batch][h][w][cin]; the picture: any strides
-  const void *weight;              // [n][kernel * kernel][cin]; the picture: [n][cin][3][3]
+  const void *weight;              // [n][kernel * kernel][cin]; the picture: [n][cin][3][3], or that too
+  int channels_last;               // the picture's weights: [n][3][3][cin]
   const void *bias;                // [n] or null
   const void *norm_weight, *norm_bias, *norm_mean, *norm_var;      // [n], all or none
   float norm_eps;

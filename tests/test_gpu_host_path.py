@@ -561,3 +561,16 @@ def test_in_place_changes_after_a_layer_are_as_before():
         m.sampling_offsets.weight.add_(1.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(out.sum(), q)
+
+
+def test_channels_last_models_keep_the_one_call_convolutions():
+    from dcnv4_amd import ext
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer
+    torch.manual_seed(5)
+    stem, down = StemLayer(3, 64).cuda().half().eval(), DownsampleLayer(64).cuda().half().eval()
+    x, y = torch.randn(2, 3, 37, 30, device="cuda").half(), torch.randn(2, 35, 64, device="cuda").half()
+    with torch.no_grad():
+        want = stem(x), down(y, (5, 7))[0]
+        stem, down = stem.to(memory_format=torch.channels_last), down.to(memory_format=torch.channels_last)
+        got = ext._native.stem_inference(stem, x), ext._native.downsample_inference(down, y, 5, 7)
+    assert all(g is not None and torch.equal(g, w) for g, w in zip(got, want))
