@@ -1,6 +1,7 @@
 """The window gathers of the DCNv4 operator at the edges of their tiles, against the oracle: every lanes-per-group and
-groups-per-workgroup variant, images smaller than a tile, one pixel into the next tile and of a row, groups left over in the last
-workgroup, points beyond the window and outside the image."""
+units-per-workgroup variant (which of them a shape takes follows from the bytes of a group, one lane for 32, and from the pixels:
+two units a workgroup up to 64, four up to 32), images smaller than a tile, one pixel into the next tile and of a row, groups left
+over in the last workgroup, points beyond the window and outside the image, offsets that are no numbers."""
 import pytest
 import torch
 
@@ -32,3 +33,37 @@ def test_window_gathers_match_oracle(oracle, shape, dtype):
     cabi.assert_close(gv, wgv, *GRAD_TOL[dtype], what="grad_value")
     cabi.assert_close(gom, wgom, *GRAD_TOL[dtype], what="grad_offset_mask")
     assert (gom[..., G * 27:] == 0).all(), "padded tail of grad_offset_mask must be exactly zero"
+
+
+# lanes and units that the shapes above leave out in 16 bits: (1, 2), two groups of 32 bytes on 33 to 64 pixels (the last stage of a
+# model at 224 pixels), and (2, 4), two groups of 64 bytes on up to 32; an odd number of groups each, and one group alone
+SMALL = [(3, 7, 7, 5, 16, 5, 3.0), (2, 1, 33, 1, 16, 0, 2.0), (2, 8, 8, 2, 16, 12, 20.0), (2, 5, 6, 3, 32, 2, 4.0), (1, 32, 1, 1, 32, 5, 3.0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("shape", SMALL, ids=lambda s: "x".join(str(v) for v in s[:5]))
+def test_window_gathers_of_small_images_match_oracle(oracle, shape, dtype):
+    test_window_gathers_match_oracle(oracle, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("width", [16, 32, 64])
+def test_window_gathers_drop_offsets_that_are_no_numbers(width, dtype):
+    """Such a point is outside the image: it adds nothing, and its gradients are zero, as for one far outside."""
+    from dcnv4_amd import ext
+    b, h, w, groups = 2, 9, 13, 3
+    case = (b, h, w, groups, width, (3, 3, 1, 1, 1, 1, 1, 1), 0, 1.0, 2.0)
+    v, om, go, (geom, G, D, scale, rc) = _dcn_inputs(case, dtype, seed=width)
+    results = []
+    for values in ((float("nan"), float("inf"), float("-inf")), (1000.0, 1000.0, -1000.0)):
+        rows = om.clone()
+        for i, value in enumerate(values):
+            rows[..., 2 * i] = value
+            rows[:, 3, :, 27 + 2 * i + 7] = value
+        with ext.launch_options(reach=4, dual="off"):
+            out = cabi.dcnv4_forward(v.cuda(), rows.cuda(), geom, G, D, scale, rc)
+            gv, gom = cabi.dcnv4_backward(v.cuda(), rows.cuda(), go.cuda(), geom, G, D, scale, rc)
+        results.append((out, gv, gom))
+    for got, want in zip(*results):
+        assert torch.isfinite(got).all()
+        cabi.assert_close(got, cabi.f64(want), *GRAD_TOL[dtype], what="against points far outside")
