@@ -1,7 +1,7 @@
 // Shared helpers of the Python extension dcnv4_amd._native: the host path of the operators in C++.
 //
 // What bounds a small call is the host: argument checks, the autograd wrapper and the C-ABI call in Python took 16 us
-// for a forward and 65 to 130 us for forward and backward (one image of 7x7 to some 30 MB of tensors, MI355X box), while
+// for a forward and 65 to 130 us for forward and backward (one image of 7x7 to some 30 MB of tensors), while
 // its kernels run 5 to 30 us.  Here a call parses its arguments with the vectorcall protocol, allocates through ATen and
 // records a C++ autograd node, so the backward runs on the engine's thread without the interpreter.
 #pragma once

@@ -294,7 +294,7 @@ int plan_grad_value_tiles(DcnLaunch *L, int dtype, int batch) {
   return fail(DCNV4_ERR_RUNTIME, "kernel with %d taps and %d group channels does not fit the tiled backward", L->Kp, D);
 }
 
-constexpr uint64_t kDirectForwardBytes = 2800u << 10;      // outputs up to this size go by the direct kernel
+constexpr uint64_t kSmallForwardBytes = 2800u << 10;      // outputs up to this size go by the kernels for small calls
 
 bool tiled_gather_enabled() { return g_opt.gather != kOptPlain; }
 
@@ -811,7 +811,7 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
   // 1x56x56x64 4.3 against 5.7, 4x56x56x64 (1.6 MB) 6.1 against 7.3, 2x64x64x128 (2.1 MB) 5.4 against 8.1, 6x56x56x64 (2.4 MB)
   // 8.3 against 8.0, 4x64x64x128 (4.2 MB) 9.3 against 8.9.
   const bool small = g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 &&
-                     (uint64_t)batch * pr.img_out_elems * pr.s <= kDirectForwardBytes;
+                     (uint64_t)batch * pr.img_out_elems * pr.s <= kSmallForwardBytes;
   const bool at_once = small && kernel_h == 3 && kernel_w == 3 && !remove_center && !softmax && pr.launch.lanes.cpt * pr.s == 16;
   const int window = small ? 0 : plan_window_gather(&pr.launch, pr.s, batch, false);
   const bool tiled = !small && window == 0 && plan_gather_tiles(&pr.launch, pr.s, false);

@@ -174,9 +174,10 @@ __device__ __forceinline__ void quad_softmax_stats(const float *m, int n, int my
 }
 
 // The softmax and sampling points of a (query, head) with four levels of four points, a lane's share of them - point my_k of every
-// level - from memory straight into its registers: no staging of rows, and every exponential once.  The staged forward, which is
-// bound by its vector instructions (277 -> 225 for 64 points), took 146 -> 140 us with it for 4 images of 128x128.., 8 heads of
-// 32, fp16, inputs not in a cache.
+// level - from memory straight into its registers: no staging of rows, and every exponential once.  The staged forward keeps its
+// CU's limit of requests to the L2 outstanding and its vector units half busy, so a fifth fewer vector instructions (277 -> 225 for
+// 64 points) took 4 %: 146 -> 140 us for 4 images of 128x128.., 8 heads of 32, fp16, inputs not in a cache.  Written for the
+// module's default of four levels and four points, whose loops are unrolled over registers; others stage their rows in LDS.
 constexpr int kFour = 4;
 template <typename Tag>
 struct QuadRow {

@@ -6,9 +6,10 @@
 // The matrix instruction leaves a lane four rows of its result; with w1's features dealt to the rows of two instructions so that
 // these are eight consecutive features, they are the lane's eight values of the depth of the second product: the activations
 // never leave the lane.  Both weights' next 32 features come straight into LDS meanwhile, shared by the four waves.
-// What bounds it then is the GELU (thirteen instructions an element; the vector units are busy 75 % of the time, the matrix cores
-// 31) and, with 224 channels, the two waves that its registers leave room for.
-// Measured, fp16, two kernels -> this one: 401408 x 112 336 -> 145 us, 100352 x 224 203 -> 134.
+// What bounds it then is the GELU (seventeen instructions an element; with 112 channels the vector units are busy 59 % of the time,
+// the matrix cores 22) and, with 224 channels, the two waves that its registers leave room for (34 and 21 %).
+// Measured, fp16, two kernels -> this one: 401408 x 112 336 -> 160 us, 100352 x 224 203 -> 140 (145 and 134 with a GELU of thirteen
+// instructions, which was less exact than the fp32 function).
 #include <algorithm>
 
 #include "launch.hpp"
