@@ -62,6 +62,12 @@ class DropPath(nn.Module):
         return x * mask / keep
 
 
+def _one_call(x):
+    """Whether a module may hand `x` to the extension and be done: a GPU tensor without gradients, in a program that runs rather
+    than one that is traced symbolically or compiled, which has to see the module's own operators."""
+    return isinstance(x, torch.Tensor) and x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+
+
 class StemLayer(nn.Module):
     def __init__(self, in_chans=3, out_chans=96, norm_layer="BN"):
         super().__init__()
@@ -72,8 +78,8 @@ class StemLayer(nn.Module):
         self.norm2 = _norm(out_chans, norm_layer, "channels_first", "channels_last")
 
     def forward(self, x):
-        if x.is_cuda and not torch.is_grad_enabled():
-            y = ext._native.stem_inference(self, x)      # csrc/binding/convolutions.cpp
+        if not torch.jit.is_scripting():
+            y = ext._native.stem_inference(self, x) if _one_call(x) else None      # csrc/binding/convolutions.cpp
             if y is not None:
                 return y
         # channels-last memory from the first convolution on: the NHWC view the blocks work on is then dense, so
@@ -91,10 +97,9 @@ class DownsampleLayer(nn.Module):
     def forward(self, x, shape):
         H, W = shape
         N, _, C = x.shape
-        if x.is_cuda and not torch.is_grad_enabled():
-            y = ext._native.downsample_inference(self, x, H, W)
-            if y is not None:
-                return y, ((H + 1) // 2, (W + 1) // 2)
+        y = ext._native.downsample_inference(self, x, H, W) if _one_call(x) else None
+        if y is not None:
+            return y, ((H + 1) // 2, (W + 1) // 2)
         x = self.norm(self.conv(x.view(N, H, W, C).permute(0, 3, 1, 2)))
         H, W = x.size(2), x.size(3)
         return x.flatten(2).permute(0, 2, 1), (H, W)
@@ -252,7 +257,7 @@ class FlashInternImage(nn.Module):
         for level in self.levels:
             x, shape = level(x, shape)
         h, w = shape
-        y = ext._native.head_inference(self.conv_head, x, h, w) if x.is_cuda and not torch.is_grad_enabled() else None
+        y = ext._native.head_inference(self.conv_head, x, h, w) if _one_call(x) else None
         x = self.conv_head(x.view(N, h, w, -1).permute(0, 3, 1, 2)) if y is None else y.permute(0, 3, 1, 2)
         return torch.flatten(self.avgpool(x), 1)
 

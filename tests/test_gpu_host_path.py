@@ -574,3 +574,13 @@ def test_channels_last_models_keep_the_one_call_convolutions():
         stem, down = stem.to(memory_format=torch.channels_last), down.to(memory_format=torch.channels_last)
         got = ext._native.stem_inference(stem, x), ext._native.downsample_inference(down, y, 5, 7)
     assert all(g is not None and torch.equal(g, w) for g, w in zip(got, want))
+
+
+def test_a_compiled_stem_is_one_graph_of_its_modules():
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer
+    torch.manual_seed(3)
+    stem, down = StemLayer(3, 64).cuda().half().eval(), DownsampleLayer(64).cuda().half().eval()
+    x, y = torch.randn(1, 3, 32, 32, device="cuda").half(), torch.randn(1, 64, 64, device="cuda").half()
+    with torch.no_grad():
+        assert _rel(torch.compile(stem, backend="eager", fullgraph=True)(x), stem(x)) < 2e-3
+        assert _rel(torch.compile(down, backend="eager", fullgraph=True)(y, (8, 8))[0], down(y, (8, 8))[0]) < 2e-3

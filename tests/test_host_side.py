@@ -357,3 +357,16 @@ def test_committed_table_records_the_library_it_was_tuned_on():
     assert isinstance(table.get("library_commit"), str) and len(table["library_commit"]) >= 7
     sha = table.get("library_sources_sha256")
     assert isinstance(sha, str) and len(sha) == 64 and len(tune.library_sources_sha256()) == 64
+
+
+@pytest.mark.parametrize("grad", [True, False], ids=["grad", "no-grad"])
+def test_the_convolutions_around_the_layers_can_be_scripted_traced_and_compiled(grad):
+    """Their one-call paths on a GPU stay out of a program that is made of the modules' operators."""
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer
+    stem, down = StemLayer(3, 16).eval(), DownsampleLayer(16).eval()
+    x, y = torch.randn(1, 3, 16, 16), torch.randn(1, 16, 16)
+    with torch.set_grad_enabled(grad):
+        want, (want_down, _) = stem(x), down(y, (4, 4))
+        for program in (torch.jit.script(stem), torch.fx.symbolic_trace(stem), torch.compile(stem, backend="eager", fullgraph=True)):
+            torch.testing.assert_close(program(x), want)
+        torch.testing.assert_close(torch.fx.symbolic_trace(down)(y, (4, 4))[0], want_down)
