@@ -143,7 +143,7 @@ class InternImageLayer(nn.Module):
         return residual + self.drop_path(layer_norm_residual(y, ln, gamma))
 
     def forward(self, x, shape):
-        if x.is_cuda and not GFX950_TABLE:
+        if x.is_cuda and shape is not None and not GFX950_TABLE:
             # one call where the kernels take the layer as it is: under autocast csrc/binding/training.cpp, else without
             # gradients csrc/binding/layers.cpp
             call = ext._native.layer_training if torch.is_autocast_enabled("cuda") else ext._native.layer_inference

@@ -584,3 +584,9 @@ def test_a_compiled_stem_is_one_graph_of_its_modules():
     with torch.no_grad():
         assert _rel(torch.compile(stem, backend="eager", fullgraph=True)(x), stem(x)) < 2e-3
         assert _rel(torch.compile(down, backend="eager", fullgraph=True)(y, (8, 8))[0], down(y, (8, 8))[0]) < 2e-3
+
+
+def test_a_layer_without_a_shape_takes_its_tokens_for_a_square():
+    layer, x = _layer().eval(), torch.randn(1, 49, 64, device="cuda").half()
+    with torch.no_grad():
+        assert _rel(layer(x, None), layer(x, (7, 7))) < 3e-3
