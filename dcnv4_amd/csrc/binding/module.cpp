@@ -101,7 +101,7 @@ bool observed() {
 
 bool in_memory(const Tensor &t) { return t.has_storage() && (t.numel() == 0 || t.const_data_ptr() != nullptr); }
 
-bool plain(const Tensor &t) { return in_memory(t) && !torch::autograd::isFwGradDefined(t); }
+bool plain(const Tensor &t) { return in_memory(t) && !t._fw_grad(/*level=*/0).defined(); }
 
 Tensor incoming(const Tensor &grad, bool aligned) {
   Tensor g = grad._is_zerotensor() ? at::zeros(grad.sizes(), grad.options()) : grad.contiguous();
