@@ -4,6 +4,8 @@
 // A picture or a few are bound by the host: 415 launches through Python took 6.5 ms for a T variant whose kernels run
 // 2.2 ms.  Here a layer is seven (pre-norm) or eight launches: the two projections in front of the operator share one,
 // bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.
+#include <cmath>
+
 #include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 
@@ -72,9 +74,10 @@ bool Layer::load(const Module &m, const Tensor &x, at::ScalarType params) {
   dilation = (int)dcn.integer("dilation", 0);
   group = (int)dcn.integer("group", 0);
   group_channels = (int)dcn.integer("group_channels", 0);
-  remove_center = (int)dcn.integer("remove_center", 0);
-  offset_scale = (float)dcn.real("offset_scale", 1.0);
-  if (kernel <= 0 || dilation <= 0 || 2 * pad != dilation * (kernel - 1) || (int64_t)group * group_channels != c) return false;
+  remove_center = (int)dcn.integer("remove_center", -1);
+  const double scale = dcn.real("offset_scale", std::nan(""));
+  offset_scale = (float)scale;
+  if (remove_center < 0 || std::isnan(scale) || kernel <= 0 || dilation <= 0 || 2 * pad != dilation * (kernel - 1) || (int64_t)group * group_channels != c) return false;
   const Module offset = dcn.child("offset_mask", kLinear);
   row = offset.integer("out_features", 0);
   if (row <= 0 || row % 8 != 0 || !load_linear(offset, x, params, c, row, &offset_w, &offset_b) ||

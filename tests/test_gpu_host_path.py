@@ -590,3 +590,25 @@ def test_a_layer_without_a_shape_takes_its_tokens_for_a_square():
     layer, x = _layer().eval(), torch.randn(1, 49, 64, device="cuda").half()
     with torch.no_grad():
         assert _rel(layer(x, None), layer(x, (7, 7))) < 3e-3
+
+
+@pytest.mark.parametrize("kind", ["inference", "autocast"])
+def test_settings_of_another_type_keep_their_value(kind):
+    """What the operator's call converts to a number - a tensor of one element, a numpy integer - is no number to a reader of
+    attributes."""
+    import numpy as np
+    layer = _layer(dtype=torch.float16 if kind == "inference" else torch.float32).eval()
+    x = torch.randn(2, 42, 64, device="cuda", dtype=layer.norm1[0].weight.dtype)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=kind == "autocast"):
+            return layer(x, (6, 7))
+
+    layer.dcn.offset_scale = 2.0
+    want = run()
+    layer.dcn.offset_scale = torch.tensor(2.0)
+    assert _rel(run(), want) < 3e-3
+    layer.dcn.offset_scale, layer.dcn.remove_center = 2.0, 1
+    want = run()
+    layer.dcn.remove_center = np.int64(1)
+    assert _rel(run(), want) < 3e-3
