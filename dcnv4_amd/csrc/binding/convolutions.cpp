@@ -97,7 +97,7 @@ PyObject *py_stem(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!stem.computes(kStemLayer) || a.overridden({0}) || !inference(x) || x.dim() != 4 || x.size(0) * x.size(2) * x.size(3) >= (1ll << 31)) Py_RETURN_NONE;
   const Module norm1 = stem.child("norm1", kSequential), norm2 = stem.child("norm2", kSequential), act = stem.child("act", kGelu);
   Convolution c1, c2;
-  if (!norm1 || norm1.child("1") || !norm2.child("1", kToChannelsLast) || norm2.child("2") || !act || !exact_gelu(act) ||
+  if (norm1.children() != 1 || !norm2.child("1", kToChannelsLast) || norm2.children() != 2 || !act || !exact_gelu(act) ||
       !c1.load(stem.child("conv1", kConv2d), x, x.size(1), 3, 2, 1) || !c1.load_norm(norm1.child("0", kBatchNorm2d), x) ||
       !c2.load(stem.child("conv2", kConv2d), x, c1.n, 3, 2, 1) || !c2.load_norm(norm2.child("0", kBatchNorm2d), x))
     Py_RETURN_NONE;
@@ -134,7 +134,7 @@ PyObject *py_downsample(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!m.computes(kDownsampleLayer) || a.overridden({0}) || !inference(x) || !usable_input(x, h, w)) Py_RETURN_NONE;
   const Module norm = m.child("norm", kSequential);
   Convolution conv;
-  if (!norm || !norm.child("0", kToChannelsLast) || !norm.child("2", kToChannelsFirst) || norm.child("3") ||
+  if (!norm || !norm.child("0", kToChannelsLast) || !norm.child("2", kToChannelsFirst) || norm.children() != 3 ||
       !conv.load(m.child("conv", kConv2d), x, x.size(2), 3, 2, 1))
     Py_RETURN_NONE;
   const Module ln = norm.child("1", kLayerNorm);
@@ -172,7 +172,7 @@ PyObject *py_head(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (a.overridden({0}) || !inference(x) || !usable_input(x, h, w) || !head.is(kSequential) || head.hooked()) Py_RETURN_NONE;
   const Module norm = head.child("1", kSequential), act = head.child("2", kGelu);
   Convolution conv;
-  if (!norm || norm.child("1") || !act || !exact_gelu(act) || head.child("3") || !conv.load(head.child("0", kConv2d), x, x.size(2), 1, 1, 0) ||
+  if (norm.children() != 1 || !act || !exact_gelu(act) || head.children() != 3 || !conv.load(head.child("0", kConv2d), x, x.size(2), 1, 1, 0) ||
       !conv.load_norm(norm.child("0", kBatchNorm2d), x))
     Py_RETURN_NONE;
   const ConvLaunch p = conv.launch((int)x.size(0), h, w, x.size(2), 1, 1, 0, true);

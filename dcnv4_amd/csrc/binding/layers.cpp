@@ -23,7 +23,7 @@ namespace {
 
 bool load_norm(const Module &sequential, const Tensor &x, at::ScalarType dtype, int64_t channels, NormParams *out) {
   const Module norm = sequential.child("0", kLayerNorm);
-  if (!norm || sequential.child("1")) return false;
+  if (!norm || sequential.children() != 1) return false;
   out->weight = norm.parameter("weight");
   out->bias = norm.parameter("bias");
   out->eps = (float)norm.real("eps", -1.0);

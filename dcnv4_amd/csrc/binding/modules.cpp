@@ -76,6 +76,11 @@ Module Module::child(const char *name) const {
   return Module(c == Py_None ? nullptr : c);
 }
 
+Py_ssize_t Module::children() const {
+  PyObject *all = o_ != nullptr ? item(dict_of(o_), "_modules") : nullptr;
+  return all != nullptr && PyDict_Check(all) ? PyDict_GET_SIZE(all) : 0;
+}
+
 Module Module::child(const char *name, ModuleKind kind) const {
   const Module c = child(name);
   return c.is(kind) && !c.hooked() ? c : Module();

@@ -16,6 +16,7 @@ class Module {
   explicit operator bool() const { return o_ != nullptr; }
   Module child(const char *name, ModuleKind kind) const;      // null unless there is one of exactly that class
   Module child(const char *name) const;
+  Py_ssize_t children() const;
   Tensor parameter(const char *name) const;                   // undefined: registered as None
   Tensor buffer(const char *name) const;
   PyObject *attribute(const char *name) const;                // borrowed; null: absent

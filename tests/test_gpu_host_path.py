@@ -612,3 +612,26 @@ def test_settings_of_another_type_keep_their_value(kind):
     want = run()
     layer.dcn.remove_center = np.int64(1)
     assert _rel(run(), want) < 3e-3
+
+
+def test_modules_added_to_a_sequential_run():
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer, StemLayer, _norm
+    torch.manual_seed(4)
+    stem, down, layer = StemLayer(3, 64).cuda().half().eval(), DownsampleLayer(64).cuda().half().eval(), _layer(post_norm=True).eval()
+    calls = []
+
+    class Count(torch.nn.Module):
+        def forward(self, x):
+            calls.append(1)
+            return x
+
+    head = torch.nn.Sequential(torch.nn.Conv2d(64, 96, 1), _norm(96, "BN", "channels_first", "channels_first"), torch.nn.GELU()).cuda().half().eval()
+    for sequential in (stem.norm1, stem.norm2, down.norm, layer.norm2, head, head[1]):
+        sequential.add_module("extra", Count())
+    from dcnv4_amd import ext
+    with torch.no_grad():
+        y = stem(torch.randn(1, 3, 32, 32, device="cuda").half()).reshape(1, 64, 64)
+        down(y, (8, 8))
+        layer(y, (8, 8))
+        assert ext._native.head_inference(head, y, 8, 8) is None
+    assert len(calls) == 4
