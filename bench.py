@@ -286,7 +286,7 @@ def main():
                 return
         sys.exit(f"--only-op {args.only_op}: no such DCNv4 shape")
 
-    # ------------------------------------------------------------------ the step (configs[1])
+    # ------------------------------------------------------------------ the step
     work = []
     for dtype, s in ((torch.float16, 2), (torch.float32, 4)):
         for name, B, H, W, C, G in CFG2:
@@ -399,7 +399,7 @@ def main():
                 time_op(lambda: ext.flash_deform_attn_backward(v, shapes, starts, sla, go, 64, K, 0, 0), args.op_iters), bb)
             del v, sla, go
 
-    # ------------------------------------------------------------------ FlashInternImage-B end to end (configs[4])
+    # ------------------------------------------------------------------ FlashInternImage-B end to end
     model_line = None
     if not args.no_model:
         from dcnv4_amd.models import flash_intern_image
@@ -461,7 +461,7 @@ def main():
     # ------------------------------------------------------------------ CPU baseline (rank 0, bounded sample)
     # The pure-PyTorch grid_sample formulation on the host cores: 2 warm-ups, median of 5, forward and
     # forward+backward separately.  `value` is the forward+backward rate over the step's own four shapes on a batch
-    # sample; `detail` adds configs[0] (its full size, batch 2) and one image of the attention configuration.
+    # sample; `detail` adds the first stage alone (batch 2) and one image of the attention configuration.
     cpu = None
     if not args.no_cpu_baseline:
         import statistics
@@ -513,7 +513,7 @@ def main():
         cpu = {"value": round(cpu_bytes / cpu_time / 1e9, 3), "unit": "GB/s", "cores": cores, "kind": "port",
                "sample": f"DCNv4 fwd+bwd, four FlashInternImage-T stage shapes at batch {Bc} (of 64), fp32, torch grid_sample "
                          f"formulation + autograd, median of 5 after 2 warm-ups, {cpu_time * 1e3:.0f} ms per pass; detail: "
-                         "configs[0] at its full batch 2, configs[1] at batch 8, configs[3] one image of 4",
+                         "the first stage alone at batch 2, the four stages at batch 8, one image of 4 of the attention shape",
                "detail": cpu_detail}
 
     line = {
