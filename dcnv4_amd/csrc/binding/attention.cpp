@@ -252,6 +252,7 @@ struct FlashDeformAttnBackward final : torch::autograd::Node {
     for (SavedVariable &v : inputs) v.reset_data();
     for (SavedVariable &v : weights) v.reset_data();
     saved.arena.release();
+    for (Tensor &p : layer.params) p = Tensor();
     released_ = true;
   }
   variable_list apply(variable_list &&grads) override {

@@ -330,6 +330,7 @@ struct InternImageLayerBackward final : torch::autograd::Node {
     for (SavedVariable &p : params) p.reset_data();
     saved.arena.release();
     saved.mid = Tensor();
+    layer.l = Layer();      // its weights
     released_ = true;
   }
   variable_list apply(variable_list &&grads) override {

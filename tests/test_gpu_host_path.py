@@ -635,3 +635,24 @@ def test_modules_added_to_a_sequential_run():
         layer(y, (8, 8))
         assert ext._native.head_inference(head, y, 8, 8) is None
     assert len(calls) == 4
+
+
+@pytest.mark.parametrize("kind", ["layer", "attention"])
+def test_a_node_lets_go_of_its_weights_after_the_backward(kind):
+    """Weights that are no parameters - computed from others for one call - are held by nothing but the graph."""
+    if kind == "layer":
+        m, inputs, amp = _layer(channels=512, dtype=torch.float32), (torch.randn(1, 9, 512, device="cuda"), (3, 3)), True
+    else:
+        (m, inputs), amp = _attention(width=512), False
+    values = {name: p.detach().clone() for name, p in m.named_parameters()}
+    weights = {name: v.clone().requires_grad_() * 1.0 for name, v in values.items()}
+    with torch.autocast("cuda", dtype=torch.float16, enabled=amp):
+        out = torch.func.functional_call(m, weights, inputs)
+    assert out.grad_fn.name() in ("InternImageLayerBackward", "FlashDeformAttnBackward")
+    size = sum(w.numel() for w in weights.values() if w.dim() == 2) * 4
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    out.sum().backward()
+    del weights
+    gc.collect()
+    assert torch.cuda.memory_allocated() <= before - size and out.grad_fn is not None
