@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <utility>
 
 #include "../../include/dcnv4_gfx950.h"
 #include "common.hpp"
@@ -188,6 +189,18 @@ __global__ void init_state_kernel(GradState *st) {
   if (threadIdx.x < sizeof(GradState) / sizeof(uint32_t)) reinterpret_cast<uint32_t *>(st)[threadIdx.x] = 0u;
 }
 static_assert(sizeof(GradState) / sizeof(uint32_t) <= 64, "init_state_kernel runs one wave");
+
+// The same, and the headers of the tiles' lists of far points: a lane each.
+__global__ void __launch_bounds__(256) init_lists_kernel(const DcnLaunch p, int elem_bytes, int lists) {
+  if (blockIdx.x == 0 && threadIdx.x < sizeof(GradState) / sizeof(uint32_t)) reinterpret_cast<uint32_t *>(p.state)[threadIdx.x] = 0u;
+  int id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= lists) return;
+  const int n_chunks = (p.G + p.ng_chunk - 1) / p.ng_chunk, nty = (p.H + p.tile_h - 1) / p.tile_h, ntx = (p.W + p.tile_w - 1) / p.tile_w;
+  const int chunk = id % n_chunks; id /= n_chunks;
+  const int tx = id % ntx; id /= ntx;
+  const FarList list(p, elem_bytes, id % nty, tx, chunk);
+  *static_cast<FarHeader *>(list.slot(p, elem_bytes, id / nty, 0)) = FarHeader{0u, 0u};
+}
 
 constexpr size_t kStateBytes = 256;     // GradState, padded
 constexpr int kMaxBackwardGroupChannels = 512;    // widest group of the backward: 64 lanes of 16 bytes in the gather, 16 lanes of 32 channels per slot
@@ -717,6 +730,31 @@ int static_scratch_of_current_device(void **out) {
   return DCNV4_OK;
 }
 
+// Whether the tiles' parts of grad_value hold lists of far points until they are overwritten.  None of the tensors that are still
+// read may lie there.  And the visits must shrink: a list's points cost a count in memory each, and the first kernel some 6 % where
+// offsets have tails, for a tile's visits over tails of about twice the near reach.  Learnt offsets (a bell of 2 pixels), grad_value /
+// grad_offset_mask, us, without and with: 2x200x334 with 10 groups of 16 in bf16 (1.9 times the visits) 244 / 109 -> 170 / 122, 64x56x56 with 4 groups
+// of 64 (2.0) 536 -> 515 together; 64x28x28 with 4 of 64 (1.7) 83 / 52 -> 80 / 58, 64x56x56 with 4 of 16 (1.4, the image's edges cut
+// the visits) 105 / 71 -> 99 / 78.  A near reach of 5 pixels serves offsets within +-4; 6, 7 and 8 took 191, 184 and 203 us for the 170
+// above, by what fits a strip.
+constexpr int kNearReach = 5;
+bool far_lists_fit(const DcnLaunch &L, const DcnProblem &pr, const void *grad_value, std::initializer_list<std::pair<const void *, size_t>> others) {
+  if (L.H / L.tile_h >= 0xffff || L.W / L.tile_w >= 0xffff) return false;      // tiles are named by 16 bits each way
+  auto visited = [](int extent, int tile, int reach) {      // rows (columns) over all tiles
+    double sum = 0.;
+    for (int at = 0; at < extent; at += tile) sum += std::min(extent, at + tile + reach) - std::max(0, at - reach);
+    return sum;
+  };
+  const int tails = 2 * kNearReach + 1;
+  if (visited(L.H, L.tile_h, tails) * visited(L.W, L.tile_w, tails) < 1.75 * visited(L.H, L.tile_h, kNearReach) * visited(L.W, L.tile_w, kNearReach)) return false;
+  const uintptr_t lo = reinterpret_cast<uintptr_t>(grad_value), hi = lo + (size_t)pr.batch * pr.img_elems * pr.s;
+  for (const auto &[ptr, image] : others) {
+    const uintptr_t from = reinterpret_cast<uintptr_t>(ptr);
+    if (from < hi && from + (size_t)pr.batch * image * pr.s > lo) return false;
+  }
+  return true;
+}
+
 const char *at(const void *base, size_t elems, int s) { return static_cast<const char *>(base) + elems * s; }
 char *at(void *base, size_t elems, int s) { return static_cast<char *>(base) + elems * s; }
 
@@ -888,7 +926,21 @@ static int dcn_backward_impl(const void *value, const void *offset_mask, const v
     if (gather_tiled) cap = std::max(cap, std::max((base.gt_h - 1) * base.sh, (base.gt_w - 1) * base.sw) + base.gt_reach + 1);
     base.gv_reach_cap = (float)cap;
   }
-  if (!base.gv_whole) {
+  // With lists of far points (the window kernel writes them) a few pixels suffice for every tile.
+  base.gv_lists = 0;
+  base.gv_near = base.gv_reach_cap;
+  if (window && !base.gv_whole && far_lists_fit(base, pr, grad_value, {{value, pr.img_elems}, {offset_mask, pr.img_om_elems},
+      {grad_output, pr.img_out_elems}, {grad_offset_mask, pr.img_om_elems}})) {
+    base.gv_lists = 1;
+    base.gv_near = (float)kNearReach;
+  }
+  if (base.gv_lists) {
+    DcnLaunch L = base;
+    L.grad_value = grad_value;
+    const int lists = batch * ((base.H + base.tile_h - 1) / base.tile_h) * ((base.W + base.tile_w - 1) / base.tile_w) * ((base.G + base.ng_chunk - 1) / base.ng_chunk);
+    hipLaunchKernelGGL(init_lists_kernel, dim3((unsigned)((lists + 255) / 256)), dim3(256), 0, st, L, pr.s, lists);
+    if (hipError_t e = hipGetLastError()) return hip_fail("state init launch", e);
+  } else if (!base.gv_whole) {
     hipLaunchKernelGGL(init_state_kernel, dim3(1), dim3(64), 0, st, base.state);
     if (hipError_t e = hipGetLastError()) return hip_fail("state init launch", e);
   }

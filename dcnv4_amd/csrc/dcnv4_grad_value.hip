@@ -5,9 +5,9 @@
 namespace dcn {
 namespace {
 
-template <typename Tag, int KP, int CW, int ROUNDS, int NT>
-__global__ void __launch_bounds__(NT) dcnv4_grad_value_kernel(const DcnLaunch p) {
-  dcnv4_grad_value_body<Tag, KP, CW, ROUNDS, NT>(p, blockIdx.x, gridDim.x);
+template <typename Tag, int KP, int CW, int ROUNDS, int NT, bool LISTS = false>
+__global__ void __launch_bounds__(NT, LISTS ? 4 : 1) dcnv4_grad_value_kernel(const DcnLaunch p) {
+  dcnv4_grad_value_body<Tag, KP, CW, ROUNDS, NT, LISTS>(p, blockIdx.x, gridDim.x);
 }
 
 constexpr int gv_rounds(int kp) { return kp > 0 ? kGradValueColumnRounds : kGradValueRounds; }
@@ -33,6 +33,8 @@ hipError_t launch_t(const DcnLaunch &p, hipStream_t stream) {
     if (p.gv_cw == 8) return go(dcnv4_grad_value_kernel<Tag, KPV, 8, gv_rounds(KPV), 1024>);       \
     return go(dcnv4_grad_value_kernel<Tag, KPV, 16, gv_rounds(KPV), 1024>);       \
   } while (0)
+  if (p.gv_lists)      // of the window kernel: 3x3 with its centre, groups of 16 channels or more
+    return p.gv_threads == 512 ? go(dcnv4_grad_value_kernel<Tag, 9, 16, gv_rounds(9), 512, true>) : go(dcnv4_grad_value_kernel<Tag, 9, 16, gv_rounds(9), 1024, true>);
   if (k3 && !p.remove_center) GV_CASE(9);
   if (k3 && p.remove_center) GV_CASE(8);
   GV_CASE(0);

@@ -22,7 +22,12 @@
 //     data needs (GradState::reach_needed, written by the grad_offset_mask kernel that runs
 //     first: what the sampling points within the reach cap need; a tile that points beyond the
 //     cap land in reads its own, larger number from GradState::far_reach), in strips of
-//     interleaved rows, so that every strip spreads its points evenly over the tile.  Per strip:
+//     interleaved rows, so that every strip spreads its points evenly over the tile.  With lists
+//     (LISTS) the reach stays at a few pixels whatever tails the offsets have, and the points
+//     that land in the tile from farther away are read from its list at the end, as many at a
+//     time as it has lanes: the visits of a tile of 20 x 21 are 930 pixels for a reach of 5 and
+//     1980 for the 12 that a bell of 2 pixels asks for (2x200x334, 10 groups of 16, bf16: 244 ->
+//     170 us).  Per strip:
 //       park   the strip's grad_out rows are copied to LDS;
 //       A      one lane per (group, pixel, kernel tap) recomputes the sampling position and links
 //              a 16-byte entry (m * hy, m * ly, lx, address of the pixel's parked grad_out | next)
@@ -57,7 +62,8 @@ __device__ __forceinline__ int fdiv_small(int n, float inv) { return (int)(((flo
 // NT: lanes per workgroup (512: two workgroups share a CU and overlap each other's phases; 1024: one workgroup with
 // the whole LDS); one (anchor, group) list per lane at most.
 // (the body of the kernel as a function of the workgroup's number, so that a grid can also hold workgroups of another role)
-template <typename Tag, int KP, int CW, int ROUNDS, int NT>
+// LISTS: 3x3 kernels with their centre only.
+template <typename Tag, int KP, int CW, int ROUNDS, int NT, bool LISTS = false>
 __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32_t bid, uint32_t nblocks) {
   constexpr int kValThreads = NT, kMaxAnchorSlots = NT;
   extern __shared__ __align__(16) uint32_t lds32[];
@@ -102,6 +108,7 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
   // how far away the output pixels of those points lie (GradState::far_reach): only such tiles pay for outliers
   const int reach = p.gv_whole ? (1 << 20)
                                : (int)min(max(p.state->reach_needed, p.state->far_reach[dcnv4_far_slot(b, ty, tx, nty, ntx, chunk, n_chunks)]), 1u << 20);
+  const bool listed = LISTS && p.state->listed != 0;
   const int ho_lo = max(0, ceil_div_signed(ty0 - reach - cy0, p.sh));
   const int ho_hi = min(Ho, ceil_div_signed(ty0 + eh + reach - cy0, p.sh));
   const int wo_lo_all = max(0, ceil_div_signed(tx0 - reach - cx0, p.sw));
@@ -138,6 +145,41 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
   auto to_f = [](elem_t raw) { float f[1]; Pack<Tag, 1>::decode(raw, f); return f[0]; };
 
   int parity = 0;                                             // which half of s_head the current strip uses
+  // Phase B: every lane walks its own anchor's list; the next entry is read while the current one is applied.
+  // Corner weights (common.h:48-58, 153-184): modulation * row weight * column weight.
+  auto walk = [&](const uint32_t *head) {
+    if (list_live) {
+      uint32_t e = head[my_list];
+      s_head[parity * kMaxAnchorSlots + my_list] = end_idx;    // the next strip's head of this list
+      const char *go_lane = s_go + my_part * kLaneBytes;
+      u32x4 ent = s_entry[e];
+      while (e != end_idx) {
+        e = ent.w >> 14;
+        const u32x4 next = s_entry[e];
+        const uint32_t a_bits = ent.x, b_bits = ent.y, fx_bits = ent.z;
+        const float wa = __builtin_bit_cast(float, a_bits), wb = __builtin_bit_cast(float, b_bits);
+        const float fxv = __builtin_bit_cast(float, fx_bits), hxv = 1.f - fxv;
+        const float w4[4] = {wa * hxv, wa * fxv, wb * hxv, wb * fxv};
+        const char *g = go_lane + ((ent.w & 0x3fffu) << 4);
+        // the row in pieces of at most 32 bytes, one piece in registers at a time
+        constexpr int kPieceBytes = kLaneBytes < 32 ? kLaneBytes : 32;
+        constexpr int kPiece = kPieceBytes / kParkBytes;       // channels per piece
+#pragma unroll
+        for (int h = 0; h < CW / kPiece; ++h) {
+          park_t gv[kPiece];
+#pragma unroll
+          for (int q = 0; q < kPieceBytes / 16; ++q)
+            *reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(gv) + 16 * q) = *reinterpret_cast<const u32x4 *>(g + kPieceBytes * h + 16 * q);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int c = 0; c < kPiece; ++c) acc[k][h * kPiece + c] = fmaf(w4[k], (float)gv[c], acc[k][h * kPiece + c]);
+          if (h + 1 < CW / kPiece) __builtin_amdgcn_sched_barrier(0);
+        }
+        ent = next;
+      }
+    }
+  };
   for (int wo_lo = wo_lo_all; wo_lo < wo_hi_all && n_rows > 0; wo_lo += cols_cap) {
     const int nwx = min(cols_cap, wo_hi_all - wo_lo);
 
@@ -303,39 +345,50 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
       if (s + 1 < n_strips) prefetch(s + 1);
       __syncthreads();
 
-      // ---- phase B: every lane walks its own anchor's list; the next entry is read while the current one is applied.
-      // Corner weights (common.h:48-58, 153-184): modulation * row weight * column weight.
-      if (list_live) {
-        uint32_t e = head[my_list];
-        s_head[parity * kMaxAnchorSlots + my_list] = end_idx;    // the next strip's head of this list
-        const char *go_lane = s_go + my_part * kLaneBytes;
-        u32x4 ent = s_entry[e];
-        while (e != end_idx) {
-          e = ent.w >> 14;
-          const u32x4 next = s_entry[e];
-          const uint32_t a_bits = ent.x, b_bits = ent.y, fx_bits = ent.z;
-          const float wa = __builtin_bit_cast(float, a_bits), wb = __builtin_bit_cast(float, b_bits);
-          const float fxv = __builtin_bit_cast(float, fx_bits), hxv = 1.f - fxv;
-          const float w4[4] = {wa * hxv, wa * fxv, wb * hxv, wb * fxv};
-          const char *g = go_lane + ((ent.w & 0x3fffu) << 4);
-          // the row in pieces of at most 32 bytes, one piece in registers at a time
-          constexpr int kPieceBytes = kLaneBytes < 32 ? kLaneBytes : 32;
-          constexpr int kPiece = kPieceBytes / kParkBytes;       // channels per piece
+      walk(head);
+      __syncthreads();
+    }
+  }
+
+  // Points of the tile's list, a lane each: its pixel's grad_out row of the point's group, and the entry as in phase A, unless the
+  // pixel was visited.
+  if (LISTS && listed) {
+    const FarList far_list(p, Tag::kBytes, ty, tx, chunk);
+    const int n_far = min(__builtin_amdgcn_readfirstlane((int)static_cast<const FarHeader *>(far_list.slot(p, Tag::kBytes, b, 0))->count), far_list.capacity);
+    const int far_stride = (Dp * kParkBytes / 16 | 1) * 16;
+    const int far_chunk = min(min(NT, (int)end_idx), p.strip_pix * go_stride / far_stride);
+    for (int f0 = 0; f0 < n_far; f0 += far_chunk) {
+      uint32_t *head = s_head + parity * kMaxAnchorSlots;
+      parity ^= 1;
+      if (tid < far_chunk && f0 + tid < n_far) {
+        const FarRecord rec = *static_cast<const FarRecord *>(far_list.slot(p, Tag::kBytes, b, 1 + f0 + tid));
+        const int k = (int)(rec.point & 0xffu), gl = (int)(rec.point >> 8);
+        const int ho = (int)rec.pixel / p.Wo, wo = (int)rec.pixel - ho * p.Wo, ti = k / 3, tjj = k - 3 * ti;
+        const bool visited = dcnv4_away(p, ty, tx, cy0 + ho * p.sh, cx0 + wo * p.sw) <= reach;
+        const elem_t *om = om_img + ((size_t)rec.pixel * p.P_pad + (size_t)((g0 + gl) * 3 * Kp));
+        const elem_t off_x = om[2 * k], off_y = om[2 * k + 1], m_raw = om[2 * Kp + k];
+        const elem_t *src = go_img + ((size_t)rec.pixel * C + (size_t)(g0 + gl) * D);
+        float *dst = reinterpret_cast<float *>(s_go + tid * far_stride);
+        constexpr int kRowVec = 16 / Tag::kBytes;               // groups of 32, 64 or 128 bytes (plan_window_gather)
+        for (int u = 0; u < D; u += kRowVec) {
+          float f[kRowVec];
+          Pack<Tag, kRowVec>::decode(*reinterpret_cast<const typename Pack<Tag, kRowVec>::raw_t *>(src + u), f);
 #pragma unroll
-          for (int h = 0; h < CW / kPiece; ++h) {
-            park_t gv[kPiece];
-#pragma unroll
-            for (int q = 0; q < kPieceBytes / 16; ++q)
-              *reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(gv) + 16 * q) = *reinterpret_cast<const u32x4 *>(g + kPieceBytes * h + 16 * q);
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-#pragma unroll
-              for (int c = 0; c < kPiece; ++c) acc[k][h * kPiece + c] = fmaf(w4[k], (float)gv[c], acc[k][h * kPiece + c]);
-            if (h + 1 < CW / kPiece) __builtin_amdgcn_sched_barrier(0);
-          }
-          ent = next;
+          for (int c = 0; c < kRowVec; c += 4) *reinterpret_cast<f32x4 *>(dst + u + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
+        }
+        const float x = add_rn(sub_rn((float)(cx0 + wo * p.sw), x_sub), mul_rn(add_rn((float)(ti * p.dw), to_f(off_x)), p.offset_scale));
+        const float y = add_rn(sub_rn((float)(cy0 + ho * p.sh), y_sub), mul_rn(add_rn((float)(tjj * p.dh), to_f(off_y)), p.offset_scale));
+        const float fy = floorf(y), fx = floorf(x);
+        const int ay = (int)fy - ty0 + 1, ax = (int)fx - tx0 + 1;
+        if (!visited && (unsigned)ay <= (unsigned)th && (unsigned)ax <= (unsigned)tw) {
+          const float m = to_f(m_raw), ly = y - fy, lx = x - fx;
+          const uint32_t succ = __hip_atomic_exchange(&head[ay * (p.ng_chunk * aw) + gl * aw + ax], (uint32_t)tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          s_entry[tid] = u32x4{__builtin_bit_cast(uint32_t, m * (1.f - ly)), __builtin_bit_cast(uint32_t, m * ly),
+                               __builtin_bit_cast(uint32_t, lx), (uint32_t)(tid * far_stride) >> 4 | (succ << 14)};
         }
       }
+      __syncthreads();
+      walk(head);
       __syncthreads();
     }
   }

@@ -130,24 +130,31 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
 }
 
 // ------------------------------------------------------------------------------- backward
+// Points beyond the near reach that a workgroup looks at one by one, of its 2304; with more it widens the visits of the tiles around.
+constexpr int kBeyondMost = 512;
+
 // grad_offset_mask (the part of dcnv4_col2im_cuda.cuh:280-350 and common.h:188-211 that does not scatter): the four
 // corner . grad_out products of a point give d/dx, d/dy and d/dmask.  Where lanes share a group each forms the gradients of the
 // points it prepared.  The rows then go through LDS, in the window's place, so that they leave as whole runs; points outside the
-// window are served in between.  Also folds the reach that the grad_value kernel has to cover into GradState.
-template <typename Tag, int LPG, int UNITS>
+// window are served in between.  Also folds the reach that the grad_value kernel has to cover into GradState, and with LISTS hands
+// it the points that lie far from their pixels (FarList): a variant of its own, because what it keeps for them in registers costs
+// 2 % (64x56x56, 4 groups of 16, fp16: 61.9 -> 63.5 us).
+template <typename Tag, int LPG, int UNITS, bool LISTS>
 __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_window_kernel(const DcnLaunch p) {
   extern __shared__ u32x4 lds128[];
-  __shared__ uint32_t s_reach;
+  __shared__ uint32_t s_reach, s_beyond_count;
+  __shared__ uint16_t s_beyond[LISTS ? kBeyondMost : 1];      // points beyond the near reach: lane | point << 8
   typedef typename RawWord<Tag::kBytes>::type elem_t;
   constexpr int kGroups = UNITS / LPG, kCell = UNITS * 32;
   char *lds = reinterpret_cast<char *>(lds128);
   const WindowTile t = window_tile<kGroups>(p, blockIdx.x, gridDim.x);
   const WindowFrame<UNITS> frame(t);
-  if (threadIdx.x == 0) s_reach = 0u;
+  if (threadIdx.x == 0) s_reach = s_beyond_count = 0u;
 
   constexpr int kPixels = kWindowThreads / UNITS, kPerGroup = kPixels * LPG;
   const int gl = threadIdx.x / kPerGroup, part = threadIdx.x & (LPG - 1), q = threadIdx.x % kPerGroup / LPG;
-  const int py = exact_div(q, __builtin_amdgcn_rcpf((float)p.gt_w)), px = q - py * p.gt_w;
+  const float inv_gt_w = __builtin_amdgcn_rcpf((float)p.gt_w);
+  const int py = exact_div(q, inv_gt_w), px = q - py * p.gt_w;
   const bool active = py < t.th && px < t.tw && t.g0 + gl < p.G;
   const int ho = t.oy0 + py, wo = t.ox0 + px;
   const size_t pixel = active ? (size_t)t.b * p.Q + (size_t)ho * p.Wo + wo : 0;
@@ -210,8 +217,8 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
   const int lane_bytes = (gl * LPG + part) * 32;
   constexpr int kOwn = PointRows<Tag, LPG>::kOwn;
   float result[kOwn][3];
-  uint32_t far = 0;
-  uint32_t reach_bits = 0;      // bits of the largest distance so far: non-negative floats order like their bits
+  uint32_t far = 0, beyond = 0;      // a bit for each point that this lane prepares: served from memory, beyond the near reach
+  uint32_t reach_bits = 0;           // bits of the largest distance so far: non-negative floats order like their bits
   if (active) {
 #pragma unroll
     for (int i = 0; i < kOwn; ++i) {
@@ -229,6 +236,8 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
         counts = inside;
       }
       const float dist = fmaxf(fabsf(x - p0xf), fabsf(y - p0yf));
+      if constexpr (LISTS)
+        if (__any(counts && dist > p.gv_near)) beyond |= (uint32_t)(counts && dist > p.gv_near && (LPG == 1 || part + i * LPG < 9)) << k;
       reach_bits = max(reach_bits, (counts && dist <= p.gv_reach_cap) ? __builtin_bit_cast(uint32_t, dist) : 0u);
       float d[4] = {0.f, 0.f, 0.f, 0.f};
       auto one = [&](auto jj) {
@@ -254,7 +263,44 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (LISTS) {
+    if (__any(beyond != 0)) {      // a wave asks for room once
+      const uint32_t mine = (uint32_t)__builtin_popcount(beyond), upto = wave_prefix_sum(mine), all = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+      uint32_t at = 0;
+      if ((threadIdx.x & 63) == 0) at = atomicAdd(&s_beyond_count, all);
+      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+      if (at + all <= kBeyondMost) {
+        at += upto - mine;
+        for (uint32_t left = beyond; left != 0; left &= left - 1) s_beyond[at++] = (uint16_t)(threadIdx.x | (uint32_t)__builtin_ctz(left) << 8);
+      }
+    }
+  }
   __syncthreads();      // nobody reads the window any more
+
+  // Records for the tiles of grad_value that a point lands in from beyond the near reach: a lane looks at a point, asks for a place
+  // in the list, and writes the record behind the rows, which the round trip overlaps.
+  const int n_beyond = LISTS ? (int)s_beyond_count : 0;
+  const bool dense = n_beyond > kBeyondMost;
+  FarPlace first_place;
+  if (n_beyond != 0 && !dense) {
+    for (int i = threadIdx.x; i < n_beyond; i += kWindowThreads) {
+      const int lane = s_beyond[i] & 255, k = s_beyond[i] >> 8;
+      const int its_q = lane % kPerGroup / LPG, its_py = exact_div(its_q, inv_gt_w), its_g = t.g0 + lane / kPerGroup;
+      const int ry = t.oy0 + its_py, rx = t.ox0 + its_q - its_py * p.gt_w, its_pixel = ry * p.Wo + rx;
+      float f3[3];
+      point_of_row<Tag>(static_cast<const char *>(p.offset_mask) + (((size_t)t.b * p.Q + its_pixel) * p.P_pad + (size_t)its_g * 27) * Tag::kBytes, k, f3);
+      const int kx = exact_div(k, 1.f / 3.f), cy = 1 - p.ph + ry, cx = 1 - p.pw + rx;
+      const float x = add_rn(sub_rn((float)cx, p.offset_scale), mul_rn(add_rn((float)kx, f3[0]), p.offset_scale));
+      const float y = add_rn(sub_rn((float)cy, p.offset_scale), mul_rn(add_rn((float)(k - 3 * kx), f3[1]), p.offset_scale));
+      const int chunk = its_g / p.ng_chunk;
+      const FarRecord record = {(uint32_t)its_pixel, (uint32_t)k | (uint32_t)(its_g - chunk * p.ng_chunk) << 8};
+      dcnv4_far_tiles(p, (int)floorf(y), (int)floorf(x), cy, cx, [&](int ty, int tx, int away) {
+        FarPlace place(p, Tag::kBytes, t.b, ty, tx, chunk, away, record);
+        if (first_place.ty < 0) first_place = place;
+        else place.keep(p, Tag::kBytes);
+      });
+    }
+  }
 
   // rows of 27 gradients in LDS, a run of kGroups of them per pixel
   constexpr int kRun = kGroups * 27, kPitch = Tag::kBytes == 2 ? (kRun + 1) / 2 * 2 : kRun;      // elements: runs start on a word
@@ -287,7 +333,10 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
         x = add_rn(x_base, mul_rn(add_rn((float)i, f3[0]), p.offset_scale));
         y = add_rn(y_base, mul_rn(add_rn((float)(k - 3 * i), f3[1]), p.offset_scale));
         const Tap tp = make_tap(y, x, p.H, p.W, base, pix_bytes);
-        if (tp.valid != 0 && fmaxf(fabsf(x - p0xf), fabsf(y - p0yf)) > p.gv_reach_cap) dcnv4_fold_far_point(p, t.b, g, tp.y0, tp.x0, p0y, p0x);
+        if (tp.valid != 0 && (!LISTS || dense) && fmaxf(fabsf(x - p0xf), fabsf(y - p0yf)) > p.gv_reach_cap) {
+          if (!LISTS) dcnv4_fold_far_point(p, t.b, g, tp.y0, tp.x0, p0y, p0x);
+          else if (part == 0) dcnv4_far_tiles(p, tp.y0, tp.x0, p0y, p0x, [&](int ty, int tx, int away) { dcnv4_widen_visit(p, t.b, ty, tx, g / p.ng_chunk, away); });
+        }
         dots([&](int cn, int v) { return buffer_load<16>(value, tp.off[cn] + 16u * v); }, d);
         gradients(d, tp.ly, tp.lx, f3[2], r);
         if (part == k % LPG) put(k, r);
@@ -300,7 +349,8 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t *dst = &p.state->reach_needed;
-    const uint32_t mine = s_reach;
+    const uint32_t mine = n_beyond != 0 ? (uint32_t)p.gv_near : s_reach;
+    if (n_beyond != 0 && p.state->listed == 0) p.state->listed = 1u;
     if (mine > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, mine);
   }
   // runs to memory, a word a lane whatever the alignment, the last element of an odd run alone
@@ -331,6 +381,17 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
       reinterpret_cast<elem_t *>(gom)[((size_t)y * p.Wo + x) * p.P_pad + run + e] = elem_t(0);
     }
   }
+  if (first_place.ty >= 0) first_place.keep(p, Tag::kBytes);
+  if (dense) {      // every tile that a point within the cap can reach from here is visited as far as the farthest of them
+    const int r = (int)s_reach, y_lo = max(1 - p.ph + t.oy0 - r, 0) / p.tile_h, y_hi = min(1 - p.ph + t.oy0 + t.th - 1 + r, p.H - 1) / p.tile_h;
+    const int x_lo = max(1 - p.pw + t.ox0 - r, 0) / p.tile_w, x_hi = min(1 - p.pw + t.ox0 + t.tw - 1 + r, p.W - 1) / p.tile_w;
+    const int chunk_lo = t.g0 / p.ng_chunk, chunks = (min(t.g0 + kGroups, p.G) - 1) / p.ng_chunk - chunk_lo + 1;
+    const int columns = x_hi - x_lo + 1, around = max((y_hi - y_lo + 1) * columns, 0) * chunks;
+    for (int i = threadIdx.x; i < around; i += kWindowThreads) {
+      const int tile = i / chunks, row = tile / columns;
+      dcnv4_widen_visit(p, t.b, y_lo + row, x_lo + tile - row * columns, chunk_lo + i - tile * chunks, r);
+    }
+  }
 }
 
 template <typename Tag, int LPG, int UNITS, bool BWD>
@@ -339,11 +400,11 @@ hipError_t launch_units(const DcnLaunch &p, hipStream_t stream) {
   const int Ho = p.Q / p.Wo;
   const unsigned tiles = (unsigned)(p.n_pix / p.Q) * ((Ho + p.gt_h - 1) / p.gt_h) * ((p.Wo + p.gt_w - 1) / p.gt_w) * ((p.G + kGroups - 1) / kGroups);
   auto go = [&](auto kernel) {
-    if (hipError_t e = ensure_dynamic_lds_limit(reinterpret_cast<const void *>(kernel), kMaxLdsPerWorkgroup - 1024)) return e;
+    if (hipError_t e = ensure_dynamic_lds_limit(reinterpret_cast<const void *>(kernel), kMaxLdsPerWorkgroup - 8192)) return e;
     hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kWindowThreads), dcnv4_window_lds_bytes(p, UNITS), stream, p);
     return hipGetLastError();
   };
-  if constexpr (BWD) return go(dcnv4_offset_mask_grad_window_kernel<Tag, LPG, UNITS>);
+  if constexpr (BWD) return p.gv_lists ? go(dcnv4_offset_mask_grad_window_kernel<Tag, LPG, UNITS, true>) : go(dcnv4_offset_mask_grad_window_kernel<Tag, LPG, UNITS, false>);
   else return go(dcnv4_forward_window_kernel<Tag, LPG, UNITS>);
 }
 

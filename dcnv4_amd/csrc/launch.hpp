@@ -22,7 +22,7 @@ constexpr size_t kMaxLdsPerWorkgroup = 160 * 1024;  // gfx950
 // Device-side scratch word block shared by the kernels of one backward call (256 bytes).
 constexpr int kFarSlots = 56;
 struct GradState {
-  uint32_t unused0;
+  uint32_t listed;         // DCNv4: not 0 if a tile may have a list of far points
   uint32_t unused1;
   uint32_t reach_needed;   // DCNv4: ceiling of the largest Chebyshev distance (pixels) of an in-range sampling point from its output pixel's reference point, over the points within the reach cap
   uint32_t reserved;       // attention backward: set when a level has more tiles than the binning kernel can count
@@ -96,7 +96,16 @@ struct DcnLaunch {
   int gt_reach;             // input pixels around an output pixel's reference point that the window covers
   int dual_interleave;      // two-role backward: workgroups of the two roles alternate in eights (else one role after the other)
   float gv_reach_cap;       // sampling points farther than this from their reference point stay out of reach_needed and are folded into GradState::far_reach
+  int gv_lists;             // 1: tiles are visited by the pixels within gv_near of them, and points that land in them from farther away are listed (FarHeader)
+  float gv_near;            // a whole number of pixels
 };
+
+// How far outside a grad_value tile a reference point lies: the pixels within the reach of it are visited.
+__host__ __device__ inline int dcnv4_away(const DcnLaunch &p, int ty, int tx, int y, int x) {
+  const int dy = y - ty * p.tile_h, dx = x - tx * p.tile_w;
+  const int oy = -dy > dy - (p.tile_h - 1) ? -dy : dy - (p.tile_h - 1), ox = -dx > dx - (p.tile_w - 1) ? -dx : dx - (p.tile_w - 1);
+  return oy > ox ? oy : ox;
+}
 
 // Slot of GradState::far_reach that the workgroup of the grad_value kernel for (image within its launch, tile, chunk of
 // groups) uses.
@@ -119,6 +128,72 @@ __device__ inline void dcnv4_fold_far_point(const DcnLaunch &p, int img, int g, 
     if (b > 0) atomicMax(&p.state->far_reach[dcnv4_far_slot(img, ty, tx, nty, ntx, chunk, n_chunks)], (uint32_t)min(b, 1 << 20));
   }
 }
+
+// Lists of far points (gv_lists): the tiles of the grad_value kernel are visited by the output pixels within a few pixels of
+// them, and a tile's list names the points that land in it from farther away.  A list lies in the tile's own part of
+// grad_value, which nobody else touches until the tile's workgroup overwrites it with its result: 8-byte slots, the header
+// first, then the records.  Where a list is full, or a workgroup of the first kernel has too many such points, far_reach widens
+// the visit instead; records of pixels that are visited count for nothing.
+struct FarHeader {
+  uint32_t count;      // places given out; the first `capacity` hold records
+  uint32_t unused;
+};
+struct FarRecord {
+  uint32_t pixel;      // of the image
+  uint32_t point;      // index among the group's points | group of the chunk << 8
+};
+constexpr int kFarSlotBytes = 8;
+static_assert(sizeof(FarHeader) == kFarSlotBytes && sizeof(FarRecord) == kFarSlotBytes, "a slot holds either");
+constexpr int kFarMost = 8191;      // records of a tile, at most
+constexpr int kFarShare = 4;        // and of its points, one in four
+struct FarList {
+  int ty0, tx0, tw, g0, cell_bytes, capacity;
+  __device__ __forceinline__ FarList(const DcnLaunch &p, int elem_bytes, int ty, int tx, int chunk) {
+    ty0 = ty * p.tile_h; tx0 = tx * p.tile_w;
+    g0 = chunk * p.ng_chunk;
+    tw = min(p.tile_w, p.W - tx0);
+    const int cells = min(p.tile_h, p.H - ty0) * tw, ng = min(p.ng_chunk, p.G - g0);
+    cell_bytes = ng * p.D * elem_bytes;
+    capacity = min(min(cells * (cell_bytes / kFarSlotBytes) - 1, cells * ng * p.Kp / kFarShare), kFarMost);
+  }
+  __device__ __forceinline__ void *slot(const DcnLaunch &p, int elem_bytes, int img, int i) const {
+    const int byte = i * kFarSlotBytes, cell = byte / cell_bytes, cy = cell / tw;
+    const size_t at = ((size_t)img * p.H + ty0 + cy) * p.W + tx0 + cell - cy * tw;
+    return static_cast<char *>(p.grad_value) + (at * (size_t)(p.G * p.D) + (size_t)g0 * p.D) * elem_bytes + (byte - cell * cell_bytes);
+  }
+};
+// The tile is visited by pixels as far as `away`.
+__device__ __forceinline__ void dcnv4_widen_visit(const DcnLaunch &p, int img, int ty, int tx, int chunk, int away) {
+  const int nty = (p.H + p.tile_h - 1) / p.tile_h, ntx = (p.W + p.tile_w - 1) / p.tile_w, n_chunks = (p.G + p.ng_chunk - 1) / p.ng_chunk;
+  uint32_t *reach = &p.state->far_reach[dcnv4_far_slot(img, ty, tx, nty, ntx, chunk, n_chunks)];
+  if ((uint32_t)away > __hip_atomic_load(reach, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(reach, (uint32_t)away);
+}
+// The tiles that a point with first corner (y0, x0), a corner of it in the image, lands in from beyond the near reach.
+template <typename F>
+__device__ __forceinline__ void dcnv4_far_tiles(const DcnLaunch &p, int y0, int x0, int p0y, int p0x, F each) {
+  const int ty_b = min(y0 + 1, p.H - 1) / p.tile_h, tx_b = min(x0 + 1, p.W - 1) / p.tile_w;
+  for (int ty = max(y0, 0) / p.tile_h; ty <= ty_b; ++ty)
+    for (int tx = max(x0, 0) / p.tile_w; tx <= tx_b; ++tx) {
+      const int away = dcnv4_away(p, ty, tx, p0y, p0x);
+      if (away > (int)p.gv_near) each(ty, tx, away);
+    }
+}
+// A record and the place it was given in a tile's list.
+struct FarPlace {
+  int img, ty = -1, tx, chunk, away;
+  uint32_t place;
+  FarRecord record;
+  __device__ __forceinline__ FarPlace() {}
+  __device__ __forceinline__ FarPlace(const DcnLaunch &p, int elem_bytes, int img_, int ty_, int tx_, int chunk_, int away_, const FarRecord &record_)
+      : img(img_), ty(ty_), tx(tx_), chunk(chunk_), away(away_), record(record_) {
+    place = atomicAdd(&static_cast<FarHeader *>(FarList(p, elem_bytes, ty, tx, chunk).slot(p, elem_bytes, img, 0))->count, 1u);
+  }
+  __device__ __forceinline__ void keep(const DcnLaunch &p, int elem_bytes) const {
+    const FarList list(p, elem_bytes, ty, tx, chunk);
+    if (place < (uint32_t)list.capacity) *static_cast<FarRecord *>(list.slot(p, elem_bytes, img, 1 + (int)place)) = record;
+    else dcnv4_widen_visit(p, img, ty, tx, chunk, away);
+  }
+};
 
 // Lower bound of the reach cap: the statistic in reach_needed then stays at what the bulk of the sampling points needs
 // when a few offsets are outliers.
