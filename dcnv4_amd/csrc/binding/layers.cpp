@@ -200,6 +200,14 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
     launch(code, p, stream);
   };
 
+  // a product and the normalisation behind it in one kernel
+  auto rows_normed = [&](const void *a, const Tensor &wt, const Tensor &b, int64_t k, const NormParams &n, const Tensor &gamma, const void *residual,
+                         void *stream_out, void *normed_out) {
+    RowsLaunch p = {a, ptr(wt), ptr(b), rows, (int)c, (int)k, {ptr(n.weight), ptr(n.bias), n.eps, ptr(gamma), residual, stream_out, normed_out, normed_out != nullptr}};
+    hip_check(launch_rows(code, p, static_cast<hipStream_t>(stream)), "linear layer launch");
+  };
+  const bool whole_rows = rows_fits(code, rows, (int)c, (int)c) && rows_fits(code, rows, (int)c, (int)l.hidden);
+
   // DCNv4 half
   const bool norm_first = !l.post_norm && l.dw_kernel == 0;      // the normalised rows go into the projections alone
   const void *source = in;
@@ -222,30 +230,47 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
   check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
                              l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
   const bool fused = mlp_fits(code, rows, (int)c, (int)l.hidden);      // the MLP in one kernel
-  auto mlp = [&](const Tensor &gamma, const void *residual, void *o) {
-    const MlpLaunch m = {middle, ptr(l.fc1_w), ptr(l.fc1_b), ptr(l.fc2_w), ptr(l.fc2_b), ptr(gamma), residual, o, rows, (int)c, (int)l.hidden};
+  auto mlp = [&](const Tensor &gamma, const void *residual, void *o, const NormParams *n) {
+    MlpLaunch m = {middle, ptr(l.fc1_w), ptr(l.fc1_b), ptr(l.fc2_w), ptr(l.fc2_b), ptr(gamma), residual, o, rows, (int)c, (int)l.hidden, {}};
+    if (n != nullptr) m.norm = {ptr(n->weight), ptr(n->bias), n->eps, ptr(gamma), residual, o, nullptr, 0};
     hip_check(launch_mlp(code, m, static_cast<hipStream_t>(stream)), "MLP launch");
   };
   LinearLaunch fc1 = {};
   fc1.p[0] = {last, ptr(l.fc1_w), ptr(l.fc1_b), nullptr, nullptr, hidden, (int)l.hidden};
   fc1.count = 1; fc1.rows = rows; fc1.k = (int)c; fc1.gelu = 1;
   if (l.post_norm) {
-    linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
-    if (fused) {
-      norm(last, l.norm1, l.gamma1, in, middle);
-      mlp(Tensor(), nullptr, last);
+    if (whole_rows) {
+      rows_normed(sampled, l.output_w, l.output_b, c, l.norm1, l.gamma1, in, middle, nullptr);
+      fc1.p[0].a = middle;
     } else {
-      normed(fc1, l.norm1, l.gamma1, in, middle);
-      linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
+      linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
+      if (fused) norm(last, l.norm1, l.gamma1, in, middle);
     }
-    norm(last, l.norm2, l.gamma2, middle, out.data_ptr());
-  } else {
-    linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
     if (fused) {
-      norm(last, l.norm2, Tensor(), nullptr, middle);
-      mlp(l.gamma2, last, out.data_ptr());
+      mlp(l.gamma2, middle, out.data_ptr(), &l.norm2);
     } else {
-      normed(fc1, l.norm2, Tensor(), nullptr, middle);
+      if (whole_rows) launch(code, fc1, stream);
+      else normed(fc1, l.norm1, l.gamma1, in, middle);
+      if (whole_rows) {
+        rows_normed(hidden, l.fc2_w, l.fc2_b, l.hidden, l.norm2, l.gamma2, middle, out.data_ptr(), nullptr);
+      } else {
+        linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, Tensor(), nullptr, last);
+        norm(last, l.norm2, l.gamma2, middle, out.data_ptr());
+      }
+    }
+  } else {
+    if (whole_rows) {
+      rows_normed(sampled, l.output_w, l.output_b, c, l.norm2, l.gamma1, in, last, middle);
+      fc1.p[0].a = middle;
+    } else {
+      linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
+      if (fused) norm(last, l.norm2, Tensor(), nullptr, middle);
+    }
+    if (fused) {
+      mlp(l.gamma2, last, out.data_ptr(), nullptr);
+    } else {
+      if (whole_rows) launch(code, fc1, stream);
+      else normed(fc1, l.norm2, Tensor(), nullptr, middle);
       linear(hidden, l.fc2_w, l.fc2_b, l.hidden, c, false, l.gamma2, last, out.data_ptr());
     }
   }

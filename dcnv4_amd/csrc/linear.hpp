@@ -57,12 +57,35 @@ bool linear_fits(int dtype, long long rows, int n, int k);
 bool linear_takes_norm(const LinearLaunch &p);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
 
+// What follows a product in a layer together with its normalisation (16-bit types), every step rounded as the kernels one by one round
+// it: after_residual  stream = gamma * (product + bias) + residual, normed = norm(stream); else the product rounded to the type and
+// stream = residual + gamma * norm(product + bias).  gamma and residual may be null, normed goes with after_residual.
+struct NormEpilogue {
+  const void *weight, *bias;      // null: no normalisation
+  float eps;
+  const void *gamma, *residual;
+  void *stream, *normed;
+  int after_residual;
+};
+
+// a [rows, k] times w [n, k] with the rows of the result whole in a workgroup (linear_rows.hip): up to 512 features, rows enough.
+struct RowsLaunch {
+  const void *a, *w, *bias;
+  long long rows;
+  int n, k;
+  NormEpilogue norm;
+};
+bool rows_fits(int dtype, long long rows, int n, int k);
+hipError_t launch_rows(int dtype, const RowsLaunch &p, hipStream_t stream);
+
 // (gelu(a w1' + b1) w2' + b2) * gamma + residual over [rows, c], w1 [hidden, c], w2 [c, hidden]; b1, b2, gamma, residual may be null.
+// With norm, without after_residual, it has gamma, residual and result: residual + gamma * norm(...).
 struct MlpLaunch {
   const void *a, *w1, *b1, *w2, *b2, *gamma, *residual;
   void *out;
   long long rows;
   int c, hidden;
+  NormEpilogue norm;
 };
 constexpr long long kMlpLeastRows = 32768;      // a workgroup of 128 rows for every CU
 // 16-bit types, up to 224 channels (more do not fit a wave's registers), hidden features in whole steps.
