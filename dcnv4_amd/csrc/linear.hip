@@ -1,6 +1,11 @@
 // Linear layers on the matrix cores, with what follows the product fused into its epilogue: bias, GELU,
-// layer scale, residual.  Two kernels:
+// layer scale, residual.  Three kernels:
 //
+//  linear_wide_kernel: wide products in 16 bits.  Eight waves own 256 rows x 128 features, 64 x 64 each; operands come by slices of
+//    64 bytes into three buffers of 24 KB, two slices under way while the matrix cores work on a third, and a CU holds two
+//    workgroups.  What an operand costs on its way into LDS bounds these products as much as the matrix cores do - the matrix
+//    instructions alone, with their reads of LDS, take half the time (25088 x 1792 x 448: 36 of 68 us, the loads alone 43, the
+//    epilogue with the GELU 42) - and a tile of twice the rows brings a quarter less.
 //  linear_tiled_kernel: many rows.  A workgroup of four waves owns BM rows x BN features; both operands come in slices of
 //    128 bytes along the depth, 16 bytes a lane, straight into LDS (two buffers, one barrier a slice: the next slice's loads are in
 //    flight while the matrix cores work on this one).  The 16-byte vectors of a row are stored at position
@@ -13,6 +18,7 @@
 //    straight from memory and meet in LDS once.  What the epilogue reads is requested first.  With a layer normalisation in
 //    front the workgroup normalises its 32 rows itself, into LDS: each does so again for every 32 features, but a launch less
 //    is 3 us less for the device and as much for the host.
+#include "fragments.hpp"
 #include "linear.hpp"
 #include "launch.hpp"
 #include "mfma.hpp"
@@ -187,6 +193,89 @@ __global__ void __launch_bounds__(256) linear_tiled_kernel(const LinearLaunch p,
 #pragma unroll
     for (int u = 0; u < 16 / rows_per_pass; ++u) {
       const int r = u * rows_per_pass + lane / lanes_per_row, row = wm * (BM / WM) + j * 16 + r;
+      const f32x4 lo = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col), hi = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col + 4);
+      float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      if (row < live_m && n < live_n) finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+constexpr int kWideRows = 256, kWideFeatures = 128, kWideBuffers = 3;
+template <typename Tag, bool EXTRA>
+__global__ void __launch_bounds__(512, 2) linear_wide_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
+  static_assert(Tag::kBytes == 2, "16-bit types");
+  constexpr int kWaves = 8, MF = 4, NF = 4, kTileBytes = (kWideRows + kWideFeatures) * 64, kLoads = kTileBytes / 1024 / kWaves;
+  __shared__ __align__(16) char lds[kWideBuffers * kTileBytes];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t tile = xcd_contiguous_block(blockIdx.x, gridDim.x);
+  const int tm = tile / tiles_n;
+  int tn = tile % tiles_n;
+  const int which = tn >= tiles_n0;
+  const LinearProblem &q = p.p[which];
+  if (which) tn -= tiles_n0;
+  const long long m0 = (long long)tm * kWideRows;
+  const int n0 = tn * kWideFeatures, k = p.k, slices = (k + 31) / 32;
+  const int live_m = (int)min((long long)kWideRows, p.rows - m0), live_n = min(kWideFeatures, q.n - n0);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const uint16_t *>(q.a) + (size_t)m0 * k, (uint32_t)live_m * k * 2);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const uint16_t *>(q.w) + (size_t)n0 * k, (uint32_t)live_n * k * 2);
+
+  // a wave's load covers sixteen rows of a tile: lane l takes row l / 4
+  const int row16 = lane >> 2, vector = (lane & 3) ^ (row16 >> 2);
+  uint32_t offset[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = (i * kWaves + wave) * 16 + row16;             // rows of the row tile, then of the feature tile
+    offset[i] = (uint32_t)((i < kWideRows / 16 / kWaves ? row : row - kWideRows) * k * 2 + vector * 16);
+  }
+  auto stage = [&](int s, int buffer) {
+    const bool in = s * 32 + vector * 8 < k;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      load_to_lds(i < kWideRows / 16 / kWaves ? ra : rw, lds + buffer * kTileBytes + (i * kWaves + wave) * 1024, in ? offset[i] + (uint32_t)s * 64u : kDropOffset);
+  };
+  const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, kb = lane >> 4;
+  const uint32_t at = lds_address(lds) + fragment_offset(r16, kb), at_m = at + wm * MF * 1024, at_n = at + kWideRows * 64 + wn * NF * 1024;
+  f32x4 acc[NF][MF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < MF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kWideBuffers - 1; ++s)
+    if (s < slices) stage(s, s);
+  int cur = 0;
+  for (int s = 0; s < slices; ++s) {
+    wait_behind<kWideBuffers - 2, kLoads, kLoads>(slices - 1 - s, false);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    u32x4 fm[MF], fn[NF];
+    read_fragments(fm, at_m + cur * kTileBytes);
+    read_fragments(fn, at_n + cur * kTileBytes);
+    if (s + kWideBuffers - 1 < slices) stage(s + kWideBuffers - 1, cur == 0 ? kWideBuffers - 1 : cur - 1);
+    fragments_arrived(fm);
+    fragments_arrived(fn);
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int j = 0; j < MF; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[i], fm[j], acc[i][j]);
+    cur = cur == kWideBuffers - 1 ? 0 : cur + 1;
+  }
+  // Epilogue as in linear_tiled_kernel, in the two buffers that the last slice does not use: nobody reads those any more.
+  constexpr int TN = NF * 16, kTurn = TN + 4, kPerBuffer = kTileBytes / (16 * kTurn * 4);
+  static_assert(kPerBuffer * (kWideBuffers - 1) >= kWaves, "two buffers hold every wave's sixteen rows");
+  const int buffer = (cur + wave / kPerBuffer) % kWideBuffers;
+  float *turn = reinterpret_cast<float *>(lds + buffer * kTileBytes) + wave % kPerBuffer * 16 * kTurn;
+  const int col = (lane & 7) * 8, n = wn * TN + col;
+  const Columns<Tag> columns(q, n0 + n, n < live_n);
+#pragma unroll
+  for (int j = 0; j < MF; ++j) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) *reinterpret_cast<f32x4 *>(turn + r16 * kTurn + i * 16 + kb * 4) = acc[i][j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = u * 8 + (lane >> 3), row = (wm * MF + j) * 16 + r;
       const f32x4 lo = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col), hi = *reinterpret_cast<const f32x4 *>(turn + r * kTurn + col + 4);
       float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       if (row < live_m && n < live_n) finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v);
@@ -371,6 +460,15 @@ hipError_t launch_tiled(const LinearLaunch &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <typename Tag, bool EXTRA>
+hipError_t launch_wide(const LinearLaunch &p, hipStream_t stream) {
+  const long long tiles_m = (p.rows + kWideRows - 1) / kWideRows;
+  const int tiles_n0 = (p.p[0].n + kWideFeatures - 1) / kWideFeatures, tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kWideFeatures - 1) / kWideFeatures : 0);
+  if (tiles_m * tiles_n > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((linear_wide_kernel<Tag, EXTRA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, stream, p, tiles_n0, tiles_n);
+  return hipGetLastError();
+}
+
 template <typename Tag, bool EXTRA, int WAVES, int NORM>
 hipError_t launch_few_waves(const LinearLaunch &p, hipStream_t stream) {
   const int tiles_m = (int)((p.rows + kFewTile - 1) / kFewTile), tiles_n0 = (p.p[0].n + kFewTile - 1) / kFewTile;
@@ -394,12 +492,14 @@ hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
   return steps <= 16 ? launch_few_waves<Tag, EXTRA, 4, 0>(p, stream) : launch_few_waves<Tag, EXTRA, 8, 0>(p, stream);
 }
 
-// Which kernel and tile: enough workgroups for the 256 CUs first, then the widest tile whose padding does not cost more
-// than it saves.  Measured (fp16, tile rows x features; us):
+// Which kernel and tile: enough workgroups for the 256 CUs first, then the tile that brings fewer bytes.  Measured (fp16, tile
+// rows x features; us):
 //   few rows against 64x64: 49 x 512 x 2048 9.5 / 11.1, 392 x 512 x 2048 9.8 / 11.4, 1568 x 256 x 1024 9.6 / 7.1
-//   128x64 against 128x128: 25088 x 448 x 448 17.7 / 18.9, 25088 x 1792 x 448 62.5 / 55.5, 6272 x 3584 x 896 59.3 / 51.4,
-//     6272 x 1512 x 896 25.4 / 30.1 (600 against 588 tiles of which the last round is a third full)
-//   256x64 where the width is not a multiple of 128: 401408 x 192 x 112 52.4 against 62.0
+//   256x128 against 128x64 or 128x128, from seven eighths of two workgroups a CU on: 25088 x 608 x 224 19.6 -> 16.1 (490 tiles),
+//     6272 x 2560 x 640 39.0 -> 36.4 (500), 12544 x 1792 x 448 with what training adds 49.7 -> 44.0, 52.9 -> 44.5 (686), 25088 x 1792 x 448
+//     73.5 -> 70.1 (1372), 100352 x 608 x 224 58.1 -> 47.6 (1960), 401408 x 304 x 112 120 -> 110; below: 25088 x 448 x 1792 56.0 -> 61.3 (392),
+//     6272 x 896 x 3584 53.6 -> 63.8 (175).  Padding to 128 features costs less than it saves up to 80 per cent (401408 x 216 x 80
+//     77 -> 62); 64 features take 256x64: 401408 x 64 x 64 23.3 against 25.3
 template <typename Tag, bool EXTRA>
 hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
   auto tiles = [&](int bm, int bn) {
@@ -413,9 +513,11 @@ hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
     return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
   } else {
     if (tiles(128, 64) < kCus) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
-    const long long wide = tiles(128, 128), narrow = tiles(128, 64);
-    if (wide < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
-    if (20 * wide <= 11 * narrow) return launch_tiled<Tag, EXTRA, 128, 128, 2, 2>(p, stream);
+    int features = 0;
+    for (int i = 0; i < p.count; ++i) features += p.p[i].n;
+    const long long wide = tiles(kWideRows, kWideFeatures), padded = tiles(1 << 30, kWideFeatures) * kWideFeatures;
+    if (wide >= 2 * kCus * 7 / 8 && 5 * padded <= 9 * features) return launch_wide<Tag, EXTRA>(p, stream);
+    if (tiles(128, 128) < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
     return launch_tiled<Tag, EXTRA, 256, 64, 4, 1>(p, stream);
   }
 }
