@@ -29,8 +29,8 @@ __device__ __forceinline__ void read_fragments(u32x4 (&f)[N], uint32_t at, std::
 }
 template <int N>
 __device__ __forceinline__ void read_fragments(u32x4 (&f)[N], uint32_t at) { read_fragments(f, at, std::make_integer_sequence<int, N>{}); }
-template <int N>
-__device__ __forceinline__ void fragments_arrived(u32x4 (&f)[N]) {
+template <typename T, int N>
+__device__ __forceinline__ void fragments_arrived(T (&f)[N]) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));

@@ -2,28 +2,45 @@
 //
 // linear_weight_grad_kernel: grad_w[n, k] = sum over rows of grad_out[row, n] * in[row, k], for all the linear layers of a
 // block in one launch.  The reduction runs over the slow axis of both operands, so a fragment's eight values lie a row
-// apart: slices of 64 rows (32 in fp32) come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns them
-// on the way into registers (16 lanes read 4 rows x 16 columns; lane i gets column i).  A row's 32-byte units are stored at
+// apart: slices of 8 KB of either operand come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns
+// them on the way into registers (16 lanes read 4 rows x 16 columns; lane i gets column i).  A row's 32-byte units are stored at
 // unit ^ f(row), f taking each value once over the eight rows that half a wave reads, so those reads fall into different
 // banks.  The rows are split over workgroups until the chip is full, partial sums are fp32 and are added in split order by
 // linear_grad_reduce_kernel: no atomics, the same bits every time.  The bias gradient is one more matrix instruction per
 // fragment, against a vector of ones.
+//   What bounds it is the operands' way into LDS (10 to 13 TB/s over the chip, most of it from L2), so the tile is as large as the
+// registers allow, and the latency of a slice: three buffers keep two slices under way behind the one that is multiplied, 48 KB,
+// three workgroups to a CU.  Two buffers, each waited for in full, were 64 KB with the 128-wide tile, two workgroups to a CU.
+// Sums included, us, before -> now, five layers of C channels, fp16: 12544 x 448 121 -> 103, 3136 x 896 119 -> 88, 50176 x 224 247 ->
+// 135, 200704 x 112 257 -> 155, 50176 x 128 72 -> 47, 25088 x 64 33 -> 17, 392 x 256 7.0 -> 6.4; 200704 x 64 87 -> 89 (its operands
+// alone are 69 at the rate of a copy).  The four products of 256 channels, 40394 rows, fp32: 231 -> 204, where the matrix cores alone
+// take 120.  Tiles of 256 x 128, eight waves, gave no more: 109 to 98, 135 to 129, 155 to 212.
 //   12544 rows, five layers of 448 channels (59 GFLOP): the library's one product at a time left 49 workgroups for each
 //   (82 us, five of them, 412 us) and its column sums took 65 us more.
 #include <type_traits>
 
+#include "fragments.hpp"
 #include "linear.hpp"
 #include "mfma.hpp"
 
 namespace dcn {
 namespace {
 
-template <typename Tag> constexpr int kRowsOf = 128 / Tag::kBytes;      // rows of a slice
+template <typename Tag, int W> constexpr int kRowsOf = 8192 / (W * Tag::kBytes);      // rows of a slice
+constexpr int kGradBuffers = 3;
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ u32x2 read_turned(const char *lds) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)lds));
+// Reads of LDS past the compiler, as in fragments.hpp: between them and fragments_arrived nothing may use the registers.
+template <int OFFSET>
+__device__ __forceinline__ u32x2 read_turned(uint32_t at) {
+  u32x2 v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFFSET));
+  return v;
+}
+template <int OFFSET>
+__device__ __forceinline__ float read_word(uint32_t at) {
+  float v;
+  asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFFSET));
+  return v;
 }
 
 // Sixteen columns of a row - 32 bytes, or 64 of fp32 - are a unit, stored at unit ^ swizzle(row).
@@ -33,15 +50,39 @@ __device__ __forceinline__ int unit_swizzle(int row) {
   else return WIDTH == 128 ? (row & 3) | ((row >> 1) & 4) : ((row >> 1) & 1) | ((row >> 2) & 2);
 }
 
+template <int STEP_BYTES, int F, int... U, int STEPS>
+__device__ __forceinline__ void read_words(float (&v)[STEPS][F], const uint32_t (&low)[F], uint32_t base, std::integer_sequence<int, U...>) {
+  auto one = [&](auto u) {
+    constexpr int kStep = decltype(u)::value;
+#pragma unroll
+    for (int i = 0; i < F; ++i) v[kStep][i] = read_word<kStep * STEP_BYTES>(base + low[i]);
+  };
+  (one(std::integral_constant<int, U>{}), ...);
+}
+// A lane's eight values of a step are two reads, four rows apart.
+template <int ROW_BYTES, int F, int... U, int STEPS>
+__device__ __forceinline__ void read_halves(u32x2 (&v)[STEPS][2 * F], const uint32_t (&low)[F], uint32_t base, std::integer_sequence<int, U...>) {
+  auto one = [&](auto u) {
+    constexpr int kStep = decltype(u)::value;
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      v[kStep][2 * i] = read_turned<kStep * 32 * ROW_BYTES>(base + low[i]);
+      v[kStep][2 * i + 1] = read_turned<(kStep * 32 + 4) * ROW_BYTES>(base + low[i]);
+    }
+  };
+  (one(std::integral_constant<int, U>{}), ...);
+}
+
 template <typename Tag, int W>
 __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGradLaunch p) {
   static_assert(W == 64 || W == 128, "tile side");
-  constexpr int kBytes = Tag::kBytes, kRows = kRowsOf<Tag>, kRowBytes = W * kBytes, kUnit = 16 * kBytes;
+  constexpr int kBytes = Tag::kBytes, kRows = kRowsOf<Tag, W>, kRowBytes = W * kBytes, kUnit = 16 * kBytes, kPart = kRows * kRowBytes;
   constexpr int F = W / 2 / 16;                                 // a wave takes W/2 x W/2
   constexpr int kRowsPerLoad = 64 * 16 / kRowBytes, kLoads = kRows / kRowsPerLoad / 4;
-  __shared__ __align__(16) char lds[2][2][kRows * kRowBytes];   // [buffer][grad_out, in]
+  __shared__ __align__(16) char lds[kGradBuffers][2][kPart];    // grad_out, in
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int split = blockIdx.x % p.splits, tile = blockIdx.x / p.splits;
+  const int tiles = gridDim.x / p.splits;
+  const int id = xcd_contiguous_block(blockIdx.x, gridDim.x), split = id / tiles, tile = id % tiles;
   int which = 0;
   while (which + 1 < p.count && tile >= p.tile_end[which]) ++which;
   const WeightGradProblem &q = p.p[which];
@@ -52,7 +93,7 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
 
   // a wave's load covers kRowsPerLoad rows; a lane's 16 bytes go to position lane, which holds a unit's piece of the row
   const int load_row = lane * 16 / kRowBytes, load_chunk = lane % (kRowBytes / 16);
-  auto stage = [&](long long row0, char (&buf)[2][kRows * kRowBytes]) {
+  auto stage = [&](long long row0, char (&buf)[2][kPart]) {
     const int live = (int)max(0ll, min((long long)kRows, row_end - row0));
     const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.n * kBytes, (uint32_t)live * q.n * kBytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char *>(q.in) + (size_t)row0 * q.k * kBytes, (uint32_t)live * q.k * kBytes);
@@ -66,27 +107,17 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
     }
   };
 
-  // Fragments of a slice: for 16-bit types two steps of 32 rows, a lane's eight values by two turned reads; for fp32 eight
-  // steps of four rows, a lane's value as it lies.
+  // Fragments of a slice: for 16-bit types steps of 32 rows, for fp32 of four, a lane's value as it lies.  A fragment's unit is
+  // the wave's first one + i, under the swizzle.
   typedef typename std::conditional<kBytes == 2, u32x4, float>::type frag_t;
-  constexpr int kSteps = kBytes == 2 ? 2 : kRows / 4;
+  constexpr int kSteps = kBytes == 2 ? kRows / 32 : kRows / 4;
   const int wn = wave >> 1, wk = wave & 1, kb = lane >> 4, i16 = lane & 15;
-  const int frag_row = kBytes == 2 ? kb * 8 + (i16 >> 2) : kb, f = unit_swizzle<Tag, W>(frag_row);
-  const int in_unit = kBytes == 2 ? (i16 & 3) * 8 : i16 * 4;
-  int at_n[F], at_k[F];
+  const int frag_row = kBytes == 2 ? kb * 8 + (i16 >> 2) : kb, in_unit = kBytes == 2 ? (i16 & 3) * 8 : i16 * 4, f = unit_swizzle<Tag, W>(frag_row);
+  uint32_t low[F];
 #pragma unroll
-  for (int i = 0; i < F; ++i) {
-    at_n[i] = frag_row * kRowBytes + ((wn * F + i) ^ f) * kUnit + in_unit;
-    at_k[i] = frag_row * kRowBytes + ((wk * F + i) ^ f) * kUnit + in_unit;
-  }
-  auto fragment = [&](const char *base, int at, int s) -> frag_t {
-    if constexpr (kBytes == 2) {
-      const u32x2 lo = read_turned(base + at + s * 32 * kRowBytes), hi = read_turned(base + at + (s * 32 + 4) * kRowBytes);
-      return u32x4{lo.x, lo.y, hi.x, hi.y};
-    } else {
-      return *reinterpret_cast<const float *>(base + at + s * 4 * kRowBytes);
-    }
-  };
+  for (int i = 0; i < F; ++i) low[i] = (i ^ (f & (F - 1))) * kUnit + in_unit;
+  const uint32_t at_n = lds_address(lds) + frag_row * kRowBytes + ((wn * F) ^ (f & ~(F - 1))) * kUnit;
+  const uint32_t at_k = lds_address(lds) + kPart + frag_row * kRowBytes + ((wk * F) ^ (f & ~(F - 1))) * kUnit;
   auto multiply = [](frag_t a, frag_t b, f32x4 c) {
     if constexpr (kBytes == 2) return mfma_64_bytes<Tag>(a, b, c);
     else return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -100,42 +131,74 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   }
   const bool with_bias = q.grad_bias != nullptr && k0 == 0 && wk == 0;
 
-  f32x4 acc[F][F], bias[F];
+  f32x4 acc[F][F];
+  float bias[F], group[F];
 #pragma unroll
   for (int i = 0; i < F; ++i) {
-    bias[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bias[i] = group[i] = 0.f;
 #pragma unroll
     for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  if (row_begin < row_end) stage(row_begin, lds[0]);
+  const int slices = (int)((max(row_end - row_begin, 0ll) + kRows - 1) / kRows);
+#pragma unroll
+  for (int s = 0; s < kGradBuffers - 1; ++s)
+    if (s < slices) stage(row_begin + s * kRows, lds[s]);
+  // the bias by groups of rows: one running sum over a split's rows was three times as far from 64 bits as the framework's sum
+  constexpr int kGroup = (kBytes == 2 ? 64 : 32) / kRows;      // slices
   int cur = 0;
-  for (long long row0 = row_begin; row0 < row_end; row0 += kRows, cur ^= 1) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+  for (int s = 0; s < slices; ++s) {
+    wait_behind<kGradBuffers - 2, 2 * kLoads, 2 * kLoads>(slices - 1 - s, false);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t in_n = at_n + (uint32_t)(cur * 2 * kPart), in_k = at_k + (uint32_t)(cur * 2 * kPart);
+    auto stage_ahead = [&] {
+      if (s + kGradBuffers - 1 < slices) stage(row_begin + (long long)(s + kGradBuffers - 1) * kRows, lds[cur == 0 ? kGradBuffers - 1 : cur - 1]);
+    };
     frag_t fn[kSteps][F], fk[kSteps][F];
+    constexpr auto steps = std::make_integer_sequence<int, kSteps>{};
+    if constexpr (kBytes == 2) {
+      u32x2 half_n[kSteps][2 * F], half_k[kSteps][2 * F];
+      read_halves<kRowBytes>(half_n, low, in_n, steps);
+      read_halves<kRowBytes>(half_k, low, in_k, steps);
+      stage_ahead();
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s)
+      for (int u = 0; u < kSteps; ++u) {
+        fragments_arrived(half_n[u]);
+        fragments_arrived(half_k[u]);
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+          fn[u][i] = u32x4{half_n[u][2 * i].x, half_n[u][2 * i].y, half_n[u][2 * i + 1].x, half_n[u][2 * i + 1].y};
+          fk[u][i] = u32x4{half_k[u][2 * i].x, half_k[u][2 * i].y, half_k[u][2 * i + 1].x, half_k[u][2 * i + 1].y};
+        }
+      }
+    } else {
+      read_words<4 * kRowBytes>(fn, low, in_n, steps);
+      read_words<4 * kRowBytes>(fk, low, in_k, steps);
+      stage_ahead();
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) {
+        fragments_arrived(fn[u]);
+        fragments_arrived(fk[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u)
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = multiply(fk[u][j], fn[u][i], acc[i][j]);
+    if (with_bias) {
+      const bool closes = (s + 1) % kGroup == 0 || s + 1 == slices;
 #pragma unroll
       for (int i = 0; i < F; ++i) {
-        fn[s][i] = fragment(lds[cur][0], at_n[i], s);
-        fk[s][i] = fragment(lds[cur][1], at_k[i], s);
+        f32x4 sum = {group[i], 0.f, 0.f, 0.f};      // every row of this result is the same sum: the first is kept
+#pragma unroll
+        for (int u = 0; u < kSteps; ++u) sum = multiply(ones, fn[u][i], sum);
+        group[i] = closes ? 0.f : sum.x;
+        if (closes) bias[i] += sum.x;
       }
-    if (row0 + kRows < row_end) stage(row0 + kRows, lds[cur ^ 1]);
-    // the bias by slices: one running sum over a split's rows was three times as far from 64 bits as the framework's sum
-    f32x4 slice[F];
-#pragma unroll
-    for (int i = 0; i < F; ++i) slice[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-      for (int i = 0; i < F; ++i) {
-#pragma unroll
-        for (int j = 0; j < F; ++j) acc[i][j] = multiply(fk[s][j], fn[s][i], acc[i][j]);
-        if (with_bias) slice[i] = multiply(ones, fn[s][i], slice[i]);
-      }
-    if (with_bias)
-#pragma unroll
-      for (int i = 0; i < F; ++i) bias[i] += slice[i];
+    }
+    cur = cur == kGradBuffers - 1 ? 0 : cur + 1;
   }
   // results: rows of the fragment are the depth, so a lane stores four consecutive k of one n
   float *grad_w = q.grad_w + (size_t)split * p.split_stride, *grad_b = q.grad_bias + (size_t)split * p.split_stride;
@@ -143,7 +206,7 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   for (int i = 0; i < F; ++i) {
     const int n = n0 + (wn * F + i) * 16 + i16;
     if (n >= q.n) continue;
-    if (with_bias && kb == 0) grad_b[n] = bias[i].x;
+    if (with_bias && kb == 0) grad_b[n] = bias[i];
 #pragma unroll
     for (int j = 0; j < F; ++j) {
       const int k = k0 + (wk * F + j) * 16 + kb * 4;
@@ -297,43 +360,48 @@ __global__ void __launch_bounds__(256) narrow_rows_kernel(const void *src, u32x4
 }
 
 template <typename Tag, int W>
-hipError_t launch_grad_t(const WeightGradLaunch &p, hipStream_t stream) {
-  hipLaunchKernelGGL((linear_weight_grad_kernel<Tag, W>), dim3((unsigned)(p.tile_end[p.count - 1] * p.splits)), dim3(256), 0, stream, p);
+hipError_t launch_grad_t(WeightGradLaunch p, hipStream_t stream) {
+  constexpr int kRows = kRowsOf<Tag, W>;
+  p.rows_per_split = ((p.rows + p.splits - 1) / p.splits + kRows - 1) / kRows * kRows;
+  int end = 0;
+  for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + W - 1) / W) * ((p.p[i].k + W - 1) / W);
+  hipLaunchKernelGGL((linear_weight_grad_kernel<Tag, W>), dim3((unsigned)(end * p.splits)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
 }  // namespace
 
-// Tile and split.  A split is a power of two: consecutive workgroups go to the eight XCDs in turn, and the tiles that read
-// the same rows then share an L2 (12544 rows, 256 channels: 22 splits 67 us, 16 splits 53).  Measured over five layers of C
-// channels, us, 128 / 64 wide tiles at their best split: 12544 x 448 127 / 119, 12544 x 256 48 / 42, 50176 x 128 50 / 44,
-// 50176 x 224 151 / 185, 200704 x 112 169 / 238, 200704 x 64 106 / 84 - the wide tile is for many rows, where it reads its
-// operands half as often, unless most of it is padding.  Best splits: about 3136 rows each for the small tile (42, 44, 84,
-// 119 us above; 2 to 4 times as many cost 15 to 30 % more), about 400 workgroups for the wide one.
+// Tile and split.  Three workgroups live on a CU: splits, a power of two, double while the chip's 768 places hold them and a split
+// keeps rows enough to be worth its partial sums - 1200 with the wide tile, 750 with the small one (25088 x 64: 784 rows each 17 us,
+// 392 20), 150 in fp32, which is slower by the row (600 rows, three products: one split 21 us, four 11).  A long sum in 32 bits
+// is cut all the same: most_rows.
+// The wide tile reads its operands half as often; the small one pads less and fills the chip sooner.  us, wide / small at the best
+// split: 12544 x 448 102 / 115, 3136 x 896 96 / 125, 50176 x 224 132 / 180, 200704 x 112 155 / 228, 40394 x 256 (four products)
+// 37 / 44; 50176 x 128 (384 wide workgroups) 46 / 46, 12544 x 256 (384) 43 / 41, 3136 x 512 (376) 45 / 39, 40394 x 256 (one
+// product, 128) 24 / 19; 50176 x 160, half of it padding, 98 / 98.  A last round that is nearly empty costs a whole one: 120000 x 256 in fp32, 896 wide
+// workgroups, 711 / 602.
 WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p) {
   auto tiles = [&](int w) {
     long long n = 0;
     for (int i = 0; i < p.count; ++i) n += (long long)((p.p[i].n + w - 1) / w) * ((p.p[i].k + w - 1) / w);
     return n;
   };
-  WeightGradPlan plan;
+  const bool fp32 = dtype == F32::kCode;
   const long long wide = tiles(128), small = tiles(64);
-  plan.tile = p.rows >= 32768 && wide * 4 * 5 <= small * 6 ? 128 : 64;
-  // fp32 is bound by the matrix cores: even shares of the chip count
-  if (dtype == F32::kCode) plan.tile = 64;
-  const double want = dtype == F32::kCode ? (double)p.rows / 1300 : plan.tile == 64 ? (double)p.rows / 3136 : std::min(400.0 / (double)wide, (double)p.rows / 1500);
-  plan.splits = 1;
-  while (plan.splits < 64 && want >= 1.5 * plan.splits) plan.splits *= 2;
-  return plan;
+  const long long most_rows = fp32 ? 1950 : wide <= 32 && p.rows >= 32768 ? 1600 : 4704;
+  auto splits = [&](long long count, long long least_rows) {
+    int s = 1;
+    while (s < 64 && (p.rows >= most_rows * s || (count * 2 * s <= 768 && p.rows >= least_rows * 2 * s))) s *= 2;
+    return s;
+  };
+  const int wide_splits = splits(wide, 1200);
+  const long long groups = wide * wide_splits, last_round = (groups - 1) % 768 + 1;
+  if (last_round >= 400 && wide * 8 <= small * 3) return {128, wide_splits};
+  return {64, splits(small, fp32 ? 150 : 750)};
 }
 
-hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &launch, int tile, hipStream_t stream) {
-  WeightGradLaunch p = launch;
-  const int slice = dtype == F32::kCode ? kRowsOf<F32> : kRowsOf<F16>;
-  p.rows_per_split = ((p.rows + p.splits - 1) / p.splits + slice - 1) / slice * slice;
-  int end = 0;
-  for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + tile - 1) / tile) * ((p.p[i].k + tile - 1) / tile);
-  if (dtype == F32::kCode) return launch_grad_t<F32, 64>(p, stream);
+hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &p, int tile, hipStream_t stream) {
+  if (dtype == F32::kCode) return tile == 128 ? launch_grad_t<F32, 128>(p, stream) : launch_grad_t<F32, 64>(p, stream);
   if (dtype == F16::kCode) return tile == 128 ? launch_grad_t<F16, 128>(p, stream) : launch_grad_t<F16, 64>(p, stream);
   return tile == 128 ? launch_grad_t<BF16, 128>(p, stream) : launch_grad_t<BF16, 64>(p, stream);
 }
