@@ -5,16 +5,16 @@
 // apart: slices of 8 KB of either operand come 16 bytes a lane straight into LDS as they lie in memory and ds_read_b64_tr_b16 turns
 // them on the way into registers (16 lanes read 4 rows x 16 columns; lane i gets column i).  A row's 32-byte units are stored at
 // unit ^ f(row), f taking each value once over the eight rows that half a wave reads, so those reads fall into different
-// banks.  The rows are split over workgroups until the chip is full, partial sums are fp32 and are added in split order by
+// banks.  The rows are split over workgroups until the chip is full, partial sums are fp32 and are added in a fixed order by
 // linear_grad_reduce_kernel: no atomics, the same bits every time.  The bias gradient is one more matrix instruction per
 // fragment, against a vector of ones.
 //   What bounds it is the operands' way into LDS (10 to 13 TB/s over the chip, most of it from L2), so the tile is as large as the
 // registers allow, and the latency of a slice: three buffers keep two slices under way behind the one that is multiplied, 48 KB,
 // three workgroups to a CU.  Two buffers, each waited for in full, were 64 KB with the 128-wide tile, two workgroups to a CU.
-// Sums included, us, before -> now, five layers of C channels, fp16: 12544 x 448 121 -> 103, 3136 x 896 119 -> 88, 50176 x 224 247 ->
-// 135, 200704 x 112 257 -> 155, 50176 x 128 72 -> 47, 25088 x 64 33 -> 17, 392 x 256 7.0 -> 6.4; 200704 x 64 87 -> 89 (its operands
-// alone are 69 at the rate of a copy).  The four products of 256 channels, 40394 rows, fp32: 231 -> 204, where the matrix cores alone
-// take 120.  Tiles of 256 x 128, eight waves, gave no more: 109 to 98, 135 to 129, 155 to 212.
+// Sums included, us, before -> now, five layers of C channels, fp16: 12544 x 448 122 -> 102, 3136 x 896 119 -> 90, 50176 x 224 246 ->
+// 120, 200704 x 112 256 -> 146, 50176 x 128 73 -> 47, 25088 x 64 33 -> 16, 392 x 256 7.0 -> 6.4; 200704 x 64 87 -> 88 (its operands
+// alone are 69 at the rate of a copy).  The four products of 256 channels, 40394 rows, fp32: 232 -> 187, where the matrix cores alone
+// take 120.  Tiles of 256 x 128, eight waves, gave no more: 102 to 98, 126 to 129, 145 to 212.
 //   12544 rows, five layers of 448 channels (59 GFLOP): the library's one product at a time left 49 workgroups for each
 //   (82 us, five of them, 412 us) and its column sums took 65 us more.
 #include <type_traits>
@@ -223,15 +223,25 @@ __global__ void __launch_bounds__(256) linear_grad_reduce_kernel(const WeightGra
   for (int i = blockIdx.x * 256 + threadIdx.x; i * 4 < s.count; i += stride) {
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     const float *src = p.partial + s.offset + (size_t)i * 4;
+    // sixteen splits under way, added in pairs: closer to 64 bits than one after the other (the bias of 25088 x 64, 33 splits, 6.8e-8
+    // of its norm against 1.2e-7)
     int split = 0;
-    for (; split + 4 <= p.splits; split += 4) {
-      f32x4 v[4];
+    auto add = [&](auto at_once) {
+      constexpr int kAtOnce = decltype(at_once)::value;
+      for (; split + kAtOnce <= p.splits; split += kAtOnce) {
+        f32x4 v[kAtOnce];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const f32x4 *>(src + (size_t)(split + u) * p.split_stride);
+        for (int u = 0; u < kAtOnce; ++u) v[u] = *reinterpret_cast<const f32x4 *>(src + (size_t)(split + u) * p.split_stride);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sum += v[u];
-    }
-    for (; split < p.splits; ++split) sum += *reinterpret_cast<const f32x4 *>(src + (size_t)split * p.split_stride);
+        for (int step = 1; step < kAtOnce; step *= 2)
+#pragma unroll
+          for (int u = 0; u + step < kAtOnce; u += 2 * step) v[u] += v[u + step];
+        sum += v[0];
+      }
+    };
+    add(std::integral_constant<int, 16>{});
+    add(std::integral_constant<int, 4>{});
+    add(std::integral_constant<int, 1>{});
     if (i * 4 + 4 <= s.count) {
       *reinterpret_cast<f32x4 *>(s.grad + (size_t)i * 4) = sum;
     } else {
@@ -371,15 +381,16 @@ hipError_t launch_grad_t(WeightGradLaunch p, hipStream_t stream) {
 
 }  // namespace
 
-// Tile and split.  Three workgroups live on a CU: splits, a power of two, double while the chip's 768 places hold them and a split
-// keeps rows enough to be worth its partial sums - 1200 with the wide tile, 750 with the small one (25088 x 64: 784 rows each 17 us,
-// 392 20), 150 in fp32, which is slower by the row (600 rows, three products: one split 21 us, four 11).  A long sum in 32 bits
-// is cut all the same: most_rows.
-// The wide tile reads its operands half as often; the small one pads less and fills the chip sooner.  us, wide / small at the best
-// split: 12544 x 448 102 / 115, 3136 x 896 96 / 125, 50176 x 224 132 / 180, 200704 x 112 155 / 228, 40394 x 256 (four products)
-// 37 / 44; 50176 x 128 (384 wide workgroups) 46 / 46, 12544 x 256 (384) 43 / 41, 3136 x 512 (376) 45 / 39, 40394 x 256 (one
-// product, 128) 24 / 19; 50176 x 160, half of it padding, 98 / 98.  A last round that is nearly empty costs a whole one: 120000 x 256 in fp32, 896 wide
-// workgroups, 711 / 602.
+// Tile and split.  The chip's 256 CUs are to have the same work each: two workgroups, or three (the wide tile, 14 tiles in fp32,
+// 40394 rows: 36 splits 187 us, 54 188, 40 and 48 - some CUs get three, some two - 245 and 208; 12 tiles of 200704 rows in fp16: 42 splits
+// 144, 48 173).  A split keeps rows enough to be worth its partial sums: 1500 with the wide tile, 750 with the small one (25088 x
+// 64: 784 rows each 17 us, 392 20), 1000 and 150 in fp32, which is slower by the row (600 rows, three products: one split 21 us,
+// four 11).  `least`: a long sum in 32 bits is cut all the same.
+// The wide tile reads its operands half as often; the small one pads less and fills the chip sooner.  us, wide / small: 12544 x 448
+// 102 / 115, 3136 x 896 90 / 125, 50176 x 224 120 / 184, 200704 x 112 145 / 231, 50176 x 160 (half of it padding) 87 / 98, 40394 x 256
+// (four products) 38 / 41; 50176 x 128 (384 wide workgroups) 48 / 46, 12544 x 256 (384) 43 / 41, 3136 x 512 (376) 45 / 39, 40394 x
+// 256 (one product, 128) 24 / 19.  More workgroups than live at once end in a round that should not be nearly empty: 120000 x 256 in
+// fp32, 896 wide workgroups, 711 / 602.
 WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p) {
   auto tiles = [&](int w) {
     long long n = 0;
@@ -388,14 +399,18 @@ WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p) {
   };
   const bool fp32 = dtype == F32::kCode;
   const long long wide = tiles(128), small = tiles(64);
-  const long long most_rows = fp32 ? 1950 : wide <= 32 && p.rows >= 32768 ? 1600 : 4704;
+  const double want = fp32 ? (double)p.rows / 1300 : p.rows >= 32768 && wide * 20 <= small * 6 ? std::min(400.0 / (double)wide, (double)p.rows / 1500) : (double)p.rows / 3136;
+  int least = 1;
+  while (least < 64 && want >= 1.5 * least) least *= 2;
   auto splits = [&](long long count, long long least_rows) {
-    int s = 1;
-    while (s < 64 && (p.rows >= most_rows * s || (count * 2 * s <= 768 && p.rows >= least_rows * 2 * s))) s *= 2;
-    return s;
+    long long s = 512 / count;
+    if (s * count < 480) s = std::max(1ll, 768 / count);
+    s = std::clamp(std::min(s, p.rows / least_rows), 1ll, 64ll);
+    for (int per = 1; s < least; ++per) s = std::min(64ll, std::max(s, 256 * per / count));
+    return (int)s;
   };
-  const int wide_splits = splits(wide, 1200);
-  const long long groups = wide * wide_splits, last_round = (groups - 1) % 768 + 1;
+  const int wide_splits = splits(wide, fp32 ? 1000 : 1500);
+  const long long last_round = (wide * wide_splits - 1) % 768 + 1;
   if (last_round >= 400 && wide * 8 <= small * 3) return {128, wide_splits};
   return {64, splits(small, fp32 ? 150 : 750)};
 }

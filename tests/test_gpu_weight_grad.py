@@ -13,7 +13,7 @@ PIXELS = sum(h * w for h, w in LEVELS)
 
 
 # rows: one slice and its remainders, two and three of them, four splits (the last one short); as many as the features, and then all
-# products are one launch: the small tile with 32 splits (the last one empty), the wide one
+# products are one launch: the small tile with 54 splits (64 in fp32, the last ones empty), the wide one with 32 (36)
 @pytest.mark.parametrize("amp", [None, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
 @pytest.mark.parametrize("width,rows", [(64, 1), (64, 31), (64, 33), (128, 65), (256, 129), (256, 601), (64, PIXELS), (256, PIXELS)])
 def test_weight_gradients_match_fp64(width, rows, amp):
@@ -44,7 +44,7 @@ def test_weight_gradients_match_fp64(width, rows, amp):
     assert _rel(got_w, g.t() @ x) < tol and _rel(got_b, g.sum(0)) < 1e-6
 
 
-# 80, 160 and 448 channels: 128-wide tiles of 64, 16 and 4 splits
+# 80, 160 and 448 channels: 128-wide tiles of 51, 12 and 3 splits
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
 @pytest.mark.parametrize("channels,groups,size", [(80, 5, (5, 124, 124)), (160, 10, (1, 139, 139)), (448, 28, (3, 40, 41)), (64, 4, (1, 3, 11))])
 def test_layer_weight_gradients_in_wide_tiles_match_the_composition(channels, groups, size, dtype):
