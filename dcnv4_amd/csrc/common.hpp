@@ -138,6 +138,20 @@ __device__ __forceinline__ float sub_rn(float a, float b) {
   return a - b;
 }
 
+// An element of a 16-bit pair plus c, one instruction in fp16.
+template <typename Tag, int HI>
+__device__ __forceinline__ float plus_half(uint32_t pair, float c) {
+  if constexpr (Tag::kCode == F16::kCode) {
+    float r;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(c));
+    else asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(c));
+    return r;
+  } else {
+    return __builtin_bit_cast(float, HI ? pair & 0xffff0000u : pair << 16) + c;
+  }
+}
+__device__ __forceinline__ uint32_t lds_address(const void *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p; }
+
 // ---------------------------------------------------------------- bilinear tap
 // Corner order: (y0,x0) (y0,x0+1) (y0+1,x0) (y0+1,x0+1), as common.h:48-58.
 // `off` are byte offsets into the descriptor, kDropOffset for a corner outside the image

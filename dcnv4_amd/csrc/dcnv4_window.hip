@@ -9,12 +9,11 @@ namespace {
 
 template <typename Tag, int LPG, int UNITS>
 __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel(const DcnLaunch p) {
-  extern __shared__ u32x4 lds128[];
+  extern __shared__ __align__(32) u32x4 lds128[];      // window_corner turns a bit of the address
   constexpr int kGroups = UNITS / LPG, EPV = 16 / Tag::kBytes, kCell = UNITS * 32;
   typedef Pack<Tag, EPV> pack;
   char *lds = reinterpret_cast<char *>(lds128);
   const WindowTile t = window_tile<kGroups>(p, blockIdx.x, gridDim.x);
-  const WindowFrame<UNITS> frame(t);
 
   // lane -> (pixel of the tile, group of the workgroup, part of the group): a wave stays within one group
   constexpr int kPixels = kWindowThreads / UNITS, kPerGroup = kPixels * LPG;
@@ -35,25 +34,25 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
   const float x_base = sub_rn((float)(1 - p.pw + wo), p.offset_scale), y_base = sub_rn((float)(1 - p.ph + ho), p.offset_scale);
   auto position = [&](int own, int k, float &y, float &x, float &m) {
     float ox, oy;
-    rows.get(own, ox, oy, m);
     const int i = LPG == 1 ? k / 3 : exact_div(k, 1.f / 3.f), j = k - 3 * i;
-    x = add_rn(x_base, mul_rn(add_rn((float)i, ox), p.offset_scale));
-    y = add_rn(y_base, mul_rn(add_rn((float)j, oy), p.offset_scale));
+    rows.get(own, i, j, ox, oy, m);
+    x = add_rn(x_base, mul_rn(ox, p.offset_scale));
+    y = add_rn(y_base, mul_rn(oy, p.offset_scale));
   };
-  const int lane_bytes = (gl * LPG + part) * 32;
-  float acc[2][EPV];
+  const int half = lane_half<LPG>(), lane_bytes = (int)lds_address(lds) + (gl * LPG + part) * 32 + half;
+  const WindowFrame<UNITS> frame(t, LPG == 1 ? lane_bytes : 0);
+  float acc[2][EPV];      // of the lane's first half, then the other
 #pragma unroll
   for (int v = 0; v < 2; ++v)
 #pragma unroll
     for (int c = 0; c < EPV; ++c) acc[v][c] = 0.f;
   uint32_t far = 0;      // a bit for each point this lane prepares that is inside the image but outside the window
   auto gather = [&](int addr, const float (&w)[4]) {
-    const char *src = lds + addr;
     u32x4 raw[4][2];
 #pragma unroll
     for (int cn = 0; cn < 4; ++cn)
 #pragma unroll
-      for (int v = 0; v < 2; ++v) raw[cn][v] = *reinterpret_cast<const u32x4 *>(src + (cn & 1) * kCell + (cn >> 1) * frame.row_bytes + 16 * v);
+      for (int v = 0; v < 2; ++v) raw[cn][v] = window_corner<kCell>((uint32_t)addr, frame.row_bytes, cn, v);
 #pragma unroll
     for (int cn = 0; cn < 4; ++cn)
 #pragma unroll
@@ -71,7 +70,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
     float y, x, m;
     position(i, k, y, x, m);
     const WindowPoint pt = window_point<UNITS>(frame, y, x, m);
-    if (!__all(pt.ok)) {
+    if (__builtin_amdgcn_ballot_w64(!pt.ok) != 0) {
       const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
       far |= (uint32_t)(inside && !pt.ok) << k;
     }
@@ -80,7 +79,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
       if constexpr (J < LPG) {
         if (i * LPG + J < 9) {
           const float w[4] = {share<LPG, J>(pt.w[0]), share<LPG, J>(pt.w[1]), share<LPG, J>(pt.w[2]), share<LPG, J>(pt.w[3])};
-          gather(share<LPG, J>(pt.addr) + lane_bytes, w);
+          gather(LPG == 1 ? pt.addr : share<LPG, J>(pt.addr) + lane_bytes, w);
         }
       }
     };
@@ -117,7 +116,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
           float f[EPV];
-          pack::decode(buffer_load<16>(value, tp.off[cn] + 16u * v), f);      // a dropped corner stays out of range
+          pack::decode(buffer_load<16>(value, tp.off[cn] + (uint32_t)(half ^ 16 * v)), f);      // a dropped corner stays out of range
           const float w = f3[2] * tp.w[cn];
 #pragma unroll
           for (int c = 0; c < EPV; ++c) acc[v][c] = fmaf(w, f[c], acc[v][c]);
@@ -126,7 +125,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
   }
   char *dst = static_cast<char *>(p.out) + (pixel * (size_t)(p.G * p.D) + (size_t)g * p.D) * Tag::kBytes + part * 32;
 #pragma unroll
-  for (int v = 0; v < 2; ++v) *reinterpret_cast<u32x4 *>(dst + 16 * v) = pack::encode(acc[v]);
+  for (int v = 0; v < 2; ++v) *reinterpret_cast<u32x4 *>(dst + (half ^ 16 * v)) = pack::encode(acc[v]);
 }
 
 // ------------------------------------------------------------------------------- backward
@@ -141,14 +140,13 @@ constexpr int kBeyondMost = 512;
 // 2 % (64x56x56, 4 groups of 16, fp16: 61.9 -> 63.5 us).
 template <typename Tag, int LPG, int UNITS, bool LISTS>
 __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_window_kernel(const DcnLaunch p) {
-  extern __shared__ u32x4 lds128[];
+  extern __shared__ __align__(32) u32x4 lds128[];      // window_corner turns a bit of the address
   __shared__ uint32_t s_reach, s_beyond_count;
   __shared__ uint16_t s_beyond[LISTS ? kBeyondMost : 1];      // points beyond the near reach: lane | point << 8
   typedef typename RawWord<Tag::kBytes>::type elem_t;
   constexpr int kGroups = UNITS / LPG, kCell = UNITS * 32;
   char *lds = reinterpret_cast<char *>(lds128);
   const WindowTile t = window_tile<kGroups>(p, blockIdx.x, gridDim.x);
-  const WindowFrame<UNITS> frame(t);
   if (threadIdx.x == 0) s_reach = s_beyond_count = 0u;
 
   constexpr int kPixels = kWindowThreads / UNITS, kPerGroup = kPixels * LPG;
@@ -162,10 +160,11 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
   const void *row = static_cast<const char *>(p.offset_mask) + (pixel * p.P_pad + (size_t)g * 27) * Tag::kBytes;
   PointRows<Tag, LPG> rows;
   rows.load(row, part);
-  u32x4 go_raw[2];
+  const int half = lane_half<LPG>();
+  u32x4 go_raw[2];        // the lane's first half, then the other
   const char *go_src = static_cast<const char *>(p.grad_out) + (pixel * (size_t)(p.G * p.D) + (size_t)g * p.D) * Tag::kBytes + part * 32;
 #pragma unroll
-  for (int v = 0; v < 2; ++v) go_raw[v] = *reinterpret_cast<const u32x4 *>(go_src + 16 * v);
+  for (int v = 0; v < 2; ++v) go_raw[v] = *reinterpret_cast<const u32x4 *>(go_src + (half ^ 16 * v));
   stage_window<Tag, UNITS>(p, t, lds);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -173,10 +172,12 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
   const int p0x = 1 - p.pw + wo, p0y = 1 - p.ph + ho;      // reference point
   const float p0xf = (float)p0x, p0yf = (float)p0y;
   const float x_base = sub_rn(p0xf, p.offset_scale), y_base = sub_rn(p0yf, p.offset_scale);
-  auto at = [&](int k, float ox, float oy, float &y, float &x) {
+  auto position = [&](int own, int k, float &y, float &x, float &m) {
+    float ox, oy;
     const int i = LPG == 1 ? k / 3 : exact_div(k, 1.f / 3.f), j = k - 3 * i;
-    x = add_rn(x_base, mul_rn(add_rn((float)i, ox), p.offset_scale));
-    y = add_rn(y_base, mul_rn(add_rn((float)j, oy), p.offset_scale));
+    rows.get(own, i, j, ox, oy, m);
+    x = add_rn(x_base, mul_rn(ox, p.offset_scale));
+    y = add_rn(y_base, mul_rn(oy, p.offset_scale));
   };
   // corner . grad_out over this lane's channels
   auto dots = [&](auto fetch, float (&d)[4]) {
@@ -214,7 +215,8 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
     r[2] = hy * hx * d[0] + hy * lx * d[1] + ly * hx * d[2] + ly * lx * d[3];
   };
 
-  const int lane_bytes = (gl * LPG + part) * 32;
+  const int lane_bytes = (int)lds_address(lds) + (gl * LPG + part) * 32 + half;
+  const WindowFrame<UNITS> frame(t, LPG == 1 ? lane_bytes : 0);
   constexpr int kOwn = PointRows<Tag, LPG>::kOwn;
   float result[kOwn][3];
   uint32_t far = 0, beyond = 0;      // a bit for each point that this lane prepares: served from memory, beyond the near reach
@@ -223,14 +225,13 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
 #pragma unroll
     for (int i = 0; i < kOwn; ++i) {
       const int k = LPG == 1 ? i : min(part + i * LPG, 8);
-      float ox, oy, y, x, m;
-      rows.get(i, ox, oy, m);
-      at(k, ox, oy, y, x);
+      float y, x, m;
+      position(i, k, y, x, m);
       const WindowPoint pt = window_point<UNITS>(frame, y, x, 1.f);
       // Chebyshev distance of the point from its reference point: its ceiling is how far the weighted corners of its 2x2 block
       // lie from it at most.  Points beyond the cap - which exceeds what a window covers - are folded where they are served.
       bool counts = pt.ok;
-      if (!__all(pt.ok)) {
+      if (__builtin_amdgcn_ballot_w64(!pt.ok) != 0) {
         const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
         far |= (uint32_t)(inside && !pt.ok) << k;
         counts = inside;
@@ -244,9 +245,9 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
         constexpr int J = decltype(jj)::value;
         if constexpr (J < LPG) {
           if (i * LPG + J < 9) {
-            const char *src = lds + share<LPG, J>(pt.addr) + lane_bytes;
+            const int addr = LPG == 1 ? pt.addr : share<LPG, J>(pt.addr) + lane_bytes;
             float dj[4];
-            dots([&](int cn, int v) { return *reinterpret_cast<const u32x4 *>(src + (cn & 1) * kCell + (cn >> 1) * frame.row_bytes + 16 * v); }, dj);
+            dots([&](int cn, int v) { return window_corner<kCell>((uint32_t)addr, frame.row_bytes, cn, v); }, dj);
 #pragma unroll
             for (int cn = 0; cn < 4; ++cn) d[cn] = LPG == 1 || part == J ? dj[cn] : d[cn];
           }
@@ -337,7 +338,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
           if (!LISTS) dcnv4_fold_far_point(p, t.b, g, tp.y0, tp.x0, p0y, p0x);
           else if (part == 0) dcnv4_far_tiles(p, tp.y0, tp.x0, p0y, p0x, [&](int ty, int tx, int away) { dcnv4_widen_visit(p, t.b, ty, tx, g / p.ng_chunk, away); });
         }
-        dots([&](int cn, int v) { return buffer_load<16>(value, tp.off[cn] + 16u * v); }, d);
+        dots([&](int cn, int v) { return buffer_load<16>(value, tp.off[cn] + (uint32_t)(half ^ 16 * v)); }, d);
         gradients(d, tp.ly, tp.lx, f3[2], r);
         if (part == k % LPG) put(k, r);
       }

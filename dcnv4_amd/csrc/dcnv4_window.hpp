@@ -10,9 +10,11 @@
 //     through LDS;
 //   * the range test of a point is one against the window, which is clipped to the image: the reference's own test
 //     (dcnv4_im2col_cuda.cuh:227) only runs in a wave that has a point outside.
-// What bounds them is LDS reads (128 bytes a point and lane) and the sums, about evenly.  64x56x56, 4 groups of 16, share of the time
-// in which the vector units / the LDS are busy (two thirds of the latter are bank conflicts): forward fp16 75 / 63 %, fp32 63 /
-// 70 %, grad_offset_mask fp32 72 / 51 %.
+//   * of its 32 bytes every other lane reads the second half first, or a read's lanes share every other of the LDS's slots
+//     (128x56x56, 7 groups of 16 in fp16: 36 million cycles of the LDS, 48 with one order for all), and the address of a point takes
+//     four instructions: offsets and window come with what all addresses of a lane start from.
+// What bounds them is the sums and, less, the LDS reads (128 bytes a point and lane), behind the latency of the window: vector units
+// / LDS busy, 128x56x56 in fp16, 73 / 46 % of the time.
 // Measured, us, offsets within +-3, tiled -> window kernel (forward | grad_offset_mask):
 //   64x56x56, 4 groups of 16    fp16   48 -> 32 |  62 -> 56     fp32   66 -> 52
 //   128x56x56, 7 groups of 16   fp16  174 -> 130
@@ -20,6 +22,8 @@
 //   64x56x56, 4 groups of 32    fp16  103 -> 59                 fp32  150 -> 84
 //   64x28x28, 4 groups of 64    fp16   40 -> 27 |  61 -> 35
 //   64x7x7, 32 groups of 16     fp16   12 ->  8
+// and without -> with the halves' order and the shorter address: 64x14x14, 16 groups, fp32 forward 18.0 -> 16.8; 2x200x334, 10 groups,
+// bf16, offsets with tails, 84 -> 80 | 123 -> 120; 64x56x56, 4 groups, fp16 35.1 -> 34.4 | 62.2 -> 60.5.
 #pragma once
 #include "common.hpp"
 #include "launch.hpp"
@@ -84,28 +88,41 @@ __device__ __forceinline__ void stage_window(const DcnLaunch &p, const WindowTil
   }
 }
 
+// Which 16 bytes of its 32 a lane reads first: every other (pixel, group) the second.  All cells start at a multiple of 32 bytes, and
+// with one order for all a read's sixteen lanes had only every other of the sixteen slots of 256 bytes to fall into.
+template <int LPG>
+__device__ __forceinline__ int lane_half() { return (threadIdx.x / LPG & 1) * 16; }
+
+// The v-th half of corner cn, the first of which lies at addr.
+template <int CELL>
+__device__ __forceinline__ u32x4 window_corner(uint32_t addr, int row_bytes, int cn, int v) {
+  return *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)((addr ^ 16u * v) + (uint32_t)((cn >> 1) * row_bytes + (cn & 1) * CELL));
+}
+
 // What a sampling point needs of the window, the same for every lane: bounds of the points it serves, and LDS strides.
 template <int UNITS>
 struct WindowFrame {
   static constexpr int kCell = UNITS * 32;
   float y_lo, y_hi, x_lo, x_hi;
   int row_bytes, origin, zeros;
-  __device__ __forceinline__ explicit WindowFrame(const WindowTile &t) {
+  // bytes: what every address starts from
+  __device__ __forceinline__ WindowFrame(const WindowTile &t, int bytes) {
     // from the window's first row to before its last; a window that starts at the ring excludes -1 itself
     y_lo = t.wy0 < 0 ? -0.99999994f : (float)t.wy0;
     x_lo = t.wx0 < 0 ? -0.99999994f : (float)t.wx0;
     y_hi = (float)(t.wy0 + t.wh - 1);
     x_hi = (float)(t.wx0 + t.ww - 1);
     row_bytes = t.ww * kCell;
-    origin = -(t.wy0 * row_bytes + t.wx0 * kCell);
-    zeros = t.wh * row_bytes;
+    origin = bytes - (t.wy0 * row_bytes + t.wx0 * kCell);
+    zeros = bytes + t.wh * row_bytes;
+    asm("" : "+v"(origin), "+v"(zeros));      // left alone the compiler adds the parts up again for every point
   }
 };
 
 struct WindowPoint {
   float w[4];        // corner weights times the modulation
   float ly, lx;
-  int addr;          // of corner 0, without the lane's own bytes
+  int addr;          // of corner 0
   bool ok;
 };
 
@@ -117,10 +134,12 @@ __device__ __forceinline__ WindowPoint window_point(const WindowFrame<UNITS> &f,
   x = r.ok ? x : 0.f;
   const float fy = floorf(y), fx = floorf(x);
   r.ly = y - fy; r.lx = x - fx;
-  const int at = __mul24((int)fx, WindowFrame<UNITS>::kCell) + (__mul24((int)fy, f.row_bytes) + f.origin);
+  int at = (int)fx * WindowFrame<UNITS>::kCell + (__mul24((int)fy, f.row_bytes) + f.origin);
+  asm("" : "+v"(at));      // or else computed in a branch of its own
   r.addr = r.ok ? at : f.zeros;
-  const float hx = 1.f - r.lx, upper = m * (1.f - r.ly), lower = m * r.ly;
-  r.w[0] = upper * hx; r.w[1] = upper * r.lx; r.w[2] = lower * hx; r.w[3] = lower * r.lx;
+  // m (1 - ly) as m - m ly, rounded once, and so on: no 1 - ly, no 1 - lx
+  const float upper = fmaf(-m, r.ly, m), lower = m * r.ly;
+  r.w[0] = fmaf(-upper, r.lx, upper); r.w[1] = upper * r.lx; r.w[2] = fmaf(-lower, r.lx, lower); r.w[3] = lower * r.lx;
   return r;
 }
 
@@ -164,12 +183,20 @@ struct PointRows {
       for (int i = 0; i < kOwn; ++i) point_of_row<Tag>(row, min(part + i * LPG, 8), own[i]);
     }
   }
-  // x offset, y offset, modulation of the lane's i-th point
-  __device__ __forceinline__ void get(int i, float &x, float &y, float &m) const {
-    if constexpr (LPG == 1) {
-      x = element(2 * i); y = element(2 * i + 1); m = element(18 + i);
+  // i + x offset, j + y offset and modulation of the lane's n-th point, tap (i, j)
+  __device__ __forceinline__ void get(int n, int i, int j, float &x, float &y, float &m) const {
+    if constexpr (LPG == 1 && Tag::kCode == F16::kCode) {      // conversion and sum in one instruction
+      x = i == 0 ? element(2 * n) : plus_half<Tag, 0>(raw[n], (float)i);
+      y = j == 0 ? element(2 * n + 1) : plus_half<Tag, 1>(raw[n], (float)j);
+      m = element(18 + n);
+    } else if constexpr (LPG == 1) {
+      x = add_rn((float)i, element(2 * n));
+      y = add_rn((float)j, element(2 * n + 1));
+      m = element(18 + n);
     } else {
-      x = own[i][0]; y = own[i][1]; m = own[i][2];
+      x = add_rn((float)i, own[n][0]);
+      y = add_rn((float)j, own[n][1]);
+      m = own[n][2];
     }
   }
 

@@ -14,7 +14,6 @@ namespace dcn {
 // The reads are written out because a read in C++ waits for every load into LDS that is under way - the compiler cannot tell
 // the buffers apart - and the point of several buffers is that it does not.  Between read_fragments and fragments_arrived nothing
 // may use the registers.
-__device__ __forceinline__ uint32_t lds_address(const void *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p; }
 __device__ __forceinline__ uint32_t fragment_offset(int r16, int kb) { return (uint32_t)(r16 * 64 + (kb ^ ((r16 >> 2) & 3)) * 16); }
 
 template <int OFFSET>
@@ -73,18 +72,6 @@ __device__ __forceinline__ f32x4 load4(const char *vector, int element) {
   return f32x4{f[0], f[1], f[2], f[3]};
 }
 
-// An element of a pair of them plus c, one instruction in fp16.
-template <typename Tag, int HI>
-__device__ __forceinline__ float plus_half(uint32_t pair, float c) {
-  if constexpr (Tag::kCode == F16::kCode) {
-    float r;
-    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(c));
-    else asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(c));
-    return r;
-  } else {
-    return __builtin_bit_cast(float, HI ? pair & 0xffff0000u : pair << 16) + c;
-  }
-}
 template <typename Tag>
 __device__ __forceinline__ f32x4 plus_halves(u32x2 v, f32x4 c) {
   const uint32_t lo = v.x, hi = v.y;
