@@ -5,7 +5,7 @@
 //    64 bytes into three buffers of 24 KB, two slices under way while the matrix cores work on a third, and a CU holds two
 //    workgroups.  What an operand costs on its way into LDS bounds these products as much as the matrix cores do - the matrix
 //    instructions alone, with their reads of LDS, take half the time (25088 x 1792 x 448: 36 of 68 us, the loads alone 43, the
-//    epilogue with the GELU 42) - and a tile of twice the rows brings a quarter less.
+//    epilogue with a GELU of six more issue slots 42) - and a tile of twice the rows brings a quarter less.
 //  linear_tiled_kernel: many rows.  A workgroup of four waves owns BM rows x BN features; both operands come in slices of
 //    128 bytes along the depth, 16 bytes a lane, straight into LDS (two buffers, one barrier a slice: the next slice's loads are in
 //    flight while the matrix cores work on this one).  The 16-byte vectors of a row are stored at position

@@ -6,12 +6,12 @@
 // The matrix instruction leaves a lane four rows of its result; with w1's features dealt to the rows of two instructions so that
 // these are eight consecutive features, they are the lane's eight values of the depth of the second product: the activations
 // never leave the lane.  Both weights' next 32 features come straight into LDS meanwhile, shared by the four waves.
-// What bounds it then is the GELU (seventeen instructions an element; with 112 channels the vector units are busy 59 % of the time,
-// the matrix cores 22) and, with 224 channels, the two waves that its registers leave room for (34 and 21 %).
+// What bounds it then is the GELU (seventeen issue slots an element, 23 in bf16; with 112 channels and 23 the vector units were busy
+// 59 % of the time, the matrix cores 22) and, with 224 channels, the two waves that its registers leave room for (34 and 21 %).
 // A layer normalisation behind the MLP (NORM: residual + gamma * norm(mlp)) takes the sums of a row from the registers of the four
-// lanes that hold it.
-// Measured, fp16, two kernels -> this one: 401408 x 112 336 -> 160 us, 100352 x 224 203 -> 140 (145 and 134 with a GELU of thirteen
-// instructions, which was less exact than the fp32 function).
+// lanes that hold it: two kernels -> one, us, 401408 x 112 163 + 46 -> 165 to 185, 100352 x 224 142 + 23 -> 153 to 168.
+// Measured, fp16, two kernels -> this one: 401408 x 112 336 -> 160 us, 100352 x 224 203 -> 140, both with the GELU of 23 slots (145 and 134 with one of
+// thirteen instructions, which was less exact than the fp32 function).
 #include <algorithm>
 
 #include "fragments.hpp"
