@@ -406,7 +406,7 @@ WeightGradPlan plan_weight_grad(int dtype, const WeightGradLaunch &p) {
     long long s = 512 / count;
     if (s * count < 480) s = std::max(1ll, 768 / count);
     s = std::clamp(std::min(s, p.rows / least_rows), 1ll, 64ll);
-    for (int per = 1; s < least; ++per) s = std::min(64ll, std::max(s, 256 * per / count));
+    if (s < least) s = std::min(64ll, 256 * ((least * count + 255) / 256) / count);      // the next even share
     return (int)s;
   };
   const int wide_splits = splits(wide, fp32 ? 1000 : 1500);
