@@ -8,7 +8,7 @@ namespace dcn {
 namespace {
 
 template <typename Tag, int LPG, int UNITS>
-__global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel(const DcnLaunch p) {
+__global__ void __launch_bounds__(kWindowThreads, 5) dcnv4_forward_window_kernel(const DcnLaunch p) {
   extern __shared__ __align__(32) u32x4 lds128[];      // window_corner turns a bit of the address
   constexpr int kGroups = UNITS / LPG, EPV = 16 / Tag::kBytes, kCell = UNITS * 32;
   typedef Pack<Tag, EPV> pack;
@@ -102,11 +102,14 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_forward_window_kernel
     const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
     const uint32_t pix_bytes = (uint32_t)(p.G * p.D) * Tag::kBytes;
     const uint32_t base = (uint32_t)t.b * (uint32_t)(p.H * p.W) * pix_bytes + (uint32_t)(g * p.D) * Tag::kBytes + (uint32_t)part * 32u;
-#pragma unroll 1
-    for (int k = 0; k < 9; ++k) {
-      if (((far >> k) & 1) == 0) continue;
-      float f3[3];
-      point_of_row<Tag>(row, k, f3);
+    // a lane's own next one: a turn is a chain of two latencies, the first of which the turn before covers
+    float next[3] = {0.f, 0.f, 0.f};
+    if (far != 0) point_of_row<Tag>(row, __builtin_ctz(far), next);
+    while (far != 0) {
+      const int k = __builtin_ctz(far);
+      const float f3[3] = {next[0], next[1], next[2]};
+      far &= far - 1;
+      if (far != 0) point_of_row<Tag>(row, __builtin_ctz(far), next);
       const int i = exact_div(k, 1.f / 3.f), j = k - 3 * i;
       const float x = add_rn(x_base, mul_rn(add_rn((float)i, f3[0]), p.offset_scale));
       const float y = add_rn(y_base, mul_rn(add_rn((float)j, f3[1]), p.offset_scale));
@@ -325,11 +328,14 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
       const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
       const uint32_t pix_bytes = (uint32_t)(p.G * p.D) * Tag::kBytes;
       const uint32_t base = (uint32_t)t.b * (uint32_t)(p.H * p.W) * pix_bytes + (uint32_t)(g * p.D) * Tag::kBytes + (uint32_t)part * 32u;
-#pragma unroll 1
-      for (int k = 0; k < 9; ++k) {
-        if (((far >> k) & 1) == 0) continue;
-        float f3[3], y, x, d[4], r[3];
-        point_of_row<Tag>(row, k, f3);
+      float next[3] = {0.f, 0.f, 0.f};      // as in the forward
+      if (far != 0) point_of_row<Tag>(row, __builtin_ctz(far), next);
+      while (far != 0) {
+        const int k = __builtin_ctz(far);
+        const float f3[3] = {next[0], next[1], next[2]};
+        float y, x, d[4], r[3];
+        far &= far - 1;
+        if (far != 0) point_of_row<Tag>(row, __builtin_ctz(far), next);
         const int i = exact_div(k, 1.f / 3.f);
         x = add_rn(x_base, mul_rn(add_rn((float)i, f3[0]), p.offset_scale));
         y = add_rn(y_base, mul_rn(add_rn((float)(k - 3 * i), f3[1]), p.offset_scale));

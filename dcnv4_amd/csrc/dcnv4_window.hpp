@@ -24,6 +24,8 @@
 //   64x7x7, 32 groups of 16     fp16   12 ->  8
 // and without -> with the halves' order and the shorter address: 64x14x14, 16 groups, fp32 forward 18.0 -> 16.8; 2x200x334, 10 groups,
 // bf16, offsets with tails, 84 -> 80 | 123 -> 120; 64x56x56, 4 groups, fp16 35.1 -> 34.4 | 62.2 -> 60.5.
+// Points outside the window are served a turn at a time, a lane's own next one in each: with all lanes on the same of the nine taps a
+// wave made a turn for every tap that any lane had outside.  2x200x334 as above 80 -> 73 | 120 -> 114, 64x14x14 fp32 forward 16.8 -> 15.3.
 #pragma once
 #include "common.hpp"
 #include "launch.hpp"
