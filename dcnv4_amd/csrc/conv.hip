@@ -1,8 +1,11 @@
 // Dense convolutions on the matrix cores, with bias, batch normalisation and GELU in the epilogue.  A convolution is the product
 // of linear.hip whose rows are output pixels and whose depth runs over (tap, channel): the 16-byte vector that a lane brings in
 // is eight channels of one tap, at the pixel's address plus an offset that depends on the tap alone, or zeros outside the
-// image.  Three kernels:
+// image.  Four kernels:
 //
+//  conv_wide_kernel        very many: the tiles, slices and buffers of linear_wide_kernel.  What bounds the tiles here is the way of
+//                          the gathered operands into LDS: 256 x 128 instead of 128 x 128 brings a quarter less, and two slices
+//                          stay under way where the other kernel waits for its one.
 //  conv_tiled_kernel       many pixels: the tiles, slices and epilogue of linear_tiled_kernel.
 //  conv_few_rows_kernel    a picture at the later stages: 32 pixels x 32 features, the eight waves share the depth, which is
 //                          up to 4032, in registers straight from memory (49 x 512 x 2304 in tiles is 36 slices one after the other).
@@ -11,9 +14,10 @@
 //
 // Measured, 128 pictures of 224 x 224, fp16 (MIOpen's convolution alone | all of it here): picture 3 -> 56, with normalisation and
 // GELU 700 us and two more passes | 114 (180 MB written: 36 at the rate of a copy; the gathered loads and the GELU bound it);
-// 56 -> 112 226 and a pass | 79; 112 -> 224 226 | 95; 224 -> 448 144 | 76; 448 -> 896 97 | 70 (45 GFLOP each, 600 TFLOP/s: what
-// the tiles of linear.hip reach).  One picture, 14 x 14 x 256 -> 512: 9 us.
+// 56 -> 112 226 and a pass | 129, 115 with wide tiles; 112 -> 224 226 | 87, 82; 224 -> 448 144 | 79, 63; 448 -> 896 97 | 60 (45 GFLOP
+// each, 390 to 750 TFLOP/s).  One picture, 14 x 14 x 256 -> 512: 9 us.
 #include "conv.hpp"
+#include "fragments.hpp"
 #include "launch.hpp"
 #include "mfma.hpp"
 
@@ -173,6 +177,97 @@ __global__ void __launch_bounds__(256) conv_tiled_kernel(const ConvLaunch p, int
   }
 }
 
+constexpr int kWideRows = 256, kWideFeatures = 128, kWideBuffers = 3;
+template <typename Tag>
+__global__ void __launch_bounds__(512, 2) conv_wide_kernel(const ConvLaunch p, int rows, int tiles_n) {
+  constexpr int kWaves = 8, MF = 4, NF = 4, kTileBytes = (kWideRows + kWideFeatures) * 64, kLoads = kTileBytes / 1024 / kWaves;
+  constexpr int kPixelLoads = kWideRows / 16 / kWaves;
+  __shared__ __align__(16) char lds[kWideBuffers * kTileBytes];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t tile = xcd_contiguous_block(blockIdx.x, gridDim.x);
+  const int m0 = (int)(tile / tiles_n) * kWideRows, n0 = (int)(tile % tiles_n) * kWideFeatures;
+  const int live_m = min(kWideRows, rows - m0), live_n = min(kWideFeatures, p.n - n0);
+  const int vectors = p.kernel * p.kernel * p.cin / 8, slices = (vectors + 3) / 4;
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.in, (uint32_t)(p.batch * p.h * p.w) * (uint32_t)p.cin * 2u);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(p.weight) + (size_t)n0 * vectors * 16, (uint32_t)live_n * vectors * 16);
+  const float inv_per_tap = __builtin_amdgcn_rcpf((float)(p.cin / 8));
+
+  // a wave's load covers sixteen rows of a tile: lane l takes row l / 4
+  const int row16 = lane >> 2, vector = (lane & 3) ^ (row16 >> 2);
+  int start[kPixelLoads];
+  uint32_t taps[kPixelLoads], weight[kLoads - kPixelLoads];
+#pragma unroll
+  for (int i = 0; i < kPixelLoads; ++i) {
+    const int row = (i * kWaves + wave) * 16 + row16;
+    const PixelWindow window(p, m0 + min(row, live_m - 1), row < live_m);
+    start[i] = window.start;
+    taps[i] = window.taps;
+  }
+#pragma unroll
+  for (int i = 0; i < kLoads - kPixelLoads; ++i) weight[i] = (uint32_t)(((i * kWaves + wave) * 16 + row16) * vectors + vector) * 16;
+  auto stage = [&](int s, int buffer) {
+    const DepthVector d(p, s * 4 + vector, vectors, inv_per_tap);
+    char *to = lds + buffer * kTileBytes + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < kPixelLoads; ++i)
+      load_to_lds(ra, to + i * kWaves * 1024, d.in && ((taps[i] >> d.tap) & 1) ? (uint32_t)(start[i] + d.offset) : kDropOffset);
+#pragma unroll
+    for (int i = 0; i < kLoads - kPixelLoads; ++i)
+      load_to_lds(rw, to + (kPixelLoads + i) * kWaves * 1024, d.in ? weight[i] + (uint32_t)s * 64u : kDropOffset);
+  };
+  const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, kb = lane >> 4;
+  const uint32_t at = lds_address(lds) + fragment_offset(r16, kb), at_m = at + wm * MF * 1024, at_n = at + kWideRows * 64 + wn * NF * 1024;
+  f32x4 acc[NF][MF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int j = 0; j < MF; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kWideBuffers - 1; ++s)
+    if (s < slices) stage(s, s);
+  int cur = 0;
+  for (int s = 0; s < slices; ++s) {
+    wait_behind<kWideBuffers - 2, kLoads, kLoads>(slices - 1 - s, false);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    u32x4 fm[MF], fn[NF];
+    read_fragments(fm, at_m + cur * kTileBytes);
+    read_fragments(fn, at_n + cur * kTileBytes);
+    if (s + kWideBuffers - 1 < slices) stage(s + kWideBuffers - 1, cur == 0 ? kWideBuffers - 1 : cur - 1);
+    fragments_arrived(fm);
+    fragments_arrived(fn);
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int j = 0; j < MF; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[i], fm[j], acc[i][j]);
+    cur = cur == kWideBuffers - 1 ? 0 : cur + 1;
+  }
+  // the fragments turned through the two buffers that the last slice does not use, as in linear_wide_kernel
+  constexpr int TN = NF * 16, kTurn = TN + 4, kPerBuffer = kTileBytes / (16 * kTurn * 4);
+  static_assert(kPerBuffer * (kWideBuffers - 1) >= kWaves, "two buffers hold every wave's sixteen rows");
+  float *turn = reinterpret_cast<float *>(lds + (cur + wave / kPerBuffer) % kWideBuffers * kTileBytes) + wave % kPerBuffer * 16 * kTurn;
+  const int col = (lane & 7) * 8, n = wn * TN + col;
+  const Affine<Tag, 8> affine(p, n0 + n);
+#pragma unroll
+  for (int j = 0; j < MF; ++j) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i) *reinterpret_cast<f32x4 *>(turn + r16 * kTurn + i * 16 + kb * 4) = acc[i][j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = u * 8 + (lane >> 3), row = (wm * MF + j) * 16 + r;
+      float v[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] = fmaf(turn[r * kTurn + col + c], affine.scale[c], affine.shift[c]);
+      if (p.gelu)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] = gelu_exact<Tag>(v[c]);
+      if (row < live_m && n < live_n) store8<Tag>(p.out, (size_t)(m0 + row) * p.n + n0 + n, v);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 constexpr int kFewTile = 32, kFewWaves = 8;
 
 template <typename Tag>
@@ -300,6 +395,21 @@ hipError_t launch_tiled(const ConvLaunch &p, int rows, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Wide tiles where they cover the chip, their columns are not mostly padding, and a pixel is no long run of whole lines: there the
+// 128-byte slices request each line once, which the 64-byte ones do twice.  fp16, output pixels x channels -> features, wide tiles,
+// us tiled | wide:
+//     25088 x 112 -> 224   196   24.1 |  26.2       401408 x  32 ->  64  1568   47.5 |  48.0
+//     31360 x 112 -> 224   246   25.7 |  27.5       100352 x  64 -> 128   392   29.4 |  26.3
+//     37632 x 112 -> 224   294   41.4 |  40.8        50176 x 128 -> 256   392   43.7 |  41.4
+//    100352 x 112 -> 224   784   87.2 |  82.2        50176 x 192 -> 384   588   86.4 |  91.9
+//     25088 x 224 -> 448   392   78.0 |  62.8        25088 x 256 -> 512   392   74.7 |  76.6
+//     31360 x 224 -> 448   492   99.9 |  72.5        25088 x 352 -> 704   588    172 |   160
+//    401408 x  56 -> 112  1568    128 |   117        15680 x 448 -> 896   434    134 |   147
+bool wide_pays(const ConvLaunch &p, long long wide) {
+  const int padded = (p.n + kWideFeatures - 1) / kWideFeatures * kWideFeatures;
+  return wide >= kCus * 9 / 8 && 5 * padded <= 9 * p.n && (p.cin % 64 != 0 || p.cin <= 128);
+}
+
 template <typename Tag>
 hipError_t launch_t(const ConvLaunch &p, hipStream_t stream) {
   const int rows = p.batch * p.ho * p.wo;
@@ -312,6 +422,11 @@ hipError_t launch_t(const ConvLaunch &p, hipStream_t stream) {
     return hipGetLastError();
   }
   if (tiles(128, 64) < 2 * kCus) return launch_tiled<Tag, 64, 64, 2, 2>(p, rows, stream);
+  if (wide_pays(p, tiles(kWideRows, kWideFeatures))) {
+    const int tiles_n = (p.n + kWideFeatures - 1) / kWideFeatures;
+    hipLaunchKernelGGL((conv_wide_kernel<Tag>), dim3((unsigned)((rows + kWideRows - 1) / kWideRows * tiles_n)), dim3(512), 0, stream, p, rows, tiles_n);
+    return hipGetLastError();
+  }
   if (20 * tiles(128, 128) <= 11 * tiles(128, 64)) return launch_tiled<Tag, 128, 128, 2, 2>(p, rows, stream);
   return launch_tiled<Tag, 128, 64, 4, 1>(p, rows, stream);
 }

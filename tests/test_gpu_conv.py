@@ -52,6 +52,23 @@ def test_downsampling_matches_its_modules_in_fp32(channels, size, dtype, tol):
     assert shape == want_shape and got.dtype == dtype and got.shape == want.shape and _rel(got, want) < tol
 
 
+# Wide tiles (256 pixels x 128 features, at least 288 of them): a last tile of 232 pixels and a depth of 45 vectors in slices of four;
+# a second tile of 16 features; channels that straddle lines; whole tiles of whole lines.  The convolution's result and the
+# normalisation's are rounded once each to the type: within two units of roundoff.
+@pytest.mark.parametrize("dtype,unit", [(torch.float16, 2.0**-11), (torch.bfloat16, 2.0**-8)], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("channels,size", [(40, (24, 113, 110)), (72, (12, 111, 113)), (120, (13, 106, 107)), (64, (96, 56, 56))])
+def test_wide_downsampling_matches_its_modules_in_fp32(channels, size, dtype, unit):
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer
+    torch.manual_seed(channels)
+    layer = _settled(DownsampleLayer(channels), dtype)
+    n, h, w = size
+    x = torch.randn(n, h * w, channels, device="cuda").to(dtype)
+    with torch.no_grad():
+        got, _ = layer(x, (h, w))
+        want, _ = layer.float()(x.float(), (h, w))
+    assert _rel(got, want) < 2 * unit
+
+
 @pytest.mark.parametrize("rows", [1, 49, 5000])
 def test_the_heads_convolution_matches_its_modules_in_fp32(rows):
     from dcnv4_amd import ext
