@@ -139,9 +139,10 @@ __device__ __forceinline__ WindowPoint window_point(const WindowFrame<UNITS> &f,
   int at = (int)fx * WindowFrame<UNITS>::kCell + (__mul24((int)fy, f.row_bytes) + f.origin);
   asm("" : "+v"(at));      // or else computed in a branch of its own
   r.addr = r.ok ? at : f.zeros;
-  // m (1 - ly) as m - m ly, rounded once, and so on: no 1 - ly, no 1 - lx
-  const float upper = fmaf(-m, r.ly, m), lower = m * r.ly;
-  r.w[0] = fmaf(-upper, r.lx, upper); r.w[1] = upper * r.lx; r.w[2] = fmaf(-lower, r.lx, lower); r.w[3] = lower * r.lx;
+  // an infinite m stays infinite: products, not m - m ly and so on, and none for zeros
+  m = r.ok ? m : 0.f;
+  const float hx = 1.f - r.lx, upper = m * (1.f - r.ly), lower = m * r.ly;
+  r.w[0] = upper * hx; r.w[1] = upper * r.lx; r.w[2] = lower * hx; r.w[3] = lower * r.lx;
   return r;
 }
 

@@ -67,3 +67,30 @@ def test_window_gathers_drop_offsets_that_are_no_numbers(width, dtype):
     for got, want in zip(*results):
         assert torch.isfinite(got).all()
         cabi.assert_close(got, cabi.f64(want), *GRAD_TOL[dtype], what="against points far outside")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("reach", [4, 0], ids=["window", "beyond"])
+@pytest.mark.parametrize("width", [16, 32, 64])
+def test_window_gathers_carry_infinite_modulations(oracle, width, reach, dtype):
+    """An infinite modulation times corners of one sign is infinite, not NaN, whether the window serves the point or memory (reach 0,
+    for a part of the points).  Pixels whose points all lie inside the image, between its pixels: no corner has the weight zero."""
+    from dcnv4_amd import ext
+    b, h, w, groups = 2, 11, 13, 3
+    case = (b, h, w, groups, width, (3, 3, 1, 1, 1, 1, 1, 1), 0, 1.0, 2.0)
+    v, om, _, (geom, G, D, scale, rc) = _dcn_inputs(case, dtype, seed=width)
+    gen = torch.Generator().manual_seed(width)
+    v = v.abs() + 0.5
+    rows = om[..., :groups * 27].view(b, h, w, groups, 27)
+    rows[..., :18] = ((torch.rand(rows[..., :18].shape, generator=gen) * 0.6 + 0.2) * torch.randn(rows[..., :18].shape, generator=gen).sign()).to(dtype)
+    rows[..., 18:] = (torch.rand(rows[..., 18:].shape, generator=gen) + 0.1).to(dtype)
+    number = torch.arange(b * h * w * groups).view(b, h, w, groups) % 10
+    for tap in range(9):                          # one in ten of every tap, of either sign
+        rows[..., 18 + tap][number == tap] = float("inf") if tap % 2 else float("-inf")
+    want = oracle.dcnv4_forward(cabi.f64(v), cabi.f64(om), *_oracle_args(geom, G, D, scale, rc), coord_f32=True)
+    with ext.launch_options(reach=reach, dual="off"):
+        out = cabi.dcnv4_forward(v.cuda(), om.cuda(), geom, G, D, scale, rc)
+    got, want = cabi.f64(out)[:, 2:-2, 2:-2], want[:, 2:-2, 2:-2]
+    infinite = abs(want) == float("inf")
+    assert infinite.any() and not infinite.all() and (got[infinite] == want[infinite]).all()
+    cabi.assert_close(got[~infinite], want[~infinite], *FWD_TOL[dtype], what="the others")
