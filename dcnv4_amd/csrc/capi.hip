@@ -735,7 +735,10 @@ int static_scratch_of_current_device(void **out) {
 // offsets have tails, for a tile's visits over tails of about twice the near reach.  Learnt offsets (a bell of 2 pixels), grad_value /
 // grad_offset_mask, us, without and with: 2x200x334 with 10 groups of 16 in bf16 (1.9 times the visits) 244 / 109 -> 170 / 122, 64x56x56 with 4 groups
 // of 64 (2.0) 536 -> 515 together; 64x28x28 with 4 of 64 (1.7) 83 / 52 -> 80 / 58, 64x56x56 with 4 of 16 (1.4, the image's edges cut
-// the visits) 105 / 71 -> 99 / 78.  A near reach of 5 pixels serves offsets within +-4; 6, 7 and 8 took 191, 184 and 203 us for the 170
+// the visits) 105 / 71 -> 99 / 78.  Without tails (offsets within +-2) lists are the worse side by what their room costs the first kernel
+// and their word the second; backward, fp16, us, without and with, +-2 | bell: 2x200x334, 10 groups of 16 232 / 234 | 332 / 272, 4 of 64
+// 259 / 260 | 458 / 359; 2x100x167, 20 of 16 130 / 132 | 191 / 161; 2x50x84, 40 of 16 73.5 / 74.5 | 101 / 92; 32x56x56, 8 of 32 213 / 213 |
+// 308 / 268; the least gain for its cost 64x56x56, 4 of 64 377 / 384 | 511 / 503.  A near reach of 5 pixels serves offsets within +-4; 6, 7 and 8 took 191, 184 and 203 us for the 170
 // above, by what fits a strip.
 constexpr int kNearReach = 5;
 bool far_lists_fit(const DcnLaunch &L, const DcnProblem &pr, const void *grad_value, std::initializer_list<std::pair<const void *, size_t>> others) {

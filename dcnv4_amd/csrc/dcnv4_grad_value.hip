@@ -7,7 +7,15 @@ namespace {
 
 template <typename Tag, int KP, int CW, int ROUNDS, int NT, bool LISTS = false>
 __global__ void __launch_bounds__(NT, LISTS ? 4 : 1) dcnv4_grad_value_kernel(const DcnLaunch p) {
-  dcnv4_grad_value_body<Tag, KP, CW, ROUNDS, NT, LISTS>(p, blockIdx.x, gridDim.x);
+  if constexpr (LISTS) {
+    float acc[4][CW] = {};
+    int reach;
+    const GradPlace place = grad_place(p, blockIdx.x, gridDim.x, reach);
+    if (p.state->listed != 0) dcnv4_grad_value_listed<Tag, CW, NT>(kernel_argument(), place, reach, acc);
+    dcnv4_grad_value_strips<Tag, KP, CW, ROUNDS, NT>(p, place, reach, acc);
+  } else {
+    dcnv4_grad_value_body<Tag, KP, CW, ROUNDS, NT>(p, blockIdx.x, gridDim.x);
+  }
 }
 
 constexpr int gv_rounds(int kp) { return kp > 0 ? kGradValueColumnRounds : kGradValueRounds; }

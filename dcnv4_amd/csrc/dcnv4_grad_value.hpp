@@ -23,11 +23,11 @@
 //     first: what the sampling points within the reach cap need; a tile that points beyond the
 //     cap land in reads its own, larger number from GradState::far_reach), in strips of
 //     interleaved rows, so that every strip spreads its points evenly over the tile.  With lists
-//     (LISTS) the reach stays at a few pixels whatever tails the offsets have, and the points
-//     that land in the tile from farther away are read from its list at the end, as many at a
-//     time as it has lanes: the visits of a tile of 20 x 21 are 930 pixels for a reach of 5 and
-//     1980 for the 12 that a bell of 2 pixels asks for (2x200x334, 10 groups of 16, bf16: 244 ->
-//     170 us).  Per strip:
+//     (dcnv4_grad_value_listed) the reach stays at a few pixels whatever tails the offsets have,
+//     and the points that land in the tile from farther away are read from its list first, as
+//     many at a time as it has lanes: the visits of a tile of 20 x 21 are 930 pixels for a reach
+//     of 5 and 1980 for the 12 that a bell of 2 pixels asks for (2x200x334, 10 groups of 16,
+//     bf16: 244 -> 170 us).  Per strip:
 //       park   the strip's grad_out rows are copied to LDS;
 //       A      one lane per (group, pixel, kernel tap) recomputes the sampling position and links
 //              a 16-byte entry (m * hy, m * ly, lx, address of the pixel's parked grad_out | next)
@@ -57,14 +57,65 @@ template <typename Tag> struct ParkType { typedef float type; };
 __device__ __forceinline__ int fdiv_small(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }   // exact for n < 2^20
 
 
+// The workgroup's image, tile and chunk of groups.
+struct GradPlace {
+  int b, ty, tx, chunk;
+};
+// How far the tile's visit goes: the reach that the bulk of the sampling points needs, or - for a tile that points beyond the reach
+// cap land in - how far away the output pixels of those points lie (GradState::far_reach): only such tiles pay for outliers.
+__device__ __forceinline__ GradPlace grad_place(const DcnLaunch &p, uint32_t bid, uint32_t nblocks, int &reach) {
+  const int n_chunks = (p.G + p.ng_chunk - 1) / p.ng_chunk;
+  const int nty = (p.H + p.tile_h - 1) / p.tile_h, ntx = (p.W + p.tile_w - 1) / p.tile_w;
+  uint32_t id = xcd_contiguous_block(bid, nblocks);
+  GradPlace r;
+  r.chunk = id % n_chunks; id /= n_chunks;
+  r.tx = id % ntx; id /= ntx;
+  r.ty = id % nty;
+  r.b = id / nty;
+  reach = p.gv_whole ? (1 << 20)
+                     : (int)min(max(p.state->reach_needed, p.state->far_reach[dcnv4_far_slot(r.b, r.ty, r.tx, nty, ntx, r.chunk, n_chunks)]), 1u << 20);
+  return r;
+}
+
+// Walks one list: the next entry is read while the current one is applied.
+// Corner weights (common.h:48-58, 153-184): modulation * row weight * column weight.
+template <int CW>
+__device__ __forceinline__ void grad_walk(uint32_t e, uint32_t end_idx, const u32x4 *s_entry, const char *go_lane, float (&acc)[4][CW]) {
+  u32x4 ent = s_entry[e];
+  while (e != end_idx) {
+    e = ent.w >> 14;
+    const u32x4 next = s_entry[e];
+    const uint32_t a_bits = ent.x, b_bits = ent.y, fx_bits = ent.z;
+    const float wa = __builtin_bit_cast(float, a_bits), wb = __builtin_bit_cast(float, b_bits);
+    const float fxv = __builtin_bit_cast(float, fx_bits), hxv = 1.f - fxv;
+    const float w4[4] = {wa * hxv, wa * fxv, wb * hxv, wb * fxv};
+    const char *g = go_lane + ((ent.w & 0x3fffu) << 4);
+    // the row in pieces of at most 32 bytes, one piece in registers at a time
+    constexpr int kLaneBytes = CW * 4, kPieceBytes = kLaneBytes < 32 ? kLaneBytes : 32, kPiece = kPieceBytes / 4;
+#pragma unroll
+    for (int h = 0; h < CW / kPiece; ++h) {
+      float gv[kPiece];
+#pragma unroll
+      for (int q = 0; q < kPieceBytes / 16; ++q)
+        *reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(gv) + 16 * q) = *reinterpret_cast<const u32x4 *>(g + kPieceBytes * h + 16 * q);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int c = 0; c < kPiece; ++c) acc[k][h * kPiece + c] = fmaf(w4[k], gv[c], acc[k][h * kPiece + c]);
+      if (h + 1 < CW / kPiece) __builtin_amdgcn_sched_barrier(0);
+    }
+    ent = next;
+  }
+}
+
 // CW: channels a lane accumulates for each of the four corners (8 or 16): the group width rounded up, or 16 with
 // several lanes per (anchor, group).
 // NT: lanes per workgroup (512: two workgroups share a CU and overlap each other's phases; 1024: one workgroup with
 // the whole LDS); one (anchor, group) list per lane at most.
 // (the body of the kernel as a function of the workgroup's number, so that a grid can also hold workgroups of another role)
-// LISTS: 3x3 kernels with their centre only.
-template <typename Tag, int KP, int CW, int ROUNDS, int NT, bool LISTS = false>
-__device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32_t bid, uint32_t nblocks) {
+// acc: the sums so far.
+template <typename Tag, int KP, int CW, int ROUNDS, int NT>
+__device__ __forceinline__ void dcnv4_grad_value_strips(const DcnLaunch &p, const GradPlace &place, int reach, float (&acc)[4][CW]) {
   constexpr int kValThreads = NT, kMaxAnchorSlots = NT;
   extern __shared__ __align__(16) uint32_t lds32[];
   typedef typename ParkType<Tag>::type park_t;
@@ -72,14 +123,8 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
   constexpr int kParkBytes = sizeof(park_t);
   constexpr int kLaneBytes = CW * kParkBytes;                 // bytes of a parked row a lane reads per entry
   const int Kp = p.Kp, D = p.D, C = p.G * p.D;
-  const int n_chunks = (p.G + p.ng_chunk - 1) / p.ng_chunk;
   const int eh = p.tile_h, ew = p.tile_w;                     // tile extent; cells are indexed with the power-of-two stride
-  const int nty = (p.H + eh - 1) / eh, ntx = (p.W + ew - 1) / ew;
-  uint32_t id = xcd_contiguous_block(bid, nblocks);
-  const int chunk = id % n_chunks; id /= n_chunks;
-  const int tx = id % ntx; id /= ntx;
-  const int ty = id % nty;
-  const int b = id / nty;
+  const auto [b, ty, tx, chunk] = place;
   const int g0 = chunk * p.ng_chunk, ng = min(p.ng_chunk, p.G - g0);
   const int ty0 = ty * eh, tx0 = tx * ew;
   const int th = min(eh, p.H - ty0), tw = min(ew, p.W - tx0);
@@ -104,11 +149,6 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
   // output pixels this tile visits: reference point (centre tap at zero offset) within `reach` of the tile
   const int half_w = (p.dw * (p.kw - 1)) >> 1, half_h = (p.dh * (p.kh - 1)) >> 1;
   const int cy0 = half_h - p.ph, cx0 = half_w - p.pw, Ho = p.Q / p.Wo;
-  // the reach that the bulk of the sampling points needs, or - for a tile that points beyond the reach cap land in -
-  // how far away the output pixels of those points lie (GradState::far_reach): only such tiles pay for outliers
-  const int reach = p.gv_whole ? (1 << 20)
-                               : (int)min(max(p.state->reach_needed, p.state->far_reach[dcnv4_far_slot(b, ty, tx, nty, ntx, chunk, n_chunks)]), 1u << 20);
-  const bool listed = LISTS && p.state->listed != 0;
   const int ho_lo = max(0, ceil_div_signed(ty0 - reach - cy0, p.sh));
   const int ho_hi = min(Ho, ceil_div_signed(ty0 + eh + reach - cy0, p.sh));
   const int wo_lo_all = max(0, ceil_div_signed(tx0 - reach - cx0, p.sw));
@@ -126,12 +166,6 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
     const int ay = fdiv_small(row, 1.f / (float)p.ng_chunk), gl = row - ay * p.ng_chunk;
     list_live = my_list < n_lists && ay <= th && ax <= tw && gl < ng;
   }
-  float acc[4][CW];
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int c = 0; c < CW; ++c) acc[k][c] = 0.f;
-
   s_head[tid] = end_idx;
   s_head[kMaxAnchorSlots + tid] = end_idx;
   if (tid == 0) s_entry[end_idx] = u32x4{0u, 0u, 0u, end_idx << 14};
@@ -145,41 +179,6 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
   auto to_f = [](elem_t raw) { float f[1]; Pack<Tag, 1>::decode(raw, f); return f[0]; };
 
   int parity = 0;                                             // which half of s_head the current strip uses
-  // Phase B: every lane walks its own anchor's list; the next entry is read while the current one is applied.
-  // Corner weights (common.h:48-58, 153-184): modulation * row weight * column weight.
-  auto walk = [&](const uint32_t *head) {
-    if (list_live) {
-      uint32_t e = head[my_list];
-      s_head[parity * kMaxAnchorSlots + my_list] = end_idx;    // the next strip's head of this list
-      const char *go_lane = s_go + my_part * kLaneBytes;
-      u32x4 ent = s_entry[e];
-      while (e != end_idx) {
-        e = ent.w >> 14;
-        const u32x4 next = s_entry[e];
-        const uint32_t a_bits = ent.x, b_bits = ent.y, fx_bits = ent.z;
-        const float wa = __builtin_bit_cast(float, a_bits), wb = __builtin_bit_cast(float, b_bits);
-        const float fxv = __builtin_bit_cast(float, fx_bits), hxv = 1.f - fxv;
-        const float w4[4] = {wa * hxv, wa * fxv, wb * hxv, wb * fxv};
-        const char *g = go_lane + ((ent.w & 0x3fffu) << 4);
-        // the row in pieces of at most 32 bytes, one piece in registers at a time
-        constexpr int kPieceBytes = kLaneBytes < 32 ? kLaneBytes : 32;
-        constexpr int kPiece = kPieceBytes / kParkBytes;       // channels per piece
-#pragma unroll
-        for (int h = 0; h < CW / kPiece; ++h) {
-          park_t gv[kPiece];
-#pragma unroll
-          for (int q = 0; q < kPieceBytes / 16; ++q)
-            *reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(gv) + 16 * q) = *reinterpret_cast<const u32x4 *>(g + kPieceBytes * h + 16 * q);
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int c = 0; c < kPiece; ++c) acc[k][h * kPiece + c] = fmaf(w4[k], (float)gv[c], acc[k][h * kPiece + c]);
-          if (h + 1 < CW / kPiece) __builtin_amdgcn_sched_barrier(0);
-        }
-        ent = next;
-      }
-    }
-  };
   for (int wo_lo = wo_lo_all; wo_lo < wo_hi_all && n_rows > 0; wo_lo += cols_cap) {
     const int nwx = min(cols_cap, wo_hi_all - wo_lo);
 
@@ -345,50 +344,13 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
       if (s + 1 < n_strips) prefetch(s + 1);
       __syncthreads();
 
-      walk(head);
-      __syncthreads();
-    }
-  }
-
-  // Points of the tile's list, a lane each: its pixel's grad_out row of the point's group, and the entry as in phase A, unless the
-  // pixel was visited.
-  if (LISTS && listed) {
-    const FarList far_list(p, Tag::kBytes, ty, tx, chunk);
-    const int n_far = min(__builtin_amdgcn_readfirstlane((int)static_cast<const FarHeader *>(far_list.slot(p, Tag::kBytes, b, 0))->count), far_list.capacity);
-    const int far_stride = (Dp * kParkBytes / 16 | 1) * 16;
-    const int far_chunk = min(min(NT, (int)end_idx), p.strip_pix * go_stride / far_stride);
-    for (int f0 = 0; f0 < n_far; f0 += far_chunk) {
-      uint32_t *head = s_head + parity * kMaxAnchorSlots;
-      parity ^= 1;
-      if (tid < far_chunk && f0 + tid < n_far) {
-        const FarRecord rec = *static_cast<const FarRecord *>(far_list.slot(p, Tag::kBytes, b, 1 + f0 + tid));
-        const int k = (int)(rec.point & 0xffu), gl = (int)(rec.point >> 8);
-        const int ho = (int)rec.pixel / p.Wo, wo = (int)rec.pixel - ho * p.Wo, ti = k / 3, tjj = k - 3 * ti;
-        const bool visited = dcnv4_away(p, ty, tx, cy0 + ho * p.sh, cx0 + wo * p.sw) <= reach;
-        const elem_t *om = om_img + ((size_t)rec.pixel * p.P_pad + (size_t)((g0 + gl) * 3 * Kp));
-        const elem_t off_x = om[2 * k], off_y = om[2 * k + 1], m_raw = om[2 * Kp + k];
-        const elem_t *src = go_img + ((size_t)rec.pixel * C + (size_t)(g0 + gl) * D);
-        float *dst = reinterpret_cast<float *>(s_go + tid * far_stride);
-        constexpr int kRowVec = 16 / Tag::kBytes;               // groups of 32, 64 or 128 bytes (plan_window_gather)
-        for (int u = 0; u < D; u += kRowVec) {
-          float f[kRowVec];
-          Pack<Tag, kRowVec>::decode(*reinterpret_cast<const typename Pack<Tag, kRowVec>::raw_t *>(src + u), f);
-#pragma unroll
-          for (int c = 0; c < kRowVec; c += 4) *reinterpret_cast<f32x4 *>(dst + u + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
-        }
-        const float x = add_rn(sub_rn((float)(cx0 + wo * p.sw), x_sub), mul_rn(add_rn((float)(ti * p.dw), to_f(off_x)), p.offset_scale));
-        const float y = add_rn(sub_rn((float)(cy0 + ho * p.sh), y_sub), mul_rn(add_rn((float)(tjj * p.dh), to_f(off_y)), p.offset_scale));
-        const float fy = floorf(y), fx = floorf(x);
-        const int ay = (int)fy - ty0 + 1, ax = (int)fx - tx0 + 1;
-        if (!visited && (unsigned)ay <= (unsigned)th && (unsigned)ax <= (unsigned)tw) {
-          const float m = to_f(m_raw), ly = y - fy, lx = x - fx;
-          const uint32_t succ = __hip_atomic_exchange(&head[ay * (p.ng_chunk * aw) + gl * aw + ax], (uint32_t)tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          s_entry[tid] = u32x4{__builtin_bit_cast(uint32_t, m * (1.f - ly)), __builtin_bit_cast(uint32_t, m * ly),
-                               __builtin_bit_cast(uint32_t, lx), (uint32_t)(tid * far_stride) >> 4 | (succ << 14)};
-        }
+      // ---- phase B: every lane walks its own anchor's list
+      if (list_live) {
+        const uint32_t first = head[my_list];
+        s_head[parity * kMaxAnchorSlots + my_list] = end_idx;    // the next strip's head of this list
+        __builtin_amdgcn_s_waitcnt(0x0f70);      // of memory: nothing is under way, and left unsaid the walk waits for it at every entry
+        grad_walk<CW>(first, end_idx, s_entry, s_go + my_part * kLaneBytes, acc);
       }
-      __syncthreads();
-      walk(head);
       __syncthreads();
     }
   }
@@ -450,6 +412,86 @@ __device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32
       const float f[1] = {s_sum[(cy * ew + cx) * row_floats + gl * Dp + ch]};
       gv_img[(size_t)((ty0 + cy) * p.W + tx0 + cx) * C + (g0 + gl) * D + ch] = Pack<Tag, 1>::encode(f);
     }
+  }
+}
+
+
+template <typename Tag, int KP, int CW, int ROUNDS, int NT>
+__device__ __forceinline__ void dcnv4_grad_value_body(const DcnLaunch &p, uint32_t bid, uint32_t nblocks) {
+  float acc[4][CW] = {};
+  int reach;
+  const GradPlace place = grad_place(p, bid, nblocks, reach);
+  dcnv4_grad_value_strips<Tag, KP, CW, ROUNDS, NT>(p, place, reach, acc);
+}
+
+// The kernel's argument, read again where it is asked for.
+__device__ __forceinline__ DcnLaunch kernel_argument() {
+  auto *p = (const __attribute__((address_space(4))) DcnLaunch *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const DcnLaunch *)p;
+}
+
+// Points of the tile's list (3x3 kernels with their centre, groups of 32, 64 or 128 bytes), as many at a time as there are lanes: a
+// lane parks its point's grad_out row of the point's group and links an entry as phase A does, unless the pixel will be visited.
+// Ahead of the strips, with the kernel's argument read again: behind them, what it needs was kept over the strips, which have no
+// register to spare, and cost them one to four spilled ones, also where no point is far (64x56x56, 4 groups of 64, fp16, offsets
+// within +-2: 278 us, now 271; without lists 267).
+template <typename Tag, int CW, int NT>
+__device__ __forceinline__ void dcnv4_grad_value_listed(const DcnLaunch &p, const GradPlace &place, int reach, float (&acc)[4][CW]) {
+  extern __shared__ __align__(16) uint32_t lds32[];
+  typedef typename RawWord<Tag::kBytes>::type elem_t;
+  const int tid = threadIdx.x, C = p.G * p.D, aw = p.tile_w + 1, lps_log2 = p.gv_lps_log2;
+  const int ty0 = place.ty * p.tile_h, tx0 = place.tx * p.tile_w, g0 = place.chunk * p.ng_chunk;
+  const int th = min(p.tile_h, p.H - ty0), tw = min(p.tile_w, p.W - tx0);
+  uint32_t *s_head = lds32;
+  char *s_go = reinterpret_cast<char *>(lds32 + 2 * NT);
+  u32x4 *s_entry = reinterpret_cast<u32x4 *>(s_go + (size_t)p.strip_pix * p.gv_go_stride);
+  const uint32_t end_idx = (uint32_t)(p.strip_pix * 9 * p.ng_chunk);
+  const FarList list(p, Tag::kBytes, place.ty, place.tx, place.chunk);
+  const int count = min(__builtin_amdgcn_readfirstlane((int)static_cast<const FarHeader *>(list.slot(p, Tag::kBytes, place.b, 0))->count), list.capacity);
+  const int stride = ((CW << lps_log2) / 4 | 1) * 16;
+  const int together = min(min(NT, (int)end_idx), p.strip_pix * p.gv_go_stride / stride);
+  const int cy0 = 1 - p.ph, cx0 = 1 - p.pw;
+  const int my_list = tid >> lps_log2, my_part = tid & ((1 << lps_log2) - 1);
+  if (tid == 0) s_entry[end_idx] = u32x4{0u, 0u, 0u, end_idx << 14};
+  for (int first = 0; first < count; first += together) {
+    s_head[tid] = end_idx;
+    __syncthreads();
+    int mine = tid;
+    asm volatile("" : "+v"(mine));      // what is made of it below is not kept over the turns
+    if (mine < together && first + mine < count) {
+      const FarRecord rec = *static_cast<const FarRecord *>(list.slot(p, Tag::kBytes, place.b, 1 + first + mine));
+      const int k = (int)(rec.point & 0xffu), gl = (int)(rec.point >> 8);
+      const int ho = (int)rec.pixel / p.Wo, wo = (int)rec.pixel - ho * p.Wo, ti = k / 3, tjj = k - 3 * ti;
+      const bool visited = dcnv4_away(p, place.ty, place.tx, cy0 + ho, cx0 + wo) <= reach;
+      const size_t pixel = (size_t)place.b * p.Q + rec.pixel;
+      const elem_t *om = static_cast<const elem_t *>(p.offset_mask) + (pixel * p.P_pad + (size_t)((g0 + gl) * 27));
+      const elem_t *src = static_cast<const elem_t *>(p.grad_out) + (pixel * C + (size_t)(g0 + gl) * p.D);
+      auto widened = [](elem_t raw) { float f[1]; Pack<Tag, 1>::decode(raw, f); return f[0]; };
+      const elem_t off_x = om[2 * k], off_y = om[2 * k + 1], m_raw = om[18 + k];
+      float *dst = reinterpret_cast<float *>(s_go + mine * stride);
+      constexpr int kRowVec = 16 / Tag::kBytes;
+      for (int u = 0; u < p.D; u += kRowVec) {
+        float f[kRowVec];
+        Pack<Tag, kRowVec>::decode(*reinterpret_cast<const typename Pack<Tag, kRowVec>::raw_t *>(src + u), f);
+#pragma unroll
+        for (int c = 0; c < kRowVec; c += 4) *reinterpret_cast<f32x4 *>(dst + u + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
+      }
+      const float x = add_rn(sub_rn((float)(cx0 + wo), p.offset_scale), mul_rn(add_rn((float)ti, widened(off_x)), p.offset_scale));
+      const float y = add_rn(sub_rn((float)(cy0 + ho), p.offset_scale), mul_rn(add_rn((float)tjj, widened(off_y)), p.offset_scale));
+      const float fy = floorf(y), fx = floorf(x);
+      const int ay = (int)fy - ty0 + 1, ax = (int)fx - tx0 + 1;
+      if (!visited && (unsigned)ay <= (unsigned)th && (unsigned)ax <= (unsigned)tw) {
+        const float m = widened(m_raw), ly = y - fy, lx = x - fx;
+        const uint32_t succ = __hip_atomic_exchange(&s_head[ay * (p.ng_chunk * aw) + gl * aw + ax], (uint32_t)mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        s_entry[mine] = u32x4{__builtin_bit_cast(uint32_t, m * (1.f - ly)), __builtin_bit_cast(uint32_t, m * ly),
+                             __builtin_bit_cast(uint32_t, lx), (uint32_t)(mine * stride) >> 4 | (succ << 14)};
+      }
+    }
+    __syncthreads();
+    // only lists of live anchors have entries
+    grad_walk<CW>(s_head[my_list], end_idx, s_entry, s_go + my_part * CW * 4, acc);
+    __syncthreads();
   }
 }
 
