@@ -179,8 +179,9 @@ def main():
         # LDS read patterns: ticks per wave-level 16-byte read, and each pattern against the best one
         names = ["consecutive addresses (slot = lane, one cell per wave)", "random cells, slot = lane & 15 (16 lanes cover 256 B)",
                  "random cells, slot = lane & 7 (8 lanes cover 128 B)", "random cells, random slots (a gather of rows)",
-                 "random cells, every lane on slot 0"]
-        ticks = [min(ext.lds_read_probe(pat, 4000) for _ in range(3)) for pat in range(5)]
+                 "random cells, every lane on slot 0", "a fragment of 16 rows of 64 bytes, as the matrix kernels place it",
+                 "the same, vectors at lane / 16 ^ (-(row / 4) & 3)"]
+        ticks = [min(ext.lds_read_probe(pat, 4000) for _ in range(3)) for pat in range(7)]
         print(json.dumps({"only_op": "lds_probe", "unit": "cycle-counter ticks per wave instruction (ds_read_b128, 16 waves, 8 reads in flight)",
                           "patterns": [{"pattern": n, "ticks": round(t, 2), "vs_best": round(t / min(ticks), 2)} for n, t in zip(names, ticks)]}))
         return

@@ -15,6 +15,7 @@
 
 #include "../../include/dcnv4_gfx950.h"
 #include "common.hpp"
+#include "fragments.hpp"
 #include "launch.hpp"
 
 namespace dcn {
@@ -111,6 +112,9 @@ __global__ void __launch_bounds__(256) stream_copy_kernel(const u32x4 *src, u32x
 //   2  a random cell per lane, slot = lane & 7: 8 consecutive lanes cover the 8 slots of 128 bytes
 //   3  a random cell and a random slot per lane (what a gather from rows at data-dependent cells looks like)
 //   4  a random cell per lane, slot 0 for every lane (the worst case)
+//   5  all lanes of a wave in one cell, as the matrix kernels read a fragment: sixteen rows of 64 bytes, vectors where fragment_offset puts
+//      them.  Any 16 consecutive lanes cover 16 different slots, the 16 lanes of a pass do not.
+//   6  the same with a row's vectors at vector ^ (-(row / 4) & 3): the lanes of a pass cover 16 different slots
 __global__ void __launch_bounds__(1024) lds_read_probe_kernel(int pattern, int iters, uint32_t *ticks_per_1000) {
   __shared__ u32x4 cells[4096];                   // 64 KB
   for (int i = threadIdx.x; i < 4096; i += 1024) cells[i] = u32x4{(uint32_t)i, 0u, 0u, 0u};
@@ -118,7 +122,8 @@ __global__ void __launch_bounds__(1024) lds_read_probe_kernel(int pattern, int i
   const int lane = threadIdx.x & 63;
   uint32_t seed = threadIdx.x * 131u + 7u;
   u32x4 acc = {0u, 0u, 0u, 0u};
-  const int fixed_slot = pattern == 0 ? lane : (pattern == 1 ? (lane & 15) : (pattern == 2 ? (lane & 7) : 0));
+  const int row = lane & 15, vector = lane >> 4;
+  const int fixed_slot = pattern == 0 ? lane : pattern == 1 ? lane & 15 : pattern == 2 ? lane & 7 : pattern == 5 ? (int)fragment_offset(row, vector) / 16 : pattern == 6 ? row * 4 + (vector ^ (-(row >> 2) & 3)) : 0;
   __syncthreads();
   const long long t0 = clock64();
   for (int i = 0; i < iters; ++i) {
@@ -127,7 +132,7 @@ __global__ void __launch_bounds__(1024) lds_read_probe_kernel(int pattern, int i
     u32x4 v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int cell = pattern == 0 ? ((i + u) & 63) : (int)((r >> (3 * u)) & 63u);
+      const int cell = pattern == 0 || pattern >= 5 ? ((i + u) & 63) : (int)((r >> (3 * u)) & 63u);
       const int slot = pattern == 3 ? (int)((r >> (2 * u + 1)) & 63u) : fixed_slot;
       v[u] = cells[cell * 64 + slot];
     }
@@ -1457,8 +1462,8 @@ int dcnv4_gfx950_center_feature_blend_backward(const void *grad_output, const vo
 }
 
 int dcnv4_gfx950_lds_read_probe(int pattern, int iters, unsigned int *ticks_per_1000_reads, void *stream) {
-  if (pattern < 0 || pattern > 4 || iters < 1 || iters > (1 << 20))
-    return fail(DCNV4_ERR_INVALID_ARGUMENT, "LDS read probe: pattern %d (0..4), %d rounds (1..2^20)", pattern, iters);
+  if (pattern < 0 || pattern > 6 || iters < 1 || iters > (1 << 20))
+    return fail(DCNV4_ERR_INVALID_ARGUMENT, "LDS read probe: pattern %d (0..6), %d rounds (1..2^20)", pattern, iters);
   if (ticks_per_1000_reads == nullptr) return fail(DCNV4_ERR_RUNTIME, "null tensor pointer");
   hipLaunchKernelGGL(lds_read_probe_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), pattern, iters, ticks_per_1000_reads);
   if (hipError_t e = hipGetLastError()) return hip_fail("LDS read probe launch", e);

@@ -36,8 +36,8 @@ __global__ void __launch_bounds__(256, KF <= 4 ? 3 : 2) mlp_kernel(const MlpLaun
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const uint16_t *>(p.a) + (size_t)m0 * c, (uint32_t)live * c * 2);
   const __amdgpu_buffer_rsrc_t r1 = make_rsrc(p.w1, (uint32_t)p.hidden * c * 2), r2 = make_rsrc(p.w2, (uint32_t)p.hidden * c * 2);
 
-  // w1: [unit of 32 channels][feature][piece of 16 bytes ^ feature / 8], w2: [output feature][piece ^ feature / 4]: the sixteen rows
-  // that a fragment read touches fall into different banks
+  // w1: [unit of 32 channels][feature][piece of 16 bytes ^ feature / 8], w2: [output feature][piece ^ feature / 4]: any
+  // sixteen consecutive lanes of a fragment read fall into different banks, the lanes of a pass by twos into the same (fragments.hpp)
   uint32_t offset[KF];      // of the lane's pieces in the first chunk's weights
 #pragma unroll
   for (int i = 0; i < KF; ++i) {

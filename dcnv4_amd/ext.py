@@ -343,7 +343,8 @@ def stream_copy(src, dst):
 
 def lds_read_probe(pattern, iters=4000, device=None):
     """Ticks of the cycle counter per wave-level 16-byte LDS read for one of the probe's address patterns (0 consecutive,
-    1 random cells with slot = lane & 15, 2 slot = lane & 7, 3 random cells and slots, 4 all lanes on one slot)."""
+    1 random cells with slot = lane & 15, 2 slot = lane & 7, 3 random cells and slots, 4 all lanes on one slot, 5 a fragment of the
+    matrix kernels, 6 the same with vectors at lane / 16 ^ (-(row / 4) & 3))."""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else device
     with _on_device(device):
         out = torch.zeros(1, dtype=torch.int32, device=device)

@@ -334,6 +334,8 @@ int dcnv4_gfx950_stream_copy(const void *src, void *dst, size_t bytes, void *str
  *           2  a random cell per lane, slot = lane & 7
  *           3  a random cell and a random slot per lane (a gather of rows at data-dependent cells)
  *           4  a random cell per lane, slot 0 for all (worst case)
+ *           5  one cell per wave, sixteen rows of 64 bytes, as the matrix kernels read a fragment (lane & 15 the row)
+ *           6  the same with the vectors at lane / 16 ^ (-(row / 4) & 3)
  * The ratios between the patterns say which address patterns the sampling kernels' LDS reads can hope for.
  */
 int dcnv4_gfx950_lds_read_probe(int pattern, int iters, unsigned int *ticks_per_1000_reads, void *stream);

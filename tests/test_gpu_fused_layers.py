@@ -249,3 +249,14 @@ def test_lds_read_probe_orders_its_patterns():
     assert 0 < best < gather < worst and worst > 3 * best
     with pytest.raises(ValueError, match="pattern"):
         ext.lds_read_probe(9)
+
+
+def test_lanes_that_share_a_pass_of_the_lds():
+    """Which lanes a pass of ds_read_b128 takes together (fragments.hpp): sixteen rows of 64 bytes cost what consecutive addresses do with
+    their vectors at vector ^ (-(row / 4) & 3), and twice that in the LDS at vector ^ row / 4.  Of that the probe shows 1.15: its own
+    address arithmetic takes 4.78 ticks a read, beside the 2.8 that the LDS needs without conflicts and the 5.5 with them.  The bounds
+    lie half way."""
+    from dcnv4_amd import ext
+    consecutive, met, apart = (min(ext.lds_read_probe(pattern, 4000) for _ in range(3)) for pattern in (0, 5, 6))
+    print(f"LDS probe: consecutive {consecutive:.2f}, by twos {met:.2f}, apart {apart:.2f} ticks per read", flush=True)
+    assert apart < 1.07 * consecutive and met > 1.07 * apart
