@@ -9,7 +9,8 @@
 // What bounds it then is the GELU (seventeen issue slots an element, 23 in bf16; with 112 channels and 23 the vector units were busy
 // 59 % of the time, the matrix cores 22) and, with 224 channels, the two waves that its registers leave room for (34 and 21 %).
 // A layer normalisation behind the MLP (NORM: residual + gamma * norm(mlp)) takes the sums of a row from the registers of the four
-// lanes that hold it: two kernels -> one, us, 401408 x 112 163 + 46 -> 165 to 185, 100352 x 224 142 + 23 -> 153 to 168.
+// lanes that hold it: two kernels -> one, us, 401408 x 112 163 + 46 -> 149 to 163, 100352 x 224 142 + 23 -> 134 to 148
+// (in a model; 144 to 158 while 37 of its registers spilled).
 // Measured, fp16, two kernels -> this one: 401408 x 112 336 -> 160 us, 100352 x 224 203 -> 140, both with the GELU of 23 slots (145 and 134 with one of
 // thirteen instructions, which was less exact than the fp32 function).
 #include <algorithm>
