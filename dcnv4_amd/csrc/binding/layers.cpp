@@ -206,7 +206,7 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
     RowsLaunch p = {a, ptr(wt), ptr(b), rows, (int)c, (int)k, {ptr(n.weight), ptr(n.bias), n.eps, ptr(gamma), residual, stream_out, normed_out, normed_out != nullptr}};
     hip_check(launch_rows(code, p, static_cast<hipStream_t>(stream)), "linear layer launch");
   };
-  const bool whole_rows = rows_fits(code, rows, (int)c, (int)c) && rows_fits(code, rows, (int)c, (int)l.hidden);
+  const bool whole_rows = rows_fits(code, rows, (int)c, (int)c, !l.post_norm) && (!l.post_norm || rows_fits(code, rows, (int)c, (int)l.hidden, false));
 
   // DCNv4 half
   const bool norm_first = !l.post_norm && l.dw_kernel == 0;      // the normalised rows go into the projections alone
@@ -328,9 +328,22 @@ PyObject *py_layer_inference(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// rows_fits(x, width, after_residual): whether a product x @ [width, k].T and the normalisation behind it are one kernel
+PyObject *py_rows_fits(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("rows_fits", args, n, 3);
+  const Tensor &x = a.tensor();
+  const int width = a.integer();
+  const bool after_residual = a.integer() != 0;
+  const int64_t k = x.dim() ? x.size(-1) : 0;
+  return PyBool_FromLong(k != 0 && rows_fits(dtype_code(x, "input"), x.numel() / k, width, (int)k, after_residual));
+  END_HANDLE_TH_ERRORS
+}
+
 }  // namespace
 
 PyMethodDef layer_methods[] = {
+    {"rows_fits", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_rows_fits)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear)), METH_FASTCALL, nullptr},
     {"layer_inference", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_layer_inference)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -75,7 +75,7 @@ struct RowsLaunch {
   int n, k;
   NormEpilogue norm;
 };
-bool rows_fits(int dtype, long long rows, int n, int k);
+bool rows_fits(int dtype, long long rows, int n, int k, bool after_residual);
 hipError_t launch_rows(int dtype, const RowsLaunch &p, hipStream_t stream);
 
 // (gelu(a w1' + b1) w2' + b2) * gamma + residual over [rows, c], w1 [hidden, c], w2 [c, hidden]; b1, b2, gamma, residual may be null.

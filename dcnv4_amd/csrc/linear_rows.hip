@@ -146,20 +146,35 @@ hipError_t launch_t(const RowsLaunch &p, hipStream_t stream) {
 
 }  // namespace
 
-// Up to 256 features the workgroups run two and more to a CU: from half a chip of them on.  With more a CU holds one, and they pay where their
-// rounds over the chip are fuller than those of the 128 x 64 tiles that the product alone takes, three to a CU.  Measured against the
-// product and the normalisation by themselves, fp16, us (first figure a depth of n, second of 4 n):
-//   401408 x 64 49 -> 33, 86 -> 67; x 112 95 -> 60, 155 -> 127; 100352 x 160 40 -> 26, 59 -> 47; x 224 50 -> 49, 104 -> 108;
-//   25088 x 256 21 -> 19, 35 -> 30; 16384 x 128 9.6 -> 6.6, 12.0 -> 10.2
-//   25088 (77 % of a round) x 320 (64 % of the tiles' rounds) 26 -> 19, 46 -> 37; x 512 (68 %) 39 -> 37, 91 -> 77;
-//   x 448 (89 %) 32 -> 30, 66 -> 65, in a model 28 -> 32, 66 -> 70; 12544 (38 %) x 448 (89 %) 20 -> 28, 36 -> 58
-bool rows_fits(int dtype, long long rows, int n, int k) {
+// Where enough workgroups are there, by how many a CU holds: two and more up to 256 features, and beyond one, whose last round must not
+// be half empty; from the second round on what a rest may be differs by width, and six sevenths are full enough for all.  With
+// after_residual two tensors leave, and more is needed above 160 features.  Measured against the product, in the tile that launch_t of linear.hip gives it, and the normalisation by themselves,
+// fp16, time as a share of theirs: behind the product at a depth of n, of 4 n, | with after_residual at a depth of n.
+//   workgroups    64 features       112              160              192              224              256
+//      128      0.68 0.77|0.83  0.78 0.84|0.85  0.83 0.99|0.95  0.89 1.04|1.06  0.95 1.14|1.06  0.99 1.15|1.19
+//      160      0.63 0.73|0.80  0.74 0.79|0.82  0.76 0.90|0.89  0.82 0.94|1.00  0.81 0.92|0.91  0.87 0.88|1.05
+//      196                                      0.68 0.80|0.82  0.75 0.79|0.92                  0.72 0.73|0.81
+//      392                                                      0.67 0.86|0.86  0.67 0.73|0.72  0.68 0.74|0.76
+//      784                                      0.63 0.78|0.77  0.69 0.84|0.85  0.73 0.87|0.90  0.78 0.89|0.91
+//   rounds        320               384              448              512
+//      0.59     0.94 1.00|1.10  0.86 0.84|0.98  0.89 0.95|0.96  0.85 0.93|0.93
+//      0.64     0.76 0.77|0.85  0.89 0.82|0.96  0.81 0.93|0.90  0.83 0.91|0.88
+//      0.77     0.76 0.74|0.84  0.71 0.81|0.78  0.77 0.86|0.84  0.73 0.77|0.77
+//      1.29     0.90 1.11|1.04  0.99 1.20|1.14  0.99 1.17|1.06  1.02 1.15|1.12
+//      1.53     0.75 0.87|0.86  0.82 0.94|0.93  0.88 1.00|0.93  0.94 0.99|0.98
+//      1.83     0.70 0.84|0.82                  0.81 0.90|0.89  0.85 0.90|0.92
+//      2.50     0.79 0.94|0.94  0.87 1.00|1.01  0.92 1.02|0.97  0.94 1.03|1.02
+//      2.73     0.73 0.82|0.85  0.81 0.87|0.88  0.84 0.91|0.87  0.85 0.91|0.89
+//      3.06     0.85 1.00|0.98  0.93 1.06|1.05  0.93 1.03|0.97  0.97 1.05|1.00
+//      3.52     0.76 0.87|0.88  0.82 0.92|0.92  0.88 0.92|0.88  0.88 0.92|0.92
+// (100352 x 224 47 us for 65, at 896 93 for 107; 25088 x 448 32 for 41, at 1792 73 for 84; 25088 x 512 36 for 49, at 2048 84 for 109)
+bool rows_fits(int dtype, long long rows, int n, int k, bool after_residual) {
   if ((dtype != F16::kCode && dtype != BF16::kCode) || n <= 0 || n % 8 != 0 || n > kRowsMost || k <= 0 || k % 8 != 0 || k > (1 << 20) || rows <= 0 || rows >= (1ll << 31))
     return false;
   const long long workgroups = (rows + kRowsTile - 1) / kRowsTile;
-  if (n <= 256) return workgroups >= kCus / 2;
-  auto full = [](long long count, long long round) { return (double)count / (double)((count + round - 1) / round * round); };
-  return full(workgroups, kCus) > full(workgroups * ((n + 63) / 64), 3 * kCus);
+  if (n <= 256) return 8 * workgroups >= (n <= 160 ? 4 : after_residual ? 6 : 5) * kCus;
+  if (workgroups <= kCus) return 5 * workgroups >= 3 * kCus;
+  return 7 * workgroups >= 6 * ((workgroups + kCus - 1) / kCus * kCus);
 }
 
 hipError_t launch_rows(int dtype, const RowsLaunch &p, hipStream_t stream) {
