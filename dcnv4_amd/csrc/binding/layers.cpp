@@ -340,9 +340,28 @@ PyObject *py_rows_fits(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// weight_grad_plan(x, widths): tile side and splits of the weight gradients of linear layers over the rows of x in one launch
+PyObject *py_weight_grad_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("weight_grad_plan", args, n, 2);
+  const Tensor &x = a.tensor(), widths = a.tensor().cpu();
+  WeightGradLaunch launch = {};
+  if (x.dim() != 2 || widths.scalar_type() != at::kLong || widths.numel() < 1 || widths.numel() > kMaxWeightGrads) raise_runtime("a matrix and one to %d widths", kMaxWeightGrads);
+  launch.rows = x.size(0);
+  for (; launch.count < (int)widths.numel(); ++launch.count) {
+    launch.p[launch.count].n = (int)widths.data_ptr<int64_t>()[launch.count];
+    launch.p[launch.count].k = (int)x.size(1);
+    if (launch.p[launch.count].n < 1 || x.size(1) < 1) raise_runtime("widths and depth are positive");
+  }
+  const WeightGradPlan plan = plan_weight_grad(dtype_code(x, "input"), launch);
+  return Py_BuildValue("ii", plan.tile, plan.splits);
+  END_HANDLE_TH_ERRORS
+}
+
 }  // namespace
 
 PyMethodDef layer_methods[] = {
+    {"weight_grad_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_weight_grad_plan)), METH_FASTCALL, nullptr},
     {"rows_fits", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_rows_fits)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear)), METH_FASTCALL, nullptr},
     {"layer_inference", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_layer_inference)), METH_FASTCALL, nullptr},
