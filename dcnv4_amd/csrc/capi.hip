@@ -747,7 +747,6 @@ int static_scratch_of_current_device(void **out) {
 // above, by what fits a strip.
 constexpr int kNearReach = 5;
 bool far_lists_fit(const DcnLaunch &L, const DcnProblem &pr, const void *grad_value, std::initializer_list<std::pair<const void *, size_t>> others) {
-  if (L.H / L.tile_h >= 0xffff || L.W / L.tile_w >= 0xffff) return false;      // tiles are named by 16 bits each way
   auto visited = [](int extent, int tile, int reach) {      // rows (columns) over all tiles
     double sum = 0.;
     for (int at = 0; at < extent; at += tile) sum += std::min(extent, at + tile + reach) - std::max(0, at - reach);

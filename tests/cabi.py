@@ -28,7 +28,8 @@ def dcnv4_forward(value, om, geom, G, D, scale, rc=0, softmax=0, im2col_step=256
     return out
 
 
-def dcnv4_backward(value, om, go, geom, G, D, scale, rc=0, softmax=0, im2col_step=256, d_stride=0, block_thread=0):
+def dcnv4_backward(value, om, go, geom, G, D, scale, rc=0, softmax=0, im2col_step=256, d_stride=0, block_thread=0, state=None):
+    """state: a list that receives the workspace as 32-bit words."""
     L = _lib.load()
     B, H, W, _ = value.shape
     gv = torch.full_like(value, float("nan"))
@@ -39,6 +40,8 @@ def dcnv4_backward(value, om, go, geom, G, D, scale, rc=0, softmax=0, im2col_ste
                                   ws.data_ptr(), nbytes, CODES[value.dtype], B, H, W, G, D, *geom, float(scale),
                                   im2col_step, rc, om.shape[-1], softmax, d_stride, block_thread, _stream())
     _lib.check(rc_)
+    if state is not None:
+        state.append(ws[:nbytes // 4 * 4].view(torch.int32))
     return gv, gom
 
 
