@@ -1,9 +1,10 @@
 """Products wide and many-rowed enough for the 256 x 128 tile (448 of them and more): remainders of rows, features and depth, one slice
-and many, two products in a launch by way of a layer, every epilogue.  Against fp32."""
+and many, and the inference epilogues, against fp32; two products in a launch and what training adds to the epilogue by way of a
+layer, against its composition."""
 import pytest
 import torch
 
-from tests.test_gpu_layers import _rel
+from tests.test_gpu_layers import _composed, _rel
 
 pytestmark = pytest.mark.gpu
 
@@ -22,3 +23,24 @@ def test_wide_products_match_fp32(rows, depth, width, dtype):
     want = torch.nn.functional.gelu(product + b.float())
     assert _rel(ext.linear_forward(a, w, b, gelu=True), want) < tol
     assert _rel(ext.linear_forward(a, w, b, gamma, res, gelu=True), want * gamma.float() + res.float()) < tol
+
+
+# 56 tiles of rows, the last one short, by 8 of both projections' features (320 and 540) and by 10 of the hidden ones (1280)
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 3e-3), (torch.bfloat16, 2e-2)], ids=["fp16", "bf16"])      # as in test_gpu_layers.py
+def test_layer_training_in_wide_products_matches_the_composition(dtype, tol):
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    torch.manual_seed(3)
+    layer = InternImageLayer(320, 20, post_norm=True, layer_scale=0.3, dcn_output_bias=True, mlp_fc2_bias=True).cuda()
+    with torch.no_grad():
+        layer.dcn.offset_mask.weight.normal_(0, 0.02)
+        layer.dcn.offset_mask.bias.normal_(0, 0.5)
+    x, grad = torch.randn(2, 5, 2862, 320, device="cuda").unbind()
+    results = []
+    for run in (layer, lambda *a: _composed(layer, *a)):
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=dtype):
+            out = run(xi, (54, 53))
+        results.append([out.detach(), *torch.autograd.grad(out, [xi, *layer.parameters()], grad)])
+    assert results[0][0].dtype == results[1][0].dtype
+    for name, got, want in zip(["output", "x"] + [k for k, _ in layer.named_parameters()], *results):
+        assert got.dtype == want.dtype and _rel(got, want) < tol, (name, _rel(got, want))
