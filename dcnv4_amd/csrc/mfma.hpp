@@ -76,11 +76,13 @@ __device__ __forceinline__ NormalTail normal_tail(float x) {
   r.tail = p * r.bell;
   return r;
 }
-// Phi(-|x|) = 2^P(|x|), P of degree 10 fitted the same way where an fp16 result sees it: to 4.7e-8 of Phi down to |x| = 4.2, from there
-// to 4.7e-8 of the first subnormal's spacing; P falls without end beyond.  16 bits of result need no more, and without the reciprocal
-// and the bell's argument it takes 14 issue slots in place of 20.  Of 10 million inputs 920 round to another fp16 than the exact value
-// (normal_tail: 1023), of all fp16 inputs 3 (6).  A model whose MLPs' epilogues are bound by these instructions, 128 pictures: 10.76 ->
-// 10.49 ms.  bf16 reaches 1e-38, where no such P is close enough.
+// Phi(-|x|) = 2^P(|x|), P of degree 10 fitted the same way where an fp16 result sees it: relative to Phi down to |x| = 4.2, from there
+// to the first subnormal's spacing; P falls without end beyond.  With its coefficients rounded to fp32 it is within 1e-7 of Phi there
+// and within 1.3e-6 computed in fp32; beyond it is off by 1.8e-6 up to 5, 4e-4 up to 6 and 13 % up to 8, of a subnormal result and at
+// most 5e-5 of the spacing.  16 bits of result need no more (a layer scale in the tens of thousands behind it would show it), and without
+// the reciprocal and the bell's argument it takes 14 issue slots in place of 20.  Of 10 million inputs 920 round to another fp16 than
+// the exact value (normal_tail: 1023), of all fp16 inputs 3 (6).  A model whose MLPs' epilogues are bound by these instructions, 128
+// pictures: 10.76 -> 10.49 ms.  bf16 reaches 1e-38, where no such P is close enough.
 __device__ __forceinline__ float normal_tail_fp16(float x) {
   const float a = fabsf(x);
   float p = -2.7233665989001565e-08f;
