@@ -329,6 +329,26 @@ PyObject *py_layer_inference(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linear_tile(x, widths, result32): rows and features of the tile that one or two products of x in a launch take
+PyObject *py_linear_tile(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("linear_tile", args, n, 3);
+  const Tensor &x = a.tensor(), widths = a.tensor().cpu();
+  float result32;
+  const bool wants32 = a.integer() != 0;
+  LinearLaunch p = {};
+  if (x.dim() != 2 || widths.scalar_type() != at::kLong || widths.numel() < 1 || widths.numel() > 2) raise_runtime("a matrix and one or two widths");
+  p.rows = x.size(0); p.k = (int)x.size(1);
+  for (; p.count < (int)widths.numel(); ++p.count) {
+    p.p[p.count].n = (int)widths.data_ptr<int64_t>()[p.count];
+    if (wants32) p.p[p.count].out32 = &result32;
+    if (!linear_fits(dtype_code(x, "input"), p.rows, p.p[p.count].n, p.k)) raise_runtime("linear takes a depth and width in multiples of 8");
+  }
+  const LinearTile tile = linear_tile(dtype_code(x, "input"), p);
+  return Py_BuildValue("ii", tile.rows, tile.features);
+  END_HANDLE_TH_ERRORS
+}
+
 // rows_fits(x, width, after_residual): whether a product x @ [width, k].T and the normalisation behind it are one kernel
 PyObject *py_rows_fits(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -363,6 +383,7 @@ PyObject *py_weight_grad_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
 
 PyMethodDef layer_methods[] = {
     {"weight_grad_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_weight_grad_plan)), METH_FASTCALL, nullptr},
+    {"linear_tile", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear_tile)), METH_FASTCALL, nullptr},
     {"rows_fits", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_rows_fits)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear)), METH_FASTCALL, nullptr},
     {"layer_inference", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_layer_inference)), METH_FASTCALL, nullptr},

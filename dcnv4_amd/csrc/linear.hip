@@ -500,29 +500,48 @@ hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
 //     73.5 -> 70.1 (1372), 100352 x 608 x 224 58.1 -> 47.6 (1960), 401408 x 304 x 112 120 -> 110; below: 25088 x 448 x 1792 56.0 -> 61.3 (392),
 //     6272 x 896 x 3584 53.6 -> 63.8 (175).  Padding to 128 features costs less than it saves up to 80 per cent (401408 x 216 x 80
 //     77 -> 62); 64 features take 256x64: 401408 x 64 x 64 23.3 against 25.3
-template <typename Tag, bool EXTRA>
-hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
-  auto tiles = [&](int bm, int bn) {
+//   Not where the second round of two workgroups a CU is a sixth or less and the narrow tile pads less: 26624 x (320 + 216) x 448 22.7 ->
+//     27.4 (520 tiles), 17920 x (448 + 432) x 640 31.6 -> 38.0, 35840 x 448 x 192 16.7 -> 18.7 (560), 50176 x 320 x 320 20.7 -> 23.8, 50176 x
+//     (112 + 192) x 112 14.9 -> 16.7 (588); from a fifth on 39680 x 448 x 448 38.0 -> 35.0, 22511 x (320 + 432) x 224 22.4 -> 19.6.  Nor for results in fp32
+//     (onto a residual in fp32) where the narrow tile pads a quarter less: 200704 x 192 x 192 92.2 -> 103.7, x 160 x 640 139.7 -> 150.8.  Over 800 products of
+//     448 tiles and more the wide tile takes 0.91 of the others' time; a depth of 112, whose slices share lines, without an activation 0.84
+//     to 1.1.
+LinearTile plan_linear(int dtype, const LinearLaunch &p) {
+  auto tiles = [&](long long bm, int bn) {
     long long n = 0;
     for (int i = 0; i < p.count; ++i) n += (p.p[i].n + bn - 1) / bn;
     return n * ((p.rows + bm - 1) / bm);
   };
+  if (tiles(64, 64) < 64 || p.norm.weight != nullptr) return {kFewTile, kFewTile};
   // fp32 is bound by the matrix cores (157 TFLOP/s): the tile that spreads most evenly
-  if (tiles(64, 64) < 64 || p.norm.weight != nullptr) return launch_few<Tag, EXTRA>(p, stream);
+  if (dtype == F32::kCode || tiles(128, 64) < kCus) return {64, 64};
+  int features = 0;
+  for (int i = 0; i < p.count; ++i) features += p.p[i].n;
+  const long long wide = tiles(kWideRows, kWideFeatures), padded = tiles(p.rows, kWideFeatures) * kWideFeatures, narrow = tiles(p.rows, 64) * 64;
+  const bool thin = wide > 2 * kCus && wide <= 2 * kCus * 7 / 6 && 10 * padded > 11 * narrow;
+  const bool result32 = (p.p[0].out32 != nullptr || (p.count > 1 && p.p[1].out32 != nullptr)) && 4 * narrow <= 3 * padded;
+  if (wide >= 2 * kCus * 7 / 8 && 5 * padded <= 9 * features && !thin && !result32) return {kWideRows, kWideFeatures};
+  if (tiles(128, 128) < 4 * kCus) return {128, 64};
+  return {256, 64};
+}
+
+template <typename Tag, bool EXTRA>
+hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
+  const LinearTile tile = plan_linear(Tag::kCode, p);
+  if (tile.rows == kFewTile) return launch_few<Tag, EXTRA>(p, stream);
+  if (tile.rows == 64) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
   if constexpr (Tag::kBytes == 4) {
-    return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
+    return hipErrorInvalidValue;
   } else {
-    if (tiles(128, 64) < kCus) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
-    int features = 0;
-    for (int i = 0; i < p.count; ++i) features += p.p[i].n;
-    const long long wide = tiles(kWideRows, kWideFeatures), padded = tiles(1 << 30, kWideFeatures) * kWideFeatures;
-    if (wide >= 2 * kCus * 7 / 8 && 5 * padded <= 9 * features) return launch_wide<Tag, EXTRA>(p, stream);
-    if (tiles(128, 128) < 4 * kCus) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
+    if (tile.features == kWideFeatures) return launch_wide<Tag, EXTRA>(p, stream);
+    if (tile.rows == 128) return launch_tiled<Tag, EXTRA, 128, 64, 4, 1>(p, stream);
     return launch_tiled<Tag, EXTRA, 256, 64, 4, 1>(p, stream);
   }
 }
 
 }  // namespace
+
+LinearTile linear_tile(int dtype, const LinearLaunch &p) { return plan_linear(dtype, p); }
 
 bool linear_fits(int dtype, long long rows, int n, int k) {
   return (dtype == F32::kCode || dtype == F16::kCode || dtype == BF16::kCode) && rows > 0 && n > 0 && k > 0 && n % 8 == 0 && k % 8 == 0 && k <= (1 << 20) &&

@@ -56,6 +56,9 @@ bool linear_fits(int dtype, long long rows, int n, int k);
 // Whether the rows may come normalised: few enough that a workgroup normalising its own costs less than a launch.
 bool linear_takes_norm(const LinearLaunch &p);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
+// The tile of launch_linear's kernel: 32 x 32 few rows, 256 x 128 the wide one.
+struct LinearTile { int rows, features; };
+LinearTile linear_tile(int dtype, const LinearLaunch &p);
 
 // What follows a product in a layer together with its normalisation (16-bit types), every step rounded as the kernels one by one round
 // it: after_residual  stream = gamma * (product + bias) + residual, normed = norm(stream); else the product rounded to the type and

@@ -9,10 +9,27 @@ from tests.test_gpu_layers import _composed, _rel
 pytestmark = pytest.mark.gpu
 
 
+def _tile(rows, depth, *widths, result32=0):
+    from dcnv4_amd import ext
+    return ext._native.linear_tile(torch.empty(rows, depth, dtype=torch.float16, device="meta"), torch.tensor(widths), result32)
+
+
+def test_the_wide_tile_is_taken_where_it_pays():
+    """From 448 tiles on, up to 80 per cent of padding; not with a second round of a sixth or less, nor for results in fp32, where the
+    tile of 64 features pads less."""
+    assert _tile(56 * 256, 64, 1024) == (256, 128) and _tile(56 * 256 - 256, 64, 1024) == (128, 64)
+    assert _tile(401408, 64, 64) == (256, 64) and _tile(401408, 64, 72) == (256, 128)
+    # 512 tiles of two workgroups a CU: 513 to 597 of them
+    assert _tile(171 * 256 - 256, 64, 320) == (256, 128) and _tile(171 * 256, 64, 320) == (256, 64) == _tile(199 * 256, 448, 320) and _tile(200 * 256, 64, 320) == (256, 128)
+    assert _tile(104 * 256, 448, 320, 216) == (256, 64) and _tile(130 * 256, 448, 512) == (256, 128)
+    assert _tile(200704, 192, 192) == _tile(200704, 192, 256, result32=1) == _tile(200704, 192, 320, result32=1) == (256, 128) != _tile(200704, 192, 192, result32=1)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
 @pytest.mark.parametrize("rows,depth,width", [(57601, 72, 264), (57400, 8, 144), (57345, 32, 256), (19201, 200, 776), (28800, 96, 512), (9000, 104, 1792)])
 def test_wide_products_match_fp32(rows, depth, width, dtype):
     from dcnv4_amd import ext
+    assert _tile(rows, depth, width) == (256, 128)
     g = torch.Generator(device="cuda").manual_seed(rows)
     rand = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
     a, w, b, gamma, res = rand(rows, depth), rand(width, depth) / depth ** 0.5, rand(width), rand(width), rand(rows, width)
@@ -34,6 +51,7 @@ def test_layer_training_in_wide_products_matches_the_composition(dtype, tol):
     with torch.no_grad():
         layer.dcn.offset_mask.weight.normal_(0, 0.02)
         layer.dcn.offset_mask.bias.normal_(0, 0.5)
+    assert _tile(14310, 320, 320, 544) == _tile(14310, 320, 1280) == (256, 128)
     x, grad = torch.randn(2, 5, 2862, 320, device="cuda").unbind()
     results = []
     for run in (layer, lambda *a: _composed(layer, *a)):
