@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(HERE, "libdcnv4_gfx950.so")
 SOURCES = ["capi.hip", "dcnv4_kernels.hip", "dcnv4_tiled_gather.hip", "dcnv4_window.hip", "dcnv4_grad_value.hip", "dcnv4_backward_dual.hip", "fda_kernels.hip", "fda_grad_value.hip",
            "depthwise_conv.hip", "layer_norm.hip", "center_feature.hip",
            "linear.hip", "linear_rows.hip", "linear_grad.hip", "mlp.hip", "conv.hip"]
-HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "mfma.hpp"), os.path.join(CSRC, "fragments.hpp"), os.path.join(CSRC, "layer_norm.hpp"), os.path.join(CSRC, "linear.hpp"), os.path.join(CSRC, "conv.hpp"), os.path.join(CSRC, "launch.hpp"),
+HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "mfma.hpp"), os.path.join(CSRC, "fragments.hpp"), os.path.join(CSRC, "dcnv4_at_once.hpp"), os.path.join(CSRC, "layer_norm.hpp"), os.path.join(CSRC, "linear.hpp"), os.path.join(CSRC, "conv.hpp"), os.path.join(CSRC, "launch.hpp"),
            os.path.join(CSRC, "dcnv4_tiled_gather.hpp"), os.path.join(CSRC, "dcnv4_window.hpp"), os.path.join(CSRC, "dcnv4_grad_value.hpp"),
            os.path.join(os.path.dirname(HERE), "include", "dcnv4_gfx950.h")]
 

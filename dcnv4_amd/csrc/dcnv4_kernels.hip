@@ -14,29 +14,10 @@
 // tensor needs no separate clearing); the value gradient is the tiled gather of dcnv4_grad_value.hip.
 #include <algorithm>
 
-#include "common.hpp"
-#include "launch.hpp"
+#include "dcnv4_at_once.hpp"
 
 namespace dcn {
 namespace {
-
-struct PixelGeom {
-  float x_base, y_base;   // tap (0,0) position before the learned offset, dcnv4_im2col_cuda.cuh:203-210
-  uint32_t img_base;      // byte offset of this image + this lane's channels
-};
-
-template <typename Tag>
-__device__ __forceinline__ PixelGeom pixel_geometry(const DcnLaunch &p, int pix, int g, int chunk) {
-  const int b = pix / p.Q, q = pix - b * p.Q;
-  const int ho = q / p.Wo, wo = q - ho * p.Wo;
-  const int half_w = (p.dw * (p.kw - 1)) >> 1, half_h = (p.dh * (p.kh - 1)) >> 1;
-  PixelGeom geo;
-  geo.x_base = sub_rn((float)(half_w - p.pw + wo * p.sw), mul_rn((float)half_w, p.offset_scale));
-  geo.y_base = sub_rn((float)(half_h - p.ph + ho * p.sh), mul_rn((float)half_h, p.offset_scale));
-  geo.img_base = ((uint32_t)b * (uint32_t)(p.H * p.W) * (uint32_t)(p.G * p.D) +
-                  (uint32_t)(g * p.D + chunk * p.lanes.cpt)) * Tag::kBytes;
-  return geo;
-}
 
 // ------------------------------------------------------------------------------- forward
 template <typename Tag, int CPT, int KP>
@@ -112,60 +93,22 @@ __global__ void __launch_bounds__(kBlockThreads) dcnv4_forward_kernel(const DcnL
   }
 }
 
-// Small calls, a 3x3 kernel in 16-byte vectors: too few waves to hide a latency behind each other, so a lane asks for everything
-// it needs at once - its row of offsets straight from memory, then the 36 corners of its nine taps - and waits twice.
-// 1x14x14, 16 groups of 16, fp16, behind another kernel: 7.8 us with the kernel above, whose 56 registers hold two taps' corners
-// at a time.
-template <typename Tag, int CPT>
+// Small calls, a 3x3 kernel in 16-byte vectors (dcnv4_at_once.hpp).  1x14x14, 16 groups of 16, fp16, behind another kernel: 7.8 us with
+// the kernel above, whose 56 registers hold two taps' corners at a time.
+template <typename Tag, int CPT, int SHARE>
 __global__ void __launch_bounds__(kBlockThreads, 2) dcnv4_forward_small_kernel(const DcnLaunch p) {
   typedef Pack<Tag, CPT> pack;
   const __amdgpu_buffer_rsrc_t value = make_rsrc(p.value, p.value_bytes);
-  const int tpg = p.lanes.tpg, per_pixel = p.G * tpg;
-  const int it = (int)(xcd_contiguous_block(blockIdx.x, gridDim.x) * kBlockThreads + threadIdx.x);
+  const int tpg = p.lanes.tpg, per_pixel = p.G * tpg, part = threadIdx.x % SHARE;
+  const int it = (int)(xcd_contiguous_block(blockIdx.x, gridDim.x) * (kBlockThreads / SHARE) + threadIdx.x / SHARE);
   const int pix = it / per_pixel, gc = it - pix * per_pixel, g = gc / tpg, chunk = gc - g * tpg;
   if (pix >= p.n_pix) return;
-  uint32_t raw_row[(27 * Tag::kBytes + 3) / 4];
-  __builtin_memcpy(raw_row, static_cast<const char *>(p.offset_mask) + ((size_t)pix * p.P_pad + (size_t)g * 27) * Tag::kBytes, 27 * Tag::kBytes);
-  auto element = [&](int e) {
-    if constexpr (Tag::kBytes == 4) {
-      return __builtin_bit_cast(float, raw_row[e]);
-    } else {
-      float f[2];
-      Pack<Tag, 2>::decode(raw_row[e >> 1], f);
-      return f[e & 1];
-    }
-  };
-  const PixelGeom geo = pixel_geometry<Tag>(p, pix, g, chunk);
-  const uint32_t pix_bytes = (uint32_t)(p.G * p.D) * Tag::kBytes;
-  typename pack::raw_t raw[9][4];
-  float w[9][4];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const float x = add_rn(geo.x_base, mul_rn(add_rn((float)(k / 3 * p.dw), element(2 * k)), p.offset_scale));
-    const float y = add_rn(geo.y_base, mul_rn(add_rn((float)(k % 3 * p.dh), element(2 * k + 1)), p.offset_scale));
-    const float m = element(18 + k);
-    const Tap t = make_tap(y, x, p.H, p.W, geo.img_base, pix_bytes);
-#pragma unroll
-    for (int cn = 0; cn < 4; ++cn) {
-      raw[k][cn] = buffer_load<pack::kBytes>(value, t.off[cn]);
-      w[k][cn] = m * t.w[cn];
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
+  TapShare<Tag, SHARE> taps;
+  taps.request(p, pix, g, part);
   float acc[CPT];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) acc[c] = 0.f;
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-#pragma unroll
-    for (int cn = 0; cn < 4; ++cn) {
-      float v[CPT];
-      pack::decode(raw[k][cn], v);
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) acc[c] = fmaf(w[k][cn], v[c], acc[c]);
-    }
+  taps.sample(p, value, pix, g, chunk, part, acc);
   char *dst = static_cast<char *>(p.out) + ((size_t)pix * per_pixel + gc) * pack::kBytes;
-  *reinterpret_cast<typename pack::raw_t *>(dst) = pack::encode(acc);
+  if (part == 0) *reinterpret_cast<typename pack::raw_t *>(dst) = pack::encode(acc);
 }
 
 // ------------------------------------------------------------------------------- backward
@@ -366,12 +309,20 @@ size_t dcnv4_backward_lds_bytes(const DcnLaunch &p) { return 2 * dcnv4_forward_l
 hipError_t launch_dcnv4_forward(int dtype, const DcnLaunch &p, hipStream_t stream) {
   return launch_by_dtype<false>(dtype, p, stream);
 }
+// Where the chip stays empty enough a quad shares a lane's nine taps.  Behind each other in a graph, us, a lane | a quad: 3136 16-byte
+// vectors (1x7x7, 32 groups of 16, fp16) 4.04 | 3.33, 6272 4.10 | 3.45, 12544 4.14 | 3.50, 25088 4.17 | 4.18 (fp32 3.70 | 4.25), 50176 4.23 | 5.99.
+constexpr int64_t kSharedItems = 16384;
 hipError_t launch_dcnv4_forward_small(int dtype, const DcnLaunch &p, hipStream_t stream) {
-  const dim3 grid((unsigned)(((int64_t)p.n_pix * p.G * p.lanes.tpg + kBlockThreads - 1) / kBlockThreads)), block(kBlockThreads);
-  if (dtype == F32::kCode) hipLaunchKernelGGL((dcnv4_forward_small_kernel<F32, 4>), grid, block, 0, stream, p);
-  else if (dtype == F16::kCode) hipLaunchKernelGGL((dcnv4_forward_small_kernel<F16, 8>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((dcnv4_forward_small_kernel<BF16, 8>), grid, block, 0, stream, p);
-  return hipGetLastError();
+  const int64_t items = (int64_t)p.n_pix * p.G * p.lanes.tpg;
+  const int share = items <= kSharedItems ? 4 : 1;
+  const dim3 grid((unsigned)((items * share + kBlockThreads - 1) / kBlockThreads)), block(kBlockThreads);
+  auto go = [&](auto one, auto four) {
+    hipLaunchKernelGGL(share == 1 ? one : four, grid, block, 0, stream, p);
+    return hipGetLastError();
+  };
+  if (dtype == F32::kCode) return go(dcnv4_forward_small_kernel<F32, 4, 1>, dcnv4_forward_small_kernel<F32, 4, 4>);
+  if (dtype == F16::kCode) return go(dcnv4_forward_small_kernel<F16, 8, 1>, dcnv4_forward_small_kernel<F16, 8, 4>);
+  return go(dcnv4_forward_small_kernel<BF16, 8, 1>, dcnv4_forward_small_kernel<BF16, 8, 4>);
 }
 hipError_t launch_dcnv4_offset_mask_grad(int dtype, const DcnLaunch &p, hipStream_t stream) {
   return launch_by_dtype<true>(dtype, p, stream);
