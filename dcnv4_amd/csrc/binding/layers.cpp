@@ -3,8 +3,9 @@
 //
 // A picture or a few are bound by the host: 415 launches through Python took 6.5 ms for a T variant whose kernels run
 // 2.2 ms.  Here a layer is seven (pre-norm) or eight launches: the two projections in front of the operator share one,
-// bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.  With rows enough it is fewer: a product
-// takes the normalisation behind it (rows_fits), one kernel the MLP (mlp_fits).
+// bias, GELU, layer scale and the pre-norm residual are epilogues of the matrix products.  Of a handful of pixels it is fewer - a
+// normalisation goes with the product behind it (linear_takes_norm), the operator with its projection (launch_sampled_linear) - and of
+// many: a product takes the normalisation behind it (rows_fits), one kernel the MLP (mlp_fits).
 #include <cmath>
 
 #include <ATen/SavedTensorHooks.h>
@@ -228,8 +229,16 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
   both.count = 2; both.rows = rows; both.k = (int)c;
   if (norm_first) normed(both, l.norm1, Tensor(), nullptr, middle);
   else launch(code, both, stream);
-  check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
-                             l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
+  // the operator; its output projection may go with it
+  LinearProblem output = {sampled, ptr(l.output_w), ptr(l.output_b), nullptr, nullptr, last, (int)c};
+  if (!l.post_norm) { output.gamma = ptr(l.gamma1); output.residual = in; }
+  const SampledLinear sampling = {value, offsets, batch, h, w, l.group, l.group_channels, l.kernel, l.pad, l.dilation, l.remove_center, (int)l.row, l.offset_scale, output};
+  const bool projected = !whole_rows && sampled_linear_fits(code, sampling);
+  if (projected)
+    hip_check(launch_sampled_linear(code, sampling, static_cast<hipStream_t>(stream)), "DCNv4 with its projection launch");
+  else
+    check(dcnv4_gfx950_forward(value, offsets, sampled, code, batch, h, w, l.group, l.group_channels, l.kernel, l.kernel, 1, 1, l.pad,
+                               l.pad, l.dilation, l.dilation, l.offset_scale, 256, l.remove_center, (int)l.row, 0, 0, 0, stream));
   const bool fused = mlp_fits(code, rows, (int)c, (int)l.hidden);      // the MLP in one kernel
   auto mlp = [&](const Tensor &gamma, const void *residual, void *o, const NormParams *n) {
     MlpLaunch m = {middle, ptr(l.fc1_w), ptr(l.fc1_b), ptr(l.fc2_w), ptr(l.fc2_b), ptr(gamma), residual, o, rows, (int)c, (int)l.hidden, {}};
@@ -244,7 +253,7 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
       rows_normed(sampled, l.output_w, l.output_b, c, l.norm1, l.gamma1, in, middle, nullptr);
       fc1.p[0].a = middle;
     } else {
-      linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
+      if (!projected) linear(sampled, l.output_w, l.output_b, c, c, false, Tensor(), nullptr, last);
       if (fused) norm(last, l.norm1, l.gamma1, in, middle);
     }
     if (fused) {
@@ -264,7 +273,7 @@ Tensor layer_inference(const Layer &l, const Tensor &x, int batch, int h, int w)
       rows_normed(sampled, l.output_w, l.output_b, c, l.norm2, l.gamma1, in, last, middle);
       fc1.p[0].a = middle;
     } else {
-      linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
+      if (!projected) linear(sampled, l.output_w, l.output_b, c, c, false, l.gamma1, in, last);
       if (fused) norm(last, l.norm2, Tensor(), nullptr, middle);
     }
     if (fused) {
@@ -361,6 +370,20 @@ PyObject *py_rows_fits(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// sampled_linear_fits(x, h, w, group, kernel): whether DCNv4 over x [batch, h * w, channels] and its output projection are one kernel
+PyObject *py_sampled_linear_fits(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("sampled_linear_fits", args, n, 5);
+  const Tensor &x = a.tensor();
+  const int h = a.integer(), w = a.integer(), group = a.integer(), kernel = a.integer();
+  if (x.dim() != 3 || group <= 0 || x.size(2) % group != 0) raise_runtime("rows of whole groups");
+  const int c = (int)x.size(2);
+  SampledLinear p = {nullptr, nullptr, (int)x.size(0), h, w, group, c / group, kernel, kernel / 2, 1, 0, (group * kernel * kernel * 3 + 7) / 8 * 8, 1.f, {}};
+  p.q.n = c;
+  return PyBool_FromLong(sampled_linear_fits(dtype_code(x, "input"), p));
+  END_HANDLE_TH_ERRORS
+}
+
 // weight_grad_plan(x, widths): tile side and splits of the weight gradients of linear layers over the rows of x in one launch
 PyObject *py_weight_grad_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -383,6 +406,7 @@ PyObject *py_weight_grad_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
 
 PyMethodDef layer_methods[] = {
     {"weight_grad_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_weight_grad_plan)), METH_FASTCALL, nullptr},
+    {"sampled_linear_fits", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_sampled_linear_fits)), METH_FASTCALL, nullptr},
     {"linear_tile", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear_tile)), METH_FASTCALL, nullptr},
     {"rows_fits", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_rows_fits)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_linear)), METH_FASTCALL, nullptr},

@@ -312,7 +312,7 @@ int plan_grad_value_tiles(DcnLaunch *L, int dtype, int batch) {
   return fail(DCNV4_ERR_RUNTIME, "kernel with %d taps and %d group channels does not fit the tiled backward", L->Kp, D);
 }
 
-constexpr uint64_t kSmallForwardBytes = 2800u << 10;      // outputs up to this size go by the kernels for small calls
+constexpr uint64_t kSmallForwardBytes = 2800u << 10;      // outputs up to this size go by the kernels for small calls (small_forward)
 
 bool tiled_gather_enabled() { return g_opt.gather != kOptPlain; }
 
@@ -762,6 +762,11 @@ bool far_lists_fit(const DcnLaunch &L, const DcnProblem &pr, const void *grad_va
   return true;
 }
 
+// Whether a forward goes by the kernels for small calls.
+bool small_forward(const DcnProblem &pr, int batch) {
+  return g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 && (uint64_t)batch * pr.img_out_elems * pr.s <= kSmallForwardBytes;
+}
+
 const char *at(const void *base, size_t elems, int s) { return static_cast<const char *>(base) + elems * s; }
 char *at(void *base, size_t elems, int s) { return static_cast<char *>(base) + elems * s; }
 
@@ -769,6 +774,29 @@ char *at(void *base, size_t elems, int s) { return static_cast<char *>(base) + e
 }  // namespace dcn
 
 namespace dcn {
+
+static bool prepare_sampled_linear(DcnProblem *pr, int dtype, const SampledLinear &p) {
+  if (dcn_prepare(pr, false, dtype, p.batch, p.height, p.width, p.group, p.group_channels, p.kernel, p.kernel, 1, 1, p.pad, p.pad, p.dilation,
+                  p.dilation, p.offset_scale, 256, p.remove_center, p.row, 0, 0, 0) != DCNV4_OK)
+    return false;      // the operator's own call says why
+  DcnLaunch &L = pr->launch;
+  L.value = p.value;
+  L.offset_mask = p.offsets;
+  L.value_bytes = (uint32_t)((size_t)p.batch * pr->img_elems * pr->s);
+  L.n_pix = p.batch * L.Q;
+  return small_forward(*pr, p.batch);
+}
+
+bool sampled_linear_fits(int dtype, const SampledLinear &p) {
+  DcnProblem pr;
+  return prepare_sampled_linear(&pr, dtype, p) && sampled_linear_fits(pr.launch, dtype, p.q.n);
+}
+
+hipError_t launch_sampled_linear(int dtype, const SampledLinear &p, hipStream_t stream) {
+  DcnProblem pr;
+  if (!prepare_sampled_linear(&pr, dtype, p)) return hipErrorInvalidValue;
+  return launch_sampled_linear(dtype, pr.launch, p.q, stream);
+}
 
 int prepare_layer_norm(LnLaunch *L, int dtype, long long rows, int channels, float eps) {
   const int s = elem_bytes(dtype);
@@ -855,8 +883,7 @@ int dcnv4_gfx950_forward(const void *value, const void *offset_mask, void *outpu
   // the direct one), where the others first stage a window behind a barrier.  Measured (fp16, us, small against window):
   // 1x56x56x64 4.3 against 5.7, 4x56x56x64 (1.6 MB) 6.1 against 7.3, 2x64x64x128 (2.1 MB) 5.4 against 8.1, 6x56x56x64 (2.4 MB)
   // 8.3 against 8.0, 4x64x64x128 (4.2 MB) 9.3 against 8.9.
-  const bool small = g_opt.gather == kOptAuto && g_opt.reach < 0 && g_opt.gather_tile == 0 &&
-                     (uint64_t)batch * pr.img_out_elems * pr.s <= kSmallForwardBytes;
+  const bool small = small_forward(pr, batch);
   const bool at_once = small && kernel_h == 3 && kernel_w == 3 && !remove_center && !softmax && pr.launch.lanes.cpt * pr.s == 16;
   const int window = small ? 0 : plan_window_gather(&pr.launch, pr.s, batch, false);
   const bool tiled = !small && window == 0 && plan_gather_tiles(&pr.launch, pr.s, false);

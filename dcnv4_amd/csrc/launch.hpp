@@ -312,6 +312,10 @@ hipError_t launch_depthwise_grad_weight_partials(int dtype, const DwLaunch &p, h
 hipError_t launch_depthwise_grad_weight_reduce(int dtype, const DwLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_forward_small(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_forward(int dtype, const DcnLaunch &p, hipStream_t stream);
+// DCNv4 and a product of n features behind it in one kernel (linear.hip); d.out is not used, nor q.a.
+struct LinearProblem;
+bool sampled_linear_fits(const DcnLaunch &d, int dtype, int n);
+hipError_t launch_sampled_linear(int dtype, const DcnLaunch &d, const LinearProblem &q, hipStream_t stream);
 hipError_t launch_dcnv4_offset_mask_grad(int dtype, const DcnLaunch &p, hipStream_t stream);
 hipError_t launch_dcnv4_grad_value(int dtype, const DcnLaunch &p, hipStream_t stream);
 // Both kernels of the backward as one launch with two workgroup roles, for shapes whose grad_value tiles are whole images

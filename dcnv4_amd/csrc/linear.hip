@@ -15,9 +15,11 @@
 //    four consecutive features of one row and stores 8 bytes.
 //  linear_few_rows_kernel: a picture or two at the later stages, where a launch has a handful of tiles and its time is load
 //    latency.  A workgroup owns 32 rows x 32 features; its four or eight waves share the depth between them, take their fragments
-//    straight from memory and meet in LDS once.  What the epilogue reads is requested first.  With a layer normalisation in
+//    straight from memory and meet in LDS once.  What the epilogue reads is requested first, the residual into registers of its own (with
+//    a pointer that was either it or memory it went through scratch memory: 0.7 us of a launch behind another).  With a layer normalisation in
 //    front the workgroup normalises its 32 rows itself, into LDS: each does so again for every 32 features, but a launch less
 //    is 3 us less for the device and as much for the host.
+#include "dcnv4_at_once.hpp"
 #include "fragments.hpp"
 #include "linear.hpp"
 #include "launch.hpp"
@@ -65,9 +67,9 @@ __device__ __forceinline__ void to_locations(const SamplingLocations &l, long lo
 
 // The epilogue for eight consecutive features of one row: 16 bytes in and out (32 of fp32).  EXTRA: with what training adds,
 // which costs the small tiles a third more registers.
-template <typename Tag, bool EXTRA>
-__device__ __forceinline__ void finish(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8],
-                                       const float *residual = nullptr) {      // residual: q.residual's values, where they are at hand
+// AT_HAND: residual holds q.residual's values, if there is one.
+template <typename Tag, bool EXTRA, bool AT_HAND>
+__device__ __forceinline__ void finish_with(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8], const float (&residual)[8]) {
   const LinearProblem &q = p.p[which];
   if (col.has_bias)
 #pragma unroll
@@ -91,14 +93,11 @@ __device__ __forceinline__ void finish(const LinearLaunch &p, int which, const C
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] *= s;
   }
-  if (residual != nullptr) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] += residual[c];
-  } else if (q.residual != nullptr) {
+  if (q.residual != nullptr) {
     float r[8];
-    load8<Tag>(q.residual, at, r);
+    if constexpr (!AT_HAND) load8<Tag>(q.residual, at, r);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] += r[c];
+    for (int c = 0; c < 8; ++c) v[c] += AT_HAND ? residual[c] : r[c];
   }
   if (EXTRA && q.residual32 != nullptr) {
     float r[8];
@@ -112,6 +111,11 @@ __device__ __forceinline__ void finish(const LinearLaunch &p, int which, const C
     for (int c = 0; c < 8; ++c) v[c] = 0.f;
   if (EXTRA && q.out32 != nullptr) store8<F32>(q.out32, at, v);
   else store8<Tag>(q.out, at, v);
+}
+
+template <typename Tag, bool EXTRA>
+__device__ __forceinline__ void finish(const LinearLaunch &p, int which, const Columns<Tag> &col, long long row, int n, float (&v)[8]) {
+  finish_with<Tag, EXTRA, false>(p, which, col, row, n, v, v);
 }
 
 template <typename Tag, int BM, int BN, int WM, int WN, bool EXTRA>
@@ -406,7 +410,7 @@ __global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const Linea
   const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
   const bool finishes = threadIdx.x < 128 && row < live_m && n < live_n;
   const Columns<Tag> columns(q, n0 + n, finishes);
-  float residual[8];
+  float residual[8] = {};
   if (finishes && q.residual != nullptr) load8<Tag>(q.residual, (size_t)(m0 + row) * q.n + n0 + n, residual);
   if constexpr (NORM > 0) {
     normalise_rows<Tag, NORM>(p, m0, live_m, first_tile, rows);
@@ -447,7 +451,102 @@ __global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const Linea
     for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4 *>(&part[w][row][n + c]);
     v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
   }
-  finish<Tag, EXTRA>(p, which, columns, m0 + row, n0 + n, v, q.residual != nullptr ? residual : nullptr);
+  finish_with<Tag, EXTRA, true>(p, which, columns, m0 + row, n0 + n, v, residual);
+}
+
+// DCNv4 (3x3) and the output projection behind it for few pixels.  A workgroup owns up to 16 pixels x 64 features: its lanes, a quad a
+// 16-byte vector, sample all channels of the pixels into LDS, each rounded to the type, while its share of the weights is on its
+// way; four waves and four more, half the depth each, then form the product.  Every 64 features the sampling is done again, which
+// costs nothing where the chip is empty; a launch in between would.  What bounds it is the chain: offsets, corners, LDS, product, LDS.
+constexpr int kSampledRows = 16, kSampledFeatures = 64, kSampledWaves = 8, kSampledSplits = kSampledWaves / 4, kSampledItems = kSampledWaves * 16;
+constexpr int kSampledDepth = 1024;      // of rows that fit the LDS a workgroup has without asking for more
+template <typename Tag>
+__global__ void __launch_bounds__(kSampledWaves * 64) sampled_linear_kernel(const DcnLaunch d, const LinearLaunch p, int tiles_n, int tile_rows) {
+  static_assert(Tag::kBytes == 2, "16-bit types");
+  constexpr int kTurn = kSampledFeatures + 4;
+  extern __shared__ u32x4 lds[];
+  float (*part)[kSampledRows][kTurn] = reinterpret_cast<float (*)[kSampledRows][kTurn]>(lds);
+  char *rows = reinterpret_cast<char *>(part + kSampledSplits);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
+  const LinearProblem &q = p.p[0];
+  const int m0 = tm * tile_rows, n0 = tn * kSampledFeatures, k = p.k;
+  const int live_m = min(tile_rows, d.n_pix - m0), live_n = min(kSampledFeatures, q.n - n0);
+  const __amdgpu_buffer_rsrc_t value = make_rsrc(d.value, d.value_bytes);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const uint16_t *>(q.w) + (size_t)n0 * k, (uint32_t)live_n * k * 2);
+
+  const int vectors = k / 8, items = live_m * vectors, tpg = d.lanes.tpg, quad = threadIdx.x & 3;
+  const float inv_vectors = __builtin_amdgcn_rcpf((float)vectors), inv_tpg = __builtin_amdgcn_rcpf((float)tpg);
+  auto place = [&](int it, int &pix, int &gc, int &g) {      // it < 2^20
+    pix = (int)(((float)it + 0.5f) * inv_vectors);
+    gc = it - pix * vectors;
+    g = (int)(((float)gc + 0.5f) * inv_tpg);
+  };
+  TapShare<Tag, 4> taps;
+  int pix, gc, g, it = threadIdx.x / 4;
+  place(it, pix, gc, g);
+  if (it < items) taps.request(d, m0 + pix, g, quad);
+
+  const int fragment = wave & 3, split = wave >> 2, r16 = lane & 15, kb = lane >> 4, steps = (k + 31) / 32;
+  constexpr int kTogether = 8;
+  u32x4 fn[kTogether];
+  auto request = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u) {
+      const int kk = (s0 + u * kSampledSplits) * 32 + kb * 8;
+      if (u == 0 || s0 + u * kSampledSplits < steps)
+        fn[u] = buffer_load<16>(rw, kk < k ? (uint32_t)((fragment * 16 + r16) * k + kk) * 2 : kDropOffset);
+    }
+  };
+  request(split);
+  const int out_row = threadIdx.x >> 3, n = (threadIdx.x & 7) * 8;
+  const bool finishes = threadIdx.x < 128 && out_row < live_m && n < live_n;
+  const Columns<Tag> columns(q, n0 + n, finishes);
+  float residual[8] = {};
+  if (finishes && q.residual != nullptr) load8<Tag>(q.residual, (size_t)(m0 + out_row) * q.n + n0 + n, residual);
+
+  while (it < items) {
+    float acc[8];
+    taps.sample(d, value, m0 + pix, g, gc - g * tpg, quad, acc);
+    if (quad == 0) *reinterpret_cast<u32x4 *>(rows + pix * norm_row_bytes(k) + gc * 16) = Pack<Tag, 8>::encode(acc);
+    it += kSampledItems;
+    place(it, pix, gc, g);
+    if (it < items) taps.request(d, m0 + pix, g, quad);
+  }
+  __syncthreads();
+
+  // rows beyond the live ones hold whatever the LDS held: theirs are columns of the result of their own, which go nowhere
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = split; s0 < steps; s0 += kTogether * kSampledSplits) {
+    if (s0 != split) request(s0);
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u) {
+      const int s = s0 + u * kSampledSplits, kk = s * 32 + kb * 8;
+      if (s >= steps) break;
+      const u32x4 fm = kk < k ? *reinterpret_cast<const u32x4 *>(rows + r16 * norm_row_bytes(k) + kk * 2) : u32x4{0u, 0u, 0u, 0u};
+      acc = mfma_64_bytes<Tag>(fn[u], fm, acc);
+    }
+  }
+  *reinterpret_cast<f32x4 *>(&part[split][r16][fragment * 16 + kb * 4]) = acc;
+  __syncthreads();
+  if (!finishes) return;
+  float v[8];
+#pragma unroll
+  for (int c = 0; c < 8; c += 4) {
+    f32x4 sum = *reinterpret_cast<const f32x4 *>(&part[0][out_row][n + c]);
+#pragma unroll
+    for (int s = 1; s < kSampledSplits; ++s) sum += *reinterpret_cast<const f32x4 *>(&part[s][out_row][n + c]);
+    v[c] = sum.x; v[c + 1] = sum.y; v[c + 2] = sum.z; v[c + 3] = sum.w;
+  }
+  finish_with<Tag, false, true>(p, 0, columns, m0 + out_row, n0 + n, v, residual);
+}
+
+template <typename Tag>
+hipError_t launch_sampled(const DcnLaunch &d, const LinearLaunch &p, int tile_rows, hipStream_t stream) {
+  const int tiles_m = (d.n_pix + tile_rows - 1) / tile_rows, tiles_n = (p.p[0].n + kSampledFeatures - 1) / kSampledFeatures;
+  const size_t lds = (size_t)kSampledSplits * kSampledRows * (kSampledFeatures + 4) * 4 + (size_t)kSampledRows * norm_row_bytes(p.k);
+  hipLaunchKernelGGL(sampled_linear_kernel<Tag>, dim3((unsigned)(tiles_m * tiles_n)), dim3(kSampledWaves * 64), lds, stream, d, p, tiles_n, tile_rows);
+  return hipGetLastError();
 }
 
 template <typename Tag, bool EXTRA, int BM, int BN, int WM, int WN>
@@ -552,6 +651,34 @@ bool linear_takes_norm(const LinearLaunch &p) {
   long long tiles = 0;
   for (int i = 0; i < p.count; ++i) tiles += (p.p[i].n + kFewTile - 1) / kFewTile;
   return p.k <= kNormDepth && tiles * ((p.rows + kFewTile - 1) / kFewTile) <= kNormTiles;
+}
+
+// Pixels of a workgroup: one round of its lanes, or as many as leave every CU one workgroup.
+static int sampled_tile_rows(const DcnLaunch &d, int n) {
+  const int vectors = d.G * d.D / 8, tiles_n = (n + kSampledFeatures - 1) / kSampledFeatures;
+  const long long even = ((long long)d.n_pix * tiles_n + kCus - 1) / kCus;
+  return (int)std::min<long long>(kSampledRows, std::max<long long>(std::max(1, kSampledItems / vectors), even));
+}
+
+// One round of workgroups on the chip, and little more than one of a workgroup's lanes: beyond that the sampling that every 64 features
+// do again costs more than the launch.  A layer, us, two kernels | one: 3136 pixels of 64 channels 24.3 | 22.9, 784 of 128 21.9 | 20.4,
+// 196 of 256 22.8 | 21.4, 49 of 512 29.2 | 27.7 (1 round each); 196 of 320 35.2 | 34.4, 49 of 640 41.9 | 41.3 (1.25); 784 of 160 29.1 |
+// 29.4 (1.6), 1568 of 128 26.5 | 26.9 (1.6), 392 of 256 26.2 | 26.4 (1.75), 529 of 256 29.1 | 30.6, 196 of 448 41.2 | 43.4 (2.6).
+// FlashInternImage-T, one picture of 224: 874 -> 790 us with what linear_few_rows_kernel and dcnv4_forward_small_kernel gained.
+bool sampled_linear_fits(const DcnLaunch &d, int dtype, int n) {
+  if (dtype == F32::kCode || d.kh != 3 || d.kw != 3 || d.remove_center || d.softmax || d.lanes.cpt != 8) return false;
+  const int k = d.G * d.D;
+  if (n <= 0 || n % 8 != 0 || k % 8 != 0 || k > kSampledDepth) return false;
+  const int rows = sampled_tile_rows(d, n);
+  const long long tiles_m = (d.n_pix + rows - 1) / rows, tiles_n = (n + kSampledFeatures - 1) / kSampledFeatures;
+  return tiles_m * tiles_n <= kCus && rows * (k / 8) <= kSampledItems * 5 / 4;
+}
+
+hipError_t launch_sampled_linear(int dtype, const DcnLaunch &d, const LinearProblem &q, hipStream_t stream) {
+  LinearLaunch p = {};
+  p.p[0] = q; p.count = 1; p.rows = d.n_pix; p.k = d.G * d.D;
+  const int rows = sampled_tile_rows(d, q.n);
+  return dtype == F16::kCode ? launch_sampled<F16>(d, p, rows, stream) : launch_sampled<BF16>(d, p, rows, stream);
 }
 
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream) {

@@ -60,6 +60,16 @@ hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
 struct LinearTile { int rows, features; };
 LinearTile linear_tile(int dtype, const LinearLaunch &p);
 
+// DCNv4 over value and offset rows of a batch of pictures, and the product behind it, q.a not used: one kernel for a handful of pixels.
+struct SampledLinear {
+  const void *value, *offsets;
+  int batch, height, width, group, group_channels, kernel, pad, dilation, remove_center, row;
+  float offset_scale;
+  LinearProblem q;
+};
+bool sampled_linear_fits(int dtype, const SampledLinear &p);
+hipError_t launch_sampled_linear(int dtype, const SampledLinear &p, hipStream_t stream);
+
 // What follows a product in a layer together with its normalisation (16-bit types), every step rounded as the kernels one by one round
 // it: after_residual  stream = gamma * (product + bias) + residual, normed = norm(stream); else the product rounded to the type and
 // stream = residual + gamma * norm(product + bias).  gamma and residual may be null, normed goes with after_residual.

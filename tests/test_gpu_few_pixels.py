@@ -1,4 +1,4 @@
-"""Calls of a handful of pixels: DCNv4's taps shared by the lanes of a quad."""
+"""Calls of a handful of pixels: DCNv4's taps shared by the lanes of a quad, and the operator with its output projection in one kernel."""
 import pytest
 import torch
 
@@ -27,3 +27,41 @@ def test_forward_of_few_pixels_matches_the_direct_kernel(B, H, W, G, D, dilation
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     keep = torch.isfinite(want)
     assert _rel(got[keep], want[keep]) < bound
+
+
+# one round of workgroups and a round and a quarter of a workgroup's lanes at most: pixels in whole and ragged tiles, widths that are no
+# multiple of 64, one vector a group and several, one pixel
+LAYERS = [(16, 1, False, None, (1, 1, 1)), (64, 4, False, None, (1, 56, 56)), (64, 2, True, 0.3, (1, 33, 29)), (80, 5, True, 0.3, (1, 31, 33)),
+          (128, 8, False, 0.5, (3, 13, 17)), (128, 4, True, 3.0, (1, 28, 28)), (256, 16, False, None, (1, 14, 14)), (320, 20, True, 0.3, (1, 14, 14)),
+          (448, 7, False, None, (1, 5, 6)), (512, 32, False, 0.5, (1, 7, 7)), (640, 40, True, 0.3, (1, 7, 7)), (1024, 64, False, None, (1, 3, 4))]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("channels,groups,post_norm,scale,size", LAYERS, ids=[f"{c[0]}-{'post' if c[2] else 'pre'}" for c in LAYERS])
+def test_layer_of_few_pixels_matches_the_modules_in_fp32(channels, groups, post_norm, scale, size, dtype):
+    from dcnv4_amd import ext
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    torch.manual_seed(channels)
+    layer = InternImageLayer(channels, groups, post_norm=post_norm, layer_scale=scale, dw_kernel_size=3 if post_norm else None,
+                             dcn_output_bias=post_norm).cuda()
+    with torch.no_grad():
+        layer.dcn.offset_mask.weight.normal_(0, 0.02)
+        layer.dcn.offset_mask.bias.normal_(0, 0.5)
+    layer = layer.to(dtype).eval()
+    n, h, w = size
+    x = torch.randn(n, h * w, channels, device="cuda").to(dtype)
+    assert ext._native.sampled_linear_fits(x, h, w, groups, 3)
+    with torch.no_grad():
+        got = layer(x, (h, w))
+        want = layer.float()(x.float(), (h, w))
+    tol = 2e-3 if dtype == torch.float16 else 1.5e-2      # a chain of roundings to the type, as in test_gpu_layers.py
+    assert got.dtype == dtype and _rel(got, want) < tol
+    assert _rel(got[-1, -1], want[-1, -1]) < 4 * tol and _rel(got[..., -8:], want[..., -8:]) < 2 * tol
+
+
+def test_the_rule_of_the_kernel_for_few_pixels():
+    from dcnv4_amd import ext
+    fits = lambda n, h, w, c, kernel=3, dtype=torch.float16: ext._native.sampled_linear_fits(torch.empty(n, h * w, c, dtype=dtype, device="meta"), h, w, c // 16, kernel)
+    assert fits(1, 64, 64, 64) and not fits(1, 64, 65, 64)              # 256 workgroups of 16 pixels
+    assert fits(1, 14, 14, 256) and not fits(1, 14, 23, 256)            # 5 pixels a workgroup are a round and a quarter of its lanes, 6 are not
+    assert not fits(1, 14, 14, 256, kernel=5) and not fits(1, 14, 14, 256, dtype=torch.float32) and not fits(1, 2, 2, 1040)
