@@ -7,7 +7,7 @@
 //                          the gathered operands into LDS: 256 x 128 instead of 128 x 128 brings a quarter less, and two slices
 //                          stay under way where the other kernel waits for its one.
 //  conv_tiled_kernel       many pixels: the tiles, slices and epilogue of linear_tiled_kernel.
-//  conv_few_rows_kernel    a picture at the later stages: 32 pixels x 32 features, the eight waves share the depth, which is
+//  conv_few_rows_kernel    a picture at the later stages: 32 pixels x 32 features or 16 x 16, the eight waves share the depth, which is
 //                          up to 4032, in registers straight from memory (49 x 512 x 2304 in tiles is 36 slices one after the other).
 //  picture_conv_kernel     the first layer, three channels to some fifty: 27 values a pixel make one instruction's depth, a wave
 //                          gathers sixteen pixels' and writes their features as one run.
@@ -15,7 +15,7 @@
 // Measured, 128 pictures of 224 x 224, fp16 (MIOpen's convolution alone | all of it here): picture 3 -> 56, with normalisation and
 // GELU 700 us and two more passes | 114 (180 MB written: 36 at the rate of a copy; the gathered loads and the GELU bound it);
 // 56 -> 112 226 and a pass | 129, 115 with wide tiles; 112 -> 224 226 | 87, 82; 224 -> 448 144 | 79, 63; 448 -> 896 97 | 60 (45 GFLOP
-// each, 390 to 750 TFLOP/s).  One picture, 14 x 14 x 256 -> 512: 9 us.
+// each, 390 to 750 TFLOP/s).  One picture, 14 x 14 x 256 -> 512: 5 us.
 #include "conv.hpp"
 #include "fragments.hpp"
 #include "launch.hpp"
@@ -268,41 +268,61 @@ __global__ void __launch_bounds__(512, 2) conv_wide_kernel(const ConvLaunch p, i
   }
 }
 
-constexpr int kFewTile = 32, kFewWaves = 8;
+constexpr int kFewWaves = 8;
 
-template <typename Tag>
+// F: fragments of sixteen pixels and features in a tile
+template <typename Tag, int F>
 __global__ void __launch_bounds__(kFewWaves * 64) conv_few_rows_kernel(const ConvLaunch p, int rows, int tiles_n) {
-  __shared__ __align__(16) float part[kFewWaves][kFewTile][kFewTile + 4];
+  constexpr int kTile = F * 16;
+  __shared__ __align__(16) float part[kFewWaves][kTile][kTile + 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m0 = (int)(blockIdx.x / tiles_n) * kFewTile, n0 = (int)(blockIdx.x % tiles_n) * kFewTile;
-  const int live_m = min(kFewTile, rows - m0), live_n = min(kFewTile, p.n - n0);
+  const int m0 = (int)(blockIdx.x / tiles_n) * kTile, n0 = (int)(blockIdx.x % tiles_n) * kTile;
+  const int live_m = min(kTile, rows - m0), live_n = min(kTile, p.n - n0);
   const int vectors = p.kernel * p.kernel * p.cin / 8, steps = (vectors + 3) / 4;
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.in, (uint32_t)(p.batch * p.h * p.w) * (uint32_t)p.cin * 2u);
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(p.weight) + (size_t)n0 * vectors * 16, (uint32_t)live_n * vectors * 16);
   const float inv_per_tap = __builtin_amdgcn_rcpf((float)(p.cin / 8));
   const int r16 = lane & 15, kb = lane >> 4;
-  const PixelWindow w0(p, m0 + min(r16, live_m - 1), r16 < live_m), w1(p, m0 + min(16 + r16, live_m - 1), 16 + r16 < live_m);
-  f32x4 acc[2][2] = {};
-#pragma unroll 4
-  for (int s = wave; s < steps; s += kFewWaves) {
-    const DepthVector d(p, s * 4 + kb, vectors, inv_per_tap);
-    u32x4 fm[2], fn[2];
-    fm[0] = buffer_load<16>(ra, d.in && ((w0.taps >> d.tap) & 1) ? (uint32_t)(w0.start + d.offset) : kDropOffset);
-    fm[1] = buffer_load<16>(ra, d.in && ((w1.taps >> d.tap) & 1) ? (uint32_t)(w1.start + d.offset) : kDropOffset);
+  int start[F];
+  uint32_t taps[F];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) fn[i] = buffer_load<16>(rw, d.in ? (uint32_t)((i * 16 + r16) * vectors + s * 4 + kb) * 16u : kDropOffset);
+  for (int j = 0; j < F; ++j) {
+    const PixelWindow window(p, m0 + min(j * 16 + r16, live_m - 1), j * 16 + r16 < live_m);
+    start[j] = window.start;
+    taps[j] = window.taps;
+  }
+  f32x4 acc[F][F] = {};
+  // a wave's steps are requested eight (four) at a time
+  constexpr int kTogether = 8 / F;
+  for (int s0 = wave; s0 < steps; s0 += kTogether * kFewWaves) {
+    u32x4 fm[kTogether][F], fn[kTogether][F];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int u = 0; u < kTogether; ++u) {
+      const int s = s0 + u * kFewWaves;
+      if (s >= steps) break;
+      const DepthVector d(p, s * 4 + kb, vectors, inv_per_tap);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[i], fm[j], acc[i][j]);
+      for (int j = 0; j < F; ++j) fm[u][j] = buffer_load<16>(ra, d.in && ((taps[j] >> d.tap) & 1) ? (uint32_t)(start[j] + d.offset) : kDropOffset);
+#pragma unroll
+      for (int i = 0; i < F; ++i) fn[u][i] = buffer_load<16>(rw, d.in ? (uint32_t)((i * 16 + r16) * vectors + s * 4 + kb) * 16u : kDropOffset);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u) {
+      if (s0 + u * kFewWaves >= steps) break;
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[u][i], fm[u][j], acc[i][j]);
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
+    for (int j = 0; j < F; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
   __syncthreads();
-  if (threadIdx.x >= 128) return;
-  const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
+  const int row = threadIdx.x / (2 * F), n = threadIdx.x % (2 * F) * 8;
+  if (row >= kTile) return;
   const Affine<Tag, 8> affine(p, n0 + n);
   float v[8];
 #pragma unroll
@@ -417,9 +437,14 @@ hipError_t launch_t(const ConvLaunch &p, hipStream_t stream) {
   // few rows against 64 x 64 tiles: a tile's depth is 9 to 63 slices one after the other, so the split pays up to half a chip of
   // tiles; then the rules of linear.hip
   if (tiles(64, 64) < kCus / 2) {
-    const int tiles_n = (p.n + kFewTile - 1) / kFewTile;
-    hipLaunchKernelGGL((conv_few_rows_kernel<Tag>), dim3((unsigned)((rows + kFewTile - 1) / kFewTile * tiles_n)), dim3(kFewWaves * 64), 0, stream, p, rows, tiles_n);
-    return hipGetLastError();
+    auto go = [&](auto kernel, int tile) {
+      const int tiles_n = (p.n + tile - 1) / tile;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + tile - 1) / tile * tiles_n)), dim3(kFewWaves * 64), 0, stream, p, rows, tiles_n);
+      return hipGetLastError();
+    };
+    // a picture's downsampling, normalisation and turned weights with it, us 32 x 32 | 16 x 16: 14 x 14 x 256 -> 512 (128 tiles of 16 x 16) 17.8 |
+    // 14.0, 14 x 14 x 448 -> 896 (224) 31.9 | 22.1, 28 x 28 x 160 -> 320 (260) 14.1 | 12.3, 56 x 56 x 64 -> 128 (392) 10.5 | 10.1, 28 x 28 x 256 -> 512 (416) 18.2 | 17.9
+    return tiles(16, 16) <= 2 * kCus ? go(conv_few_rows_kernel<Tag, 1>, 16) : go(conv_few_rows_kernel<Tag, 2>, 32);
   }
   if (tiles(128, 64) < 2 * kCus) return launch_tiled<Tag, 64, 64, 2, 2>(p, rows, stream);
   if (wide_pays(p, tiles(kWideRows, kWideFeatures))) {

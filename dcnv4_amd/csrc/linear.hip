@@ -14,7 +14,7 @@
 //    fp32: at depths of 2 to 28 slices nothing covers the first loads and the epilogue.  The features are the rows of the matrix instruction's result, so a lane ends up with
 //    four consecutive features of one row and stores 8 bytes.
 //  linear_few_rows_kernel: a picture or two at the later stages, where a launch has a handful of tiles and its time is load
-//    latency.  A workgroup owns 32 rows x 32 features; its four or eight waves share the depth between them, take their fragments
+//    latency.  A workgroup owns 32 rows x 32 features, or 16 x 16; its four or eight waves share the depth between them, take their fragments
 //    straight from memory and meet in LDS once.  What the epilogue reads is requested first, the residual into registers of its own (with
 //    a pointer that was either it or memory it went through scratch memory: 0.7 us of a launch behind another).  With a layer normalisation in
 //    front the workgroup normalises its 32 rows itself, into LDS: each does so again for every 32 features, but a launch less
@@ -370,45 +370,47 @@ __device__ __forceinline__ void normalise_rows(const LinearLaunch &p, long long 
   }
 }
 
-// NORM: vectors of a normalised row in a lane, 0 without normalisation
-template <typename Tag, int WAVES, bool EXTRA, int NORM>
+// F: fragments of sixteen rows and features in a tile.  NORM: vectors of a normalised row in a lane, 0 without normalisation
+template <typename Tag, int WAVES, int F, bool EXTRA, int NORM>
 __global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const LinearLaunch p, int tiles_n0, int tiles_n) {
-  constexpr int kBytes = Tag::kBytes;
+  static_assert(NORM == 0 || F * 16 == kFewTile, "whole tiles of rows are normalised");
+  constexpr int kBytes = Tag::kBytes, kTile = F * 16;
   extern __shared__ u32x4 lds[];
-  float (*part)[kFewTile][kFewTile + 4] = reinterpret_cast<float (*)[kFewTile][kFewTile + 4]>(lds);
+  float (*part)[kTile][kTile + 4] = reinterpret_cast<float (*)[kTile][kTile + 4]>(lds);
   char *rows = reinterpret_cast<char *>(part + WAVES);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tm = blockIdx.x / tiles_n;
   int tn = blockIdx.x % tiles_n;
   const int which = tn >= tiles_n0;
   const LinearProblem &q = p.p[which];
-  const int m0 = tm * kFewTile, k = p.k;
-  const int live_m = (int)min((long long)kFewTile, p.rows - m0);
+  const int m0 = tm * kTile, k = p.k;
+  const int live_m = (int)min((long long)kTile, p.rows - m0);
   const bool first_tile = tn == 0;
   if (which) tn -= tiles_n0;
-  const int n0 = tn * kFewTile, live_n = min(kFewTile, q.n - n0);
+  const int n0 = tn * kTile, live_n = min(kTile, q.n - n0);
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(static_cast<const char *>(q.a) + (size_t)m0 * k * kBytes, (uint32_t)live_m * k * kBytes);
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(static_cast<const char *>(q.w) + (size_t)n0 * k * kBytes, (uint32_t)live_n * k * kBytes);
   const int r16 = lane & 15, kb = lane >> 4;
   constexpr int kStep = 64 / kBytes;
   const int steps = (k + kStep - 1) / kStep;
 
-  // wave w takes every WAVES-th 64 bytes of the depth, two of them requested together (four: 1 % slower)
-  constexpr int kTogether = 2;
-  u32x4 fm[kTogether][2], fn[kTogether][2];
-  auto request = [&](int s0, const __amdgpu_buffer_rsrc_t &r, u32x4 (&f)[kTogether][2]) {
+  // wave w takes every WAVES-th 64 bytes of the depth, two of them requested together (four: 1 % slower), eight of a single fragment
+  constexpr int kTogether = F == 1 ? 8 : 2;
+  u32x4 fm[kTogether][F], fn[kTogether][F];
+  auto request = [&](int s0, const __amdgpu_buffer_rsrc_t &r, u32x4 (&f)[kTogether][F]) {
 #pragma unroll
     for (int u = 0; u < kTogether; ++u) {
+      if (F == 1 && u > 0 && s0 + u * WAVES >= steps) break;
       const int kk = (s0 + u * WAVES) * kStep + kb * (16 / kBytes);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) f[u][j] = buffer_load<16>(r, kk < k ? (uint32_t)((j * 16 + r16) * k + kk) * kBytes : kDropOffset);
+      for (int j = 0; j < F; ++j) f[u][j] = buffer_load<16>(r, kk < k ? (uint32_t)((j * 16 + r16) * k + kk) * kBytes : kDropOffset);
     }
   };
   request(wave, rw, fn);
   if constexpr (NORM == 0) request(wave, ra, fm);
   // what the epilogue needs, by the lanes that run it
-  const int row = threadIdx.x >> 2, n = (threadIdx.x & 3) * 8;
-  const bool finishes = threadIdx.x < 128 && row < live_m && n < live_n;
+  const int row = threadIdx.x / (2 * F), n = threadIdx.x % (2 * F) * 8;
+  const bool finishes = row < kTile && row < live_m && n < live_n;
   const Columns<Tag> columns(q, n0 + n, finishes);
   float residual[8] = {};
   if (finishes && q.residual != nullptr) load8<Tag>(q.residual, (size_t)(m0 + row) * q.n + n0 + n, residual);
@@ -417,7 +419,7 @@ __global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const Linea
     __syncthreads();
   }
 
-  f32x4 acc[2][2] = {};
+  f32x4 acc[F][F] = {};
   for (int s0 = wave; s0 < steps; s0 += kTogether * WAVES) {
     if (s0 != wave) {
       request(s0, rw, fn);
@@ -429,18 +431,18 @@ __global__ void __launch_bounds__(WAVES * 64) linear_few_rows_kernel(const Linea
       if constexpr (NORM > 0) {
         const int kk = (s0 + u * WAVES) * kStep + kb * (16 / kBytes);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) fm[u][j] = kk < k ? *reinterpret_cast<const u32x4 *>(rows + (j * 16 + r16) * norm_row_bytes(k) + kk * 2) : u32x4{0u, 0u, 0u, 0u};
+        for (int j = 0; j < F; ++j) fm[u][j] = kk < k ? *reinterpret_cast<const u32x4 *>(rows + (j * 16 + r16) * norm_row_bytes(k) + kk * 2) : u32x4{0u, 0u, 0u, 0u};
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < F; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[u][i], fm[u][j], acc[i][j]);
+        for (int j = 0; j < F; ++j) acc[i][j] = mfma_64_bytes<Tag>(fn[u][i], fm[u][j], acc[i][j]);
     }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
+    for (int j = 0; j < F; ++j) *reinterpret_cast<f32x4 *>(&part[wave][j * 16 + r16][i * 16 + kb * 4]) = acc[i][j];
   __syncthreads();
   if (!finishes) return;
   float v[8];
@@ -568,27 +570,35 @@ hipError_t launch_wide(const LinearLaunch &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename Tag, bool EXTRA, int WAVES, int NORM>
+template <typename Tag, bool EXTRA, int WAVES, int F, int NORM>
 hipError_t launch_few_waves(const LinearLaunch &p, hipStream_t stream) {
-  const int tiles_m = (int)((p.rows + kFewTile - 1) / kFewTile), tiles_n0 = (p.p[0].n + kFewTile - 1) / kFewTile;
-  const int tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kFewTile - 1) / kFewTile : 0);
-  const auto kernel = linear_few_rows_kernel<Tag, WAVES, EXTRA, NORM>;
-  const size_t lds = (size_t)WAVES * kFewTile * (kFewTile + 4) * 4 + (NORM > 0 ? (size_t)kFewTile * norm_row_bytes(p.k) : 0);
+  constexpr int kTile = F * 16;
+  const int tiles_m = (int)((p.rows + kTile - 1) / kTile), tiles_n0 = (p.p[0].n + kTile - 1) / kTile;
+  const int tiles_n = tiles_n0 + (p.count > 1 ? (p.p[1].n + kTile - 1) / kTile : 0);
+  const auto kernel = linear_few_rows_kernel<Tag, WAVES, F, EXTRA, NORM>;
+  const size_t lds = (size_t)WAVES * kTile * (kTile + 4) * 4 + (NORM > 0 ? (size_t)kFewTile * norm_row_bytes(p.k) : 0);
   if (NORM > 0)
     if (hipError_t e = ensure_dynamic_lds_limit(reinterpret_cast<const void *>(kernel), 112 * 1024)) return e;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(WAVES * 64), lds, stream, p, tiles_n0, tiles_n);
   return hipGetLastError();
 }
 
-// Eight waves where four would take more than four turns each (196 x 256 x 1024 8.4 -> 7.0 us; sixteen gain nothing further, the
-// bytes that a CU reads then bound it).
+// Tiles of 16 x 16 where one round of the chip, or little more, holds them: four times the CUs read half the bytes each, and what a CU
+// reads bounds these products.  32 x 32 | 16 x 16, us a launch behind another, with bias, layer scale and residual, fp16: 49 x 512 x 2048
+// (128 tiles of 16 x 16) 9.3 | 5.9, 196 x 256 x 1024 (208) 5.9 | 4.3, 196 x 256 x 256 3.5 | 3.1, 196 x 320 x 1280 (260) 6.8 | 6.3, 196 x 448 x 1792 (364)
+// 8.6 | 8.5, 392 x 256 x 1024 (400) 5.9 | 6.0, 600 x 256 x 256 (608) 3.6 | 4.5; fp32: 49 x 512 x 2048 16.8 | 10.0, 196 x 320 x 1280 11.6 | 10.2.
+// Of 32 x 32, eight waves where four would take more than four turns each (196 x 256 x 1024 8.4 -> 7.0 us; sixteen gain nothing further).
+constexpr int kFewSmallTiles = kCus * 5 / 4;
 template <typename Tag, bool EXTRA>
 hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
   if constexpr (!EXTRA && Tag::kBytes == 2) {
-    if (p.norm.weight != nullptr) return p.k <= 256 ? launch_few_waves<Tag, false, kNormWaves, 2>(p, stream) : launch_few_waves<Tag, false, kNormWaves, 4>(p, stream);
+    if (p.norm.weight != nullptr) return p.k <= 256 ? launch_few_waves<Tag, false, kNormWaves, 2, 2>(p, stream) : launch_few_waves<Tag, false, kNormWaves, 2, 4>(p, stream);
   }
   const long long steps = (long long)p.k * Tag::kBytes / 64;
-  return steps <= 16 ? launch_few_waves<Tag, EXTRA, 4, 0>(p, stream) : launch_few_waves<Tag, EXTRA, 8, 0>(p, stream);
+  long long tiles = 0;
+  for (int i = 0; i < p.count; ++i) tiles += (p.p[i].n + 15) / 16;
+  if (tiles * ((p.rows + 15) / 16) <= kFewSmallTiles) return launch_few_waves<Tag, EXTRA, 8, 1, 0>(p, stream);
+  return steps <= 16 ? launch_few_waves<Tag, EXTRA, 4, 2, 0>(p, stream) : launch_few_waves<Tag, EXTRA, 8, 2, 0>(p, stream);
 }
 
 // Which kernel and tile: enough workgroups for the 256 CUs first, then the tile that brings fewer bytes.  Measured (fp16, tile

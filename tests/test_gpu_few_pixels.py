@@ -65,3 +65,32 @@ def test_the_rule_of_the_kernel_for_few_pixels():
     assert fits(1, 64, 64, 64) and not fits(1, 64, 65, 64)              # 256 workgroups of 16 pixels
     assert fits(1, 14, 14, 256) and not fits(1, 14, 23, 256)            # 5 pixels a workgroup are a round and a quarter of its lanes, 6 are not
     assert not fits(1, 14, 14, 256, kernel=5) and not fits(1, 14, 14, 256, dtype=torch.float32) and not fits(1, 2, 2, 1040)
+
+
+# tiles of 16 x 16 up to 320 of them: one element, ragged tiles, depths below a slice, that are no whole slice and beyond what a
+# workgroup requests at once; 325 tiles go by 32 x 32
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("rows,width,depth", [(1, 8, 8), (17, 24, 40), (49, 512, 2048), (2, 96, 2088), (33, 40, 4168), (320, 256, 64), (400, 208, 64)])
+def test_products_of_few_rows(rows, width, depth, dtype):
+    from dcnv4_amd import ext
+    torch.manual_seed(rows + depth)
+    a, w, res = (torch.randn(*s, device="cuda").to(dtype) for s in ((rows, depth), (width, depth), (rows, width)))
+    b, gamma = (torch.randn(width, device="cuda").to(dtype) for _ in range(2))
+    product = a.double() @ w.double().t()
+    # sums in fp32, of which a lane's chain has a sixteenth (fp32: a quarter), then one rounding of the result
+    unit = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    assert _rel(ext.linear_forward(a, w), product) < unit + 1e-6
+    assert _rel(ext.linear_forward(a, w, b, gamma, res), (product + b.double()) * gamma.double() + res.double()) < unit + 1e-6
+
+
+# pixels x features in tiles of 16 x 16 (252 of them, the depth in one request and in two) and of 32 x 32
+@pytest.mark.parametrize("channels,size", [(112, (5, 15, 14)), (456, (1, 3, 5)), (112, (8, 28, 28))])
+def test_downsampling_of_few_pixels(channels, size):
+    from dcnv4_amd.models.flash_intern_image import DownsampleLayer
+    torch.manual_seed(channels)
+    n, h, w = size
+    layer = DownsampleLayer(channels, "LN").cuda().half().eval()
+    x = torch.randn(n, h * w, channels, device="cuda").half()
+    with torch.no_grad():
+        got, want = layer(x, (h, w)), layer.float()(x.float(), (h, w))
+    assert got[1] == want[1] and _rel(got[0], want[0]) < 2e-3      # as in test_gpu_conv.py
