@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(kWindowThreads, 5) dcnv4_forward_window_kernel
     float y, x, m;
     position(i, k, y, x, m);
     const WindowPoint pt = window_point<UNITS>(frame, y, x, m);
-    if (__builtin_amdgcn_ballot_w64(!pt.ok) != 0) {
+    if (!pt.all) {
       const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
       far |= (uint32_t)(inside && !pt.ok) << k;
     }
@@ -189,24 +189,21 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
     for (int cn = 0; cn < 4; ++cn)
 #pragma unroll
       for (int v = 0; v < 2; ++v) raw[cn][v] = fetch(cn, v);
+    // a sum of each corner, the corners in turn: consecutive instructions do not wait for each other
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) d[cn] = 0.f;
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int cn = 0; cn < 4; ++cn) {
+          const uint32_t a = raw[cn][v][c], b = go_raw[v][c];
+          if constexpr (Tag::kBytes == 2) d[cn] = dot2_pair<Tag>(a, b, d[cn]);      // two channels per instruction, products and sums in fp32
+          else d[cn] = fmaf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), d[cn]);
+        }
 #pragma unroll
     for (int cn = 0; cn < 4; ++cn) {
-      float sum[2] = {0.f, 0.f};      // two running sums: consecutive instructions do not wait for each other
-#pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const u32x4 a = raw[cn][v], b = go_raw[v];
-        if constexpr (Tag::kBytes == 2) {      // two channels per instruction, products and sums in fp32
-#pragma unroll
-          for (int c = 0; c < 4; ++c) sum[c & 1] = dot2_pair<Tag>(a[c], b[c], sum[c & 1]);
-        } else {
-          float fa[4], fb[4];
-          Pack<Tag, 4>::decode(a, fa);
-          Pack<Tag, 4>::decode(b, fb);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) sum[c & 1] = fmaf(fa[c], fb[c], sum[c & 1]);
-        }
-      }
-      d[cn] = sum[0] + sum[1];
       if constexpr (LPG >= 2) d[cn] += dcn::dpp_quad_xor1(d[cn]);
       if constexpr (LPG >= 4) d[cn] += dcn::dpp_quad_xor2(d[cn]);
     }
@@ -234,7 +231,7 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
       // Chebyshev distance of the point from its reference point: its ceiling is how far the weighted corners of its 2x2 block
       // lie from it at most.  Points beyond the cap - which exceeds what a window covers - are folded where they are served.
       bool counts = pt.ok;
-      if (__builtin_amdgcn_ballot_w64(!pt.ok) != 0) {
+      if (!pt.all) {
         const bool inside = y > -1.f && x > -1.f && y < (float)p.H && x < (float)p.W;      // dcnv4_im2col_cuda.cuh:227
         far |= (uint32_t)(inside && !pt.ok) << k;
         counts = inside;
@@ -360,23 +357,37 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
     if (n_beyond != 0 && p.state->listed == 0) p.state->listed = 1u;
     if (mine > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, mine);
   }
-  // runs to memory, a word a lane whatever the alignment, the last element of an odd run alone
+  // runs to memory, a word a lane whatever the alignment, the last element of an odd run alone.  kTeam lanes take every (256 / kTeam)-th
+  // pixel, whose place advances as the window's cells do (stage_window): 27 -> 12 vector instructions a word.
   const int groups = min(kGroups, p.G - t.g0), run = groups * 27;
   char *gom = static_cast<char *>(p.grad_offset_mask) + (((size_t)t.b * p.Q + (size_t)t.oy0 * p.Wo + t.ox0) * p.P_pad + (size_t)t.g0 * 27) * Tag::kBytes;
-  constexpr int kPerWord = 4 / Tag::kBytes;
-  const int words = (run + kPerWord - 1) / kPerWord, total = t.th * t.tw * words;
-  const float inv_words = __builtin_amdgcn_rcpf((float)words), inv_tw = __builtin_amdgcn_rcpf((float)t.tw);
-  for (int idx = threadIdx.x; idx < total; idx += kWindowThreads) {
-    const int pix = exact_div(idx, inv_words), w = idx - pix * words;
-    const int y = exact_div(pix, inv_tw), x = pix - y * t.tw;
-    const elem_t *src = reinterpret_cast<const elem_t *>(lds) + (size_t)(y * p.gt_w + x) * kPitch + w * kPerWord;
-    char *dst = gom + (((size_t)y * p.Wo + x) * p.P_pad + (size_t)w * kPerWord) * Tag::kBytes;
-    if (w * kPerWord + kPerWord <= run) {
-      const uint32_t word = *reinterpret_cast<const uint32_t *>(src);
-      if constexpr (Tag::kBytes == 4) __builtin_nontemporal_store(word, reinterpret_cast<uint32_t *>(dst));
-      else __builtin_memcpy(dst, &word, 4);
-    } else {
-      *reinterpret_cast<elem_t *>(dst) = *src;
+  constexpr int kPerWord = 4 / Tag::kBytes, kWords = (kRun + kPerWord - 1) / kPerWord, kTeam = kWords <= 16 ? 16 : kWords <= 32 ? 32 : 64;
+  static_assert(kWords <= kTeam, "a word a lane");
+  const float inv_tw = __builtin_amdgcn_rcpf((float)t.tw);
+  const int word = threadIdx.x & (kTeam - 1);
+  if (word * kPerWord < run) {
+    constexpr int kStep = kWindowThreads / kTeam;
+    const int step_rows = __builtin_amdgcn_readfirstlane(exact_div(kStep, inv_tw)), step_cols = kStep - step_rows * t.tw;
+    const int pix_pitch = p.P_pad * Tag::kBytes, row_pitch = p.Wo * pix_pitch;
+    const int pix = threadIdx.x / kTeam, y = exact_div(pix, inv_tw);
+    int x = pix - y * t.tw, from = (y * p.gt_w + x) * kPitch + word * kPerWord;
+    size_t to = (size_t)y * row_pitch + (size_t)x * pix_pitch + (size_t)word * 4;
+    const bool whole = word * kPerWord + kPerWord <= run;
+    for (int left = t.th * t.tw - pix; left > 0; left -= kStep) {
+      const elem_t *src = reinterpret_cast<const elem_t *>(lds) + from;
+      char *dst = gom + to;
+      if (whole) {
+        const uint32_t w = *reinterpret_cast<const uint32_t *>(src);
+        if constexpr (Tag::kBytes == 4) __builtin_nontemporal_store(w, reinterpret_cast<uint32_t *>(dst));
+        else __builtin_memcpy(dst, &w, 4);
+      } else {
+        *reinterpret_cast<elem_t *>(dst) = *src;
+      }
+      x += step_cols; from += (step_rows * p.gt_w + step_cols) * kPitch; to += (size_t)(step_rows * row_pitch + step_cols * pix_pitch);
+      const bool over = x >= t.tw;
+      x -= over ? t.tw : 0;
+      from += over ? (p.gt_w - t.tw) * kPitch : 0;
+      to += over ? (size_t)(row_pitch - t.tw * pix_pitch) : 0;
     }
   }
   const int tail = p.P_pad - p.G * 27;
