@@ -233,7 +233,6 @@ int reach_setting() { return g_opt.reach < 0 ? kDefaultReach : std::min(g_opt.re
 // Flash attention backward: head widths the tiled grad_value kernel handles (whole 8-channel blocks; a launch
 // accumulates up to 32 channels - 8 lanes x 4 - and wider heads take a launch per window of 32 over the same point
 // records and lists), with point counts that fit its 32-bit point ids.
-constexpr int kFdaWindowChannels = 32;
 bool fda_tiled_shape(int D, int L, int Q, int K) {
   return D % 8 == 0 && D <= 4 * kFdaWindowChannels && L >= 1 && K >= 1 && (long long)Q * K < (1ll << 31);
 }
@@ -1113,9 +1112,10 @@ int flash_deform_attn_gfx950_forward_split(const void *value, const int64_t *spa
 }
 
 // Scratch of the tiled attention backward, in this order: GradState, keys, point records, grad_out regrouped by head,
-// tile table, sorted point lists.  The last two are sized for the images of one launch and reused by the next.
+// tile table, sorted point lists, counters of items handed out.  The last three are sized for the images of one launch and reused by the
+// next.
 struct FdaScratch {
-  size_t keys, recs, go_rows, table, regions, total;     // byte offsets, total bytes
+  size_t keys, recs, go_rows, table, regions, taken, total;     // byte offsets, total bytes
   int n_chunks, tile_stride, per;
 };
 
@@ -1135,7 +1135,8 @@ FdaScratch fda_scratch(int s, int batch, int N, int G, int D, int L, int Q, int 
   sc.go_rows = sc.recs + round16((size_t)batch * points * 16);
   sc.table = sc.go_rows + round16((size_t)batch * G * Q * D * s);
   sc.regions = sc.table + round16(segs * sc.tile_stride * sizeof(uint32_t));
-  sc.total = sc.regions + round16(segs * 4 * kFdaChunkPoints * sizeof(uint32_t));
+  sc.taken = (sc.regions + segs * 4 * kFdaChunkPoints * sizeof(uint32_t) + 255) / 256 * 256;
+  sc.total = sc.taken + 16 * kFdaTakenStride * sizeof(uint32_t);
   return sc;
 }
 
@@ -1160,11 +1161,14 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
   // the tiled grad_value kernel addresses one image's sampling_loc_attn and grad_out with 32-bit byte offsets
   const unsigned long long row_bytes = (unsigned long long)std::max(num_heads, 1) *
                                        std::max(3 * num_levels * num_points, head_channels) * 4ull;
-  // fp32 tensors with few sampling points per image (a decoder's few hundred queries against an encoder's pyramid):
-  // the atomic scatter adds straight into grad_value and is done before the binned kernels have walked the pyramid's
-  // tiles (2 images of 100x152.., 100 queries: 0.028 against 0.057 ms; 900 queries: 0.107 against 0.067 ms)
+  // fp32 tensors with few sampling points (a decoder's few hundred queries against an encoder's pyramid): the atomic scatter adds straight
+  // into grad_value.  It costs 35 ns a query of 8 heads of 32 channels and 16 points, where the binned kernels cost 8, and the clearing
+  // of grad_value; the binned kernels 15 us to begin with and 0.7 ns a pixel, each of which is in a tile somebody walks.  us, binned /
+  // atomic, images of a pyramid from 100 x 152: 2 images, 300 queries 58 / 41, 500 60 / 59, 900 63 / 98; 6 images, 200 122 / 78, 300
+  // 126 / 110, 500 133 / 158.  From 44 x 36: 2 images, 200 33 / 24, 300 34 / 30, 500 36 / 42; 6 images, 100 44 / 32, 200 46 / 54.
+  const double channels = (double)num_heads * head_channels * batch;
   const bool sparse = g_opt.scatter == kOptAuto && elem_bytes(dtype) == 4 &&
-                      3ll * num_query * num_levels * num_points < (long long)spatial_size;
+                      5.0 * num_query * num_levels * num_points * channels < spatial_size * channels + 11e6;
   const bool tiled = fda_tiled_shape(head_channels, num_levels, num_query, num_points) && fda_tiled_enabled() && !sparse &&
                      (unsigned long long)num_query * row_bytes < (1ull << 31);
   // the tiled path gathers only: 16-byte lanes; the atomic path wants one channel per lane
@@ -1197,6 +1201,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
     char *go_rows = ws + sc.go_rows;
     base.table = reinterpret_cast<uint32_t *>(ws + sc.table);
     base.regions = reinterpret_cast<uint32_t *>(ws + sc.regions);
+    base.taken = reinterpret_cast<uint32_t *>(ws + sc.taken);
     base.n_chunks = sc.n_chunks;
     base.tile_stride = sc.tile_stride;
     // The state block (the binning kernel's flag) is cleared by the first kernel itself, which runs to its end
@@ -1221,6 +1226,11 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
         F.value_bytes = (uint32_t)(nb * pr.img_elems * pr.s);
         F.n_row = nb * F.Q;
         F.n_img = nb;
+        // A tile is worked on by one workgroup: no more points than about a share of them all, or it is what the launch waits for; smaller
+        // tiles than that list more points twice.  us of a backward, shares of 350 / 800 / 2000: 1 image of a pyramid from 100 x 152, every
+        // pixel a query, fp32 214 / 199 / 199, fp16 185 / 147 / 147; 1 of 160 x 160 352 / 317 / 317; 4 of 128 x 128 727 / 728 / 763, fp16 506 /
+        // 505 / 550; 8 of 60 x 60 319 / 319 / 348; 2 of 100 x 152 340 / 346 / 353; 2 of 43 x 89 110 / 118 / 119.
+        F.tile_points = (int)std::clamp<long long>((long long)num_query * num_points * num_levels * nb * num_heads / 800, 1024, 0x7fffffff);
         hipError_t e = hipSuccess;
         if (pass == 0) fda_choose_order(&F, pr, spatial_size, num_heads, head_channels, num_levels, num_points, true);
         F.clear_state = (pass == 0 && b0 == 0) ? 1 : 0;

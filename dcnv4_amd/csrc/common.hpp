@@ -11,6 +11,7 @@
 namespace dcn {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -44,6 +45,11 @@ __device__ __forceinline__ typename RawWord<BYTES>::type buffer_load(__amdgpu_bu
   else if constexpr (BYTES == 8) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
   else return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
+
+// Stores that the caches need not keep (nt).
+__device__ __forceinline__ void buffer_store_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t v) { __builtin_amdgcn_raw_buffer_store_b32(v, r, off, 0, 2); }
+__device__ __forceinline__ void buffer_store_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x2 v) { __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, 2); }
+__device__ __forceinline__ void buffer_store_nt(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 2); }
 
 // ---------------------------------------------------------------- element <-> fp32 conversion
 // N contiguous elements of dtype Tag, held as one raw word, to / from N floats.

@@ -14,18 +14,24 @@
 //     listed under each of them) and writes the sorted point ids to the chunk's region of the
 //     workspace plus one (offset, count) word per tile to a table - no global atomics, no host
 //     round trip, every chunk independent;
-//   * fda_grad_value_kernel: persistent workgroups walk (tile, image, head) items, an XCD staying with one
-//     (image, head) pair and going through its levels coarsest first.  An item collects its tile's slices of all
-//     chunk lists into LDS and applies them in batches of 256 points: records and grad_out rows are requested one
-//     batch ahead; per batch every corner inside the tile draws a rank in its cell's list with an integer LDS
-//     atomic, a 64-entry scan gives every cell a segment, the (weight, parked row) entries are placed, and the
-//     lanes of a cell walk the cell's entries with fp32 sums in registers.  The arithmetic is the reference's
-//     (every term rounded to fp32, summed in fp32, rounded once to the tensor dtype); the order of the terms of a
-//     cell follows the ranks, which the atomics fix per run, like the reference's atomics do;
+//   * fda_grad_value_kernel: persistent workgroups walk (tile, image, head) items, the coarsest levels first, in steps of up to 256
+//     listed points: every corner inside the tile draws a rank in its cell's list with an integer LDS atomic, a 64-entry scan gives
+//     every cell a segment, the (weight, parked row) entries are placed, and the lanes of a cell walk the cell's entries with fp32
+//     sums in registers.  The arithmetic is the reference's (every term rounded to fp32, summed in fp32, rounded once to the tensor
+//     dtype); the order of the terms of a cell follows the ranks, which the atomics fix per run, like the reference's atomics do;
 //   * the finished tile is written to grad_value with plain stores in the tensor dtype.
 //
-// Tiles are at most 8x8 cells and every level is cut into 16 of them or more, so items stay
-// small (several workgroups share a CU and hide each other's latencies) and comparable in size.
+// A step's operands are four loads behind each other: where the tile's points lie in the chunks' lists, their numbers, their records
+// and the rows of grad_out.  An item at a time these were waited for one by one, which was most of the time of a decoder's sparse
+// tiles and a third of an encoder's.  So the steps of all items are one stream: each step adds up its own points while the records and
+// rows of the next, the numbers of the one behind it and the place of the next item's lists are on their way.  The points of a tile
+// come in the order of the queries, neighbours hit the same cells, and a step waits for its longest cell: a step takes every n-th block
+// of 32 (a line of numbers) of the list instead of 256 in a row.  What bounds it now are the VALU (two thirds busy) and LDS (half).
+//   us, before -> now, 8 heads of 32 channels, levels from 100 x 152, four points: 2 images, every pixel a query, fp32 285 -> 171;
+// 300 queries, fp16 72 -> 26.  The whole backward: fp16, 1 image 244 -> 147, 2 images of 100 x 100 253 -> 179 (calls).
+//
+// Tiles are at most 8x8 cells and every level is cut into 16 of them or more, into 64 where a tile would hold more than its share of
+// the points (FdaLaunch::tile_points), so items stay small (several workgroups share a CU and hide each other's latencies).
 // Levels and tile shapes are derived on the device from the spatial_shapes tensor; the host never
 // reads it.  A level with more tiles than the binning kernel's LDS histogram holds raises a flag in
 // GradState: this kernel then writes zeros and the atomic fallback kernel adds everything (in fp32).
@@ -39,13 +45,14 @@ namespace dcn {
 namespace {
 
 constexpr int kBinThreads = 1024;
-constexpr int kBinWordsPerLane = kFdaChunkPoints / 2 / kBinThreads;      // dwords of two keys per lane: 4
+constexpr int kBinPointsPerLane = kFdaChunkPoints / kBinThreads;         // 8; a wave's are consecutive: those of a query stay together
 constexpr int kBinSortedCap = 2 * kFdaChunkPoints;                       // list entries of a chunk put together in LDS
 constexpr int kBatch = 256;                  // listed points per batch: one per lane of the first four waves
-constexpr int kListCap = 1024;               // listed point ids held in LDS at a time
-constexpr int kTabCap = 256;                 // chunk table entries held in LDS at a time
+constexpr int kTabCap = kWave;               // chunk table entries held in LDS at a time
+static_assert(kWave == 64);
+constexpr int kBlock = 32;                   // of an item's listed points: a step takes one in `rounds` of these
 constexpr int kTileCells = 64;               // tiles have at most 8 x 8 cells
-constexpr int kSubLists = 1;                 // sub-lists (groups of lanes) every cell has at least; small tiles get more
+constexpr int kItemSlots = 8;                // items known at a time: added up, fetched, listed, and the one behind them
 
 struct LevelPlan {
   int H, W, start;
@@ -57,6 +64,10 @@ __device__ __forceinline__ LevelPlan level_plan(const FdaLaunch &p, int l) {
   lp.H = (int)p.shapes[2 * l]; lp.W = (int)p.shapes[2 * l + 1]; lp.start = (int)p.level_start[l];
   lp.th = max(1, min(8, (lp.H + 3) / 4));
   lp.tw = max(1, min(8, (lp.W + 3) / 4));
+  if ((long long)p.Q * p.K * ((lp.th + 1) * (lp.tw + 1)) > (long long)p.tile_points * lp.H * lp.W) {
+    lp.th = max(1, min(lp.th, (lp.H + 7) / 8));
+    lp.tw = max(1, min(lp.tw, (lp.W + 7) / 8));
+  }
   lp.nty = lp.H > 0 ? (lp.H + lp.th - 1) / lp.th : 0;
   lp.ntx = lp.W > 0 ? (lp.W + lp.tw - 1) / lp.tw : 0;
   return lp;
@@ -73,6 +84,14 @@ __device__ __forceinline__ float elem_at(const void *base, size_t i) {
 // n / d for small non-negative n and 1 <= d <= 8
 __device__ __forceinline__ int div_small(int n, float inv) { return (int)(((float)n + 0.5f) * inv); }
 
+// n / d for n >= 0, d >= 1: the estimate is off by one at most below 2^22, and the remainder tells; beyond, the long way
+__device__ __forceinline__ int quotient(int n, int d) {
+  if (n >= 1 << 22) return n / d;
+  int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
+  const int rest = n - q * d;
+  return rest < 0 ? q - 1 : rest >= d ? q + 1 : q;
+}
+
 // ------------------------------------------------------------------------------- binning
 // The tiles a sampling point touches: the tile of the first in-level row and column of its corner
 // block, and whether the block continues into the next tile column / row.
@@ -88,6 +107,7 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   __shared__ __align__(16) uint16_t s_sorted[kBinSortedCap];      // the sorted list's first entries, as point numbers inside the chunk
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int QK = p.Q * p.K;
+  if (blockIdx.x == 0 && tid < kXcds) p.taken[tid * kFdaTakenStride] = 0u;        // for the kernel behind this one
   const int chunk = blockIdx.x % p.n_chunks, seg = blockIdx.x / p.n_chunks;       // seg = (image * G + head) * L + level
   const int l = seg % p.L;
   const LevelPlan lp = level_plan(p, l);
@@ -100,8 +120,7 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   __syncthreads();
 
   const size_t QKp = fda_key_stride(p.Q, p.K);
-  const uint32_t *keys = reinterpret_cast<const uint32_t *>(p.keys + (size_t)seg * QKp);
-  const int n_words = (int)(QKp / 2);
+  const uint16_t *keys = p.keys + (size_t)seg * QKp;
   const float inv_th = 1.f / (float)lp.th, inv_tw = 1.f / (float)lp.tw;
 
   auto touch_of = [&](uint32_t k16, uint32_t pt) {
@@ -125,21 +144,19 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   };
 
   // ---- pass 1: count
-  Touch touch[2 * kBinWordsPerLane];
+  Touch touch[kBinPointsPerLane];
+  uint32_t key[kBinPointsPerLane];
 #pragma unroll
-  for (int u = 0; u < kBinWordsPerLane; ++u) {
-    const int w = chunk * (kFdaChunkPoints / 2) + u * kBinThreads + tid;
-    const uint32_t word = __builtin_nontemporal_load(keys + min(w, n_words - 1));
+  for (int u = 0; u < kBinPointsPerLane; ++u) key[u] = __builtin_nontemporal_load(keys + min(chunk * kFdaChunkPoints + u * kBinThreads + tid, QK - 1));
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const Touch t = touch_of((word >> (16 * h)) & 0xffffu, w < n_words ? 2u * (uint32_t)w + h : 0xffffffffu);
-      touch[2 * u + h] = t;
-      if (t.t00 != 0xffffffffu) {
-        atomicAdd(&s_hist[t.t00], 1u);
-        if (t.dx) atomicAdd(&s_hist[t.t00 + 1], 1u);
-        if (t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx], 1u);
-        if (t.dx && t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx + 1], 1u);
-      }
+  for (int u = 0; u < kBinPointsPerLane; ++u) {
+    const Touch t = touch_of(key[u], (uint32_t)(chunk * kFdaChunkPoints + u * kBinThreads + tid));
+    touch[u] = t;
+    if (t.t00 != 0xffffffffu) {
+      atomicAdd(&s_hist[t.t00], 1u);
+      if (t.dx) atomicAdd(&s_hist[t.t00 + 1], 1u);
+      if (t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx], 1u);
+      if (t.dx && t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx + 1], 1u);
     }
   }
   __syncthreads();
@@ -187,17 +204,14 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
     else region[at] = pt0 + local;
   };
 #pragma unroll
-  for (int u = 0; u < kBinWordsPerLane; ++u) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const Touch t = touch[2 * u + h];
-      if (t.t00 == 0xffffffffu) continue;
-      const uint32_t local = 2u * (uint32_t)(u * kBinThreads + tid) + h;
-      place(t.t00, local);
-      if (t.dx) place(t.t00 + 1, local);
-      if (t.dy) place(t.t00 + lp.ntx, local);
-      if (t.dx && t.dy) place(t.t00 + lp.ntx + 1, local);
-    }
+  for (int u = 0; u < kBinPointsPerLane; ++u) {
+    const Touch t = touch[u];
+    if (t.t00 == 0xffffffffu) continue;
+    const uint32_t local = (uint32_t)(u * kBinThreads + tid);
+    place(t.t00, local);
+    if (t.dx) place(t.t00 + 1, local);
+    if (t.dy) place(t.t00 + lp.ntx, local);
+    if (t.dx && t.dy) place(t.t00 + lp.ntx + 1, local);
   }
   __syncthreads();
   const uint32_t n_lds = min(total, (uint32_t)kBinSortedCap);
@@ -224,56 +238,72 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
   return v;
 }
 
+// An item: a tile of one level of one (image, head) pair.
+struct Item {
+  int pair, seg, tile;       // -1: none; (pair, level); tile within the level
+  int y0, x0;                // first cell
+  int shape;                 // height | width << 8 | level << 16
+  int H, W;                  // of the level
+};
+// Up to kBatch listed points of an item.  A step without points is one too: the tile's zeros have to be written.
+struct Step {
+  int n, slot;               // points, where the item lies
+  bool first, last, live;    // of the item; not live: behind the last item
+};
+
 // CW: channels a lane accumulates (at most 16 bytes of the tensor dtype); LPC lanes (4 or 8) share a cell, so a cell
 // holds DP = LPC * CW channels (the head width rounded up to 8, 16 or 32).  A workgroup has one lane per (cell, part):
 // 64 * LPC lanes.  grad_out rows are parked in LDS in the tensor dtype.
-template <typename Tag, int CW, int LPC, int SUBS>
-__global__ void __launch_bounds__(kTileCells * LPC * SUBS) fda_grad_value_kernel(const FdaLaunch p) {
+template <typename Tag, int CW, int LPC>
+__global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_value_kernel(const FdaLaunch p) {
   extern __shared__ __align__(16) uint32_t lds32[];      // 16-byte aligned behind the static arrays: LDS stalls on 8- and 16-byte accesses that are not
   typedef typename RawWord<Tag::kBytes>::type elem_t;
-  constexpr int kSlots = kTileCells * SUBS;                   // every cell has at least SUBS sub-lists
-  constexpr int kApplyThreads = kSlots * LPC;
-  static_assert(kBatch <= kApplyThreads && (kBatch * LPC) % kApplyThreads == 0, "a lane per point, whole rows per lane");
-  constexpr int kCellLanes = LPC;
+  constexpr int kThreads = kTileCells * LPC;
+  static_assert(kBatch <= kThreads, "a lane per point");
   constexpr int kCellLanesLog2 = LPC == 8 ? 3 : 2;
-  constexpr int DP = CW * kCellLanes;
-  constexpr int kParkBytes = Tag::kBytes;
-  constexpr int kGoStride = (((DP * kParkBytes + 15) / 16) | 1) * 16;     // an odd number of 16-byte units per parked row
+  constexpr int DP = CW * LPC;
+  constexpr int kGoStride = (((DP * Tag::kBytes + 15) / 16) | 1) * 16;     // an odd number of 16-byte units per parked row
   // D: the head's channels in memory; this launch accumulates the window [c0, c0 + Dc) of them (heads wider than 32
   // channels take several launches over the same records and lists)
   const int D = p.D, c0 = p.gv_c0, Dc = p.gv_dc, QK = p.Q * p.K;
   uint32_t *s_count = lds32;                                  // [kTileCells] entries per cell in this batch
   uint32_t *s_offs = s_count + kTileCells;                    // [kTileCells + 4] first entry of every cell, then the total
-  uint32_t *s_list = s_offs + kTileCells + 4;                 // [kListCap] listed point ids
-  uint32_t *s_tab = s_list + kListCap;                        // [kTabCap] (offset | count << 16) of the item's tile per chunk
-  uint32_t *s_pre = s_tab + kTabCap;                          // [kTabCap + 4] exclusive prefix of the counts
+  uint32_t *s_query = s_offs + kTileCells + 4;                // [kBatch] queries of the next step's points
+  uint32_t *s_tab = s_query + kBatch;                         // [kTabCap] where the tile's points start in each chunk's list
+  uint32_t *s_pre = s_tab + kTabCap;                          // [kTabCap + 4] exclusive prefix of their counts
   u32x2 *s_entry = reinterpret_cast<u32x2 *>(s_pre + kTabCap + 4);      // [4 * kBatch + 2] (weight, parked row), sorted by cell
   char *s_go = reinterpret_cast<char *>(s_entry + 4 * kBatch + 2);      // [kBatch + 1] parked grad_out rows of the batch, then a row of zeros
   __shared__ LevelPlan s_plan[kMaxLevels];
   __shared__ int s_first[kMaxLevels + 1];                     // rank of each level's first tile in the walk
+  __shared__ bool s_gaps;
+  __shared__ Item s_item[kItemSlots];
 
-  const int tid = threadIdx.x;
-  if (tid == 0) {
-    int rank = 0;                                             // walk order: last level first
-    for (int l = p.L - 1; l >= 0; --l) {
-      s_plan[l] = level_plan(p, l);
-      s_first[l] = rank;
-      rank += s_plan[l].nty * s_plan[l].ntx;
-    }
-    s_first[p.L] = rank;                                      // total
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const uint32_t gave_up = p.state->reserved;                 // then the atomic fallback kernel adds everything
+  if (wave == 0) {
+    const int l = p.L - 1 - lane;                             // walk order: last level first
+    LevelPlan lp = {};
+    if (l >= 0) s_plan[l] = lp = level_plan(p, l);
+    const int tiles = (int)wave_inclusive_scan((uint32_t)(lp.nty * lp.ntx));
+    if (l >= 0) s_first[l] = tiles - lp.nty * lp.ntx;
+    // whether every row belongs to a level: they lie one behind the other from the first row to the last
+    const int cells = (int)wave_inclusive_scan((uint32_t)(lp.H * lp.W));
+    const bool apart = l >= 0 && lp.start + cells != p.N;
+    const bool gaps = __ballot(apart) != 0 || __builtin_amdgcn_readlane(cells, kWave - 1) != p.N;
+    if (lane == kWave - 1) { s_first[p.L] = tiles; s_gaps = gaps; }
   }
   if (tid < kTileCells) s_count[tid] = 0u;
   if (tid < kGoStride / 4) reinterpret_cast<uint32_t *>(s_go + kBatch * kGoStride)[tid] = 0u;      // the row of zeros
   __syncthreads();
-  const int n_tiles = s_first[p.L];
+  const int n_tiles = __builtin_amdgcn_readfirstlane(s_first[p.L]);
   const int BG = p.n_img * p.G;
 
   // value rows that no level covers (spatial_size beyond the levels, gaps between them) get zeros, like the
   // reference's zeros_like(value) (flash_deform_attn_cuda.cu:118); whole rows, by the launch of the first window
-  if (c0 == 0) {
+  if (c0 == 0 && s_gaps) {
     const long long rows = (long long)p.n_img * p.N;
     const int row_elems = p.G * p.D;
-    for (long long r = (long long)blockIdx.x * kApplyThreads + tid; r < rows; r += (long long)gridDim.x * kApplyThreads) {
+    for (long long r = (long long)blockIdx.x * kThreads + tid; r < rows; r += (long long)gridDim.x * kThreads) {
       const int n = (int)(r % p.N);
       bool covered = false;
       for (int l = 0; l < p.L; ++l) covered |= n >= s_plan[l].start && n < s_plan[l].start + s_plan[l].H * s_plan[l].W;
@@ -284,9 +314,9 @@ __global__ void __launch_bounds__(kTileCells * LPC * SUBS) fda_grad_value_kernel
     }
   }
 
-  const bool usable = p.state->reserved == 0u;               // else the atomic fallback kernel adds everything
+  const bool usable = gave_up == 0u;
   const size_t QKp = fda_key_stride(p.Q, p.K);
-  const int my_slot = tid >> kCellLanesLog2, my_part = tid & (kCellLanes - 1);      // slot: (cell, sub-list), 64 of them
+  const int my_slot = tid >> kCellLanesLog2, my_part = tid & (LPC - 1);      // slot: (cell, sub-list), 64 of them
 
   // Item order.  The hardware deals consecutive workgroup ids to the 8 XCDs in turn.  When the (image, head) pairs
   // divide evenly among them, an XCD works through its pairs one after the other, and through a pair level by level
@@ -294,246 +324,286 @@ __global__ void __launch_bounds__(kTileCells * LPC * SUBS) fda_grad_value_kernel
   // stay in that XCD's L2 while its points are gathered.  Otherwise tiles are dealt over everything, in the same
   // level order.
   const bool by_pair = BG % kXcds == 0 && (int)gridDim.x % kXcds == 0;
-  const int n_items = n_tiles * BG;
-  const int xcd = blockIdx.x % kXcds, wg_in_xcd = blockIdx.x / kXcds, wgs_per_xcd = gridDim.x / kXcds;
-  const int items_per_xcd = n_items / kXcds;
-  for (int it = by_pair ? wg_in_xcd : (int)blockIdx.x; it < (by_pair ? items_per_xcd : n_items); it += by_pair ? wgs_per_xcd : (int)gridDim.x) {
-    int rank, bg;
-    if (by_pair) {
-      const int j = it / n_tiles;                             // the XCD's j-th pair
-      rank = it - j * n_tiles;
-      bg = j * kXcds + xcd;
-    } else {
-      rank = it / BG;
-      bg = it - rank * BG;
+  const int workers = by_pair ? gridDim.x / kXcds : gridDim.x, me = by_pair ? blockIdx.x / kXcds : blockIdx.x;
+  const int all_items = by_pair ? n_tiles * (BG / kXcds) : n_tiles * BG;
+  // A workgroup's first two are given, the others go to whoever comes next: a tile of a coarse level holds ten times the points of
+  // one of the finest.  Launches for windows of channels take turns with the counters, each clears those of the one behind it.
+  const bool shared = (long long)QK * p.L >= (long long)kBatch * n_tiles;
+  const int turn = c0 / kFdaWindowChannels & 1;
+  uint32_t *taken = p.taken + (turn * kXcds + (by_pair ? blockIdx.x % kXcds : 0)) * kFdaTakenStride;
+  if (blockIdx.x == 0 && tid < kXcds) p.taken[((turn ^ 1) * kXcds + tid) * kFdaTakenStride] = 0u;
+  const int pairs = by_pair ? BG / kXcds : BG;
+  // by a whole wave, a level a lane
+  auto item_at = [&](long long it, int slot) {
+    if (it >= all_items) {
+      if (lane == 0) s_item[slot] = Item{-1, 0, 0, 0, 0, 0, 0, 0};
+      return;
     }
-    const int b = bg / p.G, g = bg - b * p.G;
-    int l = 0;
-    for (int i = 0; i < p.L; ++i)       // first ranks fall with the level index: the first level whose rank fits
-      if (s_first[i] <= rank && s_plan[i].nty * s_plan[i].ntx > 0) { l = i; break; }
-    const LevelPlan lp = s_plan[l];
-    const int t_in = rank - s_first[l];
-    const int ty = t_in / lp.ntx, tx = t_in - ty * lp.ntx;
-    const int ty0 = ty * lp.th, tx0 = tx * lp.tw;
-    const int th = min(lp.th, lp.H - ty0), tw = min(lp.tw, lp.W - tx0);
-    const int n_cells = th * tw;                             // <= 64
-    // A tile of few cells gives every cell several lanes: cells rounded up to a power of two, 64 / that many sub-lists
-    // per cell; lane (cell, sub) takes the cell's entries sub, sub + n_sub, ...; the partial sums meet at the end.
-    int cells_log2 = 0;
-    while ((1 << cells_log2) < n_cells) ++cells_log2;
-    const int n_sub = kSlots >> cells_log2;
+    const int rank = quotient((int)it, pairs);
+    int pair = (int)it - rank * pairs;
+    if (by_pair) pair = pair * kXcds + blockIdx.x % kXcds;
+    const int begin = lane < p.L ? s_first[lane] : all_items;
+    const int level = __builtin_ctzll(__ballot(rank >= begin));      // first ranks fall with the level
+    const LevelPlan lp = s_plan[level];
+    const int tile = rank - __builtin_amdgcn_readlane(begin, level), ty = quotient(tile, lp.ntx), y0 = ty * lp.th, x0 = (tile - ty * lp.ntx) * lp.tw;
+    if (lane == 0)
+      s_item[slot] = Item{pair, pair * p.L + level, tile, y0, x0, min(lp.th, lp.H - y0) | min(lp.tw, lp.W - x0) << 8 | level << 16, lp.H, lp.W};      // <= 64 cells
+  };
+
+  // Everything a step needs is on its way at least a step before it: the (offset, count) words of an item's tile when its
+  // predecessor begins, point ids two steps ahead, records and grad_out rows one.  All loads are range-checked or clamped raw
+  // words: no branches around them, so they fly together.
+  const int groups = (p.n_chunks + kTabCap - 1) / kTabCap;    // of chunks, whose words fit LDS
+  uint32_t tab = 0, id = 0, ticket = 0;
+  auto request_tab = [&](int slot, int group) {               // by the second wave
+    int stride = p.tile_stride;
+    asm volatile("" : "+s"(stride));                          // products with it are not worth registers all the time
+    const int chunks = min(kTabCap, p.n_chunks - group * kTabCap);
+    const size_t row = (size_t)__builtin_amdgcn_readfirstlane(s_item[slot].seg) * p.n_chunks + group * kTabCap;
+    const __amdgpu_buffer_rsrc_t words = make_rsrc(p.table + row * stride, (uint32_t)(chunks * stride) * 4u);
+    tab = buffer_load<4>(words, lane < chunks && usable ? (uint32_t)(lane * stride + __builtin_amdgcn_readfirstlane(s_item[slot].tile)) * 4u : kDropOffset);
+  };
+  typedef typename RawWord<CW * Tag::kBytes>::type goN_t;
+  constexpr int kRowsPerLane = kBatch * LPC / kThreads, kRowStep = kThreads / LPC;
+  u32x3 rec = {0u, 0u, 0u};                                   // this lane's point of the step: x, y, probability
+  goN_t go[kRowsPerLane] = {};                                // LPC lanes fetch a listed point's grad_out row, CW channels each
+
+  const int k_shift = (p.K & (p.K - 1)) == 0 ? 31 - __builtin_clz(p.K) : -1;
+
+  // the cursor: what the point ids are requested of.  `enter`: its group of chunks is new.
+  int at_item = 0, at_group = 0, round = 0, rounds = 1, whole = 0, over = 0, total = 0;
+  const uint32_t *region = p.regions;
+  bool enter = me < all_items, live = enter;
+  if (wave == kThreads / kWave - 1) item_at(me, 0);
+  __syncthreads();
+  if (wave == 1 && live) request_tab(0, 0);
+  Step now = {0, 0, false, false, true}, ahead = now;         // two steps of nothing while the first loads come
+
+  float acc[CW];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) acc[c] = 0.f;
+  int y0 = 0, x0 = 0, th = 0, tw = 0;
+  float Hf = 0.f, Wf = 0.f;
+  int cells_log2 = 0;
+  while (now.live) {
+    if (now.first) {
+      const Item i = s_item[now.slot];
+      const int shape = __builtin_amdgcn_readfirstlane(i.shape);
+      y0 = __builtin_amdgcn_readfirstlane(i.y0); x0 = __builtin_amdgcn_readfirstlane(i.x0);
+      th = shape & 0xff; tw = shape >> 8 & 0xff;
+      Hf = (float)i.H; Wf = (float)i.W;
+      // A tile of few cells gives every cell several lanes: cells rounded up to a power of two, 64 / that many sub-lists
+      // per cell; lane (cell, sub) takes the cell's entries sub, sub + n_sub, ...; the partial sums meet at the end.
+      cells_log2 = th * tw > 1 ? 32 - __builtin_clz(th * tw - 1) : 0;
+    }
+    const int n_cells = th * tw, n_sub = kTileCells >> cells_log2;
     const int my_cell = my_slot & ((1 << cells_log2) - 1), my_sub = my_slot >> cells_log2;
-    const int seg = bg * p.L + l;
-    const float Hf = (float)lp.H, Wf = (float)lp.W;
 
-    float acc[CW];
-#pragma unroll
-    for (int c = 0; c < CW; ++c) acc[c] = 0.f;
-
-    // Everything a batch needs is requested through range-checked buffer loads of raw words: no branches
-    // around the loads, so they all fly together, and nothing is converted before it is needed.
-    const __amdgpu_buffer_rsrc_t rec_rs = make_rsrc(p.recs + (size_t)seg * QKp, (uint32_t)QK * 16u);
-    const __amdgpu_buffer_rsrc_t go_rs = make_rsrc(reinterpret_cast<const elem_t *>(p.go_rows) + (size_t)bg * p.Q * D,
-                                                   (uint32_t)((size_t)p.Q * D * Tag::kBytes));
-    // kCellLanes lanes fetch a listed point's grad_out row, CW channels each; a lane serves kRowsPerLane rows of a batch.
-    typedef typename RawWord<CW * Tag::kBytes>::type goN_t;
-    constexpr int kRowsPerLane = kBatch * kCellLanes / kApplyThreads;
-    constexpr int kRowStep = kApplyThreads / kCellLanes;
-    struct Ahead {
-      u32x4 rec;                       // this lane's point of the batch: x, y, probability
-      goN_t go[kRowsPerLane];
-    };
-    auto fetch = [&](uint32_t b0, int nb) {
-      Ahead a;
-      {
-        const uint32_t pt = s_list[min((int)b0 + min(tid, max(nb - 1, 0)), kListCap - 1)];
-        a.rec = buffer_load<16>(rec_rs, tid < nb ? pt * 16u : kDropOffset);
-      }
-#pragma unroll
-      for (int u = 0; u < kRowsPerLane; ++u) {
-        const int h = my_slot + u * kRowStep;
-        const bool live = h < nb && my_part * CW < Dc;
-        const uint32_t q = s_list[min((int)b0 + min(h, max(nb - 1, 0)), kListCap - 1)] / (uint32_t)p.K;
-        a.go[u] = buffer_load<CW * Tag::kBytes>(go_rs, live ? (q * (uint32_t)D + (uint32_t)(c0 + my_part * CW)) * Tag::kBytes : kDropOffset);
-      }
-      return a;
-    };
-
-    // Applies the first n entries of s_list in batches of kBatch points, one lane per point:
-    //   A      the lane rebuilds its point's position; each corner inside the tile draws a rank in its cell
-    //          (integer LDS atomic) - barrier
-    //   scan   exclusive prefix sum of the 64 cell counts (one wave); all lanes park the batch's grad_out rows - barrier
-    //   place  (weight, parked row) entries go to cell start + rank; the next batch's loads are requested - barrier
-    //   B      four lanes per cell walk the cell's entries: sum += weight * grad_out row, fp32, in registers.
-    // No barrier after B: the next batch's phase A only touches the counters, and everything B reads is rewritten
-    // after that batch's first barrier.
-    auto apply_list = [&](uint32_t n) {
-      if (n == 0) return;
-      int nb = (int)min((uint32_t)kBatch, n);
-      Ahead cur = fetch(0, nb);
-      for (uint32_t b0 = 0; b0 < n; b0 += kBatch) {
-        // ---- phase A
-        float rec_w[4] = {0.f, 0.f, 0.f, 0.f};
-        uint32_t rec_cr[4] = {~0u, ~0u, ~0u, ~0u};            // cell << 16 | rank
-        if (tid < nb) {
-          // the position the first backward kernel formed (flash_deform_im2col_cuda.cuh:188-189), and the probability
-          // (a vector element is copied to a scalar first: a bit cast of the element expression itself reads element 0)
-          const uint32_t rx = cur.rec.x, ry = cur.rec.y, rz = cur.rec.z;
-          const float x = __builtin_bit_cast(float, rx), y = __builtin_bit_cast(float, ry);
-          if ((y > -1.f) && (x > -1.f) && (y < Hf) && (x < Wf)) {
-            const float fy = floorf(y), fx = floorf(x);
-            const float ly = y - fy, lx = x - fx, hy = 1.f - ly, hx = 1.f - lx;
-            const float pr = __builtin_bit_cast(float, rz);
-            const float w4[4] = {hy * hx, hy * lx, ly * hx, ly * lx};
-            // corner 0 relative to the tile; a corner inside the tile is inside the level (tiles are clipped to it)
-            const int cy0 = (int)fy - ty0, cx0 = (int)fx - tx0;
-#pragma unroll
-            for (int cn = 0; cn < 4; ++cn) {
-              const int cy = cy0 + (cn >> 1), cx = cx0 + (cn & 1);
-              if ((unsigned)cy < (unsigned)th && (unsigned)cx < (unsigned)tw) {
-                const uint32_t cell = (uint32_t)(cy * tw + cx);
-                rec_w[cn] = pr * w4[cn];
-                rec_cr[cn] = (cell << 16) | __hip_atomic_fetch_add(&s_count[cell], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              }
-            }
-          }
-        }
-        __syncthreads();
-
-        // ---- scan (first wave) and park (everyone)
-        if (tid < kWave) {
-          const uint32_t c = s_count[tid];
-          const uint32_t incl = wave_inclusive_scan(c);
-          s_offs[tid] = incl - c;
-          if (tid == kWave - 1) s_offs[kWave] = incl;
-        }
-#pragma unroll
-        for (int u = 0; u < kRowsPerLane; ++u) {
-          const int h = my_slot + u * kRowStep;
-          if (h >= nb) break;
-          *reinterpret_cast<goN_t *>(s_go + h * kGoStride + my_part * (CW * kParkBytes)) = cur.go[u];
-        }
-        __syncthreads();
-
-        // ---- place
-        if (tid < kTileCells) s_count[tid] = 0u;              // for the next batch; the scan has read them
+    // ---- rank: a lane per point rebuilds its position; each corner inside the tile draws a rank in its cell (integer LDS atomic)
+    float rec_w[4];
+    uint32_t rank[4];                                         // of corner i, if inside & 1 << i
+    int cell0 = 0, inside = 0;
+    if (tid < now.n) {
+      // the position the first backward kernel formed (flash_deform_im2col_cuda.cuh:188-189), and the probability
+      // (a vector element is copied to a scalar first: a bit cast of the element expression itself reads element 0)
+      const uint32_t rx = rec.x, ry = rec.y, rz = rec.z;
+      const float x = __builtin_bit_cast(float, rx), y = __builtin_bit_cast(float, ry);
+      if ((y > -1.f) && (x > -1.f) && (y < Hf) && (x < Wf)) {
+        const float fy = floorf(y), fx = floorf(x);
+        const float ly = y - fy, lx = x - fx, hy = 1.f - ly, hx = 1.f - lx;
+        const float pr = __builtin_bit_cast(float, rz);
+        const float w4[4] = {hy * hx, hy * lx, ly * hx, ly * lx};
+        // corner 0 relative to the tile; a corner inside the tile is inside the level (tiles are clipped to it)
+        const int cy0 = (int)fy - y0, cx0 = (int)fx - x0;
+        cell0 = cy0 * tw + cx0;
 #pragma unroll
         for (int cn = 0; cn < 4; ++cn) {
-          const uint32_t cr = rec_cr[cn];
-          if (cr == ~0u) continue;
-          s_entry[s_offs[cr >> 16] + (cr & 0xffffu)] = u32x2{__builtin_bit_cast(uint32_t, rec_w[cn]), (uint32_t)(tid * kGoStride)};
-        }
-        const int nb_next = b0 + kBatch < n ? (int)min((uint32_t)kBatch, n - b0 - kBatch) : 0;
-        cur = fetch(b0 + kBatch, nb_next);      // flies while this batch is applied (after the last batch: nothing is read)
-        __syncthreads();
-
-        // ---- phase B: a lane walks every n_sub-th entry of its cell, two at a time and without branches inside
-        // (past the end of the list: weight 0 times the row of zeros), so that all LDS reads of a step are in
-        // flight together
-        if (my_cell < n_cells) {
-          const uint32_t beg = s_offs[my_cell], end = s_offs[my_cell + 1];
-          const char *go_lane = s_go + my_part * (CW * kParkBytes);
-          const uint32_t step = (uint32_t)n_sub;
-          for (uint32_t e = beg + (uint32_t)my_sub; e < end; e += 2u * step) {
-            const bool two = e + step < end;
-            const u32x2 ent0 = s_entry[e];
-            u32x2 ent1 = s_entry[two ? e + step : e];
-            ent1.x = two ? ent1.x : 0u;
-            ent1.y = two ? ent1.y : (uint32_t)(kBatch * kGoStride);
-            const goN_t row0 = *reinterpret_cast<const goN_t *>(go_lane + ent0.y);
-            const goN_t row1 = *reinterpret_cast<const goN_t *>(go_lane + ent1.y);
-            const uint32_t w0_bits = ent0.x, w1_bits = ent1.x;
-            const float w0 = __builtin_bit_cast(float, w0_bits), w1 = __builtin_bit_cast(float, w1_bits);
-            float g0[CW], g1[CW];
-            Pack<Tag, CW>::decode(row0, g0);
-            Pack<Tag, CW>::decode(row1, g1);
-#pragma unroll
-            for (int c = 0; c < CW; ++c) acc[c] = fmaf(w1, g1[c], fmaf(w0, g0[c], acc[c]));
+          rec_w[cn] = pr * w4[cn];
+          if ((unsigned)(cy0 + (cn >> 1)) < (unsigned)th && (unsigned)(cx0 + (cn & 1)) < (unsigned)tw) {
+            inside |= 1 << cn;
+            rank[cn] = __hip_atomic_fetch_add(&s_count[cell0 + (cn >> 1) * tw + (cn & 1)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           }
         }
-        nb = nb_next;
       }
-    };
+    }
+    if (tid < kBatch) {
+      uint32_t points = (uint32_t)p.K;
+      asm volatile("" : "+s"(points));
+      s_query[tid] = k_shift >= 0 ? id >> k_shift : id / points;
+    }
+    if (enter && at_group == 0 && wave == kThreads / kWave - 1) {
+      const uint32_t handed = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
+      item_at(at_item == 0 || !shared ? (at_item + 1ll) * workers + me : 2ll * workers + handed, (at_item + 1) & (kItemSlots - 1));
+    }
+    __syncthreads();
 
-    // ---- collect this tile's slices of the chunk lists (a group of chunks at a time) and apply them
-    if (usable) {
-      for (int c0 = 0; c0 < p.n_chunks; c0 += kTabCap) {
-        const int nc = min(kTabCap, p.n_chunks - c0);
-        __syncthreads();
-        for (int c = tid; c < nc; c += kApplyThreads)
-          s_tab[c] = p.table[((size_t)seg * p.n_chunks + c0 + c) * p.tile_stride + t_in];
-        __syncthreads();
-        if (tid < kWave) {            // exclusive prefix of the counts, one wave
-          uint32_t run = 0;
-          for (int base = 0; base < nc; base += kWave) {
-            const int c = base + tid;
-            const uint32_t v = c < nc ? s_tab[c] >> 16 : 0u;
-            const uint32_t incl = wave_inclusive_scan(v);
-            if (c < nc) s_pre[c] = run + incl - v;
-            run += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    // ---- scan the counts (first wave) and the words of the cursor's tile (second), park the rows
+    if (wave == 0) {
+      const uint32_t c = s_count[tid];
+      const uint32_t incl = wave_inclusive_scan(c);
+      s_offs[tid] = incl - c;
+      if (tid == kWave - 1) s_offs[kWave] = incl;
+    }
+    if (wave == 1 && enter) {
+      const uint32_t incl = wave_inclusive_scan(tab >> 16);
+      s_tab[lane] = tab & 0xffffu;
+      s_pre[lane] = incl - (tab >> 16);
+      if (lane == kWave - 1) s_pre[kTabCap] = incl;
+    }
+#pragma unroll
+    for (int u = 0; u < kRowsPerLane; ++u) *reinterpret_cast<goN_t *>(s_go + (my_slot + u * kRowStep) * kGoStride + my_part * (CW * Tag::kBytes)) = go[u];
+    __syncthreads();
+
+    // ---- place (weight, parked row) entries at cell start + rank
+    if (tid < kTileCells) s_count[tid] = 0u;                  // for the next step; the scan has read them
+    uint32_t first_of[4], at[kRowsPerLane];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) first_of[cn] = s_offs[inside >> cn & 1 ? cell0 + (cn >> 1) * tw + (cn & 1) : 0];
+#pragma unroll
+    for (int u = 0; u < kRowsPerLane; ++u) at[u] = s_query[my_slot + u * kRowStep];
+    const int ahead_seg = s_item[ahead.slot].seg, ahead_pair = s_item[ahead.slot].pair;
+    // all of these reads at once, not each where it is used
+    asm volatile("" : "+v"(first_of[0]), "+v"(first_of[1]), "+v"(first_of[2]), "+v"(first_of[3]), "+v"(at[0]), "+v"(at[1]), "+v"(at[2]), "+v"(at[3]));
+    static_assert(kRowsPerLane == 4, "rows a lane fetches");
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn)
+      if (inside >> cn & 1) s_entry[first_of[cn] + rank[cn]] = u32x2{__builtin_bit_cast(uint32_t, rec_w[cn]), (uint32_t)(tid * kGoStride)};
+    // ---- request: ids of the step after the next and words of the next item, then records and rows of the next step, in the order
+    // in which they are waited for
+    const uint32_t listed = id;
+    Step next = {0, at_item & (kItemSlots - 1), false, false, live};
+    if (live) {
+      if (enter) {
+        total = __builtin_amdgcn_readfirstlane((int)s_pre[kTabCap]);
+        const int blocks = (total + kBlock - 1) / kBlock;
+        round = 0;
+        rounds = max(1, (blocks + kBatch / kBlock - 1) / (kBatch / kBlock));
+        whole = quotient(blocks, rounds);
+        over = blocks - whole * rounds;
+        region = p.regions + ((size_t)__builtin_amdgcn_readfirstlane(s_item[next.slot].seg) * p.n_chunks + at_group * kTabCap) * (4 * kFdaChunkPoints);
+      }
+      next.n = (whole + (round < over ? 1 : 0)) * kBlock - (round == (over > 0 ? over : rounds) - 1 ? -total & (kBlock - 1) : 0);
+      next.first = enter && at_group == 0;
+      const int slot = next.slot, group = at_group;
+      if (enter && shared && group == 0 && tid == kThreads - kWave) {
+        uint32_t *mine = taken;
+        asm volatile("" : "+v"(mine));                         // known to be uniform, it would be waited for at once
+        ticket = atomicAdd(mine, 1u);
+      }
+      if (enter && wave == 1) {
+        if (group + 1 < groups) request_tab(slot, group + 1);
+        else request_tab((at_item + 1) & (kItemSlots - 1), 0);
+      }
+      if (wave < kBatch / kWave) {      // lane -> entry -> chunk: the last that starts at it or before
+        const uint32_t starts = s_pre[lane], skip = (uint32_t)lane * (4 * kFdaChunkPoints) + s_tab[lane] - starts;
+        const uint32_t e = (uint32_t)((tid / kBlock * rounds + round) * kBlock + tid % kBlock);
+        uint32_t to[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {      // a block's first entry, and the chunks that start within it
+          const uint32_t e0 = (uint32_t)(((2 * wave + h) * rounds + round) * kBlock);
+          to[h] = (uint32_t)__builtin_amdgcn_readlane((int)skip, 63 - __builtin_clzll(__ballot(starts <= e0)));
+          for (uint64_t more = __ballot(starts > e0 && starts < e0 + kBlock && starts < (uint32_t)total); more != 0; more &= more - 1) {
+            const int c = __builtin_ctzll(more);
+            to[h] = e >= (uint32_t)__builtin_amdgcn_readlane((int)starts, c) ? (uint32_t)__builtin_amdgcn_readlane((int)skip, c) : to[h];
           }
-          if (tid == 0) s_pre[nc] = run;
         }
-        __syncthreads();
-        const uint32_t total = s_pre[nc];
-        // copy the slices into s_list, kListCap entries at a time; lane -> entry -> chunk by bisection
-        for (uint32_t e0 = 0; e0 < total; e0 += kListCap) {
-          const uint32_t ne = min((uint32_t)kListCap, total - e0);
-          __syncthreads();                                     // the previous list has been fetched from
-          for (uint32_t i = tid; i < ne; i += kApplyThreads) {
-            const uint32_t e = e0 + i;
-            int lo = 0, hi = nc;                       // largest c with s_pre[c] <= e
-            while (hi - lo > 1) {
-              const int mid = (lo + hi) >> 1;
-              if (s_pre[mid] <= e) lo = mid; else hi = mid;
-            }
-            const uint32_t *region = p.regions + ((size_t)seg * p.n_chunks + c0 + lo) * (4 * kFdaChunkPoints);
-            s_list[i] = __builtin_nontemporal_load(region + (s_tab[lo] & 0xffffu) + (e - s_pre[lo]));      // read once
-          }
-          __syncthreads();
-          apply_list(ne);
-        }
+        const __amdgpu_buffer_rsrc_t list = make_rsrc(region, kTabCap * 4 * kFdaChunkPoints * 4u);
+        id = buffer_load<4>(list, tid < next.n ? ((lane < kBlock ? to[0] : to[1]) + e) * 4u : kDropOffset);
+      }
+      enter = ++round == rounds;
+      if (enter && ++at_group == groups) {
+        next.last = true;
+        at_group = 0;
+        ++at_item;
+        live = __builtin_amdgcn_readfirstlane(s_item[at_item & (kItemSlots - 1)].pair) >= 0;
+        enter = live;
+      }
+    }
+    {
+      const int seg = __builtin_amdgcn_readfirstlane(ahead_seg), pair = __builtin_amdgcn_readfirstlane(ahead_pair);
+      const bool any = ahead.n > 0;
+      const __amdgpu_buffer_rsrc_t rec_rs = make_rsrc(p.recs + (any ? (size_t)seg * QKp : 0), (uint32_t)QK * 16u);
+      const __amdgpu_buffer_rsrc_t go_rs = make_rsrc(reinterpret_cast<const elem_t *>(p.go_rows) + (any ? (size_t)pair * p.Q * D : 0),
+                                                     (uint32_t)((size_t)p.Q * D * Tag::kBytes));
+      rec = __builtin_amdgcn_raw_buffer_load_b96(rec_rs, tid < ahead.n ? listed * 16u : kDropOffset, 0, 0);
+#pragma unroll
+      for (int u = 0; u < kRowsPerLane; ++u) {
+        const bool wanted = my_slot + u * kRowStep < ahead.n && my_part * CW < Dc;
+        go[u] = buffer_load<CW * Tag::kBytes>(go_rs, wanted ? (at[u] * (uint32_t)D + (uint32_t)(c0 + my_part * CW)) * Tag::kBytes : kDropOffset);
+      }
+    }
+    __syncthreads();
+
+    // ---- add up: a lane walks every n_sub-th entry of its cell, fp32 sums in registers, two entries at a time and without
+    // branches inside (past the end of the list: weight 0 times the row of zeros), so that all LDS reads of a round are in
+    // flight together.  No barrier behind it: the next step's ranks only touch the counters, and everything read here is
+    // rewritten after that step's first barrier.
+    if (my_cell < n_cells) {
+      const uint32_t end = s_offs[my_cell + 1], step = (uint32_t)n_sub;
+      const char *go_lane = s_go + my_part * (CW * Tag::kBytes);
+      uint32_t e = s_offs[my_cell] + (uint32_t)my_sub;
+      u32x2 ent0 = s_entry[e], ent1 = s_entry[e + step];      // past the end: some word of LDS, not used
+      for (; e < end; e += 2u * step) {
+        const bool two = e + step < end;
+        const uint32_t w0_bits = ent0.x, w1_bits = two ? ent1.x : 0u;
+        const goN_t row0 = *reinterpret_cast<const goN_t *>(go_lane + ent0.y);
+        const goN_t row1 = *reinterpret_cast<const goN_t *>(go_lane + (two ? ent1.y : (uint32_t)(kBatch * kGoStride)));
+        ent0 = s_entry[e + 2u * step];
+        ent1 = s_entry[e + 3u * step];
+        const float w0 = __builtin_bit_cast(float, w0_bits), w1 = __builtin_bit_cast(float, w1_bits);
+        float g0[CW], g1[CW];
+        Pack<Tag, CW>::decode(row0, g0);
+        Pack<Tag, CW>::decode(row1, g1);
+#pragma unroll
+        for (int c = 0; c < CW; ++c) acc[c] = fmaf(w1, g1[c], fmaf(w0, g0[c], acc[c]));
       }
     }
 
     // ---- the tile is complete: the sub-lists' partial sums meet in LDS, then registers -> memory (zeros when the
     // binning gave up: the fallback kernel then adds everything).  The lanes of a cell write DP contiguous channels.
-    if (n_sub > 1) {
-      __syncthreads();                                       // the last phase B is over: lists, entries and rows are free
-      float *s_part = reinterpret_cast<float *>(s_list);     // [kSlots][kCellLanes][CW]
+    if (now.last) {
+      if (n_sub > 1) {      // those of a wave by exchange, the waves' through LDS
+        constexpr int kWaveSlotsLog2 = 6 - kCellLanesLog2;
+        for (int bit = cells_log2; bit < kWaveSlotsLog2; ++bit) {
 #pragma unroll
-      for (int c = 0; c < CW; ++c) s_part[(tid * CW) + c] = acc[c];
-      __syncthreads();
-      if (my_sub == 0) {
-        for (int j = 1; j < n_sub; ++j) {
-          const float *o = s_part + ((((j << cells_log2) + my_cell) << kCellLanesLog2) + my_part) * CW;
+          for (int c = 0; c < CW; ++c) acc[c] += __shfl_xor(acc[c], LPC << bit, kWave);
+        }
+        __syncthreads();                                     // the entries have been read
+        float *s_part = reinterpret_cast<float *>(s_entry);  // [kTileCells][LPC][CW]
+        static_assert(kTileCells * LPC * CW * sizeof(float) <= (4 * kBatch + 2) * sizeof(u32x2), "room for the partial sums");
 #pragma unroll
-          for (int c = 0; c < CW; ++c) acc[c] += o[c];
+        for (int c = 0; c < CW; ++c) s_part[tid * CW + c] = acc[c];
+        __syncthreads();
+        if (my_sub == 0) {
+          const int each = 1 << max(0, kWaveSlotsLog2 - cells_log2);
+          for (int j = each; j < n_sub; j += each) {
+            const float *o = s_part + ((((j << cells_log2) + my_cell) << kCellLanesLog2) + my_part) * CW;
+#pragma unroll
+            for (int c = 0; c < CW; ++c) acc[c] += o[c];
+          }
         }
       }
-      __syncthreads();                                       // read before the row of zeros is restored
-      if (tid < kGoStride / 4) reinterpret_cast<uint32_t *>(s_go + kBatch * kGoStride)[tid] = 0u;
-    }
-    if (my_cell < n_cells && my_sub == 0) {
-      const int cy = my_cell / tw, cx = my_cell - cy * tw;
-      const long long n = (long long)lp.start + (long long)(ty0 + cy) * lp.W + tx0 + cx;      // level tables are not validated
-      if (n >= 0 && n < p.N) {
-        elem_t *dst = reinterpret_cast<elem_t *>(p.grad_value) + (((size_t)b * p.N + (size_t)n) * p.G + g) * D + c0 + my_part * CW;
-        if ((D % CW) == 0 && (Dc % CW) == 0 && (CW * Tag::kBytes) % 4 == 0) {
-          if (my_part * CW < Dc) __builtin_nontemporal_store(Pack<Tag, CW>::encode(acc), reinterpret_cast<goN_t *>(dst));
-        } else {
-#pragma unroll
-          for (int c = 0; c < CW; ++c)
-            if (my_part * CW + c < Dc) { const float f[1] = {acc[c]}; dst[c] = Pack<Tag, 1>::encode(f); }
+      if (my_cell < n_cells && my_sub == 0) {
+        const Item i = s_item[now.slot];
+        const LevelPlan &lp = s_plan[__builtin_amdgcn_readfirstlane(i.shape) >> 16];
+        const int pair = __builtin_amdgcn_readfirstlane(i.pair), b = pair / p.G, g = pair - b * p.G;
+        const int cy = div_small(my_cell, 1.f / (float)tw), cx = my_cell - cy * tw;
+        const long long n = (long long)lp.start + (long long)(y0 + cy) * lp.W + x0 + cx;      // level tables are not validated
+        if (n >= 0 && n < p.N) {
+          const uint32_t at = (uint32_t)((((size_t)b * p.N + (size_t)n) * p.G + g) * D + c0 + my_part * CW) * Tag::kBytes;
+          if (my_part * CW < Dc) buffer_store_nt(make_rsrc(p.grad_value, p.value_bytes), at, Pack<Tag, CW>::encode(acc));
         }
       }
+#pragma unroll
+      for (int c = 0; c < CW; ++c) acc[c] = 0.f;
     }
+    now = ahead;
+    ahead = next;
   }
 }
 
 // lanes per cell: four, or eight when four lanes of 16 bytes do not cover the (padded) head width
 int fda_cell_lanes(int D, int elem_bytes) { return fda_padded_channels(D) * elem_bytes > 64 ? 8 : 4; }
-int fda_sub_lists_for(int) { return kSubLists; }
 
 template <typename Tag>
 hipError_t launch_t(const FdaLaunch &p, hipStream_t stream) {
@@ -550,9 +620,7 @@ hipError_t launch_t(const FdaLaunch &p, hipStream_t stream) {
   }
   const size_t lds = fda_grad_value_lds_bytes(p, Tag::kBytes);
   const int lpc = fda_cell_lanes(p.gv_dc, Tag::kBytes), cw = fda_padded_channels(p.gv_dc) / lpc;
-  const int subs = fda_sub_lists_for(lpc);
-  const int threads = kTileCells * lpc * subs;
-  // persistent workgroups: as many per CU as LDS and wave slots (32 per CU) allow
+  const int threads = kTileCells * lpc;
   // persistent workgroups: as many as are resident at once (registers, LDS and wave slots decide)
   const dim3 block((unsigned)threads);
   auto go = [&](auto kernel) -> hipError_t {
@@ -564,15 +632,15 @@ hipError_t launch_t(const FdaLaunch &p, hipStream_t stream) {
   };
   if (lpc == 8) {
     if constexpr (Tag::kBytes == 4) {
-      if (cw == 4) return go(fda_grad_value_kernel<Tag, 4, 8, kSubLists>);      // fp32 heads of 17 .. 32 channels
+      if (cw == 4) return go(fda_grad_value_kernel<Tag, 4, 8>);      // fp32 heads of 17 .. 32 channels
     }
     return hipErrorInvalidValue;
   }
   switch (cw) {
-    case 2: return go(fda_grad_value_kernel<Tag, 2, 4, kSubLists>);
-    case 4: return go(fda_grad_value_kernel<Tag, 4, 4, kSubLists>);
+    case 2: return go(fda_grad_value_kernel<Tag, 2, 4>);
+    case 4: return go(fda_grad_value_kernel<Tag, 4, 4>);
     case 8:
-      if constexpr (Tag::kBytes == 2) return go(fda_grad_value_kernel<Tag, 8, 4, kSubLists>);
+      if constexpr (Tag::kBytes == 2) return go(fda_grad_value_kernel<Tag, 8, 4>);
       break;
   }
   return hipErrorInvalidValue;      // wider heads take the atomic path (the entry point checks)
@@ -583,11 +651,7 @@ hipError_t launch_t(const FdaLaunch &p, hipStream_t stream) {
 size_t fda_grad_value_lds_bytes(const FdaLaunch &p, int elem_bytes) {
   const size_t go_stride = ((((size_t)fda_padded_channels(p.gv_dc) * elem_bytes + 15) / 16) | 1) * 16;
   const size_t head = ((size_t)2 * kTileCells + 4) * sizeof(uint32_t);
-  const size_t batch = head + ((size_t)kListCap + 2 * kTabCap + 4) * sizeof(uint32_t) + ((size_t)4 * kBatch + 2) * sizeof(u32x2) +
-                       (size_t)(kBatch + 1) * go_stride;
-  // the sub-lists' partial sums meet in LDS behind the counters: a float per lane and channel it holds
-  const size_t meet = head + (size_t)kTileCells * kSubLists * fda_padded_channels(p.gv_dc) * sizeof(float);
-  return std::max(batch, meet);
+  return head + ((size_t)kBatch + 2 * kTabCap + 4) * sizeof(uint32_t) + ((size_t)4 * kBatch + 2) * sizeof(u32x2) + (size_t)(kBatch + 1) * go_stride;
 }
 
 hipError_t launch_fda_grad_value(int dtype, const FdaLaunch &p, hipStream_t stream) {

@@ -244,9 +244,11 @@ struct FdaLaunch {
   void *go_rows;            // [n_img, G, Q, D] grad_out regrouped by head, tensor dtype: a head's rows lie densely
   uint32_t *table;          // [n_img * G * L * n_chunks][tile_stride] (offset | count << 16) of every tile in every chunk's sorted list
   uint32_t *regions;        // [n_img * G * L * n_chunks][4 * kFdaChunkPoints] point ids of a chunk, sorted by tile
+  uint32_t *taken;          // [2 * 8] counters, each kFdaTakenStride words from the next: items of the grad_value kernel handed out, by XCD
   int n_chunks;             // chunks of kFdaChunkPoints points per (image, head, level)
   int tile_stride;          // table row length: an upper bound of the tiles of one level
   int n_img;
+  int tile_points;          // a level whose tiles would collect more of them is cut finer
   int gv_c0, gv_dc;         // tiled grad_value kernel: the window [gv_c0, gv_c0 + gv_dc) of a head's channels this launch accumulates (at most 32)
 };
 
@@ -257,6 +259,8 @@ constexpr uint32_t kFdaKeyOutside = 0xfeffu;
 constexpr uint32_t kFdaKeySaturated = 0xffffu;
 constexpr int kFdaKeyFieldMax = 0xfe;
 constexpr int kFdaChunkPoints = 8192;          // points one binning workgroup sorts
+constexpr int kFdaTakenStride = 64;            // words: dies that count in one cache line wait for each other
+constexpr int kFdaWindowChannels = 32;         // of a head, that the grad_value kernel adds up at a time
 constexpr int kFdaMaxTilesPerLevel = 8192;     // LDS histogram of the binning kernel
 __host__ __device__ inline size_t fda_key_stride(int Q, int K) { return ((size_t)Q * K + 1) & ~size_t(1); }
 

@@ -1,0 +1,58 @@
+"""grad_value of flash deformable attention by tiles: where the walk over tiles and their points turns a corner, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from dcnv4_amd import ext
+from tests import cabi
+from tests.inputs import make_fda_inputs
+
+pytestmark = pytest.mark.gpu
+
+# B, levels, G, D, K, Q
+CASES = {
+    # 69 chunks of points: the words of a tile come in two groups; one level, cut finer because a tile holds thousands of points
+    "two_groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000),
+    # tiles handed out as workgroups come free, pairs by die: levels of 1, 5 and many tiles, one of a single cell
+    "handed_out": (2, [(70, 90), (9, 7), (1, 1), (12, 12)], 8, 32, 4, 3000),
+    # ... two windows of channels, whose launches take turns with the counters, and a third of them
+    "windows_take_turns": (1, [(30, 40), (4, 4)], 8, 72, 4, 1500),
+    # pairs that the dies do not share evenly, points that are no power of two, a part of a block and of a step at every list's end
+    "odd_pairs": (1, [(33, 17), (5, 3)], 3, 16, 6, 1111),
+    # hardly a point to a tile: most steps are empty
+    "empty_tiles": (1, [(100, 120), (50, 60)], 8, 32, 4, 9),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["fp32", "fp16"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_grad_value_by_tiles(oracle, name, dtype):
+    B, levels, G, D, K, Q = CASES[name]
+    print(f"case {name} dtype {dtype}", flush=True)
+    v, shp, st, sla, go = make_fda_inputs(B, levels, G, D, K, Q, seed=len(name), dtype=dtype, loc_lo=-0.05, loc_hi=1.05)
+    args = (cabi.f64(v), shp.numpy(), st.numpy(), cabi.f64(sla))
+    want, _ = oracle.flash_deform_attn_backward(*args, cabi.f64(go), K, coord_f32=True)
+    sizes, _ = oracle.flash_deform_attn_backward(*args, np.abs(cabi.f64(go)), K, coord_f32=True)      # of a sum's terms: all weights are positive
+    with ext.launch_options(scatter="tiled"):
+        got = [cabi.fda_backward(v.cuda(), shp.cuda(), st.cuda(), sla.cuda(), go.cuda(), K)[0] for _ in range(2)]
+    torch.cuda.synchronize()
+    # a weight is right to a few units of fp32 (16 for the exponential's argument), an n-term sum to n of them, and a cell has about
+    # 4 * Q * K / cells terms; the result is rounded to the type
+    terms = 4 * 4 * Q * K / min(h * w for h, w in levels)
+    bound = sizes * (16 + terms) * 2.0 ** -24 + (np.abs(want) * 2.0 ** -11 + 2.0 ** -24 if dtype == torch.float16 else 1e-30)
+    for g in got:
+        assert (np.abs(cabi.f64(g) - want) <= bound).all(), float((np.abs(cabi.f64(g) - want) / bound).max())
+
+
+# fp32 tensors with few points take the atomic scatter by themselves: on either side of where, both ways against each other
+@pytest.mark.parametrize("batch,queries", [(2, 280), (2, 320), (6, 100), (6, 120)])
+def test_few_points_choose_a_way(batch, queries):
+    v, shp, st, sla, go = (t.cuda() for t in make_fda_inputs(batch, [(30, 34), (15, 17), (8, 9), (4, 5)], 8, 32, 4, queries, seed=3, dtype=torch.float32))
+    auto, rows = cabi.fda_backward(v, shp, st, sla, go, 4)
+    sizes, _ = cabi.fda_backward(v, shp, st, sla, go.abs(), 4)
+    for scatter in ("tiled", "atomic"):
+        with ext.launch_options(scatter=scatter):
+            one, one_rows = cabi.fda_backward(v, shp, st, sla, go, 4)
+        # the same terms in another order, at most 4 * queries * 4 of them
+        assert ((one - auto).abs() <= sizes * (2 * 16 * queries * 2.0 ** -24) + 1e-30).all(), scatter
+        torch.testing.assert_close(one_rows, rows, rtol=1e-4, atol=1e-5)
