@@ -9,7 +9,7 @@
 //   * the grad_sampling_loc_attn kernel, which runs first, leaves per sampling point a 16-bit key (integer position
 //     of the first corner, or "outside") and a 16-byte record (position, softmax probability), both laid out
 //     [image][head][level][query][point], and grad_out regrouped by head;
-//   * fda_bin_points_kernel: one workgroup per chunk of 8192 points of one (image, head, level)
+//   * fda_bin_points_kernel: one workgroup per chunk of 4096 points of one (image, head, level)
 //     counting-sorts the chunk by tile in LDS (a point whose 2x2 corner block straddles tiles is
 //     listed under each of them) and writes the sorted point ids to the chunk's region of the
 //     workspace plus one (offset, count) word per tile to a table - no global atomics, no host
@@ -44,7 +44,7 @@ namespace dcn {
 
 namespace {
 
-constexpr int kBinThreads = 1024;
+constexpr int kBinThreads = 512;
 constexpr int kBinPointsPerLane = kFdaChunkPoints / kBinThreads;         // 8; a wave's are consecutive: those of a query stay together
 constexpr int kBinSortedCap = 2 * kFdaChunkPoints;                       // list entries of a chunk put together in LDS
 constexpr int kBatch = 256;                  // listed points per batch: one per lane of the first four waves
@@ -100,9 +100,13 @@ struct Touch {
   uint32_t dx, dy;
 };
 
+// Bound by LDS atomics: neighbouring points fall into few tiles, and an atomic takes its lanes on one address one by one. So they are
+// counted once: a point's rank in a tile is what its count returned, and placing it only reads. Counting a tile's lanes together took
+// longer (two tiles at a time 65 us). 2 images of a pyramid from 100 x 152, every pixel a query, 8 heads, four points: 1024 lanes to
+// 8192 points, counted twice 52 us, once 39, 512 to 4096 - three workgroups on a CU where the ranks left room for one - 32.
 template <typename Tag>
 __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLaunch p) {
-  __shared__ uint32_t s_hist[kFdaMaxTilesPerLevel];       // counts, then running cursors
+  __shared__ uint32_t s_hist[kFdaMaxTilesPerLevel];       // counts, then starts
   __shared__ uint32_t s_wave_sum[kBinThreads / kWave];
   __shared__ __align__(16) uint16_t s_sorted[kBinSortedCap];      // the sorted list's first entries, as point numbers inside the chunk
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -146,6 +150,7 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   // ---- pass 1: count
   Touch touch[kBinPointsPerLane];
   uint32_t key[kBinPointsPerLane];
+  uint32_t rank[kBinPointsPerLane][4];      // within the tile
 #pragma unroll
   for (int u = 0; u < kBinPointsPerLane; ++u) key[u] = __builtin_nontemporal_load(keys + min(chunk * kFdaChunkPoints + u * kBinThreads + tid, QK - 1));
 #pragma unroll
@@ -153,16 +158,16 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
     const Touch t = touch_of(key[u], (uint32_t)(chunk * kFdaChunkPoints + u * kBinThreads + tid));
     touch[u] = t;
     if (t.t00 != 0xffffffffu) {
-      atomicAdd(&s_hist[t.t00], 1u);
-      if (t.dx) atomicAdd(&s_hist[t.t00 + 1], 1u);
-      if (t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx], 1u);
-      if (t.dx && t.dy) atomicAdd(&s_hist[t.t00 + lp.ntx + 1], 1u);
+      rank[u][0] = atomicAdd(&s_hist[t.t00], 1u);
+      if (t.dx) rank[u][1] = atomicAdd(&s_hist[t.t00 + 1], 1u);
+      if (t.dy) rank[u][2] = atomicAdd(&s_hist[t.t00 + lp.ntx], 1u);
+      if (t.dx && t.dy) rank[u][3] = atomicAdd(&s_hist[t.t00 + lp.ntx + 1], 1u);
     }
   }
   __syncthreads();
 
-  // ---- exclusive prefix over the tiles (8 consecutive tiles per lane), table row out
-  constexpr int kPer = kFdaMaxTilesPerLevel / kBinThreads;      // 8
+  // ---- exclusive prefix over the tiles (consecutive ones per lane), table row out
+  constexpr int kPer = kFdaMaxTilesPerLevel / kBinThreads;      // 16
   uint32_t cnt[kPer], sum = 0;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
@@ -184,8 +189,8 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   for (int j = 0; j < kPer; ++j) {
     const int i = tid * kPer + j;
     if (i < n_tiles) {
-      table[i] = before | (cnt[j] << 16);                 // offset <= 32767 and count <= 32768 for 8192 points
-      s_hist[i] = before;                                 // now the running cursor of the tile
+      table[i] = before | (cnt[j] << 16);                 // both fit: a point is listed four times at most, in a tile once
+      s_hist[i] = before;                                 // now where the tile's list starts
     }
     before += cnt[j];
   }
@@ -198,8 +203,8 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
   for (int w = 0; w < kBinThreads / kWave; ++w) total += s_wave_sum[w];
   uint32_t *region = p.regions + (size_t)blockIdx.x * (4 * kFdaChunkPoints);
   const uint32_t pt0 = (uint32_t)chunk * kFdaChunkPoints;
-  auto place = [&](uint32_t tile, uint32_t local) {
-    const uint32_t at = atomicAdd(&s_hist[tile], 1u);
+  auto place = [&](uint32_t tile, uint32_t rank, uint32_t local) {
+    const uint32_t at = s_hist[tile] + rank;
     if (at < (uint32_t)kBinSortedCap) s_sorted[at] = (uint16_t)local;
     else region[at] = pt0 + local;
   };
@@ -208,10 +213,10 @@ __global__ void __launch_bounds__(kBinThreads) fda_bin_points_kernel(const FdaLa
     const Touch t = touch[u];
     if (t.t00 == 0xffffffffu) continue;
     const uint32_t local = (uint32_t)(u * kBinThreads + tid);
-    place(t.t00, local);
-    if (t.dx) place(t.t00 + 1, local);
-    if (t.dy) place(t.t00 + lp.ntx, local);
-    if (t.dx && t.dy) place(t.t00 + lp.ntx + 1, local);
+    place(t.t00, rank[u][0], local);
+    if (t.dx) place(t.t00 + 1, rank[u][1], local);
+    if (t.dy) place(t.t00 + lp.ntx, rank[u][2], local);
+    if (t.dx && t.dy) place(t.t00 + lp.ntx + 1, rank[u][3], local);
   }
   __syncthreads();
   const uint32_t n_lds = min(total, (uint32_t)kBinSortedCap);

@@ -258,7 +258,7 @@ struct FdaLaunch {
 constexpr uint32_t kFdaKeyOutside = 0xfeffu;
 constexpr uint32_t kFdaKeySaturated = 0xffffu;
 constexpr int kFdaKeyFieldMax = 0xfe;
-constexpr int kFdaChunkPoints = 8192;          // points one binning workgroup sorts
+constexpr int kFdaChunkPoints = 4096;          // points one binning workgroup sorts
 constexpr int kFdaTakenStride = 64;            // words: dies that count in one cache line wait for each other
 constexpr int kFdaWindowChannels = 32;         // of a head, that the grad_value kernel adds up at a time
 constexpr int kFdaMaxTilesPerLevel = 8192;     // LDS histogram of the binning kernel

@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 # B, levels, G, D, K, Q
 CASES = {
-    # 69 chunks of points: the words of a tile come in two groups; one level, cut finer because a tile holds thousands of points
-    "two_groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000),
+    # 137 chunks of points: the words of a tile come in three groups; one level, cut finer because a tile holds thousands of points
+    "groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000),
     # tiles handed out as workgroups come free, pairs by die: levels of 1, 5 and many tiles, one of a single cell
     "handed_out": (2, [(70, 90), (9, 7), (1, 1), (12, 12)], 8, 32, 4, 3000),
     # ... two windows of channels, whose launches take turns with the counters, and a third of them
