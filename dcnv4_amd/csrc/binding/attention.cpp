@@ -53,7 +53,7 @@ class LevelCheck {
 struct AttentionSaved {
   Arena arena;
   size_t query, features, value, locations, logits, sampled;      // query, features: their 16-bit copies under autocast
-  size_t value_wt, offsets_wt, logits_wt, output_wt;
+  size_t value_wt, rows_wt, output_wt;
 };
 
 struct Attention {
@@ -112,16 +112,19 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
   size_t as_is[kInputs], turned[kInputs];
   auto narrowed = [&](Input i, int64_t n, int64_t k) {
     as_is[i] = half ? a.take((size_t)(n * k) * 2) : 0;
-    turned[i] = n > 1 && keep ? a.take((size_t)(n * k) * bytes()) : 0;
+    turned[i] = n > 1 && keep && i != kOffsetsW && i != kLogitsW ? a.take((size_t)(n * k) * bytes()) : 0;
   };
   narrowed(kValueW, width, width);
   narrowed(kOffsetsW, n_loc, width);
   narrowed(kLogitsW, n_log, width);
   narrowed(kOutputW, width, width);
+  // the offsets' and the logits' turned side by side, [width][n_loc + n_log]: one product gives the gradient of the query
+  turned[kOffsetsW] = !keep ? 0 : a.take((size_t)((n_loc + n_log) * width) * bytes());
+  turned[kLogitsW] = turned[kOffsetsW] + (size_t)n_loc * bytes();
   for (Input i : {kValueB, kOffsetsB, kLogitsB, kOutputB})
     if (params[i].defined()) narrowed(i, 1, params[i].numel());
   a.allocate(query);
-  s->value_wt = turned[kValueW]; s->offsets_wt = turned[kOffsetsW]; s->logits_wt = turned[kLogitsW]; s->output_wt = turned[kOutputW];
+  s->value_wt = turned[kValueW]; s->rows_wt = turned[kOffsetsW]; s->output_wt = turned[kOutputW];
   for (int i = kValueW; i < kInputs; ++i) {
     const Tensor &t = params[i];
     const bool matrix = t.defined() && t.dim() == 2, turn = matrix && keep;
@@ -130,23 +133,26 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
     q.from = static_cast<const float *>(t.const_data_ptr());
     q.to = half ? a.at(as_is[i]) : nullptr;
     q.turned = turn ? a.at(turned[i]) : nullptr;
+    if (i == kOffsetsW || i == kLogitsW) q.turned_pitch = (int)(n_loc + n_log);
     q.n = matrix ? (int)t.size(0) : 1;
     q.k = matrix ? (int)t.size(1) : (int)t.numel();
   }
-  if (cast.count > 0) hip_check(launch_cast_weights(code, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
-  auto param = [&](Input i) -> const void * { return !params[i].defined() ? nullptr : half ? a.at(as_is[i]) : params[i].const_data_ptr(); };
+  // and the inputs that come in fp32
   auto input = [&](const Tensor &t, bool is32, size_t at, int64_t rows) -> const void * {
     if (!half || !is32) return t.const_data_ptr();
-    hip_check(launch_narrow_rows(code, t.const_data_ptr(), true, a.at(at), (size_t)(rows * width), nullptr, 0, static_cast<hipStream_t>(stream)),
-              "conversion launch");
+    CastWeights &q = cast.p[cast.count++];
+    q.from = static_cast<const float *>(t.const_data_ptr());
+    q.to = a.at(at);
+    q.flat = (size_t)(rows * width);
     return a.at(at);
   };
+  const void *features_in = input(features, features32, s->features, feature_rows()), *query_in = input(query, query32, s->query, query_rows());
+  if (cast.count > 0) hip_check(launch_cast_weights(code, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
+  auto param = [&](Input i) -> const void * { return !params[i].defined() ? nullptr : half ? a.at(as_is[i]) : params[i].const_data_ptr(); };
 
-  LinearLaunch value = product(input(features, features32, s->features, feature_rows()), param(kValueW), param(kValueB), feature_rows(),
-                               width, width, a.at(s->value));
+  LinearLaunch value = product(features_in, param(kValueW), param(kValueB), feature_rows(), width, width, a.at(s->value));
   value.p[0].zero_rows = static_cast<const uint8_t *>(ptr(padding));
   launch(code, value, stream);
-  const void *query_in = input(query, query32, s->query, query_rows());
   levels_check.finish(pixels);
   LinearLaunch rows = product(query_in, param(kOffsetsW), param(kOffsetsB), query_rows(), width, n_loc,
                               a.at(s->locations));
@@ -183,8 +189,7 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
 
   Arena t;
   const size_t d_sampled = t.take((size_t)(query_rows() * width) * bytes()), d_value = t.take((size_t)(feature_rows() * width) * bytes()),
-               d_locations = t.take((size_t)(query_rows() * n_loc) * location_bytes()), d_logits = t.take((size_t)(query_rows() * n_log) * bytes()),
-               d_offsets = t.take((size_t)(query_rows() * n_loc) * bytes());
+               d_rows = t.take((size_t)(query_rows() * (n_loc + n_log)) * bytes());      // of the offsets and the logits, side by side
   const size_t ws_bytes = flash_deform_attn_gfx950_backward_workspace_bytes(code, batch, (int)pixels, heads, (int)width / heads, levels,
                                                                             (int)queries, points);
   const size_t ws = t.take(ws_bytes);
@@ -192,53 +197,43 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
 
   if (through) {
     launch(code, product(grad.const_data_ptr(), a.at(s.output_wt), nullptr, query_rows(), width, width, t.at(d_sampled)), stream);
-    check(flash_deform_attn_gfx950_backward_split(a.at(s.value), shapes.const_data_ptr<int64_t>(), starts.const_data_ptr<int64_t>(),
-                                                  a.at(s.locations), a.at(s.logits), t.at(d_sampled), t.at(d_value), t.at(d_locations),
-                                                  t.at(d_logits), t.at(ws), ws_bytes, code, location_code(), batch, (int)pixels, heads,
-                                                  (int)width / heads, levels, (int)queries, points, 64, 0, 0, stream));
+    FdaLayerBackward p = {};
+    p.value = a.at(s.value); p.locations = a.at(s.locations); p.logits = a.at(s.logits);
+    p.shapes = shapes.const_data_ptr<int64_t>(); p.starts = starts.const_data_ptr<int64_t>();
+    p.grad_output = t.at(d_sampled); p.grad_value = t.at(d_value); p.grad_rows = t.at(d_rows);
+    p.workspace = t.at(ws); p.workspace_bytes = ws_bytes;
+    p.dtype = code; p.location_dtype = location_code();
+    p.batch = (int)batch; p.spatial_size = (int)pixels; p.heads = heads; p.head_channels = (int)width / heads;
+    p.levels = levels; p.queries = (int)queries; p.points = points;
+    p.reference = static_cast<const float *>(ptr(reference)); p.reference_kind = kind;
+    p.zero_rows = static_cast<const uint8_t *>(ptr(padding));
+    check(fda_layer_backward(p, hip));
   }
-  if (into_value && padding.defined())
-    hip_check(launch_zero_rows(bytes(), t.at(d_value), static_cast<const uint8_t *>(padding.const_data_ptr()), feature_rows(), (int)width, hip),
-              "padding launch");
-  if (into_offsets)
-    hip_check(launch_location_grad(code, sampling(reference, shapes), t.at(d_locations), location_code() == DCNV4_DTYPE_F32, t.at(d_offsets),
-                                   query_rows(), (int)n_loc, hip),
-              "location gradient launch");
   // results in the type of the input: fp32 beside 16-bit products
-  auto result = [&](LinearLaunch p, const Tensor &out, bool is32, bool add) {
+  auto result = [&](LinearLaunch p, const Tensor &out, bool is32) {
     LinearProblem &q = p.p[0];
-    if (half && is32) {
-      q.out32 = static_cast<float *>(out.data_ptr());
-      if (add) q.residual32 = q.out32;
-    } else {
-      q.out = out.data_ptr();
-      if (add) q.residual = q.out;
-    }
+    if (half && is32) q.out32 = static_cast<float *>(out.data_ptr());
+    else q.out = out.data_ptr();
     launch(code, p, stream);
   };
   if (want[kFeatures]) {
     g[kFeatures] = at::empty({batch, pixels, width}, features_options);
-    result(product(t.at(d_value), a.at(s.value_wt), nullptr, feature_rows(), width, width, nullptr), g[kFeatures], features32, false);
+    result(product(t.at(d_value), a.at(s.value_wt), nullptr, feature_rows(), width, width, nullptr), g[kFeatures], features32);
   }
   if (want[kQuery]) {
     g[kQuery] = at::empty({batch, queries, width}, query_options);
-    result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc, width, nullptr), g[kQuery], query32, false);
-    result(product(t.at(d_logits), a.at(s.logits_wt), nullptr, query_rows(), n_log, width, nullptr), g[kQuery], query32, true);
+    result(product(t.at(d_rows), a.at(s.rows_wt), nullptr, query_rows(), n_loc + n_log, width, nullptr), g[kQuery], query32);
   }
   const void *q_in = half && query32 ? a.at(s.query) : ptr(query), *f_in = half && features32 ? a.at(s.features) : ptr(features);
   const auto fp32 = params[kValueW].options();
-  auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n) -> WeightGradient {
-    return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1]};
+  auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n, int64_t pitch) -> WeightGradient {
+    return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1], pitch};
   };
-  const WeightGradient value = gradient(kValueW, t.at(d_value), f_in, width), offsets = gradient(kOffsetsW, t.at(d_offsets), q_in, n_loc),
-                       logit = gradient(kLogitsW, t.at(d_logits), q_in, n_log),
-                       output = gradient(kOutputW, grad.const_data_ptr(), a.at(s.sampled), width);
-  if (query_rows() == feature_rows()) {
-    weight_gradients(code, query_rows(), fp32, {output, offsets, value, logit}, stream);
-  } else {
-    weight_gradients(code, query_rows(), fp32, {output, offsets, logit}, stream);
-    weight_gradients(code, feature_rows(), fp32, {value}, stream);
-  }
+  const WeightGradient value = gradient(kValueW, t.at(d_value), f_in, width, 0), offsets = gradient(kOffsetsW, t.at(d_rows), q_in, n_loc, n_loc + n_log),
+                       logit = gradient(kLogitsW, t.at(d_rows + (size_t)n_loc * bytes()), q_in, n_log, n_loc + n_log),
+                       output = gradient(kOutputW, grad.const_data_ptr(), a.at(s.sampled), width, 0);
+  if (query_rows() == feature_rows()) weight_gradients(code, fp32, {{query_rows(), {output, offsets, value, logit}}}, stream);
+  else weight_gradients(code, fp32, {{query_rows(), {output, offsets, logit}}, {feature_rows(), {value}}}, stream);
   return g;
 }
 

@@ -110,50 +110,56 @@ void hip_check(hipError_t e, const char *what) {
   if (e != hipSuccess) raise_runtime("%s: %s", what, hipGetErrorString(e));
 }
 
-void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream) {
-  WeightGradLaunch launch = {};
-  launch.rows = rows;
-  struct { Tensor weight, bias; } grads[kMaxWeightGrads];
-  for (const WeightGradient &l : layers) {
-    if (!l.want_w && !l.want_b) continue;
-    auto &g = grads[launch.count];
-    g.weight = at::empty(l.weight->sizes(), fp32);
-    if (l.want_w) *l.grad_w = g.weight;
-    if (l.want_b) *l.grad_b = g.bias = at::empty(l.bias->sizes(), fp32);
-    WeightGradProblem &q = launch.p[launch.count++];
-    q.grad_out = l.grad_out; q.in = l.in; q.n = (int)l.n; q.k = (int)l.k;
-  }
-  if (launch.count == 0) return;
-  const WeightGradPlan plan = plan_weight_grad(code, launch);
-  launch.splits = plan.splits;
-  // one split writes the gradients themselves, several their partial sums
+void weight_gradients(int code, const at::TensorOptions &fp32, const std::vector<WeightGradients> &groups, void *stream) {
   WeightGradReduce reduce = {};
-  reduce.splits = plan.splits;
-  size_t floats = 0;
-  auto place = [&](const Tensor &grad) {
-    reduce.s[reduce.count++] = {static_cast<float *>(grad.data_ptr()), floats, (int)grad.numel()};
-    floats += (size_t)(grad.numel() + 3) / 4 * 4;
-  };
-  for (int i = 0; i < launch.count; ++i) {
-    place(grads[i].weight);
-    if (grads[i].bias.defined()) place(grads[i].bias);
+  std::vector<Tensor> partials;      // given back behind the last launch
+  for (const WeightGradients &group : groups) {
+    WeightGradLaunch launch = {};
+    launch.rows = group.rows;
+    struct { Tensor weight, bias; } grads[kMaxWeightGrads];
+    for (const WeightGradient &l : group.layers) {
+      if (!l.want_w && !l.want_b) continue;
+      auto &g = grads[launch.count];
+      g.weight = at::empty(l.weight->sizes(), fp32);
+      if (l.want_w) *l.grad_w = g.weight;
+      if (l.want_b) *l.grad_b = g.bias = at::empty(l.bias->sizes(), fp32);
+      WeightGradProblem &q = launch.p[launch.count++];
+      q.grad_out = l.grad_out; q.in = l.in; q.n = (int)l.n; q.k = (int)l.k;
+      q.pitch = (int)(l.pitch != 0 ? l.pitch : l.n);
+    }
+    if (launch.count == 0) continue;
+    const WeightGradPlan plan = plan_weight_grad(code, launch);
+    launch.splits = plan.splits;
+    // one split writes the gradients themselves, several their partial sums
+    size_t floats = 0, offsets[2 * kMaxWeightGrads];
+    int segments = 0;
+    auto place = [&](const Tensor &grad) {
+      offsets[segments++] = floats;
+      floats += (size_t)(grad.numel() + 3) / 4 * 4;
+    };
+    for (int i = 0; i < launch.count; ++i) {
+      place(grads[i].weight);
+      if (grads[i].bias.defined()) place(grads[i].bias);
+    }
+    float *base = nullptr;
+    if (plan.splits > 1) {
+      partials.push_back(at::empty({(int64_t)(floats * plan.splits)}, fp32));
+      base = static_cast<float *>(partials.back().data_ptr());
+    }
+    launch.split_stride = floats;
+    segments = 0;
+    auto target = [&](const Tensor &grad) {
+      float *g = static_cast<float *>(grad.data_ptr()), *sum = base == nullptr ? g : base + offsets[segments++];
+      if (base != nullptr) reduce.s[reduce.count++] = {g, sum, floats, (int)grad.numel(), plan.splits};
+      return sum;
+    };
+    for (int i = 0; i < launch.count; ++i) {
+      launch.p[i].grad_w = target(grads[i].weight);
+      if (grads[i].bias.defined()) launch.p[i].grad_bias = target(grads[i].bias);
+    }
+    hip_check(launch_weight_grad(code, launch, plan.tile, static_cast<hipStream_t>(stream)), "weight gradient launch");
   }
-  Tensor partial;
-  if (plan.splits > 1) partial = at::empty({(int64_t)(floats * plan.splits)}, fp32);
-  float *base = plan.splits > 1 ? static_cast<float *>(partial.data_ptr()) : nullptr;
-  reduce.partial = base;
-  reduce.split_stride = launch.split_stride = floats;
-  int segment = 0;
-  auto target = [&] {
-    const WeightGradSegment &s = reduce.s[segment++];
-    return base != nullptr ? base + s.offset : s.grad;
-  };
-  for (int i = 0; i < launch.count; ++i) {
-    launch.p[i].grad_w = target();
-    if (grads[i].bias.defined()) launch.p[i].grad_bias = target();
-  }
-  hip_check(launch_weight_grad(code, launch, plan.tile, static_cast<hipStream_t>(stream)), "weight gradient launch");
-  if (plan.splits > 1) hip_check(launch_weight_grad_reduce(reduce, static_cast<hipStream_t>(stream)), "weight gradient sum launch");
+  if (reduce.count > 0) hip_check(launch_weight_grad_reduce(reduce, static_cast<hipStream_t>(stream)), "weight gradient sum launch");
 }
 
 bool usable_input(const Tensor &x, int h, int w) {

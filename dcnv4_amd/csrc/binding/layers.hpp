@@ -63,8 +63,14 @@ struct WeightGradient {
   const Tensor *weight, *bias;
   Tensor *grad_w, *grad_b;
   bool want_w, want_b;
+  int64_t pitch = 0;      // elements between grad_out's rows, n if 0
 };
-void weight_gradients(int code, int64_t rows, const at::TensorOptions &fp32, std::initializer_list<WeightGradient> layers, void *stream);
+// Those of the same rows go in one launch, the sums of their parts in one for all.
+struct WeightGradients {
+  int64_t rows;
+  std::vector<WeightGradient> layers;
+};
+void weight_gradients(int code, const at::TensorOptions &fp32, const std::vector<WeightGradients> &groups, void *stream);
 
 extern PyMethodDef training_methods[];
 extern PyMethodDef attention_methods[];

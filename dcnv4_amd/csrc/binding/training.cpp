@@ -137,6 +137,12 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s, bool keep) const {
     cast.p[i].to = a.at(placed[i].second.as_is);
     cast.p[i].turned = placed[i].first ? a.at(placed[i].second.turned) : nullptr;
   }
+  if (l.post_norm && stream32) {      // the stream enters the products as it is
+    CastWeights &q = cast.p[cast.count++];
+    q.from = static_cast<const float *>(x.const_data_ptr());
+    q.to = a.at(s->half_x);
+    q.flat = (size_t)(rows * c);
+  }
   hip_check(launch_cast_weights(c16, cast, static_cast<hipStream_t>(stream)), "parameter conversion launch");
   auto bias = [&](long at) -> const void * { return at < 0 ? nullptr : a.at((size_t)at); };
 
@@ -145,8 +151,9 @@ Tensor LayerTraining::forward(const Tensor &x, Saved *s, bool keep) const {
   Tensor out = at::empty(x.sizes(), x.options());
 
   // DCNv4 half.  The stream enters the products as it is (post-norm) or normalised (pre-norm).
-  if (l.post_norm) narrow(in, stream32, a.at(s->half_x), Tensor(), stream);
-  else normalise(l.norm1, in, stream32, a.at(s->half_x), false, Tensor(), Tensor(), nullptr, nullptr, stream);
+  if (l.post_norm) {
+    if (!stream32) narrow(in, false, a.at(s->half_x), Tensor(), stream);
+  } else normalise(l.norm1, in, stream32, a.at(s->half_x), false, Tensor(), Tensor(), nullptr, nullptr, stream);
   if (l.dw_kernel)
     check(dcnv4_gfx950_depthwise_conv_forward(a.at(s->half_x), a.at(s->w_dw), bias(dw_b), a.at(s->pre), c16, batch, h, w, (int)c,
                                               l.dw_kernel, (l.dw_kernel - 1) / 2, stream));
@@ -297,12 +304,12 @@ variable_list LayerTraining::backward(const Tensor &x, const Tensor &grad, const
   auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n, int64_t k, const Tensor &wt, const Tensor &b) -> WeightGradient {
     return {grad_out, in, n, k, &wt, &b, &g[weight], &g[weight + 1], want[weight], want[weight + 1]};
   };
-  weight_gradients(c16, rows, f32,
-                   {gradient(kFc2W, last, a.at(s.hidden), c, l.hidden, l.fc2_w, l.fc2_b),
+  weight_gradients(c16, f32,
+                   {{rows, {gradient(kFc2W, last, a.at(s.hidden), c, l.hidden, l.fc2_w, l.fc2_b),
                     gradient(kFc1W, t.at(d_hidden), a.at(s.half_mid), l.hidden, c, l.fc1_w, l.fc1_b),
                     gradient(kOutputW, projected, a.at(s.sampled), c, c, l.output_w, l.output_b),
                     gradient(kValueW, t.at(d_value), a.at(s.half_x), c, c, l.value_w, l.value_b),
-                    gradient(kOffsetW, t.at(d_offsets), a.at(s.pre), l.row, c, l.offset_w, l.offset_b)},
+                    gradient(kOffsetW, t.at(d_offsets), a.at(s.pre), l.row, c, l.offset_w, l.offset_b)}}},
                    stream);
   return g;
 }

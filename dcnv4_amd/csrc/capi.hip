@@ -17,6 +17,7 @@
 #include "common.hpp"
 #include "fragments.hpp"
 #include "launch.hpp"
+#include "linear.hpp"
 
 namespace dcn {
 namespace {
@@ -1039,6 +1040,11 @@ struct FdaRows {
   const void *sla, *loc, *logits;
   void *grad_sla, *grad_loc, *grad_logits;
   int loc_bytes;      // 0: packed rows
+  // a layer's (FdaLayerBackward), in place of grad_loc and grad_logits
+  void *grad_rows = nullptr;
+  const float *reference = nullptr;
+  int reference_kind = 0;
+  const uint8_t *zero_rows = nullptr;
 };
 
 static void fda_set_rows(FdaLaunch *F, const FdaRows &r, const FdaProblem &pr, int b0, int LK) {
@@ -1050,6 +1056,9 @@ static void fda_set_rows(FdaLaunch *F, const FdaRows &r, const FdaProblem &pr, i
   F->logits = r.logits ? at(r.logits, pairs * LK, pr.s) : nullptr;
   F->grad_logits = r.grad_logits ? at(r.grad_logits, pairs * LK, pr.s) : nullptr;
   F->loc_f32 = r.loc_bytes == 4 ? 1 : 0;
+  F->grad_rows = r.grad_rows ? at(r.grad_rows, pairs * 3 * LK, pr.s) : nullptr;
+  F->reference = r.reference ? r.reference + (size_t)b0 * F->Q * F->L * r.reference_kind : nullptr;
+  F->reference_kind = r.reference_kind;
 }
 
 static int fda_check_split(int dtype, int location_dtype, int *loc_bytes) {
@@ -1175,7 +1184,8 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
   if (int rc = fda_prepare(&pr, true, !tiled, dtype, batch, spatial_size, num_heads, head_channels, num_levels, num_query,
                            num_points, im2col_step, d_stride, block_thread))
     return rc;
-  if (int rc = rows.loc_bytes == 0 ? check_ptrs({value, rows.sla, grad_output, grad_value, rows.grad_sla})
+  if (int rc = rows.loc_bytes == 0         ? check_ptrs({value, rows.sla, grad_output, grad_value, rows.grad_sla})
+               : rows.grad_rows != nullptr ? check_ptrs({value, rows.loc, rows.logits, grad_output, grad_value, rows.grad_rows})
                         : check_ptrs({value, rows.loc, rows.logits, grad_output, grad_value, rows.grad_loc, rows.grad_logits}))
     return rc;
   if (spatial_shapes == nullptr || level_start_index == nullptr) return fail(DCNV4_ERR_RUNTIME, "null level tensors");
@@ -1188,6 +1198,11 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
   hipStream_t st = static_cast<hipStream_t>(stream);
   const size_t total = (size_t)batch * pr.img_elems;
   const int per = images_per_launch(pr, true);      // equals FdaScratch::per
+  auto clear_rows = [&]() -> int {      // where the kernel that stores grad_value has not
+    if (rows.zero_rows == nullptr) return DCNV4_OK;
+    const hipError_t e = launch_zero_rows(pr.s, grad_value, rows.zero_rows, (long long)batch * spatial_size, num_heads * head_channels, st);
+    return e ? hip_fail("padding launch", e) : DCNV4_OK;
+  };
 
   if (tiled) {
     // pass 0: grad_sampling_loc_attn, keys, point records, regrouped grad_out; pass 1: tiled grad_value; pass 2: fallback
@@ -1226,6 +1241,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
         F.value_bytes = (uint32_t)(nb * pr.img_elems * pr.s);
         F.n_row = nb * F.Q;
         F.n_img = nb;
+        F.zero_rows = rows.zero_rows && !fallback_possible ? rows.zero_rows + (size_t)b0 * spatial_size : nullptr;
         // A tile is worked on by one workgroup: no more points than about a share of them all, or it is what the launch waits for; smaller
         // tiles than that list more points twice.  us of a backward, shares of 350 / 800 / 2000: 1 image of a pyramid from 100 x 152, every
         // pixel a query, fp32 214 / 199 / 199, fp16 185 / 147 / 147; 1 of 160 x 160 352 / 317 / 317; 4 of 128 x 128 727 / 728 / 763, fp16 506 /
@@ -1260,7 +1276,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
         if (e) return hip_fail("flash_deform_attn backward launch", e);
       }
     }
-    return DCNV4_OK;
+    return fallback_possible ? clear_rows() : DCNV4_OK;
   }
 
   const bool widen = pr.s == 2;
@@ -1281,7 +1297,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
   }
   if (widen)
     if (hipError_t e = narrow_async(dtype, acc, grad_value, total, st)) return hip_fail("cast launch", e);
-  return DCNV4_OK;
+  return clear_rows();
 }
 
 int flash_deform_attn_gfx950_backward(const void *value, const int64_t *spatial_shapes,
@@ -1528,6 +1544,18 @@ int depthwise_backward_fp32_grads(const void *input, const void *weight, const v
                                   int channels, int kernel_size, int pad, void *stream) {
   return dw_backward_impl(input, weight, grad_output, grad_input, grad_weight, grad_bias, workspace, workspace_bytes, dtype,
                           DCNV4_DTYPE_F32, batch, height, width, channels, kernel_size, pad, stream);
+}
+
+int fda_layer_backward(const FdaLayerBackward &p, hipStream_t stream) {
+  int loc_bytes = 0;
+  if (int rc = fda_check_split(p.dtype, p.location_dtype, &loc_bytes)) return rc;
+  FdaRows rows{nullptr, p.locations, p.logits, nullptr, nullptr, nullptr, loc_bytes};
+  rows.grad_rows = p.grad_rows;
+  rows.reference = p.reference;
+  rows.reference_kind = p.reference_kind;
+  rows.zero_rows = p.zero_rows;
+  return fda_backward_impl(p.value, p.shapes, p.starts, rows, p.grad_output, p.grad_value, p.workspace, p.workspace_bytes, p.dtype, p.batch,
+                           p.spatial_size, p.heads, p.head_channels, p.levels, p.queries, p.points, 64, 0, 0, stream);
 }
 
 }  // namespace dcn

@@ -537,6 +537,13 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
         go[u] = buffer_load<CW * Tag::kBytes>(go_rs, wanted ? (at[u] * (uint32_t)D + (uint32_t)(c0 + my_part * CW)) * Tag::kBytes : kDropOffset);
       }
     }
+    uint32_t zero = 0;                                        // not 0: the cell's gradient is
+    if (now.last && p.zero_rows != nullptr) {
+      const Item i = s_item[now.slot];
+      const int b = __builtin_amdgcn_readfirstlane(i.pair) / p.G, cy = div_small(my_cell, 1.f / (float)tw);
+      const __amdgpu_buffer_rsrc_t zeros = make_rsrc(p.zero_rows + (size_t)b * p.N, (uint32_t)p.N);
+      zero = __builtin_amdgcn_raw_buffer_load_b8(zeros, (uint32_t)(s_plan[__builtin_amdgcn_readfirstlane(i.shape) >> 16].start + (y0 + cy) * i.W + x0 + my_cell - cy * tw), 0, 0);
+    }
     __syncthreads();
 
     // ---- add up: a lane walks every n_sub-th entry of its cell, fp32 sums in registers, two entries at a time and without
@@ -595,6 +602,10 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
         const int cy = div_small(my_cell, 1.f / (float)tw), cx = my_cell - cy * tw;
         const long long n = (long long)lp.start + (long long)(y0 + cy) * lp.W + x0 + cx;      // level tables are not validated
         if (n >= 0 && n < p.N) {
+          if (zero != 0) {
+#pragma unroll
+            for (int c = 0; c < CW; ++c) acc[c] = 0.f;
+          }
           const uint32_t at = (uint32_t)((((size_t)b * p.N + (size_t)n) * p.G + g) * D + c0 + my_part * CW) * Tag::kBytes;
           if (my_part * CW < Dc) buffer_store_nt(make_rsrc(p.grad_value, p.value_bytes), at, Pack<Tag, CW>::encode(acc));
         }

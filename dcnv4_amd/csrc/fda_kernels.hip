@@ -131,6 +131,41 @@ __device__ __forceinline__ void fda_unstage_grads(const float *lds, const FdaLau
     return;
   }
   const float inv_2lk = 1.f / (float)(2 * LK), inv_lk = 1.f / (float)LK;
+  if (p.grad_rows != nullptr) {
+    // Of the offsets that the locations come from, and of the logits behind them; points come in fours (the layer asks for that), so four
+    // elements lie in one level. Each step rounded as the framework's operators round it.
+    const int per_pair = row_len / 4;
+    const float inv_pair = 1.f / (float)per_pair, inv_2k = 1.f / (float)(2 * p.K);
+    for (int i = threadIdx.x; i < pairs * per_pair; i += blockDim.x) {
+      const int j = fdiv20(i, inv_pair), e = (i - j * per_pair) * 4;
+      const int r = fdiv20(j, inv_h), g = g0 + j - r * heads_here;
+      const f32x4 in = *reinterpret_cast<const f32x4 *>(lds + j * row_len + e);
+      float v[4] = {in.x, in.y, in.z, in.w};
+      int at = p.G * 2 * LK + g * LK + e - 2 * LK;
+      if (e < 2 * LK) {
+        at = g * 2 * LK + e;
+        const int l = fdiv20(e, inv_2k);
+        auto round4 = [&] { Pack<Tag, 4>::decode(Pack<Tag, 4>::encode(v), v); };
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = (float)(_Float16)v[c];
+        if (p.reference_kind == 2) {
+          round4();
+          const float w = (float)(int)p.shapes[2 * l + 1], h = (float)(int)p.shapes[2 * l];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] /= (c & 1) ? h : w;
+        } else {
+          const float *size = p.reference + ((size_t)(row0 + r) * p.L + l) * 4 + 2;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = mul_rn(mul_rn(v[c], 0.5f), size[c & 1]);
+          round4();
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] /= (float)p.K;
+        }
+      }
+      *reinterpret_cast<typename Pack<Tag, 4>::raw_t *>(reinterpret_cast<elem_t *>(p.grad_rows) + (size_t)(row0 + r) * p.G * row_len + at) = Pack<Tag, 4>::encode(v);
+    }
+    return;
+  }
   for (int i = threadIdx.x; i < pairs * 2 * LK; i += blockDim.x) {
     const int j = fdiv20(i, inv_2lk), e = i - j * 2 * LK;
     const int r = fdiv20(j, inv_h), gh = j - r * heads_here;

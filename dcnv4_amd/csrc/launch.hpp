@@ -249,6 +249,11 @@ struct FdaLaunch {
   int tile_stride;          // table row length: an upper bound of the tiles of one level
   int n_img;
   int tile_points;          // a level whose tiles would collect more of them is cut finer
+  // a layer's backward: in place of grad_loc and grad_logits, gradients of its offsets and logits, tensor dtype
+  void *grad_rows;          // [n_row][G * 2*L*K offsets, G * L*K logits]
+  const float *reference;   // [n_row, L, reference_kind]; of the locations: 2 a point, 4 a box
+  int reference_kind;
+  const uint8_t *zero_rows; // [n_img, N]; null, or where grad_value is zero
   int gv_c0, gv_dc;         // tiled grad_value kernel: the window [gv_c0, gv_c0 + gv_dc) of a head's channels this launch accumulates (at most 32)
 };
 

@@ -112,6 +112,7 @@ struct WeightGradProblem {
   const void *grad_out, *in;
   float *grad_w, *grad_bias;
   int n, k;
+  int pitch;                          // elements between grad_out's rows
 };
 struct WeightGradLaunch {
   WeightGradProblem p[kMaxWeightGrads];
@@ -126,23 +127,26 @@ hipError_t launch_weight_grad(int dtype, const WeightGradLaunch &p, int tile, hi
 
 struct WeightGradSegment {
   float *grad;
-  size_t offset;                      // of the segment in a split's partial sums, a multiple of 4
-  int count;
+  const float *partial;               // of the first split, on a 16-byte boundary
+  size_t split_stride;
+  int count, splits;
 };
 struct WeightGradReduce {
   WeightGradSegment s[2 * kMaxWeightGrads];
-  int count, splits;
-  const float *partial;
-  size_t split_stride;
+  int count;
 };
 hipError_t launch_weight_grad_reduce(const WeightGradReduce &p, hipStream_t stream);
 
-// Copies of fp32 matrices [n, k] in the dtype, as they lie and turned [k, n] (either may be null).
+// Copies of fp32 matrices [n, k] in the dtype, as they lie and turned [k, n] (either may be null); with `flat`, a multiple of eight, of
+// so many elements as they lie.
 constexpr int kMaxCasts = 16;
+constexpr size_t kFlatCast = 8192;      // elements of a workgroup
 struct CastWeights {
   const float *from;
   void *to, *turned;
   int n, k;
+  int turned_pitch;                   // elements between rows of turned, a multiple of 4 if n and k are
+  size_t flat;
 };
 struct CastWeightsLaunch {
   CastWeights p[kMaxCasts];
@@ -150,9 +154,6 @@ struct CastWeightsLaunch {
   int count;
 };
 hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &p, hipStream_t stream);
-// grad_offsets (dtype) from the gradients of the locations (fp32, or the dtype): the backward of SamplingLocations.
-hipError_t launch_location_grad(int dtype, const SamplingLocations &l, const void *grad_locations, bool locations32, void *grad_offsets,
-                                long long rows, int n, hipStream_t stream);
 // Clears the rows of n elements whose byte is not zero.
 hipError_t launch_zero_rows(int elem_bytes, void *rows_of, const uint8_t *zero, long long rows, int n, hipStream_t stream);
 // Writes the n (up to 64) numbers to pinned host memory.
@@ -160,5 +161,21 @@ hipError_t launch_read_back(const int64_t *numbers, int n, int64_t *host, hipStr
 // dst = 16-bit src (fp32, or 16-bit with a factor per sample of scale_elements elements); n and scale_elements multiples of 8
 hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
                               hipStream_t stream);
+
+// The backward of deformable attention inside its layer (capi.hip): in place of the gradients of the locations and logits, those of the
+// offsets and logits side by side, [rows][heads * 2 * levels * points, heads * levels * points] in the dtype; grad_value is zero in rows
+// whose byte in zero_rows (may be null) is not.  Checks and errors are those of the library's entry point.
+struct FdaLayerBackward {
+  const void *value;
+  const int64_t *shapes, *starts;
+  const void *locations, *logits, *grad_output;
+  void *grad_value, *grad_rows, *workspace;
+  size_t workspace_bytes;
+  int dtype, location_dtype, batch, spatial_size, heads, head_channels, levels, queries, points;
+  const float *reference;
+  int reference_kind;
+  const uint8_t *zero_rows;
+};
+int fda_layer_backward(const FdaLayerBackward &p, hipStream_t stream);
 
 }  // namespace dcn

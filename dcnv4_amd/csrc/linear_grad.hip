@@ -95,14 +95,15 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   const int load_row = lane * 16 / kRowBytes, load_chunk = lane % (kRowBytes / 16);
   auto stage = [&](long long row0, char (&buf)[2][kPart]) {
     const int live = (int)max(0ll, min((long long)kRows, row_end - row0));
-    const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.n * kBytes, (uint32_t)live * q.n * kBytes);
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(static_cast<const char *>(q.grad_out) + (size_t)row0 * q.pitch * kBytes,
+                                                live > 0 ? (uint32_t)((live - 1) * q.pitch + q.n) * kBytes : 0u);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(static_cast<const char *>(q.in) + (size_t)row0 * q.k * kBytes, (uint32_t)live * q.k * kBytes);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int base = (i * 4 + wave) * kRowsPerLoad, row = base + load_row;
       const int col = ((load_chunk * 16 / kUnit) ^ unit_swizzle<Tag, W>(row)) * 16 + load_chunk * 16 % kUnit / kBytes;
       // columns beyond the matrix read the next row's values; they only reach results beyond the matrix
-      load_to_lds(rg, buf[0] + base * kRowBytes, (uint32_t)(row * q.n + n0 + col) * kBytes);
+      load_to_lds(rg, buf[0] + base * kRowBytes, (uint32_t)(row * q.pitch + n0 + col) * kBytes);
       load_to_lds(rx, buf[1] + base * kRowBytes, (uint32_t)(row * q.k + k0 + col) * kBytes);
     }
   };
@@ -215,23 +216,22 @@ __global__ void __launch_bounds__(256) linear_weight_grad_kernel(const WeightGra
   }
 }
 
-// partial sums [split][split_stride] -> the gradients; every segment starts on a 16-byte boundary and a whole vector of padding
-// may be read behind it
+// partial sums [split][split_stride] -> the gradients; a whole vector of padding may be read behind a segment
 __global__ void __launch_bounds__(256) linear_grad_reduce_kernel(const WeightGradReduce p) {
   const WeightGradSegment &s = p.s[blockIdx.y];
   const int stride = gridDim.x * 256;
   for (int i = blockIdx.x * 256 + threadIdx.x; i * 4 < s.count; i += stride) {
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-    const float *src = p.partial + s.offset + (size_t)i * 4;
+    const float *src = s.partial + (size_t)i * 4;
     // sixteen splits under way, added in pairs: closer to 64 bits than one after the other (the bias of 25088 x 64, 33 splits, 6.8e-8
     // of its norm against 1.2e-7)
     int split = 0;
     auto add = [&](auto at_once) {
       constexpr int kAtOnce = decltype(at_once)::value;
-      for (; split + kAtOnce <= p.splits; split += kAtOnce) {
+      for (; split + kAtOnce <= s.splits; split += kAtOnce) {
         f32x4 v[kAtOnce];
 #pragma unroll
-        for (int u = 0; u < kAtOnce; ++u) v[u] = *reinterpret_cast<const f32x4 *>(src + (size_t)(split + u) * p.split_stride);
+        for (int u = 0; u < kAtOnce; ++u) v[u] = *reinterpret_cast<const f32x4 *>(src + (size_t)(split + u) * s.split_stride);
 #pragma unroll
         for (int step = 1; step < kAtOnce; step *= 2)
 #pragma unroll
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256) linear_grad_reduce_kernel(const WeightGra
 }
 
 // Copies of fp32 parameters in the type: a matrix [n, k] as it lies and turned [k, n], in tiles of 64 x 64 through LDS; a
-// vector (n = 1, nothing turned) as a row.
+// vector (n = 1, nothing turned) as a row.  And of activations (flat): a launch less, as long as parameters go too.
 template <typename Tag>
 __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaunch p) {
   typedef typename RawWord<Tag::kBytes>::type elem_t;
@@ -260,6 +260,27 @@ __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaun
   while (which + 1 < p.count && (int)blockIdx.x >= p.tile_end[which]) ++which;
   const CastWeights &q = p.p[which];
   const int local = blockIdx.x - (which ? p.tile_end[which - 1] : 0), tiles_k = (q.k + 63) / 64;
+  if constexpr (Tag::kBytes == 2) {
+    if (q.flat != 0) {
+      const size_t first = (size_t)local * kFlatCast + threadIdx.x * 8;
+      f32x4 lo[4], hi[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t i = first + u * 2048;
+        if (i >= q.flat) break;
+        lo[u] = *reinterpret_cast<const f32x4 *>(q.from + i);
+        hi[u] = *reinterpret_cast<const f32x4 *>(q.from + i + 4);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t i = first + u * 2048;
+        if (i >= q.flat) break;
+        const float f[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
+        *reinterpret_cast<u32x4 *>(static_cast<elem_t *>(q.to) + i) = Pack<Tag, 8>::encode(f);
+      }
+      return;
+    }
+  }
   const int n0 = local / tiles_k * 64, k0 = local % tiles_k * 64;
   if (q.k % 4 == 0 && (q.turned == nullptr || q.n % 4 == 0)) {      // four columns a lane: 16 bytes in, a row's piece or a turned one out
     const int c4 = (threadIdx.x & 15) * 4;
@@ -288,7 +309,7 @@ __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaun
       for (int c = 0; c < 4; ++c) e[c] = tile[c4 + c][r];
       raw_t h;
       __builtin_memcpy(&h, e, sizeof(h));
-      if (k < q.k && n0 + c4 < q.n) *reinterpret_cast<raw_t *>(static_cast<elem_t *>(q.turned) + (size_t)k * q.n + n0 + c4) = h;
+      if (k < q.k && n0 + c4 < q.n) *reinterpret_cast<raw_t *>(static_cast<elem_t *>(q.turned) + (size_t)k * q.turned_pitch + n0 + c4) = h;
     }
     return;
   }
@@ -307,39 +328,12 @@ __global__ void __launch_bounds__(256) cast_weights_kernel(const CastWeightsLaun
 #pragma unroll 4
   for (int r = threadIdx.x >> 6; r < 64; r += 4) {
     const int k = k0 + r, n = n0 + col;
-    if (n < q.n && k < q.k) static_cast<elem_t *>(q.turned)[(size_t)k * q.n + n] = tile[col][r];
+    if (n < q.n && k < q.k) static_cast<elem_t *>(q.turned)[(size_t)k * q.turned_pitch + n] = tile[col][r];
   }
 }
 
 __global__ void __launch_bounds__(64) read_back_kernel(const int64_t *numbers, int n, int64_t *host) {
   if ((int)threadIdx.x < n) host[threadIdx.x] = numbers[threadIdx.x];
-}
-
-// Eight gradients of one (head, level) at a time: the backward of SamplingLocations, rounded where the framework rounds.
-template <typename Tag, typename LocTag>
-__global__ void __launch_bounds__(256) location_grad_kernel(const SamplingLocations l, const void *grad_locations, void *grad_offsets,
-                                                            size_t vectors, int vectors_per_row) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= vectors) return;
-  const size_t row = i / (size_t)vectors_per_row;
-  const int n = (int)(i - row * vectors_per_row) * 8, level = n / (2 * l.points) % l.levels;
-  float g[8];
-  load8<LocTag>(grad_locations, i * 8, g);
-  if (l.kind == 2) {
-    const float w = (float)l.shapes[2 * level + 1], h = (float)l.shapes[2 * level];
-    round8<Tag>(g);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) g[c] /= (c & 1) ? h : w;
-  } else {
-    const float *size = l.reference + (row * l.levels + level) * 4 + 2;
-    const float points = (float)l.points;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) g[c] = mul_rn(mul_rn(g[c], 0.5f), size[c & 1]);
-    round8<Tag>(g);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) g[c] /= points;
-  }
-  store8<Tag>(grad_offsets, i * 8, g);
 }
 
 // A wave per row.
@@ -430,11 +424,17 @@ hipError_t launch_weight_grad_reduce(const WeightGradReduce &p, hipStream_t stre
 
 hipError_t launch_cast_weights(int dtype, const CastWeightsLaunch &launch, hipStream_t stream) {
   CastWeightsLaunch p = launch;
-  int end = 0;
-  for (int i = 0; i < p.count; ++i) p.tile_end[i] = end += ((p.p[i].n + 63) / 64) * ((p.p[i].k + 63) / 64);
-  if (dtype == F32::kCode) hipLaunchKernelGGL(cast_weights_kernel<F32>, dim3(end), dim3(256), 0, stream, p);
-  else if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3(end), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(cast_weights_kernel<BF16>, dim3(end), dim3(256), 0, stream, p);
+  long long end = 0;
+  for (int i = 0; i < p.count; ++i) {
+    CastWeights &q = p.p[i];
+    if (q.turned_pitch == 0) q.turned_pitch = q.n;
+    end += q.flat != 0 ? (long long)((q.flat + kFlatCast - 1) / kFlatCast) : (long long)((q.n + 63) / 64) * ((q.k + 63) / 64);
+    if (end > 0x7fffffff) return hipErrorInvalidValue;
+    p.tile_end[i] = (int)end;
+  }
+  if (dtype == F32::kCode) hipLaunchKernelGGL(cast_weights_kernel<F32>, dim3((unsigned)end), dim3(256), 0, stream, p);
+  else if (dtype == F16::kCode) hipLaunchKernelGGL(cast_weights_kernel<F16>, dim3((unsigned)end), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL(cast_weights_kernel<BF16>, dim3((unsigned)end), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -442,19 +442,6 @@ hipError_t launch_read_back(const int64_t *numbers, int n, int64_t *host, hipStr
   if (n < 0 || n > 64) return hipErrorInvalidValue;
   hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, numbers, n, host);
   return hipGetLastError();
-}
-
-hipError_t launch_location_grad(int dtype, const SamplingLocations &l, const void *grad_locations, bool locations32, void *grad_offsets,
-                                long long rows, int n, hipStream_t stream) {
-  const size_t vectors = (size_t)rows * (n / 8);
-  const dim3 grid((unsigned)((vectors + 255) / 256)), block(256);
-  auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, l, grad_locations, grad_offsets, vectors, n / 8);
-    return hipGetLastError();
-  };
-  if (dtype == F32::kCode) return run(location_grad_kernel<F32, F32>);
-  if (dtype == F16::kCode) return locations32 ? run(location_grad_kernel<F16, F32>) : run(location_grad_kernel<F16, F16>);
-  return locations32 ? run(location_grad_kernel<BF16, F32>) : run(location_grad_kernel<BF16, BF16>);
 }
 
 hipError_t launch_zero_rows(int elem_bytes, void *rows_of, const uint8_t *zero, long long rows, int n, hipStream_t stream) {
