@@ -146,9 +146,7 @@ template <int UNITS>
 __device__ __forceinline__ WindowPoint window_point(const WindowFrame<UNITS> &f, float y, float x, float m) {
   WindowPoint r;
   r.ok = y >= f.y_lo && y < f.y_hi && x >= f.x_lo && x < f.x_hi;
-  // by the masks of the comparisons: of a bool put together the compiler makes a number in every lane, and compares that
-  r.all = (__builtin_amdgcn_ballot_w64(y >= f.y_lo) & __builtin_amdgcn_ballot_w64(y < f.y_hi) & __builtin_amdgcn_ballot_w64(x >= f.x_lo) &
-           __builtin_amdgcn_ballot_w64(x < f.x_hi)) == __builtin_amdgcn_ballot_w64(true);
+  r.all = __builtin_amdgcn_ballot_w64(!r.ok) == 0;
   y = r.ok ? y : 0.f;          // also scrubs NaN and huge coordinates
   x = r.ok ? x : 0.f;
   const float fy = floorf(y), fx = floorf(x);
