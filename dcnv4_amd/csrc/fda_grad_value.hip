@@ -324,10 +324,11 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
   const int my_slot = tid >> kCellLanesLog2, my_part = tid & (LPC - 1);      // slot: (cell, sub-list), 64 of them
 
   // Item order.  The hardware deals consecutive workgroup ids to the 8 XCDs in turn.  When the (image, head) pairs
-  // divide evenly among them, an XCD works through its pairs one after the other, and through a pair level by level
-  // (coarsest first): the pair's regrouped grad_out rows and the level's point records and lists - a few MB - then
-  // stay in that XCD's L2 while its points are gathered.  Otherwise tiles are dealt over everything, in the same
-  // level order.
+  // divide evenly among them, an XCD keeps to its pairs and works through all of them level by level, coarsest first:
+  // a tile of a coarse level holds ten times the points of a fine one's, and those that come last have to be small.
+  // One pair after the other instead: 2 images of 100x152 in fp32, whole backward 386 us instead of 330 (locations
+  // all over the picture 407, 350), 4 of 128x128 in fp16 no difference.  Otherwise tiles are dealt over everything,
+  // in the same level order.
   const bool by_pair = BG % kXcds == 0 && (int)gridDim.x % kXcds == 0;
   const int workers = by_pair ? gridDim.x / kXcds : gridDim.x, me = by_pair ? blockIdx.x / kXcds : blockIdx.x;
   const int all_items = by_pair ? n_tiles * (BG / kXcds) : n_tiles * BG;
