@@ -189,9 +189,9 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
     for (int cn = 0; cn < 4; ++cn)
 #pragma unroll
       for (int v = 0; v < 2; ++v) raw[cn][v] = fetch(cn, v);
-    // a sum of each corner, the corners in turn: consecutive instructions do not wait for each other
-#pragma unroll
-    for (int cn = 0; cn < 4; ++cn) d[cn] = 0.f;
+    // two sums of each corner - one sum of twice the terms is 9 % further from 64 bits (16 fp32 channels) - all in turn: consecutive
+    // instructions do not wait for each other
+    float sum[4][2] = {};
 #pragma unroll
     for (int v = 0; v < 2; ++v)
 #pragma unroll
@@ -199,9 +199,12 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
 #pragma unroll
         for (int cn = 0; cn < 4; ++cn) {
           const uint32_t a = raw[cn][v][c], b = go_raw[v][c];
-          if constexpr (Tag::kBytes == 2) d[cn] = dot2_pair<Tag>(a, b, d[cn]);      // two channels per instruction, products and sums in fp32
-          else d[cn] = fmaf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), d[cn]);
+          float &s = sum[cn][c & 1];
+          if constexpr (Tag::kBytes == 2) s = dot2_pair<Tag>(a, b, s);      // two channels per instruction, products and sums in fp32
+          else s = fmaf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), s);
         }
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) d[cn] = sum[cn][0] + sum[cn][1];
 #pragma unroll
     for (int cn = 0; cn < 4; ++cn) {
       if constexpr (LPG >= 2) d[cn] += dcn::dpp_quad_xor1(d[cn]);

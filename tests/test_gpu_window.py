@@ -94,3 +94,26 @@ def test_window_gathers_carry_infinite_modulations(oracle, width, reach, dtype):
     infinite = abs(want) == float("inf")
     assert infinite.any() and not infinite.all() and (got[infinite] == want[infinite]).all()
     cabi.assert_close(got[~infinite], want[~infinite], *FWD_TOL[dtype], what="the others")
+
+
+@pytest.mark.parametrize("reach", [4, 0], ids=["window", "beyond"])
+@pytest.mark.parametrize("width,dtype", [(16, torch.float32), (32, torch.float32), (16, torch.float16), (32, torch.float16), (64, torch.float16),
+                                         (16, torch.bfloat16), (32, torch.bfloat16), (64, torch.bfloat16)])
+def test_gradient_of_the_modulation_sums_neighbouring_words_apart(width, reach, dtype):
+    """A corner's product with grad_out is two sums, of every other 4-byte word: words of 2^25, 1, -2^25, 1 give the number of ones,
+    which a single sum loses next to 2^25.  Points on pixels, where the gradient of a modulation is one corner's product."""
+    from dcnv4_amd import ext
+    b, h, w, groups = 2, 9, 13, 3
+    case = (b, h, w, groups, width, (3, 3, 1, 1, 1, 1, 1, 1), 0, 1.0, 0.0)
+    v, om, go, (geom, G, D, scale, rc) = _dcn_inputs(case, dtype, seed=width)
+    om.zero_()
+    word = 1 if dtype == torch.float32 else 2      # channels
+    for t, words in ((v, (2.0 ** 13, 1.0, -2.0 ** 13, 1.0)), (go, (2.0 ** 12, 1.0, 2.0 ** 12, 1.0))):
+        pattern = torch.zeros(4, word)
+        pattern[:, 0] = torch.tensor(words)
+        t.copy_(pattern.flatten().repeat(t.numel() // (4 * word)).view(t.shape).to(dtype))
+    with ext.launch_options(reach=reach, dual="off"):
+        _, gom = cabi.dcnv4_backward(v.cuda(), om.cuda(), go.cuda(), geom, G, D, scale, rc)
+    rows = gom[:, 1:-1, 1:-1, :groups * 27].reshape(b, h - 2, w - 2, groups, 27).cpu().float()
+    assert (rows[..., 18:] == width // word // 2).all(), rows[..., 18:].unique()
+    assert (rows[..., :18] == 0).all()      # all corners alike
