@@ -54,7 +54,7 @@ class LevelCheck {
 struct AttentionSaved {
   Arena arena;
   size_t query, features, value, locations, logits, sampled;      // query, features: their 16-bit copies under autocast
-  size_t value_wt, rows_wt, output_wt;
+  size_t value_wt, offsets_wt, logits_wt, output_wt;
 };
 
 struct Attention {
@@ -70,6 +70,10 @@ struct Attention {
   int64_t query_rows() const { return batch * queries; }
   int64_t feature_rows() const { return batch * pixels; }
   int64_t logits() const { return (int64_t)heads * levels * points; }
+  // The gradients of offsets and logits, and the two matrices turned, side by side: one product gives the query's gradient, rounded to 16
+  // bits once.  Not an fp32 one: a sum over both depths is further from 64 bits than one over each, added (depths of 256 and 128, 30400
+  // queries: fp32 products 3.8e-7 against 2.7e-7, fp16 1.36e-7 against 1.02e-7; one launch more, an encoder layer in fp32 1016 -> 1048 us).
+  bool side_by_side() const { return !query32; }
   // locations are rounded through fp16 by the operator: fp16 tensors hold them as they are used
   int location_code() const { return code == DCNV4_DTYPE_F16 ? DCNV4_DTYPE_F16 : DCNV4_DTYPE_F32; }
   int location_bytes() const { return code == DCNV4_DTYPE_F16 ? 2 : 4; }
@@ -119,13 +123,13 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
   narrowed(kOffsetsW, n_loc, width);
   narrowed(kLogitsW, n_log, width);
   narrowed(kOutputW, width, width);
-  // the offsets' and the logits' turned side by side, [width][n_loc + n_log]: one product gives the gradient of the query
+  // the offsets' and the logits' turned, [width][n_loc + n_log] or one behind the other
   turned[kOffsetsW] = !keep ? 0 : a.take((size_t)((n_loc + n_log) * width) * bytes());
-  turned[kLogitsW] = turned[kOffsetsW] + (size_t)n_loc * bytes();
+  turned[kLogitsW] = turned[kOffsetsW] + (size_t)(side_by_side() ? n_loc : n_loc * width) * bytes();
   for (Input i : {kValueB, kOffsetsB, kLogitsB, kOutputB})
     if (params[i].defined()) narrowed(i, 1, params[i].numel());
   a.allocate(query);
-  s->value_wt = turned[kValueW]; s->rows_wt = turned[kOffsetsW]; s->output_wt = turned[kOutputW];
+  s->value_wt = turned[kValueW]; s->offsets_wt = turned[kOffsetsW]; s->logits_wt = turned[kLogitsW]; s->output_wt = turned[kOutputW];
   for (int i = kValueW; i < kInputs; ++i) {
     const Tensor &t = params[i];
     const bool matrix = t.defined() && t.dim() == 2, turn = matrix && keep;
@@ -134,7 +138,7 @@ Tensor Attention::forward(const Tensor &query, const Tensor &reference, const Te
     q.from = static_cast<const float *>(t.const_data_ptr());
     q.to = half ? a.at(as_is[i]) : nullptr;
     q.turned = turn ? a.at(turned[i]) : nullptr;
-    if (i == kOffsetsW || i == kLogitsW) q.turned_pitch = (int)(n_loc + n_log);
+    if (side_by_side() && (i == kOffsetsW || i == kLogitsW)) q.turned_pitch = (int)(n_loc + n_log);
     q.n = matrix ? (int)t.size(0) : 1;
     q.k = matrix ? (int)t.size(1) : (int)t.numel();
   }
@@ -190,7 +194,9 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
 
   Arena t;
   const size_t d_sampled = t.take((size_t)(query_rows() * width) * bytes()), d_value = t.take((size_t)(feature_rows() * width) * bytes()),
-               d_rows = t.take((size_t)(query_rows() * (n_loc + n_log)) * bytes());      // of the offsets and the logits, side by side
+               d_offsets = t.take((size_t)(query_rows() * (n_loc + n_log)) * bytes()),
+               d_logits = d_offsets + (size_t)(side_by_side() ? n_loc : query_rows() * n_loc) * bytes();
+  const int64_t offsets_pitch = side_by_side() ? n_loc + n_log : n_loc, logits_pitch = side_by_side() ? n_loc + n_log : n_log;
   const size_t ws_bytes = flash_deform_attn_gfx950_backward_workspace_bytes(code, batch, (int)pixels, heads, (int)width / heads, levels,
                                                                             (int)queries, points);
   const size_t ws = t.take(ws_bytes);
@@ -201,7 +207,8 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
     FdaLayerBackward p = {};
     p.value = a.at(s.value); p.locations = a.at(s.locations); p.logits = a.at(s.logits);
     p.shapes = shapes.const_data_ptr<int64_t>(); p.starts = starts.const_data_ptr<int64_t>();
-    p.grad_output = t.at(d_sampled); p.grad_value = t.at(d_value); p.grad_rows = t.at(d_rows);
+    p.grad_output = t.at(d_sampled); p.grad_value = t.at(d_value);
+    p.grad_offsets = t.at(d_offsets); p.grad_logits = t.at(d_logits); p.offsets_pitch = (int)offsets_pitch; p.logits_pitch = (int)logits_pitch;
     p.workspace = t.at(ws); p.workspace_bytes = ws_bytes;
     p.dtype = code; p.location_dtype = location_code();
     p.batch = (int)batch; p.spatial_size = (int)pixels; p.heads = heads; p.head_channels = (int)width / heads;
@@ -223,15 +230,23 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
   }
   if (want[kQuery]) {
     g[kQuery] = at::empty({batch, queries, width}, query_options);
-    result(product(t.at(d_rows), a.at(s.rows_wt), nullptr, query_rows(), n_loc + n_log, width, nullptr), g[kQuery], query32);
+    if (side_by_side()) {
+      result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc + n_log, width, nullptr), g[kQuery], query32);
+    } else {
+      result(product(t.at(d_offsets), a.at(s.offsets_wt), nullptr, query_rows(), n_loc, width, nullptr), g[kQuery], query32);
+      LinearLaunch more = product(t.at(d_logits), a.at(s.logits_wt), nullptr, query_rows(), n_log, width, nullptr);
+      if (half) more.p[0].residual32 = static_cast<const float *>(g[kQuery].const_data_ptr());
+      else more.p[0].residual = g[kQuery].const_data_ptr();
+      result(more, g[kQuery], query32);
+    }
   }
   const void *q_in = half && query32 ? a.at(s.query) : ptr(query), *f_in = half && features32 ? a.at(s.features) : ptr(features);
   const auto fp32 = params[kValueW].options();
   auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n, int64_t pitch) -> WeightGradient {
     return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1], pitch};
   };
-  const WeightGradient value = gradient(kValueW, t.at(d_value), f_in, width, 0), offsets = gradient(kOffsetsW, t.at(d_rows), q_in, n_loc, n_loc + n_log),
-                       logit = gradient(kLogitsW, t.at(d_rows + (size_t)n_loc * bytes()), q_in, n_log, n_loc + n_log),
+  const WeightGradient value = gradient(kValueW, t.at(d_value), f_in, width, 0), offsets = gradient(kOffsetsW, t.at(d_offsets), q_in, n_loc, offsets_pitch),
+                       logit = gradient(kLogitsW, t.at(d_logits), q_in, n_log, logits_pitch),
                        output = gradient(kOutputW, grad.const_data_ptr(), a.at(s.sampled), width, 0);
   if (query_rows() == feature_rows()) weight_gradients(code, fp32, {{query_rows(), {output, offsets, value, logit}}}, stream);
   else weight_gradients(code, fp32, {{query_rows(), {output, offsets, logit}}, {feature_rows(), {value}}}, stream);

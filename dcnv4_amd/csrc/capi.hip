@@ -1040,8 +1040,9 @@ struct FdaRows {
   const void *sla, *loc, *logits;
   void *grad_sla, *grad_loc, *grad_logits;
   int loc_bytes;      // 0: packed rows
-  // a layer's (FdaLayerBackward), in place of grad_loc and grad_logits
-  void *grad_rows = nullptr;
+  // a layer's (FdaLayerBackward), in place of grad_loc
+  void *grad_offsets = nullptr;
+  int offsets_pitch = 0, logits_pitch = 0;
   const float *reference = nullptr;
   int reference_kind = 0;
   const uint8_t *zero_rows = nullptr;
@@ -1054,10 +1055,13 @@ static void fda_set_rows(FdaLaunch *F, const FdaRows &r, const FdaProblem &pr, i
   F->loc = r.loc ? at(r.loc, pairs * 2 * LK, r.loc_bytes) : nullptr;
   F->grad_loc = r.grad_loc ? at(r.grad_loc, pairs * 2 * LK, r.loc_bytes) : nullptr;
   F->logits = r.logits ? at(r.logits, pairs * LK, pr.s) : nullptr;
-  F->grad_logits = r.grad_logits ? at(r.grad_logits, pairs * LK, pr.s) : nullptr;
+  const size_t row0 = (size_t)b0 * F->Q;
+  F->grad_logits = r.grad_logits ? at(r.grad_logits, r.grad_offsets ? row0 * r.logits_pitch : pairs * LK, pr.s) : nullptr;
   F->loc_f32 = r.loc_bytes == 4 ? 1 : 0;
-  F->grad_rows = r.grad_rows ? at(r.grad_rows, pairs * 3 * LK, pr.s) : nullptr;
-  F->reference = r.reference ? r.reference + (size_t)b0 * F->Q * F->L * r.reference_kind : nullptr;
+  F->grad_offsets = r.grad_offsets ? at(r.grad_offsets, row0 * r.offsets_pitch, pr.s) : nullptr;
+  F->offsets_pitch = r.offsets_pitch;
+  F->logits_pitch = r.logits_pitch;
+  F->reference = r.reference ? r.reference + row0 * F->L * r.reference_kind : nullptr;
   F->reference_kind = r.reference_kind;
 }
 
@@ -1185,7 +1189,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
                            num_points, im2col_step, d_stride, block_thread))
     return rc;
   if (int rc = rows.loc_bytes == 0         ? check_ptrs({value, rows.sla, grad_output, grad_value, rows.grad_sla})
-               : rows.grad_rows != nullptr ? check_ptrs({value, rows.loc, rows.logits, grad_output, grad_value, rows.grad_rows})
+               : rows.grad_offsets != nullptr ? check_ptrs({value, rows.loc, rows.logits, grad_output, grad_value, rows.grad_offsets, rows.grad_logits})
                         : check_ptrs({value, rows.loc, rows.logits, grad_output, grad_value, rows.grad_loc, rows.grad_logits}))
     return rc;
   if (spatial_shapes == nullptr || level_start_index == nullptr) return fail(DCNV4_ERR_RUNTIME, "null level tensors");
@@ -1549,8 +1553,10 @@ int depthwise_backward_fp32_grads(const void *input, const void *weight, const v
 int fda_layer_backward(const FdaLayerBackward &p, hipStream_t stream) {
   int loc_bytes = 0;
   if (int rc = fda_check_split(p.dtype, p.location_dtype, &loc_bytes)) return rc;
-  FdaRows rows{nullptr, p.locations, p.logits, nullptr, nullptr, nullptr, loc_bytes};
-  rows.grad_rows = p.grad_rows;
+  FdaRows rows{nullptr, p.locations, p.logits, nullptr, nullptr, p.grad_logits, loc_bytes};
+  rows.grad_offsets = p.grad_offsets;
+  rows.offsets_pitch = p.offsets_pitch;
+  rows.logits_pitch = p.logits_pitch;
   rows.reference = p.reference;
   rows.reference_kind = p.reference_kind;
   rows.zero_rows = p.zero_rows;

@@ -131,7 +131,7 @@ __device__ __forceinline__ void fda_unstage_grads(const float *lds, const FdaLau
     return;
   }
   const float inv_2lk = 1.f / (float)(2 * LK), inv_lk = 1.f / (float)LK;
-  if (p.grad_rows != nullptr) {
+  if (p.grad_offsets != nullptr) {
     // Of the offsets that the locations come from, and of the logits behind them; points come in fours (the layer asks for that), so four
     // elements lie in one level. Each step rounded as the framework's operators round it.
     const int per_pair = row_len / 4;
@@ -141,9 +141,10 @@ __device__ __forceinline__ void fda_unstage_grads(const float *lds, const FdaLau
       const int r = fdiv20(j, inv_h), g = g0 + j - r * heads_here;
       const f32x4 in = *reinterpret_cast<const f32x4 *>(lds + j * row_len + e);
       float v[4] = {in.x, in.y, in.z, in.w};
-      int at = p.G * 2 * LK + g * LK + e - 2 * LK;
+      const size_t row = (size_t)(row0 + r);
+      elem_t *dst = reinterpret_cast<elem_t *>(p.grad_logits) + row * p.logits_pitch + g * LK + e - 2 * LK;
       if (e < 2 * LK) {
-        at = g * 2 * LK + e;
+        dst = reinterpret_cast<elem_t *>(p.grad_offsets) + row * p.offsets_pitch + g * 2 * LK + e;
         const int l = fdiv20(e, inv_2k);
         auto round4 = [&] { Pack<Tag, 4>::decode(Pack<Tag, 4>::encode(v), v); };
 #pragma unroll
@@ -154,7 +155,7 @@ __device__ __forceinline__ void fda_unstage_grads(const float *lds, const FdaLau
 #pragma unroll
           for (int c = 0; c < 4; ++c) v[c] /= (c & 1) ? h : w;
         } else {
-          const float *size = p.reference + ((size_t)(row0 + r) * p.L + l) * 4 + 2;
+          const float *size = p.reference + (row * p.L + l) * 4 + 2;
 #pragma unroll
           for (int c = 0; c < 4; ++c) v[c] = mul_rn(mul_rn(v[c], 0.5f), size[c & 1]);
           round4();
@@ -162,7 +163,7 @@ __device__ __forceinline__ void fda_unstage_grads(const float *lds, const FdaLau
           for (int c = 0; c < 4; ++c) v[c] /= (float)p.K;
         }
       }
-      *reinterpret_cast<typename Pack<Tag, 4>::raw_t *>(reinterpret_cast<elem_t *>(p.grad_rows) + (size_t)(row0 + r) * p.G * row_len + at) = Pack<Tag, 4>::encode(v);
+      *reinterpret_cast<typename Pack<Tag, 4>::raw_t *>(dst) = Pack<Tag, 4>::encode(v);
     }
     return;
   }

@@ -249,8 +249,9 @@ struct FdaLaunch {
   int tile_stride;          // table row length: an upper bound of the tiles of one level
   int n_img;
   int tile_points;          // a level whose tiles would collect more of them is cut finer
-  // a layer's backward: in place of grad_loc and grad_logits, gradients of its offsets and logits, tensor dtype
-  void *grad_rows;          // [n_row][G * 2*L*K offsets, G * L*K logits]
+  // a layer's backward: in place of grad_loc the gradients of the offsets that the locations come from, tensor dtype
+  void *grad_offsets;       // [n_row][G * 2*L*K], rows offsets_pitch elements apart; those of grad_logits are then logits_pitch apart
+  int offsets_pitch, logits_pitch;      // multiples of 4
   const float *reference;   // [n_row, L, reference_kind]; of the locations: 2 a point, 4 a box
   int reference_kind;
   const uint8_t *zero_rows; // [n_img, N]; null, or where grad_value is zero

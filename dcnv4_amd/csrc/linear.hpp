@@ -162,14 +162,15 @@ hipError_t launch_read_back(const int64_t *numbers, int n, int64_t *host, hipStr
 hipError_t launch_narrow_rows(int dtype, const void *src, bool src32, void *dst, size_t n, const float *row_scale, size_t scale_elements,
                               hipStream_t stream);
 
-// The backward of deformable attention inside its layer (capi.hip): in place of the gradients of the locations and logits, those of the
-// offsets and logits side by side, [rows][heads * 2 * levels * points, heads * levels * points] in the dtype; grad_value is zero in rows
-// whose byte in zero_rows (may be null) is not.  Checks and errors are those of the library's entry point.
+// The backward of deformable attention inside its layer (capi.hip): in place of the gradients of the locations those of the offsets,
+// [rows][heads * 2 * levels * points] in the dtype, their rows and those of the logits' gradients a pitch (elements, a multiple of 4) apart;
+// grad_value is zero in rows whose byte in zero_rows (may be null) is not.  Checks and errors are those of the library's entry point.
 struct FdaLayerBackward {
   const void *value;
   const int64_t *shapes, *starts;
   const void *locations, *logits, *grad_output;
-  void *grad_value, *grad_rows, *workspace;
+  void *grad_value, *grad_offsets, *grad_logits, *workspace;
+  int offsets_pitch, logits_pitch;
   size_t workspace_bytes;
   int dtype, location_dtype, batch, spatial_size, heads, head_channels, levels, queries, points;
   const float *reference;

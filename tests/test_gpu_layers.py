@@ -176,6 +176,32 @@ def test_attention_layer_in_one_call_matches_the_composition(levels, queries, ki
         assert not results[0][2][mask].any()
 
 
+# products of few rows and of many
+@pytest.mark.parametrize("amp", [None, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("h,w", [(6, 9), (64, 100)], ids=["few", "many"])
+def test_query_gradient_in_fp32_is_two_products_added(h, w, amp):
+    """One sum over both depths would be further from 64 bits.  With a query of zeros neither weight moves a point, so that the gradients
+    of offsets and logits are the same whichever weight is zero: the gradient with both weights is the two with one of them, added."""
+    import dcnv4_amd
+    torch.manual_seed(h)
+    m = dcnv4_amd.FlashDeformAttn(256, 1, 8, 4).cuda()
+    shapes, starts = torch.tensor([[h, w]], device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    features, reference = torch.randn(1, h * w, 256, device="cuda"), torch.rand(1, h * w, 1, 2, device="cuda")
+    grad = torch.randn(1, h * w, 256, device="cuda")
+    weights = [torch.randn_like(p.weight) for p in (m.sampling_offsets, m.attention_weights)]
+    def query_gradient(*kept):
+        with torch.no_grad():
+            for p, weight, keep in zip((m.sampling_offsets, m.attention_weights), weights, kept):
+                p.weight.copy_(weight * keep)
+        query = torch.zeros(1, h * w, 256, device="cuda", requires_grad=True)
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            out = m(query, reference, features, shapes, starts)
+        assert out.grad_fn.name() == "FlashDeformAttnBackward"
+        return torch.autograd.grad(out, query, grad.to(out.dtype))[0]
+    both, offsets, logits = query_gradient(1, 1), query_gradient(1, 0), query_gradient(0, 1)
+    assert offsets.any() and logits.any() and torch.equal(both, logits + offsets)
+
+
 def test_attention_layer_reads_changed_level_shapes_again():
     import dcnv4_amd
     m = dcnv4_amd.FlashDeformAttn(64, 1, 4, 4).cuda()
