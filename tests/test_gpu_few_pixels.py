@@ -83,6 +83,16 @@ def test_products_of_few_rows(rows, width, depth, dtype):
     assert _rel(ext.linear_forward(a, w, b, gamma, res), (product + b.double()) * gamma.double() + res.double()) < unit + 1e-6
 
 
+def test_products_of_few_rows_add_their_parts_in_pairs():
+    """Eight waves share a depth of 128 in fp32, sixteen elements each: their sums 2^25, 0, 2, 2, 1, 1, 1, 1 are exact in pairs; added one
+    after the other all but the first are lost."""
+    from dcnv4_amd import ext
+    w = torch.zeros(8, 128, device="cuda")
+    w[:, ::16] = torch.tensor([2.0 ** 25, 0.0, 2.0, 2.0, 1.0, 1.0, 1.0, 1.0], device="cuda")
+    for rows in (1, 17):
+        assert (ext.linear_forward(torch.ones(rows, 128, device="cuda"), w) == 2.0 ** 25 + 8).all()
+
+
 # pixels x features in tiles of 16 x 16 (252 of them, the depth in one request and in two) and of 32 x 32
 @pytest.mark.parametrize("channels,size", [(112, (5, 15, 14)), (456, (1, 3, 5)), (112, (8, 28, 28))])
 def test_downsampling_of_few_pixels(channels, size):
