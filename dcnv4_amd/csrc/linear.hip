@@ -524,7 +524,9 @@ __global__ void __launch_bounds__(kSampledWaves * 64) sampled_linear_kernel(cons
   __syncthreads();
 
   // rows beyond the live ones hold whatever the LDS held: theirs are columns of the result of their own, which go nowhere
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // Four sums a wave, eight with the other half's: as short as the chains of eight waves that share a depth (linear_few_rows_kernel).
+  constexpr int kSums = 4;
+  f32x4 acc[kSums] = {};
   for (int s0 = split; s0 < steps; s0 += kTogether * kSampledSplits) {
     if (s0 != split) request(s0);
 #pragma unroll
@@ -532,10 +534,10 @@ __global__ void __launch_bounds__(kSampledWaves * 64) sampled_linear_kernel(cons
       const int s = s0 + u * kSampledSplits, kk = s * 32 + kb * 8;
       if (s >= steps) break;
       const u32x4 fm = kk < k ? *reinterpret_cast<const u32x4 *>(rows + r16 * norm_row_bytes(k) + kk * 2) : u32x4{0u, 0u, 0u, 0u};
-      acc = mfma_64_bytes<Tag>(fn[u], fm, acc);
+      acc[u % kSums] = mfma_64_bytes<Tag>(fn[u], fm, acc[u % kSums]);
     }
   }
-  *reinterpret_cast<f32x4 *>(&part[split][r16][fragment * 16 + kb * 4]) = acc;
+  *reinterpret_cast<f32x4 *>(&part[split][r16][fragment * 16 + kb * 4]) = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   __syncthreads();
   if (!finishes) return;
   float v[8];

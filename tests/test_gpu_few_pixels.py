@@ -59,6 +59,27 @@ def test_layer_of_few_pixels_matches_the_modules_in_fp32(channels, groups, post_
     assert _rel(got[-1, -1], want[-1, -1]) < 4 * tol and _rel(got[..., -8:], want[..., -8:]) < 2 * tol
 
 
+def test_layer_of_few_pixels_sums_a_depth_in_eight_chains():
+    """Eight chains, as many as products of few rows have: slices of 32 channels that are eight apart meet in one sum, where 2^25 and
+    -2^25 are gone before the ones of the slices between are added.  The operator's points lie on their pixels and its values are the
+    projection's biases, the MLP's are zero."""
+    from dcnv4_amd import ext
+    from dcnv4_amd.models.flash_intern_image import InternImageLayer
+    layer = InternImageLayer(512, 32).cuda().half().eval()
+    with torch.no_grad():
+        for p in (layer.dcn.value_proj.weight, layer.dcn.offset_mask.weight, layer.dcn.offset_mask.bias, layer.dcn.output_proj.weight, layer.mlp.fc2.weight):
+            p.zero_()
+        layer.dcn.value_proj.bias.fill_(1.0)
+        layer.dcn.value_proj.bias[0] = layer.dcn.value_proj.bias[8 * 32] = 2.0 ** 12
+        layer.dcn.offset_mask.bias[:32 * 27].view(32, 27)[:, 18 + 4] = 1.0
+        layer.dcn.output_proj.weight[:, 0], layer.dcn.output_proj.weight[:, 8 * 32] = 2.0 ** 13, -2.0 ** 13
+        for slice in range(1, 8):
+            layer.dcn.output_proj.weight[:, slice * 32] = 1.0
+        x = torch.zeros(1, 49, 512, device="cuda", dtype=torch.float16)
+        assert ext._native.sampled_linear_fits(x, 7, 7, 32, 3)
+        assert (layer(x, (7, 7)) == 7.0).all()
+
+
 def test_the_rule_of_the_kernel_for_few_pixels():
     from dcnv4_amd import ext
     fits = lambda n, h, w, c, kernel=3, dtype=torch.float16: ext._native.sampled_linear_fits(torch.empty(n, h * w, c, dtype=dtype, device="meta"), h, w, c // 16, kernel)
