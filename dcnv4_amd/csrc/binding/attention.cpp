@@ -392,9 +392,21 @@ PyObject *py_attention_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// attention_backward_tiled(value, levels, queries, points): whether the gradient of value [batch, pixels, heads, channels] is added up by tiles
+PyObject *py_attention_backward_tiled(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Args a("attention_backward_tiled", args, n, 4);
+  const Tensor &value = a.tensor();
+  const int levels = a.integer(), queries = a.integer(), points = a.integer();
+  if (value.dim() != 4) raise_runtime("value has four dimensions");
+  return PyBool_FromLong(fda_backward_tiled(dtype_code(value, "value"), (int)value.size(1), (int)value.size(2), (int)value.size(3), levels, queries, points));
+  END_HANDLE_TH_ERRORS
+}
+
 }  // namespace
 
 PyMethodDef attention_methods[] = {
+    {"attention_backward_tiled", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_attention_backward_tiled)), METH_FASTCALL, nullptr},
     {"attention_layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(py_attention_layer)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

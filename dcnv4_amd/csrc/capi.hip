@@ -775,6 +775,20 @@ char *at(void *base, size_t elems, int s) { return static_cast<char *>(base) + e
 
 namespace dcn {
 
+bool fda_backward_tiled(int dtype, int spatial_size, int heads, int head_channels, int levels, int queries, int points) {
+  // the tiled grad_value kernel addresses one image's sampling_loc_attn and grad_out with 32-bit byte offsets
+  const unsigned long long row_bytes = (unsigned long long)std::max(heads, 1) * std::max(3 * levels * points, head_channels) * 4ull;
+  // fp32 tensors with fewer than a point to three pixels (a decoder's few hundred queries against an encoder's pyramid): the atomic
+  // scatter adds straight into grad_value.  us, binned / atomic, four levels and points, 8 heads of 32 channels, points within some
+  // pixels of each query's, images of a pyramid from 100 x 152: 2 images, 300 queries (0.24 points a pixel) 58 / 41, 500 (0.4) 60 / 59,
+  // 900 63 / 98; 6 images, 300 126 / 110, 500 133 / 158.  Points all over the picture: 1 image of 76 x 81 (0.27) 34 / 25, 2 of 78 x 97 (0.33) 44 /
+  // 57, 2 of 104 x 99 (0.42) 56 / 86.  Not by the amount of work: with more points to a cell the atomics of one address wait for each other,
+  // one head of 8 channels, 6875 queries on 4 x 4 pixels 73 / 417, 1720 on 30 x 40 46 / 131.
+  const bool sparse = g_opt.scatter == kOptAuto && elem_bytes(dtype) == 4 && 3ll * queries * levels * points < (long long)spatial_size;
+  return fda_tiled_shape(head_channels, levels, queries, points) && fda_tiled_enabled() && !sparse &&
+         (unsigned long long)queries * row_bytes < (1ull << 31);
+}
+
 static bool prepare_sampled_linear(DcnProblem *pr, int dtype, const SampledLinear &p) {
   if (dcn_prepare(pr, false, dtype, p.batch, p.height, p.width, p.group, p.group_channels, p.kernel, p.kernel, 1, 1, p.pad, p.pad, p.dilation,
                   p.dilation, p.offset_scale, 256, p.remove_center, p.row, 0, 0, 0) != DCNV4_OK)
@@ -1171,19 +1185,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
                              int head_channels, int num_levels, int num_query, int num_points, int im2col_step,
                              int d_stride, int block_thread, void *stream) {
   FdaProblem pr;
-  // the tiled grad_value kernel addresses one image's sampling_loc_attn and grad_out with 32-bit byte offsets
-  const unsigned long long row_bytes = (unsigned long long)std::max(num_heads, 1) *
-                                       std::max(3 * num_levels * num_points, head_channels) * 4ull;
-  // fp32 tensors with few sampling points (a decoder's few hundred queries against an encoder's pyramid): the atomic scatter adds straight
-  // into grad_value.  It costs 35 ns a query of 8 heads of 32 channels and 16 points, where the binned kernels cost 8, and the clearing
-  // of grad_value; the binned kernels 15 us to begin with and 0.7 ns a pixel, each of which is in a tile somebody walks.  us, binned /
-  // atomic, images of a pyramid from 100 x 152: 2 images, 300 queries 58 / 41, 500 60 / 59, 900 63 / 98; 6 images, 200 122 / 78, 300
-  // 126 / 110, 500 133 / 158.  From 44 x 36: 2 images, 200 33 / 24, 300 34 / 30, 500 36 / 42; 6 images, 100 44 / 32, 200 46 / 54.
-  const double channels = (double)num_heads * head_channels * batch;
-  const bool sparse = g_opt.scatter == kOptAuto && elem_bytes(dtype) == 4 &&
-                      5.0 * num_query * num_levels * num_points * channels < spatial_size * channels + 11e6;
-  const bool tiled = fda_tiled_shape(head_channels, num_levels, num_query, num_points) && fda_tiled_enabled() && !sparse &&
-                     (unsigned long long)num_query * row_bytes < (1ull << 31);
+  const bool tiled = fda_backward_tiled(dtype, spatial_size, num_heads, head_channels, num_levels, num_query, num_points);
   // the tiled path gathers only: 16-byte lanes; the atomic path wants one channel per lane
   if (int rc = fda_prepare(&pr, true, !tiled, dtype, batch, spatial_size, num_heads, head_channels, num_levels, num_query,
                            num_points, im2col_step, d_stride, block_thread))

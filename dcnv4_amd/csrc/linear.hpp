@@ -178,5 +178,7 @@ struct FdaLayerBackward {
   const uint8_t *zero_rows;
 };
 int fda_layer_backward(const FdaLayerBackward &p, hipStream_t stream);
+// Whether the backward of deformable attention adds up grad_value by tiles; if not, with atomics.
+bool fda_backward_tiled(int dtype, int spatial_size, int heads, int head_channels, int levels, int queries, int points);
 
 }  // namespace dcn

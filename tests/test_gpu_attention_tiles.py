@@ -44,10 +44,12 @@ def test_grad_value_by_tiles(oracle, name, dtype):
         assert (np.abs(cabi.f64(g) - want) <= bound).all(), float((np.abs(cabi.f64(g) - want) / bound).max())
 
 
-# fp32 tensors with few points take the atomic scatter by themselves: on either side of where, both ways against each other
-@pytest.mark.parametrize("batch,queries", [(2, 280), (2, 320), (6, 100), (6, 120)])
+# fp32 tensors with fewer points than a third of the pixels take the atomic scatter by themselves: on either side of where, both ways
+# against each other
+@pytest.mark.parametrize("batch,queries", [(2, 28), (2, 29), (2, 280), (2, 320), (6, 100), (6, 120)])
 def test_few_points_choose_a_way(batch, queries):
     v, shp, st, sla, go = (t.cuda() for t in make_fda_inputs(batch, [(30, 34), (15, 17), (8, 9), (4, 5)], 8, 32, 4, queries, seed=3, dtype=torch.float32))
+    assert ext._native.attention_backward_tiled(v, 4, queries, 4) == (3 * 16 * queries >= v.shape[1]) == (queries > 28)
     auto, rows = cabi.fda_backward(v, shp, st, sla, go, 4)
     sizes, _ = cabi.fda_backward(v, shp, st, sla, go.abs(), 4)
     for scatter in ("tiled", "atomic"):
@@ -56,3 +58,15 @@ def test_few_points_choose_a_way(batch, queries):
         # the same terms in another order, at most 4 * queries * 4 of them
         assert ((one - auto).abs() <= sizes * (2 * 16 * queries * 2.0 ** -24) + 1e-30).all(), scatter
         torch.testing.assert_close(one_rows, rows, rtol=1e-4, atol=1e-5)
+
+
+def test_many_points_on_few_pixels_go_by_tiles_however_little_work_they_are():
+    """Atomics of one address wait for each other: one head of 8 channels, 6875 queries on 4 x 4 pixels, 417 us against 73."""
+    tiled = lambda pixels, heads, channels, levels, queries, dtype=torch.float32: ext._native.attention_backward_tiled(
+        torch.empty(1, pixels, heads, channels, dtype=dtype, device="meta"), levels, queries, 4)
+    assert tiled(16, 1, 8, 1, 6875) and tiled(16, 8, 32, 1, 214) and tiled(1600, 1, 8, 4, 1720) and tiled(80, 1, 8, 2, 3437)
+    assert tiled(20197, 8, 32, 4, 421) and not tiled(20197, 8, 32, 4, 420) and tiled(20197, 8, 32, 4, 300, torch.float16)
+    with ext.launch_options(scatter="tiled"):
+        assert tiled(20197, 8, 32, 4, 300)
+    with ext.launch_options(scatter="atomic"):
+        assert not tiled(16, 1, 8, 1, 6875)
