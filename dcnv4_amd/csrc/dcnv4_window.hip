@@ -373,10 +373,11 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
   if (word * kPerWord < run) {
     constexpr int kStep = kWindowThreads / kTeam;
     const int step_rows = __builtin_amdgcn_readfirstlane(exact_div(kStep, inv_tw)), step_cols = kStep - step_rows * t.tw;
-    const int pix_pitch = p.P_pad * Tag::kBytes, row_pitch = p.Wo * pix_pitch;
+    const size_t pix_pitch = (size_t)p.P_pad * Tag::kBytes, row_pitch = p.Wo * pix_pitch;      // rows of 2 GiB and more are allowed
+    const size_t step = step_rows * row_pitch + step_cols * pix_pitch, wrap = row_pitch - t.tw * pix_pitch;
     const int pix = threadIdx.x / kTeam, y = exact_div(pix, inv_tw);
     int x = pix - y * t.tw, from = (y * p.gt_w + x) * kPitch + word * kPerWord;
-    size_t to = (size_t)y * row_pitch + (size_t)x * pix_pitch + (size_t)word * 4;
+    size_t to = y * row_pitch + x * pix_pitch + (size_t)word * 4;
     const bool whole = word * kPerWord + kPerWord <= run;
     for (int left = t.th * t.tw - pix; left > 0; left -= kStep) {
       const elem_t *src = reinterpret_cast<const elem_t *>(lds) + from;
@@ -387,11 +388,11 @@ __global__ void __launch_bounds__(kWindowThreads, 4) dcnv4_offset_mask_grad_wind
       } else {
         *reinterpret_cast<elem_t *>(dst) = *src;
       }
-      x += step_cols; from += (step_rows * p.gt_w + step_cols) * kPitch; to += (size_t)(step_rows * row_pitch + step_cols * pix_pitch);
+      x += step_cols; from += (step_rows * p.gt_w + step_cols) * kPitch; to += step;
       const bool over = x >= t.tw;
       x -= over ? t.tw : 0;
       from += over ? (p.gt_w - t.tw) * kPitch : 0;
-      to += over ? (size_t)(row_pitch - t.tw * pix_pitch) : 0;
+      to += over ? wrap : 0;
     }
   }
   const int tail = p.P_pad - p.G * 27;

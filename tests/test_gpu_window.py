@@ -117,3 +117,18 @@ def test_gradient_of_the_modulation_sums_neighbouring_words_apart(width, reach, 
     rows = gom[:, 1:-1, 1:-1, :groups * 27].reshape(b, h - 2, w - 2, groups, 27).cpu().float()
     assert (rows[..., 18:] == width // word // 2).all(), rows[..., 18:].unique()
     assert (rows[..., :18] == 0).all()      # all corners alike
+
+
+def test_rows_of_offsets_that_lie_gigabytes_apart():
+    """Eight rows of 16393 pixels whose offset rows have 4096 elements are 2.1 GB, more than an int holds: the last column of tiles is one
+    pixel wide, so that a lane of grad_offset_mask's stores goes on eight rows further down."""
+    h, w = 10, 16393
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    v, go = (torch.randn(1, h, w, 16, generator=gen, device="cuda") for _ in range(2))
+    packed = torch.randn(1, h, w, 32, generator=gen, device="cuda")
+    wide = torch.zeros(1, h, w, 4096, device="cuda")
+    wide[..., :27] = packed[..., :27]
+    geom = (3, 3, 1, 1, 1, 1, 1, 1)
+    _, want = cabi.dcnv4_backward(v, packed, go, geom, 1, 16, 1.0, 0)
+    _, got = cabi.dcnv4_backward(v, wide, go, geom, 1, 16, 1.0, 0)
+    assert torch.equal(got[..., :27], want[..., :27]) and not got[..., 27:].any()
