@@ -345,10 +345,12 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
       if (lane == 0) s_item[slot] = Item{-1, 0, 0, 0, 0, 0, 0, 0};
       return;
     }
-    const int rank = quotient((int)it, pairs);
-    int pair = (int)it - rank * pairs;
+    int of = pairs, own = lane;
+    asm volatile("" : "+s"(of), "+v"(own));                   // a reciprocal and an address are not worth registers all the time
+    const int rank = quotient((int)it, of);
+    int pair = (int)it - rank * of;
     if (by_pair) pair = pair * kXcds + blockIdx.x % kXcds;
-    const int begin = lane < p.L ? s_first[lane] : all_items;
+    const int begin = own < p.L ? s_first[own] : all_items;
     const int level = __builtin_ctzll(__ballot(rank >= begin));      // first ranks fall with the level
     const LevelPlan lp = s_plan[level];
     const int tile = rank - __builtin_amdgcn_readlane(begin, level), ty = quotient(tile, lp.ntx), y0 = ty * lp.th, x0 = (tile - ty * lp.ntx) * lp.tw;
@@ -583,9 +585,11 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
         }
         __syncthreads();                                     // the entries have been read
         float *s_part = reinterpret_cast<float *>(s_entry);  // [kTileCells][LPC][CW]
+        int own = tid;
+        asm volatile("" : "+v"(own));                        // as above
         static_assert(kTileCells * LPC * CW * sizeof(float) <= (4 * kBatch + 2) * sizeof(u32x2), "room for the partial sums");
 #pragma unroll
-        for (int c = 0; c < CW; ++c) s_part[tid * CW + c] = acc[c];
+        for (int c = 0; c < CW; ++c) s_part[own * CW + c] = acc[c];
         __syncthreads();
         if (my_sub == 0) {
           const int each = 1 << max(0, kWaveSlotsLog2 - cells_log2);

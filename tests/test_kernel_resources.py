@@ -39,7 +39,8 @@ def scratch_bytes(tmp_path_factory):
 
 # kernels by what their names hold, and how many instances there are
 @pytest.mark.parametrize("kernel,instances", [(r"dcnv4_grad_value_kernel<\w+, 9, 16, 2, \d+, (true|false)>", 12),
-                                              (r"linear_rows_kernel<\w+, [1-8], (true|false)>", 32), (r"mlp_kernel<\w+, [2-7], (true|false)>", 24)])
+                                              (r"linear_rows_kernel<\w+, [1-8], (true|false)>", 32), (r"mlp_kernel<\w+, [2-7], (true|false)>", 24),
+                                              (r"fda_grad_value_kernel<\w+, [248], [48]>", 9), (r"sampled_linear_kernel<\w+>", 2)])
 def test_kernels_without_scratch_memory(scratch_bytes, kernel, instances):
     found = {name: size for name, size in scratch_bytes.items() if re.search(kernel, name)}
     assert len(found) == instances, sorted(found)
