@@ -789,6 +789,11 @@ bool fda_backward_tiled(int dtype, int spatial_size, int heads, int head_channel
          (unsigned long long)queries * row_bytes < (1ull << 31);
 }
 
+void fda_backward_tile(int h, int w, long long points, long long pairs, int *tile_h, int *tile_w) {
+  const FdaTile tile = fda_tile(h, w, points, fda_tile_points(points * pairs));
+  *tile_h = tile.h; *tile_w = tile.w;
+}
+
 static bool prepare_sampled_linear(DcnProblem *pr, int dtype, const SampledLinear &p) {
   if (dcn_prepare(pr, false, dtype, p.batch, p.height, p.width, p.group, p.group_channels, p.kernel, p.kernel, 1, 1, p.pad, p.pad, p.dilation,
                   p.dilation, p.offset_scale, 256, p.remove_center, p.row, 0, 0, 0) != DCNV4_OK)
@@ -1154,7 +1159,7 @@ FdaScratch fda_scratch(int s, int batch, int N, int G, int D, int L, int Q, int 
   sc.per = (int)std::min<uint64_t>(per, (uint64_t)batch);
   const size_t points = (size_t)G * L * fda_key_stride(Q, K);          // per image
   sc.n_chunks = (int)(((size_t)Q * K + kFdaChunkPoints - 1) / kFdaChunkPoints);
-  // a level of H x W cells is cut into tiles of min(8, ceil(dim / 4)) cells per side: at most N/8 + 64 tiles
+  // what a level is cut into at most (fda_tile)
   sc.tile_stride = (int)std::min<size_t>(kFdaMaxTilesPerLevel, (size_t)N / 8 + 64);
   const size_t segs = (size_t)sc.per * G * L * sc.n_chunks;
   sc.keys = kStateBytes;
@@ -1227,9 +1232,8 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
     base.tile_stride = sc.tile_stride;
     // The state block (the binning kernel's flag) is cleared by the first kernel itself, which runs to its end
     // before the binning kernel starts.  The fallback - three launches that return at once without the flag - can
-    // only be needed when a level has more tiles than the binning kernel counts (kFdaMaxTilesPerLevel); tiles have
-    // at least 8 cells (a level of up to four rows is cut into 1 x 8 pieces), so a tensor of fewer cells than that
-    // many tiles' worth cannot raise the flag and the launches are left out.
+    // only be needed when a level has more tiles than the binning kernel counts (kFdaMaxTilesPerLevel); a tensor
+    // that cannot have a level of so many (fda_tile) cannot raise the flag and the launches are left out.
     const bool fallback_possible = (size_t)spatial_size / 8 + 64 > (size_t)kFdaMaxTilesPerLevel;
     for (int pass = 0; pass < (fallback_possible ? 3 : 2); ++pass) {
       for (int b0 = 0; b0 < batch; b0 += per) {
@@ -1248,11 +1252,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
         F.n_row = nb * F.Q;
         F.n_img = nb;
         F.zero_rows = rows.zero_rows && !fallback_possible ? rows.zero_rows + (size_t)b0 * spatial_size : nullptr;
-        // A tile is worked on by one workgroup: no more points than about a share of them all, or it is what the launch waits for; smaller
-        // tiles than that list more points twice.  us of a backward, shares of 350 / 800 / 2000: 1 image of a pyramid from 100 x 152, every
-        // pixel a query, fp32 214 / 199 / 199, fp16 185 / 147 / 147; 1 of 160 x 160 352 / 317 / 317; 4 of 128 x 128 727 / 728 / 763, fp16 506 /
-        // 505 / 550; 8 of 60 x 60 319 / 319 / 348; 2 of 100 x 152 340 / 346 / 353; 2 of 43 x 89 110 / 118 / 119.
-        F.tile_points = (int)std::clamp<long long>((long long)num_query * num_points * num_levels * nb * num_heads / 800, 1024, 0x7fffffff);
+        F.tile_points = fda_tile_points((long long)num_query * num_points * num_levels * nb * num_heads);
         hipError_t e = hipSuccess;
         if (pass == 0) fda_choose_order(&F, pr, spatial_size, num_heads, head_channels, num_levels, num_points, true);
         F.clear_state = (pass == 0 && b0 == 0) ? 1 : 0;

@@ -30,8 +30,7 @@
 //   us, before -> now, 8 heads of 32 channels, levels from 100 x 152, four points: 2 images, every pixel a query, fp32 285 -> 171;
 // 300 queries, fp16 72 -> 26.  The whole backward: fp16, 1 image 244 -> 147, 2 images of 100 x 100 253 -> 179 (calls).
 //
-// Tiles are at most 8x8 cells and every level is cut into 16 of them or more, into 64 where a tile would hold more than its share of
-// the points (FdaLaunch::tile_points), so items stay small (several workgroups share a CU and hide each other's latencies).
+// Tiles are small (fda_tile): several workgroups share a CU and hide each other's latencies.
 // Levels and tile shapes are derived on the device from the spatial_shapes tensor; the host never
 // reads it.  A level with more tiles than the binning kernel's LDS histogram holds raises a flag in
 // GradState: this kernel then writes zeros and the atomic fallback kernel adds everything (in fp32).
@@ -62,23 +61,11 @@ struct LevelPlan {
 __device__ __forceinline__ LevelPlan level_plan(const FdaLaunch &p, int l) {
   LevelPlan lp;
   lp.H = (int)p.shapes[2 * l]; lp.W = (int)p.shapes[2 * l + 1]; lp.start = (int)p.level_start[l];
-  lp.th = max(1, min(8, (lp.H + 3) / 4));
-  lp.tw = max(1, min(8, (lp.W + 3) / 4));
-  if ((long long)p.Q * p.K * ((lp.th + 1) * (lp.tw + 1)) > (long long)p.tile_points * lp.H * lp.W) {
-    lp.th = max(1, min(lp.th, (lp.H + 7) / 8));
-    lp.tw = max(1, min(lp.tw, (lp.W + 7) / 8));
-  }
+  const FdaTile tile = fda_tile(lp.H, lp.W, (long long)p.Q * p.K, p.tile_points);
+  lp.th = tile.h; lp.tw = tile.w;
   lp.nty = lp.H > 0 ? (lp.H + lp.th - 1) / lp.th : 0;
   lp.ntx = lp.W > 0 ? (lp.W + lp.tw - 1) / lp.tw : 0;
   return lp;
-}
-
-template <typename Tag>
-__device__ __forceinline__ float elem_at(const void *base, size_t i) {
-  typedef typename RawWord<Tag::kBytes>::type elem_t;
-  float f[1];
-  Pack<Tag, 1>::decode(reinterpret_cast<const elem_t *>(base)[i], f);
-  return f[0];
 }
 
 // n / d for small non-negative n and 1 <= d <= 8

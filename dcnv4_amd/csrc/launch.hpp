@@ -268,6 +268,24 @@ constexpr int kFdaChunkPoints = 4096;          // points one binning workgroup s
 constexpr int kFdaTakenStride = 64;            // words: dies that count in one cache line wait for each other
 constexpr int kFdaWindowChannels = 32;         // of a head, that the grad_value kernel adds up at a time
 constexpr int kFdaMaxTilesPerLevel = 8192;     // LDS histogram of the binning kernel
+// The attention backward's tiles of a level of h x w cells with `points` sampling points: at most 8 x 8 cells, 16 tiles or more where there
+// are as many cells, 64 where a tile would hold more than tile_points.  No side is cut into more pieces than max(8, dim / 8 + 1), nor than
+// it has cells, so tiles are at most h * w / 8 + 64.
+struct FdaTile { int h, w; };
+__host__ __device__ inline FdaTile fda_tile(int h, int w, long long points, int tile_points) {
+  auto side = [](int dim, int pieces) { const int n = (dim + pieces - 1) / pieces; return n < 1 ? 1 : n > 8 ? 8 : n; };
+  const FdaTile coarse = {side(h, 4), side(w, 4)};
+  if (points * ((coarse.h + 1) * (coarse.w + 1)) <= (long long)tile_points * h * w) return coarse;
+  return {side(h, 8), side(w, 8)};
+}
+// A tile is worked on by one workgroup: no more points than about a share of them all, or it is what the launch waits for; smaller
+// tiles than that list more points twice.  us of a backward, shares of 350 / 800 / 2000: 1 image of a pyramid from 100 x 152, every
+// pixel a query, fp32 214 / 199 / 199, fp16 185 / 147 / 147; 1 of 160 x 160 352 / 317 / 317; 4 of 128 x 128 727 / 728 / 763, fp16 506 /
+// 505 / 550; 8 of 60 x 60 319 / 319 / 348; 2 of 100 x 152 340 / 346 / 353; 2 of 43 x 89 110 / 118 / 119.
+inline int fda_tile_points(long long all_points) {
+  const long long share = all_points / 800;
+  return (int)(share < 1024 ? 1024 : share > 0x7fffffff ? 0x7fffffff : share);
+}
 __host__ __device__ inline size_t fda_key_stride(int Q, int K) { return ((size_t)Q * K + 1) & ~size_t(1); }
 
 enum FdaBackwardMode {

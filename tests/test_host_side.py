@@ -370,3 +370,18 @@ def test_the_convolutions_around_the_layers_can_be_scripted_traced_and_compiled(
         for program in (torch.jit.script(stem), torch.fx.symbolic_trace(stem), torch.compile(stem, backend="eager", fullgraph=True)):
             torch.testing.assert_close(program(x), want)
         torch.testing.assert_close(torch.fx.symbolic_trace(down)(y, (4, 4))[0], want_down)
+
+
+def test_tiles_of_a_level_are_no_more_than_their_table_holds():
+    """The attention backward's table has room for N / 8 + 64 tiles of a level of N cells, whichever way the level is cut."""
+    from dcnv4_amd import ext
+    sides = list(range(1, 70)) + [127, 128, 129, 255, 1000, 20197]
+    finer = 0
+    for h in sides:
+        for w in sides:
+            cuts = {ext._native.attention_tile(h, w, points, pairs) for points, pairs in ((1, 1), (1 << 20, 1))}
+            finer += len(cuts) > 1
+            for tile_h, tile_w in cuts:
+                assert 1 <= tile_h <= 8 and 1 <= tile_w <= 8
+                assert -(-h // tile_h) * -(-w // tile_w) <= h * w // 8 + 64, (h, w, tile_h, tile_w)
+    assert finer > 1000
