@@ -44,6 +44,50 @@ def test_grad_value_by_tiles(oracle, name, dtype):
         assert (np.abs(cabi.f64(g) - want) <= bound).all(), float((np.abs(cabi.f64(g) - want) / bound).max())
 
 
+# The same turns with sides that are powers of two, for data whose sums are exact: one lost or doubled point of one cell shows.
+# B, levels, G, D, K, Q, then which levels are cut finer and whether tiles are handed out (fda_grad_value_kernel's `shared`)
+EXACT = {
+    "groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000, [True], True),
+    "handed_out": (2, [(64, 128), (8, 8), (1, 1), (16, 16)], 8, 32, 4, 12000, [False, True, False, True], True),
+    "windows_take_turns": (1, [(32, 64), (16, 16)], 8, 72, 4, 4000, [False, True], True),
+    "odd_pairs": (1, [(32, 16), (4, 2)], 3, 16, 6, 1111, [False, False], True),
+    "empty_tiles": (1, [(128, 128), (64, 64)], 8, 32, 4, 9, [False, False], False),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["fp32", "fp16"])
+@pytest.mark.parametrize("name", list(EXACT))
+def test_grad_value_by_tiles_has_every_point_once(oracle, name, dtype):
+    """Positions in quarters of a pixel, eight or sixteen equal probabilities a query, gradients of 1 and -1: every term is a multiple of
+    2^-8 and every sum exact in fp32, so that the result is the oracle's, rounded once."""
+    B, levels, G, D, K, Q, finer, handed_out = EXACT[name]
+    print(f"case {name} dtype {dtype}", flush=True)
+    tiles = [ext._native.attention_tile(h, w, Q * K, len(levels) * B * G) for h, w in levels]
+    assert [t != ext._native.attention_tile(h, w, 1, 1) for t, (h, w) in zip(tiles, levels)] == finer
+    assert (Q * K * len(levels) >= 256 * sum(-(-h // th) * -(-w // tw) for (h, w), (th, tw) in zip(levels, tiles))) == handed_out
+    g = torch.Generator().manual_seed(len(name))
+    v, shp, st, sla, go = make_fda_inputs(B, levels, G, D, K, Q, seed=1, dtype=torch.float32)
+    rows = sla[..., :len(levels) * K * 2].view(B, Q, G, len(levels), K, 2)
+    for level, (h, w) in enumerate(levels):
+        for axis, side in ((0, w), (1, h)):      # from a pixel outside to the last one
+            quarters = torch.randint(-3, 4 * side, (B, Q, G, K), generator=g)
+            rows[..., level, :, axis] = (quarters / 4 + 0.5) / side
+    logits = sla[..., len(levels) * K * 2:]
+    logits.zero_()
+    points = len(levels) * K
+    equal = 1 << (points.bit_length() - 1)
+    logits.scatter_(-1, torch.rand(logits.shape, generator=g).argsort(-1)[..., equal:], -1000.0)      # the others have none
+    go.copy_(torch.randint(0, 2, go.shape, generator=g) * 2 - 1)
+    v, sla, go = v.to(dtype), sla.to(dtype), go.to(dtype)
+    want, _ = oracle.flash_deform_attn_backward(cabi.f64(v), shp.numpy(), st.numpy(), cabi.f64(sla), cabi.f64(go), K, coord_f32=True)
+    assert (want * 256 == np.rint(want * 256)).all() and np.abs(want).max() * 256 < 2 ** 24 and want.any()
+    want = torch.from_numpy(want).to(dtype)
+    with ext.launch_options(scatter="tiled"):
+        for _ in range(2):
+            got = cabi.fda_backward(v.cuda(), shp.cuda(), st.cuda(), sla.cuda(), go.cuda(), K)[0].cpu()
+            assert torch.equal(got, want), (int((got != want).sum()), float((got - want).abs().max()))
+
+
 # fp32 tensors with fewer points than a third of the pixels take the atomic scatter by themselves: on either side of where, both ways
 # against each other
 @pytest.mark.parametrize("batch,queries", [(2, 28), (2, 29), (2, 280), (2, 320), (6, 100), (6, 120)])
