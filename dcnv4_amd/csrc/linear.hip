@@ -595,17 +595,14 @@ hipError_t launch_few_waves(const LinearLaunch &p, hipStream_t stream) {
 // reads bounds these products.  32 x 32 | 16 x 16, us a launch behind another, with bias, layer scale and residual, fp16: 49 x 512 x 2048
 // (128 tiles of 16 x 16) 9.3 | 5.9, 196 x 256 x 1024 (208) 5.9 | 4.3, 196 x 256 x 256 3.5 | 3.1, 196 x 320 x 1280 (260) 6.8 | 6.3, 196 x 448 x 1792 (364)
 // 8.6 | 8.5, 392 x 256 x 1024 (400) 5.9 | 6.0, 600 x 256 x 256 (608) 3.6 | 4.5; fp32: 49 x 512 x 2048 16.8 | 10.0, 196 x 320 x 1280 11.6 | 10.2.
-// Of 32 x 32, eight waves where four would take more than four turns each (196 x 256 x 1024 8.4 -> 7.0 us; sixteen gain nothing further).
 constexpr int kFewSmallTiles = kCus * 5 / 4;
+// Of 32 x 32, eight waves where four would take more than four turns each (196 x 256 x 1024 8.4 -> 7.0 us; sixteen gain nothing further).
 template <typename Tag, bool EXTRA>
 hipError_t launch_few(const LinearLaunch &p, hipStream_t stream) {
   if constexpr (!EXTRA && Tag::kBytes == 2) {
     if (p.norm.weight != nullptr) return p.k <= 256 ? launch_few_waves<Tag, false, kNormWaves, 2, 2>(p, stream) : launch_few_waves<Tag, false, kNormWaves, 2, 4>(p, stream);
   }
   const long long steps = (long long)p.k * Tag::kBytes / 64;
-  long long tiles = 0;
-  for (int i = 0; i < p.count; ++i) tiles += (p.p[i].n + 15) / 16;
-  if (tiles * ((p.rows + 15) / 16) <= kFewSmallTiles) return launch_few_waves<Tag, EXTRA, 8, 1, 0>(p, stream);
   return steps <= 16 ? launch_few_waves<Tag, EXTRA, 4, 2, 0>(p, stream) : launch_few_waves<Tag, EXTRA, 8, 2, 0>(p, stream);
 }
 
@@ -629,7 +626,8 @@ LinearTile plan_linear(int dtype, const LinearLaunch &p) {
     for (int i = 0; i < p.count; ++i) n += (p.p[i].n + bn - 1) / bn;
     return n * ((p.rows + bm - 1) / bm);
   };
-  if (tiles(64, 64) < 64 || p.norm.weight != nullptr) return {kFewTile, kFewTile};
+  if (p.norm.weight != nullptr) return {kFewTile, kFewTile};
+  if (tiles(64, 64) < 64) return tiles(16, 16) <= kFewSmallTiles ? LinearTile{16, 16} : LinearTile{kFewTile, kFewTile};
   // fp32 is bound by the matrix cores (157 TFLOP/s): the tile that spreads most evenly
   if (dtype == F32::kCode || tiles(128, 64) < kCus) return {64, 64};
   int features = 0;
@@ -645,6 +643,7 @@ LinearTile plan_linear(int dtype, const LinearLaunch &p) {
 template <typename Tag, bool EXTRA>
 hipError_t launch_t(const LinearLaunch &p, hipStream_t stream) {
   const LinearTile tile = plan_linear(Tag::kCode, p);
+  if (tile.rows == 16) return launch_few_waves<Tag, EXTRA, 8, 1, 0>(p, stream);
   if (tile.rows == kFewTile) return launch_few<Tag, EXTRA>(p, stream);
   if (tile.rows == 64) return launch_tiled<Tag, EXTRA, 64, 64, 2, 2>(p, stream);
   if constexpr (Tag::kBytes == 4) {

@@ -56,7 +56,7 @@ bool linear_fits(int dtype, long long rows, int n, int k);
 // Whether the rows may come normalised: few enough that a workgroup normalising its own costs less than a launch.
 bool linear_takes_norm(const LinearLaunch &p);
 hipError_t launch_linear(int dtype, const LinearLaunch &p, hipStream_t stream);
-// The tile of launch_linear's kernel: 32 x 32 few rows, 256 x 128 the wide one.
+// The tile of launch_linear's kernel: 16 x 16 or 32 x 32 of few rows, 256 x 128 the wide one.
 struct LinearTile { int rows, features; };
 LinearTile linear_tile(int dtype, const LinearLaunch &p);
 
