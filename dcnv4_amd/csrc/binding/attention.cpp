@@ -240,7 +240,10 @@ variable_list Attention::backward(const Tensor &query, const Tensor &reference, 
       result(more, g[kQuery], query32);
     }
   }
-  const void *q_in = half && query32 ? a.at(s.query) : ptr(query), *f_in = half && features32 ? a.at(s.features) : ptr(features);
+  // An input is not kept for frozen weights.  Their gradients, which nobody asked for, go with their biases' all the same, and are formed of
+  // rows of that many elements that are at hand.
+  const void *q_in = half && query32 ? a.at(s.query) : query.defined() ? ptr(query) : a.at(s.sampled);
+  const void *f_in = half && features32 ? a.at(s.features) : features.defined() ? ptr(features) : a.at(s.value);
   const auto fp32 = params[kValueW].options();
   auto gradient = [&](Input weight, const void *grad_out, const void *in, int64_t n, int64_t pitch) -> WeightGradient {
     return {grad_out, in, n, width, &params[weight], &params[weight + 1], &g[weight], &g[weight + 1], want[weight], want[weight + 1], pitch};

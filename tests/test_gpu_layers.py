@@ -202,6 +202,35 @@ def test_query_gradient_in_fp32_is_two_products_added(h, w, amp):
     assert offsets.any() and logits.any() and torch.equal(both, logits + offsets)
 
 
+# 16 queries of 54 pixels, and every pixel a query
+@pytest.mark.parametrize("queries", [16, 54])
+@pytest.mark.parametrize("amp", [None, torch.float16], ids=["fp32", "fp16"])
+def test_attention_layer_trains_biases_of_frozen_weights(queries, amp):
+    """The inputs, fp32 or the products' type, are kept for the weights' gradients only: biases do without."""
+    import dcnv4_amd
+    torch.manual_seed(0)
+    m = dcnv4_amd.FlashDeformAttn(64, 1, 4, 4).cuda()
+    shapes, starts = torch.tensor([[6, 9]], device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    query, features = (torch.randn(2, n, 64, device="cuda", dtype=amp or torch.float32) for n in (queries, 54))
+    reference, grad = torch.rand(2, queries, 1, 2, device="cuda"), torch.randn(2, queries, 64, device="cuda")
+
+    def gradients(wanted):
+        for p in m.parameters():
+            p.requires_grad_(False)
+        for p in wanted:
+            p.requires_grad_(True)
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            out = m(query, reference, features, shapes, starts)
+        assert out.grad_fn.name() == "FlashDeformAttnBackward"
+        return torch.autograd.grad(out, wanted, grad.to(out.dtype))
+    parameters = dict(m.named_parameters())
+    every = dict(zip(parameters, gradients(list(parameters.values()))))
+    biases = [name for name in parameters if name.endswith("bias")]
+    for names in (biases, *([name] for name in biases)):
+        for name, got in zip(names, gradients([parameters[name] for name in names])):
+            assert _rel(got, every[name]) < (1e-5 if amp is None else 1e-3), name      # grad_value's terms come in an order that varies
+
+
 def test_attention_layer_reads_changed_level_shapes_again():
     import dcnv4_amd
     m = dcnv4_amd.FlashDeformAttn(64, 1, 4, 4).cuda()
