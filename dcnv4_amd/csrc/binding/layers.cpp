@@ -112,7 +112,7 @@ void hip_check(hipError_t e, const char *what) {
 
 void weight_gradients(int code, const at::TensorOptions &fp32, const std::vector<WeightGradients> &groups, void *stream) {
   WeightGradReduce reduce = {};
-  std::vector<Tensor> partials;      // given back behind the last launch
+  std::vector<Tensor> held;      // until the last launch, which writes all gradients: partial sums, and gradients that nobody asked for
   for (const WeightGradients &group : groups) {
     WeightGradLaunch launch = {};
     launch.rows = group.rows;
@@ -122,6 +122,7 @@ void weight_gradients(int code, const at::TensorOptions &fp32, const std::vector
       auto &g = grads[launch.count];
       g.weight = at::empty(l.weight->sizes(), fp32);
       if (l.want_w) *l.grad_w = g.weight;
+      else held.push_back(g.weight);
       if (l.want_b) *l.grad_b = g.bias = at::empty(l.bias->sizes(), fp32);
       WeightGradProblem &q = launch.p[launch.count++];
       q.grad_out = l.grad_out; q.in = l.in; q.n = (int)l.n; q.k = (int)l.k;
@@ -143,8 +144,8 @@ void weight_gradients(int code, const at::TensorOptions &fp32, const std::vector
     }
     float *base = nullptr;
     if (plan.splits > 1) {
-      partials.push_back(at::empty({(int64_t)(floats * plan.splits)}, fp32));
-      base = static_cast<float *>(partials.back().data_ptr());
+      held.push_back(at::empty({(int64_t)(floats * plan.splits)}, fp32));
+      base = static_cast<float *>(held.back().data_ptr());
     }
     launch.split_stride = floats;
     segments = 0;

@@ -231,6 +231,38 @@ def test_attention_layer_trains_biases_of_frozen_weights(queries, amp):
             assert _rel(got, every[name]) < (1e-5 if amp is None else 1e-3), name      # grad_value's terms come in an order that varies
 
 
+@pytest.mark.parametrize("amp", [None, torch.float16], ids=["fp32", "fp16"])
+def test_gradients_that_nobody_asked_for_have_memory_of_their_own(amp):
+    """A frozen weight's gradient, formed with its bias's, is written by the last launch, which adds up the partial sums of all products:
+    the gradients of feature rows, allocated behind those of query rows, may not lie in its memory."""
+    import dcnv4_amd
+    from dcnv4_amd import ext
+    torch.manual_seed(0)
+    m = dcnv4_amd.FlashDeformAttn(256, 1, 8, 4).cuda()
+    with torch.no_grad():
+        m.sampling_offsets.weight.normal_(0, 0.05)
+        m.attention_weights.weight.normal_(0, 0.05)
+    h, w, q = 32, 48, 1600
+    shapes, starts = torch.tensor([[h, w]], device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    query, features = torch.randn(1, q, 256, device="cuda"), torch.randn(1, h * w, 256, device="cuda")
+    reference, grad = torch.rand(1, q, 1, 2, device="cuda"), torch.randn(1, q, 256, device="cuda")
+    splits = ext._native.weight_grad_plan(torch.empty(q, 256, dtype=amp or torch.float32, device="meta"), torch.tensor([256, 64, 32]))[1]
+    assert splits > 1      # so that there are partial sums of query rows
+
+    def gradients(names):
+        for name, p in m.named_parameters():
+            p.requires_grad_(name in names)
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            out = m(query, reference, features, shapes, starts)
+        assert out.grad_fn.name() == "FlashDeformAttnBackward"
+        return dict(zip(names, torch.autograd.grad(out, [dict(m.named_parameters())[n] for n in names], grad.to(out.dtype))))
+    every = [name for name, _ in m.named_parameters()]
+    want = gradients(every)
+    got = gradients([name for name in every if name.endswith("bias") or name.startswith("value_proj")])
+    for name, g in got.items():
+        assert _rel(g, want[name]) < (1e-5 if amp is None else 1e-3), name      # sums in fp32, grad_value's terms in an order that varies
+
+
 def test_attention_layer_reads_changed_level_shapes_again():
     import dcnv4_amd
     m = dcnv4_amd.FlashDeformAttn(64, 1, 4, 4).cuda()
