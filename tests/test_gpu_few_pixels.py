@@ -29,6 +29,22 @@ def test_forward_of_few_pixels_matches_the_direct_kernel(B, H, W, G, D, dilation
     assert _rel(got[keep], want[keep]) < bound
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("groups,shared", [(32, True), (33, False)])
+def test_a_quad_shares_the_taps_of_up_to_16384_vectors(groups, shared, dtype):
+    """Points on their pixels, values of 2^12: taps 0, 1 and 4 are 2^25, 1 and -2^25.  A lane of all nine loses the 1 next to 2^25; in a quad
+    taps 0 and 4 are one lane's and cancel before another's 1 is added."""
+    from dcnv4_amd import ext
+    h, w = (16, 16) if dtype != torch.float32 else (8, 16)
+    assert (h * w * groups * 16 * dtype.itemsize // 16 <= 16384) == shared
+    value = torch.full((1, h, w, groups * 16), 2.0 ** 12, dtype=dtype, device="cuda")
+    rows = torch.zeros(1, h, w, (groups * 27 + 7) // 8 * 8, dtype=dtype, device="cuda")
+    taps = rows[..., :groups * 27].view(1, h, w, groups, 27)[..., 18:]
+    taps[..., 0], taps[..., 1], taps[..., 4] = 2.0 ** 13, 2.0 ** -12, -2.0 ** 13
+    out = ext.dcnv4_forward(value, rows, 3, 3, 1, 1, 1, 1, 1, 1, groups, 16, 1.0, 256, 0, 0, 0, False)
+    assert (out[:, 1:-1, 1:-1] == (1 if shared else 0)).all()
+
+
 # one round of workgroups and a round and a quarter of a workgroup's lanes at most: pixels in whole and ragged tiles, widths that are no
 # multiple of 64, one vector a group and several, one pixel
 LAYERS = [(16, 1, False, None, (1, 1, 1)), (64, 4, False, None, (1, 56, 56)), (64, 2, True, 0.3, (1, 33, 29)), (80, 5, True, 0.3, (1, 31, 33)),
@@ -116,7 +132,8 @@ def test_products_of_few_rows_add_their_parts_in_pairs():
         assert (ext.linear_forward(torch.ones(rows, 128, device="cuda"), w) == 2.0 ** 25 + 8).all()
 
 
-# pixels x features in tiles of 16 x 16 (252 of them, the depth in one request and in two) and of 32 x 32
+# pixels x features in tiles of 16 x 16 (252 and 57 of them, the depth in one request and in two) and of 32 x 32 (1372 of 16 x 16): the
+# depth is cut alike, so that results do not tell
 @pytest.mark.parametrize("channels,size", [(112, (5, 15, 14)), (456, (1, 3, 5)), (112, (8, 28, 28))])
 def test_downsampling_of_few_pixels(channels, size):
     from dcnv4_amd.models.flash_intern_image import DownsampleLayer

@@ -176,6 +176,45 @@ def test_attention_layer_in_one_call_matches_the_composition(levels, queries, ki
         assert not results[0][2][mask].any()
 
 
+# either way of the gradient of value, whichever the sizes would take: by tiles the kernel that adds it up clears the padded rows
+@pytest.mark.parametrize("scatter", ["tiled", "atomic"])
+@pytest.mark.parametrize("amp", [None, torch.float16], ids=["fp32", "fp16"])
+@pytest.mark.parametrize("queries,kind", [(0, 2), (0, 4), (50, 4)], ids=["pixels-ref2", "pixels-ref4", "few-ref4"])
+def test_padded_rows_of_an_attention_layer_have_no_gradient(queries, kind, amp, scatter):
+    import dcnv4_amd
+    from dcnv4_amd import ext
+    torch.manual_seed(kind)
+    levels, batch, width = [(40, 52), (20, 26), (10, 13), (5, 7)], 2, 64
+    m = dcnv4_amd.FlashDeformAttn(width, 4, 4, 4).cuda()
+    with torch.no_grad():
+        m.sampling_offsets.weight.normal_(0, 0.05)
+        m.attention_weights.weight.normal_(0, 0.05)
+    pixels = sum(h * w for h, w in levels)
+    shapes = torch.tensor(levels, device="cuda")
+    starts = torch.tensor([sum(h * w for h, w in levels[:i]) for i in range(4)], device="cuda")
+    # a picture's right and lower edge in every level, and pixels here and there
+    mask = torch.cat([((torch.arange(h)[:, None] >= 0.8 * h) | (torch.arange(w) >= 0.7 * w)).flatten() for h, w in levels]).expand(batch, -1).clone()
+    mask = (mask & torch.tensor([[True], [False]])).cuda() | (torch.rand(batch, pixels, device="cuda") < 0.1)
+    query, features = torch.randn(batch, queries or pixels, width, device="cuda"), torch.randn(batch, pixels, width, device="cuda")
+    reference, grad = torch.rand(batch, queries or pixels, 4, kind, device="cuda"), torch.randn(batch, queries or pixels, width, device="cuda")
+    results = []
+    with ext.launch_options(scatter=scatter):
+        value = torch.empty(batch, pixels, 4, width // 4, dtype=amp or torch.float32, device="meta")
+        assert ext._native.attention_backward_tiled(value, 4, queries or pixels, 4) == (scatter == "tiled")
+        for composed in (False, True):
+            handle = m.output_proj.register_forward_hook(lambda *a: None) if composed else None
+            qi, fi = query.clone().requires_grad_(), features.clone().requires_grad_()
+            with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+                out = m(qi, reference, fi, shapes, starts, mask)
+            assert (out.grad_fn.name() == "FlashDeformAttnBackward") != composed
+            results.append(torch.autograd.grad(out, [fi, m.value_proj.weight, m.value_proj.bias], grad.to(out.dtype)))
+            if composed:
+                handle.remove()
+    for got, want in zip(*results):
+        assert _rel(got, want) < (2e-3 if amp is None else 4e-3)      # as in the comparison with the composition above
+    assert not results[0][0][mask].any() and results[0][0][~mask].any()
+
+
 # products of few rows and of many
 @pytest.mark.parametrize("amp", [None, torch.float16, torch.bfloat16], ids=["fp32", "fp16", "bf16"])
 @pytest.mark.parametrize("h,w", [(6, 9), (64, 100)], ids=["few", "many"])

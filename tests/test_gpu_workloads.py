@@ -273,6 +273,17 @@ def test_flash_deform_attn_grad_value_keeps_fp32_accuracy_on_heavy_tailed_gradie
     _assert_accumulated_like_fp32(gv, wgv, mag, dtype, "grad_value")
 
 
+# the same either way, whichever the sizes would take
+@pytest.mark.parametrize("scatter", ["tiled", "atomic"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["fp16", "bf16", "fp32"])
+def test_flash_deform_attn_grad_value_keeps_fp32_accuracy_by_tiles_and_atomics(oracle, dtype, scatter):
+    from dcnv4_amd import ext
+    with ext.launch_options(scatter=scatter):
+        value = torch.empty(2, 24 * 24 + 12 * 12, 4, 32, dtype=dtype, device="meta")
+        assert ext._native.attention_backward_tiled(value, 2, 700, 4) == (scatter == "tiled")
+        test_flash_deform_attn_grad_value_keeps_fp32_accuracy_on_heavy_tailed_gradients(oracle, dtype)
+
+
 def test_flash_deform_attn_value_rows_no_level_covers_get_zero_gradient(oracle):
     """spatial_size larger than the levels cover, and a gap between two levels: the reference returns
     zeros_like(value) there (DCNv4_op/src/cuda/flash_deform_attn_cuda.cu:118)."""
