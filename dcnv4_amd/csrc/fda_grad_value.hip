@@ -22,13 +22,14 @@
 //   * the finished tile is written to grad_value with plain stores in the tensor dtype.
 //
 // A step's operands are four loads behind each other: where the tile's points lie in the chunks' lists, their numbers, their records
-// and the rows of grad_out.  An item at a time these were waited for one by one, which was most of the time of a decoder's sparse
-// tiles and a third of an encoder's.  So the steps of all items are one stream: each step adds up its own points while the records and
+// and the rows of grad_out.  An item at a time these were waited for one by one, a third of an encoder's time.  So the steps of all items are one stream: each step adds up its own points while the records and
 // rows of the next, the numbers of the one behind it and the place of the next item's lists are on their way.  The points of a tile
 // come in the order of the queries, neighbours hit the same cells, and a step waits for its longest cell: a step takes every n-th block
 // of 32 (a line of numbers) of the list instead of 256 in a row.  What bounds it now are the VALU (two thirds busy) and LDS (half).
-//   us, before -> now, 8 heads of 32 channels, levels from 100 x 152, four points: 2 images, every pixel a query, fp32 285 -> 171;
-// 300 queries, fp16 72 -> 26.  The whole backward: fp16, 1 image 244 -> 147, 2 images of 100 x 100 253 -> 179 (calls).
+//   us under a tracer, before -> now, 8 heads of 32 channels, levels from 100 x 152, four points: 2 images, every pixel a query, fp32
+// 291 -> 182; 300 queries, fp16, 29.3 -> 28.0 (5648 tiles of which most hold a point or none: there it gains nothing).  The whole
+// backward, every pixel a query: fp16, 1 image 246 -> 136, 2 images of 100 x 100 284 -> 170, 4 of 128 x 128 589 -> 467; fp32, 1 image 265
+// -> 190, 4 of 128 x 128 805 -> 704, 8 of 60 x 60 358 -> 300.
 //
 // Tiles are small (fda_tile): several workgroups share a CU and hide each other's latencies.
 // Levels and tile shapes are derived on the device from the spatial_shapes tensor; the host never
