@@ -310,7 +310,7 @@ hipError_t launch_dcnv4_forward(int dtype, const DcnLaunch &p, hipStream_t strea
   return launch_by_dtype<false>(dtype, p, stream);
 }
 // Where the chip stays empty enough a quad shares a lane's nine taps.  Behind each other in a graph, us, a lane | a quad: 3136 16-byte
-// vectors (1x7x7, 32 groups of 16, fp16) 4.04 | 3.33, 6272 4.10 | 3.45, 12544 4.14 | 3.50, 25088 4.17 | 4.18 (fp32 3.70 | 4.25), 50176 4.23 | 5.99.
+// vectors (1x7x7, 32 groups of 16, fp16) 3.75 | 2.88, 6272 3.81 | 3.05, 12544 3.84 | 3.11, 25088 3.89 | 3.99 (fp32 3.52 | 3.95), 50176 3.94 | 5.95.
 constexpr int64_t kSharedItems = 16384;
 hipError_t launch_dcnv4_forward_small(int dtype, const DcnLaunch &p, hipStream_t stream) {
   const int64_t items = (int64_t)p.n_pix * p.G * p.lanes.tpg;
