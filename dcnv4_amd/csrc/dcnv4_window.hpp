@@ -79,30 +79,51 @@ __device__ __forceinline__ void stage_window(const DcnLaunch &p, const WindowTil
   const int piece = threadIdx.x & (kPieces - 1);
   const bool piece_in = first + piece * 16 < pix_bytes;
   const int cells = t.wh * t.ww + t.ww + 2;
-  // A lane's cells are kStep apart: place and address advance by what kStep is in rows and columns.  Rows and columns count from the first
-  // that lies in the image; every lane has one division, in place of one a cell (28 -> 13 vector instructions each).  Two cells a turn, so
-  // that the next place is at hand when a load has been given: forward and backward, 64x56x56 with 4 groups in fp32 245.4 -> 244.5 us,
-  // 64x28x28 with 8 118.2 -> 117.6, 2x200x334 with 10 in bf16 354 -> 352.5; four a turn gain half of that.
+  // A lane's cells are kStep apart.  Behind the first two, whose place is found by a division, place and address advance by what kStep is
+  // in rows and columns, counted from the first that lies in the image (28 -> 13 vector instructions a cell; two cells a turn, so that the
+  // next place is at hand when a load has been given).  What that takes is formed while the first loads are under way: small images have two
+  // to five cells a lane, and their forward waited for it.  us, fp16, every cell by division | steps from the first on | so: 128x7x7 with 56
+  // groups 20.15 | 20.41 | 20.19, 64x14x14 with 16 11.77 | 11.91 | 11.77, 40x19x23 with 11 11.60 | 11.73 | 11.63; forward and backward of
+  // 64x56x56 with 4 169.1 | 166.2 | 166.2, 2x200x334 with 10 283.1 | 273.8 | 275.2 (with what the other kernels gained beside it).
   constexpr int kStep = kWindowThreads / kPieces;
   const float inv = __builtin_amdgcn_rcpf((float)t.ww);
   const int first_row = max(-t.wy0, 0), first_col = max(-t.wx0, 0);
   const int rows_in = max(min(t.wy0 + t.wh, p.H) - (t.wy0 + first_row), 0), cols_in = piece_in ? max(min(t.wx0 + t.ww, p.W) - (t.wx0 + first_col), 0) : 0;
-  const int step_rows = __builtin_amdgcn_readfirstlane(exact_div(kStep, inv)), step_cols = kStep - step_rows * t.ww;
-  const int row_pitch = p.W * pix_bytes, step = step_rows * row_pitch + step_cols * pix_bytes, wrap = row_pitch - t.ww * pix_bytes;
-  const int cell = (wave * 64 + lane) / kPieces, cell_row = exact_div(cell, inv);
-  int row = cell_row - first_row, col = cell - cell_row * t.ww - first_col;
-  const int last_col = t.ww - first_col;
-  uint32_t off = img + (uint32_t)(((t.wy0 + cell_row) * p.W + t.wx0 + cell - cell_row * t.ww) * pix_bytes + piece * 16);
-#pragma unroll 2
-  for (int base = wave * 64; base < cells * kPieces; base += kWindowThreads) {
+  int row, col;
+  uint32_t off;
+  auto place = [&](int cell) {
+    const int cell_row = exact_div(cell, inv), cell_col = cell - cell_row * t.ww;
+    row = cell_row - first_row;
+    col = cell_col - first_col;
+    off = img + (uint32_t)(((t.wy0 + cell_row) * p.W + t.wx0 + cell_col) * pix_bytes + piece * 16);
+  };
+  auto load = [&](int base) {
     const bool in = (unsigned)row < (unsigned)rows_in && (unsigned)col < (unsigned)cols_in;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(value, (__attribute__((address_space(3))) void *)(lds + base * 16), 16,
                                              (int)(in ? off : kDropOffset), 0, 0, 0);
+  };
+  const int end = cells * kPieces;
+  int base = wave * 64;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    if (base >= end) return;
+    place((wave * 64 + lane) / kPieces + u * kStep);
+    load(base);
+    base += kWindowThreads;
+  }
+  if (base >= end) return;
+  __builtin_amdgcn_sched_barrier(0);
+  const int step_rows = __builtin_amdgcn_readfirstlane(exact_div(kStep, inv)), step_cols = kStep - step_rows * t.ww;
+  const int row_pitch = p.W * pix_bytes, step = step_rows * row_pitch + step_cols * pix_bytes, wrap = row_pitch - t.ww * pix_bytes;
+  const int last_col = t.ww - first_col;
+#pragma unroll 2
+  for (; base < end; base += kWindowThreads) {
     row += step_rows; col += step_cols; off += (uint32_t)step;
     const bool over = col >= last_col;
     row += over ? 1 : 0;
     col -= over ? t.ww : 0;
     off += over ? (uint32_t)wrap : 0u;
+    load(base);
   }
 }
 
