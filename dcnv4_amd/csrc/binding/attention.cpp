@@ -406,14 +406,14 @@ PyObject *py_attention_backward_tiled(PyObject *, PyObject *const *args, Py_ssiz
   END_HANDLE_TH_ERRORS
 }
 
-// attention_tile(h, w, points, pairs): sides of the backward's tiles of a level of h x w cells with that many sampling points in each of
-// as many pairs (image, head, level)
+// attention_tile(h, w, points, pairs, bytes): sides of the backward's tiles of a level of h x w cells with that many sampling points in each
+// of as many pairs (image, head, level), for elements of that many bytes
 PyObject *py_attention_tile(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Args a("attention_tile", args, n, 4);
-  const int h = a.integer(), w = a.integer(), points = a.integer(), pairs = a.integer();
+  Args a("attention_tile", args, n, 5);
+  const int h = a.integer(), w = a.integer(), points = a.integer(), pairs = a.integer(), bytes = a.integer();
   int tile_h, tile_w;
-  fda_backward_tile(h, w, points, pairs, &tile_h, &tile_w);
+  fda_backward_tile(h, w, points, pairs, bytes, &tile_h, &tile_w);
   return Py_BuildValue("ii", tile_h, tile_w);
   END_HANDLE_TH_ERRORS
 }

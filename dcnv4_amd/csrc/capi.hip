@@ -789,8 +789,8 @@ bool fda_backward_tiled(int dtype, int spatial_size, int heads, int head_channel
          (unsigned long long)queries * row_bytes < (1ull << 31);
 }
 
-void fda_backward_tile(int h, int w, long long points, long long pairs, int *tile_h, int *tile_w) {
-  const FdaTile tile = fda_tile(h, w, points, fda_tile_points(points * pairs));
+void fda_backward_tile(int h, int w, long long points, long long pairs, int elem_bytes, int *tile_h, int *tile_w) {
+  const FdaTile tile = fda_tile(h, w, points, fda_tile_share(points * pairs, elem_bytes));
   *tile_h = tile.h; *tile_w = tile.w;
 }
 
@@ -1252,7 +1252,7 @@ static int fda_backward_impl(const void *value, const int64_t *spatial_shapes, c
         F.n_row = nb * F.Q;
         F.n_img = nb;
         F.zero_rows = rows.zero_rows && !fallback_possible ? rows.zero_rows + (size_t)b0 * spatial_size : nullptr;
-        F.tile_points = fda_tile_points((long long)num_query * num_points * num_levels * nb * num_heads);
+        F.tile_share = fda_tile_share((long long)num_query * num_points * num_levels * nb * num_heads, pr.s);
         hipError_t e = hipSuccess;
         if (pass == 0) fda_choose_order(&F, pr, spatial_size, num_heads, head_channels, num_levels, num_points, true);
         F.clear_state = (pass == 0 && b0 == 0) ? 1 : 0;

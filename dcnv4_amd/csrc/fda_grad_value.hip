@@ -62,7 +62,7 @@ struct LevelPlan {
 __device__ __forceinline__ LevelPlan level_plan(const FdaLaunch &p, int l) {
   LevelPlan lp;
   lp.H = (int)p.shapes[2 * l]; lp.W = (int)p.shapes[2 * l + 1]; lp.start = (int)p.level_start[l];
-  const FdaTile tile = fda_tile(lp.H, lp.W, (long long)p.Q * p.K, p.tile_points);
+  const FdaTile tile = fda_tile(lp.H, lp.W, (long long)p.Q * p.K, p.tile_share);
   lp.th = tile.h; lp.tw = tile.w;
   lp.nty = lp.H > 0 ? (lp.H + lp.th - 1) / lp.th : 0;
   lp.ntx = lp.W > 0 ? (lp.W + lp.tw - 1) / lp.tw : 0;

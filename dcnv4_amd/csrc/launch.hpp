@@ -248,7 +248,7 @@ struct FdaLaunch {
   int n_chunks;             // chunks of kFdaChunkPoints points per (image, head, level)
   int tile_stride;          // table row length: an upper bound of the tiles of one level
   int n_img;
-  int tile_points;          // a level whose tiles would collect more of them is cut finer
+  long long tile_share;     // fda_tile
   // a layer's backward: in place of grad_loc the gradients of the offsets that the locations come from, tensor dtype
   void *grad_offsets;       // [n_row][G * 2*L*K], rows offsets_pitch elements apart; those of grad_logits are then logits_pitch apart
   int offsets_pitch, logits_pitch;      // multiples of 4
@@ -269,23 +269,24 @@ constexpr int kFdaTakenStride = 64;            // words: dies that count in one 
 constexpr int kFdaWindowChannels = 32;         // of a head, that the grad_value kernel adds up at a time
 constexpr int kFdaMaxTilesPerLevel = 8192;     // LDS histogram of the binning kernel
 // The attention backward's tiles of a level of h x w cells with `points` sampling points: at most 8 x 8 cells, 16 tiles or more where there
-// are as many cells, 64 where a tile would hold more than tile_points.  No side is cut into more pieces than max(8, dim / 8 + 1), nor than
-// it has cells, so tiles are at most h * w / 8 + 64.
+// are as many cells, 64 where a tile would hold too large a part of all points (fda_tile_share).  No side is cut into more pieces than
+// max(8, dim / 8 + 1), nor than it has cells, so tiles are at most h * w / 8 + 64.
 struct FdaTile { int h, w; };
-__host__ __device__ inline FdaTile fda_tile(int h, int w, long long points, int tile_points) {
+__host__ __device__ inline FdaTile fda_tile(int h, int w, long long points, long long share) {
   auto side = [](int dim, int pieces) { const int n = (dim + pieces - 1) / pieces; return n < 1 ? 1 : n > 8 ? 8 : n; };
   const FdaTile coarse = {side(h, 4), side(w, 4)};
-  if (points * ((coarse.h + 1) * (coarse.w + 1)) <= (long long)tile_points * h * w) return coarse;
+  const long long cells = (long long)h * w, listed = points * ((coarse.h + 1) * (coarse.w + 1));      // times cells: of a tile
+  if (listed <= 1024 * cells || listed * (coarse.h + coarse.w) <= share * cells) return coarse;
   return {side(h, 8), side(w, 8)};
 }
-// A tile is worked on by one workgroup: no more points than about a share of them all, or it is what the launch waits for; smaller
-// tiles than that list more points twice.  us of a backward, shares of 350 / 800 / 2000: 1 image of a pyramid from 100 x 152, every
-// pixel a query, fp32 214 / 199 / 199, fp16 185 / 147 / 147; 1 of 160 x 160 352 / 317 / 317; 4 of 128 x 128 727 / 728 / 763, fp16 506 /
-// 505 / 550; 8 of 60 x 60 319 / 319 / 348; 2 of 100 x 152 340 / 346 / 353; 2 of 43 x 89 110 / 118 / 119.
-inline int fda_tile_points(long long all_points) {
-  const long long share = all_points / 800;
-  return (int)(share < 1024 ? 1024 : share > 0x7fffffff ? 0x7fffffff : share);
-}
+// A tile is worked on by one workgroup: where it holds more than about a workgroup's part of all points, the launch waits for it.  Finer
+// tiles list more points twice, the more the smaller they are - and the lanes of a step then meet in few cells - so a tile of sides
+// th + tw is cut if it holds more than all points / (50 (th + tw)), 60 of 16 bits, whose workgroups are smaller and more.  us of a backward,
+// every pixel a query, cut where a tile holds 1 / 800 of all points | so (never cut finer), fp32: 2 images of
+// a pyramid from 64 x 64 124 | 109 (108), of 43 x 89 114 | 107 (107), 6 of 36 x 36 111 | 104, 3 of 38 x 67 113 | 106, 2 of 100 x 152 329 |
+// 325 (323), 1 of 100 x 152 189 | 190 (217), 1 of 160 x 160 306 | 306 (340); fp16: 2 of 64 x 64 93 | 80 (80), 2 of 100 x 152 255 | 246 (266), 2 of
+// 100 x 100 170 | 170 (190), 1 of 100 x 152 140 | 142 (202), 3 of 120 x 35 124 | 115 (114).
+inline long long fda_tile_share(long long all_points, int elem_bytes) { return all_points / (elem_bytes == 4 ? 50 : 60); }
 __host__ __device__ inline size_t fda_key_stride(int Q, int K) { return ((size_t)Q * K + 1) & ~size_t(1); }
 
 enum FdaBackwardMode {

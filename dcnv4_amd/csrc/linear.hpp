@@ -181,6 +181,6 @@ int fda_layer_backward(const FdaLayerBackward &p, hipStream_t stream);
 // Whether the backward of deformable attention adds up grad_value by tiles; if not, with atomics.
 bool fda_backward_tiled(int dtype, int spatial_size, int heads, int head_channels, int levels, int queries, int points);
 // The sides of its tiles of a level of h x w cells, with that many sampling points in each of `pairs` (image, head, level).
-void fda_backward_tile(int h, int w, long long points, long long pairs, int *tile_h, int *tile_w);
+void fda_backward_tile(int h, int w, long long points, long long pairs, int elem_bytes, int *tile_h, int *tile_w);
 
 }  // namespace dcn

@@ -379,7 +379,7 @@ def test_tiles_of_a_level_are_no_more_than_their_table_holds():
     finer = 0
     for h in sides:
         for w in sides:
-            cuts = {ext._native.attention_tile(h, w, points, pairs) for points, pairs in ((1, 1), (1 << 20, 1))}
+            cuts = {ext._native.attention_tile(h, w, points, 1, size) for points in (1, 1 << 20) for size in (2, 4)}
             finer += len(cuts) > 1
             for tile_h, tile_w in cuts:
                 assert 1 <= tile_h <= 8 and 1 <= tile_w <= 8
