@@ -321,10 +321,14 @@ __global__ void __launch_bounds__(kTileCells * LPC, LPC == 8 ? 6 : 5) fda_grad_v
   const int workers = by_pair ? gridDim.x / kXcds : gridDim.x, me = by_pair ? blockIdx.x / kXcds : blockIdx.x;
   const int all_items = by_pair ? n_tiles * (BG / kXcds) : n_tiles * BG;
   // A workgroup's first two are given, the others go to whoever comes next: a tile of a coarse level holds ten times the points of
-  // one of the finest.  Launches for windows of channels take turns with the counters, each clears those of the one behind it.
-  const bool shared = (long long)QK * p.L >= (long long)kBatch * n_tiles;
+  // one of the finest.  Not where all XCDs would ask one counter, which answers them one by one: us of a backward, handed out | dealt, pyramids
+  // from 50 x 70, 3 images, 5 heads of 24, fp32 126 | 118, fp16 112 | 97; 64 x 64, 3 images, 3 heads, fp32 89 | 78, fp16 76 | 62; 128 x 128, 1
+  // image, 6 heads 162 | 159, 135 | 125; 100 x 152, 2 images, 6 heads 275 | 280, 217 | 208.  (Eight counters there and every eighth tile to an
+  // XCD: 268, 204, but registers that all others pay for with 1 %.)
+  // Launches for windows of channels take turns with the counters, each clears those of the one behind it.
+  const bool shared = by_pair && (long long)QK * p.L >= (long long)kBatch * n_tiles;
   const int turn = c0 / kFdaWindowChannels & 1;
-  uint32_t *taken = p.taken + (turn * kXcds + (by_pair ? blockIdx.x % kXcds : 0)) * kFdaTakenStride;
+  uint32_t *taken = p.taken + (turn * kXcds + blockIdx.x % kXcds) * kFdaTakenStride;
   if (blockIdx.x == 0 && tid < kXcds) p.taken[((turn ^ 1) * kXcds + tid) * kFdaTakenStride] = 0u;
   const int pairs = by_pair ? BG / kXcds : BG;
   // by a whole wave, a level a lane

@@ -47,10 +47,11 @@ def test_grad_value_by_tiles(oracle, name, dtype):
 # The same turns with sides that are powers of two, for data whose sums are exact: one lost or doubled point of one cell shows.
 # B, levels, G, D, K, Q, then which levels are cut finer and whether tiles are handed out (fda_grad_value_kernel's `shared`)
 EXACT = {
-    "groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000, [True], True),
+    "groups_of_chunks": (1, [(16, 16)], 1, 8, 4, 140000, [True], False),
+    "groups_handed_out": (1, [(16, 16)], 8, 8, 4, 140000, [True], True),
     "handed_out": (1, [(64, 128), (16, 8), (1, 1), (16, 16)], 8, 32, 4, 12000, [False, True, False, True], True),
     "windows_take_turns": (1, [(32, 64), (16, 16)], 8, 72, 4, 4000, [False, True], True),
-    "odd_pairs": (1, [(32, 16), (4, 2)], 3, 16, 6, 1111, [False, False], True),
+    "odd_pairs": (1, [(32, 16), (4, 2)], 3, 16, 6, 1111, [False, False], False),
     "empty_tiles": (1, [(128, 128), (64, 64)], 8, 32, 4, 9, [False, False], False),
 }
 
@@ -64,7 +65,7 @@ def test_grad_value_by_tiles_has_every_point_once(oracle, name, dtype):
     print(f"case {name} dtype {dtype}", flush=True)
     tiles = [ext._native.attention_tile(h, w, Q * K, len(levels) * B * G, dtype.itemsize) for h, w in levels]
     assert [t != ext._native.attention_tile(h, w, 1, 1, dtype.itemsize) for t, (h, w) in zip(tiles, levels)] == finer
-    assert (Q * K * len(levels) >= 256 * sum(-(-h // th) * -(-w // tw) for (h, w), (th, tw) in zip(levels, tiles))) == handed_out
+    assert (B * G % 8 == 0 and Q * K * len(levels) >= 256 * sum(-(-h // th) * -(-w // tw) for (h, w), (th, tw) in zip(levels, tiles))) == handed_out
     g = torch.Generator().manual_seed(len(name))
     v, shp, st, sla, go = make_fda_inputs(B, levels, G, D, K, Q, seed=1, dtype=torch.float32)
     rows = sla[..., :len(levels) * K * 2].view(B, Q, G, len(levels), K, 2)
