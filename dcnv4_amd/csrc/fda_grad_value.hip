@@ -27,7 +27,7 @@
 // come in the order of the queries, neighbours hit the same cells, and a step waits for its longest cell: a step takes every n-th block
 // of 32 (a line of numbers) of the list instead of 256 in a row.  What bounds it now are the VALU (two thirds busy) and LDS (half).
 //   us under a tracer, before -> now, 8 heads of 32 channels, levels from 100 x 152, four points: 2 images, every pixel a query, fp32
-// 291 -> 182; 300 queries, fp16, 29.3 -> 28.0 (5648 tiles of which most hold a point or none: there it gains nothing).  The whole
+// 291 -> 175; 300 queries, fp16, 29.3 -> 28.0 (5648 tiles of which most hold a point or none: there it gains nothing).  The whole
 // backward, every pixel a query: fp16, 1 image 246 -> 136, 2 images of 100 x 100 284 -> 170, 4 of 128 x 128 589 -> 467; fp32, 1 image 265
 // -> 190, 4 of 128 x 128 805 -> 704, 8 of 60 x 60 358 -> 300.
 //
